@@ -1,0 +1,56 @@
+"""fp32 attention of packed queries (16-query tiles, four a workgroup, waves that share a tile splitting its keys) at
+the sizes where its tiling turns: key counts around a block of 16 and a stage of 64, query counts around a tile, a pair
+of tiles and a workgroup of four, and key counts that leave some parts of a split without a key."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import dge_oracle as orc
+from util import assert_close, randn, rng
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [1, 0, 15, 16, 17, 32, 33, 48, 49, 64, 65, 80, 97, 128, 200]
+
+
+def _run(dev, q, k, v, lengths, scale):
+    from vtpack_amd import _C
+    got = _C.batched_sparse_attention_forward(*(torch.from_numpy(t).to(dev) for t in (q, k, v)),
+                                              torch.from_numpy(lengths), scale)
+    return got.cpu()
+
+
+@pytest.mark.parametrize("d", [64, 32])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 48, 63, 64, 65, 128, 129, 257, 300])
+def test_tiles_and_key_stages(dev, n, d):
+    h = 3
+    lengths = rng(900 + n).permutation(np.array(LENGTHS, dtype=np.int64))
+    L, B = int(lengths.sum()), len(lengths)
+    q, k, v = randn(901, h, L, d), randn(902, h, B, n, d), randn(903, h, B, n, d)
+    assert_close(_run(dev, q, k, v, lengths, d ** -0.5), orc.attention(q, k, v, lengths, d ** -0.5), torch.float32,
+                 f"fp32 attention over {n} keys")
+
+
+@pytest.mark.parametrize("shape", ["ramp", "late spike", "early spike", "steps"])
+def test_scores_far_above_the_first_stage(dev, shape):
+    """Running maxima that keep rising, one key hundreds above the rest, and jumps of 60 between stages, for tiles
+    that are whole (200 rows), split two ways (20) and four ways (5)."""
+    h, d, n = 2, 64, 257
+    lengths = np.array([200, 20, 5], dtype=np.int64)
+    q, k, v = 0.05 * randn(910, h, 225, d), 0.05 * randn(911, h, 3, n, d), randn(912, h, 3, n, d)
+    j = np.arange(n, dtype=np.float32)
+    q[..., 0] = 8.0
+    k[..., 0] = {"ramp": 0.25 * j, "late spike": np.where(j == n - 7, 300.0, 0.0),
+                 "early spike": np.where(j == 5, 300.0, 0.0), "steps": 60.0 * np.floor(j / 64)}[shape]
+    got = _run(dev, q, k, v, lengths, 0.125)
+    assert bool(torch.isfinite(got).all())
+    # scores reach 300: their fp32 rounding (300 x 2^-24 in the exponent, both sides) is 4e-5 of a probability
+    want = orc.attention(q, k, v, lengths, 0.125)
+    assert float((got - torch.from_numpy(want)).abs().max()) <= 4e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.5])
+def test_scale_zero_and_negative(dev, scale):
+    lengths = np.array([30, 70], dtype=np.int64)
+    q, k, v = randn(920, 1, 100, 64), randn(921, 1, 2, 40, 64), randn(922, 1, 2, 40, 64)
+    assert_close(_run(dev, q, k, v, lengths, scale), orc.attention(q, k, v, lengths, scale), torch.float32, "scale")

@@ -1,4 +1,5 @@
-// Sparse attention of packed queries against each sample's full K/V (gfx950).
+// Sparse attention of packed queries against each sample's full K/V (gfx950): the entry point, and the bf16 kernel for
+// what attention_dma.hip does not take (head_dim 32, a scale that is not positive).  fp32: attention_f32.hip.
 //
 // One 256-thread workgroup = (sample, head, chunk of 128 packed query rows);
 // each of its 4 waves owns 32 query rows.  K/V of the sample are streamed
@@ -24,28 +25,19 @@ namespace vtdge {
 constexpr int QROWS = 128;   // query rows per workgroup
 constexpr int KSTAGE = 128;  // keys per LDS stage (4 blocks of 32)
 
-template <typename T> struct ExpFn;
-template <> struct ExpFn<float> {
-    static __device__ __forceinline__ float f(float x) { return expf(x); }
-};
-template <> struct ExpFn<bf16_t> {
-    static __device__ __forceinline__ float f(float x) { return __expf(x); }
-};
-
-template <typename T, int D>
+template <int D>
 __global__ __launch_bounds__(256) void sparse_attention_kernel(
-    const T *__restrict__ q, int64_t q_rs, int64_t q_hs, const T *__restrict__ k, const T *__restrict__ v,
-    int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets, T *__restrict__ out,
-    int64_t o_rs, int64_t o_hs, int n, int qchunks, float scale)
+    const bf16_t *__restrict__ q, int64_t q_rs, int64_t q_hs, const bf16_t *__restrict__ k,
+    const bf16_t *__restrict__ v, int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets,
+    bf16_t *__restrict__ out, int64_t o_rs, int64_t o_hs, int n, int qchunks, float scale)
 {
-    constexpr int ESZ = sizeof(T);
-    constexpr int ROWB = D * ESZ;            // bytes of one K/V row (one head)
+    constexpr int ROWB = D * 2;              // bytes of one K/V row (one head)
     constexpr int NSLAB = ROWB / 32;         // 32-byte slabs along d
     constexpr int KP = ROWB + 16;            // K row pitch in LDS
-    constexpr int VP = KSTAGE * ESZ + 16;    // V^T row pitch in LDS
+    constexpr int VP = KSTAGE * 2 + 16;      // V^T row pitch in LDS
     constexpr int CPR = ROWB / 16;           // 16-byte chunks per K/V row
     constexpr int DB = D / 32;               // 32-wide head-dim blocks
-    constexpr int VEC = 16 / ESZ;
+    constexpr int VEC = 8;
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char *Ks = smem;
@@ -82,8 +74,8 @@ __global__ __launch_bounds__(256) void sparse_attention_kernel(
         for (int e = 0; e < 16; e++) o[i][e] = 0.f;
     float m_run = -INFINITY, l_run = 0.f;
 
-    const T *kb_ptr = k + (int64_t)b * kv_bs + (int64_t)head * kv_hs;
-    const T *vb_ptr = v + (int64_t)b * kv_bs + (int64_t)head * kv_hs;
+    const bf16_t *kb_ptr = k + (int64_t)b * kv_bs + (int64_t)head * kv_hs;
+    const bf16_t *vb_ptr = v + (int64_t)b * kv_bs + (int64_t)head * kv_hs;
 
     for (int key0 = 0; key0 < n; key0 += KSTAGE) {
         // ---- stage K rows and V^T into LDS (zero beyond n)
@@ -96,17 +88,11 @@ __global__ __launch_bounds__(256) void sparse_attention_kernel(
                 vv = *reinterpret_cast<const u32x4 *>(vb_ptr + (int64_t)key * kv_ts + ch * VEC);
             }
             *reinterpret_cast<u32x4 *>(Ks + kr * KP + ch * 16) = kk;
-            if constexpr (ESZ == 2) {
-                const uint32_t w[4] = {vv.x, vv.y, vv.z, vv.w};
+            const uint32_t w[4] = {vv.x, vv.y, vv.z, vv.w};
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const uint16_t h16 = (uint16_t)(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu);
-                    *reinterpret_cast<uint16_t *>(Vt + (ch * 8 + e) * VP + kr * 2) = h16;
-                }
-            } else {
-                const uint32_t w[4] = {vv.x, vv.y, vv.z, vv.w};
-#pragma unroll
-                for (int e = 0; e < 4; e++) *reinterpret_cast<uint32_t *>(Vt + (ch * 4 + e) * VP + kr * 4) = w[e];
+            for (int e = 0; e < 8; e++) {
+                const uint16_t h16 = (uint16_t)(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu);
+                *reinterpret_cast<uint16_t *>(Vt + (ch * 8 + e) * VP + kr * 2) = h16;
             }
         }
         __syncthreads();
@@ -125,7 +111,7 @@ __global__ __launch_bounds__(256) void sparse_attention_kernel(
 #pragma unroll
                     for (int sl = 0; sl < NSLAB; sl++) {
                         const u32x4 kf = *reinterpret_cast<const u32x4 *>(kp + sl * 32);
-                        Slab<T>::mma(kf, qf[sl], s[kb]);
+                        Slab<bf16_t>::mma(kf, qf[sl], s[kb]);
                     }
 #pragma unroll
                     for (int e = 0; e < 16; e++) {
@@ -138,7 +124,7 @@ __global__ __launch_bounds__(256) void sparse_attention_kernel(
             }
             mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
             const float m_new = fmaxf(m_run, mx);
-            const float alpha = ExpFn<T>::f(m_run - m_new);
+            const float alpha = __expf(m_run - m_new);
             m_run = m_new;
             l_run *= alpha;
 #pragma unroll
@@ -151,46 +137,27 @@ __global__ __launch_bounds__(256) void sparse_attention_kernel(
                 if (kb < nb) {
 #pragma unroll
                     for (int e = 0; e < 16; e++) {
-                        const float p = ExpFn<T>::f(s[kb][e] - m_new);
+                        const float p = __expf(s[kb][e] - m_new);
                         s[kb][e] = p;
                         l_run += p;
                     }
-                    if constexpr (ESZ == 2) {
 #pragma unroll
-                        for (int t = 0; t < 2; t++) {
-                            u32x4 pf;
-                            pf.x = pack_bf16x2(s[kb][8 * t + 0], s[kb][8 * t + 1]);
-                            pf.y = pack_bf16x2(s[kb][8 * t + 2], s[kb][8 * t + 3]);
-                            pf.z = pack_bf16x2(s[kb][8 * t + 4], s[kb][8 * t + 5]);
-                            pf.w = pack_bf16x2(s[kb][8 * t + 6], s[kb][8 * t + 7]);
+                    for (int t = 0; t < 2; t++) {
+                        u32x4 pf;
+                        pf.x = pack_bf16x2(s[kb][8 * t + 0], s[kb][8 * t + 1]);
+                        pf.y = pack_bf16x2(s[kb][8 * t + 2], s[kb][8 * t + 3]);
+                        pf.z = pack_bf16x2(s[kb][8 * t + 4], s[kb][8 * t + 5]);
+                        pf.w = pack_bf16x2(s[kb][8 * t + 6], s[kb][8 * t + 7]);
 #pragma unroll
-                            for (int db = 0; db < DB; db++) {
-                                const unsigned char *vp = Vt + (db * 32 + lr) * VP + (kb * 32 + 16 * t + 4 * lg) * 2;
-                                const u32x2 lo = *reinterpret_cast<const u32x2 *>(vp);
-                                const u32x2 hi = *reinterpret_cast<const u32x2 *>(vp + 16);
-                                u32x4 vf;
-                                vf.x = lo.x; vf.y = lo.y; vf.z = hi.x; vf.w = hi.y;
-                                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf),
-                                                                               __builtin_bit_cast(bf16x8, pf), o[db],
-                                                                               0, 0, 0);
-                            }
-                        }
-                    } else {
-#pragma unroll
-                        for (int g4 = 0; g4 < 4; g4++) {
-#pragma unroll
-                            for (int db = 0; db < DB; db++) {
-                                const unsigned char *vp = Vt + (db * 32 + lr) * VP + (kb * 32 + 8 * g4 + 4 * lg) * 4;
-                                const u32x4 vf = *reinterpret_cast<const u32x4 *>(vp);
-                                o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(vf.x), s[kb][4 * g4 + 0],
-                                                                            o[db], 0, 0, 0);
-                                o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(vf.y), s[kb][4 * g4 + 1],
-                                                                            o[db], 0, 0, 0);
-                                o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(vf.z), s[kb][4 * g4 + 2],
-                                                                            o[db], 0, 0, 0);
-                                o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(vf.w), s[kb][4 * g4 + 3],
-                                                                            o[db], 0, 0, 0);
-                            }
+                        for (int db = 0; db < DB; db++) {
+                            const unsigned char *vp = Vt + (db * 32 + lr) * VP + (kb * 32 + 16 * t + 4 * lg) * 2;
+                            const u32x2 lo = *reinterpret_cast<const u32x2 *>(vp);
+                            const u32x2 hi = *reinterpret_cast<const u32x2 *>(vp + 16);
+                            u32x4 vf;
+                            vf.x = lo.x; vf.y = lo.y; vf.z = hi.x; vf.w = hi.y;
+                            o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf),
+                                                                           __builtin_bit_cast(bf16x8, pf), o[db],
+                                                                           0, 0, 0);
                         }
                     }
                 }
@@ -203,7 +170,7 @@ __global__ __launch_bounds__(256) void sparse_attention_kernel(
     const float l_tot = l_run + __shfl_xor(l_run, 32, WAVE);
     if (!row_live) return;
     const float inv = 1.0f / l_tot;
-    T *op = out + (row0 + qrow) * o_rs + (int64_t)head * o_hs;
+    bf16_t *op = out + (row0 + qrow) * o_rs + (int64_t)head * o_hs;
 #pragma unroll
     for (int db = 0; db < DB; db++) {
 #pragma unroll
@@ -212,34 +179,35 @@ __global__ __launch_bounds__(256) void sparse_attention_kernel(
             float f[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) f[e] = o[db][4 * g4 + e] * inv;
-            if constexpr (ESZ == 2) {
-                u32x2 w;
-                w.x = pack_bf16x2(f[0], f[1]);
-                w.y = pack_bf16x2(f[2], f[3]);
-                *reinterpret_cast<u32x2 *>(op + d0) = w;
-            } else {
-                *reinterpret_cast<f32x4 *>(op + d0) = f32x4{f[0], f[1], f[2], f[3]};
-            }
+            u32x2 w;
+            w.x = pack_bf16x2(f[0], f[1]);
+            w.y = pack_bf16x2(f[2], f[3]);
+            *reinterpret_cast<u32x2 *>(op + d0) = w;
         }
     }
 }
 
-template <typename T, int D>
+template <int D>
 static int launch_attention(const void *q, int64_t q_rs, int64_t q_hs, const void *k, const void *v, int64_t kv_bs,
                             int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs,
                             int64_t o_hs, int B, int h, int n, int max_rows, float scale, hipStream_t st)
 {
-    constexpr int ESZ = sizeof(T);
-    const size_t lds = (size_t)KSTAGE * (D * ESZ + 16) + (size_t)D * (KSTAGE * ESZ + 16);
+    const size_t lds = (size_t)KSTAGE * (D * 2 + 16) + (size_t)D * (KSTAGE * 2 + 16);
     const int qchunks = (int)ceil_div(max_rows, QROWS);
-    auto kern = sparse_attention_kernel<T, D>;
+    auto kern = sparse_attention_kernel<D>;
     VT_RESERVE_LDS(kern, lds, "sparse_attention");
     dim3 grid((unsigned)((int64_t)B * qchunks), (unsigned)h), block(256);
     note_kernel(reinterpret_cast<const void *>(kern));
-    kern<<<grid, block, lds, st>>>((const T *)q, q_rs, q_hs, (const T *)k, (const T *)v, kv_bs, kv_ts, kv_hs, offsets,
-                                   (T *)out, o_rs, o_hs, n, qchunks, scale);
+    kern<<<grid, block, lds, st>>>((const bf16_t *)q, q_rs, q_hs, (const bf16_t *)k, (const bf16_t *)v, kv_bs, kv_ts, kv_hs, offsets,
+                                   (bf16_t *)out, o_rs, o_hs, n, qchunks, scale);
     return check_launch("sparse_attention");
 }
+
+// fp32 (attention_f32.hip)
+template <int D>
+int launch_attention_f32(const void *q, int64_t q_rs, int64_t q_hs, const void *k, const void *v, int64_t kv_bs,
+                         int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs, int64_t o_hs,
+                         int B, int h, int n, int max_rows, float scale, hipStream_t st);
 
 // bf16 / head_dim 64 fast path (attention_dma.hip)
 int launch_attention_bf16_d64(const void *q, int64_t q_rs, int64_t q_hs, const void *k, const void *v, int64_t kv_bs,
@@ -275,16 +243,14 @@ extern "C" int vtdge_sparse_attention(const void *q, int64_t q_row_stride, int64
         return launch_attention_bf16_d64(q, q_row_stride, q_head_stride, k, v, kv_batch_stride, kv_tok_stride,
                                          kv_head_stride, offsets, out, o_row_stride, o_head_stride, B, h, n,
                                          max_rows_per_sample, scale, st);
-#define VT_ATT(T, D)                                                                                                 \
-    return launch_attention<T, D>(q, q_row_stride, q_head_stride, k, v, kv_batch_stride, kv_tok_stride,             \
-                                  kv_head_stride, offsets, out, o_row_stride, o_head_stride, B, h, n,               \
-                                  max_rows_per_sample, scale, st)
+#define VT_ATT(launch)                                                                                              \
+    return launch(q, q_row_stride, q_head_stride, k, v, kv_batch_stride, kv_tok_stride, kv_head_stride, offsets,    \
+                  out, o_row_stride, o_head_stride, B, h, n, max_rows_per_sample, scale, st)
     if (dtype == VTDGE_F32) {
-        if (d == 64) VT_ATT(float, 64);
-        VT_ATT(float, 32);
-    } else {
-        if (d == 64) VT_ATT(bf16_t, 64);
-        VT_ATT(bf16_t, 32);
+        if (d == 64) VT_ATT(launch_attention_f32<64>);
+        VT_ATT(launch_attention_f32<32>);
     }
+    if (d == 64) VT_ATT(launch_attention<64>);
+    VT_ATT(launch_attention<32>);
 #undef VT_ATT
 }

@@ -1,0 +1,277 @@
+// Sparse attention of packed queries against each sample's full K/V, fp32 (gfx950).
+//
+// What bounds it: the fp32 matrix instructions (64 flops a clock and SIMD) and the vector instructions beside them,
+// which do not overlap with them, so the split keeps every SIMD's matrix pipe fed and the softmax short.
+//   * A workgroup is 64 query rows of one (sample, head): four waves of ONE 16-query tile each, on
+//     v_mfma_f32_16x16x4_f32.  Sixteen-row tiles waste less on ragged query counts and on n = 257 keys than 32-row ones
+//     (17 key blocks of 16 against 9 of 32), and in a workgroup of one or two tiles two waves share a tile and split
+//     its keys, adding up through LDS at the end.
+//   * K/V come in stages of 32 keys by direct loads into two LDS buffers (32 KB): four workgroups share a compute unit,
+//     and a stage's loads run under the stage before it.
+//   * All first chunks of the samples are dealt out before the second ones: whole workgroups first, remainders into
+//     the holes.
+// Measured at 64 samples x 6 heads, 26 to 199 queries (6402 rows), n = 257, d = 64: 45 us; workgroups of 8 tiles with
+// a ring of 3 or 4 stages 46 us; chunks of a sample next to each other 49 us; 2 tiles a workgroup 60 us; five or six
+// workgroups a compute unit 46 and 51 us.  At 128 rows for every sample 37 us, 87 TFLOP/s (8 tiles: 46 us).  At
+// one mix of 1/4/16 queries a region (7277 rows, 17 to 257 a sample) 48 us; the kernel before this one, 32-query tiles
+// on 128-row workgroups with K/V through registers, took 104 us.
+//
+// MFMA mapping: S^T = K Q^T (keys are rows, queries columns), then O^T = V^T P^T.  Lane (l = lane % 16, g = lane / 16)
+// holds S^T of keys 4 g + r (r < 4) and query l, which is exactly the B operand of the second product when its step r
+// contracts over keys 4 g + r: P never moves between lanes.  V stays row-major: in step r a lane needs V[4 g + r] at
+// NDB values of d, one per d block, and taking d = NDB l + db for block db makes them one vector read; the output then
+// has d = NDB (4 g + r) + db.  For the first product the contraction order is d = 16 j + 4 g + e for step (j, e): one
+// 16-byte read of K per four instructions.  K and V rows are stored with their 16-byte chunks XOR-ed by the row, which
+// keeps both kinds of read free of bank conflicts without padding (direct loads cannot pad).
+#include "common.h"
+
+namespace vtdge {
+
+constexpr int AF_KEYS = 32;      // keys per stage
+constexpr int AF_TILES = 4;      // waves = query tiles of a full workgroup
+constexpr int AF_RING = 2;       // stages in LDS
+constexpr float AF_RAISE = 8.f;  // log2 units a score may exceed its query's reference by
+
+template <int D> struct AttnF32 {
+    static constexpr int ROWB = D * 4;                        // bytes of a K/V row
+    static constexpr int CPR = ROWB / 16;                     // 16-byte chunks of it
+    static constexpr int BUF = 2 * AF_KEYS * ROWB;            // one stage: K then V
+    static constexpr int NDB = D / 16;                        // d blocks of the output
+    static __device__ __forceinline__ int slot(int row, int chunk)
+    {
+        return D == 64 ? chunk ^ (row & 15) : chunk ^ ((row >> 1) & 7);
+    }
+};
+
+template <int D>
+__global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
+    const float *__restrict__ q, int64_t q_rs, int64_t q_hs, const float *__restrict__ k, const float *__restrict__ v,
+    int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets, float *__restrict__ out,
+    int64_t o_rs, int64_t o_hs, int pairs, int h, int n, int chunks, float scale_log2)
+{
+    using G = AttnF32<D>;
+    constexpr int NL = G::BUF / 1024 / AF_TILES;              // direct loads a wave and stage
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+
+    // the chunks of a (sample, head) pair run on one XCD, so its K/V are fetched into one L2
+    const int rest = blockIdx.x >> 3, pairs_x = (pairs + 7) / 8;
+    const int pair = (rest % pairs_x) * 8 + (blockIdx.x & 7), chunk = rest / pairs_x;
+    if (pair >= pairs) return;
+    const int b = pair / h, head = pair - b * h;
+    const int64_t row0 = offsets[b];
+    const int Lb = (int)(offsets[b + 1] - row0);
+    if (chunk * 16 * AF_TILES >= Lb) return;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l = lane & 15, g = lane >> 4;
+    // tiles of this workgroup, and how its waves share them
+    const int tiles = min(AF_TILES, (Lb - chunk * 16 * AF_TILES + 15) / 16);
+    const int split = tiles <= AF_TILES / 2 ? 2 : 1;
+    const int tile = wid / split, part = wid % split;
+    const bool live = tile < tiles;
+    const int qrow = (chunk * AF_TILES + tile) * 16 + l;
+    const bool row_live = live && qrow < Lb;
+
+    const unsigned char *kbase = reinterpret_cast<const unsigned char *>(k + (int64_t)b * kv_bs + (int64_t)head * kv_hs);
+    const unsigned char *vbase = reinterpret_cast<const unsigned char *>(v + (int64_t)b * kv_bs + (int64_t)head * kv_hs);
+    const uint32_t rowp = (uint32_t)(kv_ts * 4);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+    // one stage: loads [wid NL, wid NL + NL) of its BUF / 1024, K rows first.  Rows past the last key repeat it.
+    auto load_stage = [&](int st) {
+        const int key0 = st * AF_KEYS, last = n - 1 - key0;
+        const uint32_t dst = lds0 + (uint32_t)((st % AF_RING) * G::BUF + wid * NL * 1024);
+        const void *base = uniform_ptr((wid < AF_TILES / 2 ? kbase : vbase) + (int64_t)key0 * rowp);
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const int row = ((wid % (AF_TILES / 2)) * NL + i) * (64 / G::CPR) + lane / G::CPR;
+            dma16(base, (uint32_t)min(row, last) * rowp + (uint32_t)G::slot(row, lane % G::CPR) * 16u, dst + i * 1024);
+        }
+    };
+
+    const int stages = (n + AF_KEYS - 1) / AF_KEYS;
+#pragma unroll
+    for (int i = 0; i < AF_RING - 1; i++)
+        if (i < stages) load_stage(i);
+    // queries times scale * log2(e): the scores come out of the matrix pipe in log2 units
+    f32x4 qf[D / 16];
+    {
+        const float *qp = q + (row0 + qrow) * q_rs + (int64_t)head * q_hs + 4 * g;
+#pragma unroll
+        for (int j = 0; j < D / 16; j++)
+            qf[j] = (row_live ? *reinterpret_cast<const f32x4 *>(qp + 16 * j) : f32x4{0.f, 0.f, 0.f, 0.f}) * scale_log2;
+    }
+    f32x4 o[G::NDB];
+#pragma unroll
+    for (int i = 0; i < G::NDB; i++) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // The softmax's reference m of a query: the accumulators of its scores start from -m, so a probability is one
+    // exp2 of what the matrix pipe delivers.  m is the query's maximum over its first stage and is raised (and the
+    // running sums rescaled) only when a score exceeds it by more than AF_RAISE; any reference cancels in the end.
+    float neg_m = 0.f, l_run = 0.f;
+    bool first = true;
+
+    // LDS offsets of this lane's fragments in a stage: K row l, V rows 4 g + r, of the block this part starts with
+    int koff[D / 16], voff[4];
+#pragma unroll
+    for (int j = 0; j < D / 16; j++) koff[j] = (part * 16 + l) * G::ROWB + G::slot(l, 4 * j + g) * 16;
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        voff[r] = (AF_KEYS + part * 16 + 4 * g + r) * G::ROWB +
+                  (D == 64 ? G::slot(4 * g + r, l) * 16 : G::slot(4 * g + r, l >> 1) * 16 + (l & 1) * 8);
+
+    // one stage of a wave: NB blocks of 16 keys (this part's only one, or both), keys >= n masked where TAIL
+    auto compute = [&](auto nbc, auto tailc, int st) {
+        constexpr int NB = decltype(nbc)::value;
+        constexpr bool TAIL = decltype(tailc)::value;
+        const unsigned char *S = smem + (st % AF_RING) * G::BUF;
+        const int key0 = st * AF_KEYS + part * 16 + 4 * g;    // this lane's first key of block 0
+        f32x4 s[NB];
+#pragma unroll
+        for (int i = 0; i < NB; i++) s[i] = f32x4{neg_m, neg_m, neg_m, neg_m};
+#pragma unroll
+        for (int j = 0; j < D / 16; j++)
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                const f32x4 kf = *reinterpret_cast<const f32x4 *>(S + koff[j] + i * 16 * G::ROWB);
+#pragma unroll
+                for (int e = 0; e < 4; e++) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[j][e], s[i], 0, 0, 0);
+            }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if constexpr (TAIL)
+                    if (key0 + 16 * i + r >= n) s[i][r] = -INFINITY;
+                mx = fmaxf(mx, s[i][r]);
+            }
+        if (first || __any(mx > AF_RAISE)) {
+            mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+            const float d = first ? mx : fmaxf(mx, 0.f);
+            neg_m -= d;
+#pragma unroll
+            for (int i = 0; i < NB; i++) s[i] -= d;
+            if (!first) {
+                const float alpha = __builtin_amdgcn_exp2f(-d);
+                l_run *= alpha;
+#pragma unroll
+                for (int i = 0; i < G::NDB; i++) o[i] *= alpha;
+            }
+            first = false;
+        }
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float p = __builtin_amdgcn_exp2f(s[i][r]);
+                l_run += p;
+                float vf[G::NDB];
+                const unsigned char *vp = S + voff[r] + i * 16 * G::ROWB;
+                if constexpr (D == 64) {
+                    const f32x4 t = *reinterpret_cast<const f32x4 *>(vp);
+                    vf[0] = t[0]; vf[1] = t[1]; vf[2] = t[2]; vf[3] = t[3];
+                } else {
+                    const f32x2 t = *reinterpret_cast<const f32x2 *>(vp);
+                    vf[0] = t[0]; vf[1] = t[1];
+                }
+                if constexpr (TAIL)                           // a repeated row: nothing of it, not even 0 * infinity
+                    if (key0 + 16 * i + r >= n)
+#pragma unroll
+                        for (int db = 0; db < G::NDB; db++) vf[db] = 0.f;
+#pragma unroll
+                for (int db = 0; db < G::NDB; db++)
+                    o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[db], p, o[db], 0, 0, 0);
+            }
+    };
+
+    for (int st = 0; st < stages; st++) {
+        // this wave's loads of stage st have landed once only those of the younger stages are outstanding
+        if (st + AF_RING - 2 < stages) wait_vmcnt<(AF_RING - 2) * NL>();
+        else wait_vmcnt<0>();
+        block_barrier();                                      // stage st is whole; the buffer of st - 1 is free
+        if (st + AF_RING - 1 < stages) load_stage(st + AF_RING - 1);
+        if (!live) continue;
+        const int left = n - st * AF_KEYS - part * 16;        // keys of this part's blocks of the stage, and beyond
+        if (split == 1) {
+            if (left >= 32) compute(std::integral_constant<int, 2>{}, std::false_type{}, st);
+            else if (left > 16) compute(std::integral_constant<int, 2>{}, std::true_type{}, st);
+            else compute(std::integral_constant<int, 1>{}, std::true_type{}, st);
+        } else {
+            if (left >= 16) compute(std::integral_constant<int, 1>{}, std::false_type{}, st);
+            else if (left > 0) compute(std::integral_constant<int, 1>{}, std::true_type{}, st);
+        }
+    }
+    float m_run = first ? -INFINITY : -neg_m;                 // a part without keys has no maximum
+
+    l_run += __shfl_xor(l_run, 16, WAVE);
+    l_run += __shfl_xor(l_run, 32, WAVE);
+    if (split > 1) {
+        // the parts of a tile meet in LDS: maximum, sum and accumulators of every part but the first
+        float *sh = reinterpret_cast<float *>(smem) + wid * (4 * G::NDB + 2) * 64 + lane;
+        lds_barrier();                                        // the last stage has been read
+        if (part > 0) {
+            sh[0] = m_run;
+            sh[64] = l_run;
+#pragma unroll
+            for (int db = 0; db < G::NDB; db++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) sh[(2 + 4 * db + r) * 64] = o[db][r];
+        }
+        lds_barrier();
+        if (part > 0) return;
+        for (int p = 1; p < split; p++) {
+            const float *sp = sh + p * (4 * G::NDB + 2) * 64;
+            const float m_new = fmaxf(m_run, sp[0]);
+            const float fa = __builtin_amdgcn_exp2f(m_run - m_new), fb = __builtin_amdgcn_exp2f(sp[0] - m_new);
+            m_run = m_new;
+            l_run = l_run * fa + sp[64] * fb;
+#pragma unroll
+            for (int db = 0; db < G::NDB; db++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) o[db][r] = o[db][r] * fa + sp[(2 + 4 * db + r) * 64] * fb;
+        }
+    }
+    if (!row_live) return;
+    const float inv = 1.0f / l_run;
+    float *op = out + (row0 + qrow) * o_rs + (int64_t)head * o_hs + 4 * G::NDB * g;
+    if constexpr (D == 64) {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            *reinterpret_cast<f32x4 *>(op + 4 * r) = f32x4{o[0][r] * inv, o[1][r] * inv, o[2][r] * inv, o[3][r] * inv};
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r += 2)
+            *reinterpret_cast<f32x4 *>(op + 2 * r) =
+                f32x4{o[0][r] * inv, o[1][r] * inv, o[0][r + 1] * inv, o[1][r + 1] * inv};
+    }
+}
+
+template <int D>
+int launch_attention_f32(const void *q, int64_t q_rs, int64_t q_hs, const void *k, const void *v, int64_t kv_bs,
+                         int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs, int64_t o_hs,
+                         int B, int h, int n, int max_rows, float scale, hipStream_t st)
+{
+    constexpr size_t lds = AF_RING * AttnF32<D>::BUF;
+    const int64_t pairs = (int64_t)B * h, chunks = ceil_div(max_rows, 16 * AF_TILES);
+    const int64_t grid = ceil_div(pairs, 8) * 8 * chunks;
+    VT_REQUIRE(grid < (1ll << 31), VTDGE_ERR_UNSUPPORTED, "sparse_attention: %lld workgroups exceed one launch",
+               (long long)grid);
+    VT_REQUIRE(kv_ts >= 0 && kv_ts < (1 << 23), VTDGE_ERR_UNSUPPORTED, "sparse_attention: token stride %lld",
+               (long long)kv_ts);
+    auto kern = attention_f32_kernel<D>;
+    VT_RESERVE_LDS(kern, lds, "sparse_attention");
+    note_kernel(reinterpret_cast<const void *>(kern));
+    kern<<<dim3((unsigned)grid), dim3(64 * AF_TILES), lds, st>>>(
+        (const float *)q, q_rs, q_hs, (const float *)k, (const float *)v, kv_bs, kv_ts, kv_hs, offsets, (float *)out,
+        o_rs, o_hs, (int)pairs, h, n, (int)chunks, scale * 1.44269504088896340736f);
+    return check_launch("sparse_attention");
+}
+template int launch_attention_f32<64>(const void *, int64_t, int64_t, const void *, const void *, int64_t, int64_t,
+                                      int64_t, const int64_t *, void *, int64_t, int64_t, int, int, int, int, float,
+                                      hipStream_t);
+template int launch_attention_f32<32>(const void *, int64_t, int64_t, const void *, const void *, int64_t, int64_t,
+                                      int64_t, const int64_t *, void *, int64_t, int64_t, int, int, int, int, float,
+                                      hipStream_t);
+
+}  // namespace vtdge
