@@ -349,7 +349,7 @@ static int go(const LinArgs &a, const PatchGeom &pg = PatchGeom{0, 0, 0, 0, 0, 0
     constexpr bool LATE = (BM / WGM) * (BN / WGN) > 64 * 64;      // wave tiles beyond 64 x 64
     constexpr size_t lds = (size_t)NSTAGE * (BM + BN) * DKB;
     static_assert(lds <= 160 * 1024, "LDS budget");
-    constexpr int WGS_PER_CU = lds <= 80 * 1024 ? 2 : 1;
+    constexpr int WGS_PER_CU = lds <= 53 * 1024 ? 3 : lds <= 80 * 1024 ? 2 : 1;
     auto kern = linear_dma_kernel<T, BM, BN, WGM, WGN, NWP, ACT, HB, HR, NSTAGE, LATE, PATCH>;
     VT_RESERVE_LDS(kern, lds, "linear");
     // persistent grid: what fits on the 256 CUs at once, but never more workgroups than tiles per XCD
@@ -397,6 +397,13 @@ int launch_linear_dma(const void *A, int64_t lda, const void *W, const void *bia
     // wide outputs: 256x128 tiles on 8 MFMA waves; narrow ones (N <= 512), and matrices that have fewer large tiles
     // than the chip has compute units (a classifier on 256 rows): 128x128 on 4, for more tiles.  Other shapes of the
     // same template (2 loader waves, 128x256 and 128x384 tiles on a two-stage ring) measured no faster.
+    // fp32: an instruction of 4096 flops takes 64 clocks, so the operand traffic of small tiles is hidden and what counts
+    // is how evenly they fill the chip: 64x64 tiles on four 32x32 waves, three workgroups a compute unit.  Measured
+    // against the two shapes below (rows, N, K): 32896, 384, 192: 62 against 70 us; 14300, 768, 192 + GELU: 54.5 against
+    // 69; 14300, 192, 768: 47 against 58.6; 24000, 64, 512: 24 against 41; 113, 384, 1536: 35 against 104.  From eight
+    // 256x128 tiles a compute unit on the larger tile wins: 65536, 1536, 384: 641 against 688 us.
+    if constexpr (sizeof(T) == 4)
+        if (ceil_div(rows, 256) * ceil_div(N, 128) < 2048) return pick_epilogue<T, 64, 64, 2, 2, 4>(a);
     if (N >= 768 && ceil_div(rows, 256) * ceil_div(N, 128) >= 256) return pick_epilogue<T, 256, 128, 4, 2, 4>(a);
     return pick_epilogue<T, 128, 128, 2, 2, 4>(a);
 }
@@ -423,6 +430,7 @@ int launch_patch_embed(const void *images, const void *W, const void *bias, cons
     // 78 us, when launches are timed back to back and the tail of one hides under the head of the next).
     // Eight loader waves instead of four (they also work out the patch addresses): 77.5 against 83.5 us; with two,
     // 201 us.  64x128 tiles: 108 us, 256x128 with eight loaders: 98 us.
+    if constexpr (sizeof(T) == 4) return go<T, 64, 64, 2, 2, 8, VTDGE_ACT_NONE, true, true, true>(a, pg);
     if (N >= 768) return go<T, 256, 128, 4, 2, 4, VTDGE_ACT_NONE, true, true, true>(a, pg);
     return go<T, 128, 128, 2, 2, 8, VTDGE_ACT_NONE, true, true, true>(a, pg);
 }
@@ -444,6 +452,7 @@ int launch_patch_linear(const void *tokens, const void *W, const void *bias, voi
     const PatchGeom pg{P, 0, 1, 0, 0, C, H, Wd};
     const int64_t rows = (int64_t)B * (H / P) * (Wd / P);
     LinArgs a{tokens, 0, W, bias, nullptr, 0, out, N, nullptr, rows, N, P * P * C, VTDGE_ACT_NONE, st};
+    if constexpr (sizeof(T) == 4) return go<T, 64, 64, 2, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
     if (N >= 768 || ceil_div(rows, 256) * ceil_div(N, 128) >= 512)
         return go<T, 256, 128, 4, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
     return go<T, 128, 128, 2, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
