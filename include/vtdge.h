@@ -400,6 +400,41 @@ int vtdge_batched_sparse_gemm(const void *a, const void *b, const int64_t *a_off
                               int trans_b, int64_t out_rows, int64_t out_cols, int64_t max_m, int dtype,
                               void *stream);
 
+/* A chain of DGE transformer blocks on one token grid (vtpack/models/dge/deit_dge.py:101-131 or pvt_dge.py:111-140,
+ * `depth` of them in a row), issued by one host call: the launches are those of the entry points above, in the order a
+ * caller that composes a block from them would issue them, with nothing of the host between them.
+ *   chain        what the blocks have in common.  H, W multiples of 4 and split sizes that divide 4 (`splits_124`: all
+ *                of them out of {1, 2, 4}); head dim 32 or 64; sr > 1 only without extra tokens
+ *   params_host  HOST table of device pointers, VTDGE_CHAIN_PARAMS per block, in this order (NULL where absent):
+ *                norm1 weight, bias, norm2 weight, bias, router weight, bias, splits (int64); q weight, bias, kv weight,
+ *                bias, proj weight, bias, fc1 weight, bias, fc2 weight, bias; packed copies (vtdge_linear_prepack) of
+ *                the q, kv, proj, fc1, fc2 weights; folded weight, column records (vtdge_layernorm_fold) and packed
+ *                copy of the folded weight for norm1 -> q, norm1 -> kv, norm2 -> fc1; with sr > 1 the reduction's
+ *                weight in [C, sr, sr, C] order, bias, and its norm's weight, bias.  The folded entries are needed
+ *                where vtdge_chain_layout says so
+ *   front_rows   nullable [extra, C]: stored as the extra tokens of every sample of x before anything reads them
+ *   x            [B, extra + H*W, C], the first block's input; out: the last block's output, same shape
+ *   ints, big, scratch   device buffers of the sizes vtdge_chain_layout returns, 256-byte aligned, nothing else using
+ *                them until the call's work is done.  `scratch` may be reused as soon as later work on `stream` runs
+ *   side_stream  nullable: a second stream for the routing half of every block where it helps; the call orders it
+ *                against `stream` on both ends
+ * vtdge_chain_layout fills layout_host[VTDGE_CHAIN_LAYOUT_HEAD + depth * VTDGE_CHAIN_LAYOUT_BLOCK]:
+ *   [0..2] bytes of ints, big, scratch; [3] bytes of status words per block or 0; [4] 1 if folded weights are needed;
+ *   then per block: offsets in `ints` of the gate logits, of offsets int64 [B+1], of lengths int64 [B] (-1: the
+ *   differences of the offsets), of the status words of the scatter-back that packed the block (-1: none; word 0 stays
+ *   0 unless it failed); offsets in `big` of its input tokens (-1: x itself), of its packed queries before and after
+ *   the block [B * (extra + H*W), C], of its patch descriptors int64 [B * (extra + H*W), 4]. */
+typedef struct {
+    int32_t B, H, W, C, heads, hidden, extra, S, depth, dtype, sr, splits_124;
+    float eps1, eps2, sr_eps, scale;
+} vtdge_chain;
+#define VTDGE_CHAIN_PARAMS 35
+#define VTDGE_CHAIN_LAYOUT_HEAD 8
+#define VTDGE_CHAIN_LAYOUT_BLOCK 8
+int vtdge_chain_layout(const vtdge_chain *chain, int64_t *layout_host);
+int vtdge_chain_forward(const vtdge_chain *chain, const void *const *params_host, const void *front_rows, void *x,
+                        void *ints, void *big, void *scratch, void *out, void *stream, void *side_stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,123 @@
+"""A chain of blocks issued by one call into the library against the same blocks composed launch by launch: the same
+kernels in the same order, so every output and every value of `states` is the same bit for bit."""
+import copy
+
+import pytest
+import torch
+
+from vtpack_amd import engine
+from vtpack_amd.models.dge.deit_dge import VisionTransformer
+from vtpack_amd.models.dge.pvt_dge import PyramidVisionTransformer
+from vtpack_amd.synthetic import set_synthetic_router, synthetic_images
+
+pytestmark = pytest.mark.gpu
+KEYS = ("comp", "input", "patches", "batches", "batches_device", "offsets_device", "gate", "queries", "size",
+        "num_extra_tokens")
+
+
+def _deit(dev, dtype, dim, img=128, depth=3, **kw):
+    torch.manual_seed(dim + depth)
+    m = VisionTransformer(img_size=img, patch_size=16, embed_dim=dim, depth=depth, num_heads=dim // 64, num_classes=40,
+                          split_sizes=[4, 2, 1], **kw)
+    return set_synthetic_router(m, 3).eval().to(dev).to(dtype)
+
+
+def _pvt(dev, dtype, img=128):
+    torch.manual_seed(9)
+    m = PyramidVisionTransformer(img_size=img, patch_size=4, embed_dims=[64, 128, 320, 512], num_heads=[1, 2, 5, 8],
+                                 mlp_ratios=[2, 2, 2, 2], qkv_bias=True, depths=[2, 1, 2, 1], sr_ratios=[8, 4, 2, 1],
+                                 split_sizes=[[4, 2, 1]] * 4, num_classes=30)
+    return set_synthetic_router(m, 4).eval().to(dev).to(dtype)
+
+
+def _blocks(m):
+    return list(m.blocks) if hasattr(m, "blocks") else [b for i in range(4) for b in getattr(m, f"block{i + 1}")]
+
+
+def _run(m, images, native):
+    engine.NATIVE_CHAIN = native
+    try:
+        with torch.no_grad():
+            out = m(images).clone()
+        return out, [{k: b.dge.states[k] for k in KEYS} for b in _blocks(m)]
+    finally:
+        engine.NATIVE_CHAIN = True
+
+
+def _same(a, b):
+    return torch.equal(a, b) if torch.is_tensor(a) else a == b
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim,batch,kw", [(64, 1, {}), (192, 3, {}), (384, 1, {}), (384, 33, {}), (384, 40, {"img": 192}),
+                                          (768, 2, {}), (384, 31, {"distilled": True}), (192, 2, {"cls_token": False}),
+                                          (384, 32, {"depth": 1})])
+@pytest.mark.parametrize("two_streams", [False, True])
+def test_deit(dev, dtype, dim, batch, kw, two_streams):
+    kw = dict(kw)
+    img = kw.get("img", 128)
+    m = _deit(dev, dtype, dim, **kw)
+    images = synthetic_images(batch, img, seed=5, dtype=dtype, device=dev)
+    before = engine.OVERLAP_FROM
+    engine.OVERLAP_FROM = 0 if two_streams else 1 << 62
+    try:
+        got, st = _run(m, images, True)
+    finally:
+        engine.OVERLAP_FROM = before
+    assert getattr(m.blocks[0], "_vtdge_chain").common is not None
+    want, wst = _run(m, images, False)
+    assert torch.equal(got, want)
+    for i, (a, b) in enumerate(zip(st, wst)):
+        for k in KEYS:
+            assert _same(a[k], b[k]), (i, k)
+
+
+@pytest.mark.parametrize("dtype,batch", [(torch.float32, 1), (torch.bfloat16, 3), (torch.bfloat16, 9)])
+def test_pvt(dev, dtype, batch):
+    m = _pvt(dev, dtype)
+    images = synthetic_images(batch, 128, seed=6, dtype=dtype, device=dev)
+    got, st = _run(m, images, True)
+    want, wst = _run(m, images, False)
+    assert torch.equal(got, want)
+    assert all(_same(a[k], b[k]) for a, b in zip(st, wst) for k in KEYS)
+
+
+def test_changes_of_the_parameters_are_seen(dev):
+    """In-place edits, a parameter or a module replaced, another data type, a copy of the model: each call works with
+    the parameters as they are then."""
+    m = _deit(dev, torch.bfloat16, 384)
+    images = synthetic_images(33, 128, seed=7, dtype=torch.bfloat16, device=dev)
+    first, _ = _run(m, images, True)
+    other = copy.deepcopy(m)
+    assert torch.equal(_run(other, images, True)[0], first)
+
+    def check(model, im=images, changed=True):
+        got = _run(model, im, True)[0]
+        assert torch.equal(got, _run(model, im, False)[0])
+        assert torch.equal(got, first) != changed
+
+    with torch.no_grad():
+        m.blocks[1].norm2.weight.mul_(1.5)
+    check(m)
+    check(other, changed=False)
+    other.blocks[2].attn.kv.weight = torch.nn.Parameter(other.blocks[2].attn.kv.weight.detach() * 2)
+    check(other)
+    fresh = torch.nn.Linear(384, 768)
+    with torch.no_grad():
+        fresh.weight.mul_(0.1)
+    m.blocks[0].mlp.fc1, m.blocks[0].mlp.fc2 = fresh.to(dev).bfloat16(), torch.nn.Linear(768, 384).to(dev).bfloat16()
+    check(m)                                     # the blocks are no longer alike: composed
+    m32 = copy.deepcopy(other).float()
+    assert torch.equal(_run(m32, images.float(), True)[0], _run(m32, images.float(), False)[0])
+
+
+def test_outputs_and_states_belong_to_their_call(dev):
+    m = _deit(dev, torch.bfloat16, 384)
+    a, b = (synthetic_images(n, 128, seed=8 + n, dtype=torch.bfloat16, device=dev) for n in (33, 40))
+    with torch.no_grad():
+        first = m(a)
+        kept, gate = first.clone(), m.blocks[1].dge.states["gate"]
+        gate_kept = gate.clone()
+        m(b)
+        m(b)
+    assert torch.equal(first, kept) and torch.equal(gate, gate_kept)

@@ -60,7 +60,19 @@ SIGNATURES = {
                                     _i, _i, _i, _p],
     "vtdge_sparse_attention": [_p, _l, _l, _p, _p, _l, _l, _l, _p, _p, _l, _l, _i, _i, _i, _i, _i, _f, _i, _p],
     "vtdge_batched_sparse_gemm": [_p, _p, _p, _p, _p, _i, _i, _l, _i, _l, _i, _i, _i, _l, _l, _l, _i, _p],
+    "vtdge_chain_layout": [_p, _p],
+    "vtdge_chain_forward": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p],
 }
+CHAIN_PARAMS, CHAIN_LAYOUT_HEAD, CHAIN_LAYOUT_BLOCK = 35, 8, 8      # include/vtdge.h
+
+
+class Chain(ctypes.Structure):
+    """vtdge_chain of include/vtdge.h."""
+    _fields_ = [(n, ctypes.c_int32) for n in ("B", "H", "W", "C", "heads", "hidden", "extra", "S", "depth", "dtype", "sr",
+                                              "splits_124")] + \
+               [(n, ctypes.c_float) for n in ("eps1", "eps2", "sr_eps", "scale")]
+
+
 EXPORTS = ["vtdge_version", "vtdge_last_error", "vtdge_last_kernel"] + list(SIGNATURES)
 
 _lib = None

@@ -8,10 +8,13 @@ elsewhere, with the packed query count kept in device memory: buffers are sized 
 token) and every packed kernel reads the live row count itself.  Nothing here synchronises, so the whole forward can
 be captured into a HIP graph.
 """
+import array
+import ctypes
+
 import torch
 
-from . import ops
-from .layers.dge import Deferred
+from . import _lib, ops
+from .layers.dge import BlockView, Deferred
 
 # Where the block runs on two streams, it has two independent chains before attention: the routing chain (router -> index->patch -> compress ->
 # q projection: small, latency-bound launches) and the key/value chain (LayerNorm of all tokens -> kv projection:
@@ -80,6 +83,23 @@ REGION_ROWS = True
 PACK_NEXT = True
 
 
+# A chain of blocks as one call into the library (`vtdge_chain_forward`): the same kernels in the same order, without
+# the 25 - 30 us of interpreter time each of them costs when it is issued from here (77 launches of a 12-block model:
+# 2.2 ms of host time, more than the GPU needs below a batch of about 150).  Taken where every switch above is at its
+# default and no per-launch timer is set; otherwise the blocks are composed by `block_forward`.
+NATIVE_CHAIN = True
+# Values of a natively issued chain (tokens times channels) from which the routing half of a block goes to a second
+# stream, where the block has no folded kernels.  Below, the fork and the join cost more than the overlap gives: one
+# stream against two, GPU time of a forward: 1001 against 1098 us (one 256 px picture, 384 channels), 1497 against 1515
+# (five, 768 channels); above: 4293 against 4174 (128, 192 channels fp32), 4654 against 4561 (99, 768 channels), 6847
+# against 6572 (256, PVT-Small).
+OVERLAP_FROM = 2 << 20
+_SWITCHES = ("OVERLAP", "FUSE_NEXT_NORM", "FUSE_ROUTER_NORM", "FUSE_NEXT_ROUTER", "FOLD_NORMS", "FUSE_PATCH_EMBED",
+             "ROUTING_ON_SIDE", "Q_AFTER_JOIN", "REGION_COMPRESS", "SERIAL_BESIDE_WEIGHT_STATIONARY", "ROUTING_FIRST",
+             "Q_BEFORE_KV", "PAIR_KV_Q", "ROUTER_STATS", "REGION_ROWS", "PACK_NEXT", "NATIVE_CHAIN")
+_defaults = tuple(globals()[name] for name in _SWITCHES)
+
+
 def _side_stream(device, slot=0):
     s = _side_streams.get((device, slot))
     if s is None:
@@ -109,6 +129,21 @@ def prepare(model):
                 if (w is not None and w.is_cuda and w.dtype == torch.bfloat16 and w.shape[1] == 384
                         and w.shape[0] % 384 == 0 and w.shape[0] <= 3072):
                     ops.folded_weight(w, lin.bias, norm.weight, norm.bias)
+    # and the address tables of its chains of blocks
+    chains = [list(model.blocks)] if hasattr(model, "blocks") else \
+        [list(getattr(model, f"block{i + 1}")) for i in range(getattr(model, "num_stages", 0))]
+    for i, blocks in enumerate(chains):
+        w = getattr(getattr(blocks[0].attn, "q", None), "weight", None) if blocks and hasattr(blocks[0], "attn") else None
+        if w is None or not w.is_cuda:
+            continue
+        extra = model.num_tokens if hasattr(model, "blocks") else int(i == len(chains) - 1)
+        plan = _chain_plan(blocks, w.dtype, w.device, w.shape[1], extra)
+        if plan is not None:
+            _chain_table(plan, blocks, False, False)
+            if w.dtype == torch.bfloat16:
+                c = plan.common
+                _chain_table(plan, blocks, c["C"] == 384 and c["sr"] == 1 and c["hidden"] % 384 == 0
+                             and c["hidden"] <= 3072, True)
     return model
 
 
@@ -379,9 +414,215 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
     return out
 
 
+class _ChainPlan:
+    """What a chain of blocks needs besides its input: the table of its parameters' addresses with the packed and
+    folded copies of its weights, and what the blocks have in common.  Checked against the parameters on every call
+    (`_chain_plan`) and made again when any of them has changed; never copied or pickled with its model."""
+
+    def __init__(self, key, common):
+        self.key, self.common = key, common
+        self.tables = {}        # (folded, packed copies wanted) -> (addresses, the derived tensors behind them)
+        self.layouts = {}       # (B, H, W) -> (vtdge_chain, layout)
+
+    def __deepcopy__(self, memo):
+        return None
+
+    def __reduce__(self):
+        return type(None), ()
+
+
+def _block_tensors(blk):
+    """The parameters of a block in the order of vtdge_chain_forward's table (the first 17 entries, then the spatial
+    reduction's four)."""
+    m = blk._modules
+    at, mlp, dge = m["attn"]._modules, m["mlp"]._modules, m["dge"]
+    gate = dge._modules["router"]._modules["gate"]._parameters
+    out = []
+    for mod in (m["norm1"], m["norm2"]):
+        pr = mod._parameters
+        out += (pr["weight"], pr["bias"])
+    out += (gate["weight"], gate["bias"], dge._parameters["splits"])
+    for mod in (at["q"], at["kv"], at["proj"], mlp["fc1"], mlp["fc2"]):
+        pr = mod._parameters
+        out += (pr["weight"], pr["bias"])
+    if "sr" in at:
+        for mod in (at["sr"], at["norm"]):
+            pr = mod._parameters
+            out += (pr["weight"], pr["bias"])
+    return out
+
+
+def _common_of(blocks, tensors, dtype, device, channels, extra):
+    """The numbers vtdge_chain wants, or None where the blocks are not alike or not of the shapes it takes."""
+    seen = None
+    for blk in blocks:
+        dge, attn, mlp = blk.dge, blk.attn, blk.mlp
+        C, hidden, sr = attn.q.weight.shape[0], mlp.fc1.weight.shape[0], getattr(attn, "sr_ratio", 1)
+        S = dge.router.gate.weight.shape[0]
+        shapes = [(attn.q, C, C), (attn.kv, 2 * C, C), (attn.proj, C, C), (mlp.fc1, hidden, C), (mlp.fc2, C, hidden),
+                  (dge.router.gate, S, C)]
+        norms = [blk.norm1, blk.norm2]
+        if sr > 1:
+            norms.append(attn.norm)
+            if (type(attn.sr) is not torch.nn.Conv2d or tuple(attn.sr.weight.shape) != (C, C, sr, sr) or attn.sr.bias is None
+                    or (C * dtype.itemsize) % 128):
+                return None
+        if any(type(n) is not torch.nn.LayerNorm or n.weight is None or n.bias is None or tuple(n.weight.shape) != (C,)
+               for n in norms):
+            return None
+        if any(type(lin) is not torch.nn.Linear or tuple(lin.weight.shape) != (n, k) for lin, n, k in shapes):
+            return None
+        splits = tuple(int(v) for v in dge.router.split_sizes)
+        if (C != channels or C % attn.num_heads or C // attn.num_heads not in (32, 64) or dge.router.gate.bias is None
+                or dge.region_size != 4 or len(splits) != S or S > _lib.MAX_SPLITS or dge.splits.numel() != S):
+            return None
+        if type(mlp.act) is not torch.nn.GELU or getattr(mlp.act, "approximate", "none") != "none":
+            return None
+        mine = dict(C=C, heads=attn.num_heads, hidden=hidden, S=S, sr=sr, splits_124=int(set(splits) <= {1, 2, 4}),
+                    eps1=blk.norm1.eps, eps2=blk.norm2.eps, sr_eps=attn.norm.eps if sr > 1 else 0.0,
+                    scale=float(attn.scale))
+        if seen is not None and mine != seen:
+            return None
+        seen = mine
+    for ts in tensors:
+        for i, t in enumerate(ts):
+            if t is not None and (t.device != device or not t.is_contiguous() or t.data_ptr() % 16
+                                  or t.dtype != (torch.int64 if i == 6 else dtype)):
+                return None
+    return dict(seen, extra=extra, depth=len(blocks), dtype=_lib.BF16 if dtype == torch.bfloat16 else _lib.F32)
+
+
+def _chain_plan(blocks, dtype, device, channels, extra):
+    """The plan of a chain of blocks for tokens of this kind, made anew where a parameter has changed since; None where
+    the blocks are composed one by one."""
+    if _lib.timer is not None or not ops.PACK_WEIGHTS or dtype not in (torch.float32, torch.bfloat16):
+        return None
+    g = globals()
+    if tuple(g[name] for name in _SWITCHES) != _defaults:
+        return None
+    try:
+        tensors = [_block_tensors(blk) for blk in blocks]
+        flat = [t for ts in tensors for t in ts]
+        key = ([0 if t is None else t.data_ptr() for t in flat], [0 if t is None else t._version for t in flat],
+               [None if t is None else t.dtype for t in flat], dtype, device, extra, channels,
+               [blk.attn.scale for blk in blocks], ops._pack_epoch, ops._plan_epoch)
+    except (KeyError, AttributeError):
+        return None
+    plan = getattr(blocks[0], "_vtdge_chain", None)
+    if plan is None or plan.key != key:
+        plan = _ChainPlan(key, _common_of(blocks, tensors, dtype, device, channels, extra))
+        object.__setattr__(blocks[0], "_vtdge_chain", plan)
+    return plan if plan.common is not None else None
+
+
+def _chain_layout(plan, B, H, W):
+    """(vtdge_chain, layout words) of a call on [B, extra + H*W, C], or None where the library refuses the shape (which
+    is left to the composition: it says what is wrong)."""
+    lay = plan.layouts.get((B, H, W))
+    if lay is None:
+        desc = _lib.Chain(B=B, H=H, W=W, **plan.common)
+        words = (ctypes.c_int64 * (_lib.CHAIN_LAYOUT_HEAD + desc.depth * _lib.CHAIN_LAYOUT_BLOCK))()
+        rc = _lib.load().vtdge_chain_layout(ctypes.addressof(desc), ctypes.addressof(words))
+        if len(plan.layouts) >= 64:
+            plan.layouts.clear()
+        lay = plan.layouts[(B, H, W)] = (desc, list(words)) if rc == 0 else (None, None)
+    return lay if lay[0] is not None else None
+
+
+def _chain_table(plan, blocks, folded, packs):
+    """The address table of the blocks' parameters (vtdge_chain_forward): with the packed copies of the weights, and of
+    the folded ones where those are used instead."""
+    made = plan.tables.get((folded, packs))
+    if made is None:
+        table, keep = [], []
+        for blk in blocks:
+            at, mlp = blk.attn, blk.mlp
+            ts = _block_tensors(blk)
+            derived = [ops.packed_weight(lin.weight) if packs and not (folded and lin in (at.q, at.kv, mlp.fc1)) else None
+                       for lin in (at.q, at.kv, at.proj, mlp.fc1, mlp.fc2)]
+            for norm, lin in ((blk.norm1, at.q), (blk.norm1, at.kv), (blk.norm2, mlp.fc1)):
+                derived += ops.folded_weight(lin.weight, lin.bias, norm.weight, norm.bias) if folded else (None,) * 3
+            tail = ([_khwc_weight(at.sr)] + ts[18:]) if len(ts) > 17 else [None] * 4
+            keep += derived + tail[:1]
+            table += [0 if t is None else t.data_ptr() for t in ts[:17] + derived + tail]
+        made = plan.tables[(folded, packs)] = (array.array("Q", table), keep)
+    return made[0]
+
+
+class _ChainBlock(BlockView):
+    """Block `i` of a chain that ran natively: its `states` values, made from the chain's buffers when they are read."""
+
+    KEYS = ("comp", "input", "patches", "batches", "batches_device", "offsets_device", "gate", "queries")
+
+    def __init__(self, run, i):
+        self.run, self.i = run, i
+
+    def _view(self, buf, at, dtype, *shape):
+        n = dtype.itemsize
+        for s in shape:
+            n *= s
+        return buf[at:at + n].view(dtype).view(shape)
+
+    def get(self, key):
+        x, ints, big, (desc, lay) = self.run
+        B, N, C = x.shape
+        o = lay[_lib.CHAIN_LAYOUT_HEAD + self.i * _lib.CHAIN_LAYOUT_BLOCK:][:_lib.CHAIN_LAYOUT_BLOCK]
+        if key == "input":
+            return x if o[4] < 0 else self._view(big, o[4], x.dtype, B, N, C)
+        if key == "gate":
+            return self._view(ints, o[0], x.dtype, B, desc.H // 4, desc.W // 4, desc.S)
+        offsets = self._view(ints, o[1], torch.int64, B + 1)
+        if key == "offsets_device":
+            return offsets
+        # the host-side counts and the tensors cut to the live rows: one device->host copy per read, nothing cached (a
+        # replay of a captured graph rewrites the buffers without running this code)
+        if o[3] >= 0 and int(self._view(ints, o[3], torch.int64, 1)) != 0:
+            raise RuntimeError("the scatter-back that packed this block's queries gave up waiting (see "
+                               "vtdge_decompress_router_compress): rows are missing")
+        live = offsets[1:] - offsets[:-1] if o[2] < 0 else self._view(ints, o[2], torch.int64, B)
+        if key == "batches_device":
+            return live
+        if key == "batches":
+            return live.cpu()
+        rows = int(live.sum())
+        if key == "patches":
+            return self._view(big, o[7], torch.int64, B * N, 4)[:rows]
+        return self._view(big, o[5 if key == "comp" else 6], x.dtype, B * N, C)[:rows]
+
+
+def _run_chain(blocks, x, H, W, front, plan, lay):
+    """`blocks` on x through vtdge_chain_forward."""
+    desc, words = lay
+    table = _chain_table(plan, blocks, bool(words[4]), x.dtype == torch.bfloat16 and x.shape[0] * x.shape[1] >= 2048)
+    for blk in blocks:      # what the last call left is about to be replaced: its buffers can serve this one
+        st = blk.dge.states
+        if isinstance(dict.get(st, "comp"), _ChainBlock):
+            st.update(dict.fromkeys(_ChainBlock.KEYS))
+    main = torch.cuda.current_stream(x.device)
+    side = 0
+    if not words[4] and x.numel() >= OVERLAP_FROM:
+        side = _side_stream(x.device, main.cuda_stream).cuda_stream
+    ints, big, scratch = (torch.empty((n,), dtype=torch.uint8, device=x.device) for n in words[:3])
+    out = torch.empty_like(x)
+    _lib.call("vtdge_chain_forward", ctypes.addressof(desc), table.buffer_info()[0],
+              0 if front is None else front.data_ptr(), x.data_ptr(), ints.data_ptr(), big.data_ptr(), scratch.data_ptr(),
+              out.data_ptr(), main.cuda_stream, side)
+    run = (x, ints, big, lay)
+    for i, blk in enumerate(blocks):
+        st = blk.dge.states
+        dict.update(st, dict.fromkeys(_ChainBlock.KEYS, _ChainBlock(run, i)))
+        st["size"], st["num_extra_tokens"] = (H, W), desc.extra
+    return out
+
+
 def _run_blocks(blocks, x, H, W, front=None):
     """A chain of blocks on one token grid, each handing the next what it has already computed for it.  `front`
     [extra, C]: rows the first block stores as the extra tokens of every sample before anything reads them."""
+    x = x.contiguous()
+    plan = _chain_plan(blocks, x.dtype, x.device, x.shape[-1], x.shape[1] - H * W) if blocks and x.is_cuda else None
+    lay = _chain_layout(plan, x.shape[0], H, W) if plan is not None else None
+    if lay is not None:
+        return _run_chain(blocks, x, H, W, front, plan, lay)
     carry = {"front": front} if front is not None else {}
     R = blocks[0].dge.region_size if blocks else 0
     if (PACK_NEXT and len(blocks) > 1 and R == 4

@@ -27,6 +27,14 @@ class Deferred:
         self.make = make
 
 
+class BlockView:
+    """Stands for every value one block of a natively issued chain leaves in `states`: `get(key)` makes the value when
+    it is read, from the buffers the whole chain shares."""
+
+    def get(self, key):
+        raise NotImplementedError
+
+
 class States(dict):
     """The `states` dict of a DynamicGrainedEncoder (vtpack/layers/dge.py:35-38, :81-84).
 
@@ -41,11 +49,13 @@ class States(dict):
     dict(states), {**states} - so code written against the reference's plain dict never sees a Deferred object."""
 
     @staticmethod
-    def _resolve(value):
-        return value.make() if isinstance(value, Deferred) else value
+    def _resolve(key, value):
+        if isinstance(value, Deferred):
+            return value.make()
+        return value.get(key) if isinstance(value, BlockView) else value
 
     def __getitem__(self, key):
-        return self._resolve(dict.__getitem__(self, key))
+        return self._resolve(key, dict.__getitem__(self, key))
 
     def get(self, key, default=None):
         return self[key] if key in self else default
@@ -75,7 +85,7 @@ class States(dict):
 
     def popitem(self):
         key, value = dict.popitem(self)
-        return key, self._resolve(value)
+        return key, self._resolve(key, value)
 
     def setdefault(self, key, default=None):
         if key not in self:

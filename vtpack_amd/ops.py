@@ -483,6 +483,7 @@ def layernorm_front_rows(x, count, weight, bias, eps=1e-6):
 
 PACK_WEIGHTS = True     # module switch (tests compare the two paths)
 _pack_epoch = 0         # bumped by invalidate_packed(): every packed copy made before is stale
+_plan_epoch = 0         # bumped by every invalidate_packed() call: tables of parameter addresses are made again
 
 
 def invalidate_packed(obj=None):
@@ -494,7 +495,8 @@ def invalidate_packed(obj=None):
     NOT see writes that bypass the version counter: `w.data.copy_(...)`, `w.data.mul_(...)`, a raw kernel writing
     into the storage.  After such a write call this function (or `engine.prepare(model)`) before the next forward;
     otherwise the weight-stationary kernels keep multiplying by the old weights."""
-    global _pack_epoch
+    global _pack_epoch, _plan_epoch
+    _plan_epoch += 1
     if obj is None:
         _pack_epoch += 1
         return
