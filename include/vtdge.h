@@ -400,6 +400,21 @@ int vtdge_batched_sparse_gemm(const void *a, const void *b, const int64_t *a_off
                               int trans_b, int64_t out_rows, int64_t out_cols, int64_t max_m, int dtype,
                               void *stream);
 
+/* out = act(LayerNorm(A) W^T + bias) for few rows, the LayerNorm done inside the Linear: norm1 -> kv and norm1 -> q
+ * (vtpack/models/dge/deit_dge.py:127 with :72-73; the two products share the launch) or norm2 -> fc1 -> GELU (:128 with
+ * :38-44) of a small batch.  LayerNorm(A) is rounded to the storage type before it is multiplied, as the two modules
+ * would.
+ *   A0 [rows0, K] leading dim lda0, W0 [N0, K], bias0 [N0] nullable, out0 [rows0, N0] dense, rows_dev0 nullable; the same
+ *   for the second product with the same K and LayerNorm, absent with rows1 = 0
+ * Taken where vtdge_layernorm_linear_fits says 1 (rows of whole 128-byte pieces and at most 1024 values, few tiles);
+ * VTDGE_ERR_UNSUPPORTED otherwise. */
+int vtdge_layernorm_linear_fits(int64_t rows0, int N0, int64_t rows1, int N1, int K, int dtype);
+int vtdge_layernorm_linear(const void *A0, int64_t lda0, const void *W0, const void *bias0, void *out0,
+                           const int64_t *rows_dev0, int64_t rows0, int N0, const void *A1, int64_t lda1, const void *W1,
+                           const void *bias1, void *out1, const int64_t *rows_dev1, int64_t rows1, int N1,
+                           const void *ln_weight, const void *ln_bias, float ln_eps, int K, int act, int dtype,
+                           void *stream);
+
 /* A chain of DGE transformer blocks on one token grid (vtpack/models/dge/deit_dge.py:101-131 or pvt_dge.py:111-140,
  * `depth` of them in a row), issued by one host call: the launches are those of the entry points above, in the order a
  * caller that composes a block from them would issue them, with nothing of the host between them.

@@ -60,6 +60,8 @@ SIGNATURES = {
                                     _i, _i, _i, _p],
     "vtdge_sparse_attention": [_p, _l, _l, _p, _p, _l, _l, _l, _p, _p, _l, _l, _i, _i, _i, _i, _i, _f, _i, _p],
     "vtdge_batched_sparse_gemm": [_p, _p, _p, _p, _p, _i, _i, _l, _i, _l, _i, _i, _i, _l, _l, _l, _i, _p],
+    "vtdge_layernorm_linear_fits": [_l, _i, _l, _i, _i, _i],
+    "vtdge_layernorm_linear": [_p, _l, _p, _p, _p, _p, _l, _i, _p, _l, _p, _p, _p, _p, _l, _i, _p, _p, _f, _i, _i, _i, _p],
     "vtdge_chain_layout": [_p, _p],
     "vtdge_chain_forward": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p],
 }

@@ -35,6 +35,7 @@ struct ChainPlan {
     int esz, N, n_kv;              // tokens per sample, keys per sample
     bool folded;                   // norms folded into weight-stationary Linears, chained scatter-back (384-channel bf16)
     bool by_region, pack;          // compress by region; the scatter-back packs the next block's queries
+    bool ln_kvq, ln_fc1;           // few rows: norm1 inside the kv and q Linear, norm2 inside fc1
     int64_t ws_words;
     // byte offsets
     int64_t ints_total, big_total, scratch_total;
@@ -68,6 +69,8 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
     p.by_region = c->splits_124 && nvec > 32 && nvec <= 64 && c->extra <= 64 && p.regions <= 65536 && p.rows < (1 << 24);
     p.folded = p.by_region && c->dtype == VTDGE_BF16 && c->C == 384 && p.rows >= 2048 && c->sr == 1 &&
                c->hidden % 384 == 0 && c->hidden <= 3072;
+    p.ln_kvq = !p.folded && c->sr == 1 && vtdge_layernorm_linear_fits(p.rows, 2 * c->C, p.cap, c->C, c->C, c->dtype);
+    p.ln_fc1 = !p.folded && vtdge_layernorm_linear_fits(p.cap, c->hidden, 0, 0, c->C, c->dtype);
     p.pack = p.folded && c->depth > 1 && p.regions % 4 == 0;
     p.ws_words = p.pack ? vtdge_decompress_router_compress_workspace(c->B, c->H, c->W, 4) / 8 : 0;
 
@@ -202,37 +205,44 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
                                hipStreamWaitEvent((hipStream_t)side, fork, 0) == hipSuccess,
                            VTDGE_ERR_LAUNCH, "chain: cannot fork to the side stream");
             }
-            char *comp_ln = scratch + p.comp_ln, *xln = scratch + p.xln;
+            char *comp_ln = p.ln_kvq ? nullptr : scratch + p.comp_ln, *xln = scratch + p.xln;
             if (!routed)
                 VT_TRY(vtdge_router(x, P[P_RW], P[P_RB], gate, idx, B, H, W, C, extra, 4, S, dt, routing));
             if (p.by_region) {
                 VT_TRY(vtdge_compress_regions(x, idx, splits, have_counts ? cnt : nullptr, comp, nullptr, 0.f, patches,
                                               p.cap, offsets, lengths, rr, B, H, W, C, extra, 4, S, dt, routing));
-                VT_TRY(vtdge_layernorm(comp, P[P_N1W], P[P_N1B], comp_ln, live, p.cap, C, c->eps1, dt, routing));
+                if (comp_ln != nullptr)
+                    VT_TRY(vtdge_layernorm(comp, P[P_N1W], P[P_N1B], comp_ln, live, p.cap, C, c->eps1, dt, routing));
             } else {
                 VT_TRY(vtdge_index_to_patch(idx, splits, B, H / 4, W / 4, S, 4, extra, patches, p.cap, offsets, lengths,
                                             routing));
-                VT_TRY(vtdge_compress(x, patches, live, p.cap, comp, comp_ln, P[P_N1W], P[P_N1B], c->eps1, B, N, C, W,
-                                      extra, dt, routing));
+                VT_TRY(vtdge_compress(x, patches, live, p.cap, comp, comp_ln, comp_ln ? P[P_N1W] : nullptr,
+                                      comp_ln ? P[P_N1B] : nullptr, c->eps1, B, N, C, W, extra, dt, routing));
             }
-            VT_TRY(vtdge_layernorm(x, P[P_N1W], P[P_N1B], xln, nullptr, p.rows, C, c->eps1, dt, stream));
-            char *src = xln;
-            if (c->sr > 1) {
-                char *red = scratch + p.red;
-                VT_TRY(vtdge_patch_linear(xln, P[P_SRW], P[P_SRB], red, B, H, W, C, c->sr, C, dt, stream));
-                // the normalised rows take the place of LN1(x), which nothing reads any more
-                VT_TRY(vtdge_layernorm(red, P[P_SRNW], P[P_SRNB], xln, nullptr, (int64_t)B * p.n_kv, C, c->sr_eps, dt,
-                                       stream));
+            if (p.ln_kvq) {
+                VT_TRY(vtdge_layernorm_linear(x, C, P[P_KVW], P[P_KVB], kv, nullptr, p.rows, 2 * C, comp, C, P[P_QW], P[P_QB],
+                                              q, live, p.cap, C, P[P_N1W], P[P_N1B], c->eps1, C, VTDGE_ACT_NONE, dt,
+                                              stream));
+            } else {
+                VT_TRY(vtdge_layernorm(x, P[P_N1W], P[P_N1B], xln, nullptr, p.rows, C, c->eps1, dt, stream));
+                char *src = xln;
+                if (c->sr > 1) {
+                    char *red = scratch + p.red;
+                    VT_TRY(vtdge_patch_linear(xln, P[P_SRW], P[P_SRB], red, B, H, W, C, c->sr, C, dt, stream));
+                    // the normalised rows take the place of LN1(x), which nothing reads any more
+                    VT_TRY(vtdge_layernorm(red, P[P_SRNW], P[P_SRNB], xln, nullptr, (int64_t)B * p.n_kv, C, c->sr_eps, dt,
+                                           stream));
+                }
+                const int64_t kv_rows = (int64_t)B * p.n_kv;
+                VT_TRY(vtdge_linear_prepacked(src, C, P[P_KVW], kv_rows >= 2048 ? P[P_KVP] : nullptr, P[P_KVB], nullptr, 0, kv,
+                                              2 * C, nullptr, kv_rows, 2 * C, C, VTDGE_ACT_NONE, dt, stream));
+                if (side != nullptr)
+                    VT_REQUIRE(hipEventRecord(join, (hipStream_t)side) == hipSuccess &&
+                                   hipStreamWaitEvent((hipStream_t)stream, join, 0) == hipSuccess,
+                               VTDGE_ERR_LAUNCH, "chain: cannot join the side stream");
+                VT_TRY(vtdge_linear_prepacked(comp_ln, C, P[P_QW], pk(P_QP), P[P_QB], nullptr, 0, q, C, live, p.cap, C, C,
+                                              VTDGE_ACT_NONE, dt, stream));
             }
-            const int64_t kv_rows = (int64_t)B * p.n_kv;
-            VT_TRY(vtdge_linear_prepacked(src, C, P[P_KVW], kv_rows >= 2048 ? P[P_KVP] : nullptr, P[P_KVB], nullptr, 0, kv,
-                                          2 * C, nullptr, kv_rows, 2 * C, C, VTDGE_ACT_NONE, dt, stream));
-            if (side != nullptr)
-                VT_REQUIRE(hipEventRecord(join, (hipStream_t)side) == hipSuccess &&
-                               hipStreamWaitEvent((hipStream_t)stream, join, 0) == hipSuccess,
-                           VTDGE_ERR_LAUNCH, "chain: cannot join the side stream");
-            VT_TRY(vtdge_linear_prepacked(comp_ln, C, P[P_QW], pk(P_QP), P[P_QB], nullptr, 0, q, C, live, p.cap, C, C,
-                                          VTDGE_ACT_NONE, dt, stream));
         }
         VT_TRY(vtdge_sparse_attention(q, C, d, kv, kv + (int64_t)C * esz, (int64_t)p.n_kv * 2 * C, 2 * C, d, offsets, o, C,
                                       d, B, c->heads, d, p.n_kv, N, c->scale, dt, stream));
@@ -245,9 +255,15 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
             char *q1_ln = scratch + p.q1_ln;
             VT_TRY(vtdge_linear_prepacked(o, C, P[P_PROJW], pk(P_PROJP), P[P_PROJB], comp, C, q1, C, live, p.cap, C, C,
                                           VTDGE_ACT_NONE, dt, stream));
-            VT_TRY(vtdge_layernorm(q1, P[P_N2W], P[P_N2B], q1_ln, live, p.cap, C, c->eps2, dt, stream));
-            VT_TRY(vtdge_linear_prepacked(q1_ln, C, P[P_FC1W], pk(P_FC1P), P[P_FC1B], nullptr, 0, hid, c->hidden, live,
-                                          p.cap, c->hidden, C, VTDGE_ACT_GELU, dt, stream));
+            if (p.ln_fc1) {
+                VT_TRY(vtdge_layernorm_linear(q1, C, P[P_FC1W], P[P_FC1B], hid, live, p.cap, c->hidden, nullptr, 0, nullptr,
+                                              nullptr, nullptr, nullptr, 0, 0, P[P_N2W], P[P_N2B], c->eps2, C,
+                                              VTDGE_ACT_GELU, dt, stream));
+            } else {
+                VT_TRY(vtdge_layernorm(q1, P[P_N2W], P[P_N2B], q1_ln, live, p.cap, C, c->eps2, dt, stream));
+                VT_TRY(vtdge_linear_prepacked(q1_ln, C, P[P_FC1W], pk(P_FC1P), P[P_FC1B], nullptr, 0, hid, c->hidden, live,
+                                              p.cap, c->hidden, C, VTDGE_ACT_GELU, dt, stream));
+            }
         }
         VT_TRY(vtdge_linear_prepacked(hid, c->hidden, P[P_FC2W], pk(P_FC2P), P[P_FC2B], q1, C, q2, C, live, p.cap, C,
                                       c->hidden, VTDGE_ACT_NONE, dt, stream));
@@ -327,5 +343,5 @@ extern "C" int vtdge_chain_forward(const vtdge_chain *chain, const void *const *
         VT_REQUIRE(ok, VTDGE_ERR_ARG, "chain: block %d lacks a parameter", i);
     }
     return run_chain(chain, p, params_host, front_rows, (char *)x, (char *)ints, (char *)big, (char *)scratch, (char *)out,
-                     stream, p.folded ? nullptr : side_stream);
+                     stream, p.folded || p.ln_kvq ? nullptr : side_stream);
 }

@@ -19,35 +19,12 @@
 // wait for the prefetches still in flight.  The epilogue stays in registers
 // (a half-wave swap gives each lane 8 consecutive bf16 columns), so LDS holds
 // nothing but the operand ring.
-#include "common.h"
+#include "patch_source.h"
 #include <stdlib.h>
 
 namespace vtdge {
 
 constexpr int DKB = 128;  // K bytes per stage
-
-// GELU(x) = x * Phi(x).  fp32 keeps the exact erf form.  For bf16 outputs Phi is a degree-15 odd minimax
-// polynomial on [-4, 4] (x clamped there): no transcendental, 11 VALU instructions; |error| <= 1.3e-4 for
-// |x| <= 4 and <= 5.3e-5 * |x| beyond, i.e. below 1/30 of a bf16 rounding step of the result.
-template <typename T> __device__ __forceinline__ float gelu_fn(float v);
-template <> __device__ __forceinline__ float gelu_fn<float>(float v)
-{
-    return 0.5f * v * (1.0f + erff(v * 0.70710678118654752440f));
-}
-template <> __device__ __forceinline__ float gelu_fn<bf16_t>(float v)
-{
-    const float x = __builtin_amdgcn_fmed3f(v, -4.0f, 4.0f);
-    const float t = x * x;
-    float q = -1.580785487e-09f;
-    q = q * t + 1.217110604e-07f;
-    q = q * t - 4.100865225e-06f;
-    q = q * t + 8.066737963e-05f;
-    q = q * t - 1.048204291e-03f;
-    q = q * t + 9.664873803e-03f;
-    q = q * t - 6.617537860e-02f;
-    q = q * t + 3.988475095e-01f;
-    return v * (x * q + 0.5f);
-}
 
 // Persistent, wave-specialised kernel.  A workgroup = WGM*WGN MFMA waves + NWP loader waves.  It walks a static
 // list of output tiles; the 3-deep operand ring keeps running across tile boundaries, so the first stages of the
@@ -61,25 +38,7 @@ template <> __device__ __forceinline__ float gelu_fn<bf16_t>(float v)
 // trims each XCD's list.
 // NSTAGE = depth of the operand ring (3, or 2 for tiles whose stages are too large for three); LATE = fetch bias and
 // residual in the epilogue itself instead of during the last stage (large wave tiles have no registers to park them).
-//
-// PATCH: the kernel is a patch embedding (a convolution whose stride is its kernel size, as a Linear over the
-// patches).  A is the image batch [B, Cin, S, S] itself: row (b, gy, gx) of the product is patch (gy, gx) of image b
-// and its K index runs over (channel, row of the patch, pixel), so a 128-byte K slab of a row is a few consecutive
-// pixel rows of one channel of the patch and the loader waves fetch them straight from the image - nothing but
-// their per-lane source addresses differs from the plain kernel, no unfolded copy of the images exists.  The output
-// row goes to token `extra + gy G + gx` of sample b in [B, extra + G G, N], and the residual is row
-// `extra + gy G + gx` of one [extra + G G, N] table for every sample (the position embedding).
-//
-// The same mode reads patches of a channels-last token grid (cl_C > 0): A is [B, cl_H cl_W, cl_C] tokens, row
-// (b, gy, gx) of the product is the P x P block of tokens at (gy P, gx P) and its K index runs over (token row of
-// the block, token of that row, channel), i.e. a 128-byte K slab is a piece of one token's channels (cl_C values
-// must fill whole slabs).  This is a stride-P P x P convolution over the grid with its weight in [O, kh, kw, C]
-// order; rows of the product are stored densely (extra = 0) and there is no residual.
-struct PatchGeom {
-    int P, S, G, Cin, extra;     // patch edge, image edge, patches per edge, input channels, tokens in front
-    int cl_C, cl_H, cl_W;        // channels-last source: channels and token grid (cl_C = 0: an image batch)
-};
-
+// PATCH: the rows of A are patches of images or blocks of tokens, read in place (patch_source.h).
 template <typename T, int BM, int BN, int WGM, int WGN, int NWP, int ACT, bool HAS_BIAS, bool HAS_RES, int NSTAGE = 3,
           bool LATE = false, bool PATCH = false>
 __global__ __launch_bounds__((WGM * WGN + NWP) * 64) void linear_dma_kernel(
@@ -130,21 +89,7 @@ __global__ __launch_bounds__((WGM * WGN + NWP) * 64) void linear_dma_kernel(
                     int64_t gm = m0 + r;
                     gm = gm < M ? gm : M - 1;
                     if constexpr (PATCH) {
-                        if (pg.cl_C > 0) {
-                            // block (b, gy, gx) of the token grid: its first token; the slab's piece is added per stage
-                            const int gw = pg.cl_W / pg.P, g2 = (pg.cl_H / pg.P) * gw;
-                            const int gmi = (int)gm, b = gmi / g2, t = gmi - b * g2, gy = t / gw, gx = t - gy * gw;
-                            src[i] = reinterpret_cast<const unsigned char *>(
-                                         A + (((int64_t)b * pg.cl_H + gy * pg.P) * pg.cl_W + gx * pg.P) * pg.cl_C) +
-                                     chunk * 16;
-                        } else {
-                            // patch (b, gy, gx); the chunk is pixels `cc` of patch row `cr` of the slab's first rows
-                            const int g2 = pg.G * pg.G, cpr = pg.P * ESZ / 16;      // chunks per patch row
-                            const int gmi = (int)gm, b = gmi / g2, t = gmi - b * g2, gy = t / pg.G, gx = t - gy * pg.G;
-                            const int cr = chunk / cpr, cc = chunk % cpr;
-                            src[i] = reinterpret_cast<const unsigned char *>(
-                                         A + ((int64_t)b * pg.Cin * pg.S + gy * pg.P + cr) * pg.S + gx * pg.P) + cc * 16;
-                        }
+                        src[i] = reinterpret_cast<const unsigned char *>(A) + patch_row_offset<T>(pg, (int)gm, chunk);
                     } else {
                         src[i] = reinterpret_cast<const unsigned char *>(A + gm * lda) + chunk * 16;
                     }
@@ -160,18 +105,7 @@ __global__ __launch_bounds__((WGM * WGN + NWP) * 64) void linear_dma_kernel(
         auto issue_next = [&]() {
             unsigned char *dst = smem + (issued % NSTAGE) * STAGE + lw * NLW * 1024;
             int64_t a_off = (int64_t)it_kt * DKB;
-            if constexpr (PATCH) {
-                if (pg.cl_C > 0) {
-                    // slab it_kt of a block of tokens: which token of the block and where in its channels
-                    const int spt = pg.cl_C * ESZ / DKB;                       // slabs per token
-                    const int tk = it_kt / spt, dy = tk / pg.P, dx = tk - dy * pg.P;
-                    a_off = ((int64_t)(dy * pg.cl_W + dx) * pg.cl_C) * ESZ + (int64_t)(it_kt - tk * spt) * DKB;
-                } else {
-                    // slab it_kt of a patch: its channel and its first row in the patch
-                    const int rps = DKB / (pg.P * ESZ), spc = pg.P / rps;      // rows per slab, slabs per channel
-                    a_off = ((int64_t)(it_kt / spc) * pg.S + (it_kt % spc) * rps) * pg.S * ESZ;
-                }
-            }
+            if constexpr (PATCH) a_off = patch_slab_offset<T>(pg, it_kt);
 #pragma unroll
             for (int i = 0; i < NLW; i++) {
                 const bool a_rows = (lw * NLW + i) * 8 < BM;
@@ -201,11 +135,11 @@ __global__ __launch_bounds__((WGM * WGN + NWP) * 64) void linear_dma_kernel(
     // where row `row` of the product is stored and which row of the residual it takes
     // (32-bit arithmetic: the patch count of a batch fits, and a 64-bit division costs a hundred instructions)
     auto out_row = [&](int64_t row) -> int64_t {
-        if constexpr (PATCH) { const int g2 = pg.G * pg.G; return row + ((int)row / g2 + 1) * pg.extra; }
+        if constexpr (PATCH) return patch_out_row(pg, (int)row);
         else return row;
     };
     auto res_row = [&](int64_t row) -> int64_t {
-        if constexpr (PATCH) { const int g2 = pg.G * pg.G; return (int)row % g2 + pg.extra; }
+        if constexpr (PATCH) return patch_res_row(pg, (int)row);
         else return row;
     };
     const int wm = wid / WGN, wn = wid % WGN;
@@ -408,6 +342,12 @@ int launch_linear_dma(const void *A, int64_t lda, const void *W, const void *bia
     return pick_epilogue<T, 128, 128, 2, 2, 4>(a);
 }
 
+// few rows (linear_small.hip)
+bool patch_small_wanted(int64_t rows, int N, int K, int esz, int64_t source_bytes);
+template <typename T>
+int launch_patch_small(const void *source, const void *W, const void *bias, const void *res, void *out, int64_t rows, int N,
+                       int K, const PatchGeom &pg, hipStream_t st);
+
 // The patch embedding: images [B, Cin, S, S] -> tokens [B, extra + G G, N] rows extra.., = conv + bias + pos.
 bool patch_embed_applicable(int P, int S, int Cin, int N, int esz, const void *images, const void *weight,
                             const void *bias, const void *pos, const void *out)
@@ -425,6 +365,8 @@ int launch_patch_embed(const void *images, const void *W, const void *bias, cons
     const int G = S / P;
     const PatchGeom pg{P, S, G, Cin, extra, 0, 0, 0};
     LinArgs a{images, 0, W, bias, pos, N, out, N, nullptr, (int64_t)B * G * G, N, Cin * P * P, VTDGE_ACT_NONE, st};
+    if (patch_small_wanted(a.rows, N, a.K, sizeof(T), (int64_t)B * Cin * S * S * sizeof(T)))
+        return launch_patch_small<T>(images, W, bias, pos, out, a.rows, N, a.K, pg, st);
     // 128x128 tiles, two workgroups per CU, unless the output is wide.  At 256 x 256 patches and N = 384 a launch takes
     // 80 - 88 us against 125 - 138 us on 256x128 tiles with one workgroup per CU (which only looks faster, 67 against
     // 78 us, when launches are timed back to back and the tail of one hides under the head of the next).
@@ -452,6 +394,8 @@ int launch_patch_linear(const void *tokens, const void *W, const void *bias, voi
     const PatchGeom pg{P, 0, 1, 0, 0, C, H, Wd};
     const int64_t rows = (int64_t)B * (H / P) * (Wd / P);
     LinArgs a{tokens, 0, W, bias, nullptr, 0, out, N, nullptr, rows, N, P * P * C, VTDGE_ACT_NONE, st};
+    if (patch_small_wanted(rows, N, a.K, sizeof(T), (int64_t)B * H * Wd * C * sizeof(T)))
+        return launch_patch_small<T>(tokens, W, bias, nullptr, out, rows, N, a.K, pg, st);
     if constexpr (sizeof(T) == 4) return go<T, 64, 64, 2, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
     if (N >= 768 || ceil_div(rows, 256) * ceil_div(N, 128) >= 512)
         return go<T, 256, 128, 4, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);

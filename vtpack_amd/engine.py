@@ -40,6 +40,9 @@ FUSE_NEXT_ROUTER = True
 # takes the raw rows and a 32-byte statistics record per row, so no normalised copy of the tokens is written or read.
 # Taken where the weight-stationary kernel applies (bf16, 384 channels, 2048 rows or more, no spatial reduction).
 FOLD_NORMS = True
+# Few rows: norm1 inside the key/value and query Linears (one launch for the two) and norm2 inside fc1
+# (`vtdge_layernorm_linear`), in place of the LayerNorm kernels.
+NORM_IN_LINEAR = True
 # The patch embedding read straight from the images, position embedding added in its epilogue (`vtdge_patch_embed`),
 # instead of an unfolded copy of the images, a Linear, a copy into the token tensor and an addition.
 FUSE_PATCH_EMBED = True
@@ -96,7 +99,7 @@ NATIVE_CHAIN = True
 OVERLAP_FROM = 2 << 20
 _SWITCHES = ("OVERLAP", "FUSE_NEXT_NORM", "FUSE_ROUTER_NORM", "FUSE_NEXT_ROUTER", "FOLD_NORMS", "FUSE_PATCH_EMBED",
              "ROUTING_ON_SIDE", "Q_AFTER_JOIN", "REGION_COMPRESS", "SERIAL_BESIDE_WEIGHT_STATIONARY", "ROUTING_FIRST",
-             "Q_BEFORE_KV", "PAIR_KV_Q", "ROUTER_STATS", "REGION_ROWS", "PACK_NEXT", "NATIVE_CHAIN")
+             "Q_BEFORE_KV", "PAIR_KV_Q", "ROUTER_STATS", "REGION_ROWS", "PACK_NEXT", "NORM_IN_LINEAR", "NATIVE_CHAIN")
 _defaults = tuple(globals()[name] for name in _SWITCHES)
 
 
@@ -214,7 +217,9 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
     fold1 = (FOLD_NORMS and x_ln is None and getattr(attn, "sr_ratio", 1) <= 1
              and ops.fits_linear_layernorm(x, attn.kv.weight))
     use_regions = REGION_COMPRESS and ops.fits_compress_regions(x, H, W, R, dge.router.split_sizes)
-    overlap = overlap and OVERLAP and not (SERIAL_BESIDE_WEIGHT_STATIONARY and fold1 and use_regions)
+    norm_in = (NORM_IN_LINEAR and not fold1 and x_ln is None and not FUSE_ROUTER_NORM and getattr(attn, "sr_ratio", 1) <= 1
+               and ops.fits_layernorm_linear(x, attn.kv.weight, x, attn.q.weight))
+    overlap = overlap and OVERLAP and not norm_in and not (SERIAL_BESIDE_WEIGHT_STATIONARY and fold1 and use_regions)
     main = torch.cuda.current_stream(x.device)
     side = _side_stream(x.device, main.cuda_stream) if overlap else main
     swap = overlap and ROUTING_ON_SIDE
@@ -282,9 +287,11 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
                 want_region_rows=True)
             if cnt is not None and REGION_ROWS:
                 placed["region_rows"], placed["cur_counts"] = rrows, cnt
-            ln = None if foldq else ops.layernorm(cmp_, n1.weight, n1.bias, n1.eps, rows_dev=off[B:])
+            ln = None if foldq or norm_in else ops.layernorm(cmp_, n1.weight, n1.bias, n1.eps, rows_dev=off[B:])
             return g, idx, pat, off, lens, cmp_, ln, rec
         pat, off, lens = ops.index_to_patch(idx, dge.splits, R, extra, capacity=cap)
+        if norm_in:
+            return g, idx, pat, off, lens, ops.compress(x, pat, W, extra, rows_dev=off[B:], rows=cap), None, None
         cmp_, ln = ops.compress(x, pat, W, extra, rows_dev=off[B:], rows=cap, ln_weight=n1.weight, ln_bias=n1.bias,
                                 ln_eps=n1.eps)
         return g, idx, pat, off, lens, cmp_, ln, None
@@ -316,11 +323,15 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
             q = q_linear()
     else:
         # one stream: the routing chain, then the two Linears
-        if not ROUTING_FIRST:
+        if not ROUTING_FIRST and not norm_in:
             kv_src, kv = kv_chain()
         gate, indices, patches, offsets, lengths, comp, comp_ln, comp_rec = routing_chain()
         rows_dev = offsets[B:]
-        if PAIR_KV_Q and ROUTING_FIRST and fold1 and comp_rec is not None:
+        if norm_in:
+            kv_src = x
+            kv, q = ops.layernorm_linear(x, attn.kv.weight, attn.kv.bias, n1.weight, n1.bias, n1.eps,
+                                         second=(comp, attn.q.weight, attn.q.bias, rows_dev))
+        elif PAIR_KV_Q and ROUTING_FIRST and fold1 and comp_rec is not None:
             # the key/value and the query projection as one launch, the grid shared out by their live rows
             rec1 = carry.get("x_stats")
             if rec1 is None:
@@ -345,6 +356,9 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
 
     if fold2:
         hid = ops.linear_layernorm(q1, rec2, mlp.fc1.weight, mlp.fc1.bias, n2.weight, n2.bias, act="gelu",
+                                   rows_dev=rows_dev)
+    elif NORM_IN_LINEAR and ops.fits_layernorm_linear(q1, mlp.fc1.weight):
+        hid = ops.layernorm_linear(q1, mlp.fc1.weight, mlp.fc1.bias, n2.weight, n2.bias, n2.eps, act="gelu",
                                    rows_dev=rows_dev)
     else:
         q1_ln = ops.layernorm(q1, n2.weight, n2.bias, n2.eps, rows_dev=rows_dev)

@@ -772,6 +772,45 @@ def linear_layernorm_pair(a0, records0, weight0, bias0, a1, records1, weight1, b
     return outs[0], outs[1]
 
 
+def fits_layernorm_linear(a, weight, a1=None, weight1=None):
+    """Whether `layernorm_linear` has a kernel for these operands (few rows of whole 128-byte pieces)."""
+    for t, w in ((a, weight), (a1, weight1)):
+        if t is not None and (not t.is_cuda or not t.is_contiguous() or w.dtype != t.dtype or w.dim() != 2
+                              or w.shape[1] != t.shape[-1]):
+            return False
+    if a.dtype not in (torch.float32, torch.bfloat16):
+        return False
+    K = a.shape[-1]
+    rows1, N1 = (a1.numel() // K, weight1.shape[0]) if a1 is not None else (0, 0)
+    return bool(_lib.load().vtdge_layernorm_linear_fits(a.numel() // K, weight.shape[0], rows1, N1, K, dtype_code(a)))
+
+
+def layernorm_linear(a, weight, bias, ln_weight, ln_bias, ln_eps, act="none", rows_dev=None, second=None):
+    """act(LayerNorm(a) @ weight.T + bias) for few rows, as one launch; `second` = (a1, weight1, bias1, rows_dev1) adds a
+    product with the same LayerNorm: -> (out, out1) then.  See `fits_layernorm_linear`."""
+    K = a.shape[-1]
+    _check_vector("ln_weight", ln_weight, K)
+    _check_vector("ln_bias", ln_bias, K)
+    args, outs, shapes = [], [], ()
+    for a_, w, b, rd in ((a, weight, bias, rows_dev),) + ((second,) if second is not None else ()):
+        _need_gpu(a_, w, b, ln_weight, ln_bias)
+        _check_like(a_, weight=w, bias=b, ln_weight=ln_weight, ln_bias=ln_bias)
+        if not a_.is_contiguous() or w.dim() != 2 or w.shape[1] != K or a_.shape[-1] != K:
+            raise ValueError(f"weight {tuple(w.shape)} does not take contiguous inputs {tuple(a_.shape)} of width {K}")
+        N = w.shape[0]
+        _check_vector("bias", b, N)
+        rows = a_.numel() // K
+        outs.append(torch.empty(a_.shape[:-1] + (N,), dtype=a_.dtype, device=a_.device))
+        args += [ptr(a_), K, ptr(_contig(w)), ptr(None if b is None else _contig(b)), ptr(outs[-1]), ptr(rd), rows, N]
+        shapes += (rows, N, rd is not None)
+    if second is None:
+        args += [0, 0, 0, 0, 0, 0, 0, 0]
+    call("vtdge_layernorm_linear", *args, ptr(_contig(ln_weight)), ptr(_contig(ln_bias)), float(ln_eps), K,
+         _lib.ACT_GELU if act == "gelu" else _lib.ACT_NONE, dtype_code(a), stream_ptr(),
+         tag=("layernorm_linear", act, K) + shapes)
+    return outs[0] if second is None else tuple(outs)
+
+
 def sparse_attention(q, k, v, offsets, scale, num_heads, max_rows_per_sample, out=None):
     """Strided form.  q [L, h*d]; k, v [B, n, h*d]-like views (last dim contiguous, any batch/token strides);
     offsets int64 [B+1] on the device.  Returns [L, h*d] with channel = head*d + j."""
