@@ -128,6 +128,15 @@ int vtdge_decompress_layernorm(const void *in, const void *sub, const int64_t *p
                                const void *ln_bias, float ln_eps, int B, int N, int C, int W, int extra, int dtype,
                                void *stream);
 
+/* The adjoints of the two, for their gradients (vtpack/layers/grained_sample.py:26-38, :61-78):
+ *   vtdge_compress_sum     out[row] = the SUM of the tokens its patch covers (the gradient of vtdge_decompress's `in`)
+ *   vtdge_decompress_mean  out[token] = in[row] / area of the patch that covers it (+ add[token], nullable): the gradient of
+ *                          vtdge_compress's `x` */
+int vtdge_compress_sum(const void *x, const int64_t *patches, int64_t rows, void *out, int B, int N, int C, int W, int extra,
+                       int dtype, void *stream);
+int vtdge_decompress_mean(const void *in, const int64_t *patches, int64_t rows, const void *add, void *out, int B, int N,
+                          int C, int W, int extra, int dtype, void *stream);
+
 /* Scatter back by region, and the NEXT block's router on the tokens just written:
  *   out[b,t,:] = (in[row,:] - sub[row,:]) + ref[b,t,:]        (as vtdge_decompress with `sub` and `ref`; sub nullable)
  *   next_gate [B, H/R, W/R, S2], next_indices int64 [B, H/R, W/R] = vtdge_router(out, next_weight, next_bias)
@@ -399,6 +408,23 @@ int vtdge_batched_sparse_gemm(const void *a, const void *b, const int64_t *a_off
                               void *out, int B, int h, int64_t La, int ka, int64_t Lb, int kb, int trans_a,
                               int trans_b, int64_t out_rows, int64_t out_cols, int64_t max_m, int dtype,
                               void *stream);
+
+/* Gradients of vtdge_sparse_attention: dq, dk, dv from its operands, its output and the output's gradient, as autograd
+ * through the reference's training composition would give them (two batched products around a softmax,
+ * vtpack/models/dge/deit_dge.py:86-95), without score-sized tensors.  Strides as in vtdge_sparse_attention; `out` and
+ * `dout` share theirs.  workspace: 2 * h * L floats, L = offsets[B] = rows of q.  Gradients of keys and values of a sample
+ * without queries are zero.  Head dim 64. */
+int vtdge_sparse_attention_backward(const void *q, int64_t q_row_stride, int64_t q_head_stride, const void *k, const void *v,
+                                    int64_t kv_batch_stride, int64_t kv_tok_stride, int64_t kv_head_stride, const void *out,
+                                    const void *dout, int64_t o_row_stride, int64_t o_head_stride, const int64_t *offsets,
+                                    void *dq, int64_t dq_row_stride, int64_t dq_head_stride, void *dk, void *dv,
+                                    int64_t dkv_batch_stride, int64_t dkv_tok_stride, int64_t dkv_head_stride,
+                                    float *workspace, int64_t L, int B, int h, int d, int n, int max_rows_per_sample,
+                                    float scale, int dtype, void *stream);
+
+/* offsets int64 [B+1] (device) = 0 and the running sums of the B lengths at lengths_host (HOST memory, read before the call
+ * returns): the query counts of a batch as the reference's callers hold them, without a copy of host memory. */
+int vtdge_lengths_to_offsets(const int64_t *lengths_host, int B, int64_t *offsets, void *stream);
 
 /* out = act(LayerNorm(A) W^T + bias) for few rows, the LayerNorm done inside the Linear: norm1 -> kv and norm1 -> q
  * (vtpack/models/dge/deit_dge.py:127 with :72-73; the two products share the launch) or norm2 -> fc1 -> GELU (:128 with

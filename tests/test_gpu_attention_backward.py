@@ -1,0 +1,59 @@
+"""Gradients of the packed-query attention against float64 autograd through the same composition: query counts around a
+tile of 16, a stage of 32 and a workgroup of 64, samples without queries, key counts with a partial last tile and stage."""
+import numpy as np
+import pytest
+import torch
+
+from util import randn
+
+pytestmark = pytest.mark.gpu
+# fp32: sums of a few hundred products, 4e-6 of the largest gradient seen; bf16: P and dS are rounded to bf16 (2^-9 each)
+# and the operands of delta too
+TOL = {torch.float32: 1e-5, torch.bfloat16: 2e-2}
+
+
+def _reference(q, k, v, lengths, scale, g):
+    q, k, v = (t.double().requires_grad_(True) for t in (q, k, v))
+    outs, at = [], 0
+    for b, n in enumerate(lengths):
+        qb = q[:, at:at + n]
+        p = torch.softmax(qb @ k[:, b].transpose(1, 2).contiguous() * scale, dim=-1)
+        outs.append((p @ v[:, b]).permute(1, 0, 2).reshape(n, q.shape[0] * q.shape[2]))
+        at += n
+    out = torch.cat(outs)
+    return out.detach(), torch.autograd.grad(out, (q, k, v), g.double())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [1, 15, 33, 64, 65, 257])
+@pytest.mark.parametrize("lengths", [[1, 2], [16, 0, 17, 31], [64, 65, 33, 5, 130]])
+@pytest.mark.parametrize("scale,dense", [(0.125, False), (-0.3, True)])
+def test_against_float64(dev, dtype, n, lengths, scale, dense):
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    h, d, L, B = 3, 64, sum(lengths), len(lengths)
+    packed = torch.from_numpy(randn(n, L, h, d)).to(dtype)
+    q = packed.transpose(0, 1).contiguous() if dense else packed.transpose(0, 1)
+    k, v = (torch.from_numpy(randn(s + n, h, B, n, d)).to(dtype) for s in (1, 2))
+    g = torch.from_numpy(randn(3 + n, L, h * d)).to(dtype)
+    want, grads = _reference(q, k, v, lengths, scale, g)
+    args = [t.to(dev).requires_grad_(True) for t in (q, k, v)]
+    got = sparse_attention_train(*args, torch.tensor(lengths), scale)
+    again = torch.autograd.grad(got, args, g.to(dev), retain_graph=True)
+    assert float((got.detach().double().cpu() - want).abs().max()) <= TOL[dtype] * float(want.abs().max())
+    for name, a, b in zip("qkv", torch.autograd.grad(got, args, g.to(dev)), grads):
+        # dS is P (dP - delta) scale: two sums of 64 products of unit normals (3 sigma: 24) that cancel, entirely where
+        # there is one key; what their rounding leaves is relative to them, not to what remains
+        size = max(float(b.abs().max()), 24 * abs(scale) if name != "v" else 0)
+        assert float((a.double().cpu() - b).abs().max()) <= TOL[dtype] * size, name
+    assert all(torch.equal(a, b) for a, b in zip(again, torch.autograd.grad(sparse_attention_train(
+        *args, torch.tensor(lengths), scale), args, g.to(dev))))                      # the same bytes on every call
+
+
+@pytest.mark.parametrize("B", [1, 3, 447, 448, 449, 1000])
+def test_offsets_of_lengths(dev, B):
+    from vtpack_amd import ops
+    lengths = torch.from_numpy(np.random.RandomState(B).randint(0, 300, size=B))
+    if B > 448:
+        lengths[:448] = 0
+    got, _ = ops.lengths_to_offsets(lengths, dev)
+    assert torch.equal(got.cpu(), torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)]))

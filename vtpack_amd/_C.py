@@ -47,6 +47,20 @@ def grained_sample_index_to_patch_dense(indices, split_sizes, region_size, num_e
     return patches, torch.full((B,), per, dtype=torch.int64)
 
 
+def grained_sample_compress_sum(input, patches, height, width, num_extra_tokens):
+    """The gradient of grained_sample_decompress with respect to its packed rows (grained_sample.py:61-78)."""
+    input, C = _pad_channels(input)
+    out = ops.compress_sum(input, patches, int(width), int(num_extra_tokens))
+    return out if out.shape[-1] == C else out[:, :C].contiguous()
+
+
+def grained_sample_decompress_mean(input, patches, shape, height, width, num_extra_tokens):
+    """The gradient of grained_sample_compress with respect to its tokens (grained_sample.py:26-38)."""
+    input, C = _pad_channels(input)
+    out = ops.decompress_mean(input, patches, tuple(shape[:2]) + (input.shape[-1],), int(width), int(num_extra_tokens))
+    return out if out.shape[-1] == C else out[..., :C].contiguous()
+
+
 def _pad_channels(t):
     """The kernels move 16 bytes per lane; a channel count that is not a multiple of that (the [B, N, 1] gate map
     of sparse training, vtpack/layers/dge.py:96-106) is zero-padded here and sliced back by the caller."""
@@ -73,30 +87,20 @@ def grained_sample_decompress(input, patches, reference, height, width, num_extr
     return out if out.shape[-1] == C else out[..., :C].contiguous()
 
 
-def _offsets_from_lengths(lengths, device):
-    lengths = lengths.detach().to("cpu", torch.int64)
-    off = torch.zeros(lengths.numel() + 1, dtype=torch.int64)
-    torch.cumsum(lengths, 0, out=off[1:])
-    return off.to(device), lengths
-
-
 def batched_sparse_attention_forward(a, b, c, batch_lengths, scale):
     """a [h,L,d], b and c [h,B,n,d], batch_lengths int64 [B] (CPU) -> [h,L,d].
 
     vtpack/layers/csrc/batched_sparse_gemm/batched_sparse_gemm.cu:219-305."""
     ops._need_gpu(a, b, c)
     _check_same_dtype(a, b, c)
-    a, b, c = a.contiguous(), b.contiguous(), c.contiguous()
+    a = ops.vector_rows(a)
+    b, c = b.contiguous(), c.contiguous()
     h, L, d = a.shape
     _, B, n, _ = b.shape
-    offsets, lengths = _offsets_from_lengths(batch_lengths, a.device)
+    offsets, lengths = ops.lengths_to_offsets(batch_lengths, a.device)
     if lengths.numel() != B or int(lengths.sum()) != L:
         raise ValueError("batch_lengths must have one entry per sample and sum to the number of query rows")
-    out = torch.empty_like(a)
-    max_rows = int(lengths.max()) if B > 0 else 0
-    call("vtdge_sparse_attention", ptr(a), d, L * d, ptr(b), ptr(c), n * d, d, B * n * d, ptr(offsets), ptr(out), d,
-         L * d, B, h, d, n, max_rows, float(scale), dtype_code(a), stream_ptr())
-    return out
+    return ops.sparse_attention_heads(a, b, c, offsets, scale, int(lengths.max()) if B > 0 else 0)
 
 
 def batched_sparse_gemm_forward(a, b, a_lengths, b_lengths, is_a_transposed, is_b_transposed):
@@ -108,8 +112,8 @@ def batched_sparse_gemm_forward(a, b, a_lengths, b_lengths, is_a_transposed, is_
     a, b = a.contiguous(), b.contiguous()
     h, La, ka = a.shape
     _, Lb, kb = b.shape
-    a_off, al = _offsets_from_lengths(a_lengths, a.device)
-    b_off, bl = _offsets_from_lengths(b_lengths, a.device)
+    a_off, al = ops.lengths_to_offsets(a_lengths, a.device)
+    b_off, bl = ops.lengths_to_offsets(b_lengths, a.device)
     B = al.numel()
     if bl.numel() != B or int(al.sum()) != La or int(bl.sum()) != Lb:
         raise ValueError("length vectors must match each other and the packed row counts")

@@ -31,6 +31,8 @@ SIGNATURES = {
     "vtdge_index_to_patch_dense": [_p, _i, _i, _i, _i, _i, _i, _p, _p],
     "vtdge_compress": [_p, _p, _p, _l, _p, _p, _p, _p, _f, _i, _i, _i, _i, _i, _i, _p],
     "vtdge_decompress": [_p, _p, _p, _p, _l, _p, _p, _i, _i, _i, _i, _i, _i, _p],
+    "vtdge_compress_sum": [_p, _p, _l, _p, _i, _i, _i, _i, _i, _i, _p],
+    "vtdge_decompress_mean": [_p, _p, _l, _p, _p, _i, _i, _i, _i, _i, _i, _p],
     "vtdge_decompress_layernorm": [_p, _p, _p, _p, _l, _p, _p, _p, _p, _p, _f, _i, _i, _i, _i, _i, _i, _p],
     "vtdge_decompress_router": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _f, _p, _p, _p, _p, _i, _i, _i, _i,
                                 _i, _i, _i, _i, _i, _p],
@@ -60,6 +62,9 @@ SIGNATURES = {
                                     _i, _i, _i, _p],
     "vtdge_sparse_attention": [_p, _l, _l, _p, _p, _l, _l, _l, _p, _p, _l, _l, _i, _i, _i, _i, _i, _f, _i, _p],
     "vtdge_batched_sparse_gemm": [_p, _p, _p, _p, _p, _i, _i, _l, _i, _l, _i, _i, _i, _l, _l, _l, _i, _p],
+    "vtdge_sparse_attention_backward": [_p, _l, _l, _p, _p, _l, _l, _l, _p, _p, _l, _l, _p, _p, _l, _l, _p, _p, _l, _l, _l, _p,
+                                        _l, _i, _i, _i, _i, _i, _f, _i, _p],
+    "vtdge_lengths_to_offsets": [_p, _i, _p, _p],
     "vtdge_layernorm_linear_fits": [_l, _i, _l, _i, _i, _i],
     "vtdge_layernorm_linear": [_p, _l, _p, _p, _p, _p, _l, _i, _p, _l, _p, _p, _p, _p, _l, _i, _p, _p, _f, _i, _i, _i, _p],
     "vtdge_chain_layout": [_p, _p],

@@ -1,0 +1,467 @@
+// Gradients of the sparse attention of packed queries (gfx950): dQ, dK, dV from Q, K, V, the output and its gradient.
+//
+// The composition this stands in for (a product of queries and keys, a softmax, a product with the values, and their
+// five products backward: vtpack/models/dge/deit_dge.py:86-95) keeps four score-sized tensors in HBM, [heads, L, n] each:
+// 90 MB apiece at 14500 queries, 6 heads and 257 keys in bf16, against 45 MB of operands.  Here scores exist in registers
+// only: they are worked out again from Q and K where a gradient needs them,
+//   P = exp2(scale log2e q.k - lse),   dP = dO.v,   dS = P (dP - delta) scale,   delta = sum_d dO O,
+//   dQ = dS K,   dV = P^T dO,   dK = dS^T Q.
+// Two kernels, no atomics, so the result is the same bytes on every call: one over query tiles, which first finds lse (the
+// row's maximum plus the log of its sum, in log2 units) and delta and leaves both for the other, over key tiles.
+//
+// Both are one scheme.  A wave keeps 16 rows of two operands in registers (Q and dO, or K and V) and walks the rows of
+// the other two, which the workgroup's four waves share through LDS in stages of 32 by direct loads (two buffers).  With
+// the walked rows as rows of v_mfma_f32_16x16 tiles and the kept ones as columns, lane (l = lane % 16, g = lane / 16) holds
+// the score of walked rows 4 g + r (r < 4) with kept row l: the operand layout of the products over the walked rows, so
+// nothing moves between lanes.  Those products read the walked rows transposed: in fp32 a lane takes 4 consecutive channels
+// of row 4 g + r (block db of the output is then channels 4 i + db), in bf16 the LDS read itself transposes
+// (ds_read_b64_tr_b16: four rows of one channel).  Rows are stored with their 16-byte chunks XOR-ed by the row against bank
+// conflicts.  Every (sample, head) keeps to one XCD.
+#include "common.h"
+
+namespace vtdge {
+
+constexpr int AB_ROWS = 32;      // walked rows per stage
+constexpr int AB_WAVES = 4;      // kept tiles of 16 rows per workgroup
+
+template <typename T> struct BackTile {
+    static constexpr int ROWB = 64 * sizeof(T);               // bytes of a row (head dim 64)
+    static constexpr int CPR = ROWB / 16;
+    static constexpr int HALF = AB_ROWS * ROWB;               // one operand's stage
+    static constexpr int NF = sizeof(T) == 4 ? 4 : 2;         // register fragments of a kept row: 16 bytes a lane each
+    static __device__ __forceinline__ int slot(int row, int chunk)
+    {
+        return sizeof(T) == 4 ? chunk ^ (row & 15) : chunk ^ ((row >> 1) & 7);
+    }
+};
+
+// the four products of a stage, by storage type
+template <typename T> struct BackMath;
+template <> struct BackMath<float> {
+    typedef f32x4 Frag;
+    // walked rows 16 blk .. (rows) times the kept rows (columns), over the channels: d = 16 j + 4 g + e in step (j, e)
+    static __device__ __forceinline__ f32x4 scores(const unsigned char *S, int blk, const Frag (&x)[4], int l, int g)
+    {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const f32x4 a = *reinterpret_cast<const f32x4 *>(S + (16 * blk + l) * 256 + BackTile<float>::slot(l, 4 * j + g) * 16);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], x[j][e], acc, 0, 0, 0);
+        }
+        return acc;
+    }
+    // out[channel][kept row] += walked rows^T p, p[blk][r] = lane's value of walked row 16 blk + 4 g + r
+    static __device__ __forceinline__ void accumulate(const unsigned char *S, const f32x4 (&p)[2], f32x4 (&out)[4], int l, int g)
+    {
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const f32x4 a = *reinterpret_cast<const f32x4 *>(S + (16 * blk + 4 * g + r) * 256 +
+                                                                 BackTile<float>::slot(4 * g + r, l) * 16);
+#pragma unroll
+                for (int db = 0; db < 4; db++)
+                    out[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[db], p[blk][r], out[db], 0, 0, 0);
+            }
+    }
+    static __device__ __forceinline__ float dot(const Frag (&a)[4], const Frag (&b)[4])
+    {
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s += a[j][e] * b[j][e];
+        return s;
+    }
+    // out[db][r] is channel 16 g + 4 r + db of kept row l
+    static __device__ __forceinline__ void store(float *row, const f32x4 (&o)[4], int g)
+    {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            *reinterpret_cast<f32x4 *>(row + 16 * g + 4 * r) = f32x4{o[0][r], o[1][r], o[2][r], o[3][r]};
+    }
+};
+template <> struct BackMath<bf16_t> {
+    typedef u32x4 Frag;
+    static __device__ __forceinline__ f32x4 mma(const u32x4 &a, const u32x4 &b, const f32x4 &c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+                                                       0);
+    }
+    static __device__ __forceinline__ f32x4 scores(const unsigned char *S, int blk, const Frag (&x)[2], int l, int g)
+    {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            acc = mma(*reinterpret_cast<const u32x4 *>(S + (16 * blk + l) * 128 + BackTile<bf16_t>::slot(l, 4 * j + g) * 16),
+                      x[j], acc);
+        return acc;
+    }
+    // contraction over the stage's 32 rows in the order (4 g .. 4 g + 3, 16 + 4 g .. 16 + 4 g + 3) of lane group g
+    static __device__ __forceinline__ void accumulate(const unsigned char *S, const f32x4 (&p)[2], f32x4 (&out)[4], int l, int g)
+    {
+        u32x4 b;
+        b.x = pack_bf16x2(p[0][0], p[0][1]);
+        b.y = pack_bf16x2(p[0][2], p[0][3]);
+        b.z = pack_bf16x2(p[1][0], p[1][1]);
+        b.w = pack_bf16x2(p[1][2], p[1][3]);
+        // this lane as a source of the transposing reads: row 4 g + l / 4, channels 16 db + 4 (l % 4) .. + 3
+        const int row = 4 * g + (l >> 2);
+        const unsigned char *src = S + row * 128 + 8 * (l & 1);
+#pragma unroll
+        for (int db = 0; db < 4; db++) {
+            const unsigned char *at = src + BackTile<bf16_t>::slot(row, 2 * db + ((l & 3) >> 1)) * 16;
+            const u32x2 lo = lds_read_tr16(at), hi = lds_read_tr16(at + 16 * 128);
+            out[db] = mma(u32x4{lo.x, lo.y, hi.x, hi.y}, b, out[db]);
+        }
+    }
+    static __device__ __forceinline__ float dot(const Frag (&a)[2], const Frag (&b)[2])
+    {
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            float x[8], y[8];
+            Elem<bf16_t>::unpack(a[j], x);
+            Elem<bf16_t>::unpack(b[j], y);
+#pragma unroll
+            for (int e = 0; e < 8; e++) s += x[e] * y[e];
+        }
+        return s;
+    }
+    // out[db][r] is channel 16 db + 4 g + r of kept row l
+    static __device__ __forceinline__ void store(bf16_t *row, const f32x4 (&o)[4], int g)
+    {
+#pragma unroll
+        for (int db = 0; db < 4; db++) {
+            u32x2 w;
+            w.x = pack_bf16x2(o[db][0], o[db][1]);
+            w.y = pack_bf16x2(o[db][2], o[db][3]);
+            *reinterpret_cast<u32x2 *>(row + 16 * db + 4 * g) = w;
+        }
+    }
+};
+
+struct AttnBack {
+    const void *q, *k, *v, *out, *dout;
+    void *dq, *dk, *dv;
+    float *lse, *delta;                                   // [h, L] each
+    const int64_t *offsets;
+    int64_t q_rs, q_hs, kv_bs, kv_ts, kv_hs, o_rs, o_hs, dq_rs, dq_hs, dkv_bs, dkv_ts, dkv_hs, L;
+    int pairs, h, n, chunks;
+    float scale, scale_log2;
+};
+
+// the stages of two operands' rows in LDS: `rows` of them from base0 / base1 with the given row pitches in bytes
+template <typename T> struct Stager {
+    using B = BackTile<T>;
+    static constexpr int NL = 2 * B::HALF / 1024 / AB_WAVES;  // direct loads a wave and stage
+    const unsigned char *base;
+    uint32_t pitch, lds0;
+    int rows, wid, lane;
+    __device__ __forceinline__ void load(int st) const
+    {
+        const int r0 = st * AB_ROWS, last = rows - 1 - r0;
+        const uint32_t dst = lds0 + (uint32_t)((st & 1) * 2 * B::HALF + wid * NL * 1024);
+        const void *src = uniform_ptr(base + (int64_t)r0 * pitch);
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const int row = ((wid & 1) * NL + i) * (64 / B::CPR) + lane / B::CPR;
+            dma16(src, (uint32_t)min(row, last) * pitch + (uint32_t)B::slot(row, lane % B::CPR) * 16u, dst + i * 1024);
+        }
+    }
+};
+
+template <typename T>
+__device__ __forceinline__ void load_kept(typename BackMath<T>::Frag (&f)[BackTile<T>::NF], const T *row, bool live, int g)
+{
+    using Frag = typename BackMath<T>::Frag;
+    const unsigned char *p = reinterpret_cast<const unsigned char *>(row) + 16 * g;
+#pragma unroll
+    for (int j = 0; j < BackTile<T>::NF; j++) {
+        u32x4 z = {0u, 0u, 0u, 0u};
+        if (live) z = *reinterpret_cast<const u32x4 *>(p + 64 * j);
+        f[j] = __builtin_bit_cast(Frag, z);
+    }
+}
+
+// dQ of 64 query rows of one (sample, head), with their lse and delta
+template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_kernel(AttnBack a)
+{
+    using B = BackTile<T>;
+    using M = BackMath<T>;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * B::HALF];
+    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8;
+    const int pair = (rest % pairs_x) * 8 + (blockIdx.x & 7), chunk = rest / pairs_x;
+    if (pair >= a.pairs) return;
+    const int b = pair / a.h, head = pair - b * a.h;
+    const int64_t row0 = a.offsets[b];
+    const int Lb = (int)(a.offsets[b + 1] - row0);
+    if (chunk * 16 * AB_WAVES >= Lb) return;
+    const int lane = threadIdx.x & 63, l = lane & 15, g = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int row = (chunk * AB_WAVES + wid) * 16 + l;
+    const bool live = row < Lb, wave_live = (chunk * AB_WAVES + wid) * 16 < Lb;
+
+    const int64_t kv_at = (int64_t)b * a.kv_bs + (int64_t)head * a.kv_hs;
+    const Stager<T> kv{reinterpret_cast<const unsigned char *>((const T *)(wid < 2 ? a.k : a.v) + kv_at),
+                       (uint32_t)(a.kv_ts * sizeof(T)), (uint32_t)(uintptr_t)smem, a.n, wid, lane};
+    const int stages = (a.n + AB_ROWS - 1) / AB_ROWS;
+    if (wid < 2) kv.load(0);
+
+    typename M::Frag qf[B::NF], df[B::NF];
+    float delta;
+    {
+        typename M::Frag of[B::NF];
+        const int64_t o_at = (row0 + row) * a.o_rs + (int64_t)head * a.o_hs;
+        load_kept<T>(qf, (const T *)a.q + (row0 + row) * a.q_rs + (int64_t)head * a.q_hs, live, g);
+        load_kept<T>(df, (const T *)a.dout + o_at, live, g);
+        load_kept<T>(of, (const T *)a.out + o_at, live, g);
+        delta = M::dot(df, of);
+        delta += __shfl_xor(delta, 16, WAVE);
+        delta += __shfl_xor(delta, 32, WAVE);
+    }
+    // ---- lse of this lane's query: maximum and sum over the lane's keys, then over the four lanes that share the query
+    float m = -INFINITY, s = 0.f;
+    for (int st = 0; st < stages; st++) {
+        wait_vmcnt<0>();
+        block_barrier();
+        if (wid < 2 && st + 1 < stages) kv.load(st + 1);
+        if (!wave_live) continue;
+        const unsigned char *S = smem + (st & 1) * 2 * B::HALF;
+        f32x4 t[2];
+        float mx = m;
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            t[blk] = M::scores(S, blk, qf, l, g);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const bool in = st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
+                t[blk][r] = in ? t[blk][r] * a.scale_log2 : -INFINITY;
+                mx = fmaxf(mx, t[blk][r]);
+            }
+        }
+        if (mx > -INFINITY) {
+            s *= __builtin_amdgcn_exp2f(m - mx);
+#pragma unroll
+            for (int blk = 0; blk < 2; blk++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) s += __builtin_amdgcn_exp2f(t[blk][r] - mx);
+            m = mx;
+        }
+    }
+    float all = fmaxf(m, __shfl_xor(m, 16, WAVE));
+    all = fmaxf(all, __shfl_xor(all, 32, WAVE));
+    s *= __builtin_amdgcn_exp2f(m - all);                 // a lane without keys: exp2(-inf) = 0 times 0
+    s += __shfl_xor(s, 16, WAVE);
+    s += __shfl_xor(s, 32, WAVE);
+    const float lse = all + __builtin_amdgcn_logf(s);     // v_log_f32: base 2
+    if (live && g == 0) {
+        a.lse[(int64_t)head * a.L + row0 + row] = lse;
+        a.delta[(int64_t)head * a.L + row0 + row] = delta;
+    }
+
+    // ---- dQ^T += K^T dS^T
+    f32x4 dq[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) dq[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    block_barrier();                                      // the last stage has been read
+    kv.load(0);
+    for (int st = 0; st < stages; st++) {
+        wait_vmcnt<0>();
+        block_barrier();
+        if (st + 1 < stages) kv.load(st + 1);
+        if (!wave_live) continue;
+        const unsigned char *Ks = smem + (st & 1) * 2 * B::HALF, *Vs = Ks + B::HALF;
+        f32x4 ds[2];
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            const f32x4 t = M::scores(Ks, blk, qf, l, g), dp = M::scores(Vs, blk, df, l, g);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const bool in = st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
+                const float p = __builtin_amdgcn_exp2f(t[r] * a.scale_log2 - lse);
+                ds[blk][r] = in ? p * (dp[r] - delta) * a.scale : 0.f;
+            }
+        }
+        M::accumulate(Ks, ds, dq, l, g);
+    }
+    if (live) M::store((T *)a.dq + (row0 + row) * a.dq_rs + (int64_t)head * a.dq_hs, dq, g);
+}
+
+// dK and dV of 64 keys of one (sample, head)
+template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void attention_dkv_kernel(AttnBack a)
+{
+    using B = BackTile<T>;
+    using M = BackMath<T>;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * B::HALF];
+    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8;
+    const int pair = (rest % pairs_x) * 8 + (blockIdx.x & 7), chunk = rest / pairs_x;
+    if (pair >= a.pairs) return;
+    const int b = pair / a.h, head = pair - b * a.h;
+    const int64_t row0 = a.offsets[b];
+    const int Lb = (int)(a.offsets[b + 1] - row0);
+    const int lane = threadIdx.x & 63, l = lane & 15, g = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int key = (chunk * AB_WAVES + wid) * 16 + l;
+    const bool live = key < a.n, wave_live = (chunk * AB_WAVES + wid) * 16 < a.n;
+
+    const int stages = (Lb + AB_ROWS - 1) / AB_ROWS;      // none for a sample without queries: its gradients are zero
+    const Stager<T> qd{wid < 2 ? reinterpret_cast<const unsigned char *>((const T *)a.q + row0 * a.q_rs + (int64_t)head * a.q_hs)
+                               : reinterpret_cast<const unsigned char *>((const T *)a.dout + row0 * a.o_rs + (int64_t)head * a.o_hs),
+                       (uint32_t)((wid < 2 ? a.q_rs : a.o_rs) * sizeof(T)), (uint32_t)(uintptr_t)smem, Lb, wid, lane};
+    const float *lse = a.lse + (int64_t)head * a.L + row0, *delta = a.delta + (int64_t)head * a.L + row0;
+    // lse and delta of the lane's walked rows, one stage ahead; rows past the sample's last query: probability zero
+    f32x4 nls[2], ndl[2];
+    auto fetch = [&](int st) {
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int i = st * AB_ROWS + 16 * blk + 4 * g + r;
+                nls[blk][r] = i < Lb ? lse[i] : INFINITY;
+                ndl[blk][r] = i < Lb ? delta[i] : 0.f;
+            }
+    };
+    if (stages > 0) {
+        qd.load(0);
+        fetch(0);
+    }
+    typename M::Frag kf[B::NF], vf[B::NF];
+    const int64_t kv_at = (int64_t)b * a.kv_bs + (int64_t)key * a.kv_ts + (int64_t)head * a.kv_hs;
+    load_kept<T>(kf, (const T *)a.k + kv_at, live, g);
+    load_kept<T>(vf, (const T *)a.v + kv_at, live, g);
+    f32x4 dk[4], dv[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) dk[i] = dv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    for (int st = 0; st < stages; st++) {
+        wait_vmcnt<0>();
+        block_barrier();
+        const f32x4 ls[2] = {nls[0], nls[1]}, dl[2] = {ndl[0], ndl[1]};
+        if (st + 1 < stages) {
+            qd.load(st + 1);
+            if (wave_live) fetch(st + 1);
+        }
+        if (!wave_live) continue;
+        const unsigned char *Qs = smem + (st & 1) * 2 * B::HALF, *Ds = Qs + B::HALF;
+        f32x4 p[2], ds[2];
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            const f32x4 t = M::scores(Qs, blk, kf, l, g), dp = M::scores(Ds, blk, vf, l, g);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                p[blk][r] = __builtin_amdgcn_exp2f(t[r] * a.scale_log2 - ls[blk][r]);
+                ds[blk][r] = p[blk][r] * (dp[r] - dl[blk][r]) * a.scale;
+            }
+        }
+        M::accumulate(Ds, p, dv, l, g);
+        M::accumulate(Qs, ds, dk, l, g);
+    }
+    if (!live) return;
+    const int64_t at = (int64_t)b * a.dkv_bs + (int64_t)key * a.dkv_ts + (int64_t)head * a.dkv_hs;
+    M::store((T *)a.dk + at, dk, g);
+    M::store((T *)a.dv + at, dv, g);
+}
+
+template <typename T> static int launch_backward(AttnBack a, int max_rows, hipStream_t st)
+{
+    const int64_t pairs_x = ceil_div(a.pairs, 8);
+    const int64_t qc = ceil_div(max_rows, 16 * AB_WAVES), kc = ceil_div(a.n, 16 * AB_WAVES);
+    VT_REQUIRE(pairs_x * 8 * (qc > kc ? qc : kc) < (1ll << 31), VTDGE_ERR_UNSUPPORTED,
+               "sparse_attention_backward: too many workgroups for one launch");
+    if (qc > 0) {
+        note_kernel(reinterpret_cast<const void *>(attention_dq_kernel<T>));
+        attention_dq_kernel<T><<<dim3((unsigned)(pairs_x * 8 * qc)), dim3(64 * AB_WAVES), 0, st>>>(a);
+        const int rc = check_launch("sparse_attention_backward");
+        if (rc != VTDGE_OK) return rc;
+    }
+    note_kernel(reinterpret_cast<const void *>(attention_dkv_kernel<T>));
+    attention_dkv_kernel<T><<<dim3((unsigned)(pairs_x * 8 * kc)), dim3(64 * AB_WAVES), 0, st>>>(a);
+    return check_launch("sparse_attention_backward");
+}
+
+// offsets[base + 1 ..] of `count` lengths that travel in the kernel's arguments: no copy of host memory
+constexpr int OFF_MAX = 448;
+struct Lengths {
+    int32_t v[OFF_MAX];
+};
+__global__ __launch_bounds__(512) void lengths_offsets_kernel(Lengths len, int count, int64_t start, int64_t *__restrict__ out)
+{
+    __shared__ int64_t wave_total[8];
+    const int i = threadIdx.x, lane = i & 63;
+    int64_t v = i < count ? len.v[i] : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int64_t up = __shfl_up(v, o, WAVE);
+        if (lane >= o) v += up;
+    }
+    if (lane == 63) wave_total[i >> 6] = v;
+    __syncthreads();
+    int64_t before = start;
+    for (int w = 0; w < (i >> 6); w++) before += wave_total[w];
+    if (i < count) out[i + 1] = before + v;
+    if (i == 0 && start == 0) out[0] = 0;
+}
+
+}  // namespace vtdge
+
+using namespace vtdge;
+
+extern "C" int vtdge_lengths_to_offsets(const int64_t *lengths_host, int B, int64_t *offsets, void *stream)
+{
+    VT_REQUIRE(offsets && (lengths_host || B == 0) && B >= 0, VTDGE_ERR_ARG, "lengths_to_offsets: NULL operand");
+    int64_t start = 0;
+    for (int at = 0; at == 0 || at < B; at += OFF_MAX) {
+        Lengths len;
+        const int count = B - at < OFF_MAX ? B - at : OFF_MAX;
+        int64_t sum = 0;
+        for (int i = 0; i < count; i++) {
+            const int64_t v = lengths_host[at + i];
+            VT_REQUIRE(v >= 0 && v < (1ll << 31), VTDGE_ERR_ARG, "lengths_to_offsets: length %lld of sample %d", (long long)v,
+                       at + i);
+            len.v[i] = (int32_t)v;
+            sum += v;
+        }
+        // (`start` is zero for the first launch only, or where everything before it was empty: out[0] of a later slice
+        // is then the zero that is there already)
+        note_kernel(reinterpret_cast<const void *>(lengths_offsets_kernel));
+        lengths_offsets_kernel<<<1, 512, 0, (hipStream_t)stream>>>(len, count, start, offsets + at);
+        const int rc = check_launch("lengths_to_offsets");
+        if (rc != VTDGE_OK) return rc;
+        start += sum;
+    }
+    return VTDGE_OK;
+}
+
+extern "C" int vtdge_sparse_attention_backward(
+    const void *q, int64_t q_row_stride, int64_t q_head_stride, const void *k, const void *v, int64_t kv_batch_stride,
+    int64_t kv_tok_stride, int64_t kv_head_stride, const void *out, const void *dout, int64_t o_row_stride,
+    int64_t o_head_stride, const int64_t *offsets, void *dq, int64_t dq_row_stride, int64_t dq_head_stride, void *dk,
+    void *dv, int64_t dkv_batch_stride, int64_t dkv_tok_stride, int64_t dkv_head_stride, float *workspace, int64_t L, int B,
+    int h, int d, int n, int max_rows_per_sample, float scale, int dtype, void *stream)
+{
+    VT_REQUIRE(k && v && offsets && dk && dv && (L == 0 || (q && out && dout && dq && workspace)), VTDGE_ERR_ARG,
+               "sparse_attention_backward: NULL operand");
+    VT_REQUIRE(dtype == VTDGE_F32 || dtype == VTDGE_BF16, VTDGE_ERR_ARG, "sparse_attention_backward: unknown dtype %d", dtype);
+    VT_REQUIRE(B > 0 && h > 0 && n > 0 && L >= 0 && max_rows_per_sample >= 0 && (int64_t)B * h < (1ll << 28), VTDGE_ERR_ARG,
+               "sparse_attention_backward: bad sizes");
+    VT_REQUIRE(d == 64, VTDGE_ERR_UNSUPPORTED, "sparse_attention_backward: head_dim %d (only 64 is built)", d);
+    const int esz = dtype == VTDGE_F32 ? 4 : 2, vec = 16 / esz;
+    const int64_t strides[] = {q_row_stride,  q_head_stride, kv_batch_stride, kv_tok_stride,    kv_head_stride, o_row_stride,
+                               o_head_stride, dq_row_stride, dq_head_stride,  dkv_batch_stride, dkv_tok_stride, dkv_head_stride};
+    for (int64_t s : strides)
+        VT_REQUIRE(s >= 0 && s % vec == 0, VTDGE_ERR_UNSUPPORTED,
+                   "sparse_attention_backward: strides must keep 16-byte alignment");
+    VT_REQUIRE(q_row_stride < (1 << 23) && kv_tok_stride < (1 << 23) && o_row_stride < (1 << 23), VTDGE_ERR_UNSUPPORTED,
+               "sparse_attention_backward: row stride too large");
+    VT_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out | (uintptr_t)dout | (uintptr_t)dq | (uintptr_t)dk |
+                 (uintptr_t)dv) & 15) == 0,
+               VTDGE_ERR_ARG, "sparse_attention_backward: operands must be 16-byte aligned");
+    AttnBack a{q, k, v, out, dout, dq, dk, dv, workspace, workspace + (int64_t)h * L, offsets, q_row_stride, q_head_stride,
+               kv_batch_stride, kv_tok_stride, kv_head_stride, o_row_stride, o_head_stride, dq_row_stride, dq_head_stride,
+               dkv_batch_stride, dkv_tok_stride, dkv_head_stride, L, B * h, h, n, 0, scale,
+               scale * 1.44269504088896340736f};
+    if (dtype == VTDGE_F32) return launch_backward<float>(a, max_rows_per_sample, (hipStream_t)stream);
+    return launch_backward<bf16_t>(a, max_rows_per_sample, (hipStream_t)stream);
+}

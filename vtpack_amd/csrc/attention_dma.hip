@@ -79,13 +79,6 @@ __device__ __forceinline__ u32x4 att_read_k(const AttnTile &t, const int (&cs)[4
 // j < 4): two such reads, with k0 = 16 h + 4 lg (+ 8) and d0 = 32 db + 16 (block & 1).  Rows are stored with their
 // 16-byte chunks XOR-ed by 2 (key & 3), so the sixteen 8-byte pieces of a block come from sixteen different bank
 // groups; the XOR constant of a lane does not depend on kb, h or the +8, and db = 1 is the address XOR 64.
-typedef short att_v4s __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ u32x2 att_tr_read(const unsigned char *p)
-{
-    const att_v4s r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) att_v4s *)(uint32_t)(uintptr_t)p);
-    return __builtin_bit_cast(u32x2, r);
-}
 __device__ __forceinline__ const unsigned char *att_v_lane(const unsigned char *vbase, int lane)
 {
     const int blk = lane >> 4, i = lane & 15;
@@ -106,7 +99,7 @@ __device__ __forceinline__ void att_read_v(const AttnTile &t, int kb, u32x4 (&vf
             const unsigned char *p =
                 HI ? (db ? t.vlane_hi : t.vlane) + (kb * 32 + 16 * h) * 128
                    : reinterpret_cast<const unsigned char *>((uintptr_t)(t.vlane + (kb * 32 + 16 * h) * 128) ^ (64u * db));
-            const u32x2 lo = att_tr_read(p), hi = att_tr_read(p + 8 * 128);
+            const u32x2 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 8 * 128);
             vf[2 * h + db].x = lo.x;
             vf[2 * h + db].y = lo.y;
             vf[2 * h + db].z = hi.x;

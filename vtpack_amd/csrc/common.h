@@ -206,6 +206,16 @@ template <> struct Slab<float> {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(gptr),             \
                                      (__attribute__((address_space(3))) void *)(lptr), 16, 0, 0)
 
+// ds_read_b64_tr_b16: lane i of a block of 16 receives, as 16-bit element e, column (i & 3) of the four consecutive
+// elements that source lane 4 e + (i >> 2) of the block names - a 4 x 16 tile transposed on its way out of LDS
+typedef short lds_v4s __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x2 lds_read_tr16(const unsigned char *p)
+{
+    const lds_v4s r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) lds_v4s *)(uint32_t)(uintptr_t)p);
+    return __builtin_bit_cast(u32x2, r);
+}
+
 // s_waitcnt with only the vector-memory counter constrained (gfx9 encoding)
 template <int N> __device__ __forceinline__ void wait_vmcnt()
 {

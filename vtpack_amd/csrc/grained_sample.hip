@@ -540,7 +540,7 @@ __global__ __launch_bounds__(256, NIT == 1 ? 8 : 2) void compress_kernel(const T
                                                         const int64_t *__restrict__ rows_dev, int64_t rows,
                                                         T *__restrict__ out, T *__restrict__ ln_out,
                                                         const T *__restrict__ ln_w, const T *__restrict__ ln_b,
-                                                        float eps, int N, int C, int W, int extra)
+                                                        float eps, int N, int C, int W, int extra, bool sum)
 {
     constexpr int VEC = Elem<T>::VEC;
     static_assert(NIT == 1 || GS == 64, "several vectors per lane only with whole-wave groups");
@@ -567,20 +567,21 @@ __global__ __launch_bounds__(256, NIT == 1 ? 8 : 2) void compress_kernel(const T
                 for (int c = 0; c < VEC; c++) acc[c] = 0.f;
                 const T *base = xb + ((y0 * W + x0 + extra) * (int64_t)C + v * VEC);
                 // mean = sum / area.  The areas of the usual windows are powers of two, whose reciprocals are exact:
-                // the product is then the quotient, bit for bit, at a tenth of the instructions
+                // the product is then the quotient, bit for bit, at a tenth of the instructions.  `sum`: no division,
+                // the adjoint of the scatter back
                 if (sz == 1) {
                     window_sum<T, 1>(base, W, C, sz, acc);
                 } else if (sz == 2) {
                     window_sum<T, 2>(base, W, C, sz, acc);
 #pragma unroll
-                    for (int c = 0; c < VEC; c++) acc[c] *= 0.25f;
+                    for (int c = 0; c < VEC; c++) acc[c] *= sum ? 1.f : 0.25f;
                 } else if (sz == 4) {
                     window_sum<T, 4>(base, W, C, sz, acc);
 #pragma unroll
-                    for (int c = 0; c < VEC; c++) acc[c] *= 0.0625f;
+                    for (int c = 0; c < VEC; c++) acc[c] *= sum ? 1.f : 0.0625f;
                 } else {
                     window_sum<T, 0>(base, W, C, sz, acc);
-                    const float area = (float)(sz * sz);
+                    const float area = sum ? 1.f : (float)(sz * sz);
 #pragma unroll
                     for (int c = 0; c < VEC; c++) acc[c] = acc[c] / area;
                 }
@@ -681,8 +682,9 @@ __global__ __launch_bounds__(256) void decompress_kernel(const T *__restrict__ i
                                                           const int64_t *__restrict__ patches,
                                                           const int64_t *__restrict__ rows_dev, int64_t rows,
                                                           const T *__restrict__ ref, T *__restrict__ out, int N,
-                                                          int C, int W, int extra)
+                                                          int C, int W, int extra, bool mean)
 {
+    // mean: every token gets the row divided by its patch's area, the adjoint of compress
     constexpr int VEC = Elem<T>::VEC;
     const int lane = threadIdx.x & (GS - 1);
     const int64_t row = ((int64_t)blockIdx.x * ROWS_PER_BLOCK + (threadIdx.x >> 6)) * (WAVE / GS) + (threadIdx.x & 63) / GS;
@@ -699,6 +701,11 @@ __global__ __launch_bounds__(256) void decompress_kernel(const T *__restrict__ i
             Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(sub + row * (int64_t)C + v * VEC), s);
 #pragma unroll
             for (int c = 0; c < VEC; c++) d[c] = Elem<T>::round(d[c] - s[c]);
+        }
+        if (mean && sz > 1) {
+            const float area = (float)(sz * sz);
+#pragma unroll
+            for (int c = 0; c < VEC; c++) d[c] = d[c] / area;
         }
         const int64_t tok = y0 < 0 ? (-y0 - 1) : (y0 * W + x0 + extra);
         const int64_t off = (b * N + tok) * (int64_t)C + v * VEC;
@@ -1553,9 +1560,9 @@ extern "C" int vtdge_index_to_patch_dense(const int64_t *splits_host, int B, int
     return check_launch("index_to_patch_dense");
 }
 
-extern "C" int vtdge_compress(const void *x, const int64_t *patches, const int64_t *rows_dev, int64_t rows,
-                              void *out, void *ln_out, const void *ln_weight, const void *ln_bias, float ln_eps,
-                              int B, int N, int C, int W, int extra, int dtype, void *stream)
+static int compress_launch(const void *x, const int64_t *patches, const int64_t *rows_dev, int64_t rows, void *out,
+                           void *ln_out, const void *ln_weight, const void *ln_bias, float ln_eps, int B, int N, int C,
+                           int W, int extra, int dtype, void *stream, bool sum)
 {
     VT_REQUIRE(x && patches && out, VTDGE_ERR_ARG, "compress: NULL operand");
     VT_REQUIRE(B > 0 && N > 0 && W > 0 && extra >= 0 && rows >= 0, VTDGE_ERR_ARG, "compress: bad sizes");
@@ -1575,7 +1582,7 @@ extern "C" int vtdge_compress(const void *x, const int64_t *patches, const int64
     note_kernel(reinterpret_cast<const void *>(compress_kernel<T, LNF, GS, NIT>)),                                  \
     compress_kernel<T, LNF, GS, NIT><<<grid, block, 0, st>>>((const T *)x, patches, rows_dev, rows, (T *)out,       \
                                                              (T *)ln_out, (const T *)ln_weight, (const T *)ln_bias, \
-                                                             ln_eps, N, C, W, extra)
+                                                             ln_eps, N, C, W, extra, sum)
 #define VT_LNF(T, GS, NIT) do { if (ln) VT_LAUNCH(T, true, GS, NIT); else VT_LAUNCH(T, false, GS, NIT); } while (0)
 #define VT_GROUP(T) \
     do { if (gs == 64) { if (C / vec > WAVE) VT_LNF(T, 64, MAX_IT); else VT_LNF(T, 64, 1); } \
@@ -1587,9 +1594,24 @@ extern "C" int vtdge_compress(const void *x, const int64_t *patches, const int64
     return check_launch("compress");
 }
 
-extern "C" int vtdge_decompress(const void *in, const void *sub, const int64_t *patches, const int64_t *rows_dev,
-                                int64_t rows, const void *ref, void *out, int B, int N, int C, int W, int extra,
-                                int dtype, void *stream)
+extern "C" int vtdge_compress(const void *x, const int64_t *patches, const int64_t *rows_dev, int64_t rows,
+                              void *out, void *ln_out, const void *ln_weight, const void *ln_bias, float ln_eps,
+                              int B, int N, int C, int W, int extra, int dtype, void *stream)
+{
+    return compress_launch(x, patches, rows_dev, rows, out, ln_out, ln_weight, ln_bias, ln_eps, B, N, C, W, extra, dtype,
+                           stream, false);
+}
+
+extern "C" int vtdge_compress_sum(const void *x, const int64_t *patches, int64_t rows, void *out, int B, int N, int C, int W,
+                                  int extra, int dtype, void *stream)
+{
+    return compress_launch(x, patches, nullptr, rows, out, nullptr, nullptr, nullptr, 0.f, B, N, C, W, extra, dtype, stream,
+                           true);
+}
+
+static int decompress_launch(const void *in, const void *sub, const int64_t *patches, const int64_t *rows_dev, int64_t rows,
+                             const void *ref, void *out, int B, int N, int C, int W, int extra, int dtype, void *stream,
+                             bool mean)
 {
     VT_REQUIRE(in && patches && out, VTDGE_ERR_ARG, "decompress: NULL operand");
     VT_REQUIRE(B > 0 && N > 0 && W > 0 && extra >= 0 && rows >= 0, VTDGE_ERR_ARG, "decompress: bad sizes");
@@ -1608,7 +1630,8 @@ extern "C" int vtdge_decompress(const void *in, const void *sub, const int64_t *
 #define VT_LAUNCH(T, SUBF, ADDF, GS)                                                                              \
     note_kernel(reinterpret_cast<const void *>(decompress_kernel<T, SUBF, ADDF, GS>)),                             \
     decompress_kernel<T, SUBF, ADDF, GS><<<grid, block, 0, st>>>((const T *)in, (const T *)sub, patches, rows_dev, \
-                                                                 rows, (const T *)ref, (T *)out, N, C, W, extra)
+                                                                 rows, (const T *)ref, (T *)out, N, C, W, extra,   \
+                                                                 mean)
 #define VT_DISPATCH(T, GS)                                       \
     do {                                                         \
         if (sub && ref) VT_LAUNCH(T, true, true, GS);            \
@@ -1624,6 +1647,19 @@ extern "C" int vtdge_decompress(const void *in, const void *sub, const int64_t *
 #undef VT_DISPATCH
 #undef VT_LAUNCH
     return check_launch("decompress");
+}
+
+extern "C" int vtdge_decompress(const void *in, const void *sub, const int64_t *patches, const int64_t *rows_dev,
+                                int64_t rows, const void *ref, void *out, int B, int N, int C, int W, int extra,
+                                int dtype, void *stream)
+{
+    return decompress_launch(in, sub, patches, rows_dev, rows, ref, out, B, N, C, W, extra, dtype, stream, false);
+}
+
+extern "C" int vtdge_decompress_mean(const void *in, const int64_t *patches, int64_t rows, const void *add, void *out, int B,
+                                     int N, int C, int W, int extra, int dtype, void *stream)
+{
+    return decompress_launch(in, nullptr, patches, nullptr, rows, add, out, B, N, C, W, extra, dtype, stream, true);
 }
 
 extern "C" int vtdge_decompress_layernorm(const void *in, const void *sub, const int64_t *patches,

@@ -2,8 +2,8 @@
 
 `grained_sample_compress`, `grained_sample_decompress` and `grained_sample_index_to_patch` keep
 the reference's positional signatures.  Forward passes run on the HIP kernels; the backward rules
-are the reference's (compress and decompress are adjoint up to size**2) expressed with the same
-two kernels.
+are the reference's (compress and decompress are adjoint up to size**2) on the same two kernels, which
+leave out or put in the division by the area.
 """
 import torch
 import torch.nn.functional as F
@@ -13,25 +13,20 @@ from torch.autograd.function import once_differentiable
 from .. import _C
 
 
-def _area(patches):
-    return (patches[:, 3:4] * patches[:, 3:4])
-
-
 class _Compress(Function):
     # vtpack/layers/grained_sample.py:11-38
     @staticmethod
     def forward(ctx, input, patches, height, width, num_extra_tokens):
         input, patches = input.contiguous(), patches.contiguous()
-        ctx.geom = (height, width, num_extra_tokens)
-        ctx.save_for_backward(input, patches)
+        ctx.geom, ctx.shape = (height, width, num_extra_tokens), input.shape
+        ctx.save_for_backward(patches)
         return _C.grained_sample_compress(input, patches, height, width, num_extra_tokens)
 
     @staticmethod
     @once_differentiable
     def backward(ctx, grad):
-        input, patches = ctx.saved_tensors
-        grad = grad.contiguous() / _area(patches).to(grad.dtype)
-        return _C.grained_sample_decompress(grad, patches, input, *ctx.geom, False), None, None, None, None
+        patches, = ctx.saved_tensors
+        return _C.grained_sample_decompress_mean(grad.contiguous(), patches, ctx.shape, *ctx.geom), None, None, None, None
 
 
 class _Decompress(Function):
@@ -49,7 +44,7 @@ class _Decompress(Function):
     def backward(ctx, grad):
         patches, = ctx.saved_tensors
         grad = grad.contiguous()
-        g_in = _C.grained_sample_compress(grad, patches, *ctx.geom) * _area(patches).to(grad.dtype)
+        g_in = _C.grained_sample_compress_sum(grad, patches, *ctx.geom)
         g_ref = grad if ctx.is_add_ref else torch.zeros_like(grad)
         return g_in, None, g_ref, None, None, None, None
 

@@ -3,7 +3,7 @@ import torch
 from torch.autograd import Function
 from torch.autograd.function import once_differentiable
 
-from .. import _C
+from .. import _C, ops
 
 
 class _SparseGEMM(Function):
@@ -32,8 +32,7 @@ class _SparseAttention(Function):
     # vtpack/layers/sparse_ops.py:60-73 (forward only there as well)
     @staticmethod
     def forward(ctx, q, k, v, q_lengths, scale):
-        return _C.batched_sparse_attention_forward(q.contiguous(), k.contiguous(), v.contiguous(),
-                                                   q_lengths.contiguous(), scale)
+        return _C.batched_sparse_attention_forward(q, k, v, q_lengths, scale)
 
     @staticmethod
     def backward(ctx, grad):
@@ -44,18 +43,48 @@ batched_sparse_gemm = _SparseGEMM.apply
 batched_sparse_attention = _SparseAttention.apply
 
 
+class _SparseAttentionTrain(Function):
+    """Attention of packed queries with gradients, without score-sized tensors: the inference kernel forward, scores worked
+    out again from q and k backward.  q [h, L, d], k and v [h, B, n, d] -> [L, h * d]."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, q_lengths, scale):
+        q, k, v = ops.vector_rows(q), k.contiguous(), v.contiguous()
+        h, L, d = q.shape
+        offsets, lengths = ops.lengths_to_offsets(q_lengths, q.device)
+        out = torch.empty((L, h * d), dtype=q.dtype, device=q.device)
+        ctx.scale, ctx.max_rows = scale, int(lengths.max())
+        ops.sparse_attention_heads(q, k, v, offsets, scale, ctx.max_rows, out=out.view(L, h, d).transpose(0, 1))
+        ctx.save_for_backward(q, k, v, out, offsets)
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad):
+        q, k, v, out, offsets = ctx.saved_tensors
+        h, L, d = q.shape
+        heads = [ops.vector_rows(t.reshape(L, h, d).transpose(0, 1)) for t in (out, grad.contiguous())]
+        dq, dk, dv = ops.sparse_attention_backward(q, k, v, *heads, offsets, ctx.scale, ctx.max_rows)
+        return dq, dk, dv, None, None
+
+
 def sparse_attention_train(q, k, v, q_lengths, scale):
     """Differentiable attention of packed queries for the training branch of the models
     (vtpack/models/dge/deit_dge.py:79-95): q [h, L, d]; k, v [h, B, n, d]; -> [L, h*d].
 
-    Equal query counts (dense training: every granularity for every sample) use one batched matmul; otherwise the
-    scores and the weighted sum are two `batched_sparse_gemm` calls around a softmax over the keys."""
+    Equal query counts (dense training: every granularity for every sample) use one batched matmul.  Otherwise, on the GPU
+    with head dim 64, one attention kernel forward and two backward; other operands compose two `batched_sparse_gemm` calls
+    around a softmax over the keys."""
     h, L, d = q.shape
     B, n = k.shape[1], k.shape[2]
     if int(q_lengths.max()) == int(q_lengths.min()):
         scores = torch.matmul(q.reshape(h, B, -1, d), k.transpose(-1, -2)) * scale
         ctx = torch.matmul(scores.softmax(dim=-1, dtype=v.dtype), v)              # [h, B, Lq, d]
         return ctx.permute(1, 2, 0, 3).reshape(-1, h * d)
+    if (d == 64 and q.is_cuda and q.dtype in (torch.float32, torch.bfloat16) and q.dtype == k.dtype == v.dtype
+            and k.shape == v.shape and k.shape[0] == h and k.shape[3] == d and q_lengths.numel() == B
+            and int(q_lengths.sum()) == L):
+        return _SparseAttentionTrain.apply(q, k, v, q_lengths, float(scale))
     kv_lengths = q_lengths.new_full([B], n)
     scores = batched_sparse_gemm(q, k.reshape(h, -1, d), q_lengths, kv_lengths, False, True) * scale
     ctx = batched_sparse_gemm(scores.softmax(dim=-1, dtype=v.dtype), v.reshape(h, -1, d), q_lengths, kv_lengths,

@@ -152,6 +152,28 @@ def decompress(inp, patches, reference, width, num_extra_tokens, add_ref=True, s
     return out
 
 
+def compress_sum(x, patches, width, num_extra_tokens):
+    """x [B,N,C] -> [L,C]: the sum of the tokens each patch covers (the adjoint of the scatter back)."""
+    _need_gpu(x, patches)
+    x, patches = _contig(x), _contig(patches)
+    B, N, C = x.shape
+    out = torch.empty((patches.shape[0], C), dtype=x.dtype, device=x.device)
+    call("vtdge_compress_sum", ptr(x), ptr(patches), patches.shape[0], ptr(out), B, N, C, width, num_extra_tokens,
+         dtype_code(x), stream_ptr(), tag=("compress_sum", C))
+    return out
+
+
+def decompress_mean(inp, patches, shape, width, num_extra_tokens):
+    """inp [L,C] -> [B,N,C] = shape: every token its patch's row divided by the patch's area (the adjoint of compress)."""
+    _need_gpu(inp, patches)
+    inp, patches = _contig(inp), _contig(patches)
+    B, N, C = shape
+    out = torch.empty((B, N, C), dtype=inp.dtype, device=inp.device)
+    call("vtdge_decompress_mean", ptr(inp), ptr(patches), patches.shape[0], 0, ptr(out), B, N, C, width, num_extra_tokens,
+         dtype_code(inp), stream_ptr(), tag=("decompress_mean", C))
+    return out
+
+
 def decompress_layernorm(inp, patches, reference, width, num_extra_tokens, ln_weight, ln_bias, ln_eps=1e-6, sub=None,
                          rows_dev=None, rows=None):
     """Scatter (inp - sub) + reference back over the tokens, and the LayerNorm of the result: (out, LayerNorm(out))."""
@@ -831,3 +853,48 @@ def sparse_attention(q, k, v, offsets, scale, num_heads, max_rows_per_sample, ou
          ptr(offsets), ptr(out), out.stride(0), d, B, num_heads, d, n, int(max_rows_per_sample), float(scale),
          dtype_code(q), stream_ptr(), tag=("attention", B, num_heads, d, n))
     return out
+
+
+def lengths_to_offsets(lengths, device):
+    """CPU int64 lengths [B] -> device int64 offsets [B + 1], without a copy of host memory."""
+    lengths = lengths.detach().to("cpu", torch.int64).contiguous()
+    offsets = torch.empty((lengths.numel() + 1,), dtype=torch.int64, device=device)
+    call("vtdge_lengths_to_offsets", lengths.data_ptr(), lengths.numel(), ptr(offsets), stream_ptr(), tag=("offsets",))
+    return offsets, lengths
+
+
+def vector_rows(t):
+    """t itself where its last dimension is dense and every row starts on a 16-byte boundary, else a dense copy."""
+    vec = 16 // t.element_size()
+    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % vec == 0 for s in t.stride()[:-1]):
+        return t
+    return t.contiguous()
+
+
+def sparse_attention_heads(q, k, v, offsets, scale, max_rows_per_sample, out=None):
+    """Head-major form: q [h, L, d], k and v [h, B, n, d] (rows on 16-byte boundaries, k and v with the same strides)
+    -> out, a [h, L, d] view of any strides like q's (by default dense)."""
+    h, L, d = q.shape
+    B, n = k.shape[1], k.shape[2]
+    if out is None:
+        out = torch.empty((h, L, d), dtype=q.dtype, device=q.device)
+    call("vtdge_sparse_attention", ptr(q), q.stride(1), q.stride(0), ptr(k), ptr(v), k.stride(1), k.stride(2), k.stride(0),
+         ptr(offsets), ptr(out), out.stride(1), out.stride(0), B, h, d, n, max_rows_per_sample, float(scale), dtype_code(q),
+         stream_ptr(), tag=("attention", B, h, d, n))
+    return out
+
+
+def sparse_attention_backward(q, k, v, out, grad, offsets, scale, max_rows_per_sample):
+    """Gradients (dq, dk, dv) of `sparse_attention_heads` with head dim 64: q [h, L, d] with rows on 16-byte boundaries, k
+    and v [h, B, n, d] dense; out and grad [h, L, d] views with the same strides.  dq has q's strides order ([L, h, d] in
+    memory), dk and dv are dense."""
+    h, L, d = q.shape
+    B, n = k.shape[1], k.shape[2]
+    dq = torch.empty((L, h, d), dtype=q.dtype, device=q.device).transpose(0, 1)
+    dk, dv = torch.empty_like(k), torch.empty_like(v)
+    work = torch.empty((2 * h * L,), dtype=torch.float32, device=q.device)
+    call("vtdge_sparse_attention_backward", ptr(q), q.stride(1), q.stride(0), ptr(k), ptr(v), k.stride(1), k.stride(2),
+         k.stride(0), ptr(out), ptr(grad), out.stride(1), out.stride(0), ptr(offsets), ptr(dq), dq.stride(1), dq.stride(0),
+         ptr(dk), ptr(dv), dk.stride(1), dk.stride(2), dk.stride(0), ptr(work), L, B, h, d, n, max_rows_per_sample,
+         float(scale), dtype_code(q), stream_ptr(), tag=("attention_backward", B, h, d, n))
+    return dq, dk, dv
