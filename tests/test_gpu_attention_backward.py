@@ -49,6 +49,31 @@ def test_against_float64(dev, dtype, n, lengths, scale, dense):
         *args, torch.tensor(lengths), scale), args, g.to(dev))))                      # the same bytes on every call
 
 
+@pytest.mark.parametrize("which", ["q", "k", "v", "grad", "hook"])
+def test_operands_off_a_16_byte_boundary(dev, which):
+    """Operands that start 4 bytes behind a boundary, and saved tensors that come back from a hook that way."""
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    h, n, lengths = 2, 33, [5, 17]
+    L, B = sum(lengths), len(lengths)
+
+    def shifted(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        flat[1:] = t.reshape(-1)
+        return flat[1:].view(t.shape)
+
+    host = {name: torch.from_numpy(randn(i, *s)) for i, (name, s) in enumerate(
+        {"q": (h, L, 64), "k": (h, B, n, 64), "v": (h, B, n, 64), "grad": (L, h * 64)}.items())}
+    on = {name: shifted(t.to(dev)) if name == which else t.to(dev) for name, t in host.items()}
+    args = [on[name].requires_grad_(True) for name in "qkv"]
+    with torch.autograd.graph.saved_tensors_hooks(
+            lambda t: t, (lambda t: shifted(t) if t.is_floating_point() else t) if which == "hook" else lambda t: t):
+        got = sparse_attention_train(*args, torch.tensor(lengths), 0.125)
+    grads = torch.autograd.grad(got, args, on["grad"])
+    want, wants = _reference(host["q"], host["k"], host["v"], lengths, 0.125, host["grad"])
+    for a, b in zip((got.detach(),) + grads, (want,) + wants):
+        assert float((a.double().cpu() - b).abs().max()) <= 1e-5 * float(b.abs().max())
+
+
 @pytest.mark.parametrize("B", [1, 3, 447, 448, 449, 1000])
 def test_offsets_of_lengths(dev, B):
     from vtpack_amd import ops

@@ -54,3 +54,19 @@ def test_scale_zero_and_negative(dev, scale):
     lengths = np.array([30, 70], dtype=np.int64)
     q, k, v = randn(920, 1, 100, 64), randn(921, 1, 2, 40, 64), randn(922, 1, 2, 40, 64)
     assert_close(_run(dev, q, k, v, lengths, scale), orc.attention(q, k, v, lengths, scale), torch.float32, "scale")
+
+
+@pytest.mark.parametrize("rows", [1, 20, 64])
+def test_first_stages_without_a_finite_score(dev, rows):
+    """Scores that overflow to -infinity over the first 70 keys (more than two stages): probability zero, the rest as usual."""
+    n = 150
+    q, k, v = randn(930, 1, rows, 64), randn(931, 1, 1, n, 64), randn(932, 1, 1, n, 64)
+    q[:, ::2, 0], k[:, :, :, 0] = 1e30, 0.0
+    k[:, :, :70, 0] = -1e30
+    q[:, 1::2, 0] = 0.0                                     # every other query sees all keys
+    got = _run(dev, q, k, v, np.array([rows], dtype=np.int64), 0.125)
+    s = np.einsum("hld,hnd->hln", q[..., 1:].astype(np.float64), k[:, 0, :, 1:].astype(np.float64)) * 0.125
+    s[:, ::2, :70] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = (p / p.sum(-1, keepdims=True)) @ v[:, 0].astype(np.float64)
+    assert float(np.abs(got.numpy() - want).max()) <= 1e-5 * np.abs(want).max()

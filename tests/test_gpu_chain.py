@@ -107,6 +107,19 @@ def test_changes_of_the_parameters_are_seen(dev):
         fresh.weight.mul_(0.1)
     m.blocks[0].mlp.fc1, m.blocks[0].mlp.fc2 = fresh.to(dev).bfloat16(), torch.nn.Linear(768, 384).to(dev).bfloat16()
     check(m)                                     # the blocks are no longer alike: composed
+    # numbers of the modules, and a parameter that keeps its storage and its version but not its shape
+    other.blocks[1].norm1.eps = 0.5
+    check(other)
+    first = _run(other, images, True)[0]
+    for blk in other.blocks:
+        blk.attn.scale, blk.attn.num_heads = 0.3, 12
+    check(other)
+    first = _run(other, images, True)[0]
+    with pytest.raises(ValueError):
+        short = copy.deepcopy(other)
+        _run(short, images, True)
+        short.blocks[1].mlp.fc2.bias.data = short.blocks[1].mlp.fc2.bias.data[:192]
+        _run(short, images, True)
     m32 = copy.deepcopy(other).float()
     assert torch.equal(_run(m32, images.float(), True)[0], _run(m32, images.float(), False)[0])
 

@@ -145,20 +145,19 @@ __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
                     if (key0 + 16 * i + r >= n) s[i][r] = -INFINITY;
                 mx = fmaxf(mx, s[i][r]);
             }
-        if (first || __any(mx > AF_RAISE)) {
+        if (__any(first || mx > AF_RAISE)) {
             mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
             mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
-            const float d = first ? mx : fmaxf(mx, 0.f);
+            // a query that has met scores of -infinity only has no reference yet: its probabilities are zero, it waits
+            const float d = !first ? fmaxf(mx, 0.f) : mx == -INFINITY ? 0.f : mx;
+            const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-d);
+            first = first && mx == -INFINITY;
             neg_m -= d;
 #pragma unroll
             for (int i = 0; i < NB; i++) s[i] -= d;
-            if (!first) {
-                const float alpha = __builtin_amdgcn_exp2f(-d);
-                l_run *= alpha;
+            l_run *= alpha;
 #pragma unroll
-                for (int i = 0; i < G::NDB; i++) o[i] *= alpha;
-            }
-            first = false;
+            for (int i = 0; i < G::NDB; i++) o[i] *= alpha;
         }
 #pragma unroll
         for (int i = 0; i < NB; i++)

@@ -10,6 +10,7 @@ be captured into a HIP graph.
 """
 import array
 import ctypes
+import operator
 
 import torch
 
@@ -506,6 +507,18 @@ def _common_of(blocks, tensors, dtype, device, channels, extra):
     return dict(seen, extra=extra, depth=len(blocks), dtype=_lib.BF16 if dtype == torch.bfloat16 else _lib.F32)
 
 
+def _block_numbers(blk):
+    """What else of a block a plan is made from."""
+    m = blk._modules
+    at = m["attn"]
+    norm = at._modules.get("norm")
+    return (m["norm1"].eps, m["norm2"].eps, None if norm is None else norm.eps, m["dge"].region_size, at.scale, at.num_heads,
+            at.__dict__.get("sr_ratio", 1))
+
+
+_TENSOR_STATE = (torch.Tensor.data_ptr, torch.Tensor.is_contiguous, *map(operator.attrgetter, ("_version", "dtype", "shape")))
+
+
 def _chain_plan(blocks, dtype, device, channels, extra):
     """The plan of a chain of blocks for tokens of this kind, made anew where a parameter has changed since; None where
     the blocks are composed one by one."""
@@ -516,10 +529,9 @@ def _chain_plan(blocks, dtype, device, channels, extra):
         return None
     try:
         tensors = [_block_tensors(blk) for blk in blocks]
-        flat = [t for ts in tensors for t in ts]
-        key = ([0 if t is None else t.data_ptr() for t in flat], [0 if t is None else t._version for t in flat],
-               [None if t is None else t.dtype for t in flat], dtype, device, extra, channels,
-               [blk.attn.scale for blk in blocks], ops._pack_epoch, ops._plan_epoch)
+        flat = [t for ts in tensors for t in ts if t is not None]
+        key = (*(list(map(f, flat)) for f in _TENSOR_STATE), [t is None for ts in tensors for t in ts], dtype, device, extra,
+               channels, [_block_numbers(blk) for blk in blocks], ops._pack_epoch, ops._plan_epoch)
     except (KeyError, AttributeError):
         return None
     plan = getattr(blocks[0], "_vtdge_chain", None)

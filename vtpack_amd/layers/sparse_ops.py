@@ -49,7 +49,7 @@ class _SparseAttentionTrain(Function):
 
     @staticmethod
     def forward(ctx, q, k, v, q_lengths, scale):
-        q, k, v = ops.vector_rows(q), k.contiguous(), v.contiguous()
+        q, k, v = (ops.on_boundary(t) for t in (ops.vector_rows(q), k.contiguous(), v.contiguous()))
         h, L, d = q.shape
         offsets, lengths = ops.lengths_to_offsets(q_lengths, q.device)
         out = torch.empty((L, h * d), dtype=q.dtype, device=q.device)
@@ -63,7 +63,9 @@ class _SparseAttentionTrain(Function):
     def backward(ctx, grad):
         q, k, v, out, offsets = ctx.saved_tensors
         h, L, d = q.shape
-        heads = [ops.vector_rows(t.reshape(L, h, d).transpose(0, 1)) for t in (out, grad.contiguous())]
+        # out and the gradient share their strides in the kernel, k and v too; a saved-tensor hook may lay them out anew
+        q, k, v, out, grad = (ops.on_boundary(t) for t in (ops.vector_rows(q), *(t.contiguous() for t in (k, v, out, grad))))
+        heads = [t.view(L, h, d).transpose(0, 1) for t in (out, grad)]
         dq, dk, dv = ops.sparse_attention_backward(q, k, v, *heads, offsets, ctx.scale, ctx.max_rows)
         return dq, dk, dv, None, None
 

@@ -871,6 +871,11 @@ def vector_rows(t):
     return t.contiguous()
 
 
+def on_boundary(t):
+    """t itself where its memory starts on a 16-byte boundary, else a copy."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def sparse_attention_heads(q, k, v, offsets, scale, max_rows_per_sample, out=None):
     """Head-major form: q [h, L, d], k and v [h, B, n, d] (rows on 16-byte boundaries, k and v with the same strides)
     -> out, a [h, L, d] view of any strides like q's (by default dense)."""
