@@ -441,6 +441,20 @@ int vtdge_layernorm_linear(const void *A0, int64_t lda0, const void *W0, const v
                            const void *ln_weight, const void *ln_bias, float ln_eps, int K, int act, int dtype,
                            void *stream);
 
+/* What a block does with its packed queries behind attention (vtpack/models/dge/deit_dge.py:127-128 with :74-75 and
+ * :38-44), as one kernel without the hidden rows in memory:
+ *   q1 = o proj_weight^T + proj_bias + comp,   out = q1 + fc2(gelu(fc1(LayerNorm(q1))))
+ * q1, LayerNorm(q1) and the hidden rows are rounded to the storage type as the modules would round them.
+ *   o, comp, out  [rows, C] dense, out a buffer of its own; biases nullable, rows_dev nullable (device int64: the live rows)
+ * Taken where vtdge_block_tail_fits says 1 (bf16, 64, 128 or 192 channels, hidden a multiple of 64 and at most 4096);
+ * VTDGE_ERR_UNSUPPORTED otherwise.  vtdge_block_tail_wanted: whether it is also the faster way for that many rows. */
+int vtdge_block_tail_fits(int64_t rows, int C, int hidden, int dtype);
+int vtdge_block_tail_wanted(int64_t rows, int C, int hidden, int dtype);
+int vtdge_block_tail(const void *o, const void *comp, const void *proj_weight, const void *proj_bias,
+                     const void *ln_weight, const void *ln_bias, float ln_eps, const void *fc1_weight, const void *fc1_bias,
+                     const void *fc2_weight, const void *fc2_bias, void *out, const int64_t *rows_dev, int64_t rows, int C,
+                     int hidden, int dtype, void *stream);
+
 /* A chain of DGE transformer blocks on one token grid (vtpack/models/dge/deit_dge.py:101-131 or pvt_dge.py:111-140,
  * `depth` of them in a row), issued by one host call: the launches are those of the entry points above, in the order a
  * caller that composes a block from them would issue them, with nothing of the host between them.

@@ -50,7 +50,7 @@ def _same(a, b):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("dim,batch,kw", [(64, 1, {}), (192, 3, {}), (384, 1, {}), (384, 33, {}), (384, 40, {"img": 192}),
-                                          (768, 2, {}), (384, 31, {"distilled": True}), (192, 2, {"cls_token": False}),
+                                          (768, 2, {}), (192, 130, {}), (384, 31, {"distilled": True}), (192, 2, {"cls_token": False}),
                                           (384, 32, {"depth": 1})])
 @pytest.mark.parametrize("two_streams", [False, True])
 def test_deit(dev, dtype, dim, batch, kw, two_streams):
@@ -72,7 +72,7 @@ def test_deit(dev, dtype, dim, batch, kw, two_streams):
             assert _same(a[k], b[k]), (i, k)
 
 
-@pytest.mark.parametrize("dtype,batch", [(torch.float32, 1), (torch.bfloat16, 3), (torch.bfloat16, 9)])
+@pytest.mark.parametrize("dtype,batch", [(torch.float32, 1), (torch.bfloat16, 3), (torch.bfloat16, 9), (torch.bfloat16, 33)])
 def test_pvt(dev, dtype, batch):
     m = _pvt(dev, dtype)
     images = synthetic_images(batch, 128, seed=6, dtype=dtype, device=dev)

@@ -35,6 +35,7 @@ struct ChainPlan {
     int esz, N, n_kv;              // tokens per sample, keys per sample
     bool folded;                   // norms folded into weight-stationary Linears, chained scatter-back (384-channel bf16)
     bool by_region, pack;          // compress by region; the scatter-back packs the next block's queries
+    bool tail;                     // narrow bf16 rows: everything behind attention as one kernel
     bool ln_kvq, ln_fc1;           // few rows: norm1 inside the kv and q Linear, norm2 inside fc1
     int64_t ws_words;
     // byte offsets
@@ -70,7 +71,8 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
     p.folded = p.by_region && c->dtype == VTDGE_BF16 && c->C == 384 && p.rows >= 2048 && c->sr == 1 &&
                c->hidden % 384 == 0 && c->hidden <= 3072;
     p.ln_kvq = !p.folded && c->sr == 1 && vtdge_layernorm_linear_fits(p.rows, 2 * c->C, p.cap, c->C, c->C, c->dtype);
-    p.ln_fc1 = !p.folded && vtdge_layernorm_linear_fits(p.cap, c->hidden, 0, 0, c->C, c->dtype);
+    p.tail = vtdge_block_tail_wanted(p.rows, c->C, c->hidden, c->dtype);
+    p.ln_fc1 = !p.folded && !p.tail && vtdge_layernorm_linear_fits(p.cap, c->hidden, 0, 0, c->C, c->dtype);
     p.pack = p.folded && c->depth > 1 && p.regions % 4 == 0;
     p.ws_words = p.pack ? vtdge_decompress_router_compress_workspace(c->B, c->H, c->W, 4) / 8 : 0;
 
@@ -105,9 +107,9 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
     p.comp_ln = p.folded ? 0 : take(row);
     p.q = take(row);
     p.o = take(row);
-    p.q1 = take(row);
-    p.q1_ln = p.folded ? 0 : take(row);
-    p.hid = take(p.cap * c->hidden * p.esz);
+    p.q1 = p.tail ? 0 : take(row);
+    p.q1_ln = p.folded || p.tail ? 0 : take(row);
+    p.hid = p.tail ? 0 : take(p.cap * c->hidden * p.esz);
     p.rec2 = p.folded ? take(p.rows * 32) : 0;
     for (int i = 0; i < 2; i++) {
         p.rec_x[i] = p.folded ? take(p.rows * 32) : 0;
@@ -246,7 +248,10 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
         }
         VT_TRY(vtdge_sparse_attention(q, C, d, kv, kv + (int64_t)C * esz, (int64_t)p.n_kv * 2 * C, 2 * C, d, offsets, o, C,
                                       d, B, c->heads, d, p.n_kv, N, c->scale, dt, stream));
-        if (p.folded) {
+        if (p.tail) {
+            VT_TRY(vtdge_block_tail(o, comp, P[P_PROJW], P[P_PROJB], P[P_N2W], P[P_N2B], c->eps2, P[P_FC1W], P[P_FC1B],
+                                    P[P_FC2W], P[P_FC2B], q2, live, p.cap, C, c->hidden, dt, stream));
+        } else if (p.folded) {
             VT_TRY(vtdge_linear_stats(o, C, P[P_PROJW], P[P_PROJP], P[P_PROJB], comp, C, q1, C, scratch + p.rec2, c->eps2,
                                       live, p.cap, C, C, dt, stream));
             VT_TRY(vtdge_linear_layernorm(q1, C, scratch + p.rec2, P[P_FC1FW], P[P_FC1FP], P[P_FC1FR], hid, c->hidden,
@@ -265,8 +270,9 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
                                               p.cap, c->hidden, C, VTDGE_ACT_GELU, dt, stream));
             }
         }
-        VT_TRY(vtdge_linear_prepacked(hid, c->hidden, P[P_FC2W], pk(P_FC2P), P[P_FC2B], q1, C, q2, C, live, p.cap, C,
-                                      c->hidden, VTDGE_ACT_NONE, dt, stream));
+        if (!p.tail)
+            VT_TRY(vtdge_linear_prepacked(hid, c->hidden, P[P_FC2W], pk(P_FC2P), P[P_FC2B], q1, C, q2, C, live, p.cap, C,
+                                          c->hidden, VTDGE_ACT_NONE, dt, stream));
         if (Q == nullptr) {
             VT_TRY(vtdge_decompress(q2, comp, patches, live, p.cap, x, xout, B, N, C, W, extra, dt, stream));
             break;

@@ -87,6 +87,10 @@ REGION_ROWS = True
 PACK_NEXT = True
 
 
+# Narrow bf16 models (64, 128, 192 channels): projection, LayerNorm and MLP of the packed queries as one kernel (from some thousand rows).
+FUSE_TAIL = True
+
+
 # A chain of blocks as one call into the library (`vtdge_chain_forward`): the same kernels in the same order, without
 # the 25 - 30 us of interpreter time each of them costs when it is issued from here (77 launches of a 12-block model:
 # 2.2 ms of host time, more than the GPU needs below a batch of about 150).  Taken where every switch above is at its
@@ -100,7 +104,7 @@ NATIVE_CHAIN = True
 OVERLAP_FROM = 2 << 20
 _SWITCHES = ("OVERLAP", "FUSE_NEXT_NORM", "FUSE_ROUTER_NORM", "FUSE_NEXT_ROUTER", "FOLD_NORMS", "FUSE_PATCH_EMBED",
              "ROUTING_ON_SIDE", "Q_AFTER_JOIN", "REGION_COMPRESS", "SERIAL_BESIDE_WEIGHT_STATIONARY", "ROUTING_FIRST",
-             "Q_BEFORE_KV", "PAIR_KV_Q", "ROUTER_STATS", "REGION_ROWS", "PACK_NEXT", "NORM_IN_LINEAR", "NATIVE_CHAIN")
+             "Q_BEFORE_KV", "PAIR_KV_Q", "ROUTER_STATS", "REGION_ROWS", "PACK_NEXT", "NORM_IN_LINEAR", "FUSE_TAIL", "NATIVE_CHAIN")
 _defaults = tuple(globals()[name] for name in _SWITCHES)
 
 
@@ -348,23 +352,27 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
             if q is None:
                 q = q_linear()
     o = ops.sparse_attention(q, kv[:, :, :C], kv[:, :, C:], offsets, attn.scale, attn.num_heads, N)
-    fold2 = FOLD_NORMS and ops.fits_linear_layernorm(o, mlp.fc1.weight)
-    if fold2 and ops.fits_linear_stats(o, attn.proj.weight):
-        q1, rec2 = ops.linear(o, attn.proj.weight, attn.proj.bias, residual=comp, rows_dev=rows_dev, stats_eps=n2.eps)
+    tail = tuple((m.weight, m.bias) for m in (attn.proj, n2, mlp.fc1, mlp.fc2))
+    if FUSE_TAIL and ops.fits_block_tail(o, *tail):
+        q2 = ops.block_tail(o, comp, tail[0], tail[1], n2.eps, tail[2], tail[3], rows_dev=rows_dev)
     else:
-        q1 = ops.linear(o, attn.proj.weight, attn.proj.bias, residual=comp, rows_dev=rows_dev)
-        rec2 = ops.layernorm_stats(q1, n2.eps, rows_dev=rows_dev) if fold2 else None
+        fold2 = FOLD_NORMS and ops.fits_linear_layernorm(o, mlp.fc1.weight)
+        if fold2 and ops.fits_linear_stats(o, attn.proj.weight):
+            q1, rec2 = ops.linear(o, attn.proj.weight, attn.proj.bias, residual=comp, rows_dev=rows_dev, stats_eps=n2.eps)
+        else:
+            q1 = ops.linear(o, attn.proj.weight, attn.proj.bias, residual=comp, rows_dev=rows_dev)
+            rec2 = ops.layernorm_stats(q1, n2.eps, rows_dev=rows_dev) if fold2 else None
 
-    if fold2:
-        hid = ops.linear_layernorm(q1, rec2, mlp.fc1.weight, mlp.fc1.bias, n2.weight, n2.bias, act="gelu",
-                                   rows_dev=rows_dev)
-    elif NORM_IN_LINEAR and ops.fits_layernorm_linear(q1, mlp.fc1.weight):
-        hid = ops.layernorm_linear(q1, mlp.fc1.weight, mlp.fc1.bias, n2.weight, n2.bias, n2.eps, act="gelu",
-                                   rows_dev=rows_dev)
-    else:
-        q1_ln = ops.layernorm(q1, n2.weight, n2.bias, n2.eps, rows_dev=rows_dev)
-        hid = ops.linear(q1_ln, mlp.fc1.weight, mlp.fc1.bias, act="gelu", rows_dev=rows_dev)
-    q2 = ops.linear(hid, mlp.fc2.weight, mlp.fc2.bias, residual=q1, rows_dev=rows_dev)
+        if fold2:
+            hid = ops.linear_layernorm(q1, rec2, mlp.fc1.weight, mlp.fc1.bias, n2.weight, n2.bias, act="gelu",
+                                       rows_dev=rows_dev)
+        elif NORM_IN_LINEAR and ops.fits_layernorm_linear(q1, mlp.fc1.weight):
+            hid = ops.layernorm_linear(q1, mlp.fc1.weight, mlp.fc1.bias, n2.weight, n2.bias, n2.eps, act="gelu",
+                                       rows_dev=rows_dev)
+        else:
+            q1_ln = ops.layernorm(q1, n2.weight, n2.bias, n2.eps, rows_dev=rows_dev)
+            hid = ops.linear(q1_ln, mlp.fc1.weight, mlp.fc1.bias, act="gelu", rows_dev=rows_dev)
+        q2 = ops.linear(hid, mlp.fc2.weight, mlp.fc2.bias, residual=q1, rows_dev=rows_dev)
 
     handed = {}
     nxt = next_block.dge if next_block is not None else None

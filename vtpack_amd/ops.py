@@ -833,6 +833,39 @@ def layernorm_linear(a, weight, bias, ln_weight, ln_bias, ln_eps, act="none", ro
     return outs[0] if second is None else tuple(outs)
 
 
+def fits_block_tail(o, proj, ln, fc1, fc2):
+    """Whether `block_tail` has a kernel for these operands (bf16, narrow rows, parameters on 16-byte boundaries) and it is the
+    faster way."""
+    C, w = o.shape[-1], fc1[0]
+    return bool(o.is_cuda and o.dtype == torch.bfloat16 and w.dim() == 2
+                and all(t is None or (t.dtype == o.dtype and t.data_ptr() % 16 == 0) for t in (*proj, *ln, *fc1, *fc2))
+                and _lib.load().vtdge_block_tail_wanted(o.numel() // C, C, w.shape[0], dtype_code(o)))
+
+
+def block_tail(o, comp, proj, ln, ln_eps, fc1, fc2, rows_dev=None):
+    """q1 = o Wp^T + bp + comp -> q1 + fc2(gelu(fc1(LayerNorm(q1)))) as one kernel; proj, ln, fc1, fc2 = (weight, bias).
+    See `fits_block_tail`."""
+    C, hidden = o.shape[-1], fc1[0].shape[0]
+    _need_gpu(o, comp, *proj, *ln, *fc1, *fc2)
+    _check_like(o, comp=comp, proj=proj[0], proj_bias=proj[1], ln_weight=ln[0], ln_bias=ln[1], fc1=fc1[0], fc1_bias=fc1[1],
+                fc2=fc2[0], fc2_bias=fc2[1])
+    for name, (w, b), shape in (("proj", proj, (C, C)), ("fc1", fc1, (hidden, C)), ("fc2", fc2, (C, hidden))):
+        if tuple(w.shape) != shape:
+            raise ValueError(f"{name} weight {tuple(w.shape)} is not {shape}")
+        _check_vector(name + " bias", b, shape[0])
+    _check_vector("ln_weight", ln[0], C)
+    _check_vector("ln_bias", ln[1], C)
+    if comp.shape != o.shape:
+        raise ValueError(f"comp {tuple(comp.shape)} is not like o {tuple(o.shape)}")
+    o, comp = _contig(o), _contig(comp)
+    vecs = [None if t is None else _contig(t) for t in (*proj, *ln, *fc1, *fc2)]
+    out = torch.empty_like(o)
+    rows = o.numel() // C
+    call("vtdge_block_tail", ptr(o), ptr(comp), *map(ptr, vecs[:4]), float(ln_eps), *map(ptr, vecs[4:]), ptr(out),
+         ptr(rows_dev), rows, C, hidden, dtype_code(o), stream_ptr(), tag=("block_tail", rows, C, hidden, rows_dev is not None))
+    return out
+
+
 def sparse_attention(q, k, v, offsets, scale, num_heads, max_rows_per_sample, out=None):
     """Strided form.  q [L, h*d]; k, v [B, n, h*d]-like views (last dim contiguous, any batch/token strides);
     offsets int64 [B+1] on the device.  Returns [L, h*d] with channel = head*d + j."""
