@@ -821,6 +821,19 @@ __global__ __launch_bounds__(256) void decompress_ln_kernel(const T *__restrict_
     }
 }
 
+// Statistics records of a region's 16 tokens held by one wave, four at a time.
+template <typename T>
+__device__ __forceinline__ void region_records(const u32x4 (&tok)[16], int W, int C, bool act, u32x4 *__restrict__ rec, float eps)
+{
+#pragma unroll
+    for (int dy = 0; dy < 4; dy++) {
+        float pivot[4], st[8];
+#pragma unroll
+        for (int dx = 0; dx < 4; dx++) lane_sums<T>(tok[4 * dy + dx], act, pivot[dx], st[2 * dx], st[2 * dx + 1]);
+        write_records4(st, pivot[0], pivot[1], pivot[2], pivot[3], C, eps, rec + (int64_t)dy * W * 2);
+    }
+}
+
 // ------------------------------------------------- decompress + next router
 // Scatter back by REGION instead of by packed row, so that the same wave can route the next block: a group of GS
 // lanes owns one R x R region (R = 4) of one sample.  The packed rows of a region are consecutive (regions in
@@ -909,6 +922,62 @@ __device__ __forceinline__ void region_scatter(const T *__restrict__ in, const T
     }
 }
 
+// The same with everything the region reads requested at once and its tokens kept as stored in `tok`: 16 + 2 PS^2 vectors a
+// lane, for launches of at most a wave a SIMD, where nothing else hides a round trip to memory.  GPU time of a forward, this
+// against the loop above, by workgroups of the launch: 4 (384 channels, one 256 px picture) 582 against 590 us, 20 (768, five)
+// 1183 against 1220, 52 (384, thirteen, with packing) 773 against 803, 54 to 216 (pyramid, fp32) 1541 against 1556; 512 (192,
+// fp32) and 396 (768) even, 1024 (384, 256 pictures) 3076 against 3000.
+template <typename T, int PS, bool SUB, bool STAT>
+__device__ __forceinline__ void region_scatter_held(const T *__restrict__ in, const T *__restrict__ sub, int64_t r0,
+                                                    const T *__restrict__ refp, T *__restrict__ outp, int W, int C,
+                                                    float (&acc)[Elem<T>::VEC], u32x4 (&tok)[16], bool act,
+                                                    u32x4 *__restrict__ rec, float eps)
+{
+    constexpr int VEC = Elem<T>::VEC;
+    constexpr int STEP = 4 / PS;
+    u32x4 ir[PS * PS], sr[SUB ? PS * PS : 1];
+    const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int j = 0; j < PS * PS; j++) {
+        ir[j] = z;
+        if (act) ir[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(in + (r0 + j) * (int64_t)C));
+    }
+    if constexpr (SUB)
+#pragma unroll
+        for (int j = 0; j < PS * PS; j++) {
+            sr[j] = z;
+            if (act) sr[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(sub + (r0 + j) * (int64_t)C));
+        }
+#pragma unroll
+    for (int t = 0; t < 16; t++) {
+        tok[t] = z;
+        if (act)
+            tok[t] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(refp + ((int64_t)(t / 4) * W + t % 4) * C));
+    }
+    if constexpr (SUB)
+#pragma unroll
+        for (int j = 0; j < PS * PS; j++) {
+            float dv[VEC], sv[VEC];
+            Elem<T>::unpack(ir[j], dv);
+            Elem<T>::unpack(sr[j], sv);
+#pragma unroll
+            for (int c = 0; c < VEC; c++) dv[c] -= sv[c];
+            ir[j] = Elem<T>::pack(dv);
+        }
+#pragma unroll
+    for (int t = 0; t < 16; t++) {
+        float r[VEC], dv[VEC];
+        Elem<T>::unpack(tok[t], r);
+        Elem<T>::unpack(ir[(t / 4 / STEP) * PS + t % 4 / STEP], dv);
+#pragma unroll
+        for (int c = 0; c < VEC; c++) r[c] += dv[c];
+        tok[t] = Elem<T>::pack(r);
+        if (act) *reinterpret_cast<u32x4 *>(outp + ((int64_t)(t / 4) * W + t % 4) * C) = tok[t];
+        add_vector<T>(acc, tok[t]);                       // as stored: what the next block's router reads
+    }
+    if constexpr (STAT) region_records<T>(tok, W, C, act, rec, eps);
+}
+
 // The same pass over a region without the scatter (SCATTER = false below): the tokens are read, summed for the
 // router and, with STAT, their records written; nothing is stored to the tokens.
 template <typename T, bool STAT>
@@ -975,8 +1044,10 @@ constexpr int CHAIN_SPIN_LIMIT = 1 << 20;
 // rows (the first block of a model, which no scatter-back precedes); `in` then points, if anywhere, at `extra`
 // rows [extra, C] that are first copied into the extra-token rows of every sample of `out` (class / distillation
 // token plus their position embedding, the same for every sample).
-template <typename T, int GS, bool SUB, bool STAT = false, bool SCATTER = true, bool CHAIN = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CHAIN ? 4 : 1, CHAIN ? 4 : 8)))
+// HELD: a region's reads are all in flight at once and its tokens stay in registers (region_scatter_held), from which the
+// chained variant packs them.
+template <typename T, int GS, bool SUB, bool STAT = false, bool SCATTER = true, bool CHAIN = false, bool HELD = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HELD ? 1 : CHAIN ? 4 : 1, HELD ? 2 : CHAIN ? 4 : 8)))
 void decompress_route_kernel(
     const T *__restrict__ in, const T *__restrict__ sub, const int64_t *__restrict__ cur_indices,
     const int64_t *__restrict__ splits, const int64_t *__restrict__ offsets, const T *__restrict__ ref,
@@ -988,6 +1059,7 @@ void decompress_route_kernel(
 {
     static_assert(!STAT || (GS == WAVE && std::is_same<T, bf16_t>::value), "records: one wave per region, bf16 rows");
     static_assert(!CHAIN || (STAT && SCATTER), "the chained variant is the bf16 scatter-back with records");
+    static_assert(!HELD || SCATTER, "what is held are the tokens of the scatter-back");
     constexpr int VEC = Elem<T>::VEC;
     constexpr int R = 4;
     const int lane = threadIdx.x & (GS - 1);
@@ -1042,6 +1114,7 @@ void decompress_route_kernel(
     // STAT: the host sends rows of at most GS vectors, and every lane makes the one trip (lanes past the row idle
     // inside it, present for the sums over the wave)
     const int vend = STAT ? GS : nvec;
+    u32x4 tok[HELD ? 16 : 1];             // HELD: the region's tokens as stored
     u32x4 pooled = {0u, 0u, 0u, 0u};      // CHAIN: this lane's vector of the region's mean as the router rounds it
     for (int v0 = lane; v0 < vend; v0 += GS) {
         const bool act = !STAT || v0 < nvec;
@@ -1054,6 +1127,12 @@ void decompress_route_kernel(
         const T *subv = SUB ? sub + v * VEC : nullptr;
         u32x4 *rec = STAT ? records + ((int64_t)b * N + tok0) * 2 : nullptr;
         if constexpr (!SCATTER) region_read<T, STAT>(ref + off, W, C, acc, act, rec, eps);
+        else if constexpr (HELD) {
+            if (ps == 4) region_scatter_held<T, 4, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, tok, act, rec, eps);
+            else if (ps == 2)
+                region_scatter_held<T, 2, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, tok, act, rec, eps);
+            else region_scatter_held<T, 1, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, tok, act, rec, eps);
+        }
         else if (ps == 4) region_scatter<T, 4, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
         else if (ps == 2) region_scatter<T, 2, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
         else region_scatter<T, 1, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
@@ -1259,6 +1338,9 @@ void decompress_route_kernel(
             u32x4 lo, hi;
             row_record(pivot, sums[0], sums[1], C, chain.comp_eps, lo, hi);
             if (lane < 2) chain.comp_records[n0 * 2 + lane] = lane ? hi : lo;
+        } else if constexpr (HELD) {
+            pack_held<bf16_t>(tok, chain.comp + n0 * (int64_t)C + v * 8, chain.comp_records + n0 * 2, ps_n, C, chain.comp_eps,
+                              act);
         } else {
             pack_region<bf16_t, true>(xs + tok0 * C, chain.comp + n0 * (int64_t)C + v * 8,
                                       chain.comp_records + n0 * 2, ps_n, W, C, chain.comp_eps, act, lane);
@@ -1739,6 +1821,8 @@ static int decompress_router_launch(const void *in, const void *sub, const int64
     const int gs = group_size(C / (dtype == VTDGE_BF16 ? 8 : 4));
     dim3 grid((unsigned)ceil_div(regions, ROWS_PER_BLOCK * (WAVE / gs))), block(256);
     hipStream_t st = (hipStream_t)stream;
+    // at most a workgroup a compute unit: see region_scatter_held
+    const bool held = sub != nullptr && grid.x <= 256;
     if (out_records != nullptr) {
         VT_REQUIRE(dtype == VTDGE_BF16 && gs == WAVE && C / 8 <= WAVE, VTDGE_ERR_UNSUPPORTED,
                    "decompress_router: statistics records are written for bf16 rows of 264 to 512 channels (C=%d)", C);
@@ -1752,13 +1836,15 @@ static int decompress_router_launch(const void *in, const void *sub, const int64
                        (long long)regions, ROWS_PER_BLOCK, extra, WAVE);
             VT_REQUIRE(next_weight && next_splits && next_counts, VTDGE_ERR_ARG,
                        "decompress_router_compress: needs the next router, its splits and the count bytes");
-#define VT_CHAIN(SUBF)                                                                                               \
-    note_kernel(reinterpret_cast<const void *>(decompress_route_kernel<bf16_t, WAVE, SUBF, true, true, true>)),      \
-    decompress_route_kernel<bf16_t, WAVE, SUBF, true, true, true><<<grid, block, 0, st>>>(                           \
+#define VT_CHAIN(SUBF, HELDF)                                                                                        \
+    note_kernel(reinterpret_cast<const void *>(decompress_route_kernel<bf16_t, WAVE, SUBF, true, true, true, HELDF>)), \
+    decompress_route_kernel<bf16_t, WAVE, SUBF, true, true, true, HELDF><<<grid, block, 0, st>>>(                    \
         (const bf16_t *)in, (const bf16_t *)sub, cur_indices, splits, offsets, (const bf16_t *)ref, (bf16_t *)out,   \
         (const bf16_t *)next_weight, (const bf16_t *)next_bias, (bf16_t *)next_gate, next_indices, B, H, W, C, extra, \
         S, S2, (u32x4 *)out_records, records_eps, next_splits, next_counts, region_rows, cur_counts, *chain)
-            if (sub) VT_CHAIN(true); else VT_CHAIN(false);
+            if (held) VT_CHAIN(true, true);
+            else if (sub) VT_CHAIN(true, false);
+            else VT_CHAIN(false, false);
 #undef VT_CHAIN
             return check_launch("decompress_router_compress");
         }
@@ -1772,13 +1858,18 @@ static int decompress_router_launch(const void *in, const void *sub, const int64
 #undef VT_STAT
         return check_launch("decompress_router");
     }
-#define VT_LAUNCH2(T, GS, SUBF)                                                                                    \
-    note_kernel(reinterpret_cast<const void *>(decompress_route_kernel<T, GS, SUBF>)),                             \
-    decompress_route_kernel<T, GS, SUBF><<<grid, block, 0, st>>>(                                                  \
+#define VT_LAUNCH2(T, GS, SUBF, HELDF)                                                                             \
+    note_kernel(reinterpret_cast<const void *>(decompress_route_kernel<T, GS, SUBF, false, true, false, HELDF>)),  \
+    decompress_route_kernel<T, GS, SUBF, false, true, false, HELDF><<<grid, block, 0, st>>>(                       \
         (const T *)in, (const T *)sub, cur_indices, splits, offsets, (const T *)ref, (T *)out,                     \
         (const T *)next_weight, (const T *)next_bias, (T *)next_gate, next_indices, B, H, W, C, extra, S, S2,      \
         nullptr, 0.f, next_splits, next_counts, region_rows, cur_counts)
-#define VT_LAUNCH(T, GS) do { if (sub) VT_LAUNCH2(T, GS, true); else VT_LAUNCH2(T, GS, false); } while (0)
+#define VT_LAUNCH(T, GS)                             \
+    do {                                             \
+        if (held) VT_LAUNCH2(T, GS, true, true);     \
+        else if (sub) VT_LAUNCH2(T, GS, true, false); \
+        else VT_LAUNCH2(T, GS, false, false);        \
+    } while (0)
 #define VT_GROUP(T) \
     do { if (gs == 64) VT_LAUNCH(T, 64); else if (gs == 32) VT_LAUNCH(T, 32); else if (gs == 16) VT_LAUNCH(T, 16); \
          else VT_LAUNCH(T, 8); } while (0)

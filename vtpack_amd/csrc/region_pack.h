@@ -146,4 +146,46 @@ __device__ __forceinline__ void pack_region(const T *xp, T *cp, u32x4 *rec, int 
     }
 }
 
+// pack_region for a region of 4 or 16 queries whose tokens the wave holds in registers; the same sums in the same order.
+template <typename T>
+__device__ __forceinline__ void pack_held(const u32x4 (&tok)[16], T *cp, u32x4 *rec, int ps, int C, float eps, bool act)
+{
+    constexpr int VEC = Elem<T>::VEC;
+    float acc[VEC];
+    if (ps == 4) {
+#pragma unroll
+        for (int dy = 0; dy < 4; dy++) {
+            float pivot[4], st[8];
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+#pragma unroll
+                for (int c = 0; c < VEC; c++) acc[c] = 0.f;
+                add_vector<T>(acc, tok[4 * dy + t]);
+                const u32x4 packed = Elem<T>::pack(acc);
+                if (act) *reinterpret_cast<u32x4 *>(cp + (int64_t)(4 * dy + t) * C) = packed;
+                lane_sums<T>(packed, act, pivot[t], st[2 * t], st[2 * t + 1]);
+            }
+            write_records4(st, pivot[0], pivot[1], pivot[2], pivot[3], C, eps, rec + 4 * dy * 2);
+        }
+        return;
+    }
+    float pivot[4], st[8];
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const int t0 = (w / 2) * 8 + (w % 2) * 2;
+#pragma unroll
+        for (int c = 0; c < VEC; c++) acc[c] = 0.f;
+        add_vector<T>(acc, tok[t0]);
+        add_vector<T>(acc, tok[t0 + 1]);
+        add_vector<T>(acc, tok[t0 + 4]);
+        add_vector<T>(acc, tok[t0 + 5]);
+#pragma unroll
+        for (int c = 0; c < VEC; c++) acc[c] *= 0.25f;
+        const u32x4 packed = Elem<T>::pack(acc);
+        if (act) *reinterpret_cast<u32x4 *>(cp + (int64_t)w * C) = packed;
+        lane_sums<T>(packed, act, pivot[w], st[2 * w], st[2 * w + 1]);
+    }
+    write_records4(st, pivot[0], pivot[1], pivot[2], pivot[3], C, eps, rec);
+}
+
 }  // namespace vtdge
