@@ -162,14 +162,17 @@ __global__ __launch_bounds__((WGM * WGN + NWP) * 64) void linear_dma_kernel(
     constexpr int EPL = 16 / ESZ;          // output elements per lane and store
     constexpr int NQ = 32 / (2 * EPL);     // stores per 32x32 block and lane: bf16 2 (8 columns each), fp32 4
     u32x4 braw[JN][NQ], rraw[IM][JN][NQ];  // bias / residual vectors of the tile, fetched during its last stage
-    int kt = 0, tk = 0;
+    int kt = 0, tk = 0, slot = 0;
+    int64_t m0 = 0;
+    int n0 = 0;
     for (int g = 0; g < G; g++) {
         const bool last = kt == nk - 1;
         block_barrier();
-        // output coordinates of the tile being accumulated
-        const int u = wg + tk * nwg;
-        const int64_t m0 = (int64_t)((u / tiles_n) * 8 + xcd) * BM;
-        const int n0 = (u % tiles_n) * BN;
+        if (last) {                                   // output coordinates of the tile being accumulated
+            const int u = wg + tk * nwg;
+            m0 = (int64_t)((u / tiles_n) * 8 + xcd) * BM;
+            n0 = (u % tiles_n) * BN;
+        }
         if (last && !LATE) {
             // issue the epilogue's reads now; they return while the last stage is multiplied
 #pragma unroll
@@ -191,18 +194,30 @@ __global__ __launch_bounds__((WGM * WGN + NWP) * 64) void linear_dma_kernel(
                     }
                 }
         }
-        const unsigned char *st = smem + (g % NSTAGE) * STAGE;
+        const unsigned char *st = smem + slot * STAGE;
+        slot = slot + 1 == NSTAGE ? 0 : slot + 1;
+        // the fragments of step s + 1 are requested before the products of step s are issued (left to itself the compiler
+        // keeps one set of registers and waits for LDS in every step)
+        u32x4 fa[2][IM], fw[2][JN];
+        auto fetch = [&](int s) {
+#pragma unroll
+            for (int i = 0; i < IM; i++)
+                fa[s & 1][i] = *reinterpret_cast<const u32x4 *>(st + a_row + i * 32 * DKB + cs[s]);
+#pragma unroll
+            for (int j = 0; j < JN; j++)
+                fw[s & 1][j] = *reinterpret_cast<const u32x4 *>(st + w_row + j * 32 * DKB + cs[s]);
+        };
+        fetch(0);
 #pragma unroll
         for (int s = 0; s < 4; s++) {
-            u32x4 fa[IM], fw[JN];
-#pragma unroll
-            for (int i = 0; i < IM; i++) fa[i] = *reinterpret_cast<const u32x4 *>(st + a_row + i * 32 * DKB + cs[s]);
-#pragma unroll
-            for (int j = 0; j < JN; j++) fw[j] = *reinterpret_cast<const u32x4 *>(st + w_row + j * 32 * DKB + cs[s]);
+            if (s < 3) fetch(s + 1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < IM; i++)
 #pragma unroll
-                for (int j = 0; j < JN; j++) Slab<T>::mma(fw[j], fa[i], acc[i][j]);   // D = W_blk * A_blk^T
+                for (int j = 0; j < JN; j++)
+                    Slab<T>::mma(fw[s & 1][j], fa[s & 1][i], acc[i][j]);      // D = W_blk * A_blk^T
+            __builtin_amdgcn_sched_barrier(0);
         }
         if (++kt < nk) continue;
         kt = 0;
@@ -275,11 +290,13 @@ struct LinArgs {
     void *out; int64_t ldo; const int64_t *rows_dev; int64_t rows; int N; int K; int act; hipStream_t st;
 };
 
-template <typename T, int BM, int BN, int WGM, int WGN, int NWP, int ACT, bool HB, bool HR, bool PATCH = false>
+constexpr int deepest_ring(int rows) { return (size_t)3 * rows * DKB <= 160 * 1024 ? 3 : 2; }
+
+template <typename T, int BM, int BN, int WGM, int WGN, int NWP, int ACT, bool HB, bool HR, bool PATCH = false,
+          int NSTAGE = deepest_ring(BM + BN)>
 static int go(const LinArgs &a, const PatchGeom &pg = PatchGeom{0, 0, 0, 0, 0, 0, 0, 0})
 {
     constexpr int NW = WGM * WGN + NWP;
-    constexpr int NSTAGE = (size_t)3 * (BM + BN) * DKB <= 160 * 1024 ? 3 : 2;
     constexpr bool LATE = (BM / WGM) * (BN / WGN) > 64 * 64;      // wave tiles beyond 64 x 64
     constexpr size_t lds = (size_t)NSTAGE * (BM + BN) * DKB;
     static_assert(lds <= 160 * 1024, "LDS budget");
@@ -297,6 +314,15 @@ static int go(const LinArgs &a, const PatchGeom &pg = PatchGeom{0, 0, 0, 0, 0, 0
     return check_launch("linear");
 }
 
+template <typename T, int BM, int BN, int WGM, int WGN, int NWP, int NSTAGE = deepest_ring(BM + BN)>
+static int pick_plain_epilogue(const LinArgs &a)          // without a residual
+{
+    if (a.act == VTDGE_ACT_GELU)
+        return a.bias ? go<T, BM, BN, WGM, WGN, NWP, VTDGE_ACT_GELU, true, false, false, NSTAGE>(a)
+                      : go<T, BM, BN, WGM, WGN, NWP, VTDGE_ACT_GELU, false, false, false, NSTAGE>(a);
+    return a.bias ? go<T, BM, BN, WGM, WGN, NWP, VTDGE_ACT_NONE, true, false, false, NSTAGE>(a)
+                  : go<T, BM, BN, WGM, WGN, NWP, VTDGE_ACT_NONE, false, false, false, NSTAGE>(a);
+}
 template <typename T, int BM, int BN, int WGM, int WGN, int NWP>
 static int pick_epilogue(const LinArgs &a)
 {
@@ -328,9 +354,6 @@ int launch_linear_dma(const void *A, int64_t lda, const void *W, const void *bia
                       hipStream_t st)
 {
     LinArgs a{A, lda, W, bias, res, ldr, out, ldo, rows_dev, rows, N, K, act, st};
-    // wide outputs: 256x128 tiles on 8 MFMA waves; narrow ones (N <= 512), and matrices that have fewer large tiles
-    // than the chip has compute units (a classifier on 256 rows): 128x128 on 4, for more tiles.  Other shapes of the
-    // same template (2 loader waves, 128x256 and 128x384 tiles on a two-stage ring) measured no faster.
     // fp32: an instruction of 4096 flops takes 64 clocks, so the operand traffic of small tiles is hidden and what counts
     // is how evenly they fill the chip: 64x64 tiles on four 32x32 waves, three workgroups a compute unit.  Measured
     // against the two shapes below (rows, N, K): 32896, 384, 192: 62 against 70 us; 14300, 768, 192 + GELU: 54.5 against
@@ -338,8 +361,23 @@ int launch_linear_dma(const void *A, int64_t lda, const void *W, const void *bia
     // 256x128 tiles a compute unit on the larger tile wins: 65536, 1536, 384: 641 against 688 us.
     if constexpr (sizeof(T) == 4)
         if (ceil_div(rows, 256) * ceil_div(N, 128) < 2048) return pick_epilogue<T, 64, 64, 2, 2, 4>(a);
-    if (N >= 768 && ceil_div(rows, 256) * ceil_div(N, 128) >= 256) return pick_epilogue<T, 256, 128, 4, 2, 4>(a);
-    return pick_epilogue<T, 128, 128, 2, 2, 4>(a);
+    if constexpr (sizeof(T) == 4) return pick_epilogue<T, 256, 128, 4, 2, 4>(a);
+    else {
+        // bf16.  Wide outputs: 128x256 tiles on eight MFMA waves, one workgroup a compute unit.  Otherwise 128x128 tiles on
+        // four: with a two-stage ring two workgroups a compute unit run out of step, which pays where tiles are short; long
+        // ones (and those that also fetch a residual) do better with a third stage.  Measured (rows, N, K; the 256x128 tiles
+        // that served N >= 768 before / 128x256 / 128x128 two stages / three stages, us): 25443, 1536, 768: 75 / 64 / 75 / 82;
+        // 11000, 3072, 768 + GELU: 71 / 69 / 67 / 83; 11000, 768, 768: 28 / 28 / 25 / 25; 28000, 1280, 320 + GELU: 44 / 42 /
+        // 38 / 48; 16640, 1024, 512: 31 / 30 / 27 / 30; 459000, 64, 64: 24 / 37 / 21 / 26; with a residual 11000, 768, 3072:
+        // 91 / 90 / 111 / 79; 14000, 768, 768: 33 / 33 / 34 / 29; 28000, 320, 1280: 45 / 44 / 52 / 39.
+        // (64-byte stages in deeper rings, 64x128 and 128x64 tiles and K started at another slab per tile: no faster.)
+        // Fewer tiles than two a compute unit are dealt with the deeper ring (1285 rows of 768 channels, a whole model: 1185
+        // against 1206 us with the shorter one, 1284 on 128x256).
+        const int64_t tiles = ceil_div(rows, 128) * ceil_div(N, 128);
+        if (res != nullptr || K >= 2048 || tiles < 512) return pick_epilogue<T, 128, 128, 2, 2, 4>(a);
+        if (N >= 1536) return pick_plain_epilogue<T, 128, 256, 2, 4, 4>(a);
+        return pick_plain_epilogue<T, 128, 128, 2, 2, 4, 2>(a);
+    }
 }
 
 // few rows (linear_small.hip)
@@ -373,7 +411,6 @@ int launch_patch_embed(const void *images, const void *W, const void *bias, cons
     // Eight loader waves instead of four (they also work out the patch addresses): 77.5 against 83.5 us; with two,
     // 201 us.  64x128 tiles: 108 us, 256x128 with eight loaders: 98 us.
     if constexpr (sizeof(T) == 4) return go<T, 64, 64, 2, 2, 8, VTDGE_ACT_NONE, true, true, true>(a, pg);
-    if (N >= 768) return go<T, 256, 128, 4, 2, 4, VTDGE_ACT_NONE, true, true, true>(a, pg);
     return go<T, 128, 128, 2, 2, 8, VTDGE_ACT_NONE, true, true, true>(a, pg);
 }
 
