@@ -246,3 +246,15 @@ def test_fused_forward_refuses_a_distillation_token_without_a_class_token():
         engine.model_forward(m, img)
     with pytest.raises(ValueError, match="class token"):
         m.embed_tokens(img)
+
+
+def test_parameters_made_in_inference_mode_have_no_chain_plan():
+    """Such parameters carry no version to check a plan against: their blocks are composed one by one."""
+    from vtpack_amd import engine
+    from vtpack_amd.models.dge.deit_dge import VisionTransformer
+    args = dict(img_size=64, patch_size=16, embed_dim=64, depth=2, num_heads=1, qkv_bias=True, split_sizes=[4, 2, 1])
+    blocks = list(VisionTransformer(**args).eval().blocks)
+    assert engine._chain_plan(blocks, torch.float32, torch.device("cpu"), 64, 1) is not None
+    with torch.inference_mode():
+        blocks = list(VisionTransformer(**args).eval().blocks)
+        assert engine._chain_plan(blocks, torch.float32, torch.device("cpu"), 64, 1) is None

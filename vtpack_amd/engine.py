@@ -540,7 +540,7 @@ def _chain_plan(blocks, dtype, device, channels, extra):
         flat = [t for ts in tensors for t in ts if t is not None]
         key = (*(list(map(f, flat)) for f in _TENSOR_STATE), [t is None for ts in tensors for t in ts], dtype, device, extra,
                channels, [_block_numbers(blk) for blk in blocks], ops._pack_epoch, ops._plan_epoch)
-    except (KeyError, AttributeError):
+    except (KeyError, AttributeError, RuntimeError):    # RuntimeError: parameters made in inference mode have no version
         return None
     plan = getattr(blocks[0], "_vtdge_chain", None)
     if plan is None or plan.key != key:
