@@ -431,12 +431,24 @@ int launch_patch_linear(const void *tokens, const void *W, const void *bias, voi
     const PatchGeom pg{P, 0, 1, 0, 0, C, H, Wd};
     const int64_t rows = (int64_t)B * (H / P) * (Wd / P);
     LinArgs a{tokens, 0, W, bias, nullptr, 0, out, N, nullptr, rows, N, P * P * C, VTDGE_ACT_NONE, st};
-    if (patch_small_wanted(rows, N, a.K, sizeof(T), (int64_t)B * H * Wd * C * sizeof(T)))
+    const bool few = sizeof(T) == 4 || ceil_div(rows, 32) * ceil_div(N, 32) <= 512;
+    if (few && patch_small_wanted(rows, N, a.K, sizeof(T), (int64_t)B * H * Wd * C * sizeof(T)))
         return launch_patch_small<T>(tokens, W, bias, nullptr, out, rows, N, a.K, pg, st);
     if constexpr (sizeof(T) == 4) return go<T, 64, 64, 2, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
-    if (N >= 768 || ceil_div(rows, 256) * ceil_div(N, 128) >= 512)
-        return go<T, 256, 128, 4, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
-    return go<T, 128, 128, 2, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
+    else {
+        // bf16.  Narrow outputs and much to read: 128x64 tiles, two workgroups a compute unit (of 73 KB each) whose waits for
+        // tokens fill each other; 64x64 where even those leave half the chip idle; 128x128 where they come out even and are
+        // still two a compute unit.  Measured (rows, N, K; 256x128, which served wide outputs and many tiles before /
+        // 128x128 / 128x64 / 64x64 / few rows' kernel, us): 262144, 128, 256: 87 / 51 / 52 / 59; 65536, 320, 512: 84 / 49 /
+        // 47 / 55; 16384, 512, 1280: 52 / 32 / 34 / 39; 16384, 320, 1280: 46 / 30 / 25 / 26 / 70; 16384, 128, 2048: 78 / 26 /
+        // 23 / 23 / 42; 16384, 64, 4096: 142 / 47 / 43 / 37 / 44; 4096, 320, 1280: 44 / 17 / 13 / 15 / 21; 4096, 128, 2048:
+        // 61 / 23 / 17 / 14 / 12; 4096, 64, 4096: 112 / 40 / 28 / 23 / 12; 1024, 512, 1280: 43 / 17 / 13 / 10.5 / 10.4.
+        // PVT-Small at 256 pictures, a whole pass: 5183 -> 5060 us.
+        const int64_t tiles = ceil_div(rows, 128) * ceil_div(N, 64);
+        if (tiles <= 128) return go<T, 64, 64, 2, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
+        if (N % 128 == 0 && tiles >= 1024) return go<T, 128, 128, 2, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
+        return go<T, 128, 64, 2, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
+    }
 }
 
 template int launch_patch_linear<float>(const void *, const void *, const void *, void *, int, int, int, int, int, int,
