@@ -409,10 +409,10 @@ int vtdge_batched_sparse_gemm(const void *a, const void *b, const int64_t *a_off
                               int trans_b, int64_t out_rows, int64_t out_cols, int64_t max_m, int dtype,
                               void *stream);
 
-/* Gradients of vtdge_sparse_attention: dq, dk, dv from its operands, its output and the output's gradient, as autograd
+/* Gradients of vtdge_sparse_attention: dq, dk, dv from its operands and the output's gradient, as autograd
  * through the reference's training composition would give them (two batched products around a softmax,
- * vtpack/models/dge/deit_dge.py:86-95), without score-sized tensors.  Strides as in vtdge_sparse_attention; `out` and
- * `dout` share theirs.  workspace: 2 * h * L floats, L = offsets[B] = rows of q.  Gradients of keys and values of a sample
+ * vtpack/models/dge/deit_dge.py:86-95), without score-sized tensors.  Strides as in vtdge_sparse_attention, those of
+ * `dout` under o_*.  `out` is not read and may be NULL.  workspace: 2 * h * L floats, L = offsets[B] = rows of q.  Gradients of keys and values of a sample
  * without queries are zero.  Head dim 64. */
 int vtdge_sparse_attention_backward(const void *q, int64_t q_row_stride, int64_t q_head_stride, const void *k, const void *v,
                                     int64_t kv_batch_stride, int64_t kv_tok_stride, int64_t kv_head_stride, const void *out,

@@ -49,6 +49,26 @@ def test_against_float64(dev, dtype, n, lengths, scale, dense):
         *args, torch.tensor(lengths), scale), args, g.to(dev))))                      # the same bytes on every call
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("common", [1.0, 2.0])
+def test_keys_and_values_with_a_common_component(dev, dtype, common):
+    """What a kv bias gives: every key and every value shifted by the same vector.  A row of dS adds up to zero, so the
+    gradients do not see the shift; an error in delta would reach dQ times the mean key.  bf16: dS is rounded once, 2^-9 at
+    most and 2^-9 / sqrt(3) rms, and multiplies keys sqrt(1 + common^2) times as large as what remains of them: 2.5e-3 of
+    dQ at common = 2; bound: four times that."""
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    h, n, lengths = 3, 257, [113, 17, 64]
+    L, B = sum(lengths), len(lengths)
+    q, g = (torch.from_numpy(randn(s, L, h * 64)).to(dtype) for s in (1, 4))
+    q = q.view(L, h, 64).transpose(0, 1)
+    k, v = (torch.from_numpy(randn(s, h, B, n, 64) + common * randn(s + 7, h, 1, 1, 64)).to(dtype) for s in (2, 3))
+    want, grads = _reference(q, k, v, lengths, 0.125, g)
+    args = [t.to(dev).requires_grad_(True) for t in (q, k, v)]
+    got = sparse_attention_train(*args, torch.tensor(lengths), 0.125)
+    for name, a, b in zip("qkv", torch.autograd.grad(got, args, g.to(dev)), grads):
+        assert float((a.double().cpu() - b).norm()) <= (1e-5 if dtype == torch.float32 else 1e-2) * float(b.norm()), name
+
+
 @pytest.mark.parametrize("which", ["q", "k", "v", "grad", "hook"])
 def test_operands_off_a_16_byte_boundary(dev, which):
     """Operands that start 4 bytes behind a boundary, and saved tensors that come back from a hook that way."""

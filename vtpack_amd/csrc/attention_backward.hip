@@ -1,13 +1,16 @@
-// Gradients of the sparse attention of packed queries (gfx950): dQ, dK, dV from Q, K, V, the output and its gradient.
+// Gradients of the sparse attention of packed queries (gfx950): dQ, dK, dV from Q, K, V and the output's gradient.
 //
 // The composition this stands in for (a product of queries and keys, a softmax, a product with the values, and their
 // five products backward: vtpack/models/dge/deit_dge.py:86-95) keeps four score-sized tensors in HBM, [heads, L, n] each:
 // 90 MB apiece at 14500 queries, 6 heads and 257 keys in bf16, against 45 MB of operands.  Here scores exist in registers
 // only: they are worked out again from Q and K where a gradient needs them,
-//   P = exp2(scale log2e q.k - lse),   dP = dO.v,   dS = P (dP - delta) scale,   delta = sum_d dO O,
+//   P = exp2(scale log2e q.k - lse),   dP = dO.v,   dS = P (dP - delta) scale,   delta = sum_k P dP,
 //   dQ = dS K,   dV = P^T dO,   dK = dS^T Q.
 // Two kernels, no atomics, so the result is the same bytes on every call: one over query tiles, which first finds lse (the
 // row's maximum plus the log of its sum, in log2 units) and delta and leaves both for the other, over key tiles.
+// delta equals dO.O, but is summed from the P and dP that dS is made of: a row of dS then adds up to zero within fp32, where
+// dO times an output rounded to bf16 leaves a remainder that multiplies the mean key (relative error of dQ with a common
+// component of twice the spread in keys and values: 5.1e-2 from the rounded output, 3.6e-3 this way).
 //
 // Both are one scheme.  A wave keeps 16 rows of two operands in registers (Q and dO, or K and V) and walks the rows of
 // the other two, which the workgroup's four waves share through LDS in stages of 32 by direct loads (two buffers).  With
@@ -65,15 +68,6 @@ template <> struct BackMath<float> {
                     out[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[db], p[blk][r], out[db], 0, 0, 0);
             }
     }
-    static __device__ __forceinline__ float dot(const Frag (&a)[4], const Frag (&b)[4])
-    {
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) s += a[j][e] * b[j][e];
-        return s;
-    }
     // out[db][r] is channel 16 g + 4 r + db of kept row l
     static __device__ __forceinline__ void store(float *row, const f32x4 (&o)[4], int g)
     {
@@ -116,19 +110,6 @@ template <> struct BackMath<bf16_t> {
             out[db] = mma(u32x4{lo.x, lo.y, hi.x, hi.y}, b, out[db]);
         }
     }
-    static __device__ __forceinline__ float dot(const Frag (&a)[2], const Frag (&b)[2])
-    {
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            float x[8], y[8];
-            Elem<bf16_t>::unpack(a[j], x);
-            Elem<bf16_t>::unpack(b[j], y);
-#pragma unroll
-            for (int e = 0; e < 8; e++) s += x[e] * y[e];
-        }
-        return s;
-    }
     // out[db][r] is channel 16 db + 4 g + r of kept row l
     static __device__ __forceinline__ void store(bf16_t *row, const f32x4 (&o)[4], int g)
     {
@@ -143,12 +124,12 @@ template <> struct BackMath<bf16_t> {
 };
 
 struct AttnBack {
-    const void *q, *k, *v, *out, *dout;
+    const void *q, *k, *v, *dout;
     void *dq, *dk, *dv;
     float *lse, *delta;                                   // [h, L] each
     const int64_t *offsets;
     int64_t q_rs, q_hs, kv_bs, kv_ts, kv_hs, o_rs, o_hs, dq_rs, dq_hs, dkv_bs, dkv_ts, dkv_hs, L;
-    int pairs, h, n, chunks;
+    int pairs, h, n;
     float scale, scale_log2;
 };
 
@@ -207,55 +188,60 @@ template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_ker
     const Stager<T> kv{reinterpret_cast<const unsigned char *>((const T *)(wid < 2 ? a.k : a.v) + kv_at),
                        (uint32_t)(a.kv_ts * sizeof(T)), (uint32_t)(uintptr_t)smem, a.n, wid, lane};
     const int stages = (a.n + AB_ROWS - 1) / AB_ROWS;
-    if (wid < 2) kv.load(0);
+    kv.load(0);
 
     typename M::Frag qf[B::NF], df[B::NF];
-    float delta;
-    {
-        typename M::Frag of[B::NF];
-        const int64_t o_at = (row0 + row) * a.o_rs + (int64_t)head * a.o_hs;
-        load_kept<T>(qf, (const T *)a.q + (row0 + row) * a.q_rs + (int64_t)head * a.q_hs, live, g);
-        load_kept<T>(df, (const T *)a.dout + o_at, live, g);
-        load_kept<T>(of, (const T *)a.out + o_at, live, g);
-        delta = M::dot(df, of);
-        delta += __shfl_xor(delta, 16, WAVE);
-        delta += __shfl_xor(delta, 32, WAVE);
-    }
-    // ---- lse of this lane's query: maximum and sum over the lane's keys, then over the four lanes that share the query
-    float m = -INFINITY, s = 0.f;
+    load_kept<T>(qf, (const T *)a.q + (row0 + row) * a.q_rs + (int64_t)head * a.q_hs, live, g);
+    load_kept<T>(df, (const T *)a.dout + (row0 + row) * a.o_rs + (int64_t)head * a.o_hs, live, g);
+    // ---- lse and delta of this lane's query: maximum, sum of e and sum of e dP over the lane's keys, then over the four
+    // lanes that share the query
+    float m = -INFINITY, s = 0.f, sd = 0.f;
     for (int st = 0; st < stages; st++) {
         wait_vmcnt<0>();
         block_barrier();
-        if (wid < 2 && st + 1 < stages) kv.load(st + 1);
+        if (st + 1 < stages) kv.load(st + 1);
         if (!wave_live) continue;
-        const unsigned char *S = smem + (st & 1) * 2 * B::HALF;
-        f32x4 t[2];
+        const unsigned char *Ks = smem + (st & 1) * 2 * B::HALF, *Vs = Ks + B::HALF;
+        f32x4 t[2], dp[2];
         float mx = m;
 #pragma unroll
         for (int blk = 0; blk < 2; blk++) {
-            t[blk] = M::scores(S, blk, qf, l, g);
+            t[blk] = M::scores(Ks, blk, qf, l, g);
+            dp[blk] = M::scores(Vs, blk, df, l, g);
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const bool in = st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
                 t[blk][r] = in ? t[blk][r] * a.scale_log2 : -INFINITY;
+                dp[blk][r] = in ? dp[blk][r] : 0.f;
                 mx = fmaxf(mx, t[blk][r]);
             }
         }
         if (mx > -INFINITY) {
-            s *= __builtin_amdgcn_exp2f(m - mx);
+            const float down = __builtin_amdgcn_exp2f(m - mx);
+            s *= down;
+            sd *= down;
 #pragma unroll
             for (int blk = 0; blk < 2; blk++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) s += __builtin_amdgcn_exp2f(t[blk][r] - mx);
+                for (int r = 0; r < 4; r++) {
+                    const float e = __builtin_amdgcn_exp2f(t[blk][r] - mx);
+                    s += e;
+                    sd += e * dp[blk][r];
+                }
             m = mx;
         }
     }
     float all = fmaxf(m, __shfl_xor(m, 16, WAVE));
     all = fmaxf(all, __shfl_xor(all, 32, WAVE));
-    s *= __builtin_amdgcn_exp2f(m - all);                 // a lane without keys: exp2(-inf) = 0 times 0
+    const float down = __builtin_amdgcn_exp2f(m - all);   // a lane without keys: exp2(-inf) = 0 times 0
+    s *= down;
+    sd *= down;
     s += __shfl_xor(s, 16, WAVE);
+    sd += __shfl_xor(sd, 16, WAVE);
     s += __shfl_xor(s, 32, WAVE);
+    sd += __shfl_xor(sd, 32, WAVE);
     const float lse = all + __builtin_amdgcn_logf(s);     // v_log_f32: base 2
+    const float delta = sd / s;
     if (live && g == 0) {
         a.lse[(int64_t)head * a.L + row0 + row] = lse;
         a.delta[(int64_t)head * a.L + row0 + row] = delta;
@@ -441,7 +427,7 @@ extern "C" int vtdge_sparse_attention_backward(
     void *dv, int64_t dkv_batch_stride, int64_t dkv_tok_stride, int64_t dkv_head_stride, float *workspace, int64_t L, int B,
     int h, int d, int n, int max_rows_per_sample, float scale, int dtype, void *stream)
 {
-    VT_REQUIRE(k && v && offsets && dk && dv && (L == 0 || (q && out && dout && dq && workspace)), VTDGE_ERR_ARG,
+    VT_REQUIRE(k && v && offsets && dk && dv && (L == 0 || (q && dout && dq && workspace)), VTDGE_ERR_ARG,
                "sparse_attention_backward: NULL operand");
     VT_REQUIRE(dtype == VTDGE_F32 || dtype == VTDGE_BF16, VTDGE_ERR_ARG, "sparse_attention_backward: unknown dtype %d", dtype);
     VT_REQUIRE(B > 0 && h > 0 && n > 0 && L >= 0 && max_rows_per_sample >= 0 && (int64_t)B * h < (1ll << 28), VTDGE_ERR_ARG,
@@ -455,12 +441,12 @@ extern "C" int vtdge_sparse_attention_backward(
                    "sparse_attention_backward: strides must keep 16-byte alignment");
     VT_REQUIRE(q_row_stride < (1 << 23) && kv_tok_stride < (1 << 23) && o_row_stride < (1 << 23), VTDGE_ERR_UNSUPPORTED,
                "sparse_attention_backward: row stride too large");
-    VT_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out | (uintptr_t)dout | (uintptr_t)dq | (uintptr_t)dk |
-                 (uintptr_t)dv) & 15) == 0,
+    VT_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)dout | (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) &
+                15) == 0,
                VTDGE_ERR_ARG, "sparse_attention_backward: operands must be 16-byte aligned");
-    AttnBack a{q, k, v, out, dout, dq, dk, dv, workspace, workspace + (int64_t)h * L, offsets, q_row_stride, q_head_stride,
+    AttnBack a{q, k, v, dout, dq, dk, dv, workspace, workspace + (int64_t)h * L, offsets, q_row_stride, q_head_stride,
                kv_batch_stride, kv_tok_stride, kv_head_stride, o_row_stride, o_head_stride, dq_row_stride, dq_head_stride,
-               dkv_batch_stride, dkv_tok_stride, dkv_head_stride, L, B * h, h, n, 0, scale,
+               dkv_batch_stride, dkv_tok_stride, dkv_head_stride, L, B * h, h, n, scale,
                scale * 1.44269504088896340736f};
     if (dtype == VTDGE_F32) return launch_backward<float>(a, max_rows_per_sample, (hipStream_t)stream);
     return launch_backward<bf16_t>(a, max_rows_per_sample, (hipStream_t)stream);

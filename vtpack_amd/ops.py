@@ -924,7 +924,7 @@ def sparse_attention_heads(q, k, v, offsets, scale, max_rows_per_sample, out=Non
 
 def sparse_attention_backward(q, k, v, out, grad, offsets, scale, max_rows_per_sample):
     """Gradients (dq, dk, dv) of `sparse_attention_heads` with head dim 64: q [h, L, d] with rows on 16-byte boundaries, k
-    and v [h, B, n, d] dense; out and grad [h, L, d] views with the same strides.  dq has q's strides order ([L, h, d] in
+    and v [h, B, n, d] dense; grad a [h, L, d] view, `out` is not read.  dq has q's strides order ([L, h, d] in
     memory), dk and dv are dense."""
     h, L, d = q.shape
     B, n = k.shape[1], k.shape[2]
@@ -932,7 +932,7 @@ def sparse_attention_backward(q, k, v, out, grad, offsets, scale, max_rows_per_s
     dk, dv = torch.empty_like(k), torch.empty_like(v)
     work = torch.empty((2 * h * L,), dtype=torch.float32, device=q.device)
     call("vtdge_sparse_attention_backward", ptr(q), q.stride(1), q.stride(0), ptr(k), ptr(v), k.stride(1), k.stride(2),
-         k.stride(0), ptr(out), ptr(grad), out.stride(1), out.stride(0), ptr(offsets), ptr(dq), dq.stride(1), dq.stride(0),
+         k.stride(0), 0, ptr(grad), grad.stride(1), grad.stride(0), ptr(offsets), ptr(dq), dq.stride(1), dq.stride(0),
          ptr(dk), ptr(dv), dk.stride(1), dk.stride(2), dk.stride(0), ptr(work), L, B, h, d, n, max_rows_per_sample,
          float(scale), dtype_code(q), stream_ptr(), tag=("attention_backward", B, h, d, n))
     return dq, dk, dv
