@@ -94,6 +94,20 @@ def test_operands_off_a_16_byte_boundary(dev, which):
         assert float((a.double().cpu() - b).abs().max()) <= 1e-5 * float(b.abs().max())
 
 
+def test_the_result_may_be_changed_in_place(dev):
+    """As the composition's could: the backward pass does not need it."""
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    lengths = [5, 17]
+    args = [torch.from_numpy(randn(i, *s)).to(dev).requires_grad_(True)
+            for i, s in enumerate([(2, 22, 64), (2, 2, 33, 64), (2, 2, 33, 64)])]
+    g = torch.from_numpy(randn(3, 22, 128)).to(dev)
+    want = torch.autograd.grad(sparse_attention_train(*args, torch.tensor(lengths), 0.125), args, g)
+    out = sparse_attention_train(*args, torch.tensor(lengths), 0.125)
+    out -= 1
+    out *= 1
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(out, args, g), want))
+
+
 @pytest.mark.parametrize("B", [1, 3, 447, 448, 449, 1000])
 def test_offsets_of_lengths(dev, B):
     from vtpack_amd import ops

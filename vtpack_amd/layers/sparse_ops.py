@@ -55,18 +55,18 @@ class _SparseAttentionTrain(Function):
         out = torch.empty((L, h * d), dtype=q.dtype, device=q.device)
         ctx.scale, ctx.max_rows = scale, int(lengths.max())
         ops.sparse_attention_heads(q, k, v, offsets, scale, ctx.max_rows, out=out.view(L, h, d).transpose(0, 1))
-        ctx.save_for_backward(q, k, v, out, offsets)
+        ctx.save_for_backward(q, k, v, offsets)      # not the result: a caller may change that in place
         return out
 
     @staticmethod
     @once_differentiable
     def backward(ctx, grad):
-        q, k, v, out, offsets = ctx.saved_tensors
+        q, k, v, offsets = ctx.saved_tensors
         h, L, d = q.shape
-        # out and the gradient share their strides in the kernel, k and v too; a saved-tensor hook may lay them out anew
-        q, k, v, out, grad = (ops.on_boundary(t) for t in (ops.vector_rows(q), *(t.contiguous() for t in (k, v, out, grad))))
-        heads = [t.view(L, h, d).transpose(0, 1) for t in (out, grad)]
-        dq, dk, dv = ops.sparse_attention_backward(q, k, v, *heads, offsets, ctx.scale, ctx.max_rows)
+        # k and v share their strides in the kernel; a saved-tensor hook may lay them out anew
+        q, k, v, grad = (ops.on_boundary(t) for t in (ops.vector_rows(q), *(t.contiguous() for t in (k, v, grad))))
+        grad = grad.view(L, h, d).transpose(0, 1)
+        dq, dk, dv = ops.sparse_attention_backward(q, k, v, None, grad, offsets, ctx.scale, ctx.max_rows)
         return dq, dk, dv, None, None
 
 
