@@ -409,6 +409,14 @@ int vtdge_batched_sparse_gemm(const void *a, const void *b, const int64_t *a_off
                               int trans_b, int64_t out_rows, int64_t out_cols, int64_t max_m, int dtype,
                               void *stream);
 
+/* vtdge_sparse_attention for training: bf16, head dim 64, scores of the queries as given (not rounded once more, times the
+ * scale) and of any value, -infinity among the first ones included; the probabilities are those that
+ * vtdge_sparse_attention_backward works out again. */
+int vtdge_sparse_attention_train(const void *q, int64_t q_row_stride, int64_t q_head_stride, const void *k, const void *v,
+                                 int64_t kv_batch_stride, int64_t kv_tok_stride, int64_t kv_head_stride,
+                                 const int64_t *offsets, void *out, int64_t o_row_stride, int64_t o_head_stride, int B, int h,
+                                 int d, int n, int max_rows_per_sample, float scale, int dtype, void *stream);
+
 /* Gradients of vtdge_sparse_attention: dq, dk, dv from its operands and the output's gradient, as autograd
  * through the reference's training composition would give them (two batched products around a softmax,
  * vtpack/models/dge/deit_dge.py:86-95), without score-sized tensors.  Strides as in vtdge_sparse_attention, those of

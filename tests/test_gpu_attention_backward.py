@@ -94,6 +94,40 @@ def test_operands_off_a_16_byte_boundary(dev, which):
         assert float((a.double().cpu() - b).abs().max()) <= 1e-5 * float(b.abs().max())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("first", [1, 32, 40])
+def test_first_scores_of_minus_infinity(dev, dtype, first):
+    """Keys whose scores overflow to -infinity have probability zero, also where they are the first of their sample."""
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    h, n, lengths = 2, 65, [5, 17]
+    L, B = sum(lengths), len(lengths)
+    q, k, v = (torch.from_numpy(randn(i, *s)) for i, s in enumerate([(h, L, 64), (h, B, n, 64), (h, B, n, 64)]))
+    q[..., 3], k[..., 3] = 1e20, 0
+    k[:, :, :first, 3] = -1e20                               # -1e40: past the range of fp32
+    q, k, v, g = (t.to(dtype) for t in (q, k, v, torch.from_numpy(randn(3, L, h * 64))))
+    want, grads = _reference(q, k, v, lengths, 0.125, g)
+    args = [t.to(dev).requires_grad_(True) for t in (q, k, v)]
+    got = sparse_attention_train(*args, torch.tensor(lengths), 0.125)
+    pairs = list(zip((got.detach(),) + torch.autograd.grad(got, args, g.to(dev)), (want,) + grads))
+    keep = [c for c in range(64) if c != 3]                  # (the gradient of the huge channel is as huge)
+    pairs[2] = tuple(t[..., keep] for t in pairs[2])
+    for a, b in pairs:
+        assert float((a.double().cpu() - b).abs().max()) <= TOL[dtype] * float(b.abs().max())
+
+
+def test_scores_are_those_of_the_queries_as_given(dev):
+    """Scores of spread 8 in bf16: a query rounded once more, times the scale, would be off by 2^-9 / sqrt(3) of its score,
+    i.e. 9e-3 of a probability.  What remains are the roundings of the probabilities and of the result, 1.1e-3 each."""
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    h, n, lengths = 3, 257, [113, 64]
+    L, B = sum(lengths), len(lengths)
+    q, k, v = (torch.from_numpy(randn(i, *s)).bfloat16()
+               for i, s in enumerate([(h, L, 64), (h, B, n, 64), (h, B, n, 64)]))
+    want, _ = _reference(q, k, v, lengths, 0.9, torch.ones(L, h * 64))
+    got = sparse_attention_train(*(t.to(dev) for t in (q, k, v)), torch.tensor(lengths), 0.9)
+    assert float((got.double().cpu() - want).norm()) <= 2.5 * 1.6e-3 * float(want.norm())
+
+
 def test_the_result_may_be_changed_in_place(dev):
     """As the composition's could: the backward pass does not need it."""
     from vtpack_amd.layers.sparse_ops import sparse_attention_train

@@ -62,6 +62,7 @@ SIGNATURES = {
                                     _i, _i, _i, _p],
     "vtdge_sparse_attention": [_p, _l, _l, _p, _p, _l, _l, _l, _p, _p, _l, _l, _i, _i, _i, _i, _i, _f, _i, _p],
     "vtdge_batched_sparse_gemm": [_p, _p, _p, _p, _p, _i, _i, _l, _i, _l, _i, _i, _i, _l, _l, _l, _i, _p],
+    "vtdge_sparse_attention_train": [_p, _l, _l, _p, _p, _l, _l, _l, _p, _p, _l, _l, _i, _i, _i, _i, _i, _f, _i, _p],
     "vtdge_sparse_attention_backward": [_p, _l, _l, _p, _p, _l, _l, _l, _p, _p, _l, _l, _p, _p, _l, _l, _p, _p, _l, _l, _l, _p,
                                         _l, _i, _i, _i, _i, _i, _f, _i, _p],
     "vtdge_lengths_to_offsets": [_p, _i, _p, _p],

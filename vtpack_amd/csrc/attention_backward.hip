@@ -92,14 +92,18 @@ template <> struct BackMath<bf16_t> {
                       x[j], acc);
         return acc;
     }
-    // contraction over the stage's 32 rows in the order (4 g .. 4 g + 3, 16 + 4 g .. 16 + 4 g + 3) of lane group g
+    static __device__ __forceinline__ u32x4 pack(const f32x4 (&p)[2])
+    {
+        return u32x4{pack_bf16x2(p[0][0], p[0][1]), pack_bf16x2(p[0][2], p[0][3]), pack_bf16x2(p[1][0], p[1][1]),
+                     pack_bf16x2(p[1][2], p[1][3])};
+    }
     static __device__ __forceinline__ void accumulate(const unsigned char *S, const f32x4 (&p)[2], f32x4 (&out)[4], int l, int g)
     {
-        u32x4 b;
-        b.x = pack_bf16x2(p[0][0], p[0][1]);
-        b.y = pack_bf16x2(p[0][2], p[0][3]);
-        b.z = pack_bf16x2(p[1][0], p[1][1]);
-        b.w = pack_bf16x2(p[1][2], p[1][3]);
+        accumulate(S, pack(p), out, l, g);
+    }
+    // contraction over the stage's 32 rows in the order (4 g .. 4 g + 3, 16 + 4 g .. 16 + 4 g + 3) of lane group g
+    static __device__ __forceinline__ void accumulate(const unsigned char *S, const u32x4 &b, f32x4 (&out)[4], int l, int g)
+    {
         // this lane as a source of the transposing reads: row 4 g + l / 4, channels 16 db + 4 (l % 4) .. + 3
         const int row = 4 * g + (l >> 2);
         const unsigned char *src = S + row * 128 + 8 * (l & 1);
@@ -121,6 +125,16 @@ template <> struct BackMath<bf16_t> {
             *reinterpret_cast<u32x2 *>(row + 16 * db + 4 * g) = w;
         }
     }
+};
+
+// the forward pass
+struct AttnTrain {
+    const bf16_t *q, *k, *v;
+    bf16_t *out;
+    const int64_t *offsets;
+    int64_t q_rs, q_hs, kv_bs, kv_ts, kv_hs, o_rs, o_hs;
+    int pairs, h, n;
+    float scale_log2;
 };
 
 struct AttnBack {
@@ -164,6 +178,83 @@ __device__ __forceinline__ void load_kept(typename BackMath<T>::Frag (&f)[BackTi
         if (live) z = *reinterpret_cast<const u32x4 *>(p + 64 * j);
         f[j] = __builtin_bit_cast(Frag, z);
     }
+}
+
+// The forward pass in bf16, from the same scores as the gradients: the inference kernels round the queries once more, times
+// the scale, and take their reference score from the first 32 keys, so that a row whose first scores are all -infinity comes
+// out as NaN.  Here a query's reference is its running maximum; until a finite score comes there is none and nothing is
+// added.  The row sum is taken of the probabilities as rounded for the product with the values.
+__global__ __launch_bounds__(256, 4) void attention_train_kernel(AttnTrain a)
+{
+    using B = BackTile<bf16_t>;
+    using M = BackMath<bf16_t>;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * B::HALF];
+    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8;
+    const int pair = (rest % pairs_x) * 8 + (blockIdx.x & 7), chunk = rest / pairs_x;
+    if (pair >= a.pairs) return;
+    const int b = pair / a.h, head = pair - b * a.h;
+    const int64_t row0 = a.offsets[b];
+    const int Lb = (int)(a.offsets[b + 1] - row0);
+    if (chunk * 16 * AB_WAVES >= Lb) return;
+    const int lane = threadIdx.x & 63, l = lane & 15, g = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int row = (chunk * AB_WAVES + wid) * 16 + l;
+    const bool live = row < Lb, wave_live = (chunk * AB_WAVES + wid) * 16 < Lb;
+
+    const int64_t kv_at = (int64_t)b * a.kv_bs + (int64_t)head * a.kv_hs;
+    const Stager<bf16_t> kv{reinterpret_cast<const unsigned char *>((wid < 2 ? a.k : a.v) + kv_at), (uint32_t)(a.kv_ts * 2),
+                            (uint32_t)(uintptr_t)smem, a.n, wid, lane};
+    const int stages = (a.n + AB_ROWS - 1) / AB_ROWS;
+    kv.load(0);
+    typename M::Frag qf[B::NF];
+    load_kept<bf16_t>(qf, a.q + (row0 + row) * a.q_rs + (int64_t)head * a.q_hs, live, g);
+    f32x4 o[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, s = 0.f;                         // of this lane's query; s of this lane's keys
+    for (int st = 0; st < stages; st++) {
+        wait_vmcnt<0>();
+        block_barrier();
+        if (st + 1 < stages) kv.load(st + 1);
+        unsigned char *Ks = smem + (st & 1) * 2 * B::HALF, *Vs = Ks + B::HALF;
+        const int left = a.n - st * AB_ROWS;
+        if (left < AB_ROWS) {                             // values past the last key: nothing of them, not even 0 * infinity
+            for (int i = left * B::CPR + threadIdx.x; i < AB_ROWS * B::CPR; i += 64 * AB_WAVES)
+                *reinterpret_cast<u32x4 *>(Vs + i * 16) = u32x4{0u, 0u, 0u, 0u};
+            lds_barrier();
+        }
+        if (!wave_live) continue;
+        f32x4 p[2];
+        float mx = m;
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            p[blk] = M::scores(Ks, blk, qf, l, g);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                p[blk][r] = 16 * blk + 4 * g + r < left ? p[blk][r] * a.scale_log2 : -INFINITY;
+                mx = fmaxf(mx, p[blk][r]);
+            }
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+        const float ref = mx == -INFINITY ? 0.f : mx, down = __builtin_amdgcn_exp2f(m - ref);
+        m = mx;
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) p[blk][r] = __builtin_amdgcn_exp2f(p[blk][r] - ref);
+        const u32x4 pb = M::pack(p);
+        s = bf16_pair_sum(pb.w, bf16_pair_sum(pb.z, bf16_pair_sum(pb.y, bf16_pair_sum(pb.x, s * down))));
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[i] *= down;
+        M::accumulate(Vs, pb, o, l, g);
+    }
+    s += __shfl_xor(s, 16, WAVE);
+    s += __shfl_xor(s, 32, WAVE);
+    const float inv = 1.0f / s;
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] *= inv;
+    if (live) M::store(a.out + (row0 + row) * a.o_rs + (int64_t)head * a.o_hs, o, g);
 }
 
 // dQ of 64 query rows of one (sample, head), with their lse and delta
@@ -418,6 +509,35 @@ extern "C" int vtdge_lengths_to_offsets(const int64_t *lengths_host, int B, int6
         start += sum;
     }
     return VTDGE_OK;
+}
+
+extern "C" int vtdge_sparse_attention_train(const void *q, int64_t q_row_stride, int64_t q_head_stride, const void *k,
+                                            const void *v, int64_t kv_batch_stride, int64_t kv_tok_stride,
+                                            int64_t kv_head_stride, const int64_t *offsets, void *out, int64_t o_row_stride,
+                                            int64_t o_head_stride, int B, int h, int d, int n, int max_rows_per_sample,
+                                            float scale, int dtype, void *stream)
+{
+    VT_REQUIRE(q && k && v && offsets && out, VTDGE_ERR_ARG, "sparse_attention_train: NULL operand");
+    VT_REQUIRE(B > 0 && h > 0 && n > 0 && max_rows_per_sample >= 0 && (int64_t)B * h < (1ll << 28), VTDGE_ERR_ARG,
+               "sparse_attention_train: bad sizes");
+    VT_REQUIRE(d == 64 && dtype == VTDGE_BF16, VTDGE_ERR_UNSUPPORTED,
+               "sparse_attention_train: head_dim %d, dtype %d (only 64 and bf16 are built)", d, dtype);
+    const int64_t strides[] = {q_row_stride, q_head_stride, kv_batch_stride, kv_tok_stride, kv_head_stride, o_row_stride,
+                               o_head_stride};
+    for (int64_t s : strides)
+        VT_REQUIRE(s >= 0 && s % 8 == 0, VTDGE_ERR_UNSUPPORTED, "sparse_attention_train: strides must keep 16-byte alignment");
+    VT_REQUIRE(kv_tok_stride < (1 << 23), VTDGE_ERR_UNSUPPORTED, "sparse_attention_train: row stride too large");
+    VT_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15) == 0, VTDGE_ERR_ARG,
+               "sparse_attention_train: operands must be 16-byte aligned");
+    const int64_t chunks = ceil_div(max_rows_per_sample, 16 * AB_WAVES), grid = ceil_div((int64_t)B * h, 8) * 8 * chunks;
+    VT_REQUIRE(grid < (1ll << 31), VTDGE_ERR_UNSUPPORTED, "sparse_attention_train: too many workgroups for one launch");
+    if (grid == 0) return VTDGE_OK;
+    const AttnTrain a{(const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (bf16_t *)out, offsets, q_row_stride,
+                      q_head_stride, kv_batch_stride, kv_tok_stride, kv_head_stride, o_row_stride, o_head_stride, B * h, h, n,
+                      scale * 1.44269504088896340736f};
+    note_kernel(reinterpret_cast<const void *>(attention_train_kernel));
+    attention_train_kernel<<<dim3((unsigned)grid), dim3(64 * AB_WAVES), 0, (hipStream_t)stream>>>(a);
+    return check_launch("sparse_attention_train");
 }
 
 extern "C" int vtdge_sparse_attention_backward(

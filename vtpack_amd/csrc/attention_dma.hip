@@ -37,13 +37,6 @@ __device__ __forceinline__ void attn_store(bf16_t *op, const f32x16 (&o)[2], flo
 constexpr float ATT_RESCALE = 8.0f;   // log2 units a score may exceed its row's reference by before that is raised
 constexpr int ATT_TBL = 512;          // items per workgroup whose first row and query count are kept in LDS
 
-// acc + lo + hi of a packed bf16 pair in fp32 (v_dot2c_f32_bf16 against (1, 1))
-__device__ __forceinline__ float bf16_pair_sum(uint32_t pair, float acc)
-{
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, 0x3f803f80u),
-                                           acc, false);
-}
-
 // ---------------------------------------------------------------------------------------------------------
 // One 32-query tile against all resident keys, software-pipelined over blocks of 32 keys: while the vector ALU
 // turns the scores of block kb into probabilities, the matrix pipe already multiplies K of block kb+1 with Q, and

@@ -216,6 +216,13 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const unsigned char *p)
     return __builtin_bit_cast(u32x2, r);
 }
 
+// acc + lo + hi of a packed bf16 pair in fp32 (v_dot2c_f32_bf16 against (1, 1))
+__device__ __forceinline__ float bf16_pair_sum(uint32_t pair, float acc)
+{
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, 0x3f803f80u),
+                                           acc, false);
+}
+
 // s_waitcnt with only the vector-memory counter constrained (gfx9 encoding)
 template <int N> __device__ __forceinline__ void wait_vmcnt()
 {

@@ -44,8 +44,8 @@ batched_sparse_attention = _SparseAttention.apply
 
 
 class _SparseAttentionTrain(Function):
-    """Attention of packed queries with gradients, without score-sized tensors: the inference kernel forward, scores worked
-    out again from q and k backward.  q [h, L, d], k and v [h, B, n, d] -> [L, h * d]."""
+    """Attention of packed queries with gradients, without score-sized tensors: scores are worked out from q and k forward
+    and again backward.  q [h, L, d], k and v [h, B, n, d] -> [L, h * d]."""
 
     @staticmethod
     def forward(ctx, q, k, v, q_lengths, scale):
@@ -54,7 +54,7 @@ class _SparseAttentionTrain(Function):
         offsets, lengths = ops.lengths_to_offsets(q_lengths, q.device)
         out = torch.empty((L, h * d), dtype=q.dtype, device=q.device)
         ctx.scale, ctx.max_rows = scale, int(lengths.max())
-        ops.sparse_attention_heads(q, k, v, offsets, scale, ctx.max_rows, out=out.view(L, h, d).transpose(0, 1))
+        ops.sparse_attention_heads(q, k, v, offsets, scale, ctx.max_rows, out=out.view(L, h, d).transpose(0, 1), train=True)
         ctx.save_for_backward(q, k, v, offsets)      # not the result: a caller may change that in place
         return out
 

@@ -909,14 +909,16 @@ def on_boundary(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
-def sparse_attention_heads(q, k, v, offsets, scale, max_rows_per_sample, out=None):
+def sparse_attention_heads(q, k, v, offsets, scale, max_rows_per_sample, out=None, train=False):
     """Head-major form: q [h, L, d], k and v [h, B, n, d] (rows on 16-byte boundaries, k and v with the same strides)
-    -> out, a [h, L, d] view of any strides like q's (by default dense)."""
+    -> out, a [h, L, d] view of any strides like q's (by default dense).  `train`: the scores that
+    `sparse_attention_backward` works out again (in bf16 a kernel of its own, head dim 64)."""
     h, L, d = q.shape
     B, n = k.shape[1], k.shape[2]
     if out is None:
         out = torch.empty((h, L, d), dtype=q.dtype, device=q.device)
-    call("vtdge_sparse_attention", ptr(q), q.stride(1), q.stride(0), ptr(k), ptr(v), k.stride(1), k.stride(2), k.stride(0),
+    call("vtdge_sparse_attention_train" if train and q.dtype == torch.bfloat16 else "vtdge_sparse_attention",
+         ptr(q), q.stride(1), q.stride(0), ptr(k), ptr(v), k.stride(1), k.stride(2), k.stride(0),
          ptr(offsets), ptr(out), out.stride(1), out.stride(0), B, h, d, n, max_rows_per_sample, float(scale), dtype_code(q),
          stream_ptr(), tag=("attention", B, h, d, n))
     return out
