@@ -128,6 +128,23 @@ def test_scores_are_those_of_the_queries_as_given(dev):
     assert float((got.double().cpu() - want).norm()) <= 2.5 * 1.6e-3 * float(want.norm())
 
 
+@pytest.mark.parametrize("shape", [(), (2, 1, 1)])
+def test_a_scale_that_is_a_tensor(dev, shape):
+    """One for all heads or one each, with a gradient of its own."""
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    lengths = [5, 17]
+    q, k, v = (torch.from_numpy(randn(i, *s)) for i, s in enumerate([(2, 22, 64), (2, 2, 33, 64), (2, 2, 33, 64)]))
+    g = torch.from_numpy(randn(3, 22, 128))
+    scale = (torch.arange(1, 1 + int(np.prod(shape))) * 0.1).view(shape).double().requires_grad_(True)
+    outs = [torch.softmax(q[:, a:b].double() @ k[:, i].double().transpose(1, 2) * scale, -1) @ v[:, i].double()
+            for i, (a, b) in enumerate([(0, 5), (5, 22)])]
+    want, = torch.autograd.grad(torch.cat(outs, 1).permute(1, 0, 2).reshape(22, 128), scale, g.double())
+    got = scale.detach().float().to(dev).requires_grad_(True)
+    out = sparse_attention_train(*(t.to(dev) for t in (q, k, v)), torch.tensor(lengths), got)
+    gs, = torch.autograd.grad(out, got, g.to(dev))
+    assert float((gs.double().cpu() - want).abs().max()) <= 1e-4 * float(want.abs().max())
+
+
 def test_the_result_may_be_changed_in_place(dev):
     """As the composition's could: the backward pass does not need it."""
     from vtpack_amd.layers.sparse_ops import sparse_attention_train

@@ -75,17 +75,17 @@ def sparse_attention_train(q, k, v, q_lengths, scale):
     (vtpack/models/dge/deit_dge.py:79-95): q [h, L, d]; k, v [h, B, n, d]; -> [L, h*d].
 
     Equal query counts (dense training: every granularity for every sample) use one batched matmul.  Otherwise, on the GPU
-    with head dim 64, one attention kernel forward and two backward; other operands compose two `batched_sparse_gemm` calls
-    around a softmax over the keys."""
+    with head dim 64, one attention kernel forward and two backward; other operands, and a scale that is a tensor (it may want
+    a gradient or differ by head), compose two `batched_sparse_gemm` calls around a softmax over the keys."""
     h, L, d = q.shape
     B, n = k.shape[1], k.shape[2]
     if int(q_lengths.max()) == int(q_lengths.min()):
         scores = torch.matmul(q.reshape(h, B, -1, d), k.transpose(-1, -2)) * scale
         ctx = torch.matmul(scores.softmax(dim=-1, dtype=v.dtype), v)              # [h, B, Lq, d]
         return ctx.permute(1, 2, 0, 3).reshape(-1, h * d)
-    if (d == 64 and q.is_cuda and q.dtype in (torch.float32, torch.bfloat16) and q.dtype == k.dtype == v.dtype
-            and k.shape == v.shape and k.shape[0] == h and k.shape[3] == d and q_lengths.numel() == B
-            and int(q_lengths.sum()) == L):
+    if (d == 64 and not torch.is_tensor(scale) and q.is_cuda and q.dtype in (torch.float32, torch.bfloat16)
+            and q.dtype == k.dtype == v.dtype and k.shape == v.shape and k.shape[0] == h and k.shape[3] == d
+            and q_lengths.numel() == B and int(q_lengths.sum()) == L):
         return _SparseAttentionTrain.apply(q, k, v, q_lengths, float(scale))
     kv_lengths = q_lengths.new_full([B], n)
     scores = batched_sparse_gemm(q, k.reshape(h, -1, d), q_lengths, kv_lengths, False, True) * scale
