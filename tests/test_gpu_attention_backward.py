@@ -128,6 +128,33 @@ def test_scores_are_those_of_the_queries_as_given(dev):
     assert float((got.double().cpu() - want).norm()) <= 2.5 * 1.6e-3 * float(want.norm())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("h,B,n,step", [(1, 2, 33, 64), (1, 1, 1, 64), (2, 1, 33, 64), (1, 2, 3, 1 << 23)])
+def test_strides_of_single_heads_samples_and_keys(dev, dtype, h, B, n, step):
+    """Dimensions of size one may carry any stride, queries may lie far apart: the same bytes as from dense operands."""
+    from vtpack_amd import _C
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    lengths = [3, 5][:B]
+    L = sum(lengths)
+
+    def odd(t, row=None):
+        st = [3 if s == 1 else d for s, d in zip(t.shape, t.stride())]
+        if row is not None:
+            st[-2], st[0] = row, (3 if t.shape[0] == 1 else t.stride(0))
+        out = torch.empty_strided(t.shape, st, dtype=t.dtype, device=dev)
+        return out.copy_(t)
+
+    q, k, v, g = (torch.from_numpy(randn(i, *s)).to(dtype).to(dev)
+                  for i, s in enumerate([(h, L, 64), (h, B, n, 64), (h, B, n, 64), (L, h * 64)]))
+    runs = []
+    for a in ((q, k, v), (odd(q, step if step > 64 else None), odd(k), odd(v))):
+        a = [t.detach().requires_grad_(True) for t in a]
+        out = _C.batched_sparse_attention_forward(*(t.detach() for t in a), torch.tensor(lengths), 0.125)
+        res = sparse_attention_train(*a, torch.tensor(lengths), 0.125)
+        runs.append((out, res.detach()) + torch.autograd.grad(res, a, g))
+    assert all(torch.equal(x, y) for x, y in zip(*runs))
+
+
 @pytest.mark.parametrize("shape", [(), (2, 1, 1)])
 def test_a_scale_that_is_a_tensor(dev, shape):
     """One for all heads or one each, with a gradient of its own."""

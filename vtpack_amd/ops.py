@@ -896,10 +896,23 @@ def lengths_to_offsets(lengths, device):
     return offsets, lengths
 
 
+def steps(t):
+    """The strides of t, with a dense tensor's in place of those of dimensions of size one: there they are never taken, and
+    torch leaves any number in them (a contiguous tensor's too), which the kernels would refuse as misaligned."""
+    if 1 not in t.shape:
+        return t.stride()
+    out, dense = [], 1
+    for n, s in zip(reversed(t.shape), reversed(t.stride())):
+        out.append(s if n > 1 else dense)
+        dense *= max(n, 1)
+    return out[::-1]
+
+
 def vector_rows(t):
-    """t itself where its last dimension is dense and every row starts on a 16-byte boundary, else a dense copy."""
-    vec = 16 // t.element_size()
-    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % vec == 0 for s in t.stride()[:-1]):
+    """t itself where its last dimension is dense and every row starts on a 16-byte boundary, less than 2^23 values from the
+    next, else a dense copy."""
+    vec, st = 16 // t.element_size(), steps(t)
+    if st[-1] == 1 and t.data_ptr() % 16 == 0 and all(s % vec == 0 for s in st[:-1]) and st[-2] < 1 << 23:
         return t
     return t.contiguous()
 
@@ -917,10 +930,10 @@ def sparse_attention_heads(q, k, v, offsets, scale, max_rows_per_sample, out=Non
     B, n = k.shape[1], k.shape[2]
     if out is None:
         out = torch.empty((h, L, d), dtype=q.dtype, device=q.device)
+    qs, ks, os = steps(q), steps(k), steps(out)
     call("vtdge_sparse_attention_train" if train and q.dtype == torch.bfloat16 else "vtdge_sparse_attention",
-         ptr(q), q.stride(1), q.stride(0), ptr(k), ptr(v), k.stride(1), k.stride(2), k.stride(0),
-         ptr(offsets), ptr(out), out.stride(1), out.stride(0), B, h, d, n, max_rows_per_sample, float(scale), dtype_code(q),
-         stream_ptr(), tag=("attention", B, h, d, n))
+         ptr(q), qs[1], qs[0], ptr(k), ptr(v), ks[1], ks[2], ks[0], ptr(offsets), ptr(out), os[1], os[0], B, h, d, n,
+         max_rows_per_sample, float(scale), dtype_code(q), stream_ptr(), tag=("attention", B, h, d, n))
     return out
 
 
@@ -933,8 +946,8 @@ def sparse_attention_backward(q, k, v, out, grad, offsets, scale, max_rows_per_s
     dq = torch.empty((L, h, d), dtype=q.dtype, device=q.device).transpose(0, 1)
     dk, dv = torch.empty_like(k), torch.empty_like(v)
     work = torch.empty((2 * h * L,), dtype=torch.float32, device=q.device)
-    call("vtdge_sparse_attention_backward", ptr(q), q.stride(1), q.stride(0), ptr(k), ptr(v), k.stride(1), k.stride(2),
-         k.stride(0), 0, ptr(grad), grad.stride(1), grad.stride(0), ptr(offsets), ptr(dq), dq.stride(1), dq.stride(0),
-         ptr(dk), ptr(dv), dk.stride(1), dk.stride(2), dk.stride(0), ptr(work), L, B, h, d, n, max_rows_per_sample,
-         float(scale), dtype_code(q), stream_ptr(), tag=("attention_backward", B, h, d, n))
+    qs, ks, gs, dqs, dks = (steps(t) for t in (q, k, grad, dq, dk))
+    call("vtdge_sparse_attention_backward", ptr(q), qs[1], qs[0], ptr(k), ptr(v), ks[1], ks[2], ks[0], 0, ptr(grad), gs[1],
+         gs[0], ptr(offsets), ptr(dq), dqs[1], dqs[0], ptr(dk), ptr(dv), dks[1], dks[2], dks[0], ptr(work), L, B, h, d,
+         n, max_rows_per_sample, float(scale), dtype_code(q), stream_ptr(), tag=("attention_backward", B, h, d, n))
     return dq, dk, dv
