@@ -258,3 +258,28 @@ def test_parameters_made_in_inference_mode_have_no_chain_plan():
     with torch.inference_mode():
         blocks = list(VisionTransformer(**args).eval().blocks)
         assert engine._chain_plan(blocks, torch.float32, torch.device("cpu"), 64, 1) is None
+
+
+def test_a_parameter_replaced_at_the_same_address_has_a_new_chain_plan():
+    """An allocator hands the storage of a parameter that is gone to the one that replaces it: same address, version and
+    shape, other values - and packed copies of the weights of before."""
+    from vtpack_amd import engine
+    from vtpack_amd.models.dge.deit_dge import VisionTransformer
+    blocks = list(VisionTransformer(img_size=64, patch_size=16, embed_dim=64, depth=2, num_heads=1, qkv_bias=True,
+                                    split_sizes=[4, 2, 1]).eval().blocks)
+
+    def plan():
+        return engine._chain_plan(blocks, torch.float32, torch.device("cpu"), 64, 1)
+
+    for module in (blocks[1].attn.proj, blocks[0].mlp.fc2):    # as load_state_dict(assign=True) leaves them: version 0
+        module.weight = torch.nn.Parameter(module.weight.detach().clone())
+    first = plan()
+    assert first is not None and plan() is first
+    for module in (blocks[1].attn.proj, blocks[0].mlp.fc2):
+        values, version = module.weight.detach().numpy(), module.weight._version      # the storage outlives the parameter
+        module.weight = torch.nn.Parameter(torch.from_numpy(values))
+        values += 1
+        assert module.weight.data_ptr() == values.ctypes.data and module.weight._version == version
+        second = plan()
+        assert second is not first and plan() is second
+        first = second

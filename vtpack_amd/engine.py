@@ -11,6 +11,7 @@ be captured into a HIP graph.
 import array
 import ctypes
 import operator
+import weakref
 
 import torch
 
@@ -442,8 +443,11 @@ class _ChainPlan:
     folded copies of its weights, and what the blocks have in common.  Checked against the parameters on every call
     (`_chain_plan`) and made again when any of them has changed; never copied or pickled with its model."""
 
-    def __init__(self, key, common):
+    def __init__(self, key, common, tensors):
         self.key, self.common = key, common
+        # the key names the parameters by their ids, which hold as long as all of them live: `whole` ends with the first
+        self.whole = whole = [True]
+        self.refs = [weakref.ref(t, lambda _: whole.clear()) for t in tensors]
         self.tables = {}        # (folded, packed copies wanted) -> (addresses, the derived tensors behind them)
         self.layouts = {}       # (B, H, W) -> (vtdge_chain, layout)
 
@@ -538,13 +542,13 @@ def _chain_plan(blocks, dtype, device, channels, extra):
     try:
         tensors = [_block_tensors(blk) for blk in blocks]
         flat = [t for ts in tensors for t in ts if t is not None]
-        key = (*(list(map(f, flat)) for f in _TENSOR_STATE), [t is None for ts in tensors for t in ts], dtype, device, extra,
+        key = (list(map(id, flat)), *(list(map(f, flat)) for f in _TENSOR_STATE), [t is None for ts in tensors for t in ts], dtype, device, extra,
                channels, [_block_numbers(blk) for blk in blocks], ops._pack_epoch, ops._plan_epoch)
     except (KeyError, AttributeError, RuntimeError):    # RuntimeError: parameters made in inference mode have no version
         return None
     plan = getattr(blocks[0], "_vtdge_chain", None)
-    if plan is None or plan.key != key:
-        plan = _ChainPlan(key, _common_of(blocks, tensors, dtype, device, channels, extra))
+    if plan is None or not plan.whole or plan.key != key:
+        plan = _ChainPlan(key, _common_of(blocks, tensors, dtype, device, channels, extra), flat)
         object.__setattr__(blocks[0], "_vtdge_chain", plan)
     return plan if plan.common is not None else None
 
