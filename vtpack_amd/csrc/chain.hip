@@ -147,6 +147,36 @@ static int fork_events(hipEvent_t &fork, hipEvent_t &join)
     return VTDGE_OK;
 }
 
+// The side stream of a chain: begin() lets it start behind the main stream, end() orders the main stream behind it.  Every
+// way out of the chain goes through end(), a failed launch's too: the caller frees the buffers when the call returns, on the
+// main stream, and a capture must not end with a stream that was forked and not joined.
+struct SideStream {
+    hipStream_t main, side;
+    hipEvent_t fork = nullptr, join = nullptr;
+    bool open = false;
+    SideStream(void *m, void *s) : main((hipStream_t)m), side((hipStream_t)s) {}
+    ~SideStream() { end(); }
+    int begin()
+    {
+        if (fork == nullptr) {
+            const int rc = fork_events(fork, join);
+            if (rc != VTDGE_OK) return rc;
+        }
+        VT_REQUIRE(hipEventRecord(fork, main) == hipSuccess && hipStreamWaitEvent(side, fork, 0) == hipSuccess, VTDGE_ERR_LAUNCH,
+                   "chain: cannot fork to the side stream");
+        open = true;
+        return VTDGE_OK;
+    }
+    int end()
+    {
+        if (!open) return VTDGE_OK;
+        open = false;
+        VT_REQUIRE(hipEventRecord(join, side) == hipSuccess && hipStreamWaitEvent(main, join, 0) == hipSuccess, VTDGE_ERR_LAUNCH,
+                   "chain: cannot join the side stream");
+        return VTDGE_OK;
+    }
+};
+
 static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const *params, const void *front, char *x0,
                      char *ints, char *big, char *scratch, char *out, void *stream, void *side)
 {
@@ -155,8 +185,7 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
     char *x = x0;
     int cur = 0;                 // which of the double buffers holds what the previous block left for this one
     bool routed = false, packed = false, have_counts = false;
-    hipEvent_t fork = nullptr, join = nullptr;
-    if (side != nullptr) VT_TRY(fork_events(fork, join));
+    SideStream beside(stream, side);
 
     for (int i = 0; i < c->depth; i++) {
         const void *const *P = params + (int64_t)i * P_COUNT;
@@ -203,9 +232,7 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
             if (side != nullptr) {
                 // the routing chain beside the key/value chain, joined before attention
                 routing = side;
-                VT_REQUIRE(hipEventRecord(fork, (hipStream_t)stream) == hipSuccess &&
-                               hipStreamWaitEvent((hipStream_t)side, fork, 0) == hipSuccess,
-                           VTDGE_ERR_LAUNCH, "chain: cannot fork to the side stream");
+                VT_TRY(beside.begin());
             }
             char *comp_ln = p.ln_kvq ? nullptr : scratch + p.comp_ln, *xln = scratch + p.xln;
             if (!routed)
@@ -238,10 +265,7 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
                 const int64_t kv_rows = (int64_t)B * p.n_kv;
                 VT_TRY(vtdge_linear_prepacked(src, C, P[P_KVW], kv_rows >= 2048 ? P[P_KVP] : nullptr, P[P_KVB], nullptr, 0, kv,
                                               2 * C, nullptr, kv_rows, 2 * C, C, VTDGE_ACT_NONE, dt, stream));
-                if (side != nullptr)
-                    VT_REQUIRE(hipEventRecord(join, (hipStream_t)side) == hipSuccess &&
-                                   hipStreamWaitEvent((hipStream_t)stream, join, 0) == hipSuccess,
-                               VTDGE_ERR_LAUNCH, "chain: cannot join the side stream");
+                VT_TRY(beside.end());
                 VT_TRY(vtdge_linear_prepacked(comp_ln, C, P[P_QW], pk(P_QP), P[P_QB], nullptr, 0, q, C, live, p.cap, C, C,
                                               VTDGE_ACT_NONE, dt, stream));
             }
