@@ -116,7 +116,7 @@ def _ordered(log):
 
 def test_a_whole_chain_joins_its_streams(program):
     log = program()
-    assert log[-1] == "rc 0" and _ordered(log)
+    assert "rc 0" in log and _ordered(log)
     assert sum(line.startswith("launch") and line.endswith(SIDE) for line in log) >= 6
 
 
@@ -129,4 +129,10 @@ def test_a_launch_that_fails_leaves_the_streams_joined(program, name, count):
     assert sum(line.split()[1] == name for line in whole if line.startswith("launch")) == count
     for at in range(count):
         log = program(name, at)
-        assert log[-1] != "rc 0" and _ordered(log), (name, at)
+        assert "rc 0" not in log and _ordered(log), (name, at)
+
+
+def test_the_events_of_a_thread_end_with_it(program):
+    log = program(5)
+    made = sum(line.startswith("create") for line in log)
+    assert made >= 2 and made == sum(line.startswith("destroy") for line in log)

@@ -11,6 +11,7 @@
 // the patch descriptors, `scratch` everything that dies inside the call.  vtdge_chain_layout says how large they are
 // and where each block's results lie.
 #include "common.h"
+#include <unistd.h>
 
 namespace vtdge {
 
@@ -129,9 +130,19 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
     } while (0)
 
 // A pair of events per host thread and device for the fork to the side stream and the join behind it; each is recorded
-// anew before it is waited for.
+// anew before it is waited for.  They end with their thread (not in a process forked from it, where the runtime is not to be
+// called any more).
 struct ForkEvents {
     hipEvent_t fork[16] = {}, join[16] = {};
+    const pid_t owner = getpid();
+    ~ForkEvents()
+    {
+        if (getpid() != owner) return;
+        for (int i = 0; i < 16; i++) {
+            if (fork[i] != nullptr) (void)hipEventDestroy(fork[i]);
+            if (join[i] != nullptr) (void)hipEventDestroy(join[i]);
+        }
+    }
 };
 static int fork_events(hipEvent_t &fork, hipEvent_t &join)
 {
