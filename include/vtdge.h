@@ -441,8 +441,9 @@ int vtdge_lengths_to_offsets(const int64_t *lengths_host, int B, int64_t *offset
  *   A0 [rows0, K] leading dim lda0, W0 [N0, K], bias0 [N0] nullable, out0 [rows0, N0] dense, rows_dev0 nullable; the same
  *   for the second product with the same K and LayerNorm, absent with rows1 = 0
  * Taken where vtdge_layernorm_linear_fits says 1 (rows of whole 128-byte pieces and at most 1024 values, few tiles);
- * VTDGE_ERR_UNSUPPORTED otherwise. */
+ * VTDGE_ERR_UNSUPPORTED otherwise.  vtdge_layernorm_linear_wanted: whether it is also the faster way. */
 int vtdge_layernorm_linear_fits(int64_t rows0, int N0, int64_t rows1, int N1, int K, int dtype);
+int vtdge_layernorm_linear_wanted(int64_t rows0, int N0, int64_t rows1, int N1, int K, int dtype);
 int vtdge_layernorm_linear(const void *A0, int64_t lda0, const void *W0, const void *bias0, void *out0,
                            const int64_t *rows_dev0, int64_t rows0, int N0, const void *A1, int64_t lda1, const void *W1,
                            const void *bias1, void *out1, const int64_t *rows_dev1, int64_t rows1, int N1,

@@ -400,7 +400,7 @@ def test_forward_captured_in_a_graph_follows_its_input(dev):
     count from device memory), so it can be captured once in a HIP graph and replayed on new images written into
     the captured input buffer: the router then takes other decisions and the row counts change inside the graph.
     Every replay must give, bit for bit, what the eager forward gives for the same images - with eager work and
-    synchronisations of the program between the replays, and the two streams of a block inside the capture."""
+    synchronisations of the program between the replays.  (One stream at these sizes; two: test_gpu_chain.py.)"""
     from vtpack_amd.synthetic import synthetic_images
     m = _model("deit_dge_s124_small_patch16_256", dev, torch.bfloat16)
     static_in = synthetic_images(8, 256, seed=11, dtype=torch.bfloat16).to(dev)

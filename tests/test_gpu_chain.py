@@ -1,6 +1,7 @@
 """A chain of blocks issued by one call into the library against the same blocks composed launch by launch: the same
 kernels in the same order, so every output and every value of `states` is the same bit for bit."""
 import copy
+import threading
 
 import pytest
 import torch
@@ -152,3 +153,62 @@ def test_a_kept_value_keeps_no_more_than_itself(dev, dtype, batch):
         for key in ("gate", "offsets_device", "batches_device"):
             held = blk.dge.states[key].untyped_storage().nbytes()
             assert held <= 1 << 18, key
+
+
+def _two_stream_models(dev):
+    return [(_deit(dev, torch.float32, 192), torch.float32, 40), (_deit(dev, torch.bfloat16, 768), torch.bfloat16, 40),
+            (_pvt(dev, torch.bfloat16), torch.bfloat16, 9)]
+
+
+def test_two_streams_of_a_chain_captured_in_a_graph(dev, monkeypatch):
+    """Fork and join of the side stream inside a capture: every replay gives what the eager forward gives for its images,
+    with eager work and synchronisations between the replays."""
+    monkeypatch.setattr(engine, "OVERLAP_FROM", 0)
+    for m, dtype, batch in _two_stream_models(dev):
+        static_in = synthetic_images(batch, 128, seed=20, dtype=dtype, device=dev)
+        side = torch.cuda.Stream()
+        with torch.no_grad():
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                m(static_in)
+            torch.cuda.current_stream().wait_stream(side)
+            torch.cuda.synchronize()
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                static_out = m(static_in)
+            for seed in (20, 21, 22, 20):
+                img = synthetic_images(batch, 128, seed=seed, dtype=dtype, device=dev)
+                eager = m(img).clone()
+                torch.cuda.synchronize()
+                static_in.copy_(img)
+                g.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(static_out, eager), (dtype, seed)
+
+
+def test_host_threads_with_streams_of_their_own(dev, monkeypatch):
+    """One model called from four threads at once, each on a stream of its own (and its side stream)."""
+    monkeypatch.setattr(engine, "OVERLAP_FROM", 0)
+    for m, dtype, batch in _two_stream_models(dev):
+        images = [synthetic_images(batch, 128, seed=30 + i, dtype=dtype, device=dev) for i in range(4)]
+        with torch.no_grad():
+            want = [m(im).clone() for im in images]
+        torch.cuda.synchronize()
+        got, errors = [None] * 4, []
+
+        def work(i):
+            try:
+                with torch.no_grad(), torch.cuda.stream(torch.cuda.Stream()):
+                    for _ in range(5):
+                        got[i] = m(images[i])
+                    torch.cuda.current_stream().synchronize()
+            except Exception as e:      # noqa: BLE001
+                errors.append(e)
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not errors
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), dtype

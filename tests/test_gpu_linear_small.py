@@ -88,3 +88,20 @@ def test_patch_embedding_of_few_rows(dev, dtype, B, S, P, N, extra):
     want = F.conv2d(img.double().cpu(), w.double().cpu(), b.double().cpu(), stride=P).flatten(2).transpose(1, 2)
     assert rel_err(out[:, extra:], want + pos[extra:].double().cpu()) <= TOL[dtype]
     assert bool((out[:, :extra] == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype,rows,N,K,small", [
+    (torch.bfloat16, 257, 1536, 384, True), (torch.bfloat16, 1339, 1536, 384, False), (torch.bfloat16, 1285, 768, 768, True),
+    (torch.bfloat16, 2715, 768, 768, False), (torch.bfloat16, 4091, 320, 1280, False), (torch.float32, 1339, 768, 768, True),
+    (torch.float32, 7451, 192, 192, False)])
+def test_packed_rows_are_counted_as_if_all_were_live(dev, dtype, rows, N, K, small):
+    """An untrained router leaves every row live: the rule must not count on half of them being absent."""
+    from vtpack_amd import _lib, ops
+    a, w, b = _make(dev, dtype, rows, (rows, K), (N, K), (N,))
+    w = w / K ** 0.5
+    live = rows - 3
+    out = torch.full((rows, N), 7.0, device=dev, dtype=dtype)
+    ops.linear(a, w, b, rows_dev=torch.tensor([live], device=dev), out=out)
+    assert ("linear_small" if small else "linear_dma") in _lib.last_kernel()
+    assert rel_err(out[:live], a[:live].double() @ w.double().T + b.double()) <= TOL[dtype]
+    assert bool((out[live:] == 7.0).all())

@@ -283,3 +283,16 @@ def test_a_parameter_replaced_at_the_same_address_has_a_new_chain_plan():
         second = plan()
         assert second is not first and plan() is second
         first = second
+
+
+def test_layernorm_linear_is_wanted_where_it_fits_and_not_beyond_its_lead():
+    from vtpack_amd import _lib
+    lib = _lib.load()
+    for rows, C, hidden, dtype, pair, fc1 in [
+            (257, 384, 1536, _lib.BF16, 1, 1), (514, 384, 1536, _lib.BF16, 1, 0), (514, 768, 3072, _lib.BF16, 1, 0),
+            (771, 768, 3072, _lib.BF16, 0, 0), (771, 320, 1280, _lib.BF16, 1, 0), (1285, 192, 768, _lib.BF16, 1, 1),
+            (514, 192, 768, _lib.F32, 1, 1), (771, 192, 768, _lib.F32, 1, 0), (3000, 192, 768, _lib.F32, 0, 0)]:
+        both, one = (rows, 2 * C, rows, C, C, dtype), (rows, hidden, 0, 0, C, dtype)
+        assert (lib.vtdge_layernorm_linear_wanted(*both), lib.vtdge_layernorm_linear_wanted(*one)) == (pair, fc1), (rows, C)
+        assert lib.vtdge_layernorm_linear_fits(*both) >= pair and lib.vtdge_layernorm_linear_fits(*one) >= fc1
+    assert lib.vtdge_layernorm_linear_fits(771, 1536, 771, 768, 768, _lib.BF16)      # what was taken before still is

@@ -67,6 +67,7 @@ SIGNATURES = {
                                         _l, _i, _i, _i, _i, _i, _f, _i, _p],
     "vtdge_lengths_to_offsets": [_p, _i, _p, _p],
     "vtdge_layernorm_linear_fits": [_l, _i, _l, _i, _i, _i],
+    "vtdge_layernorm_linear_wanted": [_l, _i, _l, _i, _i, _i],
     "vtdge_layernorm_linear": [_p, _l, _p, _p, _p, _p, _l, _i, _p, _l, _p, _p, _p, _p, _l, _i, _p, _p, _f, _i, _i, _i, _p],
     "vtdge_block_tail_fits": [_l, _i, _i, _i],
     "vtdge_block_tail_wanted": [_l, _i, _i, _i],

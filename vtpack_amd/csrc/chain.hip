@@ -71,9 +71,9 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
     p.by_region = c->splits_124 && nvec > 32 && nvec <= 64 && c->extra <= 64 && p.regions <= 65536 && p.rows < (1 << 24);
     p.folded = p.by_region && c->dtype == VTDGE_BF16 && c->C == 384 && p.rows >= 2048 && c->sr == 1 &&
                c->hidden % 384 == 0 && c->hidden <= 3072;
-    p.ln_kvq = !p.folded && c->sr == 1 && vtdge_layernorm_linear_fits(p.rows, 2 * c->C, p.cap, c->C, c->C, c->dtype);
+    p.ln_kvq = !p.folded && c->sr == 1 && vtdge_layernorm_linear_wanted(p.rows, 2 * c->C, p.cap, c->C, c->C, c->dtype);
     p.tail = vtdge_block_tail_wanted(p.rows, c->C, c->hidden, c->dtype);
-    p.ln_fc1 = !p.folded && !p.tail && vtdge_layernorm_linear_fits(p.cap, c->hidden, 0, 0, c->C, c->dtype);
+    p.ln_fc1 = !p.folded && !p.tail && vtdge_layernorm_linear_wanted(p.cap, c->hidden, 0, 0, c->C, c->dtype);
     p.pack = p.folded && c->depth > 1 && p.regions % 4 == 0;
     p.ws_words = p.pack ? vtdge_decompress_router_compress_workspace(c->B, c->H, c->W, 4) / 8 : 0;
 

@@ -203,7 +203,7 @@ int launch_patch_linear(const void *tokens, const void *W, const void *bias, voi
 // few rows (linear_small.hip)
 bool linear_small_fits(int64_t lda, int64_t ldr, int64_t ldo, int64_t rows, int N, int K, int esz, const void *bias,
                        const void *res, const void *out);
-bool linear_small_wanted(int64_t rows, int N, int esz, bool packed);
+bool linear_small_wanted(int64_t rows, int N, int K, int esz);
 template <typename T>
 int launch_linear_small(const void *A, int64_t lda, const void *W, const void *bias, const void *res, int64_t ldr,
                         void *out, int64_t ldo, const int64_t *rows_dev, int64_t rows, int N, int K, int act,
@@ -444,7 +444,7 @@ extern "C" int vtdge_linear_prepacked(const void *A, int64_t lda, const void *W,
         return launch_linear_ws8(A, lda, W, packed, bias, residual, ldr, out, ldo, rows_dev, rows, N, act, st);
     if (linear_ks_applicable(lda, ldr, ldo, rows, N, K, esz, act, bias, residual, out))
         return launch_linear_ks(A, lda, W, packed, bias, residual, ldr, out, ldo, rows_dev, rows, N, st);
-    if (linear_small_wanted(rows, N, esz, rows_dev != nullptr) &&
+    if (linear_small_wanted(rows, N, K, esz) &&
         linear_small_fits(lda, ldr, ldo, rows, N, K, esz, bias, residual, out)) {
         if (dtype == VTDGE_F32)
             return launch_linear_small<float>(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);

@@ -432,8 +432,7 @@ int launch_patch_linear(const void *tokens, const void *W, const void *bias, voi
     const PatchGeom pg{P, 0, 1, 0, 0, C, H, Wd};
     const int64_t rows = (int64_t)B * (H / P) * (Wd / P);
     LinArgs a{tokens, 0, W, bias, nullptr, 0, out, N, nullptr, rows, N, P * P * C, VTDGE_ACT_NONE, st};
-    const bool few = sizeof(T) == 4 || ceil_div(rows, 32) * ceil_div(N, 32) <= 512;
-    if (few && patch_small_wanted(rows, N, a.K, sizeof(T), (int64_t)B * H * Wd * C * sizeof(T)))
+    if (patch_small_wanted(rows, N, a.K, sizeof(T), (int64_t)B * H * Wd * C * sizeof(T)))
         return launch_patch_small<T>(tokens, W, bias, nullptr, out, rows, N, a.K, pg, st);
     if constexpr (sizeof(T) == 4) return go<T, 64, 64, 2, 2, 4, VTDGE_ACT_NONE, true, false, true>(a, pg);
     else {

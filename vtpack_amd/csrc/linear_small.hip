@@ -328,17 +328,28 @@ bool linear_small_fits(int64_t lda, int64_t ldr, int64_t ldo, int64_t rows, int 
            (int64_t)N * K * esz < (1ll << 31) && ((uintptr_t)out & piece) == 0;
 }
 
-// Which products the kernel is taken for, by their 32x32 tiles at full row capacity; of a packed operand (`packed`: the
-// live rows are counted on the device) about half the capacity is live.  Measured against the streaming kernel
-// (capacity rows, live rows, N, K; us): bf16 257, 257, 768, 384: 4.0 against 7.2; 257, 113, 384, 1536: 5.2 against 16.5;
-// 1285, 500, 768, 3072 (984 tiles): 11.2 against 29.8; 1285, 500, 3072, 768 (3936): 14.5 against 13.1; 1285, 1285, 1536,
-// 768 (1968, dense): 15.5 against 11.3.  fp32, whose instructions take eight times as long: 257, 113, 384, 1536: 9.8
-// against 35.4; 1285, 1285, 1536, 768 (1968, dense): 35 against 47; 1285, 500, 3072, 768 (3936): 33.4 against 37.3; 3341,
-// 3341, 768, 384 (2520, dense): 30.2 against 26.5.
+// Which products the kernel is taken for, by their 32x32 tiles at full row capacity: where it is no slower than the streaming
+// kernel with every row live, as a router that keeps the finest split (an untrained one) leaves them.  Of packed rows about
+// 0.44 are live for a trained mix; that only adds to its lead.  Measured, us, this kernel / streaming, all rows live and 0.44
+// of them, by tiles (rows, N, K):
+//   bf16  768 (4091, 192, 192) 5.7 / 6.1, 4.8 / 6.0     768 (507, 1536, 384) 7.3 / 8.1, 5.4 / 7.9
+//         760 (2427, 320, 1280) 13.7 / 14.0, 7.6 / 13.5 768 (1531, 512, 2048) 17.7 / 20.1, 9.2 / 19.2
+//        1008 (2011, 512, 2048) 24.0 / 19.9, 10.7 / 19.1   2016 (1339, 1536, 384) 15.1 / 8.8, 8.9 / 8.0
+//        1500 (4795, 320, 320) 12.7 / 7.3, 8.5 / 7.0    768 (4091, 192, 768) 11.7 / 10.3, 6.5 / 10.0 (narrow: half a tile
+//        of the streaming kernel's is empty, but it has many)
+//   long rows of 768 values and more, with as many outputs, leave the streaming kernel few tiles and long chains:
+//        1008 (1339, 768, 768) 10.4 / 10.0, 6.4 / 9.7   1008 (1339, 768, 3072) 30.9 / 27.7, 13.5 / 27.2 (30.2 on the tiles
+//        before the present ones)  960 (315, 3072, 768) 10.4 / 12.5, 8.3 / 12.1
+//        1488 (1979, 768, 768) 15.2 / 10.0, 8.4 / 9.6   1488 (1979, 768, 3072) 46.2 / 27.9, 20.2 / 27.2
+//   fp32 1024 (2043, 512, 2048) 54.6 / 45.7, 25.8 / 42.1   1020 (2715, 384, 1536) 42.5 / 58.0, 33.8 / 32.3
+//        1008 (1339, 768, 768) 23.7 / 31.4, 12.1 / 18.6    1020 (5435, 192, 768) 26.1 / 31.6, 19.3 / 18.1
+//        1398 (7451, 192, 192) 18.0 / 11.6, 10.9 / 7.5     2040 (5435, 384, 1536) 81.7 / 85.1, 52.0 / 33.1
+//        2700 (7195, 384, 384) 38.7 / 26.3, 25.4 / 17.9    4080 (13051, 320, 1280) 128.9 / 113.5, 70.4 / 48.3
 static int64_t small_tiles(int64_t rows, int N) { return ceil_div(rows, SM_BM) * ceil_div(N, 32); }
-bool linear_small_wanted(int64_t rows, int N, int esz, bool packed)
+bool linear_small_wanted(int64_t rows, int N, int K, int esz)
 {
-    return small_tiles(rows, N) <= (esz == 2 ? 1024 : 2048) * (packed ? 2 : 1);
+    const int64_t most = esz == 4 || (N >= 768 && K >= 768) ? 1024 : N >= 256 ? 768 : 640;
+    return small_tiles(rows, N) <= most;
 }
 
 template <typename T>
@@ -364,10 +375,14 @@ template int launch_linear_small<float>(const void *, int64_t, const void *, con
 template int launch_linear_small<bf16_t>(const void *, int64_t, const void *, const void *, const void *, int64_t, void *,
                                          int64_t, const int64_t *, int64_t, int, int, int, hipStream_t);
 
-// The patch embedding and the strided convolution over tokens (patch_source.h) for few rows.
+// The patch embedding and the strided convolution over tokens (patch_source.h) for few rows, by the same tiles (all rows
+// live).  Measured, us, this kernel / streaming (rows, N, K): images, bf16 480 (1280, 384, 768) 8.3 / 11.7, 576 12.0 / 11.8,
+// 960 14.5 / 11.9; fp32 480 15.0 / 21.1, 768 (1024, 768, 768) 21.6 / 21.8, 1920 52.0 / 37.0.  Blocks of tokens, bf16 512
+// (1024, 512, 1280) 10.3 / 10.8, (4096, 128, 256) 6.7 / 5.9; fp32 700 (2240, 320, 1280) 31.0 / 33.4, (11200, 64, 4096)
+// 79 / 93, 1000 (1984, 512, 1280) 40 / 35, 2000 74 / 54.
 bool patch_small_wanted(int64_t rows, int N, int K, int esz, int64_t source_bytes)
 {
-    return linear_small_wanted(rows, N, esz, false) && (int64_t)K * esz % SLAB_BYTES == 0 && N % 4 == 0 &&
+    return small_tiles(rows, N) <= (esz == 2 ? 512 : 768) && (int64_t)K * esz % SLAB_BYTES == 0 && N % 4 == 0 &&
            source_bytes < (1ll << 31) && (int64_t)N * K * esz < (1ll << 31);
 }
 template <typename T>
@@ -384,18 +399,29 @@ template int launch_patch_small<float>(const void *, const void *, const void *,
 template int launch_patch_small<bf16_t>(const void *, const void *, const void *, const void *, void *, int64_t, int, int,
                                         const PatchGeom &, hipStream_t);
 
-// act(LayerNorm(A) W^T + bias): one problem, or two over the same K with the same LayerNorm (rows1 = 0: none).  Every
-// column tile normalises its rows again, so what the LayerNorm kernels' launches cost is given back from some number of
-// tiles on, the sooner the longer the rows (two workgroups share a compute unit up to 1536 bytes).  Measured against the
-// separate kernels (capacity rows, K; us): keys/values and queries, bf16 257, 384: 7.3 against 14.4; 771, 384: 12.6
-// against 17.9; 257, 768: 14.3 against 18.4; fp32 257, 384: 10.5 against 17.9; 1285, 384 (1476 tiles): 26 against 30.5;
-// 257, 512 (432): 14.8 against 21; 514, 768 (1200): 44.6 against 38.2.  fc1 alone, bf16 514, 384 (816): 7.9 against 8.5;
-// fp32 771, 384 (1200): 16.5 against 15.3.
+// act(LayerNorm(A) W^T + bias): one problem, or two over the same K with the same LayerNorm (rows1 = 0: none).
 bool layernorm_linear_fits(int64_t rows0, int N0, int64_t rows1, int N1, int K, int esz)
 {
     const int64_t row = (int64_t)K * esz, tiles = small_tiles(rows0, N0) + small_tiles(rows1, N1);
     return row % SLAB_BYTES == 0 && row <= 2048 && N0 % 4 == 0 && N1 % 4 == 0 &&
            tiles <= (row > 1536 ? 512 : rows1 > 0 ? 2048 : 1024);
+}
+// Which of them the kernel is taken for: every column tile normalises its rows again, so what the LayerNorm kernels' launches
+// cost is given back from some number of tiles on, the sooner the longer the rows.  The line lies where the separate kernels
+// (streaming Linears) are even with all packed rows live, as an untrained router leaves them.  Measured, us, this kernel /
+// separate kernels (rows, K; tiles), all rows live: keys/values and queries, bf16 257, 384: 8.4 / 20.4; 1285, 384 (1476):
+// 19.8 / 21.1; 1028, 512 (1584): 23.4 / 22.8; 1285, 512 (1968): 26.4 / 23.4; 514, 768 (1224): 24.2 / 29.1; 771, 768 (1800):
+// 33.5 / 30.0; fp32 257, 384: 11.7 / 28.6; 1285, 384 (1476): 31.5 / 36.7; 3000, 192 (1692): 27.5 / 26.4; 2056, 320
+// (1950): 39.7 / 34.1.  fc1, bf16 1285, 192 (984): 9.6 / 11.4; 514, 320 (680): 11.1 / 11.2; 771, 320 (1000): 13.6 / 11.3; 514, 384
+// (816): 14.5 / 11.9; 257, 512 (576): 12.9 / 12.8; 64, 768 (192): 8.5 / 16.3; 257, 768 (864): 19.6 / 17.1; fp32 514, 192
+// (408): 10.2 / 12.0; 771, 192 (600): 15.0 / 12.4; 514, 320 (680): 18.3 / 20.0; 514, 384 (816): 22.2 / 22.3.
+static bool layernorm_linear_wanted(int64_t rows0, int N0, int64_t rows1, int N1, int K, int esz)
+{
+    const int64_t row = (int64_t)K * esz, tiles = small_tiles(rows0, N0) + small_tiles(rows1, N1);
+    if (!layernorm_linear_fits(rows0, N0, rows1, N1, K, esz)) return false;
+    if (esz == 4) return tiles <= (rows1 > 0 ? 1536 : row > 1024 ? 768 : 512);
+    if (rows1 > 0) return tiles <= (row > 1024 ? 1280 : row == 1024 ? 1600 : 2048);
+    return tiles <= (row <= 384 ? 1024 : row <= 1024 ? 640 : 512);
 }
 template <typename T>
 static int launch_layernorm_linear(const void *A0, int64_t lda0, const void *W0, const void *bias0, void *out0,
@@ -430,6 +456,12 @@ extern "C" int vtdge_layernorm_linear_fits(int64_t rows0, int N0, int64_t rows1,
 {
     if (rows0 < 0 || rows1 < 0 || N0 <= 0 || N1 < 0 || K <= 0 || (dtype != VTDGE_F32 && dtype != VTDGE_BF16)) return 0;
     return layernorm_linear_fits(rows0, N0, rows1, N1, K, dtype == VTDGE_BF16 ? 2 : 4) ? 1 : 0;
+}
+
+extern "C" int vtdge_layernorm_linear_wanted(int64_t rows0, int N0, int64_t rows1, int N1, int K, int dtype)
+{
+    if (rows0 < 0 || rows1 < 0 || N0 <= 0 || N1 < 0 || K <= 0 || (dtype != VTDGE_F32 && dtype != VTDGE_BF16)) return 0;
+    return layernorm_linear_wanted(rows0, N0, rows1, N1, K, dtype == VTDGE_BF16 ? 2 : 4) ? 1 : 0;
 }
 
 extern "C" int vtdge_layernorm_linear(const void *A0, int64_t lda0, const void *W0, const void *bias0, void *out0,

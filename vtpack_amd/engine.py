@@ -224,7 +224,7 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
              and ops.fits_linear_layernorm(x, attn.kv.weight))
     use_regions = REGION_COMPRESS and ops.fits_compress_regions(x, H, W, R, dge.router.split_sizes)
     norm_in = (NORM_IN_LINEAR and not fold1 and x_ln is None and not FUSE_ROUTER_NORM and getattr(attn, "sr_ratio", 1) <= 1
-               and ops.fits_layernorm_linear(x, attn.kv.weight, x, attn.q.weight))
+               and ops.fits_layernorm_linear(x, attn.kv.weight, x, attn.q.weight, wanted=True))
     overlap = overlap and OVERLAP and not norm_in and not (SERIAL_BESIDE_WEIGHT_STATIONARY and fold1 and use_regions)
     main = torch.cuda.current_stream(x.device)
     side = _side_stream(x.device, main.cuda_stream) if overlap else main
@@ -367,7 +367,7 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
         if fold2:
             hid = ops.linear_layernorm(q1, rec2, mlp.fc1.weight, mlp.fc1.bias, n2.weight, n2.bias, act="gelu",
                                        rows_dev=rows_dev)
-        elif NORM_IN_LINEAR and ops.fits_layernorm_linear(q1, mlp.fc1.weight):
+        elif NORM_IN_LINEAR and ops.fits_layernorm_linear(q1, mlp.fc1.weight, wanted=True):
             hid = ops.layernorm_linear(q1, mlp.fc1.weight, mlp.fc1.bias, n2.weight, n2.bias, n2.eps, act="gelu",
                                        rows_dev=rows_dev)
         else:

@@ -794,8 +794,9 @@ def linear_layernorm_pair(a0, records0, weight0, bias0, a1, records1, weight1, b
     return outs[0], outs[1]
 
 
-def fits_layernorm_linear(a, weight, a1=None, weight1=None):
-    """Whether `layernorm_linear` has a kernel for these operands (few rows of whole 128-byte pieces)."""
+def fits_layernorm_linear(a, weight, a1=None, weight1=None, wanted=False):
+    """Whether `layernorm_linear` has a kernel for these operands (few rows of whole 128-byte pieces) and, with `wanted`,
+    that is the faster way."""
     for t, w in ((a, weight), (a1, weight1)):
         if t is not None and (not t.is_cuda or not t.is_contiguous() or w.dtype != t.dtype or w.dim() != 2
                               or w.shape[1] != t.shape[-1]):
@@ -804,7 +805,9 @@ def fits_layernorm_linear(a, weight, a1=None, weight1=None):
         return False
     K = a.shape[-1]
     rows1, N1 = (a1.numel() // K, weight1.shape[0]) if a1 is not None else (0, 0)
-    return bool(_lib.load().vtdge_layernorm_linear_fits(a.numel() // K, weight.shape[0], rows1, N1, K, dtype_code(a)))
+    lib = _lib.load()
+    rule = lib.vtdge_layernorm_linear_wanted if wanted else lib.vtdge_layernorm_linear_fits
+    return bool(rule(a.numel() // K, weight.shape[0], rows1, N1, K, dtype_code(a)))
 
 
 def layernorm_linear(a, weight, bias, ln_weight, ln_bias, ln_eps, act="none", rows_dev=None, second=None):
