@@ -498,13 +498,6 @@ typedef struct {
 int vtdge_chain_layout(const vtdge_chain *chain, int64_t *layout_host);
 int vtdge_chain_forward(const vtdge_chain *chain, const void *const *params_host, const void *front_rows, void *x,
                         void *ints, void *big, void *scratch, void *out, void *stream, void *side_stream);
-/* The same with the tokens between the blocks in buffers of their own, which outlive the others as the caller likes:
- *   tokens_host  HOST table of depth - 1 device pointers [B, extra + H*W, C], 16-byte aligned (NULL: in `big`).  The first
- *                bytes of `big`, up to the first block's packed queries, are then not touched: `big` may point that far
- *                before a buffer that holds the rest. */
-int vtdge_chain_forward_tokens(const vtdge_chain *chain, const void *const *params_host, const void *front_rows, void *x,
-                               void *const *tokens_host, void *ints, void *big, void *scratch, void *out, void *stream,
-                               void *side_stream);
 
 #ifdef __cplusplus
 }

@@ -74,7 +74,6 @@ SIGNATURES = {
     "vtdge_block_tail": [_p, _p, _p, _p, _p, _p, _f, _p, _p, _p, _p, _p, _p, _l, _i, _i, _i, _p],
     "vtdge_chain_layout": [_p, _p],
     "vtdge_chain_forward": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p],
-    "vtdge_chain_forward_tokens": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p],
 }
 CHAIN_PARAMS, CHAIN_LAYOUT_HEAD, CHAIN_LAYOUT_BLOCK = 35, 8, 8      # include/vtdge.h
 

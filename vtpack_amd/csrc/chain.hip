@@ -189,7 +189,7 @@ struct SideStream {
 };
 
 static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const *params, const void *front, char *x0,
-                     void *const *tokens, char *ints, char *big, char *scratch, char *out, void *stream, void *side)
+                     char *ints, char *big, char *scratch, char *out, void *stream, void *side)
 {
     const int B = c->B, H = c->H, W = c->W, C = c->C, S = c->S, extra = c->extra, dt = c->dtype, N = p.N, esz = p.esz;
     const int d = C / c->heads;
@@ -213,7 +213,7 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
         char *recx = scratch + p.rec_x[cur], *nrecx = scratch + p.rec_x[cur ^ 1];
         char *recc = scratch + p.rec_c[cur], *nrecc = scratch + p.rec_c[cur ^ 1];
         char *kv = scratch + p.kv, *q = scratch + p.q, *o = scratch + p.o, *q1 = scratch + p.q1, *hid = scratch + p.hid;
-        char *xout = !Q ? out : tokens != nullptr ? (char *)tokens[i] : big + p.tok0 + i * p.tok_sz;
+        char *xout = Q ? big + p.tok0 + i * p.tok_sz : out;
         char *ngate = Q ? ints + p.gate0 + (i + 1) * p.gate_sz : nullptr;
         auto pk = [&](int which) { return p.rows >= 2048 ? P[which] : nullptr; };
 
@@ -364,9 +364,9 @@ extern "C" int vtdge_chain_layout(const vtdge_chain *chain, int64_t *layout_host
     return VTDGE_OK;
 }
 
-extern "C" int vtdge_chain_forward_tokens(const vtdge_chain *chain, const void *const *params_host, const void *front_rows,
-                                          void *x, void *const *tokens_host, void *ints, void *big, void *scratch, void *out,
-                                          void *stream, void *side_stream)
+extern "C" int vtdge_chain_forward(const vtdge_chain *chain, const void *const *params_host, const void *front_rows,
+                                   void *x, void *ints, void *big, void *scratch, void *out, void *stream,
+                                   void *side_stream)
 {
     VT_REQUIRE(params_host && x && ints && big && scratch && out, VTDGE_ERR_ARG, "chain: NULL operand");
     ChainPlan p;
@@ -375,9 +375,6 @@ extern "C" int vtdge_chain_forward_tokens(const vtdge_chain *chain, const void *
     VT_REQUIRE((((uintptr_t)x | (uintptr_t)ints | (uintptr_t)big | (uintptr_t)scratch | (uintptr_t)out |
                  (uintptr_t)front_rows) & 15) == 0,
                VTDGE_ERR_ARG, "chain: buffers must be 16-byte aligned");
-    for (int i = 0; tokens_host != nullptr && i + 1 < chain->depth; i++)
-        VT_REQUIRE(tokens_host[i] != nullptr && ((uintptr_t)tokens_host[i] & 15) == 0, VTDGE_ERR_ARG,
-                   "chain: the tokens behind block %d are NULL or not 16-byte aligned", i);
     for (int i = 0; i < chain->depth; i++) {
         const void *const *P = params_host + (int64_t)i * P_COUNT;
         bool ok = true;
@@ -386,12 +383,6 @@ extern "C" int vtdge_chain_forward_tokens(const vtdge_chain *chain, const void *
         if (chain->sr > 1) ok = ok && P[P_SRW] && P[P_SRB] && P[P_SRNW] && P[P_SRNB];
         VT_REQUIRE(ok, VTDGE_ERR_ARG, "chain: block %d lacks a parameter", i);
     }
-    return run_chain(chain, p, params_host, front_rows, (char *)x, tokens_host, (char *)ints, (char *)big, (char *)scratch,
-                     (char *)out, stream, p.folded || p.ln_kvq ? nullptr : side_stream);
-}
-
-extern "C" int vtdge_chain_forward(const vtdge_chain *chain, const void *const *params_host, const void *front_rows, void *x,
-                                   void *ints, void *big, void *scratch, void *out, void *stream, void *side_stream)
-{
-    return vtdge_chain_forward_tokens(chain, params_host, front_rows, x, nullptr, ints, big, scratch, out, stream, side_stream);
+    return run_chain(chain, p, params_host, front_rows, (char *)x, (char *)ints, (char *)big, (char *)scratch, (char *)out,
+                     stream, p.folded || p.ln_kvq ? nullptr : side_stream);
 }

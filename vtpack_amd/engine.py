@@ -588,10 +588,7 @@ def _chain_table(plan, blocks, folded, packs):
 
 
 class _ChainBlock(BlockView):
-    """Block `i` of a chain that ran natively: its `states` values, made from the chain's buffers when they are read.  The
-    packed rows and descriptors of all blocks share one buffer, so these come out as copies of the live rows: a value that
-    is kept must not keep the whole chain's memory.  (`gate` and the offsets are views: a captured graph's replays show in
-    them.)"""
+    """Block `i` of a chain that ran natively: its `states` values, made from the chain's buffers when they are read."""
 
     KEYS = ("comp", "input", "patches", "batches", "batches_device", "offsets_device", "gate", "queries")
 
@@ -605,11 +602,11 @@ class _ChainBlock(BlockView):
         return buf[at:at + n].view(dtype).view(shape)
 
     def get(self, key):
-        x, tokens, ints, big, (desc, lay) = self.run
+        x, ints, big, (desc, lay) = self.run
         B, N, C = x.shape
         o = lay[_lib.CHAIN_LAYOUT_HEAD + self.i * _lib.CHAIN_LAYOUT_BLOCK:][:_lib.CHAIN_LAYOUT_BLOCK]
         if key == "input":
-            return tokens[self.i - 1] if self.i else x
+            return x if o[4] < 0 else self._view(big, o[4], x.dtype, B, N, C)
         if key == "gate":
             return self._view(ints, o[0], x.dtype, B, desc.H // 4, desc.W // 4, desc.S)
         offsets = self._view(ints, o[1], torch.int64, B + 1)
@@ -627,13 +624,8 @@ class _ChainBlock(BlockView):
             return live.cpu()
         rows = int(live.sum())
         if key == "patches":
-            return self._view(big, o[7] - _first_packed(lay), torch.int64, B * N, 4)[:rows].clone()
-        return self._view(big, o[5 if key == "comp" else 6] - _first_packed(lay), x.dtype, B * N, C)[:rows].clone()
-
-
-def _first_packed(words):
-    """Where the packed rows begin in `big`: behind the room for the tokens between the blocks, which have their own."""
-    return words[_lib.CHAIN_LAYOUT_HEAD + 5]
+            return self._view(big, o[7], torch.int64, B * N, 4)[:rows]
+        return self._view(big, o[5 if key == "comp" else 6], x.dtype, B * N, C)[:rows]
 
 
 def _run_chain(blocks, x, H, W, front, plan, lay):
@@ -648,15 +640,12 @@ def _run_chain(blocks, x, H, W, front, plan, lay):
     side = 0
     if not words[4] and x.numel() >= OVERLAP_FROM:
         side = _side_stream(x.device, main.cuda_stream).cuda_stream
-    unused = _first_packed(words)
-    ints, big, scratch = (torch.empty((n,), dtype=torch.uint8, device=x.device) for n in (words[0], words[1] - unused, words[2]))
+    ints, big, scratch = (torch.empty((n,), dtype=torch.uint8, device=x.device) for n in words[:3])
     out = torch.empty_like(x)
-    tokens = [torch.empty_like(x) for _ in blocks[1:]]
-    between = array.array("Q", [t.data_ptr() for t in tokens])
-    _lib.call("vtdge_chain_forward_tokens", ctypes.addressof(desc), table.buffer_info()[0],
-              0 if front is None else front.data_ptr(), x.data_ptr(), between.buffer_info()[0], ints.data_ptr(),
-              big.data_ptr() - unused, scratch.data_ptr(), out.data_ptr(), main.cuda_stream, side)
-    run = (x, tokens, ints, big, lay)
+    _lib.call("vtdge_chain_forward", ctypes.addressof(desc), table.buffer_info()[0],
+              0 if front is None else front.data_ptr(), x.data_ptr(), ints.data_ptr(), big.data_ptr(), scratch.data_ptr(),
+              out.data_ptr(), main.cuda_stream, side)
+    run = (x, ints, big, lay)
     for i, blk in enumerate(blocks):
         st = blk.dge.states
         dict.update(st, dict.fromkeys(_ChainBlock.KEYS, _ChainBlock(run, i)))
