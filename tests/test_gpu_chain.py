@@ -137,6 +137,36 @@ def test_outputs_and_states_belong_to_their_call(dev):
     assert torch.equal(first, kept) and torch.equal(gate, gate_kept)
 
 
+@pytest.mark.parametrize("dtype,batch", [(torch.float32, 2), (torch.bfloat16, 33)])
+def test_a_kept_value_keeps_no_more_than_itself(dev, dtype, batch):
+    """The chain's blocks share buffers; a caller who collects one block's values over many batches must not hold those."""
+    m = _deit(dev, dtype, 384)
+    images = synthetic_images(batch, 128, seed=5, dtype=dtype, device=dev)
+    with torch.no_grad():
+        m(images)
+    assert getattr(m.blocks[0], "_vtdge_chain").common is not None
+    for blk in m.blocks:
+        for key in ("comp", "input", "patches", "queries", "gate", "offsets_device", "batches_device"):
+            t = blk.dge.states[key]
+            held, wanted = t.untyped_storage().nbytes(), t.numel() * t.element_size()
+            assert held <= 2 * wanted, key
+    # captured, `input`, `gate` and the offsets are the graph's own memory: its replays show in them
+    static_in = images.clone()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.graph(g):
+        m(static_in)
+    held = {key: m.blocks[1].dge.states[key] for key in ("input", "gate", "offsets_device")}
+    for seed in (5, 6, 5):
+        static_in.copy_(synthetic_images(batch, 128, seed=seed, dtype=dtype, device=dev))
+        with torch.no_grad():
+            m(static_in)
+        want = {key: m.blocks[1].dge.states[key] for key in held}
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(held[key], want[key]) for key in held), seed
+
+
 def _two_stream_models(dev):
     return [(_deit(dev, torch.float32, 192), torch.float32, 40), (_deit(dev, torch.bfloat16, 768), torch.bfloat16, 40),
             (_pvt(dev, torch.bfloat16), torch.bfloat16, 9)]

@@ -588,7 +588,10 @@ def _chain_table(plan, blocks, folded, packs):
 
 
 class _ChainBlock(BlockView):
-    """Block `i` of a chain that ran natively: its `states` values, made from the chain's buffers when they are read."""
+    """Block `i` of a chain that ran natively: its `states` values, made from the chain's buffers when they are read.  All
+    blocks share these, so a value comes out as a copy (of the live rows): one that is kept must not keep the whole chain's
+    memory.  A run that was captured into a graph keeps its buffers anyway, and its replays are to show in `input`, `gate`
+    and the offsets taken at the capture: these are views then."""
 
     KEYS = ("comp", "input", "patches", "batches", "batches_device", "offsets_device", "gate", "queries")
 
@@ -602,16 +605,22 @@ class _ChainBlock(BlockView):
         return buf[at:at + n].view(dtype).view(shape)
 
     def get(self, key):
-        x, ints, big, (desc, lay) = self.run
+        x, ints, big, (desc, lay), stream, captured = self.run
+
+        def copy(t):
+            with torch.cuda.stream(stream):       # behind the forward, wherever the reader is
+                return t.clone()
+
+        own = (lambda t: t) if captured else copy
         B, N, C = x.shape
         o = lay[_lib.CHAIN_LAYOUT_HEAD + self.i * _lib.CHAIN_LAYOUT_BLOCK:][:_lib.CHAIN_LAYOUT_BLOCK]
         if key == "input":
-            return x if o[4] < 0 else self._view(big, o[4], x.dtype, B, N, C)
+            return x if o[4] < 0 else own(self._view(big, o[4], x.dtype, B, N, C))
         if key == "gate":
-            return self._view(ints, o[0], x.dtype, B, desc.H // 4, desc.W // 4, desc.S)
+            return own(self._view(ints, o[0], x.dtype, B, desc.H // 4, desc.W // 4, desc.S))
         offsets = self._view(ints, o[1], torch.int64, B + 1)
         if key == "offsets_device":
-            return offsets
+            return own(offsets)
         # the host-side counts and the tensors cut to the live rows: one device->host copy per read, nothing cached (a
         # replay of a captured graph rewrites the buffers without running this code)
         if o[3] >= 0 and int(self._view(ints, o[3], torch.int64, 1)) != 0:
@@ -619,13 +628,13 @@ class _ChainBlock(BlockView):
                                "vtdge_decompress_router_compress): rows are missing")
         live = offsets[1:] - offsets[:-1] if o[2] < 0 else self._view(ints, o[2], torch.int64, B)
         if key == "batches_device":
-            return live
+            return live if o[2] < 0 else own(live)
         if key == "batches":
             return live.cpu()
         rows = int(live.sum())
         if key == "patches":
-            return self._view(big, o[7], torch.int64, B * N, 4)[:rows]
-        return self._view(big, o[5 if key == "comp" else 6], x.dtype, B * N, C)[:rows]
+            return copy(self._view(big, o[7], torch.int64, B * N, 4)[:rows])
+        return copy(self._view(big, o[5 if key == "comp" else 6], x.dtype, B * N, C)[:rows])
 
 
 def _run_chain(blocks, x, H, W, front, plan, lay):
@@ -645,7 +654,7 @@ def _run_chain(blocks, x, H, W, front, plan, lay):
     _lib.call("vtdge_chain_forward", ctypes.addressof(desc), table.buffer_info()[0],
               0 if front is None else front.data_ptr(), x.data_ptr(), ints.data_ptr(), big.data_ptr(), scratch.data_ptr(),
               out.data_ptr(), main.cuda_stream, side)
-    run = (x, ints, big, lay)
+    run = (x, ints, big, lay, main, torch.cuda.is_current_stream_capturing())
     for i, blk in enumerate(blocks):
         st = blk.dge.states
         dict.update(st, dict.fromkeys(_ChainBlock.KEYS, _ChainBlock(run, i)))
