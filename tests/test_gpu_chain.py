@@ -167,6 +167,25 @@ def test_a_kept_value_keeps_no_more_than_itself(dev, dtype, batch):
         assert all(torch.equal(held[key], want[key]) for key in held), seed
 
 
+def test_values_read_on_another_stream(dev):
+    """The reader's stream has not waited for the forward, which is still queued behind a long kernel."""
+    m = _deit(dev, torch.bfloat16, 384)
+    images = synthetic_images(33, 128, seed=5, dtype=torch.bfloat16, device=dev)
+    with torch.no_grad():
+        m(images)
+        want = [{k: b.dge.states[k].clone() for k in ("queries", "comp", "gate", "batches")} for b in m.blocks]
+        m(torch.zeros_like(images))
+        torch.cuda.synchronize()
+        reader = torch.cuda.Stream()
+        torch.cuda._sleep(20_000_000)
+        m(images)
+        with torch.cuda.stream(reader):
+            got = [{k: b.dge.states[k] + 0 for k in w} for b, w in zip(m.blocks, want)]
+        m(torch.zeros_like(images))             # may take the buffers that the values were read from
+    torch.cuda.synchronize()
+    assert all(torch.equal(a[k], b[k]) for a, b in zip(got, want) for k in a)
+
+
 def _two_stream_models(dev):
     return [(_deit(dev, torch.float32, 192), torch.float32, 40), (_deit(dev, torch.bfloat16, 768), torch.bfloat16, 40),
             (_pvt(dev, torch.bfloat16), torch.bfloat16, 9)]

@@ -1,5 +1,7 @@
 """Host-side logic of the package: API surface, state-dict names, error behaviour, complexity counter."""
+import contextlib
 import math
+import types
 
 import pytest
 import torch
@@ -283,6 +285,38 @@ def test_a_parameter_replaced_at_the_same_address_has_a_new_chain_plan():
         second = plan()
         assert second is not first and plan() is second
         first = second
+
+
+@pytest.mark.parametrize("captured", [False, True])
+def test_values_of_a_native_chain_are_copied_on_the_readers_stream(monkeypatch, captured):
+    """A copy made on the forward's stream would not be ordered before what the reader does with it on another one: the
+    reader's stream waits for the forward's and copies itself, and the buffers are kept for it."""
+    from vtpack_amd import engine
+    log = []
+
+    class Stream:
+        def wait_stream(self, other):
+            log.append(("wait", self, other))
+
+    reader, forward = Stream(), Stream()
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: reader)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: log.append(("on", s)) or contextlib.nullcontext())
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, s: log.append(("record", t.data_ptr(), s)))
+    monkeypatch.setattr(torch.Tensor, "clone", lambda t: log.append(("clone",)) or t + 0)
+    x, ints, big = torch.zeros(2, 17, 64), torch.zeros(4096, dtype=torch.uint8), torch.arange(255, dtype=torch.uint8).repeat(400)
+    desc = types.SimpleNamespace(H=4, W=4, S=3)
+    ints[:24].view(torch.int64)[:3] = torch.tensor([0, 5, 9])
+    layout = [0] * 8 + [512, 0, -1, -1, 0, 1024, 1024, 1024]          # gate, offsets, lengths, status, input, comp, queries, patches
+    view = engine._ChainBlock((x, ints, big, (desc, layout), forward, captured), 0)
+    for key, rows in (("comp", 9), ("queries", 9), ("patches", 9), ("gate", 2), ("input", 2), ("offsets_device", 3)):
+        log.clear()
+        assert view.get(key).shape[0] == rows
+        held = captured and key in ("gate", "input", "offsets_device")
+        assert not any(e[0] == "on" for e in log) and (("clone",) in log) == (not held), key
+        if not captured:
+            assert log[0] == ("wait", reader, forward), key
+            assert {e[1] for e in log if e[0] == "record"} == {x.data_ptr(), ints.data_ptr(), big.data_ptr()}
 
 
 def test_layernorm_linear_is_wanted_where_it_fits_and_not_beyond_its_lead():

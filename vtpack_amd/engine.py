@@ -589,9 +589,9 @@ def _chain_table(plan, blocks, folded, packs):
 
 class _ChainBlock(BlockView):
     """Block `i` of a chain that ran natively: its `states` values, made from the chain's buffers when they are read.  All
-    blocks share these, so a value comes out as a copy (of the live rows): one that is kept must not keep the whole chain's
-    memory.  A run that was captured into a graph keeps its buffers anyway, and its replays are to show in `input`, `gate`
-    and the offsets taken at the capture: these are views then."""
+    blocks share these, so a value comes out as a copy (of the live rows), made on the reader's stream: one that is kept must
+    not keep the whole chain's memory.  A run that was captured into a graph keeps its buffers anyway, and its replays are to
+    show in `input`, `gate` and the offsets taken at the capture: these are views then."""
 
     KEYS = ("comp", "input", "patches", "batches", "batches_device", "offsets_device", "gate", "queries")
 
@@ -606,12 +606,14 @@ class _ChainBlock(BlockView):
 
     def get(self, key):
         x, ints, big, (desc, lay), stream, captured = self.run
+        here = torch.cuda.current_stream(x.device)
+        if here != stream and not captured and not torch.cuda.is_current_stream_capturing():
+            # a reader on another stream: its copies come behind the forward, and the buffers stay until they are made
+            here.wait_stream(stream)
+            for t in (x, ints, big):
+                t.record_stream(here)
 
-        def copy(t):
-            with torch.cuda.stream(stream):       # behind the forward, wherever the reader is
-                return t.clone()
-
-        own = (lambda t: t) if captured else copy
+        own = (lambda t: t) if captured else torch.Tensor.clone
         B, N, C = x.shape
         o = lay[_lib.CHAIN_LAYOUT_HEAD + self.i * _lib.CHAIN_LAYOUT_BLOCK:][:_lib.CHAIN_LAYOUT_BLOCK]
         if key == "input":
@@ -633,8 +635,8 @@ class _ChainBlock(BlockView):
             return live.cpu()
         rows = int(live.sum())
         if key == "patches":
-            return copy(self._view(big, o[7], torch.int64, B * N, 4)[:rows])
-        return copy(self._view(big, o[5 if key == "comp" else 6], x.dtype, B * N, C)[:rows])
+            return self._view(big, o[7], torch.int64, B * N, 4)[:rows].clone()
+        return self._view(big, o[5 if key == "comp" else 6], x.dtype, B * N, C)[:rows].clone()
 
 
 def _run_chain(blocks, x, H, W, front, plan, lay):
