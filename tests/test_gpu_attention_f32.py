@@ -70,3 +70,21 @@ def test_first_stages_without_a_finite_score(dev, rows):
     p = np.exp(s - s.max(-1, keepdims=True))
     want = (p / p.sum(-1, keepdims=True)) @ v[:, 0].astype(np.float64)
     assert float(np.abs(got.numpy() - want).max()) <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("d", [64, 32])
+def test_keys_far_apart_and_in_reverse(dev, d):
+    """Token strides of 2^23 values and more, and negative ones: the same bytes as from dense keys and values."""
+    from vtpack_amd import _lib, ops
+    h, n, lengths = 2, 37, [20, 70]
+    L, B = sum(lengths), len(lengths)
+    q, k, v = (torch.from_numpy(randn(940 + i, *s, h * d)).to(dev) for i, s in enumerate([(L,), (B, n), (B, n)]))
+    offsets, _ = ops.lengths_to_offsets(torch.tensor(lengths), dev)
+    want = ops.sparse_attention(q, k, v, offsets, 0.2, h, max(lengths))
+    far = [torch.empty_strided(t.shape, (h * d, 1 << 23, 1), device=dev).copy_(t) for t in (k, v)]
+    assert torch.equal(ops.sparse_attention(q, *far, offsets, 0.2, h, max(lengths)), want)
+    back = [t.flip(1).contiguous() for t in (k, v)]
+    got = torch.empty_like(want)
+    _lib.call("vtdge_sparse_attention", q.data_ptr(), h * d, d, *(t[0, n - 1].data_ptr() for t in back), n * h * d, -h * d, d,
+              offsets.data_ptr(), got.data_ptr(), h * d, d, B, h, d, n, max(lengths), 0.2, _lib.F32, _lib.stream_ptr())
+    assert torch.equal(got, want)

@@ -43,7 +43,8 @@ template <int D> struct AttnF32 {
     }
 };
 
-template <int D>
+// WIDE: token strides of 2^23 values and more, or negative ones: 64-bit addresses of the direct loads
+template <int D, bool WIDE>
 __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
     const float *__restrict__ q, int64_t q_rs, int64_t q_hs, const float *__restrict__ k, const float *__restrict__ v,
     int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets, float *__restrict__ out,
@@ -75,17 +76,20 @@ __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
 
     const unsigned char *kbase = reinterpret_cast<const unsigned char *>(k + (int64_t)b * kv_bs + (int64_t)head * kv_hs);
     const unsigned char *vbase = reinterpret_cast<const unsigned char *>(v + (int64_t)b * kv_bs + (int64_t)head * kv_hs);
-    const uint32_t rowp = (uint32_t)(kv_ts * 4);
+    const int64_t rowp = kv_ts * 4;
     const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
     // one stage: loads [wid NL, wid NL + NL) of its BUF / 1024, K rows first.  Rows past the last key repeat it.
     auto load_stage = [&](int st) {
         const int key0 = st * AF_KEYS, last = n - 1 - key0;
         const uint32_t dst = lds0 + (uint32_t)((st % AF_RING) * G::BUF + wid * NL * 1024);
-        const void *base = uniform_ptr((wid < AF_TILES / 2 ? kbase : vbase) + (int64_t)key0 * rowp);
+        const unsigned char *src = (wid < AF_TILES / 2 ? kbase : vbase) + (int64_t)key0 * rowp;
+        const void *base = uniform_ptr(src);
 #pragma unroll
         for (int i = 0; i < NL; i++) {
             const int row = ((wid % (AF_TILES / 2)) * NL + i) * (64 / G::CPR) + lane / G::CPR;
-            dma16(base, (uint32_t)min(row, last) * rowp + (uint32_t)G::slot(row, lane % G::CPR) * 16u, dst + i * 1024);
+            const uint32_t piece = (uint32_t)G::slot(row, lane % G::CPR) * 16u;
+            if constexpr (WIDE) VT_GLOBAL_TO_LDS(src + min(row, last) * rowp + piece, smem + (dst - lds0) + i * 1024);
+            else dma16(base, (uint32_t)min(row, last) * (uint32_t)rowp + piece, dst + i * 1024);
         }
     };
 
@@ -246,25 +250,31 @@ __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
     }
 }
 
-template <int D>
-int launch_attention_f32(const void *q, int64_t q_rs, int64_t q_hs, const void *k, const void *v, int64_t kv_bs,
-                         int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs, int64_t o_hs,
-                         int B, int h, int n, int max_rows, float scale, hipStream_t st)
+template <int D, bool WIDE>
+static int go_attention_f32(const void *q, int64_t q_rs, int64_t q_hs, const void *k, const void *v, int64_t kv_bs,
+                            int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs, int64_t o_hs,
+                            int B, int h, int n, int max_rows, float scale, hipStream_t st)
 {
     constexpr size_t lds = AF_RING * AttnF32<D>::BUF;
     const int64_t pairs = (int64_t)B * h, chunks = ceil_div(max_rows, 16 * AF_TILES);
     const int64_t grid = ceil_div(pairs, 8) * 8 * chunks;
     VT_REQUIRE(grid < (1ll << 31), VTDGE_ERR_UNSUPPORTED, "sparse_attention: %lld workgroups exceed one launch",
                (long long)grid);
-    VT_REQUIRE(kv_ts >= 0 && kv_ts < (1 << 23), VTDGE_ERR_UNSUPPORTED, "sparse_attention: token stride %lld",
-               (long long)kv_ts);
-    auto kern = attention_f32_kernel<D>;
+    auto kern = attention_f32_kernel<D, WIDE>;
     VT_RESERVE_LDS(kern, lds, "sparse_attention");
     note_kernel(reinterpret_cast<const void *>(kern));
     kern<<<dim3((unsigned)grid), dim3(64 * AF_TILES), lds, st>>>(
         (const float *)q, q_rs, q_hs, (const float *)k, (const float *)v, kv_bs, kv_ts, kv_hs, offsets, (float *)out,
         o_rs, o_hs, (int)pairs, h, n, (int)chunks, scale * 1.44269504088896340736f);
     return check_launch("sparse_attention");
+}
+template <int D>
+int launch_attention_f32(const void *q, int64_t q_rs, int64_t q_hs, const void *k, const void *v, int64_t kv_bs,
+                         int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs, int64_t o_hs,
+                         int B, int h, int n, int max_rows, float scale, hipStream_t st)
+{
+    const auto go = kv_ts >= 0 && kv_ts < (1 << 23) ? go_attention_f32<D, false> : go_attention_f32<D, true>;
+    return go(q, q_rs, q_hs, k, v, kv_bs, kv_ts, kv_hs, offsets, out, o_rs, o_hs, B, h, n, max_rows, scale, st);
 }
 template int launch_attention_f32<64>(const void *, int64_t, int64_t, const void *, const void *, int64_t, int64_t,
                                       int64_t, const int64_t *, void *, int64_t, int64_t, int, int, int, int, float,
