@@ -115,6 +115,25 @@ def test_first_scores_of_minus_infinity(dev, dtype, first):
         assert float((a.double().cpu() - b).abs().max()) <= TOL[dtype] * float(b.abs().max())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("length", [5, 32, 45])
+def test_an_infinite_gradient_of_the_last_query(dev, dtype, length):
+    """dV takes it with the query's probabilities: infinite in its channel, finite in the others (rows past the last query,
+    which repeat it, have probability zero, and zero times infinity is NaN)."""
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    lengths = [length, 7]
+    L = sum(lengths)
+    q, k, v, g = (torch.from_numpy(randn(i, *s)).to(dtype)
+                  for i, s in enumerate([(1, L, 64), (1, 2, 33, 64), (1, 2, 33, 64), (L, 64)]))
+    g[length - 1, 3] = float("inf")
+    _, grads = _reference(q, k, v, lengths, 0.125, g)
+    args = [t.to(dev).requires_grad_(True) for t in (q, k, v)]
+    dv = torch.autograd.grad(sparse_attention_train(*args, torch.tensor(lengths), 0.125), args, g.to(dev))[2].double().cpu()
+    inf = torch.isinf(grads[2])
+    assert int(inf.sum()) == 33 and torch.equal(torch.isinf(dv), inf) and bool((dv[inf] > 0).all())
+    assert float((dv - grads[2])[~inf].abs().max()) <= TOL[dtype] * float(grads[2][~inf].abs().max())
+
+
 def test_scores_are_those_of_the_queries_as_given(dev):
     """Scores of spread 8 in bf16: a query rounded once more, times the scale, would be off by 2^-9 / sqrt(3) of its score,
     i.e. 9e-3 of a probability.  What remains are the roundings of the probabilities and of the result, 1.1e-3 each."""

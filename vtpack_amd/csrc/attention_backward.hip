@@ -420,8 +420,14 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
             qd.load(st + 1);
             if (wave_live) fetch(st + 1);
         }
+        unsigned char *Qs = smem + (st & 1) * 2 * B::HALF, *Ds = Qs + B::HALF;
+        const int left = Lb - st * AB_ROWS;
+        if (left < AB_ROWS) {                             // dO past the last query: nothing of it, not even 0 * infinity
+            for (int i = left * B::CPR + threadIdx.x; i < AB_ROWS * B::CPR; i += 64 * AB_WAVES)
+                *reinterpret_cast<u32x4 *>(Ds + i * 16) = u32x4{0u, 0u, 0u, 0u};
+            lds_barrier();
+        }
         if (!wave_live) continue;
-        const unsigned char *Qs = smem + (st & 1) * 2 * B::HALF, *Ds = Qs + B::HALF;
         f32x4 p[2], ds[2];
 #pragma unroll
         for (int blk = 0; blk < 2; blk++) {
