@@ -29,7 +29,6 @@ namespace vtdge {
 
 constexpr int AF_KEYS = 32;      // keys per stage
 constexpr int AF_TILES = 4;      // waves = query tiles of a full workgroup
-constexpr int AF_RING = 2;       // stages in LDS
 constexpr float AF_RAISE = 8.f;  // log2 units a score may exceed its query's reference by
 
 template <int D> struct AttnF32 {
@@ -48,7 +47,7 @@ template <int D, bool WIDE>
 __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
     const float *__restrict__ q, int64_t q_rs, int64_t q_hs, const float *__restrict__ k, const float *__restrict__ v,
     int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets, float *__restrict__ out,
-    int64_t o_rs, int64_t o_hs, int pairs, int h, int n, int chunks, float scale_log2)
+    int64_t o_rs, int64_t o_hs, int pairs, int h, int n, float scale_log2)
 {
     using G = AttnF32<D>;
     constexpr int NL = G::BUF / 1024 / AF_TILES;              // direct loads a wave and stage
@@ -81,7 +80,7 @@ __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
     // one stage: loads [wid NL, wid NL + NL) of its BUF / 1024, K rows first.  Rows past the last key repeat it.
     auto load_stage = [&](int st) {
         const int key0 = st * AF_KEYS, last = n - 1 - key0;
-        const uint32_t dst = lds0 + (uint32_t)((st % AF_RING) * G::BUF + wid * NL * 1024);
+        const uint32_t dst = lds0 + (uint32_t)((st & 1) * G::BUF + wid * NL * 1024);
         const unsigned char *src = (wid < AF_TILES / 2 ? kbase : vbase) + (int64_t)key0 * rowp;
         const void *base = uniform_ptr(src);
 #pragma unroll
@@ -94,9 +93,7 @@ __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
     };
 
     const int stages = (n + AF_KEYS - 1) / AF_KEYS;
-#pragma unroll
-    for (int i = 0; i < AF_RING - 1; i++)
-        if (i < stages) load_stage(i);
+    load_stage(0);
     // queries times scale * log2(e): the scores come out of the matrix pipe in log2 units
     f32x4 qf[D / 16];
     {
@@ -127,7 +124,7 @@ __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
     auto compute = [&](auto nbc, auto tailc, int st) {
         constexpr int NB = decltype(nbc)::value;
         constexpr bool TAIL = decltype(tailc)::value;
-        const unsigned char *S = smem + (st % AF_RING) * G::BUF;
+        const unsigned char *S = smem + (st & 1) * G::BUF;
         const int key0 = st * AF_KEYS + part * 16 + 4 * g;    // this lane's first key of block 0
         f32x4 s[NB];
 #pragma unroll
@@ -189,11 +186,9 @@ __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
     };
 
     for (int st = 0; st < stages; st++) {
-        // this wave's loads of stage st have landed once only those of the younger stages are outstanding
-        if (st + AF_RING - 2 < stages) wait_vmcnt<(AF_RING - 2) * NL>();
-        else wait_vmcnt<0>();
+        wait_vmcnt<0>();                                      // this wave's loads of stage st have landed
         block_barrier();                                      // stage st is whole; the buffer of st - 1 is free
-        if (st + AF_RING - 1 < stages) load_stage(st + AF_RING - 1);
+        if (st + 1 < stages) load_stage(st + 1);
         if (!live) continue;
         const int left = n - st * AF_KEYS - part * 16;        // keys of this part's blocks of the stage, and beyond
         if (split == 1) {
@@ -255,7 +250,7 @@ static int go_attention_f32(const void *q, int64_t q_rs, int64_t q_hs, const voi
                             int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs, int64_t o_hs,
                             int B, int h, int n, int max_rows, float scale, hipStream_t st)
 {
-    constexpr size_t lds = AF_RING * AttnF32<D>::BUF;
+    constexpr size_t lds = 2 * AttnF32<D>::BUF;
     const int64_t pairs = (int64_t)B * h, chunks = ceil_div(max_rows, 16 * AF_TILES);
     const int64_t grid = ceil_div(pairs, 8) * 8 * chunks;
     VT_REQUIRE(grid < (1ll << 31), VTDGE_ERR_UNSUPPORTED, "sparse_attention: %lld workgroups exceed one launch",
@@ -265,7 +260,7 @@ static int go_attention_f32(const void *q, int64_t q_rs, int64_t q_hs, const voi
     note_kernel(reinterpret_cast<const void *>(kern));
     kern<<<dim3((unsigned)grid), dim3(64 * AF_TILES), lds, st>>>(
         (const float *)q, q_rs, q_hs, (const float *)k, (const float *)v, kv_bs, kv_ts, kv_hs, offsets, (float *)out,
-        o_rs, o_hs, (int)pairs, h, n, (int)chunks, scale * 1.44269504088896340736f);
+        o_rs, o_hs, (int)pairs, h, n, scale * 1.44269504088896340736f);
     return check_launch("sparse_attention");
 }
 template <int D>

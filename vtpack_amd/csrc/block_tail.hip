@@ -16,8 +16,9 @@
 // bank conflicts.
 //
 // What bounds it: the GELU (11 vector instructions a hidden value: 69 us of the 103 below, 35 of 87, 10 of 35), the LDS reads
-// of the weights' fragments (one a matrix instruction, which is all LDS delivers) and a tile's first loads, in turns; two or
-// three waves a SIMD overlap them in part.  Measured against the launches it stands in for (rows, C, hidden):
+// of the weights' fragments (one a matrix instruction, which is all LDS delivers) and a tile's first loads, in turns.  Three
+// waves a SIMD at 64 channels and two at 128 overlap them in part; at 192 a workgroup takes 101 KB of LDS and more, so there is
+// one wave a SIMD.  Measured against the launches it stands in for (rows, C, hidden):
 //   459000,  64,  512: 103 against 393 us     7000: 13.5 against 27     1800: 13.5 against 16     200: 13.5 against 12
 //   115000, 128, 1024:  87 against 190        7000: 29.5 against 40     1800: 29.5 against 23
 //    29000, 192,  768:  35 against  69       14000: 33 against 45       3600: 32 against 34        800: 32 against 17
@@ -274,7 +275,9 @@ extern "C" int vtdge_block_tail(const void *o, const void *comp, const void *pro
     const TailArgs a{(const bf16_t *)o, (const bf16_t *)comp, (const bf16_t *)proj_weight, (const bf16_t *)proj_bias,
                      (const bf16_t *)ln_weight, (const bf16_t *)ln_bias, (const bf16_t *)fc1_weight, (const bf16_t *)fc1_bias,
                      (const bf16_t *)fc2_weight, (const bf16_t *)fc2_bias, (bf16_t *)out, rows_dev, rows, ln_eps, hidden};
-        hipStream_t st = (hipStream_t)stream;
+    hipStream_t st = (hipStream_t)stream;
+    // waves a SIMD the registers are held to: what LDS lets in at 64 and 128 channels; at 192, where that is one, two only
+    // keeps the kernel within 256 registers
     if (C == 64) return go<64, 4, 3>(a, st);
     if (C == 128) return go<128, 4, 2>(a, st);
     return go<192, 4, 2>(a, st);

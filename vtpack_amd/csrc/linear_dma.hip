@@ -405,12 +405,13 @@ int launch_patch_embed(const void *images, const void *W, const void *bias, cons
     LinArgs a{images, 0, W, bias, pos, N, out, N, nullptr, (int64_t)B * G * G, N, Cin * P * P, VTDGE_ACT_NONE, st};
     if (patch_small_wanted(a.rows, N, a.K, sizeof(T), (int64_t)B * Cin * S * S * sizeof(T)))
         return launch_patch_small<T>(images, W, bias, pos, out, a.rows, N, a.K, pg, st);
-    // 128x128 tiles, two workgroups per CU, unless the output is wide.  At 256 x 256 patches and N = 384 a launch takes
-    // 80 - 88 us against 125 - 138 us on 256x128 tiles with one workgroup per CU (which only looks faster, 67 against
-    // 78 us, when launches are timed back to back and the tail of one hides under the head of the next).
+    // bf16: 128x128 tiles, two workgroups per CU.  At 256 x 256 patches and N = 384 a launch takes 80 - 88 us against
+    // 125 - 138 us on 256x128 tiles with one workgroup per CU (which only looks faster, 67 against 78 us, when launches are
+    // timed back to back and the tail of one hides under the head of the next).
     // Eight loader waves instead of four (they also work out the patch addresses): 77.5 against 83.5 us; with two,
     // 201 us.  64x128 tiles: 108 us, 256x128 with eight loaders: 98 us; 128x64 with four and eight loaders 103 and 115,
-    // 128x128 in two stages 124; 128x192 78 us, but 73 against 65 at 25344 patches and N = 768.
+    // 128x128 in two stages 124; 128x192 78 us, but 73 against 65 at 25344 patches and N = 768.  fp32: the Linear's
+    // 64x64 tiles, which the instruction rate bounds and not the operands.
     if constexpr (sizeof(T) == 4) return go<T, 64, 64, 2, 2, 8, VTDGE_ACT_NONE, true, true, true>(a, pg);
     return go<T, 128, 128, 2, 2, 8, VTDGE_ACT_NONE, true, true, true>(a, pg);
 }

@@ -3,7 +3,7 @@
 // What bounds it is latency: below some thousand rows a Linear of these models has a few dozen tiles, each of them a
 // chain of dependent round trips (row count -> operands -> multiply, stage after stage -> store), and the 128-row tiles
 // of the streaming kernel give it few workgroups with long chains.  So here
-//   * tiles are 32 rows x 32 or 64 columns, for as many workgroups as the product has;
+//   * tiles are 32 rows x 32 columns, for as many workgroups as the product has;
 //   * the waves of a workgroup split K: wave w multiplies the 128-byte K slabs w, w + NW, ... of the whole tile, from a
 //     ring of its own in LDS that it fills by direct loads - as many slabs in flight as fit, no barrier in the K loop -
 //     and the partial tiles meet in LDS at the end.  Slab s always belongs to partial sum s mod 8 (four waves keep two
@@ -21,7 +21,7 @@
 
 namespace vtdge {
 
-constexpr int SM_BM = 32;            // rows of a tile
+constexpr int SM_BM = 32, SM_BN = 32;   // rows and columns of a tile
 constexpr int SM_PITCH = 68;         // floats between the accumulator registers of a partial tile in LDS (64 lanes + 4)
 
 struct SmallProblem {
@@ -54,18 +54,17 @@ template <int GS, int NV> __device__ __forceinline__ void small_group_sum(float 
 }
 
 // LN: 0, or how a row lies while it is normalised: the lanes that share it (up to 64), times the 16-byte vectors of each
-template <typename T, int BN, int NW, int ACT, int LN, bool PATCH>
+template <typename T, int NW, int ACT, int LN, bool PATCH>
 __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, SmallProblem p1, int K,
                                                                const T *__restrict__ ln_w, const T *__restrict__ ln_b,
                                                                float eps, PatchGeom pg, int ring)
 {
     constexpr int ESZ = sizeof(T), VEC = Elem<T>::VEC;
-    constexpr int JN = BN / 32;                              // 32-column blocks of the tile
-    constexpr int WROWS = LN ? BN : SM_BM + BN;              // rows of a ring slot
+    constexpr int WROWS = LN ? SM_BN : SM_BM + SM_BN;              // rows of a ring slot
     constexpr int NLW = WROWS / 8;                           // direct loads that fill it
     constexpr int GS = LN == 0 || LN > 64 ? 64 : LN, NV = LN > 64 ? LN / 64 : 1;
     constexpr int PARTS = 8, PW = PARTS / NW;                // partial sums of a tile, and a wave's share of them
-    constexpr int NQ = (8 * BN + NW * 64 - 1) / (NW * 64);   // four-column pieces of the output per thread
+    constexpr int NQ = (8 * SM_BN + NW * 64 - 1) / (NW * 64);   // four-column pieces of the output per thread
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
     const int total0 = p0.tiles_m * p0.tiles_n, total = total0 + p1.tiles_m * p1.tiles_n;
@@ -77,7 +76,7 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
     const SmallProblem &p = second ? p1 : p0;
     const int tiles_m = p.tiles_m, N = p.N;
     const bool down = !PATCH || ESZ == 4 || pg.cl_C == 0 || p.rows <= N;
-    const int m0 = (down ? v % tiles_m : v / p.tiles_n) * SM_BM, n0 = (down ? v / tiles_m : v % p.tiles_n) * BN;
+    const int m0 = (down ? v % tiles_m : v / p.tiles_n) * SM_BM, n0 = (down ? v / tiles_m : v % p.tiles_n) * SM_BN;
     const int M = (int)live_rows(p.rows_dev, p.rows);
     if (m0 >= M) return;
 
@@ -89,7 +88,7 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
     const uint32_t ring0 = (LN ? slabs * SM_BM * SLAB_BYTES : 0) + w * ring * WROWS * SLAB_BYTES;
 
     // per-lane source offsets: a direct load brings 8 rows of a slab, LDS slot c of row r holding chunk c ^ ((r >> 1) & 7)
-    uint32_t va[SM_BM / 8], vw[BN / 8];
+    uint32_t va[SM_BM / 8], vw[SM_BN / 8];
 #pragma unroll
     for (int i = 0; i < SM_BM / 8; i++) {
         const int r = i * 8 + (lane >> 3), chunk = (lane & 7) ^ ((r >> 1) & 7), row = min(m0 + r, M - 1);
@@ -97,7 +96,7 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
         else va[i] = (uint32_t)row * (uint32_t)(p.lda * ESZ) + chunk * 16;
     }
 #pragma unroll
-    for (int i = 0; i < BN / 8; i++) {
+    for (int i = 0; i < SM_BN / 8; i++) {
         const int r = i * 8 + (lane >> 3), chunk = (lane & 7) ^ ((r >> 1) & 7);
         vw[i] = (uint32_t)min(n0 + r, N - 1) * (uint32_t)(K * ESZ) + chunk * 16;
     }
@@ -117,7 +116,7 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
         }
         const void *base = uniform_ptr((const unsigned char *)p.W + (int64_t)slab * SLAB_BYTES);
 #pragma unroll
-        for (int i = 0; i < BN / 8; i++) dma16(base, vw[i], dst + i * 1024);
+        for (int i = 0; i < SM_BN / 8; i++) dma16(base, vw[i], dst + i * 1024);
     };
     if constexpr (LN)
         for (int j = 0; j < nj; j++) load_a(w + NW * j, lds0 + (uint32_t)(w + NW * j) * SM_BM * SLAB_BYTES);
@@ -197,19 +196,17 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
         lds_barrier();
     }
 
-    // ---- this wave's share of K.  acc[jn][v] = C[row lr][column 32 jn + 8 (v / 4) + 4 lg + v % 4]
+    // ---- this wave's share of K.  acc[v] = C[row lr][column 8 (v / 4) + 4 lg + v % 4]
     const int lr = lane & 31, lg = lane >> 5, sw = (lr >> 1) & 7;
     int cs[4];
 #pragma unroll
     for (int s = 0; s < 4; s++) cs[s] = lr * SLAB_BYTES + ((2 * s + lg) ^ sw) * 16;
-    f32x16 acc[PW][JN];
+    f32x16 acc[PW];
 #pragma unroll
     for (int h = 0; h < PW; h++)
 #pragma unroll
-        for (int jn = 0; jn < JN; jn++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) acc[h][jn][e] = 0.f;
-    auto multiply = [&](int j, f32x16 (&ac)[JN]) {
+        for (int e = 0; e < 16; e++) acc[h][e] = 0.f;
+    auto multiply = [&](int j, f32x16 &ac) {
         // the slab has landed once only the loads of the younger ones are outstanding
         const int younger = min(nj, j + ring) - 1 - j;
         if (younger >= 3) wait_vmcnt<3 * NLW>();
@@ -223,9 +220,7 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
 #pragma unroll
         for (int s = 0; s < 4; s++) {
             const u32x4 fa = *reinterpret_cast<const u32x4 *>(As + cs[s]);
-#pragma unroll
-            for (int jn = 0; jn < JN; jn++)
-                Slab<T>::mma(*reinterpret_cast<const u32x4 *>(Ws + jn * 32 * SLAB_BYTES + cs[s]), fa, ac[jn]);
+            Slab<T>::mma(*reinterpret_cast<const u32x4 *>(Ws + cs[s]), fa, ac);
         }
         if (j + ring < nj) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the slot has been read
@@ -243,23 +238,20 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
     lds_barrier();
 #pragma unroll
     for (int h = 0; h < PW; h++)
-#pragma unroll
-        for (int jn = 0; jn < JN; jn++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) sh[(((h * NW + w) * JN + jn) * 16 + e) * SM_PITCH + lane] = acc[h][jn][e];
+        for (int e = 0; e < 16; e++) sh[((h * NW + w) * 16 + e) * SM_PITCH + lane] = acc[h][e];
     lds_barrier();
 #pragma unroll
     for (int i = 0; i < NQ; i++) {
         const int qd = tid + i * NW * 64;
-        if (8 * BN % (NW * 64) != 0 && qd >= 8 * BN) return;
-        const int r = qd / (BN / 4), c4 = qd % (BN / 4), jn = c4 >> 3, src = (c4 & 1) * 32 + r, e0 = 4 * ((c4 & 7) >> 1);
+        if (8 * SM_BN % (NW * 64) != 0 && qd >= 8 * SM_BN) return;
+        const int r = qd / (SM_BN / 4), c4 = qd % (SM_BN / 4), src = (c4 & 1) * 32 + r, e0 = 4 * (c4 >> 1);
         const int row = m0 + r, col = n0 + 4 * c4;
         if (row >= M || col >= N) continue;
         float f[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ww = 0; ww < PARTS; ww++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) f[e] += sh[((ww * JN + jn) * 16 + e0 + e) * SM_PITCH + src];
+            for (int e = 0; e < 4; e++) f[e] += sh[(ww * 16 + e0 + e) * SM_PITCH + src];
         const int64_t orow = PATCH ? patch_out_row(pg, row) : row;
         if (p.bias != nullptr) {
 #pragma unroll
@@ -287,11 +279,11 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
 }
 
 // ----------------------------------------------------------------------------- host
-template <typename T, int BN, int NW, int ACT, int LN, bool PATCH>
+template <typename T, int NW, int ACT, int LN, bool PATCH>
 static int go_small(const SmallProblem &p0, const SmallProblem &p1, int K, const void *ln_w, const void *ln_b, float eps,
                     const PatchGeom &pg, hipStream_t st)
 {
-    constexpr int WROWS = LN ? BN : SM_BM + BN;
+    constexpr int WROWS = LN ? SM_BN : SM_BM + SM_BN;
     const int slabs = K * (int)sizeof(T) / SLAB_BYTES;
     const size_t a_bytes = LN ? (size_t)slabs * SM_BM * SLAB_BYTES : 0, slot = (size_t)NW * WROWS * SLAB_BYTES;
     // as many slots per wave as it has slabs, up to four, within half a compute unit's LDS (two workgroups share it)
@@ -300,10 +292,10 @@ static int go_small(const SmallProblem &p0, const SmallProblem &p1, int K, const
     ring = ring < 4 ? ring : 4;
     while (ring > (LN ? 1 : 2) && a_bytes + ring * slot > 80 * 1024) ring--;
     while (ring > 1 && a_bytes + ring * slot > 160 * 1024) ring--;
-    const size_t reduce = (size_t)8 * (BN / 32) * 16 * SM_PITCH * 4;
+    const size_t reduce = (size_t)8 * 16 * SM_PITCH * 4;
     const size_t lds = a_bytes + ring * slot > reduce ? a_bytes + ring * slot : reduce;
     VT_REQUIRE(lds <= 160 * 1024, VTDGE_ERR_UNSUPPORTED, "linear: %d values of K do not fit the LDS", K);
-    auto kern = linear_small_kernel<T, BN, NW, ACT, LN, PATCH>;
+    auto kern = linear_small_kernel<T, NW, ACT, LN, PATCH>;
     VT_RESERVE_LDS(kern, 160 * 1024, "linear");
     const int64_t total = (int64_t)p0.tiles_m * p0.tiles_n + (int64_t)p1.tiles_m * p1.tiles_n;
     note_kernel(reinterpret_cast<const void *>(kern));
@@ -313,10 +305,10 @@ static int go_small(const SmallProblem &p0, const SmallProblem &p1, int K, const
 }
 
 static SmallProblem small_problem(const void *A, int64_t lda, const void *W, const void *bias, const void *res, int64_t ldr,
-                                  void *out, int64_t ldo, const int64_t *rows_dev, int64_t rows, int N, int BN)
+                                  void *out, int64_t ldo, const int64_t *rows_dev, int64_t rows, int N)
 {
     return SmallProblem{A, W, bias, res, out, rows_dev, lda, ldr, ldo, (int)rows, N, (int)ceil_div(rows, SM_BM),
-                        (int)ceil_div(N, BN)};
+                        (int)ceil_div(N, SM_BN)};
 }
 
 // What the kernel needs of one problem: whole 128-byte slabs of K, four-column pieces of the output, 32-bit offsets.
@@ -345,7 +337,7 @@ bool linear_small_fits(int64_t lda, int64_t ldr, int64_t ldo, int64_t rows, int 
 //        1008 (1339, 768, 768) 23.7 / 31.4, 12.1 / 18.6    1020 (5435, 192, 768) 26.1 / 31.6, 19.3 / 18.1
 //        1398 (7451, 192, 192) 18.0 / 11.6, 10.9 / 7.5     2040 (5435, 384, 1536) 81.7 / 85.1, 52.0 / 33.1
 //        2700 (7195, 384, 384) 38.7 / 26.3, 25.4 / 17.9    4080 (13051, 320, 1280) 128.9 / 113.5, 70.4 / 48.3
-static int64_t small_tiles(int64_t rows, int N) { return ceil_div(rows, SM_BM) * ceil_div(N, 32); }
+static int64_t small_tiles(int64_t rows, int N) { return ceil_div(rows, SM_BM) * ceil_div(N, SM_BN); }
 bool linear_small_wanted(int64_t rows, int N, int K, int esz)
 {
     const int64_t most = esz == 4 || (N >= 768 && K >= 768) ? 1024 : N >= 256 ? 768 : 640;
@@ -358,10 +350,10 @@ int launch_linear_small(const void *A, int64_t lda, const void *W, const void *b
                         hipStream_t st)
 {
     const PatchGeom none{0, 0, 0, 0, 0, 0, 0, 0};
-    const SmallProblem p = small_problem(A, lda, W, bias, res, ldr, out, ldo, rows_dev, rows, N, 32);
+    const SmallProblem p = small_problem(A, lda, W, bias, res, ldr, out, ldo, rows_dev, rows, N);
     // eight waves where a tile has two slabs of K for each of them and there are too few tiles to fill the chip
     const bool deep = K * (int)sizeof(T) / SLAB_BYTES >= 16 && small_tiles(rows, N) <= 256;
-#define VT_SMALL(NW, ACT) return go_small<T, 32, NW, ACT, 0, false>(p, SmallProblem{}, K, nullptr, nullptr, 0.f, none, st)
+#define VT_SMALL(NW, ACT) return go_small<T, NW, ACT, 0, false>(p, SmallProblem{}, K, nullptr, nullptr, 0.f, none, st)
     if (act == VTDGE_ACT_GELU) {
         if (deep) VT_SMALL(8, VTDGE_ACT_GELU);
         VT_SMALL(4, VTDGE_ACT_GELU);
@@ -389,10 +381,10 @@ template <typename T>
 int launch_patch_small(const void *source, const void *W, const void *bias, const void *res, void *out, int64_t rows, int N,
                        int K, const PatchGeom &pg, hipStream_t st)
 {
-    const SmallProblem p = small_problem(source, 0, W, bias, res, N, out, N, nullptr, rows, N, 32);
+    const SmallProblem p = small_problem(source, 0, W, bias, res, N, out, N, nullptr, rows, N);
     if (K * (int)sizeof(T) / SLAB_BYTES >= 16 && small_tiles(rows, N) <= 256)
-        return go_small<T, 32, 8, VTDGE_ACT_NONE, 0, true>(p, SmallProblem{}, K, nullptr, nullptr, 0.f, pg, st);
-    return go_small<T, 32, 4, VTDGE_ACT_NONE, 0, true>(p, SmallProblem{}, K, nullptr, nullptr, 0.f, pg, st);
+        return go_small<T, 8, VTDGE_ACT_NONE, 0, true>(p, SmallProblem{}, K, nullptr, nullptr, 0.f, pg, st);
+    return go_small<T, 4, VTDGE_ACT_NONE, 0, true>(p, SmallProblem{}, K, nullptr, nullptr, 0.f, pg, st);
 }
 template int launch_patch_small<float>(const void *, const void *, const void *, const void *, void *, int64_t, int, int,
                                        const PatchGeom &, hipStream_t);
@@ -430,15 +422,15 @@ static int launch_layernorm_linear(const void *A0, int64_t lda0, const void *W0,
                                    int N1, const void *ln_w, const void *ln_b, float eps, int K, int act, hipStream_t st)
 {
     const PatchGeom none{0, 0, 0, 0, 0, 0, 0, 0};
-    const SmallProblem p0 = small_problem(A0, lda0, W0, bias0, nullptr, 0, out0, N0, rows_dev0, rows0, N0, 32);
-    const SmallProblem p1 = rows1 > 0 ? small_problem(A1, lda1, W1, bias1, nullptr, 0, out1, N1, rows_dev1, rows1, N1, 32)
+    const SmallProblem p0 = small_problem(A0, lda0, W0, bias0, nullptr, 0, out0, N0, rows_dev0, rows0, N0);
+    const SmallProblem p1 = rows1 > 0 ? small_problem(A1, lda1, W1, bias1, nullptr, 0, out1, N1, rows_dev1, rows1, N1)
                                       : SmallProblem{};
     const int vecs = K * (int)sizeof(T) / 16;
 #define VT_SMALL(LN)                                                                                                    \
     do {                                                                                                                \
         if (act == VTDGE_ACT_GELU)                                                                                      \
-            return go_small<T, 32, 8, VTDGE_ACT_GELU, LN, false>(p0, p1, K, ln_w, ln_b, eps, none, st);                 \
-        return go_small<T, 32, 8, VTDGE_ACT_NONE, LN, false>(p0, p1, K, ln_w, ln_b, eps, none, st);                     \
+            return go_small<T, 8, VTDGE_ACT_GELU, LN, false>(p0, p1, K, ln_w, ln_b, eps, none, st);                 \
+        return go_small<T, 8, VTDGE_ACT_NONE, LN, false>(p0, p1, K, ln_w, ln_b, eps, none, st);                     \
     } while (0)
     if (vecs <= 8) VT_SMALL(8);
     if (vecs <= 16) VT_SMALL(16);

@@ -845,13 +845,13 @@ def fits_block_tail(o, proj, ln, fc1, fc2):
                 and _lib.load().vtdge_block_tail_wanted(o.numel() // C, C, w.shape[0], dtype_code(o)))
 
 
-def block_tail(o, comp, proj, ln, ln_eps, fc1, fc2, rows_dev=None):
+def block_tail(o, comp, proj, ln, ln_eps, fc1, fc2, rows_dev=None, out=None):
     """q1 = o Wp^T + bp + comp -> q1 + fc2(gelu(fc1(LayerNorm(q1)))) as one kernel; proj, ln, fc1, fc2 = (weight, bias).
     See `fits_block_tail`."""
     C, hidden = o.shape[-1], fc1[0].shape[0]
     _need_gpu(o, comp, *proj, *ln, *fc1, *fc2)
     _check_like(o, comp=comp, proj=proj[0], proj_bias=proj[1], ln_weight=ln[0], ln_bias=ln[1], fc1=fc1[0], fc1_bias=fc1[1],
-                fc2=fc2[0], fc2_bias=fc2[1])
+                fc2=fc2[0], fc2_bias=fc2[1], out=out)
     for name, (w, b), shape in (("proj", proj, (C, C)), ("fc1", fc1, (hidden, C)), ("fc2", fc2, (C, hidden))):
         if tuple(w.shape) != shape:
             raise ValueError(f"{name} weight {tuple(w.shape)} is not {shape}")
@@ -862,7 +862,10 @@ def block_tail(o, comp, proj, ln, ln_eps, fc1, fc2, rows_dev=None):
         raise ValueError(f"comp {tuple(comp.shape)} is not like o {tuple(o.shape)}")
     o, comp = _contig(o), _contig(comp)
     vecs = [None if t is None else _contig(t) for t in (*proj, *ln, *fc1, *fc2)]
-    out = torch.empty_like(o)
+    if out is None:
+        out = torch.empty_like(o)
+    elif out.shape != o.shape or not out.is_contiguous():
+        raise ValueError(f"out {tuple(out.shape)} is not a dense tensor like o {tuple(o.shape)}")
     rows = o.numel() // C
     call("vtdge_block_tail", ptr(o), ptr(comp), *map(ptr, vecs[:4]), float(ln_eps), *map(ptr, vecs[4:]), ptr(out),
          ptr(rows_dev), rows, C, hidden, dtype_code(o), stream_ptr(), tag=("block_tail", rows, C, hidden, rows_dev is not None))
