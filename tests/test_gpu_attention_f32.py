@@ -1,5 +1,5 @@
 """fp32 attention of packed queries (16-query tiles, four a workgroup, waves that share a tile splitting its keys) at
-the sizes where its tiling turns: key counts around a block of 16 and a stage of 64, query counts around a tile, a pair
+the sizes where its tiling turns: key counts around a block of 16 and a stage of 32, query counts around a tile, a pair
 of tiles and a workgroup of four, and key counts that leave some parts of a split without a key."""
 import numpy as np
 import pytest
@@ -31,17 +31,19 @@ def test_tiles_and_key_stages(dev, n, d):
                  f"fp32 attention over {n} keys")
 
 
-@pytest.mark.parametrize("shape", ["ramp", "late spike", "early spike", "steps"])
+@pytest.mark.parametrize("shape", ["ramp", "late spike", "early spike", "steps", "stage"])
 def test_scores_far_above_the_first_stage(dev, shape):
-    """Running maxima that keep rising, one key hundreds above the rest, and jumps of 60 between stages, for tiles
-    that are whole (200 rows), split two ways (20) and four ways (5)."""
+    """Running maxima that keep rising, one key hundreds above the rest, and jumps of 60 between every second and the
+    next stage or from one stage of 32 keys to the next, for tiles of a wave each (200 rows: three
+    workgroups of four) and tiles whose keys two waves split (its last 8 rows, 20 and 5)."""
     h, d, n = 2, 64, 257
     lengths = np.array([200, 20, 5], dtype=np.int64)
     q, k, v = 0.05 * randn(910, h, 225, d), 0.05 * randn(911, h, 3, n, d), randn(912, h, 3, n, d)
     j = np.arange(n, dtype=np.float32)
     q[..., 0] = 8.0
     k[..., 0] = {"ramp": 0.25 * j, "late spike": np.where(j == n - 7, 300.0, 0.0),
-                 "early spike": np.where(j == 5, 300.0, 0.0), "steps": 60.0 * np.floor(j / 64)}[shape]
+                 "early spike": np.where(j == 5, 300.0, 0.0), "steps": 60.0 * np.floor(j / 64),
+                 "stage": np.where(j < 32, -60.0, 0.0)}[shape]
     got = _run(dev, q, k, v, lengths, 0.125)
     assert bool(torch.isfinite(got).all())
     # scores reach 300: their fp32 rounding (300 x 2^-24 in the exponent, both sides) is 4e-5 of a probability

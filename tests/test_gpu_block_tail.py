@@ -24,8 +24,10 @@ def test_against_float64(dev, C, hidden, rows, live, bias):
         g[i] = (g[i].float() * k ** -0.5).to(torch.bfloat16)
     o, comp, wp, bp, lw, lb, w1, b1, w2, b2 = [t.to(dev) for t in g]
     nb = [None] * 3 if not bias else [bp, b1, b2]
-    got = ops.block_tail(o, comp, (wp, nb[0]), (lw, lb), 1e-5, (w1, nb[1]), (w2, nb[2]),
-                         rows_dev=torch.tensor([live], device=dev))
+    got = torch.full_like(o, 7.0)
+    ops.block_tail(o, comp, (wp, nb[0]), (lw, lb), 1e-5, (w1, nb[1]), (w2, nb[2]),
+                   rows_dev=torch.tensor([live], device=dev), out=got)
+    assert bool((got[live:] == 7.0).all())                 # rows past the live ones are not written
     o, comp, wp, bp, lw, lb, w1, b1, w2, b2 = [t.double() for t in g]
     if not bias:
         bp, b1, b2 = bp * 0, b1 * 0, b2 * 0

@@ -3,6 +3,8 @@
 Integer outputs (gate indices, query counts, patch descriptors) are compared bit-exactly;
 floating point within the tolerances stated in tests/util.py.
 """
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -858,6 +860,49 @@ def test_scatter_back_with_the_next_router(dev, dtype, B, Hr, Wr, C, extra):
     assert torch.equal(alone, ops.decompress(q, patches[:L], x, W, extra, add_ref=True, sub=comp))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_divided_scatter_back_on_top_of_tokens(dev, dtype):
+    """vtdge_decompress_mean with its `add` operand: the quotient and the sum in fp32, rounded once."""
+    from vtpack_amd import _lib, ops
+    B, Hr, Wr, C, extra = 2, 3, 4, 192, 1
+    N, W = extra + 16 * Hr * Wr, 4 * Wr
+    idx = torch.from_numpy(random_indices(5, B, Hr, Wr)).to(dev)
+    patches, offsets, _ = ops.index_to_patch(idx, torch.tensor(SPLITS, device=dev), 4, extra)
+    patches = patches[:int(offsets[-1])]
+    rows, add = (_t(randn(s, *shape), dev, dtype) for s, shape in ((1, (len(patches), C)), (2, (B, N, C))))
+    out = torch.empty_like(add)
+    _lib.call("vtdge_decompress_mean", rows.data_ptr(), patches.data_ptr(), len(patches), add.data_ptr(), out.data_ptr(), B, N, C,
+              W, extra, _lib.dtype_code(rows), _lib.stream_ptr())
+    mean = rows.float() / patches[:, 3:4].square()
+    assert torch.equal(out, ops.decompress(mean, patches, add.float(), W, extra).to(dtype))
+    alone = ops.decompress(mean, patches, add.float(), W, extra, add_ref=False).to(dtype)
+    assert torch.equal(ops.decompress_mean(rows, patches, (B, N, C), W, extra), alone)
+
+
+@pytest.mark.parametrize("B,Hr,Wr,C,dtype,held", [
+    (1, 32, 32, 768, torch.bfloat16, True), (1, 25, 41, 768, torch.bfloat16, False), (66, 4, 4, 768, torch.bfloat16, False),
+    (1, 32, 32, 192, torch.float32, True), (66, 4, 4, 192, torch.float32, False), (2, 64, 64, 64, torch.bfloat16, True),
+    (2, 64, 65, 64, torch.bfloat16, False)])
+def test_scatter_back_around_a_workgroup_a_compute_unit(dev, B, Hr, Wr, C, dtype, held):
+    """256 workgroups and more: up to that the region's tokens are held in registers, beyond they are read in turn.  Both
+    against the two separate operators, bit for bit."""
+    from vtpack_amd import _lib, ops
+    H, W, extra = 4 * Hr, 4 * Wr, 1
+    g = torch.Generator(dev).manual_seed(B * 100 + C)
+    idx = torch.from_numpy(random_indices(B + C, B, Hr, Wr)).to(dev)
+    splits = torch.tensor(SPLITS, dtype=torch.int64, device=dev)
+    patches, offsets, _ = ops.index_to_patch(idx, splits, 4, extra)
+    L = int(offsets[-1])
+    q, comp, x = (torch.randn(*s, C, generator=g, device=dev).to(dtype) for s in ((L,), (L,), (B, extra + H * W)))
+    wgt = (torch.randn(3, C, generator=g, device=dev) / C ** 0.5).to(dtype)
+    bias = (torch.randn(3, generator=g, device=dev) * 0.1).to(dtype)
+    got, gate, nidx = ops.decompress_router(q, idx, splits, offsets, x, H, W, 4, sub=comp, next_weight=wgt, next_bias=bias)
+    assert re.search(r"decompress_route_kernel<.*, (true|false)>", _lib.last_kernel()).group(1) == str(held).lower()
+    want = ops.decompress(q, patches[:L], x, W, extra, add_ref=True, sub=comp)
+    want_gate, want_idx = ops.router(want, wgt, bias, H, W, 4)
+    assert torch.equal(got, want) and torch.equal(nidx, want_idx) and torch.equal(gate, want_gate)
+
+
 # ------------------------------------------------------------------ patch embedding
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("B,S,C,extra", [(3, 64, 192, 1), (2, 256, 384, 1), (2, 96, 768, 2), (5, 32, 64, 0)])
@@ -884,6 +929,25 @@ def test_patch_embed(dev, dtype, B, S, C, extra):
         patches = img.reshape(B, Cin, G, P, G, P).permute(0, 2, 4, 1, 3, 5).reshape(B * G * G, Cin * P * P)
         old = ops.linear(patches, w.reshape(C, -1), b).view(B, G * G, C) + pos[:, extra:]
         assert torch.equal(out[:, extra:], old)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_patch_embed_of_many_patches(dev, dtype):
+    """The streaming kernel (8036 patches): a ragged last tile of rows and of columns, rows in front of every sample."""
+    from vtpack_amd import _lib, ops
+    B, S, C, extra, P, Cin, G = 41, 224, 392, 1, 16, 3, 14
+    g = torch.Generator(dev).manual_seed(7)
+    img = torch.rand(B, Cin, S, S, generator=g, device=dev).to(dtype)
+    w = (torch.randn(C, Cin, P, P, generator=g, device=dev) * 0.05).to(dtype)
+    b, pos = ((torch.randn(*s, C, generator=g, device=dev) * 0.3).to(dtype) for s in ((), (1, extra + G * G)))
+    out = torch.full((B, extra + G * G, C), 7.0, dtype=dtype, device=dev)
+    ops.patch_embed(img, w, b, pos, P, extra, out=out)
+    assert "linear_dma" in _lib.last_kernel()
+    assert bool((out[:, :extra] == 7.0).all())
+    patches = img.view(B, Cin, G, P, G, P).permute(0, 2, 4, 1, 3, 5).reshape(B * G * G, Cin * P * P)
+    want = (patches.double() @ w.view(C, -1).double().T + b.double()).view(B, G * G, C) + pos.double()[:, extra:]
+    # one rounding of the result in bf16; sums of 768 products in fp32
+    assert rel_err(out[:, extra:], want.cpu()) <= (1e-5 if dtype == torch.float32 else 2 ** -8)
 
 
 def test_patch_embed_refusals(dev):
