@@ -90,6 +90,26 @@ def _fake_states(model, gate_index):
         blk.dge.states.update({"input": torch.zeros(B, N, C), "gate": gate, "num_extra_tokens": 1})
 
 
+@pytest.mark.parametrize("away", ["k", "v"])
+def test_sparse_training_attention_refuses_keys_that_are_not_on_the_gpu(monkeypatch, away):
+    """Queries on the GPU, keys or values on the CPU: refused, as the composition of products does, before any kernel."""
+    from vtpack_amd import ops
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+
+    class OnGpu(torch.Tensor):          # stands for a tensor on the GPU
+        is_cuda = property(lambda self: True)
+        device = property(lambda self: torch.device("cuda", 0))
+
+    def launched(*args, **kw):
+        raise AssertionError("a kernel was handed an address of host memory")
+    for name in ("lengths_to_offsets", "sparse_attention_heads"):
+        monkeypatch.setattr(ops, name, launched)
+    t = {"q": torch.zeros(2, 5, 64), "k": torch.zeros(2, 2, 7, 64), "v": torch.zeros(2, 2, 7, 64)}
+    args = [x if name == away else x.as_subclass(OnGpu) for name, x in t.items()]
+    with pytest.raises(RuntimeError, match="GPU only"):
+        sparse_attention_train(*args, torch.tensor([2, 3]), 0.125)
+
+
 @pytest.mark.parametrize("factory,macs", [("deit_dge_s124_small_patch16_256", 6.1e9),
                                           ("deit_dge_s124_tiny_patch16_256", 1.7e9)])
 def test_complexity_counter_reproduces_published_macs(factory, macs):

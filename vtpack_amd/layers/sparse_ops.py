@@ -49,6 +49,7 @@ class _SparseAttentionTrain(Function):
 
     @staticmethod
     def forward(ctx, q, k, v, q_lengths, scale):
+        ops._need_gpu(q, k, v)
         q, k, v = (ops.on_boundary(t) for t in (ops.vector_rows(q), k.contiguous(), v.contiguous()))
         h, L, d = q.shape
         offsets, lengths = ops.lengths_to_offsets(q_lengths, q.device)
