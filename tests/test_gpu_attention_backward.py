@@ -134,6 +134,27 @@ def test_an_infinite_gradient_of_the_last_query(dev, dtype, length):
     assert float((dv - grads[2])[~inf].abs().max()) <= TOL[dtype] * float(grads[2][~inf].abs().max())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("which", ["k", "v"])
+@pytest.mark.parametrize("n", [5, 64, 257])
+def test_a_key_or_value_that_is_nan(dev, dtype, which, n):
+    """A NaN in the last key or value (at 5 keys the only one some lanes hold) is NaN in every gradient of its sample
+    that it is in for the composition, and in none of the other sample's."""
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    h, lengths = 2, [19, 7]
+    L = sum(lengths)
+    t = {name: torch.from_numpy(randn(i, *s)).to(dtype)
+         for i, (name, s) in enumerate({"q": (h, L, 64), "k": (h, 2, n, 64), "v": (h, 2, n, 64), "g": (L, h * 64)}.items())}
+    t[which][:, 0, n - 1, 7] = float("nan")
+    want, grads = _reference(t["q"], t["k"], t["v"], lengths, 0.125, t["g"])
+    args = [t[name].to(dev).requires_grad_(True) for name in "qkv"]
+    got = sparse_attention_train(*args, torch.tensor(lengths), 0.125)
+    for a, b in zip((got.detach(),) + torch.autograd.grad(got, args, t["g"].to(dev)), (want,) + grads):
+        a, nan = a.double().cpu(), torch.isnan(b)
+        assert torch.equal(torch.isnan(a), nan)
+        assert float((a - b)[~nan].abs().max()) <= TOL[dtype] * float(b[~nan].abs().max())
+
+
 def test_scores_are_those_of_the_queries_as_given(dev):
     """Scores of spread 8 in bf16: a query rounded once more, times the scale, would be off by 2^-9 / sqrt(3) of its score,
     i.e. 9e-3 of a probability.  What remains are the roundings of the probabilities and of the result, 1.1e-3 each."""

@@ -307,20 +307,19 @@ template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_ker
                 mx = fmaxf(mx, t[blk][r]);
             }
         }
-        if (mx > -INFINITY) {
-            const float down = __builtin_amdgcn_exp2f(m - mx);
-            s *= down;
-            sd *= down;
+        // (a maximum leaves NaN out, and a lane's keys may be one that is NaN and keys past the last: those are summed too)
+        const float ref = mx == -INFINITY ? 0.f : mx, down = __builtin_amdgcn_exp2f(m - ref);
+        s *= down;
+        sd *= down;
 #pragma unroll
-            for (int blk = 0; blk < 2; blk++)
+        for (int blk = 0; blk < 2; blk++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float e = __builtin_amdgcn_exp2f(t[blk][r] - mx);
-                    s += e;
-                    sd += e * dp[blk][r];
-                }
-            m = mx;
-        }
+            for (int r = 0; r < 4; r++) {
+                const float e = __builtin_amdgcn_exp2f(t[blk][r] - ref);
+                s += e;
+                sd += e * dp[blk][r];
+            }
+        m = mx;
     }
     float all = fmaxf(m, __shfl_xor(m, 16, WAVE));
     all = fmaxf(all, __shfl_xor(all, 32, WAVE));
