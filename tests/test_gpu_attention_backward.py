@@ -69,6 +69,28 @@ def test_keys_and_values_with_a_common_component(dev, dtype, common):
         assert float((a.double().cpu() - b).norm()) <= (1e-5 if dtype == torch.float32 else 1e-2) * float(b.norm()), name
 
 
+@pytest.mark.parametrize("size,common", [(1.0, 0.0), (4.0, 0.0), (16.0, 0.0), (1.0, 2.0)])
+def test_fp32_gradients_are_as_exact_as_the_composition(dev, size, common):
+    """Against float64, beside a softmax and products in fp32 on the same operands.  Rounding m + log2(s) at its own size would
+    put 2e-7 into every P of a row, 1.4 times the composition's error of dV at size = 1; an exponent that is rounded before the
+    subtraction in one pass and not in the other, as much at size = 16; sums of e dP key by key, 1.6 times its error of dQ at
+    common = 2.  Bound: a tenth above the composition, for the spread of two rms errors over 324 rows, 1 / sqrt(2 * 324) each."""
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    h, n, lengths = 3, 257, [113, 17, 64, 130]
+    L, B = sum(lengths), len(lengths)
+    q, g = (torch.from_numpy(f * randn(s, L, h * 64)) for s, f in ((1, size), (4, 1.0)))
+    q = q.view(L, h, 64).transpose(0, 1)
+    k, v = (torch.from_numpy(randn(s, h, B, n, 64) + common * randn(s + 7, h, 1, 1, 64)) for s in (2, 3))
+    want, grads = _reference(q, k, v, lengths, 0.125, g)
+    args = [t.to(dev).requires_grad_(True) for t in (q, k, v)]
+    lens = torch.tensor(lengths)
+    got = [torch.autograd.grad(sparse_attention_train(*args, lens, scale), args, g.to(dev))
+           for scale in (0.125, torch.tensor(0.125, device=dev))]      # a scale that is a tensor: the composition
+    for name, ours, theirs, b in zip("qkv", *got, grads):
+        err, ref = (float((a.double().cpu() - b).norm() / b.norm()) for a in (ours, theirs))
+        assert err <= 1.1 * ref, (name, err, ref)
+
+
 @pytest.mark.parametrize("which", ["q", "k", "v", "grad", "hook"])
 def test_operands_off_a_16_byte_boundary(dev, which):
     """Operands that start 4 bytes behind a boundary, and saved tensors that come back from a hook that way."""
@@ -234,3 +256,27 @@ def test_offsets_of_lengths(dev, B):
         lengths[:448] = 0
     got, _ = ops.lengths_to_offsets(lengths, dev)
     assert torch.equal(got.cpu(), torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_from_a_workspace_of_two_floats_a_row(dev, dtype):
+    """The C entry whose workspace holds m + log2(s) and delta only; nothing is written behind it.  In bf16 both entries keep
+    these two and agree to the last bit."""
+    from vtpack_amd import _lib, ops
+    h, n, lengths = 2, 65, [17, 0, 64]
+    L, B = sum(lengths), len(lengths)
+    q, g = (torch.from_numpy(randn(s, h, L, 64)).to(dtype) for s in (1, 4))
+    k, v = (torch.from_numpy(randn(s, h, B, n, 64)).to(dtype) for s in (2, 3))
+    _, grads = _reference(q, k, v, lengths, 0.125, g.transpose(0, 1).reshape(L, h * 64))
+    q, k, v, g = (t.to(dev) for t in (q, k, v, g))
+    offsets, _ = ops.lengths_to_offsets(torch.tensor(lengths), dev)
+    work = torch.full((2 * h * L + 64,), 7.0, device=dev)
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    q_st, kv_st = (64, L * 64), (n * 64, 64, B * n * 64)
+    _lib.call("vtdge_sparse_attention_backward", q.data_ptr(), *q_st, k.data_ptr(), v.data_ptr(), *kv_st, 0, g.data_ptr(), *q_st,
+              offsets.data_ptr(), dq.data_ptr(), *q_st, dk.data_ptr(), dv.data_ptr(), *kv_st, work.data_ptr(), L, B, h, 64, n,
+              64, 0.125, _lib.dtype_code(q), _lib.stream_ptr())
+    assert (work[2 * h * L:] == 7).all()
+    for name, a, b, c in zip("qkv", (dq, dk, dv), ops.sparse_attention_backward(q, k, v, None, g, offsets, 0.125, 64), grads):
+        assert float((a.double().cpu() - c).abs().max()) <= TOL[dtype] * float(c.abs().max()), name
+        assert dtype == torch.float32 or torch.equal(a, b), name

@@ -65,6 +65,8 @@ SIGNATURES = {
     "vtdge_sparse_attention_train": [_p, _l, _l, _p, _p, _l, _l, _l, _p, _p, _l, _l, _i, _i, _i, _i, _i, _f, _i, _p],
     "vtdge_sparse_attention_backward": [_p, _l, _l, _p, _p, _l, _l, _l, _p, _p, _l, _l, _p, _p, _l, _l, _p, _p, _l, _l, _l, _p,
                                         _l, _i, _i, _i, _i, _i, _f, _i, _p],
+    "vtdge_sparse_attention_train_backward": [_p, _l, _l, _p, _p, _l, _l, _l, _p, _l, _l, _p, _p, _l, _l, _p, _p, _l, _l, _l, _p,
+                                              _l, _i, _i, _i, _i, _i, _f, _i, _p],
     "vtdge_lengths_to_offsets": [_p, _i, _p, _p],
     "vtdge_layernorm_linear_fits": [_l, _i, _l, _i, _i, _i],
     "vtdge_layernorm_linear_wanted": [_l, _i, _l, _i, _i, _i],

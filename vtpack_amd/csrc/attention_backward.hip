@@ -4,10 +4,14 @@
 // five products backward: vtpack/models/dge/deit_dge.py:86-95) keeps four score-sized tensors in HBM, [heads, L, n] each:
 // 90 MB apiece at 14500 queries, 6 heads and 257 keys in bf16, against 45 MB of operands.  Here scores exist in registers
 // only: they are worked out again from Q and K where a gradient needs them,
-//   P = exp2(scale log2e q.k - lse),   dP = dO.v,   dS = P (dP - delta) scale,   delta = sum_k P dP,
+//   P = exp2(scale log2e q.k - m) / s,   dP = dO.v,   dS = P (dP - delta) scale,   delta = sum_k P dP,
 //   dQ = dS K,   dV = P^T dO,   dK = dS^T Q.
-// Two kernels, no atomics, so the result is the same bytes on every call: one over query tiles, which first finds lse (the
-// row's maximum plus the log of its sum, in log2 units) and delta and leaves both for the other, over key tiles.
+// Two kernels, no atomics, so the result is the same bytes on every call: one over query tiles, which first finds m (the
+// row's maximum in log2 units), s (the sum of its exponentials) and delta and leaves them for the other, over key tiles.
+// m and 1 / s stay apart: added up to m + log2(s), rounded at its own size (8 to 9 with 257 keys), they would put 2e-7 into
+// every P of a row and the subtraction as much again (fp32, 64 samples, 3 heads, 257 keys, unit normals: relative error of dV
+// 4.2e-7 against 3.0e-7 this way; a softmax and products 2.9e-7).  In bf16, where P is rounded to 2^-9, they are added up.
+// Every exponent is one fused multiply-add: the passes have to see the same e, or dS does not add up to zero.
 // delta equals dO.O, but is summed from the P and dP that dS is made of: a row of dS then adds up to zero within fp32, where
 // dO times an output rounded to bf16 leaves a remainder that multiplies the mean key (relative error of dQ with a common
 // component of twice the spread in keys and values: 5.1e-2 from the rounded output, 3.6e-3 this way).
@@ -140,7 +144,7 @@ struct AttnTrain {
 struct AttnBack {
     const void *q, *k, *v, *dout;
     void *dq, *dk, *dv;
-    float *lse, *delta;                                   // [h, L] each
+    float *m, *inv, *delta;                               // [h, L] each; bf16, or inv NULL: m + log2(s) in m's place
     const int64_t *offsets;
     int64_t q_rs, q_hs, kv_bs, kv_ts, kv_hs, o_rs, o_hs, dq_rs, dq_hs, dkv_bs, dkv_ts, dkv_hs, L;
     int pairs, h, n;
@@ -257,7 +261,7 @@ __global__ __launch_bounds__(256, 4) void attention_train_kernel(AttnTrain a)
     if (live) M::store(a.out + (row0 + row) * a.o_rs + (int64_t)head * a.o_hs, o, g);
 }
 
-// dQ of 64 query rows of one (sample, head), with their lse and delta
+// dQ of 64 query rows of one (sample, head), with their m, 1 / s and delta
 template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_kernel(AttnBack a)
 {
     using B = BackTile<T>;
@@ -284,7 +288,7 @@ template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_ker
     typename M::Frag qf[B::NF], df[B::NF];
     load_kept<T>(qf, (const T *)a.q + (row0 + row) * a.q_rs + (int64_t)head * a.q_hs, live, g);
     load_kept<T>(df, (const T *)a.dout + (row0 + row) * a.o_rs + (int64_t)head * a.o_hs, live, g);
-    // ---- lse and delta of this lane's query: maximum, sum of e and sum of e dP over the lane's keys, then over the four
+    // ---- m, s and delta of this lane's query: maximum, sum of e and sum of e dP over the lane's keys, then over the four
     // lanes that share the query
     float m = -INFINITY, s = 0.f, sd = 0.f;
     for (int st = 0; st < stages; st++) {
@@ -302,23 +306,24 @@ template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_ker
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const bool in = st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
-                t[blk][r] = in ? t[blk][r] * a.scale_log2 : -INFINITY;
                 dp[blk][r] = in ? dp[blk][r] : 0.f;
-                mx = fmaxf(mx, t[blk][r]);
+                mx = fmaxf(mx, in ? t[blk][r] * a.scale_log2 : -INFINITY);
             }
         }
         // (a maximum leaves NaN out, and a lane's keys may be one that is NaN and keys past the last: those are summed too)
         const float ref = mx == -INFINITY ? 0.f : mx, down = __builtin_amdgcn_exp2f(m - ref);
-        s *= down;
-        sd *= down;
+        // a stage's eight keys in pairs first: fewer roundings in a row than key by key
+        f32x4 e[2], ed[2];
 #pragma unroll
         for (int blk = 0; blk < 2; blk++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const float e = __builtin_amdgcn_exp2f(t[blk][r] - ref);
-                s += e;
-                sd += e * dp[blk][r];
+                const bool in = st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
+                e[blk][r] = in ? __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -ref)) : 0.f;
+                ed[blk][r] = e[blk][r] * dp[blk][r];
             }
+        s = s * down + (((e[0][0] + e[0][1]) + (e[0][2] + e[0][3])) + ((e[1][0] + e[1][1]) + (e[1][2] + e[1][3])));
+        sd = sd * down + (((ed[0][0] + ed[0][1]) + (ed[0][2] + ed[0][3])) + ((ed[1][0] + ed[1][1]) + (ed[1][2] + ed[1][3])));
         m = mx;
     }
     float all = fmaxf(m, __shfl_xor(m, 16, WAVE));
@@ -330,11 +335,13 @@ template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_ker
     sd += __shfl_xor(sd, 16, WAVE);
     s += __shfl_xor(s, 32, WAVE);
     sd += __shfl_xor(sd, 32, WAVE);
-    const float lse = all + __builtin_amdgcn_logf(s);     // v_log_f32: base 2
-    const float delta = sd / s;
+    const float inv = 1.0f / s, delta = sd / s, scale_s = a.scale * inv;
     if (live && g == 0) {
-        a.lse[(int64_t)head * a.L + row0 + row] = lse;
-        a.delta[(int64_t)head * a.L + row0 + row] = delta;
+        const int64_t at = (int64_t)head * a.L + row0 + row;
+        const bool apart = sizeof(T) == 4 && a.inv != nullptr;
+        a.m[at] = apart ? all : all + __builtin_amdgcn_logf(s);                 // v_log_f32: base 2
+        if (apart) a.inv[at] = inv;
+        a.delta[at] = delta;
     }
 
     // ---- dQ^T += K^T dS^T
@@ -356,8 +363,8 @@ template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_ker
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const bool in = st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
-                const float p = __builtin_amdgcn_exp2f(t[r] * a.scale_log2 - lse);
-                ds[blk][r] = in ? p * (dp[r] - delta) * a.scale : 0.f;
+                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(t[r], a.scale_log2, -all));
+                ds[blk][r] = in ? e * (dp[r] - delta) * scale_s : 0.f;
             }
         }
         M::accumulate(Ks, ds, dq, l, g);
@@ -386,16 +393,19 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
     const Stager<T> qd{wid < 2 ? reinterpret_cast<const unsigned char *>((const T *)a.q + row0 * a.q_rs + (int64_t)head * a.q_hs)
                                : reinterpret_cast<const unsigned char *>((const T *)a.dout + row0 * a.o_rs + (int64_t)head * a.o_hs),
                        (uint32_t)((wid < 2 ? a.q_rs : a.o_rs) * sizeof(T)), (uint32_t)(uintptr_t)smem, Lb, wid, lane};
-    const float *lse = a.lse + (int64_t)head * a.L + row0, *delta = a.delta + (int64_t)head * a.L + row0;
-    // lse and delta of the lane's walked rows, one stage ahead; rows past the sample's last query: probability zero
-    f32x4 nls[2], ndl[2];
+    const int64_t stat = (int64_t)head * a.L + row0;
+    const bool apart = sizeof(T) == 4 && a.inv != nullptr;
+    const float *rm = a.m + stat, *rinv = apart ? a.inv + stat : nullptr, *delta = a.delta + stat;
+    // m, 1 / s and delta of the lane's walked rows, one stage ahead; rows past the sample's last query: probability zero
+    f32x4 nm[2], niv[2], ndl[2];
     auto fetch = [&](int st) {
 #pragma unroll
         for (int blk = 0; blk < 2; blk++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int i = st * AB_ROWS + 16 * blk + 4 * g + r;
-                nls[blk][r] = i < Lb ? lse[i] : INFINITY;
+                nm[blk][r] = i < Lb ? rm[i] : INFINITY;
+                niv[blk][r] = apart && i < Lb ? rinv[i] : 1.f;
                 ndl[blk][r] = i < Lb ? delta[i] : 0.f;
             }
     };
@@ -414,7 +424,7 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
     for (int st = 0; st < stages; st++) {
         wait_vmcnt<0>();
         block_barrier();
-        const f32x4 ls[2] = {nls[0], nls[1]}, dl[2] = {ndl[0], ndl[1]};
+        const f32x4 ms[2] = {nm[0], nm[1]}, iv[2] = {niv[0], niv[1]}, dl[2] = {ndl[0], ndl[1]};
         if (st + 1 < stages) {
             qd.load(st + 1);
             if (wave_live) fetch(st + 1);
@@ -433,7 +443,7 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
             const f32x4 t = M::scores(Qs, blk, kf, l, g), dp = M::scores(Ds, blk, vf, l, g);
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                p[blk][r] = __builtin_amdgcn_exp2f(t[r] * a.scale_log2 - ls[blk][r]);
+                p[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[r], a.scale_log2, -ms[blk][r])) * iv[blk][r];
                 ds[blk][r] = p[blk][r] * (dp[r] - dl[blk][r]) * a.scale;
             }
         }
@@ -545,12 +555,12 @@ extern "C" int vtdge_sparse_attention_train(const void *q, int64_t q_row_stride,
     return check_launch("sparse_attention_train");
 }
 
-extern "C" int vtdge_sparse_attention_backward(
-    const void *q, int64_t q_row_stride, int64_t q_head_stride, const void *k, const void *v, int64_t kv_batch_stride,
-    int64_t kv_tok_stride, int64_t kv_head_stride, const void *out, const void *dout, int64_t o_row_stride,
-    int64_t o_head_stride, const int64_t *offsets, void *dq, int64_t dq_row_stride, int64_t dq_head_stride, void *dk,
-    void *dv, int64_t dkv_batch_stride, int64_t dkv_tok_stride, int64_t dkv_head_stride, float *workspace, int64_t L, int B,
-    int h, int d, int n, int max_rows_per_sample, float scale, int dtype, void *stream)
+static int backward(const void *q, int64_t q_row_stride, int64_t q_head_stride, const void *k, const void *v,
+                    int64_t kv_batch_stride, int64_t kv_tok_stride, int64_t kv_head_stride, const void *dout,
+                    int64_t o_row_stride, int64_t o_head_stride, const int64_t *offsets, void *dq, int64_t dq_row_stride,
+                    int64_t dq_head_stride, void *dk, void *dv, int64_t dkv_batch_stride, int64_t dkv_tok_stride,
+                    int64_t dkv_head_stride, float *workspace, bool apart, int64_t L, int B, int h, int d, int n,
+                    int max_rows_per_sample, float scale, int dtype, void *stream)
 {
     VT_REQUIRE(k && v && offsets && dk && dv && (L == 0 || (q && dout && dq && workspace)), VTDGE_ERR_ARG,
                "sparse_attention_backward: NULL operand");
@@ -569,10 +579,36 @@ extern "C" int vtdge_sparse_attention_backward(
     VT_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)dout | (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) &
                 15) == 0,
                VTDGE_ERR_ARG, "sparse_attention_backward: operands must be 16-byte aligned");
-    AttnBack a{q, k, v, dout, dq, dk, dv, workspace, workspace + (int64_t)h * L, offsets, q_row_stride, q_head_stride,
-               kv_batch_stride, kv_tok_stride, kv_head_stride, o_row_stride, o_head_stride, dq_row_stride, dq_head_stride,
+    float *last = workspace + (int64_t)h * L;
+    AttnBack a{q, k, v, dout, dq, dk, dv, workspace, apart ? last : nullptr, apart ? last + (int64_t)h * L : last, offsets,
+               q_row_stride, q_head_stride, kv_batch_stride, kv_tok_stride, kv_head_stride, o_row_stride, o_head_stride, dq_row_stride, dq_head_stride,
                dkv_batch_stride, dkv_tok_stride, dkv_head_stride, L, B * h, h, n, scale,
                scale * 1.44269504088896340736f};
     if (dtype == VTDGE_F32) return launch_backward<float>(a, max_rows_per_sample, (hipStream_t)stream);
     return launch_backward<bf16_t>(a, max_rows_per_sample, (hipStream_t)stream);
+}
+
+extern "C" int vtdge_sparse_attention_backward(
+    const void *q, int64_t q_row_stride, int64_t q_head_stride, const void *k, const void *v, int64_t kv_batch_stride,
+    int64_t kv_tok_stride, int64_t kv_head_stride, const void *out, const void *dout, int64_t o_row_stride,
+    int64_t o_head_stride, const int64_t *offsets, void *dq, int64_t dq_row_stride, int64_t dq_head_stride, void *dk,
+    void *dv, int64_t dkv_batch_stride, int64_t dkv_tok_stride, int64_t dkv_head_stride, float *workspace, int64_t L, int B,
+    int h, int d, int n, int max_rows_per_sample, float scale, int dtype, void *stream)
+{
+    (void)out;
+    return backward(q, q_row_stride, q_head_stride, k, v, kv_batch_stride, kv_tok_stride, kv_head_stride, dout, o_row_stride,
+                    o_head_stride, offsets, dq, dq_row_stride, dq_head_stride, dk, dv, dkv_batch_stride, dkv_tok_stride,
+                    dkv_head_stride, workspace, false, L, B, h, d, n, max_rows_per_sample, scale, dtype, stream);
+}
+
+extern "C" int vtdge_sparse_attention_train_backward(
+    const void *q, int64_t q_row_stride, int64_t q_head_stride, const void *k, const void *v, int64_t kv_batch_stride,
+    int64_t kv_tok_stride, int64_t kv_head_stride, const void *dout, int64_t o_row_stride, int64_t o_head_stride,
+    const int64_t *offsets, void *dq, int64_t dq_row_stride, int64_t dq_head_stride, void *dk, void *dv,
+    int64_t dkv_batch_stride, int64_t dkv_tok_stride, int64_t dkv_head_stride, float *workspace, int64_t L, int B, int h, int d,
+    int n, int max_rows_per_sample, float scale, int dtype, void *stream)
+{
+    return backward(q, q_row_stride, q_head_stride, k, v, kv_batch_stride, kv_tok_stride, kv_head_stride, dout, o_row_stride,
+                    o_head_stride, offsets, dq, dq_row_stride, dq_head_stride, dk, dv, dkv_batch_stride, dkv_tok_stride,
+                    dkv_head_stride, workspace, true, L, B, h, d, n, max_rows_per_sample, scale, dtype, stream);
 }

@@ -951,9 +951,9 @@ def sparse_attention_backward(q, k, v, out, grad, offsets, scale, max_rows_per_s
     B, n = k.shape[1], k.shape[2]
     dq = torch.empty((L, h, d), dtype=q.dtype, device=q.device).transpose(0, 1)
     dk, dv = torch.empty_like(k), torch.empty_like(v)
-    work = torch.empty((2 * h * L,), dtype=torch.float32, device=q.device)
+    work = torch.empty((3 * h * L,), dtype=torch.float32, device=q.device)
     qs, ks, gs, dqs, dks = (steps(t) for t in (q, k, grad, dq, dk))
-    call("vtdge_sparse_attention_backward", ptr(q), qs[1], qs[0], ptr(k), ptr(v), ks[1], ks[2], ks[0], 0, ptr(grad), gs[1],
+    call("vtdge_sparse_attention_train_backward", ptr(q), qs[1], qs[0], ptr(k), ptr(v), ks[1], ks[2], ks[0], ptr(grad), gs[1],
          gs[0], ptr(offsets), ptr(dq), dqs[1], dqs[0], ptr(dk), ptr(dv), dks[1], dks[2], dks[0], ptr(work), L, B, h, d,
          n, max_rows_per_sample, float(scale), dtype_code(q), stream_ptr(), tag=("attention_backward", B, h, d, n))
     return dq, dk, dv
