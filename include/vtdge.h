@@ -307,6 +307,20 @@ int vtdge_linear_prepacked(const void *A, int64_t lda, const void *W, const void
                            const void *residual, int64_t ldr, void *out, int64_t ldo, const int64_t *rows_dev,
                            int64_t rows, int N, int K, int act, int dtype, void *stream);
 
+/* fp32 Linears on the bf16 matrix instructions: for VTDGE_F32, `packed` of vtdge_linear_prepacked is a copy of W split into
+ * three bf16 parts (6 bytes a value).  The sums of all partial products of weight 2^-18 and above, in fp32, are as exact as
+ * those of the fp32 instructions (not the same bits) and 1.2 to 1.5 times as fast.
+ *   vtdge_linear_split_size    *bytes = size of the split copy of W [N, K], or 0 when there is none (N no multiple of 64, K
+ *                              none of 32)
+ *   vtdge_linear_split         fills `split` (16-byte aligned, *bytes long) from W; VTDGE_ERR_UNSUPPORTED where the size is 0
+ *   vtdge_linear_split_wanted  1 where vtdge_linear_prepacked uses the copy for that many rows, 0 where W is multiplied as it
+ *                              is, with or without one
+ * W itself is always required: blocks of the result with infinities, NaN or values outside the range of the split are
+ * worked out from it. */
+int vtdge_linear_split_size(int N, int K, int64_t *bytes);
+int vtdge_linear_split(const void *W, int N, int K, void *split, void *stream);
+int vtdge_linear_split_wanted(int64_t rows, int N, int K);
+
 /* Patch embedding, position embedding included: the stride-P P x P convolution of the reference's PatchEmbed
  * (nn.Conv2d, vtpack/models/dge/deit_dge.py:141-155) as a Linear over the patches, read straight from the images
  * (no unfolded copy), with the addition of the position table (x = x + pos_embed, deit_dge.py:277) in its epilogue:

@@ -215,7 +215,9 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
         char *kv = scratch + p.kv, *q = scratch + p.q, *o = scratch + p.o, *q1 = scratch + p.q1, *hid = scratch + p.hid;
         char *xout = Q ? big + p.tok0 + i * p.tok_sz : out;
         char *ngate = Q ? ints + p.gate0 + (i + 1) * p.gate_sz : nullptr;
-        auto pk = [&](int which) { return p.rows >= 2048 ? P[which] : nullptr; };
+        // the copy of a weight for so many rows: bf16 packed (made from 2048 rows on), fp32 split
+        auto copy_for = [&](int which, int64_t rows) { return dt == VTDGE_F32 || rows >= 2048 ? P[which] : nullptr; };
+        auto pk = [&](int which) { return copy_for(which, p.rows); };
 
         if (p.folded) {
             if (i == 0) {
@@ -274,7 +276,7 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
                                            stream));
                 }
                 const int64_t kv_rows = (int64_t)B * p.n_kv;
-                VT_TRY(vtdge_linear_prepacked(src, C, P[P_KVW], kv_rows >= 2048 ? P[P_KVP] : nullptr, P[P_KVB], nullptr, 0, kv,
+                VT_TRY(vtdge_linear_prepacked(src, C, P[P_KVW], copy_for(P_KVP, kv_rows), P[P_KVB], nullptr, 0, kv,
                                               2 * C, nullptr, kv_rows, 2 * C, C, VTDGE_ACT_NONE, dt, stream));
                 VT_TRY(beside.end());
                 VT_TRY(vtdge_linear_prepacked(comp_ln, C, P[P_QW], pk(P_QP), P[P_QB], nullptr, 0, q, C, live, p.cap, C, C,

@@ -25,8 +25,6 @@ constexpr int KB = 128;               // K bytes per stage
 constexpr int PITCH = KB + 16;        // LDS row pitch in bytes
 constexpr int NXCD = 8;
 
-__device__ __forceinline__ float gelu_erf(float v) { return 0.5f * v * (1.0f + erff(v * 0.70710678118654752440f)); }
-
 template <typename T, int ACT, bool HAS_BIAS, bool HAS_RES>
 __global__ __launch_bounds__(256) void linear_kernel(const T *__restrict__ A, int64_t lda, const T *__restrict__ Wt,
                                                       const T *__restrict__ bias, const T *__restrict__ res,
@@ -136,7 +134,7 @@ __global__ __launch_bounds__(256) void linear_kernel(const T *__restrict__ A, in
                 const int64_t row = m0 + wm * 64 + i * 32 + 8 * (v >> 2) + 4 * lg + (v & 3);
                 if (row < M) {
                     float val = acc[i][j][v] + bv;
-                    if constexpr (ACT == VTDGE_ACT_GELU) val = gelu_erf(val);
+                    if constexpr (ACT == VTDGE_ACT_GELU) val = gelu_fn<float>(val);
                     if constexpr (HAS_RES) val += Elem<T>::load(res + row * ldr + col);
                     Elem<T>::store(out + row * ldo + col, val);
                 }
@@ -208,6 +206,13 @@ template <typename T>
 int launch_linear_small(const void *A, int64_t lda, const void *W, const void *bias, const void *res, int64_t ldr,
                         void *out, int64_t ldo, const int64_t *rows_dev, int64_t rows, int N, int K, int act,
                         hipStream_t st);
+
+// fp32 on the bf16 matrix instructions, from a weight split in advance (linear_dma_split.hip)
+int64_t linear_split_size(int N, int K);
+int split_linear_weight(const void *W, int N, int K, void *split, hipStream_t st);
+int launch_linear_dma_split(const void *A, int64_t lda, const void *W, const void *split, const void *bias, const void *res,
+                      int64_t ldr, void *out, int64_t ldo, const int64_t *rows_dev, int64_t rows, int N, int K, int act,
+                      hipStream_t st);
 
 // weight-stationary variant for bf16, K = 384 (linear_ws8.hip)
 bool linear_ws_applicable(int64_t lda, int64_t ldr, int64_t ldo, int64_t rows, int N, int K, int esz, int act,
@@ -451,6 +456,8 @@ extern "C" int vtdge_linear_prepacked(const void *A, int64_t lda, const void *W,
         return launch_linear_small<bf16_t>(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
     }
     if (linear_dma_applicable(lda, ldr, ldo, N, K, esz, bias, residual, out)) {
+        if (dtype == VTDGE_F32 && packed != nullptr && vtdge_linear_split_wanted(rows, N, K))
+            return launch_linear_dma_split(A, lda, W, packed, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
         if (dtype == VTDGE_F32)
             return launch_linear_dma<float>(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
         return launch_linear_dma<bf16_t>(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
@@ -458,6 +465,28 @@ extern "C" int vtdge_linear_prepacked(const void *A, int64_t lda, const void *W,
     if (dtype == VTDGE_F32)
         return launch_linear<float>(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
     return launch_linear<bf16_t>(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
+}
+
+extern "C" int vtdge_linear_split_size(int N, int K, int64_t *bytes)
+{
+    VT_REQUIRE(bytes != nullptr, VTDGE_ERR_ARG, "linear_split_size: NULL result");
+    VT_REQUIRE(N > 0 && K > 0, VTDGE_ERR_ARG, "linear_split_size: bad sizes N=%d K=%d", N, K);
+    *bytes = linear_split_size(N, K);
+    return VTDGE_OK;
+}
+
+extern "C" int vtdge_linear_split(const void *W, int N, int K, void *split, void *stream)
+{
+    VT_REQUIRE(W && split, VTDGE_ERR_ARG, "linear_split: NULL operand");
+    VT_REQUIRE(N > 0 && K > 0, VTDGE_ERR_ARG, "linear_split: bad sizes N=%d K=%d", N, K);
+    VT_REQUIRE(linear_split_size(N, K) > 0, VTDGE_ERR_UNSUPPORTED, "linear_split: no split copy for N=%d K=%d", N, K);
+    VT_REQUIRE((((uintptr_t)W | (uintptr_t)split) & 15) == 0, VTDGE_ERR_ARG, "linear_split: operands must be 16-byte aligned");
+    return split_linear_weight(W, N, K, split, (hipStream_t)stream);
+}
+
+extern "C" int vtdge_linear_split_wanted(int64_t rows, int N, int K)
+{
+    return rows > 0 && N > 0 && K > 0 && linear_split_size(N, K) > 0 && !linear_small_wanted(rows, N, K, 4) ? 1 : 0;
 }
 
 extern "C" int vtdge_patch_embed(const void *images, const void *weight, const void *bias, const void *pos_embed,
