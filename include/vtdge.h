@@ -209,6 +209,28 @@ int vtdge_decompress_router_compress_static(const void *in, const void *sub, con
                                             int B, int H, int W, int C, int extra, int R, int S, int S2, int dtype,
                                             void *stream);
 
+/* Few regions (see vtdge_region_step_fits): from the packed queries of one block to those of the next in one launch, a
+ * workgroup per 4 x 4 region - vtdge_decompress_router, vtdge_compress_regions (or vtdge_index_to_patch and vtdge_compress)
+ * and, of tokens and packed rows, either the statistics records or the LayerNorm, each bit for bit.
+ *   in, sub [.., C]: the packed queries after and before the block   cur_indices, splits, offsets: its gate indices, splits and
+ *   first rows   region_rows with cur_counts (nullable) as in vtdge_decompress_router   ref, out [B, extra + H*W, C]
+ *   next_*: of the block that follows, as in vtdge_decompress_router_compress; S and S2 split sizes, all of them 1, 2 or 4
+ *   out_records, next_comp_records (nullable, bf16 up to 512 channels) or out_ln [B * (extra + H*W), C], next_comp_ln
+ *   [capacity_rows, C] (nullable) with ln_weight, ln_bias; eps of either
+ *   workspace: vtdge_region_step_workspace bytes, zero; its first word stays 0 unless the kernel gave up waiting
+ * vtdge_region_step_fits: 1 for rows of 33 to 192 16-byte vectors, up to 64 extra tokens and as many regions (512 to 2048, by
+ * the width) as the launch is faster for than the separate ones. */
+int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int dtype);
+int64_t vtdge_region_step_workspace(int B, int H, int W);
+int vtdge_region_step(const void *in, const void *sub, const int64_t *cur_indices, const int64_t *splits,
+                      const int64_t *offsets, const int32_t *region_rows, const uint8_t *cur_counts, const void *ref, void *out,
+                      const void *next_weight, const void *next_bias, void *next_gate, int64_t *next_indices,
+                      const int64_t *next_splits, uint8_t *next_counts, void *out_records, void *out_ln,
+                      const void *ln_weight, const void *ln_bias, float eps, void *next_comp, void *next_comp_records,
+                      void *next_comp_ln, int64_t *next_patches, int64_t capacity_rows, int64_t *next_offsets,
+                      int32_t *next_region_rows, void *workspace, int64_t workspace_bytes, int B, int H, int W, int C, int extra,
+                      int S, int S2, int dtype, void *stream);
+
 /* The router of a model's FIRST block together with the statistics records of all its tokens (no scatter-back
  * precedes it that could leave them): vtdge_router and vtdge_layernorm_stats in one pass over x, i.e.
  * DynamicRouter.forward + argmax (vtpack/layers/dge.py:145-150, :75) and the statistics half of norm1

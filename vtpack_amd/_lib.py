@@ -51,6 +51,8 @@ SIGNATURES = {
     "vtdge_linear": [_p, _l, _p, _p, _p, _l, _p, _l, _p, _l, _i, _i, _i, _i, _p],
     "vtdge_patch_embed": [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p],
     "vtdge_patch_linear": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p],
+    "vtdge_region_step_fits": [_i] * 6,
+    "vtdge_region_step": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _f, _p, _p, _p, _p, _l, _p, _p, _p, _l, _i, _i, _i, _i, _i, _i, _i, _i, _p],
     "vtdge_linear_packed_size": [_i, _i, _i, _p],
     "vtdge_linear_prepack": [_p, _i, _i, _i, _p, _p],
     "vtdge_linear_prepacked": [_p, _l, _p, _p, _p, _p, _l, _p, _l, _p, _l, _i, _i, _i, _i, _p],
@@ -128,6 +130,8 @@ def load():
     lib.vtdge_last_kernel.argtypes = []
     lib.vtdge_decompress_router_compress_workspace.restype = _l
     lib.vtdge_decompress_router_compress_workspace.argtypes = [_i, _i, _i, _i]
+    lib.vtdge_region_step_workspace.restype = _l
+    lib.vtdge_region_step_workspace.argtypes = [_i, _i, _i]
     for name, args in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.restype = _i

@@ -23,12 +23,15 @@ enum {
 };
 static_assert(P_COUNT == VTDGE_CHAIN_PARAMS, "the parameter table's documented length");
 
-// first `n` rows of every sample of x [B, N, C] = rows [n, C] (the class tokens), 16 bytes a lane
+// first `n` rows of every sample of x [B, N, C] = rows [n, C] (the class tokens), 16 bytes a lane; `words` 64-bit words at
+// `clear` = 0 (the status words of the scatter-backs)
 __global__ __launch_bounds__(256) void front_rows_kernel(u32x4 *__restrict__ x, const u32x4 *__restrict__ rows,
-                                                         int64_t sample_vecs, int vecs, int64_t total)
+                                                         int64_t sample_vecs, int vecs, int64_t total,
+                                                         unsigned long long *__restrict__ clear, int64_t words)
 {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < total) x[i / vecs * sample_vecs + i % vecs] = rows[i % vecs];
+    if (i < words) clear[i] = 0ull;
 }
 
 struct ChainPlan {
@@ -36,6 +39,7 @@ struct ChainPlan {
     int esz, N, n_kv;              // tokens per sample, keys per sample
     bool folded;                   // norms folded into weight-stationary Linears, chained scatter-back (384-channel bf16)
     bool by_region, pack;          // compress by region; the scatter-back packs the next block's queries
+    bool step;                     // few regions: the scatter-back also writes what the next block's norm1 wants
     bool tail;                     // narrow bf16 rows: everything behind attention as one kernel
     bool ln_kvq, ln_fc1;           // few rows: norm1 inside the kv and q Linear, norm2 inside fc1
     int64_t ws_words;
@@ -74,8 +78,11 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
     p.ln_kvq = !p.folded && c->sr == 1 && vtdge_layernorm_linear_wanted(p.rows, 2 * c->C, p.cap, c->C, c->C, c->dtype);
     p.tail = vtdge_block_tail_wanted(p.rows, c->C, c->hidden, c->dtype);
     p.ln_fc1 = !p.folded && !p.tail && vtdge_layernorm_linear_wanted(p.cap, c->hidden, 0, 0, c->C, c->dtype);
-    p.pack = p.folded && c->depth > 1 && p.regions % 4 == 0;
-    p.ws_words = p.pack ? vtdge_decompress_router_compress_workspace(c->B, c->H, c->W, 4) / 8 : 0;
+    p.step = c->depth > 1 && c->splits_124 && vtdge_region_step_fits(c->B, c->H, c->W, c->C, c->extra, c->dtype);
+    p.pack = p.step || (p.folded && c->depth > 1 && p.regions % 4 == 0);
+    p.ws_words = p.step   ? vtdge_region_step_workspace(c->B, c->H, c->W) / 8
+                 : p.pack ? vtdge_decompress_router_compress_workspace(c->B, c->H, c->W, 4) / 8
+                          : 0;
 
     int64_t at = 0;
     auto take = [&](int64_t bytes) {
@@ -233,40 +240,45 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
                                                2 * C, comp, C, recc, P[P_QFW], P[P_QFP], P[P_QFR], q, C, live, p.cap, C,
                                                C, dt, stream));
         } else {
-            if (i == 0 && front != nullptr) {
+            const int64_t words = p.step ? p.ws_words * (c->depth - 1) : 0;
+            if (i == 0 && (front != nullptr || words > 0)) {
                 const int vecs = extra * C * esz / 16;
-                const int64_t total = (int64_t)B * vecs;
+                const int64_t total = front != nullptr ? (int64_t)B * vecs : 0;
                 note_kernel(reinterpret_cast<const void *>(front_rows_kernel));
-                front_rows_kernel<<<(unsigned)ceil_div(total, 256), 256, 0, (hipStream_t)stream>>>(
-                    (u32x4 *)x, (const u32x4 *)front, (int64_t)N * C * esz / 16, vecs, total);
+                front_rows_kernel<<<(unsigned)ceil_div(total > words ? total : words, 256), 256, 0, (hipStream_t)stream>>>(
+                    (u32x4 *)x, (const u32x4 *)front, (int64_t)N * C * esz / 16, vecs, total,
+                    (unsigned long long *)(ints + p.ws0), words);
                 VT_TRY(check_launch("chain"));
             }
-            void *routing = stream;
-            if (side != nullptr) {
-                // the routing chain beside the key/value chain, joined before attention
-                routing = side;
-                VT_TRY(beside.begin());
-            }
             char *comp_ln = p.ln_kvq ? nullptr : scratch + p.comp_ln, *xln = scratch + p.xln;
-            if (!routed)
-                VT_TRY(vtdge_router(x, P[P_RW], P[P_RB], gate, idx, B, H, W, C, extra, 4, S, dt, routing));
-            if (p.by_region) {
-                VT_TRY(vtdge_compress_regions(x, idx, splits, have_counts ? cnt : nullptr, comp, nullptr, 0.f, patches,
-                                              p.cap, offsets, lengths, rr, B, H, W, C, extra, 4, S, dt, routing));
-                if (comp_ln != nullptr)
-                    VT_TRY(vtdge_layernorm(comp, P[P_N1W], P[P_N1B], comp_ln, live, p.cap, C, c->eps1, dt, routing));
-            } else {
-                VT_TRY(vtdge_index_to_patch(idx, splits, B, H / 4, W / 4, S, 4, extra, patches, p.cap, offsets, lengths,
-                                            routing));
-                VT_TRY(vtdge_compress(x, patches, live, p.cap, comp, comp_ln, comp_ln ? P[P_N1W] : nullptr,
-                                      comp_ln ? P[P_N1B] : nullptr, c->eps1, B, N, C, W, extra, dt, routing));
+            if (!packed) {
+                void *routing = stream;
+                if (side != nullptr) {
+                    // the routing chain beside the key/value chain, joined before attention
+                    routing = side;
+                    VT_TRY(beside.begin());
+                }
+                if (!routed)
+                    VT_TRY(vtdge_router(x, P[P_RW], P[P_RB], gate, idx, B, H, W, C, extra, 4, S, dt, routing));
+                if (p.by_region) {
+                    VT_TRY(vtdge_compress_regions(x, idx, splits, have_counts ? cnt : nullptr, comp, nullptr, 0.f, patches,
+                                                  p.cap, offsets, lengths, rr, B, H, W, C, extra, 4, S, dt, routing));
+                    if (comp_ln != nullptr)
+                        VT_TRY(vtdge_layernorm(comp, P[P_N1W], P[P_N1B], comp_ln, live, p.cap, C, c->eps1, dt, routing));
+                } else {
+                    VT_TRY(vtdge_index_to_patch(idx, splits, B, H / 4, W / 4, S, 4, extra, patches, p.cap, offsets, lengths,
+                                                routing));
+                    VT_TRY(vtdge_compress(x, patches, live, p.cap, comp, comp_ln, comp_ln ? P[P_N1W] : nullptr,
+                                          comp_ln ? P[P_N1B] : nullptr, c->eps1, B, N, C, W, extra, dt, routing));
+                }
             }
             if (p.ln_kvq) {
                 VT_TRY(vtdge_layernorm_linear(x, C, P[P_KVW], P[P_KVB], kv, nullptr, p.rows, 2 * C, comp, C, P[P_QW], P[P_QB],
                                               q, live, p.cap, C, P[P_N1W], P[P_N1B], c->eps1, C, VTDGE_ACT_NONE, dt,
                                               stream));
             } else {
-                VT_TRY(vtdge_layernorm(x, P[P_N1W], P[P_N1B], xln, nullptr, p.rows, C, c->eps1, dt, stream));
+                if (!packed)
+                    VT_TRY(vtdge_layernorm(x, P[P_N1W], P[P_N1B], xln, nullptr, p.rows, C, c->eps1, dt, stream));
                 char *src = xln;
                 if (c->sr > 1) {
                     char *red = scratch + p.red;
@@ -315,9 +327,18 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
             break;
         }
         // where this block's regions lie: left by compress by region (or by the scatter-back before it) with the counts
-        const bool placed = p.by_region && have_counts;
-        const int64_t *nsplits = p.by_region ? (const int64_t *)Q[P_SPLITS] : nullptr;
-        if (p.pack)
+        const bool placed = (p.by_region || p.step) && have_counts;
+        const int64_t *nsplits = p.by_region || p.step ? (const int64_t *)Q[P_SPLITS] : nullptr;
+        if (p.step) {
+            const bool normed = !p.folded && !p.ln_kvq;
+            VT_TRY(vtdge_region_step(
+                q2, comp, idx, splits, offsets, placed ? rr : nullptr, placed ? cnt : nullptr, x, xout, Q[P_RW], Q[P_RB], ngate,
+                nidx, nsplits, ncnt, p.folded ? nrecx : nullptr, normed ? scratch + p.xln : nullptr,
+                normed ? Q[P_N1W] : nullptr, normed ? Q[P_N1B] : nullptr, c->eps1, big + p.comp0 + (i + 1) * p.row_sz,
+                p.folded ? nrecc : nullptr, normed ? scratch + p.comp_ln : nullptr,
+                (int64_t *)(big + p.pat0 + (i + 1) * p.pat_sz), p.cap, (int64_t *)(ints + p.off0 + (i + 1) * p.off_sz), nrr,
+                ints + p.ws0 + i * p.ws_sz, p.ws_sz, B, H, W, C, extra, S, S, dt, stream));
+        } else if (p.pack)
             VT_TRY(vtdge_decompress_router_compress(
                 q2, comp, idx, splits, offsets, x, xout, Q[P_RW], Q[P_RB], ngate, nidx, nrecx, c->eps1, nsplits, ncnt,
                 placed ? rr : nullptr, placed ? cnt : nullptr, big + p.comp0 + (i + 1) * p.row_sz, nrecc, c->eps1,
@@ -330,7 +351,7 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
                                            stream));
         routed = true;
         packed = p.pack;
-        have_counts = p.by_region;
+        have_counts = p.by_region || p.step;
         x = xout;
         cur ^= 1;
     }

@@ -1037,9 +1037,6 @@ struct ChainArgs {
     int32_t *region_rows;         // [B * regions] first packed row of every region (nullable)
     unsigned long long *status;   // [1 + workgroups]: word 0 = error flag, then one word per workgroup
 };
-constexpr unsigned long long CHAIN_AGGREGATE = 1ull << 62, CHAIN_PREFIX = 2ull << 62;
-constexpr int CHAIN_SPIN_LIMIT = 1 << 20;
-
 // SCATTER = false: no packed rows at all - the kernel routes on `ref` as it stands and writes the records of its
 // rows (the first block of a model, which no scatter-back precedes); `in` then points, if anywhere, at `extra`
 // rows [extra, C] that are first copied into the extra-token rows of every sample of `out` (class / distillation
@@ -1235,64 +1232,8 @@ void decompress_route_kernel(
         const int wg = (int)blockIdx.x;
         if (wv == 0) {
             const int agg = cnt_s[0] + cnt_s[1] + cnt_s[2] + cnt_s[3];
-            if (lane == 0)
-                __hip_atomic_store(st + wg, (wg == 0 ? CHAIN_PREFIX : CHAIN_AGGREGATE) | (unsigned long long)agg,
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            long long excl = 0;
-            if (wg > 0) {
-                // Every step looks at LOOK x 64 words, nearest first.  One load a lane is the fastest: the nearest
-                // workgroups are the last to publish, and a wider window only makes each retry dearer (measured at
-                // 1024 workgroups: 52 us for the kernel with 64 words a step, 54 with 128, 57 with 512).
-                constexpr int LOOK = 1;
-                int j = wg - 1, spins = 0;
-                bool gave_up = false;
-                while (true) {
-                    unsigned long long v[LOOK];
-#pragma unroll
-                    for (int k = 0; k < LOOK; k++) {
-                        const int idx = j - lane - WAVE * k;   // lane 0 of k = 0: the workgroup just before this one
-                        v[k] = CHAIN_PREFIX;                   // before the first workgroup: a prefix of zero
-                        if (idx >= 0) v[k] = __hip_atomic_load(st + idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    }
-                    float part = 0.f;
-                    bool found = false, wait = false;
-#pragma unroll
-                    for (int k = 0; k < LOOK; k++) {
-                        if (!found && !wait) {
-                            const int flag = (int)(v[k] >> 62);
-                            const unsigned long long missing = __builtin_amdgcn_ballot_w64(flag == 0);
-                            const unsigned long long known = __builtin_amdgcn_ballot_w64(flag == 2);
-                            const int first_known = known ? __builtin_ctzll(known) : 64;
-                            const int first_missing = missing ? __builtin_ctzll(missing) : 64;
-                            if (first_missing < first_known) {
-                                wait = true;     // somebody nearer than the first prefix has not published yet
-                            } else {
-                                const int upto = first_known < 64 ? first_known : 63;
-                                part += lane <= upto ? (float)(unsigned)(v[k] & 0xffffffffull) : 0.f;
-                                found = first_known < 64;
-                            }
-                        }
-                    }
-                    if (wait) {
-                        if (++spins > CHAIN_SPIN_LIMIT) {
-                            gave_up = true;
-                            break;
-                        }
-                        __builtin_amdgcn_s_sleep(1);
-                        continue;
-                    }
-                    excl += (long long)wave_sum(part);
-                    if (found) break;
-                    j -= WAVE * LOOK;
-                }
-                if (gave_up) {
-                    excl = chain.capacity;                 // every row of this workgroup falls past the capacity
-                    if (lane == 0) __hip_atomic_store(chain.status, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-                if (lane == 0)
-                    __hip_atomic_store(st + wg, CHAIN_PREFIX | (unsigned long long)(excl + agg), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-            }
+            chain_publish(st, wg, agg);
+            const long long excl = chain_rows_before(chain.status, wg, agg, chain.capacity);
             if (lane == 0) excl_s = excl;
         }
         __syncthreads();
