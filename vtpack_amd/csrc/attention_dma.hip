@@ -620,7 +620,7 @@ __global__ __launch_bounds__(256, 2) void sparse_attention_bf16_d64_stream_kerne
     const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     f32x16 o[2], negm;
     float l[2];
-    const int nfull = n / ASK;                        // stages of four whole blocks; then at most one shorter stage
+    const int nfull = n / ASK;                        // whole stages; then at most one shorter stage
     auto stage_tile = [&](int st) {
         const unsigned char *buf = smem + (st & 1) * ASBUF;
         const unsigned char *vl = att_v_lane(buf + ASK * 128, lane);
@@ -639,12 +639,13 @@ __global__ __launch_bounds__(256, 2) void sparse_attention_bf16_d64_stream_kerne
             if (st + 1 < nstage) issue(st + 1);
             if (wave_live) att_stage_fixed<4, FAST>(stage_tile(st), cs, st == 0, qf, o, negm, l, &bad);
         }
-        if (nfull < nstage) {                // the last, shorter stage: 1 .. 3 blocks (its own code, outside the loop)
+        if (nfull < nstage) {                // the last, shorter stage: 1 .. 4 blocks (its own code, outside the loop)
             wait_vmcnt<0>();
             __syncthreads();
             if (wave_live) {
                 const AttnTile tile = stage_tile(nfull);
                 switch ((tile.n + 31) / 32) {
+                case 4: att_stage_fixed<4, FAST>(tile, cs, nfull == 0, qf, o, negm, l, &bad); break;
                 case 3: att_stage_fixed<3, FAST>(tile, cs, nfull == 0, qf, o, negm, l, &bad); break;
                 case 2: att_stage_fixed<2, FAST>(tile, cs, nfull == 0, qf, o, negm, l, &bad); break;
                 default: att_stage_fixed<1, FAST>(tile, cs, nfull == 0, qf, o, negm, l, &bad); break;
