@@ -24,3 +24,49 @@ def test_last_stage_of_streamed_keys(dev, n):
     """The streaming kernel's last stage of one to four blocks of 32 keys, whole and partial."""
     lengths = rng(800 + n).choice([0, 1, 32, 33, 128, 129, 150], size=60)
     _check(dev, 5, n, lengths, f"300 pairs of {n} keys")
+
+
+# (sample, head) pairs that few workgroups take: the kernel whose waves split the keys.  Every number of blocks (1 .. 9), whole
+# and partial, then rounds of eight blocks with a last one that some waves sit out; empty samples, a query more and less than
+# a tile, more tiles than a workgroup takes at once.
+@pytest.mark.parametrize("lengths,h", [([1, 0, 33], 2), ([257, 32, 96, 0, 31, 150], 3), ([300], 1), ([64] * 85, 1)])
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 64, 96, 128, 129, 160, 192, 197, 224, 256, 257, 288, 289, 511, 512, 513, 1025])
+def test_few_pairs(dev, n, lengths, h):
+    _check(dev, h, n, lengths, f"{h} x {len(lengths)} pairs of {n} keys")
+
+
+def test_few_pairs_many_tiles(dev):
+    _check(dev, 2, 144, [1500], "two pairs of 47 tiles")
+
+
+@pytest.mark.parametrize("n", [257, 700])
+@pytest.mark.parametrize("place", [3, 40, 250, 256])
+def test_few_pairs_one_key_above_all(dev, n, place):
+    """A key hundreds above the others: every wave but its own adds nothing, whichever wave that is."""
+    from vtpack_amd import _C
+    q, k, v = 0.05 * randn(811, 2, 70, 64), 0.05 * randn(812, 2, 1, n, 64), randn(813, 2, 1, n, 64)
+    q[..., 0], k[..., 0] = 8.0, 0.0
+    k[:, :, place, 0] = 300.0
+    q, k, v = bf16_round(q), bf16_round(k), bf16_round(v)
+    lengths = np.array([70], dtype=np.int64)
+    got = _C.batched_sparse_attention_forward(*(torch.from_numpy(t).to(dev, torch.bfloat16) for t in (q, k, v)),
+                                              torch.from_numpy(lengths), 0.125)
+    assert_close(got.float(), orc.attention(q, k, v, lengths, 0.125), torch.bfloat16, "one key above all")
+
+
+def test_few_pairs_infinities(dev):
+    """Keys whose scores are -infinity count for nothing, in a block of their own too; all of them make NaN, as a softmax of
+    nothing does; one of +infinity makes its query NaN."""
+    from vtpack_amd import _C
+    n, h = 257, 1
+    q, k, v = torch.zeros(h, 40, 64), torch.zeros(h, 2, n, 64), torch.from_numpy(randn(821, h, 2, n, 64))
+    q[..., 0] = 1.0
+    k[:, 0, :100, 0] = -float("inf")
+    k[:, 1, :, 0] = -float("inf")
+    q[:, 3, 0] = -1.0                                 # sample 0: +infinity
+    lengths = torch.tensor([20, 20])
+    got = _C.batched_sparse_attention_forward(*(t.to(dev, torch.bfloat16) for t in (q, k, v)), lengths, 0.125).float().cpu()
+    want = v.to(torch.bfloat16).float()[:, 0, 100:].mean(1)
+    rows = [i for i in range(20) if i != 3]
+    assert float((got[:, rows] - want).abs().max()) <= 4e-3 * float(want.abs().max())
+    assert bool(got[:, 3].isnan().all()) and bool(got[:, 20:].isnan().all())
