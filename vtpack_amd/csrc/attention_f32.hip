@@ -42,21 +42,16 @@ template <int D> struct AttnF32 {
     }
 };
 
+// The 64 query rows `chunk` of (sample, head) `pair`, by a workgroup of four waves.
 // WIDE: token strides of 2^23 values and more, or negative ones: 64-bit addresses of the direct loads
 template <int D, bool WIDE>
-__global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
-    const float *__restrict__ q, int64_t q_rs, int64_t q_hs, const float *__restrict__ k, const float *__restrict__ v,
-    int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets, float *__restrict__ out,
-    int64_t o_rs, int64_t o_hs, int pairs, int h, int n, float scale_log2)
+__device__ __forceinline__ void attention_f32_rows(
+    unsigned char *smem, const float *__restrict__ q, int64_t q_rs, int64_t q_hs, const float *__restrict__ k,
+    const float *__restrict__ v, int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets,
+    float *__restrict__ out, int64_t o_rs, int64_t o_hs, int pair, int chunk, int h, int n, float scale_log2)
 {
     using G = AttnF32<D>;
     constexpr int NL = G::BUF / 1024 / AF_TILES;              // direct loads a wave and stage
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-
-    // the chunks of a (sample, head) pair run on one XCD, so its K/V are fetched into one L2
-    const int rest = blockIdx.x >> 3, pairs_x = (pairs + 7) / 8;
-    const int pair = (rest % pairs_x) * 8 + (blockIdx.x & 7), chunk = rest / pairs_x;
-    if (pair >= pairs) return;
     const int b = pair / h, head = pair - b * h;
     const int64_t row0 = offsets[b];
     const int Lb = (int)(offsets[b + 1] - row0);
@@ -246,16 +241,283 @@ __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
 }
 
 template <int D, bool WIDE>
+__global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
+    const float *__restrict__ q, int64_t q_rs, int64_t q_hs, const float *__restrict__ k, const float *__restrict__ v,
+    int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets, float *__restrict__ out,
+    int64_t o_rs, int64_t o_hs, int pairs, int h, int n, float scale_log2)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    // the chunks of a (sample, head) pair run on one XCD, so its K/V are fetched into one L2
+    const int rest = blockIdx.x >> 3, pairs_x = (pairs + 7) / 8;
+    const int pair = (rest % pairs_x) * 8 + (blockIdx.x & 7), chunk = rest / pairs_x;
+    if (pair >= pairs) return;
+    attention_f32_rows<D, WIDE>(smem, q, q_rs, q_hs, k, v, kv_bs, kv_ts, kv_hs, offsets, out, o_rs, o_hs, pair, chunk, h, n,
+                                scale_log2);
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// head_dim 64 on the bf16 matrix instructions, as exact: queries, keys, probabilities and values are each the sum of three
+// bf16 values (to 2^-26 of them), six of the nine partial products of two such sums are multiplied and added in fp32
+// (linear_dma_split.hip says why that is enough).  Per 32 keys and 16 queries that is 768 clocks of matrix instructions
+// against 2048; against float64 the output is off by 3.7e-7 against 4.1e-7 (2-norm; 257 keys, unit normals).
+// What bounds it are the vector instructions: splitting a stage of K and V (88 a wave) and the probabilities (44), the
+// exponentials and 36 reads of LDS, some 300 a wave and stage beside 48 matrix instructions.
+//   * 64 query rows a workgroup, 16 a wave; a stage of 32 keys goes through registers, is split and written to LDS as planes of
+//     bf16 rows (24 KB), the next one on its way from memory meanwhile.  One buffer and two barriers a stage leave room for
+//     four workgroups a compute unit, which fill each other's waits: 34.5 us at 128 samples, 3 heads, 257 keys, 14146 rows;
+//     with two buffers (three workgroups) 39.7, 128 rows on eight waves 39.1, two tiles of queries a wave 47.9.
+//   * V comes out of LDS transposed (ds_read_b64_tr_b16), so that the operand of step j holds the keys whose probabilities the
+//     lane has: P never moves between lanes.
+//   * A workgroup of one or two tiles takes the fp32 instructions, whose waves share a tile (20 queries of 128 samples: 17.4
+//     against 20.9 us), and so does one with anything the split is not exact for: sums that are not finite, tiny or huge
+//     ones, queries far from one.
+constexpr int AS_KEYS = 32;                          // keys per stage
+constexpr int AS_PLANE = AS_KEYS * 128;              // bytes of a plane: 32 rows of 64 bf16 values
+constexpr int AS_BUF = 6 * AS_PLANE;                 // one stage: three planes of K, then three of V
+constexpr float AS_TINY = 0x1p-80f, AS_FAR = 0x1p60f;
+
+// x[0..7] into three bf16 parts each: x = p[0] + p[1] + p[2] to 2^-26 of it (nearest parts, signed remainders)
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[3])
+{
+    float r[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) r[e] = x[e];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            p[i][e] = pack_bf16x2(r[2 * e], r[2 * e + 1]);
+            if (i < 2) {
+                r[2 * e] -= bf16lo(p[i][e]);
+                r[2 * e + 1] -= bf16hi(p[i][e]);
+            }
+        }
+}
+__device__ __forceinline__ f32x4 mma_bf16_16(const u32x4 &a, const u32x4 &b, const f32x4 &c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// The 64 query rows `chunk` of a pair as attention_f32_rows computes them -> whether it could
+__device__ __forceinline__ bool attention_f32_split_rows(
+    unsigned char *smem, const float *__restrict__ q, int64_t q_rs, int64_t q_hs, const float *__restrict__ k, const float *__restrict__ v,
+    int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets, float *__restrict__ out,
+    int64_t o_rs, int64_t o_hs, int pair, int chunk, int h, int n, float scale_log2)
+{
+    constexpr int ROWS = 16 * AF_TILES;
+    const int b = pair / h, head = pair - b * h;
+    const int64_t row0 = offsets[b];
+    const int Lb = (int)(offsets[b + 1] - row0);
+    if (chunk * ROWS >= Lb) return true;
+    const int tiles = min(AF_TILES, (Lb - chunk * ROWS + 15) / 16);
+    if (tiles <= AF_TILES / 2) return false;                  // two waves a tile do better there
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l = lane & 15, g = lane >> 4;
+    const bool live = wid < tiles;
+
+    // This thread's part of a stage: 8 values of a row of K and of V
+    const int srow = tid >> 3, schunk = tid & 7;
+    const float *kp = k + (int64_t)b * kv_bs + (int64_t)head * kv_hs + 8 * schunk;
+    const float *vp = v + (int64_t)b * kv_bs + (int64_t)head * kv_hs + 8 * schunk;
+    float rk[8], rv[8];
+    auto load_stage = [&](int st) {                          // rows past the last key repeat it
+        const int64_t off = (int64_t)min(st * AS_KEYS + srow, n - 1) * kv_ts;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const f32x4 a = *reinterpret_cast<const f32x4 *>(kp + off + 4 * i), c = *reinterpret_cast<const f32x4 *>(vp + off + 4 * i);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                rk[4 * i + e] = a[e];
+                rv[4 * i + e] = c[e];
+            }
+        }
+    };
+    const int kdst = srow * 128 + ((schunk ^ ((srow >> 1) & 7)) * 16);
+    const int vdst = 3 * AS_PLANE + srow * 128 + ((schunk ^ (2 * ((srow >> 1) & 3))) * 16);
+    auto store_stage = [&](int st) {
+        if (st * AS_KEYS + AS_KEYS > n) {                    // nothing of a repeated row, not even 0 * infinity
+            const bool past = st * AS_KEYS + srow >= n;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                rk[e] = past ? 0.f : rk[e];
+                rv[e] = past ? 0.f : rv[e];
+            }
+        }
+        u32x4 p[3];
+        split8(rk, p);
+#pragma unroll
+        for (int i = 0; i < 3; i++) *reinterpret_cast<u32x4 *>(smem + kdst + i * AS_PLANE) = p[i];
+        split8(rv, p);
+#pragma unroll
+        for (int i = 0; i < 3; i++) *reinterpret_cast<u32x4 *>(smem + vdst + i * AS_PLANE) = p[i];
+    };
+
+    load_stage(0);
+    // queries times scale * log2(e), split: step t of the contraction takes d = 32 t + 8 g + (0 .. 7)
+    const int qrow = chunk * ROWS + wid * 16 + l;
+    const bool row_live = qrow < Lb;
+    u32x4 qf[2][3];
+    bool odd = false;                                        // something the split is not exact for
+    {
+        const float *qp = q + (row0 + qrow) * q_rs + (int64_t)head * q_hs + 8 * g;
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const f32x4 a = row_live ? *reinterpret_cast<const f32x4 *>(qp + 32 * t + 4 * j) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    x[4 * j + e] = a[e] * scale_log2;
+                    const float m = fabsf(x[4 * j + e]);
+                    odd = odd || !(m <= AS_FAR) || (m < 1.f / AS_FAR && a[e] != 0.f && scale_log2 != 0.f);
+                }
+            }
+            split8(x, qf[t]);
+        }
+        odd = fresh(odd) != 0;                               // here: the compiler would keep the queries for a test at the end
+    }
+    f32x4 o[4];
+#pragma unroll
+    for (int db = 0; db < 4; db++) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float neg_m = 0.f, l_run = 0.f;                          // the reference and the row sum, as in attention_f32_rows
+    bool first = true;
+    int koff[2], voff[4];
+#pragma unroll
+    for (int t = 0; t < 2; t++) koff[t] = l * 128 + (((4 * t + g) ^ ((l >> 1) & 7)) * 16);      // K row l, chunk 4 t + g
+    {
+        // the transposing reads of V: source lane 4 e + r of a block of 16 names key 4 g + e (+ 16), channels 4 r ..
+        const int key = 4 * g + (l >> 2), r = l & 3;
+#pragma unroll
+        for (int db = 0; db < 4; db++)
+            voff[db] = 3 * AS_PLANE + key * 128 + (((2 * db + (r >> 1)) ^ (2 * ((key >> 1) & 3))) * 16) + 8 * (r & 1);
+    }
+    constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};     // partial products, the small ones first
+
+    // the 32 keys of a stage; those >= n are masked (their K and V are zero)
+    auto compute = [&](int st) {
+        f32x4 s[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; kb++) {
+            s[kb] = f32x4{neg_m, neg_m, neg_m, neg_m};
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                u32x4 kf[3];
+#pragma unroll
+                for (int p = 0; p < 3; p++) kf[p] = *reinterpret_cast<const u32x4 *>(smem + koff[t] + kb * 16 * 128 + p * AS_PLANE);
+#pragma unroll
+                for (int x = 0; x < 6; x++) s[kb] = mma_bf16_16(kf[PA[x]], qf[t][PB[x]], s[kb]);
+            }
+        }
+        if (st * AS_KEYS + AS_KEYS > n) {
+            const int left = n - st * AS_KEYS - 4 * g;       // keys from this lane's first one on
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (16 * (e / 4) + e % 4 >= left) s[e / 4][e % 4] = -INFINITY;
+        }
+        // whether a score is that far above the reference: the largest bit pattern orders positive floats as floats do
+        int bits = __float_as_int(s[0][0]);
+#pragma unroll
+        for (int e = 1; e < 8; e++) bits = max(bits, __float_as_int(s[e / 4][e % 4]));
+        if (__any(first || __int_as_float(bits) > AF_RAISE)) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int e = 0; e < 8; e++) mx = fmaxf(mx, s[e / 4][e % 4]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+            const float d = !first ? fmaxf(mx, 0.f) : mx == -INFINITY ? 0.f : mx;
+            const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-d);
+            first = first && mx == -INFINITY;
+            neg_m -= d;
+            s[0] -= d;
+            s[1] -= d;
+            l_run *= alpha;
+#pragma unroll
+            for (int db = 0; db < 4; db++) o[db] *= alpha;
+        }
+        u32x4 pf[3];
+        float p[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            p[e] = __builtin_amdgcn_exp2f(s[e / 4][e % 4]);
+            l_run += p[e];
+        }
+        split8(p, pf);
+#pragma unroll
+        for (int db = 0; db < 4; db++) {
+            u32x4 vf[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                const unsigned char *vs = smem + voff[db] + i * AS_PLANE;
+                const u32x2 lo = lds_read_tr16(vs), hi = lds_read_tr16(vs + 16 * 128);
+                vf[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
+            }
+#pragma unroll
+            for (int x = 0; x < 6; x++) o[db] = mma_bf16_16(vf[PA[x]], pf[PB[x]], o[db]);
+        }
+    };
+
+    const int stages = (n + AS_KEYS - 1) / AS_KEYS;
+    for (int st = 0; st < stages; st++) {
+        if (st > 0) lds_barrier();                           // the stage before has been read
+        store_stage(st);
+        if (st + 1 < stages) load_stage(st + 1);
+        lds_barrier();                                       // stage st is whole
+        if (live) compute(st);
+    }
+    l_run += __shfl_xor(l_run, 16, WAVE);
+    l_run += __shfl_xor(l_run, 32, WAVE);
+    if (row_live) {
+        odd = odd || !(l_run < INFINITY);
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const float m = fabsf(o[e / 4][e % 4]);
+            odd = odd || !(m <= AS_FAR) || (m < AS_TINY && m != 0.f);
+        }
+    }
+    if (__syncthreads_or(odd ? 1 : 0)) return false;
+    if (!row_live) return true;
+    const float inv = 1.0f / l_run;
+    float *op = out + (row0 + qrow) * o_rs + (int64_t)head * o_hs + 4 * g;
+#pragma unroll
+    for (int db = 0; db < 4; db++)
+        *reinterpret_cast<f32x4 *>(op + 16 * db) = f32x4{o[db][0] * inv, o[db][1] * inv, o[db][2] * inv, o[db][3] * inv};
+    return true;
+}
+
+template <bool WIDE>
+__global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_split_kernel(
+    const float *__restrict__ q, int64_t q_rs, int64_t q_hs, const float *__restrict__ k, const float *__restrict__ v,
+    int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets, float *__restrict__ out,
+    int64_t o_rs, int64_t o_hs, int pairs, int h, int n, float scale_log2)
+{
+    extern __shared__ __attribute__((aligned(128))) unsigned char smem[];
+    const int rest = blockIdx.x >> 3, pairs_x = (pairs + 7) / 8;
+    const int pair = (rest % pairs_x) * 8 + (blockIdx.x & 7), chunk = rest / pairs_x;
+    if (pair >= pairs) return;
+    if (!attention_f32_split_rows(smem, q, q_rs, q_hs, k, v, kv_bs, kv_ts, kv_hs, offsets, out, o_rs, o_hs, pair, chunk, h, n,
+                                  scale_log2))
+        attention_f32_rows<64, WIDE>(smem, q, q_rs, q_hs, k, v, kv_bs, kv_ts, kv_hs, offsets, out, o_rs, o_hs, pair, chunk, h, n,
+                                     scale_log2);
+}
+
+template <int D, bool WIDE, bool SPLIT>
 static int go_attention_f32(const void *q, int64_t q_rs, int64_t q_hs, const void *k, const void *v, int64_t kv_bs,
                             int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs, int64_t o_hs,
                             int B, int h, int n, int max_rows, float scale, hipStream_t st)
 {
     constexpr size_t lds = 2 * AttnF32<D>::BUF;
+    static_assert(!SPLIT || lds >= AS_BUF, "a stage of split keys and values");
     const int64_t pairs = (int64_t)B * h, chunks = ceil_div(max_rows, 16 * AF_TILES);
     const int64_t grid = ceil_div(pairs, 8) * 8 * chunks;
     VT_REQUIRE(grid < (1ll << 31), VTDGE_ERR_UNSUPPORTED, "sparse_attention: %lld workgroups exceed one launch",
                (long long)grid);
-    auto kern = attention_f32_kernel<D, WIDE>;
+    constexpr auto kern = [] {
+        if constexpr (SPLIT) return attention_f32_split_kernel<WIDE>;
+        else return attention_f32_kernel<D, WIDE>;
+    }();
     VT_RESERVE_LDS(kern, lds, "sparse_attention");
     note_kernel(reinterpret_cast<const void *>(kern));
     kern<<<dim3((unsigned)grid), dim3(64 * AF_TILES), lds, st>>>(
@@ -268,7 +530,17 @@ int launch_attention_f32(const void *q, int64_t q_rs, int64_t q_hs, const void *
                          int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs, int64_t o_hs,
                          int B, int h, int n, int max_rows, float scale, hipStream_t st)
 {
-    const auto go = kv_ts >= 0 && kv_ts < (1 << 23) ? go_attention_f32<D, false> : go_attention_f32<D, true>;
+    const bool wide = !(kv_ts >= 0 && kv_ts < (1 << 23));
+    auto go = wide ? go_attention_f32<D, true, false> : go_attention_f32<D, false, false>;
+    // The bf16 instructions from about as many workgroups on as put one on every compute unit and some beside it, and for long
+    // chains of keys.  Us, fp32 / bf16 instructions (samples, heads, keys, live rows): 128, 3, 257, 14146: 44.1 / 34.5;
+    // 64, 6, 257, 6596: 44.2 / 33.7; 64, 6, 145, 4834: 25.8 / 20.3; 64, 6, 64, 16384: 25.3 / 21.6; 16, 6, 257, 2021: 23.6 /
+    // 19.9; 6, 1, 144, 24192: 16.8 / 15.2; 32, 6, 1025, 15106: 302 / 191; 8, 6, 1025, 3169: 77.0 / 60.0.  Below the line:
+    // 8, 6, 257, 862: 15.3 / 15.8; 6, 5, 144, 1512: 10.1 / 10.9; 64, 3, 65, 2033: 8.4 / 9.2.
+    const int64_t wgs = (int64_t)B * h * ceil_div(max_rows, 16 * AF_TILES);
+    if constexpr (D == 64)
+        if (n > 512 || (wgs >= 320 && wgs * n >= 48000))
+            go = wide ? go_attention_f32<D, true, true> : go_attention_f32<D, false, true>;
     return go(q, q_rs, q_hs, k, v, kv_bs, kv_ts, kv_hs, offsets, out, o_rs, o_hs, B, h, n, max_rows, scale, st);
 }
 template int launch_attention_f32<64>(const void *, int64_t, int64_t, const void *, const void *, int64_t, int64_t,
