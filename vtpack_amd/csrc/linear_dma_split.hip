@@ -352,7 +352,13 @@ int launch_linear_dma_split(const void *A, int64_t lda, const void *W, const voi
     // 73 / 76 / 100; 65536, 1536, 384: 637 / 572 / 525 / 477.
     if (res != nullptr) VT_PICK(true, 64, 64, 2, 2, 4, 3);
     if (N % 128 == 0 && K >= 384 && ceil_div(rows, 128) * (N / 128) >= 1024) VT_PICK(false, 128, 128, 2, 2, 4, 3);
-    if (ceil_div(rows, 128) * (N / 64) >= 1536) VT_PICK(false, 128, 64, 2, 2, 4, 2);
+    if (ceil_div(rows, 128) * (N / 64) >= 1536) {
+        // a short K: waves of 32x64, which split half as many operands a product (14300 of 32896, 768, 192 + GELU: 41.2 on waves
+        // of 64x32, 38.0 on these; 24000 of 55296, 512, 64 + GELU: 23.5 / 21.8; 6000 of 13824, 1024, 128 + GELU: 17.2 / 16.7;
+        // from K = 384 on the others are even or faster: 7200 of 16448, 1536, 384 + GELU: 59.3 / 62.9)
+        if (K <= 256) VT_PICK(false, 128, 64, 4, 1, 4, 2);
+        VT_PICK(false, 128, 64, 2, 2, 4, 2);
+    }
     VT_PICK(false, 64, 64, 2, 2, 4, 3);
 #undef VT_PICK
 #undef VT_GO
