@@ -280,3 +280,9 @@ def test_from_a_workspace_of_two_floats_a_row(dev, dtype):
     for name, a, b, c in zip("qkv", (dq, dk, dv), ops.sparse_attention_backward(q, k, v, None, g, offsets, 0.125, 64), grads):
         assert float((a.double().cpu() - c).abs().max()) <= TOL[dtype] * float(c.abs().max()), name
         assert dtype == torch.float32 or torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("n", [32, 63, 95, 96, 97, 128, 160, 161, 256, 288, 289, 320])
+def test_scores_kept_between_the_walks(dev, n):
+    """fp32: whole and partial last stages at the edges of three, five and nine kept ones, and one beyond."""
+    test_against_float64(dev, torch.float32, n, [64, 0, 65, 33, 5, 130], 0.125, False)

@@ -261,8 +261,9 @@ __global__ __launch_bounds__(256, 4) void attention_train_kernel(AttnTrain a)
     if (live) M::store(a.out + (row0 + row) * a.o_rs + (int64_t)head * a.o_hs, o, g);
 }
 
-// dQ of 64 query rows of one (sample, head), with their m, 1 / s and delta
-template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_kernel(AttnBack a)
+// dQ of 64 query rows of one (sample, head), with their m, 1 / s and delta.
+// HELD: stages of keys whose scores and dP stay in registers between the two walks (0: they are worked out again)
+template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 : HELD <= 5 ? 3 : 2) void attention_dq_kernel(AttnBack a)
 {
     using B = BackTile<T>;
     using M = BackMath<T>;
@@ -291,13 +292,9 @@ template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_ker
     // ---- m, s and delta of this lane's query: maximum, sum of e and sum of e dP over the lane's keys, then over the four
     // lanes that share the query
     float m = -INFINITY, s = 0.f, sd = 0.f;
-    for (int st = 0; st < stages; st++) {
-        wait_vmcnt<0>();
-        block_barrier();
-        if (st + 1 < stages) kv.load(st + 1);
-        if (!wave_live) continue;
+    f32x4 held_t[HELD > 0 ? HELD : 1][2], held_dp[HELD > 0 ? HELD : 1][2];
+    auto sums = [&](int st, f32x4 (&t)[2], f32x4 (&dp)[2]) {
         const unsigned char *Ks = smem + (st & 1) * 2 * B::HALF, *Vs = Ks + B::HALF;
-        f32x4 t[2], dp[2];
         float mx = m;
 #pragma unroll
         for (int blk = 0; blk < 2; blk++) {
@@ -325,6 +322,25 @@ template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_ker
         s = s * down + (((e[0][0] + e[0][1]) + (e[0][2] + e[0][3])) + ((e[1][0] + e[1][1]) + (e[1][2] + e[1][3])));
         sd = sd * down + (((ed[0][0] + ed[0][1]) + (ed[0][2] + ed[0][3])) + ((ed[1][0] + ed[1][1]) + (ed[1][2] + ed[1][3])));
         m = mx;
+    };
+    auto next_stage = [&](int st, bool values) {
+        wait_vmcnt<0>();
+        block_barrier();
+        if (st + 1 < stages && (values || wid < 2)) kv.load(st + 1);
+    };
+    if constexpr (HELD > 0) {
+        static_for<HELD>([&](auto st_c) {
+            constexpr int st = decltype(st_c)::value;
+            if (st < stages) {
+                next_stage(st, true);
+                if (wave_live) sums(st, held_t[st], held_dp[st]);
+            }
+        });
+    } else {
+        for (int st = 0; st < stages; st++) {
+            next_stage(st, true);
+            if (wave_live) sums(st, held_t[0], held_dp[0]);
+        }
     }
     float all = fmaxf(m, __shfl_xor(m, 16, WAVE));
     all = fmaxf(all, __shfl_xor(all, 32, WAVE));
@@ -349,25 +365,40 @@ template <typename T> __global__ __launch_bounds__(256, 4) void attention_dq_ker
 #pragma unroll
     for (int i = 0; i < 4; i++) dq[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     block_barrier();                                      // the last stage has been read
-    kv.load(0);
-    for (int st = 0; st < stages; st++) {
-        wait_vmcnt<0>();
-        block_barrier();
-        if (st + 1 < stages) kv.load(st + 1);
-        if (!wave_live) continue;
-        const unsigned char *Ks = smem + (st & 1) * 2 * B::HALF, *Vs = Ks + B::HALF;
+    if (HELD == 0 || wid < 2) kv.load(0);                 // scores held: keys only
+    auto add = [&](int st, const f32x4 (&t)[2], const f32x4 (&dp)[2]) {
         f32x4 ds[2];
 #pragma unroll
-        for (int blk = 0; blk < 2; blk++) {
-            const f32x4 t = M::scores(Ks, blk, qf, l, g), dp = M::scores(Vs, blk, df, l, g);
+        for (int blk = 0; blk < 2; blk++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const bool in = st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
-                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(t[r], a.scale_log2, -all));
-                ds[blk][r] = in ? e * (dp[r] - delta) * scale_s : 0.f;
+                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -all));
+                ds[blk][r] = in ? e * (dp[blk][r] - delta) * scale_s : 0.f;
             }
+        M::accumulate(smem + (st & 1) * 2 * B::HALF, ds, dq, l, g);
+    };
+    if constexpr (HELD > 0) {
+        static_for<HELD>([&](auto st_c) {
+            constexpr int st = decltype(st_c)::value;
+            if (st < stages) {
+                next_stage(st, false);
+                if (wave_live) add(st, held_t[st], held_dp[st]);
+            }
+        });
+    } else {
+        for (int st = 0; st < stages; st++) {
+            next_stage(st, true);
+            if (!wave_live) continue;
+            const unsigned char *Ks = smem + (st & 1) * 2 * B::HALF, *Vs = Ks + B::HALF;
+            f32x4 t[2], dp[2];
+#pragma unroll
+            for (int blk = 0; blk < 2; blk++) {
+                t[blk] = M::scores(Ks, blk, qf, l, g);
+                dp[blk] = M::scores(Vs, blk, df, l, g);
+            }
+            add(st, t, dp);
         }
-        M::accumulate(Ks, ds, dq, l, g);
     }
     if (live) M::store((T *)a.dq + (row0 + row) * a.dq_rs + (int64_t)head * a.dq_hs, dq, g);
 }
@@ -463,8 +494,18 @@ template <typename T> static int launch_backward(AttnBack a, int max_rows, hipSt
     VT_REQUIRE(pairs_x * 8 * (qc > kc ? qc : kc) < (1ll << 31), VTDGE_ERR_UNSUPPORTED,
                "sparse_attention_backward: too many workgroups for one launch");
     if (qc > 0) {
-        note_kernel(reinterpret_cast<const void *>(attention_dq_kernel<T>));
-        attention_dq_kernel<T><<<dim3((unsigned)(pairs_x * 8 * qc)), dim3(64 * AB_WAVES), 0, st>>>(a);
+        // fp32, whose products bound the kernel: up to 288 keys the scores and dP of the first walk are kept for the second, the
+        // same bits in three products instead of five.  Us, both kernels, worked out again / kept (samples, heads, keys): 64, 3,
+        // 257: 161 / 127; 128, 6, 257: 366 / 322; 64, 6, 145: 104 / 80; 64, 3, 65: 36.5 / 31.3; 8, 3, 257: 58.4 / 51.6.  bf16
+        // loses more by the registers than it gains: 128, 6, 257: 86 / 101; 64, 6, 145: 30.0 / 29.4.
+        auto kern = attention_dq_kernel<T, 0>;
+        if constexpr (sizeof(T) == 4) {
+            if (a.n <= 3 * AB_ROWS) kern = attention_dq_kernel<T, 3>;
+            else if (a.n <= 5 * AB_ROWS) kern = attention_dq_kernel<T, 5>;
+            else if (a.n <= 9 * AB_ROWS) kern = attention_dq_kernel<T, 9>;
+        }
+        note_kernel(reinterpret_cast<const void *>(kern));
+        kern<<<dim3((unsigned)(pairs_x * 8 * qc)), dim3(64 * AB_WAVES), 0, st>>>(a);
         const int rc = check_launch("sparse_attention_backward");
         if (rc != VTDGE_OK) return rc;
     }
