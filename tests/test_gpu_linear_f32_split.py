@@ -40,7 +40,8 @@ def test_tile_edges(dev, cap, N, K, tile, act, res):
             assert float((got - want).norm()) <= float((plain - want).norm()) * 1.02
 
 
-@pytest.mark.parametrize("scale_a,scale_w", [(1e-30, 1.0), (1e-18, 1e-18), (1e30, 1e-3), (1.0, 1e-35), (1e18, 1e18)])
+@pytest.mark.parametrize("scale_a,scale_w", [(1e-30, 1.0), (1e-18, 1e-18), (1e30, 1e-3), (1.0, 1e-35), (1e18, 1e18),
+                                             (2.0 ** -120, 2.0 ** 60), (2.0 ** 60, 2.0 ** -120)])
 def test_magnitudes(dev, scale_a, scale_w):
     """Every magnitude whose product is an fp32 number comes out with fp32's relative error, also where the smaller bf16
     parts of the operands fall below the smallest bf16 numbers."""

@@ -14,7 +14,9 @@
 //
 // Not covered by the split: an infinity or NaN (the remainders become NaN), a value that rounds to infinity in bf16, and sums
 // that live below the precision of small bf16 values.  All of them show in the result: a block with a sum that is not
-// finite, or not zero and below 2^-80, is worked out again with the fp32 instructions from the operands in memory.
+// finite, or not zero and below 2^-80, is worked out again with the fp32 instructions from the operands in memory.  A sum of
+// 2^-80 and above hides what small bf16 values lose (2^-134 of an operand) only where the other operand is not huge: weights
+// from 2^20 on, whose activations may be that small, and those below 2^-100, are put down as NaN and so join the others.
 #include "common.h"
 
 namespace vtdge {
@@ -46,6 +48,8 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float *__restri
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         float x = __uint_as_float(e < 2 ? lo[2 * e] : hi[2 * e - 4]), y = __uint_as_float(e < 2 ? lo[2 * e + 1] : hi[2 * e - 3]);
+        x = x == 0.f || (fabsf(x) >= 0x1p-100f && fabsf(x) < 0x1p20f) ? x : __builtin_nanf("");
+        y = y == 0.f || (fabsf(y) >= 0x1p-100f && fabsf(y) < 0x1p20f) ? y : __builtin_nanf("");
 #pragma unroll
         for (int p = 0; p < 3; p++) {
             part[p][e] = pack_bf16x2(x, y);
