@@ -348,6 +348,27 @@ def test_layernorm(dev, dtype, rows, C):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("C", [64, 128, 256, 384, 512, 768, 1536])
+def test_layernorm_rows_apart(dev, dtype, C):
+    """A row's result does not depend on the rows whose sums are reduced with it: one to nine rows, constant, infinite and NaN
+    ones between, bit for bit the row alone."""
+    from vtpack_amd import ops
+    if dtype == torch.float32 and C > 768:
+        C = 640
+    x = _t(randn(37, 9, C) * 2 + 0.5, dev, dtype)
+    x[2], x[4, 3], x[6, 0] = 1.5, float("inf"), float("nan")
+    w, b = _t(randn(38, C) * 0.2 + 1, dev, dtype), _t(randn(39, C) * 0.1, dev, dtype)
+    alone = torch.cat([ops.layernorm(x[r:r + 1].clone(), w, b, 1e-6) for r in range(9)])
+    good = [0, 1, 3, 5, 7, 8]
+    want = torch.nn.functional.layer_norm(x[good].double(), (C,), w.double(), b.double(), 1e-6)
+    assert_close(alone[good].float(), want.float(), dtype, "layernorm")
+    assert torch.equal(alone[2], b) and bool(alone[[4, 6]].isnan().all())
+    for rows in range(1, 10):
+        got = ops.layernorm(x[:rows].clone(), w, b, 1e-6)
+        assert torch.equal(got.isnan(), alone[:rows].isnan()) and torch.equal(got.nan_to_num(), alone[:rows].nan_to_num())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,period,C", [(4096, 1024, 64), (1537, 29, 384), (640, 64, 512), (300, 300, 768)])
 def test_layernorm_with_rows_added(dev, dtype, rows, period, C):
     """LayerNorm followed by `+ pos_embed` in one pass: bit for bit the LayerNorm kernel's result plus the addend

@@ -1292,6 +1292,23 @@ void decompress_route_kernel(
 // --------------------------------------------------------------- layernorm
 constexpr int LN_RPW = 4;   // rows per wave: their loads are issued together so that enough bytes are in flight
 
+// f of the values of a wave's rows, which for GS = 64 are the same in all lanes
+template <int GS, int RB, class F> __device__ __forceinline__ void each_row(float (&v)[RB], F &&f)
+{
+    if constexpr (GS == 64) {
+        static_assert(RB == 4, "row r in the lanes 4 i + r");
+        const float lo = threadIdx.x & 1 ? v[1] : v[0], hi = threadIdx.x & 1 ? v[3] : v[2];
+        float x = threadIdx.x & 2 ? hi : lo;
+        x = f(x);
+#pragma unroll
+        for (int r = 0; r < RB; r++)
+            v[r] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), r));
+    } else {
+#pragma unroll
+        for (int r = 0; r < RB; r++) v[r] = f(v[r]);
+    }
+}
+
 template <typename T, int NIT, int GS>   // NIT = 16-byte vectors per lane = ceil(C / VEC / 64) (1 when GS < 64)
 __global__ __launch_bounds__(256) void layernorm_kernel(const T *__restrict__ x, const T *__restrict__ w,
                                                          const T *__restrict__ bsrc, T *__restrict__ out,
@@ -1317,6 +1334,7 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const T *__restrict__ x,
             // input rows come in groups of x_group_rows dense rows, the groups x_group_stride elements apart
             const int64_t rr = row0 + r;
             const int64_t src = x_group_rows > 0 ? (rr / x_group_rows) * x_group_stride + (rr % x_group_rows) * C : rr * C;
+            raw[r][it] = u32x4{0u, 0u, 0u, 0u};
             if (v < nvec && rr < live) raw[r][it] = *reinterpret_cast<const u32x4 *>(x + src + v * VEC);
         }
     float ww[NIT][VEC], bb[NIT][VEC];
@@ -1328,47 +1346,67 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const T *__restrict__ x,
             Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(bsrc + v * VEC), bb[it]);
         }
     }
+    // The rows' sums are reduced RB rows together, independent chains, and a wave that holds whole rows takes their quotients
+    // and roots once, row r in the lanes 4 i + r, not once a row; the same bits.  Us, a row after the other / together (rows,
+    // channels): bf16 65792, 384: 24.1 / 21.4; 65536, 320: 20.8 / 18.3; 16384, 512: 9.4 / 8.2; 25443, 768: 19.8 / 19.0; fp32
+    // 32896, 192: 11.7 / 10.9; 9000, 768: 11.1 / 10.5; 262144, 128: 52.1 / 48.9.  Short bf16 rows, several a wave, are bound by
+    // memory and lose by the registers: 1048576, 64: 49.7 / 53.8; 262144, 128: 27.9 / 30.6.
+    constexpr int RB = GS == 64 || sizeof(T) == 4 ? LN_RPW : 1;
 #pragma unroll
-    for (int r = 0; r < LN_RPW; r++) {
-        if (row0 + r >= live) break;
-        float vals[NIT][VEC];
-        float s = 0.f;
+    for (int r0 = 0; r0 < LN_RPW; r0 += RB) {
+        if (row0 + r0 >= live) break;
+        float mean[RB], rstd[RB];
 #pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            if (it * WAVE + lane < nvec) {
-                Elem<T>::unpack(raw[r][it], vals[it]);
+        for (int r = 0; r < RB; r++) {
+            mean[r] = 0.f;
 #pragma unroll
-                for (int c = 0; c < VEC; c++) s += vals[it][c];
+            for (int it = 0; it < NIT; it++) {
+                float f[VEC];
+                Elem<T>::unpack(raw[r0 + r][it], f);
+#pragma unroll
+                for (int c = 0; c < VEC; c++) mean[r] += f[c];
             }
         }
-        const float mean = group_sum<GS>(s) / (float)C;
-        float q = 0.f;
+        group_sum_n<GS, RB>(mean);
+        each_row<GS, RB>(mean, [&](float s) { return s / (float)C; });
 #pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            if (it * WAVE + lane < nvec) {
+        for (int r = 0; r < RB; r++) {
+            rstd[r] = 0.f;
 #pragma unroll
-                for (int c = 0; c < VEC; c++) {
-                    const float dlt = vals[it][c] - mean;
-                    q += dlt * dlt;
-                }
+            for (int it = 0; it < NIT; it++) {
+                float f[VEC];
+                Elem<T>::unpack(raw[r0 + r][it], f);
+                if (it * WAVE + lane < nvec)
+#pragma unroll
+                    for (int c = 0; c < VEC; c++) {
+                        const float dlt = f[c] - mean[r];
+                        rstd[r] += dlt * dlt;
+                    }
             }
         }
-        const float rstd = 1.0f / sqrtf(group_sum<GS>(q) / (float)C + eps);
+        group_sum_n<GS, RB>(rstd);
+        each_row<GS, RB>(rstd, [&](float q) { return 1.0f / sqrtf(q / (float)C + eps); });
 #pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            const int v = it * WAVE + lane;
-            if (v < nvec) {
-                float y[VEC];
+        for (int r = 0; r < RB; r++) {
+            const int64_t row = row0 + r0 + r;
+            if (row >= live) break;
 #pragma unroll
-                for (int c = 0; c < VEC; c++) y[c] = (vals[it][c] - mean) * rstd * ww[it][c] + bb[it][c];
-                if (add != nullptr) {
-                    float a[VEC];
-                    Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(add + ((row0 + r) % add_rows) * C + v * VEC), a);
-                    Elem<T>::unpack(Elem<T>::pack(y), y);
+            for (int it = 0; it < NIT; it++) {
+                const int v = it * WAVE + lane;
+                if (v < nvec) {
+                    float f[VEC], y[VEC];
+                    Elem<T>::unpack(raw[r0 + r][it], f);
 #pragma unroll
-                    for (int c = 0; c < VEC; c++) y[c] += a[c];
+                    for (int c = 0; c < VEC; c++) y[c] = (f[c] - mean[r]) * rstd[r] * ww[it][c] + bb[it][c];
+                    if (add != nullptr) {
+                        float a[VEC];
+                        Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(add + (row % add_rows) * C + v * VEC), a);
+                        Elem<T>::unpack(Elem<T>::pack(y), y);
+#pragma unroll
+                        for (int c = 0; c < VEC; c++) y[c] += a[c];
+                    }
+                    *reinterpret_cast<u32x4 *>(out + row * C + v * VEC) = Elem<T>::pack(y);
                 }
-                *reinterpret_cast<u32x4 *>(out + (row0 + r) * (int64_t)C + v * VEC) = Elem<T>::pack(y);
             }
         }
     }
