@@ -1325,6 +1325,12 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const T *__restrict__ x,
         (((int64_t)blockIdx.x * ROWS_PER_BLOCK + (threadIdx.x >> 6)) * (WAVE / GS) + (threadIdx.x & 63) / GS) * LN_RPW;
     if (row0 >= live) return;
     const int nvec = C / VEC;
+    // The rows' sums are reduced RB rows together, independent chains, and a wave that holds whole rows takes their quotients
+    // and roots once, row r in the lanes 4 i + r, not once a row; the same bits.  Us, a row after the other / together (rows,
+    // channels): bf16 65792, 384: 24.1 / 21.4; 65536, 320: 20.8 / 18.3; 16384, 512: 9.4 / 8.2; 25443, 768: 19.8 / 19.0; fp32
+    // 32896, 192: 11.7 / 10.9; 9000, 768: 11.1 / 10.5; 262144, 128: 52.1 / 48.9.  Short bf16 rows, several a wave, are bound by
+    // memory and lose by the registers: 1048576, 64: 49.7 / 53.8; 262144, 128: 27.9 / 30.6.
+    constexpr int RB = GS == 64 || sizeof(T) == 4 ? LN_RPW : 1;
     u32x4 raw[LN_RPW][NIT];
 #pragma unroll
     for (int r = 0; r < LN_RPW; r++)
@@ -1334,7 +1340,7 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const T *__restrict__ x,
             // input rows come in groups of x_group_rows dense rows, the groups x_group_stride elements apart
             const int64_t rr = row0 + r;
             const int64_t src = x_group_rows > 0 ? (rr / x_group_rows) * x_group_stride + (rr % x_group_rows) * C : rr * C;
-            raw[r][it] = u32x4{0u, 0u, 0u, 0u};
+            if (RB > 1) raw[r][it] = u32x4{0u, 0u, 0u, 0u};
             if (v < nvec && rr < live) raw[r][it] = *reinterpret_cast<const u32x4 *>(x + src + v * VEC);
         }
     float ww[NIT][VEC], bb[NIT][VEC];
@@ -1346,15 +1352,52 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const T *__restrict__ x,
             Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(bsrc + v * VEC), bb[it]);
         }
     }
-    // The rows' sums are reduced RB rows together, independent chains, and a wave that holds whole rows takes their quotients
-    // and roots once, row r in the lanes 4 i + r, not once a row; the same bits.  Us, a row after the other / together (rows,
-    // channels): bf16 65792, 384: 24.1 / 21.4; 65536, 320: 20.8 / 18.3; 16384, 512: 9.4 / 8.2; 25443, 768: 19.8 / 19.0; fp32
-    // 32896, 192: 11.7 / 10.9; 9000, 768: 11.1 / 10.5; 262144, 128: 52.1 / 48.9.  Short bf16 rows, several a wave, are bound by
-    // memory and lose by the registers: 1048576, 64: 49.7 / 53.8; 262144, 128: 27.9 / 30.6.
-    constexpr int RB = GS == 64 || sizeof(T) == 4 ? LN_RPW : 1;
+    if constexpr (RB == 1) {
 #pragma unroll
-    for (int r0 = 0; r0 < LN_RPW; r0 += RB) {
-        if (row0 + r0 >= live) break;
+        for (int r = 0; r < LN_RPW; r++) {
+            if (row0 + r >= live) break;
+            float vals[NIT][VEC];
+            float s = 0.f;
+#pragma unroll
+            for (int it = 0; it < NIT; it++) {
+                if (it * WAVE + lane < nvec) {
+                    Elem<T>::unpack(raw[r][it], vals[it]);
+#pragma unroll
+                    for (int c = 0; c < VEC; c++) s += vals[it][c];
+                }
+            }
+            const float mean = group_sum<GS>(s) / (float)C;
+            float q = 0.f;
+#pragma unroll
+            for (int it = 0; it < NIT; it++) {
+                if (it * WAVE + lane < nvec) {
+#pragma unroll
+                    for (int c = 0; c < VEC; c++) {
+                        const float dlt = vals[it][c] - mean;
+                        q += dlt * dlt;
+                    }
+                }
+            }
+            const float rstd = 1.0f / sqrtf(group_sum<GS>(q) / (float)C + eps);
+#pragma unroll
+            for (int it = 0; it < NIT; it++) {
+                const int v = it * WAVE + lane;
+                if (v < nvec) {
+                    float y[VEC];
+#pragma unroll
+                    for (int c = 0; c < VEC; c++) y[c] = (vals[it][c] - mean) * rstd * ww[it][c] + bb[it][c];
+                    if (add != nullptr) {
+                        float a[VEC];
+                        Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(add + ((row0 + r) % add_rows) * C + v * VEC), a);
+                        Elem<T>::unpack(Elem<T>::pack(y), y);
+#pragma unroll
+                        for (int c = 0; c < VEC; c++) y[c] += a[c];
+                    }
+                    *reinterpret_cast<u32x4 *>(out + (row0 + r) * (int64_t)C + v * VEC) = Elem<T>::pack(y);
+                }
+            }
+        }
+    } else {
         float mean[RB], rstd[RB];
 #pragma unroll
         for (int r = 0; r < RB; r++) {
@@ -1362,7 +1405,7 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const T *__restrict__ x,
 #pragma unroll
             for (int it = 0; it < NIT; it++) {
                 float f[VEC];
-                Elem<T>::unpack(raw[r0 + r][it], f);
+                Elem<T>::unpack(raw[r][it], f);
 #pragma unroll
                 for (int c = 0; c < VEC; c++) mean[r] += f[c];
             }
@@ -1375,7 +1418,7 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const T *__restrict__ x,
 #pragma unroll
             for (int it = 0; it < NIT; it++) {
                 float f[VEC];
-                Elem<T>::unpack(raw[r0 + r][it], f);
+                Elem<T>::unpack(raw[r][it], f);
                 if (it * WAVE + lane < nvec)
 #pragma unroll
                     for (int c = 0; c < VEC; c++) {
@@ -1388,24 +1431,23 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const T *__restrict__ x,
         each_row<GS, RB>(rstd, [&](float q) { return 1.0f / sqrtf(q / (float)C + eps); });
 #pragma unroll
         for (int r = 0; r < RB; r++) {
-            const int64_t row = row0 + r0 + r;
-            if (row >= live) break;
+            if (row0 + r >= live) break;
 #pragma unroll
             for (int it = 0; it < NIT; it++) {
                 const int v = it * WAVE + lane;
                 if (v < nvec) {
                     float f[VEC], y[VEC];
-                    Elem<T>::unpack(raw[r0 + r][it], f);
+                    Elem<T>::unpack(raw[r][it], f);
 #pragma unroll
                     for (int c = 0; c < VEC; c++) y[c] = (f[c] - mean[r]) * rstd[r] * ww[it][c] + bb[it][c];
                     if (add != nullptr) {
                         float a[VEC];
-                        Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(add + (row % add_rows) * C + v * VEC), a);
+                        Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(add + ((row0 + r) % add_rows) * C + v * VEC), a);
                         Elem<T>::unpack(Elem<T>::pack(y), y);
 #pragma unroll
                         for (int c = 0; c < VEC; c++) y[c] += a[c];
                     }
-                    *reinterpret_cast<u32x4 *>(out + row * C + v * VEC) = Elem<T>::pack(y);
+                    *reinterpret_cast<u32x4 *>(out + (row0 + r) * (int64_t)C + v * VEC) = Elem<T>::pack(y);
                 }
             }
         }
