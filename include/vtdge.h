@@ -335,12 +335,16 @@ int vtdge_linear_prepacked(const void *A, int64_t lda, const void *W, const void
  *   vtdge_linear_split_size    *bytes = size of the split copy of W [N, K], or 0 when there is none (N no multiple of 64, K
  *                              none of 32)
  *   vtdge_linear_split         fills `split` (16-byte aligned, *bytes long) from W; VTDGE_ERR_UNSUPPORTED where the size is 0
+ *   vtdge_linear_split_set     the same for `count` weights in one launch: weights_host[i] [N_host[i], K_host[i]] to byte
+ *                              at_host[i] of `split` (all four tables on the host)
  *   vtdge_linear_split_wanted  1 where vtdge_linear_prepacked uses the copy for that many rows, 0 where W is multiplied as it
  *                              is, with or without one
  * W itself is always required: blocks of the result with infinities, NaN or values outside the range of the split are
  * worked out from it. */
 int vtdge_linear_split_size(int N, int K, int64_t *bytes);
 int vtdge_linear_split(const void *W, int N, int K, void *split, void *stream);
+int vtdge_linear_split_set(const void *const *weights_host, const int32_t *N_host, const int32_t *K_host, const int64_t *at_host,
+                           int count, void *split, void *stream);
 int vtdge_linear_split_wanted(int64_t rows, int N, int K);
 
 /* Patch embedding, position embedding included: the stride-P P x P convolution of the reference's PatchEmbed
@@ -518,8 +522,8 @@ int vtdge_block_tail(const void *o, const void *comp, const void *proj_weight, c
  *                of them out of {1, 2, 4}); head dim 32 or 64; sr > 1 only without extra tokens
  *   params_host  HOST table of device pointers, VTDGE_CHAIN_PARAMS per block, in this order (NULL where absent):
  *                norm1 weight, bias, norm2 weight, bias, router weight, bias, splits (int64); q weight, bias, kv weight,
- *                bias, proj weight, bias, fc1 weight, bias, fc2 weight, bias; packed copies (vtdge_linear_prepack) of
- *                the q, kv, proj, fc1, fc2 weights; folded weight, column records (vtdge_layernorm_fold) and packed
+ *                bias, proj weight, bias, fc1 weight, bias, fc2 weight, bias; packed copies (vtdge_linear_prepack, bf16;
+ *                split copies of fp32 weights are made in `scratch`) of the q, kv, proj, fc1, fc2 weights; folded weight, column records (vtdge_layernorm_fold) and packed
  *                copy of the folded weight for norm1 -> q, norm1 -> kv, norm2 -> fc1; with sr > 1 the reduction's
  *                weight in [C, sr, sr, C] order, bias, and its norm's weight, bias.  The folded entries are needed
  *                where vtdge_chain_layout says so

@@ -58,6 +58,7 @@ SIGNATURES = {
     "vtdge_linear_prepacked": [_p, _l, _p, _p, _p, _p, _l, _p, _l, _p, _l, _i, _i, _i, _i, _p],
     "vtdge_linear_split_size": [_i, _i, _p],
     "vtdge_linear_split": [_p, _i, _i, _p, _p],
+    "vtdge_linear_split_set": [_p, _p, _p, _p, _i, _p, _p],
     "vtdge_linear_split_wanted": [_l, _i, _i],
     "vtdge_linear_stats": [_p, _l, _p, _p, _p, _p, _l, _p, _l, _p, _f, _p, _l, _i, _i, _i, _p],
     "vtdge_layernorm_stats": [_p, _p, _p, _l, _i, _f, _i, _p],

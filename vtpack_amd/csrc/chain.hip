@@ -34,6 +34,8 @@ __global__ __launch_bounds__(256) void front_rows_kernel(u32x4 *__restrict__ x, 
     if (i < words) clear[i] = 0ull;
 }
 
+constexpr int LINEARS = 5;         // of a block: q, kv, proj, fc1, fc2, as in the parameter table
+
 struct ChainPlan {
     int64_t rows, cap, regions;
     int esz, N, n_kv;              // tokens per sample, keys per sample
@@ -43,6 +45,9 @@ struct ChainPlan {
     bool tail;                     // narrow bf16 rows: everything behind attention as one kernel
     bool ln_kvq, ln_fc1;           // few rows: norm1 inside the kv and q Linear, norm2 inside fc1
     int64_t ws_words;
+    bool split[LINEARS];           // fp32 Linears on split weights
+    int split_blocks;              // blocks whose weights are split in one launch, 0: none are
+    int64_t split_at[LINEARS], split_sz, split0;                         // in `scratch`, of one block
     // byte offsets
     int64_t ints_total, big_total, scratch_total;
     int64_t gate0, off0, len0, ws0, gate_sz, off_sz, len_sz, ws_sz;      // in `ints`, block i at start + i * size
@@ -50,7 +55,58 @@ struct ChainPlan {
     int64_t xln, red, kv, comp_ln, q, o, q1, q1_ln, hid, rec_x[2], rec_c[2], rec2, idx[2], cnt[2], rrows[2];   // in `scratch`
 };
 
+#define VT_TRY(expr)                      \
+    do {                                  \
+        const int vt_rc = (expr);         \
+        if (vt_rc != VTDGE_OK) return vt_rc; \
+    } while (0)
+
 static int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
+
+// A block's Linears in the order of the parameter table: what they multiply, and whether on split weights where that is faster
+struct SplitShape {
+    int64_t rows;
+    int N, K;
+    bool wanted;
+};
+static SplitShape split_shape(const vtdge_chain *c, const ChainPlan &p, int linear)
+{
+    const bool f32 = c->dtype == VTDGE_F32;
+    switch (linear) {
+    case 0: return {p.cap, c->C, c->C, f32 && !p.ln_kvq};
+    case 1: return {(int64_t)c->B * p.n_kv, 2 * c->C, c->C, f32 && !p.ln_kvq};
+    case 2: return {p.cap, c->C, c->C, f32};
+    case 3: return {p.cap, c->hidden, c->C, f32 && !p.ln_fc1};
+    default: return {p.cap, c->C, c->hidden, f32};
+    }
+}
+
+// Split weights are made anew by every call: it multiplies by the weights as they are when it runs, in a replayed graph and
+// beside calls on other streams too.  As many blocks a launch as stay in the last-level cache until they are read.  GPU time of
+// a forward at 256 px, us, without split weights / split by the call / kept from an earlier one (pictures, channels): 128, 192:
+// 3367 / 3023 / 3001; 12, 384: 1730 / 1528 / 1485; 32, 384: 2880 / 2546 / 2500; 8, 768: 3162 / 2863 / 2668; 2, 768: 1804 / 1741 /
+// 1685.
+constexpr int64_t SPLIT_ROOM = 64 << 20;
+constexpr int SPLIT_BLOCKS = 16;
+
+static int split_block_weights(const vtdge_chain *c, const ChainPlan &p, const void *const *params, int first, char *scratch,
+                               void *stream)
+{
+    const void *W[SPLIT_BLOCKS * LINEARS];
+    int32_t N[SPLIT_BLOCKS * LINEARS], K[SPLIT_BLOCKS * LINEARS];
+    int64_t at[SPLIT_BLOCKS * LINEARS];
+    int count = 0;
+    for (int b = 0; b < p.split_blocks && first + b < c->depth; b++)
+        for (int j = 0; j < LINEARS; j++) {
+            if (!p.split[j]) continue;
+            const SplitShape w = split_shape(c, p, j);
+            W[count] = params[(int64_t)(first + b) * P_COUNT + P_QW + 2 * j];
+            N[count] = w.N;
+            K[count] = w.K;
+            at[count++] = b * p.split_sz + p.split_at[j];
+        }
+    return vtdge_linear_split_set(W, N, K, at, count, scratch + p.split0, stream);
+}
 
 static int plan_chain(const vtdge_chain *c, ChainPlan &p)
 {
@@ -126,15 +182,24 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
         p.cnt[i] = take((p.regions + 15) / 16 * 16);
         p.rrows[i] = take(p.regions * 4);
     }
+    p.split_sz = p.split_blocks = 0;
+    for (int j = 0; j < LINEARS; j++) {
+        const SplitShape w = split_shape(c, p, j);
+        int64_t bytes = 0;
+        if (w.wanted && vtdge_linear_split_wanted(w.rows, w.N, w.K)) VT_TRY(vtdge_linear_split_size(w.N, w.K, &bytes));
+        p.split[j] = bytes > 0;
+        p.split_at[j] = p.split_sz;
+        p.split_sz += align256(bytes);
+    }
+    if (p.split_sz > 0) {
+        const int64_t fit = SPLIT_ROOM / p.split_sz;
+        p.split_blocks = fit < 1 ? 1 : fit > SPLIT_BLOCKS ? SPLIT_BLOCKS : (int)fit;
+        if (p.split_blocks > c->depth) p.split_blocks = c->depth;
+        p.split0 = take(p.split_sz * p.split_blocks);
+    }
     p.scratch_total = at;
     return VTDGE_OK;
 }
-
-#define VT_TRY(expr)                      \
-    do {                                  \
-        const int vt_rc = (expr);         \
-        if (vt_rc != VTDGE_OK) return vt_rc; \
-    } while (0)
 
 // A pair of events per host thread and device for the fork to the side stream and the join behind it; each is recorded
 // anew before it is waited for.  They end with their thread (not in a process forked from it, where the runtime is not to be
@@ -222,8 +287,12 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
         char *kv = scratch + p.kv, *q = scratch + p.q, *o = scratch + p.o, *q1 = scratch + p.q1, *hid = scratch + p.hid;
         char *xout = Q ? big + p.tok0 + i * p.tok_sz : out;
         char *ngate = Q ? ints + p.gate0 + (i + 1) * p.gate_sz : nullptr;
-        // the copy of a weight for so many rows: bf16 packed (made from 2048 rows on), fp32 split
-        auto copy_for = [&](int which, int64_t rows) { return dt == VTDGE_F32 || rows >= 2048 ? P[which] : nullptr; };
+        // the copy of a weight for so many rows: bf16 packed (from 2048 rows on), fp32 split
+        auto copy_for = [&](int which, int64_t rows) -> const void * {
+            if (dt != VTDGE_F32) return rows >= 2048 ? P[which] : nullptr;
+            const int j = which - P_QP;
+            return p.split[j] ? scratch + p.split0 + i % p.split_blocks * p.split_sz + p.split_at[j] : nullptr;
+        };
         auto pk = [&](int which) { return copy_for(which, p.rows); };
 
         if (p.folded) {
@@ -272,6 +341,8 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
                                           comp_ln ? P[P_N1B] : nullptr, c->eps1, B, N, C, W, extra, dt, routing));
                 }
             }
+            if (p.split_blocks > 0 && i % p.split_blocks == 0)       // on the stream of the Linears that read them, and read the last
+                VT_TRY(split_block_weights(c, p, params, i, scratch, stream));
             if (p.ln_kvq) {
                 VT_TRY(vtdge_layernorm_linear(x, C, P[P_KVW], P[P_KVB], kv, nullptr, p.rows, 2 * C, comp, C, P[P_QW], P[P_QB],
                                               q, live, p.cap, C, P[P_N1W], P[P_N1B], c->eps1, C, VTDGE_ACT_NONE, dt,

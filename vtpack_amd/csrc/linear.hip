@@ -207,9 +207,10 @@ int launch_linear_small(const void *A, int64_t lda, const void *W, const void *b
                         void *out, int64_t ldo, const int64_t *rows_dev, int64_t rows, int N, int K, int act,
                         hipStream_t st);
 
-// fp32 on the bf16 matrix instructions, from a weight split in advance (linear_dma_split.hip)
+// fp32 on the bf16 matrix instructions, from a split weight (linear_dma_split.hip)
 int64_t linear_split_size(int N, int K);
-int split_linear_weight(const void *W, int N, int K, void *split, hipStream_t st);
+int split_linear_weights(const void *const *W, const int32_t *N, const int32_t *K, const int64_t *at, int count, void *split,
+                         hipStream_t st);
 int launch_linear_dma_split(const void *A, int64_t lda, const void *W, const void *split, const void *bias, const void *res,
                       int64_t ldr, void *out, int64_t ldo, const int64_t *rows_dev, int64_t rows, int N, int K, int act,
                       hipStream_t st);
@@ -475,13 +476,26 @@ extern "C" int vtdge_linear_split_size(int N, int K, int64_t *bytes)
     return VTDGE_OK;
 }
 
+extern "C" int vtdge_linear_split_set(const void *const *weights_host, const int32_t *N_host, const int32_t *K_host,
+                                      const int64_t *at_host, int count, void *split, void *stream)
+{
+    VT_REQUIRE(weights_host && N_host && K_host && at_host && split, VTDGE_ERR_ARG, "linear_split: NULL operand");
+    VT_REQUIRE(count > 0, VTDGE_ERR_ARG, "linear_split: %d weights", count);
+    for (int j = 0; j < count; j++) {
+        const int N = N_host[j], K = K_host[j];
+        VT_REQUIRE(weights_host[j] != nullptr, VTDGE_ERR_ARG, "linear_split: NULL operand");
+        VT_REQUIRE(N > 0 && K > 0, VTDGE_ERR_ARG, "linear_split: bad sizes N=%d K=%d", N, K);
+        VT_REQUIRE(linear_split_size(N, K) > 0, VTDGE_ERR_UNSUPPORTED, "linear_split: no split copy for N=%d K=%d", N, K);
+        VT_REQUIRE((((uintptr_t)weights_host[j] | (uintptr_t)split | (uintptr_t)at_host[j]) & 15) == 0 && at_host[j] >= 0,
+                   VTDGE_ERR_ARG, "linear_split: operands must be 16-byte aligned");
+    }
+    return split_linear_weights(weights_host, N_host, K_host, at_host, count, split, (hipStream_t)stream);
+}
+
 extern "C" int vtdge_linear_split(const void *W, int N, int K, void *split, void *stream)
 {
-    VT_REQUIRE(W && split, VTDGE_ERR_ARG, "linear_split: NULL operand");
-    VT_REQUIRE(N > 0 && K > 0, VTDGE_ERR_ARG, "linear_split: bad sizes N=%d K=%d", N, K);
-    VT_REQUIRE(linear_split_size(N, K) > 0, VTDGE_ERR_UNSUPPORTED, "linear_split: no split copy for N=%d K=%d", N, K);
-    VT_REQUIRE((((uintptr_t)W | (uintptr_t)split) & 15) == 0, VTDGE_ERR_ARG, "linear_split: operands must be 16-byte aligned");
-    return split_linear_weight(W, N, K, split, (hipStream_t)stream);
+    const int64_t at = 0;
+    return vtdge_linear_split_set(&W, &N, &K, &at, 1, split, stream);
 }
 
 extern "C" int vtdge_linear_split_wanted(int64_t rows, int N, int K)

@@ -34,15 +34,29 @@ constexpr int DKB = 128;                   // bytes of a row of A per stage
 // a phase of a fragment read, lie in 16 different bank groups.
 __device__ __forceinline__ int64_t packed_block(int n16, int kt, int nk, int p) { return (((int64_t)n16 * nk + kt) * 3 + p) * 1024; }
 
-__global__ __launch_bounds__(256) void split_weight_kernel(const float *__restrict__ W, unsigned char *__restrict__ packed, int K,
-                                                           int64_t pieces)
+// Weights of one launch, and the workgroups up to and including each one's (vtdge_linear_split_set)
+constexpr int SPLIT_SET = 80;
+struct SplitSet {
+    struct {
+        const float *W;
+        unsigned char *packed;
+        int N, K;
+    } of[SPLIT_SET];
+    int end[SPLIT_SET], count;
+};
+
+__global__ __launch_bounds__(256) void split_weights_kernel(const SplitSet set)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;      // piece q of (row, slab)
-    if (i >= pieces) return;
-    const int nk = K / 32;
-    const int q = (int)(i & 3), kt = (int)(i / 4 % nk);
-    const int64_t n = i / 4 / nk;
-    const float *src = W + n * K + kt * 32 + 16 * (q >> 1) + 4 * (q & 1);
+    int j = 0;
+    for (int step = 64; step > 0; step >>= 1)               // the first weight that ends behind this workgroup
+        if (j + step <= set.count - 1 && (int)blockIdx.x >= set.end[j + step - 1]) j += step;
+    const float *W = set.of[j].W;
+    unsigned char *packed = set.of[j].packed;
+    const int K = set.of[j].K;
+    const int i = ((int)blockIdx.x - (j > 0 ? set.end[j - 1] : 0)) * 256 + threadIdx.x;      // piece q of (row, slab)
+    const int nk = K / 32, q = i & 3, n = i / 4 / nk, kt = i / 4 - n * nk;
+    if (n >= set.of[j].N) return;
+    const float *src = W + (int64_t)n * K + kt * 32 + 16 * (q >> 1) + 4 * (q & 1);
     const u32x4 lo = *reinterpret_cast<const u32x4 *>(src), hi = *reinterpret_cast<const u32x4 *>(src + 8);
     u32x4 part[3];
 #pragma unroll
@@ -59,8 +73,7 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float *__restri
     }
 #pragma unroll
     for (int p = 0; p < 3; p++)
-        *reinterpret_cast<u32x4 *>(packed + packed_block((int)(n / 16), kt, nk, p) + (n & 15) * 64 +
-                                   ((q ^ ((int)(n >> 2) & 3)) << 4)) = part[p];
+        *reinterpret_cast<u32x4 *>(packed + packed_block(n / 16, kt, nk, p) + (n & 15) * 64 + ((q ^ (n >> 2 & 3)) << 4)) = part[p];
 }
 
 // The walk over the tiles is that of linear_dma_kernel: m-tile t on XCD t % 8, n-fastest inside an XCD.
@@ -323,14 +336,31 @@ static int go(const float *A, int64_t lda, const float *W, const void *packed, c
     return check_launch("linear");
 }
 
-int64_t linear_split_size(int N, int K) { return N % 64 == 0 && K % 32 == 0 ? (int64_t)N * K * 6 : 0; }
-
-int split_linear_weight(const void *W, int N, int K, void *split, hipStream_t st)
+int64_t linear_split_size(int N, int K)
 {
-    const int64_t pieces = (int64_t)N * K / 8;
-    note_kernel(reinterpret_cast<const void *>(split_weight_kernel));
-    split_weight_kernel<<<(unsigned)ceil_div(pieces, 256), 256, 0, st>>>((const float *)W, (unsigned char *)split, K, pieces);
-    return check_launch("linear_split");
+    return N % 64 == 0 && K % 32 == 0 && (int64_t)N * K < (1ll << 33) ? (int64_t)N * K * 6 : 0;      // pieces in 31 bits
+}
+
+int split_linear_weights(const void *const *W, const int32_t *N, const int32_t *K, const int64_t *at, int count, void *split,
+                         hipStream_t st)
+{
+    for (int first = 0; first < count; first += SPLIT_SET) {
+        SplitSet set;
+        int64_t end = 0;
+        set.count = count - first < SPLIT_SET ? count - first : SPLIT_SET;
+        for (int j = 0; j < set.count; j++) {
+            const int x = first + j;
+            set.of[j] = {(const float *)W[x], (unsigned char *)split + at[x], N[x], K[x]};
+            end += ceil_div((int64_t)N[x] * K[x] / 8, 256);
+            VT_REQUIRE(end < (1ll << 31), VTDGE_ERR_UNSUPPORTED, "linear_split: too many workgroups for one launch");
+            set.end[j] = (int)end;
+        }
+        note_kernel(reinterpret_cast<const void *>(split_weights_kernel));
+        split_weights_kernel<<<(unsigned)end, 256, 0, st>>>(set);
+        const int rc = check_launch("linear_split");
+        if (rc != VTDGE_OK) return rc;
+    }
+    return VTDGE_OK;
 }
 
 int launch_linear_dma_split(const void *A, int64_t lda, const void *W, const void *split, const void *bias, const void *res, int64_t ldr,

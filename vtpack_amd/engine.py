@@ -130,8 +130,6 @@ def prepare(model):
             mod._vtdge_khwc = None
         if isinstance(mod, torch.nn.Linear) and mod.weight.is_cuda and mod.weight.dtype == torch.bfloat16:
             ops.packed_weight(mod.weight)
-        if isinstance(mod, torch.nn.Linear) and mod.weight.is_cuda and mod.weight.dtype == torch.float32:
-            ops.split_weight(mod.weight)
         # a block's LayerNorms folded into the Linears behind them (see FOLD_NORMS)
         if FOLD_NORMS and all(hasattr(mod, name) for name in ("norm1", "norm2", "attn", "mlp")):
             for norm, lin in ((mod.norm1, getattr(mod.attn, "kv", None)), (mod.norm1, getattr(mod.attn, "q", None)),
@@ -150,11 +148,11 @@ def prepare(model):
         extra = model.num_tokens if hasattr(model, "blocks") else int(i == len(chains) - 1)
         plan = _chain_plan(blocks, w.dtype, w.device, w.shape[1], extra)
         if plan is not None:
-            _chain_table(plan, blocks, False, (False,) * 5)
+            _chain_table(plan, blocks, False, False)
             if w.dtype == torch.bfloat16:
                 c = plan.common
                 _chain_table(plan, blocks, c["C"] == 384 and c["sr"] == 1 and c["hidden"] % 384 == 0
-                             and c["hidden"] <= 3072, (True,) * 5)
+                             and c["hidden"] <= 3072, True)
     return model
 
 
@@ -263,7 +261,7 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
         if x_ln is None:
             x_ln = ops.layernorm(x, n1.weight, n1.bias, n1.eps)
         src = _key_value_source(attn, x_ln, H, W, extra)
-        return src, ops.linear(src, attn.kv.weight, attn.kv.bias, keep_split=True)             # [B, n, 2C] = [B, n, 2, h, d]
+        return src, ops.linear(src, attn.kv.weight, attn.kv.bias, keep_split=True)   # [B, n, 2C] = [B, n, 2, h, d]
 
     cap = B * N
     placed = {}      # where compress_regions has put every region's rows, for the scatter-back of this block
@@ -450,7 +448,7 @@ class _ChainPlan:
         # the key names the parameters by their ids, which hold as long as all of them live: `whole` ends with the first
         self.whole = whole = [True]
         self.refs = [weakref.ref(t, lambda _: whole.clear()) for t in tensors]
-        self.tables = {}        # (folded, copies wanted) -> (addresses, the derived tensors behind them)
+        self.tables = {}        # (folded, packed copies wanted) -> (addresses, the derived tensors behind them)
         self.layouts = {}       # (B, H, W) -> (vtdge_chain, layout)
 
     def __deepcopy__(self, memo):
@@ -566,33 +564,20 @@ def _chain_layout(plan, B, H, W):
         if len(plan.layouts) >= 64:
             plan.layouts.clear()
         lay = plan.layouts[(B, H, W)] = (desc, list(words)) if rc == 0 else (None, None)
-        if rc == 0:
-            desc.copies = _chain_copies(plan.common, B, H, W)
     return lay if lay[0] is not None else None
 
 
-def _chain_copies(common, B, H, W):
-    """Which of a block's five Linears (q, kv, proj, fc1, fc2) use a packed (bf16) or split (fp32) copy of their weight."""
-    rows, C, hidden, sr = B * (common["extra"] + H * W), common["C"], common["hidden"], common["sr"]
-    if common["dtype"] == _lib.BF16:
-        return (rows >= 2048,) * 5
-    kv_rows = B * (H // sr) * (W // sr) if sr > 1 else rows
-    return tuple(ops.wants_split_weight(*s) for s in ((rows, C, C), (kv_rows, 2 * C, C), (rows, C, C), (rows, hidden, C),
-                                                      (rows, C, hidden)))
-
-
 def _chain_table(plan, blocks, folded, packs):
-    """The address table of the blocks' parameters (vtdge_chain_forward): with the packed or split copies of the weights
-    that `packs` names, and of the folded ones where those are used instead."""
+    """The address table of the blocks' parameters (vtdge_chain_forward): with the packed copies of the weights, and of
+    the folded ones where those are used instead."""
     made = plan.tables.get((folded, packs))
     if made is None:
         table, keep = [], []
         for blk in blocks:
             at, mlp = blk.attn, blk.mlp
             ts = _block_tensors(blk)
-            make = ops.packed_weight if plan.common["dtype"] == _lib.BF16 else ops.split_weight
-            derived = [make(lin.weight) if want and not (folded and lin in (at.q, at.kv, mlp.fc1)) else None
-                       for lin, want in zip((at.q, at.kv, at.proj, mlp.fc1, mlp.fc2), packs)]
+            derived = [ops.packed_weight(lin.weight) if packs and not (folded and lin in (at.q, at.kv, mlp.fc1)) else None
+                       for lin in (at.q, at.kv, at.proj, mlp.fc1, mlp.fc2)]
             for norm, lin in ((blk.norm1, at.q), (blk.norm1, at.kv), (blk.norm2, mlp.fc1)):
                 derived += ops.folded_weight(lin.weight, lin.bias, norm.weight, norm.bias) if folded else (None,) * 3
             tail = ([_khwc_weight(at.sr)] + ts[18:]) if len(ts) > 17 else [None] * 4
@@ -657,7 +642,7 @@ class _ChainBlock(BlockView):
 def _run_chain(blocks, x, H, W, front, plan, lay):
     """`blocks` on x through vtdge_chain_forward."""
     desc, words = lay
-    table = _chain_table(plan, blocks, bool(words[4]), desc.copies)
+    table = _chain_table(plan, blocks, bool(words[4]), x.dtype == torch.bfloat16 and x.shape[0] * x.shape[1] >= 2048)
     for blk in blocks:      # what the last call left is about to be replaced: its buffers can serve this one
         st = blk.dge.states
         if isinstance(dict.get(st, "comp"), _ChainBlock):

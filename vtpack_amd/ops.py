@@ -528,45 +528,45 @@ def invalidate_packed(obj=None):
             t._vtdge_packed = None
         if getattr(t, "_vtdge_folded", None) is not None:
             t._vtdge_folded = None
-        if getattr(t, "_vtdge_split", None) is not None:
-            t._vtdge_split = None
-
-
-def _weight_copy(weight, attr, size_of, fill, *args):
-    """A derived copy of a Linear weight [N, K], made once per weight tensor and version by the library's `fill` and kept
-    on the tensor object under `attr`; None where `size_of` says there is none for this shape."""
-    key = (weight.data_ptr(), weight._version, tuple(weight.shape), weight.dtype, weight.device, _pack_epoch)
-    cached = getattr(weight, attr, None)
-    if cached is not None and cached[0] == key:
-        return cached[1]
-    N, K = weight.shape
-    lib = _lib.load()        # not through call(): these two are no part of a timed step
-    size = ctypes.c_int64(0)
-    if getattr(lib, size_of)(N, K, *args, ctypes.addressof(size)) != 0:
-        raise _lib.VtdgeError(lib.vtdge_last_error().decode("utf-8", "replace"))
-    made = None
-    if size.value:
-        made = torch.empty((size.value,), dtype=torch.uint8, device=weight.device)
-        if getattr(lib, fill)(ptr(weight), N, K, *args, ptr(made), stream_ptr()) != 0:
-            raise _lib.VtdgeError(lib.vtdge_last_error().decode("utf-8", "replace"))
-    try:
-        setattr(weight, attr, (key, made))
-    except AttributeError:      # an object that takes no attributes: made again next time
-        pass
-    return made
 
 
 def packed_weight(weight):
     """The copy of a Linear weight [N, K] in the register order of the weight-stationary kernels, made once per
     weight tensor and version and kept on the tensor object; None when the kernels for this shape take W as it is.
     See `invalidate_packed` for the one kind of edit the key cannot detect."""
-    return _weight_copy(weight, "_vtdge_packed", "vtdge_linear_packed_size", "vtdge_linear_prepack", dtype_code(weight))
+    key = (weight.data_ptr(), weight._version, tuple(weight.shape), weight.dtype, weight.device, _pack_epoch)
+    cached = getattr(weight, "_vtdge_packed", None)
+    if cached is not None and cached[0] == key:
+        return cached[1]
+    N, K = weight.shape
+    lib = _lib.load()        # not through call(): these two are no part of a timed step
+    size = ctypes.c_int64(0)
+    if lib.vtdge_linear_packed_size(N, K, dtype_code(weight), ctypes.addressof(size)) != 0:
+        raise _lib.VtdgeError(lib.vtdge_last_error().decode("utf-8", "replace"))
+    packed = None
+    if size.value:
+        packed = torch.empty((size.value,), dtype=torch.uint8, device=weight.device)
+        if lib.vtdge_linear_prepack(ptr(weight), N, K, dtype_code(weight), ptr(packed), stream_ptr()) != 0:
+            raise _lib.VtdgeError(lib.vtdge_last_error().decode("utf-8", "replace"))
+    try:
+        weight._vtdge_packed = (key, packed)
+    except AttributeError:      # an object that takes no attributes: pack again next time
+        pass
+    return packed
 
 
 def split_weight(weight):
-    """The copy of an fp32 Linear weight [N, K] split into three bf16 parts (6 bytes a value), from which the fp32 Linear
-    runs on the bf16 matrix instructions; kept like `packed_weight`.  None where there is none for the shape."""
-    return _weight_copy(weight, "_vtdge_split", "vtdge_linear_split_size", "vtdge_linear_split")
+    """A copy of a contiguous fp32 Linear weight [N, K] split into three bf16 parts (6 bytes a value), from which the fp32
+    Linear runs on the bf16 matrix instructions; None where there is none for the shape.  Made anew by every call and kept nowhere:
+    whatever happens to the weight, on whichever stream, the next Linear sees it."""
+    N, K = weight.shape
+    size = ctypes.c_int64(0)
+    _lib.load().vtdge_linear_split_size(N, K, ctypes.addressof(size))
+    if not size.value:
+        return None
+    made = torch.empty((size.value,), dtype=torch.uint8, device=weight.device)
+    call("vtdge_linear_split", ptr(weight), N, K, ptr(made), stream_ptr(), tag=("linear_split", N, K))
+    return made
 
 
 def wants_split_weight(rows, N, K):
@@ -581,8 +581,8 @@ def fits_linear_stats(a, weight):
 
 def linear(a, weight, bias=None, residual=None, act="none", rows_dev=None, out=None, stats_eps=None, keep_split=False):
     """out = act(a @ weight.T + bias) + residual; a [..., K] (last dim contiguous), weight [N, K].
-    `keep_split` (fp32; a weight that is used again and again): where it is faster, a split copy of the weight is made on
-    the first call, kept on it and multiplied on the bf16 matrix instructions (`split_weight`; not the same bits).
+    `keep_split` (fp32): where it is faster, the products are made on the bf16 matrix instructions from a split copy of the
+    weight (`split_weight`; as exact, not the same bits).
     With `stats_eps` (a LayerNorm's eps; see `fits_linear_stats`) -> (out, statistics records of the rows of out) for a
     `linear_layernorm` that takes `out` next."""
     _need_gpu(a, weight, bias, residual)
