@@ -1,5 +1,7 @@
 """fp32 attention of many pairs, on the bf16 matrix instructions with operands split in three: at the sizes where its tiling
 turns, against float64, and with what the split does not cover, which the fp32 instructions have to give as before."""
+import math
+
 import pytest
 import torch
 
@@ -98,6 +100,23 @@ def test_what_the_split_does_not_cover(dev, what):
     assert torch.equal(got[rows].isnan(), want.isnan()) and torch.equal(got[rows].isinf(), want.isinf())
     err = (got[rows] - want)[finite].double()
     assert float(err.norm()) <= 1.5e-6 * float(want[finite].double().norm())
+
+
+@pytest.mark.parametrize("below", [90, 104, 112, 118, 124])
+@pytest.mark.parametrize("size", [2.0 ** 30, 2.0 ** 60, 2.0 ** 100])
+def test_large_values_of_improbable_keys(dev, below, size):
+    """Probabilities of 2^-`below` lose parts under the smallest bf16 number, which shows where the keys that matter have no
+    values to add.  The rounding of scores of some 80 in the exponent leaves 4e-6 of each probability, over 129 of them less."""
+    lengths = [113, 70, 200, 64] * 5
+    q, k, v = _inputs(dev, 130, lengths)
+    q.zero_()
+    q[:, ::64] = 1.0
+    k[:, :, ::64] = -8 * math.log(2) * (below + torch.rand(20, 130, HEADS, generator=torch.Generator().manual_seed(below))).to(dev)
+    k[:, 0, ::64] = 0.0
+    v *= size
+    v[:, 0] = 0.0
+    got, want = _run(q, k, v, lengths).cpu().double(), _float64(q, k, v, lengths)
+    assert float((got - want).norm() / want.norm()) <= 4e-6
 
 
 def test_keys_far_apart_and_in_reverse(dev):

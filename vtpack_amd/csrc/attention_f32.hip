@@ -270,11 +270,14 @@ __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
 //     lane has: P never moves between lanes.
 //   * A workgroup of one or two tiles takes the fp32 instructions, whose waves share a tile (20 queries of 128 samples: 17.4
 //     against 20.9 us), and so does one with anything the split is not exact for: sums that are not finite, tiny or huge
-//     ones, queries far from one.
+//     ones, queries far from one, large values.
 constexpr int AS_KEYS = 32;                          // keys per stage
 constexpr int AS_PLANE = AS_KEYS * 128;              // bytes of a plane: 32 rows of 64 bf16 values
 constexpr int AS_BUF = 6 * AS_PLANE;                 // one stage: three planes of K, then three of V
 constexpr float AS_TINY = 0x1p-80f, AS_FAR = 0x1p60f;
+// A probability below 2^-108 loses parts under the smallest bf16 number, up to 2^-134: over values below 2^20 that is less than
+// 2^-34 a key of a sum that is not tiny.
+constexpr float AS_LARGE = 0x1p20f;
 
 // x[0..7] into three bf16 parts each: x = p[0] + p[1] + p[2] to 2^-26 of it (nearest parts, signed remainders)
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[3])
@@ -322,6 +325,7 @@ __device__ __forceinline__ bool attention_f32_split_rows(
     const float *kp = k + (int64_t)b * kv_bs + (int64_t)head * kv_hs + 8 * schunk;
     const float *vp = v + (int64_t)b * kv_bs + (int64_t)head * kv_hs + 8 * schunk;
     float rk[8], rv[8];
+    bool large = false;                                      // a value of this wave's that is
     auto load_stage = [&](int st) {                          // rows past the last key repeat it
         const int64_t off = (int64_t)min(st * AS_KEYS + srow, n - 1) * kv_ts;
 #pragma unroll
@@ -349,6 +353,10 @@ __device__ __forceinline__ bool attention_f32_split_rows(
         split8(rk, p);
 #pragma unroll
         for (int i = 0; i < 3; i++) *reinterpret_cast<u32x4 *>(smem + kdst + i * AS_PLANE) = p[i];
+        float most = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) most = __builtin_amdgcn_fmed3f(fabsf(rv[e]), most, INFINITY);            // the maximum
+        large = large || __builtin_amdgcn_ballot_w64(!(most < AS_LARGE)) != 0;
         split8(rv, p);
 #pragma unroll
         for (int i = 0; i < 3; i++) *reinterpret_cast<u32x4 *>(smem + vdst + i * AS_PLANE) = p[i];
@@ -469,6 +477,7 @@ __device__ __forceinline__ bool attention_f32_split_rows(
     }
     l_run += __shfl_xor(l_run, 16, WAVE);
     l_run += __shfl_xor(l_run, 32, WAVE);
+    odd = odd || large;
     if (row_live) {
         odd = odd || !(l_run < INFINITY);
 #pragma unroll
