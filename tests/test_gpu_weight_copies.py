@@ -5,7 +5,8 @@ import torch
 
 from vtpack_amd import _lib, engine
 from vtpack_amd.models.dge.deit_dge import VisionTransformer
-from vtpack_amd.synthetic import set_synthetic_router
+from vtpack_amd.models.dge.pvt_dge import PyramidVisionTransformer
+from vtpack_amd.synthetic import set_synthetic_router, synthetic_images
 
 pytestmark = pytest.mark.gpu
 BATCH, GRID = 32, 16
@@ -125,3 +126,51 @@ def test_f32_parameters_made_in_inference_mode(dev):
         engine.prepare(m)
         got = _run(list(m.blocks), x)
     assert torch.equal(got, want)
+
+
+def _model(kind, dtype, dev):
+    torch.manual_seed(2)
+    if kind == "pvt":
+        m = PyramidVisionTransformer(img_size=128, patch_size=4, embed_dims=[64, 128, 320, 512], num_heads=[1, 2, 5, 8],
+                                     mlp_ratios=[2, 2, 2, 2], qkv_bias=True, depths=[2, 1, 2, 1], sr_ratios=[8, 4, 2, 1],
+                                     split_sizes=[[4, 2, 1]] * 4, num_classes=30)
+    else:
+        m = VisionTransformer(img_size=128, patch_size=16, embed_dim=384, depth=2, num_heads=6, num_classes=30, qkv_bias=True,
+                              split_sizes=[4, 2, 1])
+    return set_synthetic_router(m, 3).eval().to(dev).to(dtype)
+
+
+@pytest.mark.parametrize("kind,dtype", [("deit", torch.bfloat16), ("pvt", torch.bfloat16), ("pvt", torch.float32)])
+def test_copies_that_are_kept(dev, kind, dtype, native):
+    """Packed, folded and reordered weights and the class-token rows, which stay between calls: first used on two streams at
+    once, and in a capture that no call came before."""
+    images = synthetic_images(48, 128, seed=6, dtype=dtype, device=dev)
+
+    def forward(m):
+        with torch.no_grad():
+            return m(images)
+
+    def fresh():
+        m = _model(kind, dtype, dev)
+        torch.cuda.synchronize()
+        return m
+
+    want = forward(fresh()).clone()
+    m = fresh()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        torch.cuda._sleep(100_000_000)
+        one = forward(m)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        two = forward(m)
+    torch.cuda.synchronize()
+    assert torch.equal(one, want) and torch.equal(two, want)
+
+    m = fresh()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = forward(m)
+    assert torch.equal(forward(m), want)            # before the first replay
+    for _ in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(forward(m), want)

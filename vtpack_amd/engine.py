@@ -164,7 +164,9 @@ def _khwc_weight(conv):
     cached = getattr(conv, "_vtdge_khwc", None)
     if cached is None or cached[0] != key:
         flat = w.detach().permute(0, 2, 3, 1).reshape(w.shape[0], -1).contiguous()
-        conv._vtdge_khwc = cached = (key, flat)
+        cached = (key, flat)
+        if w.is_cuda and ops.done_before_shared():
+            conv._vtdge_khwc = cached
     return cached[1]
 
 
@@ -583,8 +585,10 @@ def _chain_table(plan, blocks, folded, packs):
             tail = ([_khwc_weight(at.sr)] + ts[18:]) if len(ts) > 17 else [None] * 4
             keep += derived + tail[:1]
             table += [0 if t is None else t.data_ptr() for t in ts[:17] + derived + tail]
-        made = plan.tables[(folded, packs)] = (array.array("Q", table), keep)
-    return made[0]
+        made = (array.array("Q", table), keep)
+        if not torch.cuda.is_current_stream_capturing():      # the copies made in a capture belong to its graph
+            plan.tables[(folded, packs)] = made
+    return made
 
 
 class _ChainBlock(BlockView):
@@ -642,7 +646,7 @@ class _ChainBlock(BlockView):
 def _run_chain(blocks, x, H, W, front, plan, lay):
     """`blocks` on x through vtdge_chain_forward."""
     desc, words = lay
-    table = _chain_table(plan, blocks, bool(words[4]), x.dtype == torch.bfloat16 and x.shape[0] * x.shape[1] >= 2048)
+    table, _keep = _chain_table(plan, blocks, bool(words[4]), x.dtype == torch.bfloat16 and x.shape[0] * x.shape[1] >= 2048)
     for blk in blocks:      # what the last call left is about to be replaced: its buffers can serve this one
         st = blk.dge.states
         if isinstance(dict.get(st, "comp"), _ChainBlock):
@@ -700,7 +704,8 @@ def _front_rows(model, front):
         with torch.no_grad():
             rows = (torch.cat([t.detach() for t in front], dim=1) + model.pos_embed.detach()[:, :len(front), :])[0]
         cached = (key, rows.contiguous())
-        object.__setattr__(model, "_vtdge_front", cached)
+        if rows.is_cuda and ops.done_before_shared():
+            object.__setattr__(model, "_vtdge_front", cached)
     return cached[1]
 
 

@@ -516,7 +516,9 @@ def invalidate_packed(obj=None):
     `load_state_dict`, `.to()` / `.bfloat16()`, optimiser steps and every in-place torch op on the parameter.  It does
     NOT see writes that bypass the version counter: `w.data.copy_(...)`, `w.data.mul_(...)`, a raw kernel writing
     into the storage.  After such a write call this function (or `engine.prepare(model)`) before the next forward;
-    otherwise the weight-stationary kernels keep multiplying by the old weights."""
+    otherwise the weight-stationary kernels keep multiplying by the old weights.  Copies made inside a graph
+    capture are made again by every replay and kept nowhere else; a graph that was captured when they were there names them,
+    and is captured again after a change of the weights."""
     global _pack_epoch, _plan_epoch
     _plan_epoch += 1
     if obj is None:
@@ -528,6 +530,15 @@ def invalidate_packed(obj=None):
             t._vtdge_packed = None
         if getattr(t, "_vtdge_folded", None) is not None:
             t._vtdge_folded = None
+
+
+def done_before_shared():
+    """Waits until the current stream is done with what it has been given, so that a derived copy just made on it can be kept
+    for calls on any stream.  False in a capture, where nothing has run yet and what is made belongs to the graph."""
+    if torch.cuda.is_current_stream_capturing():
+        return False
+    torch.cuda.current_stream().synchronize()
+    return True
 
 
 def packed_weight(weight):
@@ -548,6 +559,8 @@ def packed_weight(weight):
         packed = torch.empty((size.value,), dtype=torch.uint8, device=weight.device)
         if lib.vtdge_linear_prepack(ptr(weight), N, K, dtype_code(weight), ptr(packed), stream_ptr()) != 0:
             raise _lib.VtdgeError(lib.vtdge_last_error().decode("utf-8", "replace"))
+    if packed is not None and not done_before_shared():
+        return packed
     try:
         weight._vtdge_packed = (key, packed)
     except AttributeError:      # an object that takes no attributes: pack again next time
@@ -683,6 +696,8 @@ def folded_weight(weight, bias, ln_weight, ln_bias):
                                 dtype_code(weight), ptr(wf), ptr(rec), stream_ptr()) != 0:
         raise _lib.VtdgeError(lib.vtdge_last_error().decode("utf-8", "replace"))
     value = (wf, rec, packed_weight(wf) if PACK_WEIGHTS else None)
+    if not done_before_shared():
+        return value
     try:
         weight._vtdge_folded = (key, value)
     except AttributeError:
