@@ -49,6 +49,8 @@ const char *vtdge_last_error(void);
 /* The demangled name of the kernel that the calling thread's latest launch was (the last one, for an entry point
  * that launches several), as a profiler lists it; "" before the first launch.  For measurement tools. */
 const char *vtdge_last_kernel(void);
+/* The same of the launch `back` (0 .. 7) before the latest one; "" where the thread has made fewer. */
+const char *vtdge_recent_kernel(int back);
 
 /* Router: region mean of the spatial tokens, Linear(C -> S), argmax.
  * Replaces DynamicRouter.forward + argmax (vtpack/layers/dge.py:145-150, :75).

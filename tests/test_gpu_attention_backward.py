@@ -285,4 +285,12 @@ def test_from_a_workspace_of_two_floats_a_row(dev, dtype):
 @pytest.mark.parametrize("n", [32, 63, 95, 96, 97, 128, 160, 161, 256, 288, 289, 320])
 def test_scores_kept_between_the_walks(dev, n):
     """fp32: whole and partial last stages at the edges of three, five and nine kept ones, and one beyond."""
-    test_against_float64(dev, torch.float32, n, [64, 0, 65, 33, 5, 130], 0.125, False)
+    from vtpack_amd import _lib, ops
+    lengths = [64, 0, 65, 33, 5, 130]
+    test_against_float64(dev, torch.float32, n, lengths, 0.125, False)
+    q, g = (torch.ones(3, sum(lengths), 64, device=dev) for _ in range(2))
+    k, v = (torch.ones(3, len(lengths), n, 64, device=dev) for _ in range(2))
+    offsets, _ = ops.lengths_to_offsets(torch.tensor(lengths), dev)
+    ops.sparse_attention_backward(q, k, v, None, g, offsets, 0.125, max(lengths))
+    held = next((stages for stages in (3, 5, 9) if n <= 32 * stages), 0)
+    assert f"attention_dq_kernel<float, {held}>" in _lib.last_kernel(1)

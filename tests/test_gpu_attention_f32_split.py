@@ -18,17 +18,19 @@ def _inputs(dev, n, lengths, h=HEADS):
     return [torch.from_numpy(randn(950 + i, *shape)).to(dev) for i, shape in enumerate([(L, h * 64), (B, n, h * 64), (B, n, h * 64)])]
 
 
-def _run(q, k, v, lengths, h=HEADS, scale=0.125):
-    from vtpack_amd import ops
+def _run(q, k, v, lengths, h=HEADS, scale=0.125, split=True):
+    from vtpack_amd import _lib, ops
     offsets, _ = ops.lengths_to_offsets(torch.tensor(lengths), q.device)
-    return ops.sparse_attention(q, k, v, offsets, scale, h, max(lengths))
+    out = ops.sparse_attention(q, k, v, offsets, scale, h, max(lengths))
+    assert ("attention_f32_split_kernel<" if split else "attention_f32_kernel<64") in _lib.last_kernel()
+    return out
 
 
 def _alone(q, k, v, lengths, sample, h=HEADS):
     """One sample by itself: few pairs, so the fp32 instructions."""
     at = sum(lengths[:sample])
     return _run(q[at:at + lengths[sample]].contiguous(), k[sample:sample + 1].contiguous(), v[sample:sample + 1].contiguous(),
-                lengths[sample:sample + 1], h)
+                lengths[sample:sample + 1], h, split=False)
 
 
 def _float64(q, k, v, lengths, h=HEADS, scale=0.125):
@@ -122,16 +124,18 @@ def test_large_values_of_improbable_keys(dev, below, size):
 def test_keys_far_apart_and_in_reverse(dev):
     """Token strides of 2^23 values and negative ones, for both kinds of workgroups: the same bytes as from dense operands."""
     from vtpack_amd import _lib, ops
-    n, lengths, h = 40, [113, 20, 64] * 6, HEADS
+    n, lengths, h = 70, [113, 20, 64] * 6, HEADS
     q, k, v = _inputs(dev, n, lengths)
     v[0, 30, 2] = float("inf")                          # and for a workgroup that starts again
     want = _run(q, k, v, lengths)
     far = [torch.empty_strided(t.shape, (h * 64, 1 << 23, 1), device=dev).copy_(t) for t in (k, v)]
     got = _run(q, *far, lengths)
+    assert "attention_f32_split_kernel<true>" in _lib.last_kernel()
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
     offsets, _ = ops.lengths_to_offsets(torch.tensor(lengths), dev)
     back = [t.flip(1).contiguous() for t in (k, v)]
     _lib.call("vtdge_sparse_attention", q.data_ptr(), h * 64, 64, *(t[0, n - 1].data_ptr() for t in back), n * h * 64, -h * 64, 64,
               offsets.data_ptr(), got.data_ptr(), h * 64, 64, len(lengths), h, 64, n, max(lengths), 0.125, _lib.F32,
               _lib.stream_ptr())
+    assert "attention_f32_split_kernel<true>" in _lib.last_kernel()
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())

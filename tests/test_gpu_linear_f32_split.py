@@ -52,6 +52,18 @@ def test_magnitudes(dev, scale_a, scale_w):
     assert float((got.double() - want).norm() / want.norm()) <= 1e-6
 
 
+@pytest.mark.parametrize("K", [192, 768])
+def test_partial_products_left_out_add_up(dev, K):
+    """All operands just below 1 + 2^-8, where the second and third part are largest and of opposite signs: the three partial
+    products that are left out are 2^-24 of every product, all on one side.  Beside them one rounding of the sum for each of
+    the 6 K / 16 instructions that make it."""
+    x = 1.0038986
+    a, w = torch.full((16500, K), x, device=dev), torch.full((192, K), x, device=dev)
+    got = _run(a, w, None, None, "none", 16500, True, dev)
+    want = K * float(a[0, 0].double()) ** 2
+    assert float((got.double() - want).abs().max()) <= (1 + 6 * K / 16) * 2.0 ** -24 * want
+
+
 def test_values_outside_the_split(dev):
     """Infinities, NaN and numbers that round to infinity in bf16: the same results as on the fp32 instructions, in the
     rows and columns that hold them and beside them."""

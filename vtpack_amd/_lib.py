@@ -93,7 +93,7 @@ class Chain(ctypes.Structure):
                [(n, ctypes.c_float) for n in ("eps1", "eps2", "sr_eps", "scale")]
 
 
-EXPORTS = ["vtdge_version", "vtdge_last_error", "vtdge_last_kernel"] + list(SIGNATURES)
+EXPORTS = ["vtdge_version", "vtdge_last_error", "vtdge_last_kernel", "vtdge_recent_kernel"] + list(SIGNATURES)
 
 _lib = None
 
@@ -129,6 +129,8 @@ def load():
     lib.vtdge_last_error.argtypes = []
     lib.vtdge_last_kernel.restype = ctypes.c_char_p
     lib.vtdge_last_kernel.argtypes = []
+    lib.vtdge_recent_kernel.restype = ctypes.c_char_p
+    lib.vtdge_recent_kernel.argtypes = [_i]
     lib.vtdge_decompress_router_compress_workspace.restype = _l
     lib.vtdge_decompress_router_compress_workspace.argtypes = [_i, _i, _i, _i]
     lib.vtdge_region_step_workspace.restype = _l
@@ -157,10 +159,10 @@ def call(name, *args, tag=None):
         raise VtdgeError(f"{name} failed ({rc}): {msg}")
 
 
-def last_kernel():
-    """Name of the kernel the latest libvtdge launch of this thread was, as rocprofv3 lists it (without the
-    namespace and the argument list)."""
-    name = load().vtdge_last_kernel().decode("utf-8", "replace")
+def last_kernel(back=0):
+    """Name of the kernel the latest libvtdge launch of this thread was, or the launch `back` before it, as rocprofv3 lists
+    it (without the namespace and the argument list)."""
+    name = load().vtdge_recent_kernel(back).decode("utf-8", "replace")
     if name.startswith("void "):
         name = name[5:]
     depth, cut = 0, len(name)

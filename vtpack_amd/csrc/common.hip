@@ -15,19 +15,22 @@ void set_error(const char *fmt, ...)
     va_end(ap);
 }
 
-// The kernel of the latest launch made from this thread, for tools that want to tell a caller's entry points from
-// the kernels a profiler lists (vtdge_last_kernel).  Only the pointer is kept at launch time; the name is looked up
+// The kernels of the latest launches made from this thread, for tools that want to tell a caller's entry points from
+// the kernels a profiler lists (vtdge_last_kernel).  Only the pointers are kept at launch time; a name is looked up
 // and demangled when somebody asks.
-static thread_local const void *last_kernel_fn = nullptr;
+constexpr unsigned NOTED = 8;
+static thread_local const void *noted[NOTED];
+static thread_local unsigned notes = 0;
 static thread_local char last_kernel_name[512];
 
-void note_kernel(const void *host_function) { last_kernel_fn = host_function; }
+void note_kernel(const void *host_function) { noted[notes++ % NOTED] = host_function; }
 
-extern "C" const char *vtdge_last_kernel(void)
+extern "C" const char *vtdge_recent_kernel(int back)
 {
     last_kernel_name[0] = 0;
-    if (last_kernel_fn == nullptr) return last_kernel_name;
-    const char *mangled = hipKernelNameRefByPtr(last_kernel_fn, nullptr);
+    const void *fn = back >= 0 && back < (int)NOTED ? noted[(notes - 1 - back) % NOTED] : nullptr;
+    if (fn == nullptr) return last_kernel_name;
+    const char *mangled = hipKernelNameRefByPtr(fn, nullptr);
     if (mangled == nullptr) return last_kernel_name;
     int status = 1;
     char *plain = abi::__cxa_demangle(mangled, nullptr, nullptr, &status);
@@ -35,6 +38,8 @@ extern "C" const char *vtdge_last_kernel(void)
     free(plain);
     return last_kernel_name;
 }
+
+extern "C" const char *vtdge_last_kernel(void) { return vtdge_recent_kernel(0); }
 
 int check_launch(const char *what)
 {
