@@ -332,8 +332,9 @@ int vtdge_linear_prepacked(const void *A, int64_t lda, const void *W, const void
                            int64_t rows, int N, int K, int act, int dtype, void *stream);
 
 /* fp32 Linears on the bf16 matrix instructions: for VTDGE_F32, `packed` of vtdge_linear_prepacked is a copy of W split into
- * three bf16 parts (6 bytes a value).  The sums of all partial products of weight 2^-18 and above, in fp32, are as exact as
- * those of the fp32 instructions (not the same bits) and 1.2 to 1.5 times as fast.
+ * three bf16 parts (6 bytes a value).  The sums of the partial products of weight 2^-17 and above, in fp32, are as exact as
+ * those of the fp32 instructions (not the same bits; up to 2^-24 of a product is left out) and 1.2 to 1.5 times as fast, the
+ * split (3 to 16 us for the weights of a block) aside.
  *   vtdge_linear_split_size    *bytes = size of the split copy of W [N, K], or 0 when there is none (N no multiple of 64, K
  *                              none of 32)
  *   vtdge_linear_split         fills `split` (16-byte aligned, *bytes long) from W; VTDGE_ERR_UNSUPPORTED where the size is 0
@@ -518,8 +519,8 @@ int vtdge_block_tail(const void *o, const void *comp, const void *proj_weight, c
                      int hidden, int dtype, void *stream);
 
 /* A chain of DGE transformer blocks on one token grid (vtpack/models/dge/deit_dge.py:101-131 or pvt_dge.py:111-140,
- * `depth` of them in a row), issued by one host call: the launches are those of the entry points above, in the order a
- * caller that composes a block from them would issue them, with nothing of the host between them.
+ * `depth` of them in a row), issued by one host call: the launches are those of the entry points above
+ * (vtdge_region_step and vtdge_linear_split_set among them), with nothing of the host between them.
  *   chain        what the blocks have in common.  H, W multiples of 4 and split sizes that divide 4 (`splits_124`: all
  *                of them out of {1, 2, 4}); head dim 32 or 64; sr > 1 only without extra tokens
  *   params_host  HOST table of device pointers, VTDGE_CHAIN_PARAMS per block, in this order (NULL where absent):

@@ -256,10 +256,10 @@ __global__ __launch_bounds__(64 * AF_TILES, 4) void attention_f32_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// head_dim 64 on the bf16 matrix instructions, as exact: queries, keys, probabilities and values are each the sum of three
-// bf16 values (to 2^-26 of them), six of the nine partial products of two such sums are multiplied and added in fp32
-// (linear_dma_split.hip says why that is enough).  Per 32 keys and 16 queries that is 768 clocks of matrix instructions
-// against 2048; against float64 the output is off by 3.7e-7 against 4.1e-7 (2-norm; 257 keys, unit normals).
+// head_dim 64 on the bf16 matrix instructions, as exact: queries, keys, probabilities and values are each the sum of three bf16
+// values (exactly, where the third is no smaller than bf16 goes), six of the nine partial products of two such sums are multiplied
+// and added in fp32 (linear_dma_split.hip says what the other three are).  Per 32 keys and 16 queries that is 768 clocks of matrix
+// instructions against 2048; against float64 the output is off by 3.7e-7 against 4.1e-7 (2-norm; 257 keys, unit normals).
 // What bounds it are the vector instructions: splitting a stage of K and V (88 a wave) and the probabilities (44), the
 // exponentials and 36 reads of LDS, some 300 a wave and stage beside 48 matrix instructions.
 //   * 64 query rows a workgroup, 16 a wave; a stage of 32 keys goes through registers, is split and written to LDS as planes of
@@ -279,7 +279,7 @@ constexpr float AS_TINY = 0x1p-80f, AS_FAR = 0x1p60f;
 // 2^-34 a key of a sum that is not tiny.
 constexpr float AS_LARGE = 0x1p20f;
 
-// x[0..7] into three bf16 parts each: x = p[0] + p[1] + p[2] to 2^-26 of it (nearest parts, signed remainders)
+// x[0..7] into three bf16 parts each: x = p[0] + p[1] + p[2] (nearest parts, signed remainders)
 __device__ __forceinline__ void split8(const float (&x)[8], u32x4 (&p)[3])
 {
     float r[8];

@@ -99,9 +99,12 @@ FUSE_TAIL = True
 NATIVE_CHAIN = True
 # Values of a natively issued chain (tokens times channels) from which the routing half of a block goes to a second
 # stream, where the block has no folded kernels.  Below, the fork and the join cost more than the overlap gives: one
-# stream against two, GPU time of a forward: 1001 against 1098 us (one 256 px picture, 384 channels), 1497 against 1515
-# (five, 768 channels); above: 4293 against 4174 (128, 192 channels fp32), 4654 against 4561 (99, 768 channels), 6847
-# against 6572 (256, PVT-Small).
+# stream against two, GPU time of a forward, us: 1030 against 1088 (five 256 px pictures, 768 channels), 1505 against 1561
+# (12, 384 channels fp32).  Far above it gives more: 4531 against 4509 (99, 768 channels), 3203 against 3134 (128,
+# PVT-Small), 5176 against 5003 (256).  From the line to some 16 M values it depends on the model: 1698 against 1667 (12 of
+# 384 px, PVT-Tiny fp32), 2600 against 2545 (24), but 1737 against 1787 (32, PVT-Small) and, where few regions route the
+# next block in their scatter-back (`vtdge_region_step`) so that only the first block forks, 1462 against 1515 (12, 768
+# channels) and 2907 against 2926 (128, 192 channels fp32).
 OVERLAP_FROM = 2 << 20
 _SWITCHES = ("OVERLAP", "FUSE_NEXT_NORM", "FUSE_ROUTER_NORM", "FUSE_NEXT_ROUTER", "FOLD_NORMS", "FUSE_PATCH_EMBED",
              "ROUTING_ON_SIDE", "Q_AFTER_JOIN", "REGION_COMPRESS", "SERIAL_BESIDE_WEIGHT_STATIONARY", "ROUTING_FIRST",
