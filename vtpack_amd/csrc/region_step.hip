@@ -45,8 +45,8 @@ template <typename T> struct RegionStep {
 
 // layernorm_kernel's arithmetic for one row held by a wave, a vector or several a lane
 template <typename T, int NV>
-__device__ __forceinline__ void norm_row(const u32x4 (&row)[NV], const bool (&act)[NV], const float (&w)[NV][Elem<T>::VEC],
-                                         const float (&bb)[NV][Elem<T>::VEC], float eps, int C, T *dst)
+__device__ __forceinline__ void norm_row(const u32x4 (&row)[NV], const bool (&act)[NV], const u32x4 (&w)[NV],
+                                         const u32x4 (&bb)[NV], float eps, int C, T *dst)
 {
     constexpr int VEC = Elem<T>::VEC;
     float vals[NV][VEC];
@@ -72,11 +72,74 @@ __device__ __forceinline__ void norm_row(const u32x4 (&row)[NV], const bool (&ac
 #pragma unroll
     for (int it = 0; it < NV; it++)
         if (act[it]) {
-            float y[VEC];
+            float y[VEC], wf[VEC], bf[VEC];
+            Elem<T>::unpack(w[it], wf);
+            Elem<T>::unpack(bb[it], bf);
 #pragma unroll
-            for (int c = 0; c < VEC; c++) y[c] = (vals[it][c] - mean) * rstd * w[it][c] + bb[it][c];
+            for (int c = 0; c < VEC; c++) y[c] = (vals[it][c] - mean) * rstd * wf[c] + bf[c];
             *reinterpret_cast<u32x4 *>(dst + it * WAVE * VEC) = Elem<T>::pack(y);
         }
+}
+
+// The same for the four rows of a wave, one step of all of them after the other: their sums are four independent chains, and
+// their quotients and roots are taken once, in four lanes side by side (the same operations on the same values).  With that,
+// the LayerNorm of a region that stays 16 queries taken over from its tokens, and registers for four waves a SIMD, a launch at
+// 2048 regions of 192 fp32 channels went from 39.9 to 36.3 us (119 MB), at 80 regions of 768 bf16 channels from 15.5 to 13.9.
+template <typename T, int NV>
+__device__ __forceinline__ void norm_rows4(const u32x4 (&row)[4][NV], const bool (&act)[NV], const u32x4 (&w)[NV],
+                                           const u32x4 (&bb)[NV], float eps, int C, T *dst, u32x4 (&y4)[4][NV])
+{
+    constexpr int VEC = Elem<T>::VEC;
+    const int lane = threadIdx.x & 63;
+    // (the values come by value: behind a reference the selection turns into a load through a computed address)
+    auto per_row = [&](float v0, float v1, float v2, float v3, auto f, float (&out)[4]) {
+        const float r = f(lane & 2 ? (lane & 1 ? v3 : v2) : (lane & 1 ? v1 : v0));
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            out[t] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r), t));
+    };
+    float vals[4][NV][VEC], s[4], q[4], mean[4], rstd[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        s[t] = 0.f;
+#pragma unroll
+        for (int it = 0; it < NV; it++)
+            if (act[it]) {
+                Elem<T>::unpack(row[t][it], vals[t][it]);
+#pragma unroll
+                for (int c = 0; c < VEC; c++) s[t] += vals[t][it][c];
+            }
+    }
+    wave_sum_n<4>(s);
+    per_row(s[0], s[1], s[2], s[3], [&](float v) { return v / (float)C; }, mean);
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        q[t] = 0.f;
+#pragma unroll
+        for (int it = 0; it < NV; it++)
+            if (act[it]) {
+#pragma unroll
+                for (int c = 0; c < VEC; c++) {
+                    const float dlt = vals[t][it][c] - mean[t];
+                    q[t] += dlt * dlt;
+                }
+            }
+    }
+    wave_sum_n<4>(q);
+    per_row(q[0], q[1], q[2], q[3], [&](float v) { return 1.0f / sqrtf(v / (float)C + eps); }, rstd);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int it = 0; it < NV; it++)
+            if (act[it]) {
+                float y[VEC], wf[VEC], bf[VEC];
+                Elem<T>::unpack(w[it], wf);
+                Elem<T>::unpack(bb[it], bf);
+#pragma unroll
+                for (int c = 0; c < VEC; c++) y[c] = (vals[t][it][c] - mean[t]) * rstd[t] * wf[c] + bf[c];
+                y4[t][it] = Elem<T>::pack(y);
+                *reinterpret_cast<u32x4 *>(dst + (int64_t)t * C + it * WAVE * VEC) = y4[t][it];
+            }
 }
 
 // the record of one row, from wave-wide sums
@@ -95,7 +158,7 @@ __device__ __forceinline__ void record_row(const u32x4 &row, bool act, float eps
 }  // namespace
 
 template <typename T, int NV, bool REC>
-__global__ __launch_bounds__(256) void region_step_kernel(const RegionStep<T> a)
+__global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_step_kernel(const RegionStep<T> a)
 {
     static_assert(!REC || (NV == 1 && sizeof(T) == 2), "records: bf16 rows of one vector a lane");
     constexpr int VEC = Elem<T>::VEC;
@@ -133,14 +196,14 @@ __global__ __launch_bounds__(256) void region_step_kernel(const RegionStep<T> a)
             rsplit = (int)a.next_splits[lane];
         }
     }
-    float lw[NV][VEC], lb[NV][VEC];
+    u32x4 lw[NV], lb[NV];
     const bool normed = !REC && a.out_ln != nullptr;
     if (normed) {
 #pragma unroll
         for (int it = 0; it < NV; it++)
             if (act[it]) {
-                Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(a.ln_w + (it * WAVE + lane) * VEC), lw[it]);
-                Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(a.ln_b + (it * WAVE + lane) * VEC), lb[it]);
+                lw[it] = *reinterpret_cast<const u32x4 *>(a.ln_w + (it * WAVE + lane) * VEC);
+                lb[it] = *reinterpret_cast<const u32x4 *>(a.ln_b + (it * WAVE + lane) * VEC);
             }
     }
 
@@ -268,11 +331,14 @@ __global__ __launch_bounds__(256) void region_step_kernel(const RegionStep<T> a)
             for (int c = 0; c < VEC; c++) acc[c] = 0.f;
             pooled[it] = z;
             if (act[it]) {
-                u32x4 t16[16];
 #pragma unroll
-                for (int t = 0; t < 16; t++) t16[t] = held[t * nvec + it * WAVE + lane];
+                for (int h = 0; h < 16; h += 8) {
+                    u32x4 t8[8];
 #pragma unroll
-                for (int t = 0; t < 16; t++) add_vector<T>(acc, t16[t]);
+                    for (int t = 0; t < 8; t++) t8[t] = held[(h + t) * nvec + it * WAVE + lane];
+#pragma unroll
+                    for (int t = 0; t < 8; t++) add_vector<T>(acc, t8[t]);
+                }
 #pragma unroll
                 for (int c = 0; c < VEC; c++) acc[c] = Elem<T>::round(acc[c] / 16.f);
                 pooled[it] = Elem<T>::pack(acc);
@@ -312,6 +378,7 @@ __global__ __launch_bounds__(256) void region_step_kernel(const RegionStep<T> a)
     }
 
     // ---- what LayerNorm wants of this wave's tokens
+    u32x4 y4[4][NV];                                               // their LayerNorm, which rows of one token take over
     const int64_t row0 = (int64_t)b * N + extra + (int64_t)(ry * 4 + wv) * a.W + rx * 4;
     if constexpr (REC) {
         float pivot[4], st[8];
@@ -319,8 +386,7 @@ __global__ __launch_bounds__(256) void region_step_kernel(const RegionStep<T> a)
         for (int t = 0; t < 4; t++) lane_sums<T>(tok[t][0], act[0], pivot[t], st[2 * t], st[2 * t + 1]);
         write_records4(st, pivot[0], pivot[1], pivot[2], pivot[3], C, a.eps, a.records + row0 * 2);
     } else if (normed) {
-#pragma unroll
-        for (int t = 0; t < 4; t++) norm_row<T, NV>(tok[t], act, lw, lb, a.eps, C, a.out_ln + (row0 + t) * C + lane * VEC);
+        norm_rows4<T, NV>(tok, act, lw, lb, a.eps, C, a.out_ln + row0 * C + lane * VEC, y4);
     }
 
     // ---- the region's place among the next block's queries
@@ -351,10 +417,13 @@ __global__ __launch_bounds__(256) void region_step_kernel(const RegionStep<T> a)
     if (n0 + nq > a.capacity) return;                              // never outside the buffers
 
     // ---- the queries themselves: 16, four a wave; 4, one a wave; or the mean that the router has taken
-    auto put = [&](const u32x4 (&row)[NV], int64_t r) {
+    auto store = [&](T *to, const u32x4 (&row)[NV], int64_t r) {
 #pragma unroll
         for (int it = 0; it < NV; it++)
-            if (act[it]) *reinterpret_cast<u32x4 *>(a.comp + r * C + (it * WAVE + lane) * VEC) = row[it];
+            if (act[it]) *reinterpret_cast<u32x4 *>(to + r * C + (it * WAVE + lane) * VEC) = row[it];
+    };
+    auto put = [&](const u32x4 (&row)[NV], int64_t r) {
+        store(a.comp, row, r);
         if (normed) norm_row<T, NV>(row, act, lw, lb, a.eps, C, a.comp_ln + r * C + lane * VEC);
     };
     if (ps_n == 4) {
@@ -369,7 +438,8 @@ __global__ __launch_bounds__(256) void region_step_kernel(const RegionStep<T> a)
                 add_vector<T>(acc, tok[t][it]);                    // 0 + x: the mean of a window of one
                 tok[t][it] = Elem<T>::pack(acc);
             }
-            put(tok[t], n0 + 4 * wv + t);
+            store(a.comp, tok[t], n0 + 4 * wv + t);
+            if (normed) store(a.comp_ln, y4[t], n0 + 4 * wv + t);
             if constexpr (REC) lane_sums<T>(tok[t][0], act[0], pivot[t], st[2 * t], st[2 * t + 1]);
         }
         if constexpr (REC)
