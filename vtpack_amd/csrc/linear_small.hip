@@ -440,6 +440,27 @@ static int launch_layernorm_linear(const void *A0, int64_t lda0, const void *W0,
 #undef VT_SMALL
 }
 
+// A0 W0^T + bias0 and A1 W1^T + bias1 over the same K in one launch: the key/value and the query projection of few rows whose
+// LayerNorm the kernel that produced them has written.  For sizes that layernorm_linear_fits takes.
+template <typename T>
+static int launch_pair(const void *A0, const void *W0, const void *bias0, void *out0, int64_t rows0, int N0, const void *A1,
+                       const void *W1, const void *bias1, void *out1, const int64_t *rows_dev1, int64_t rows1, int N1, int K,
+                       hipStream_t st)
+{
+    const PatchGeom none{0, 0, 0, 0, 0, 0, 0, 0};
+    const SmallProblem p0 = small_problem(A0, K, W0, bias0, nullptr, 0, out0, N0, nullptr, rows0, N0);
+    const SmallProblem p1 = small_problem(A1, K, W1, bias1, nullptr, 0, out1, N1, rows_dev1, rows1, N1);
+    return go_small<T, 4, VTDGE_ACT_NONE, 0, false>(p0, p1, K, nullptr, nullptr, 0.f, none, st);
+}
+int launch_linear_pair(const void *A0, const void *W0, const void *bias0, void *out0, int64_t rows0, int N0, const void *A1,
+                       const void *W1, const void *bias1, void *out1, const int64_t *rows_dev1, int64_t rows1, int N1, int K,
+                       int dtype, hipStream_t st)
+{
+    if (dtype == VTDGE_F32)
+        return launch_pair<float>(A0, W0, bias0, out0, rows0, N0, A1, W1, bias1, out1, rows_dev1, rows1, N1, K, st);
+    return launch_pair<bf16_t>(A0, W0, bias0, out0, rows0, N0, A1, W1, bias1, out1, rows_dev1, rows1, N1, K, st);
+}
+
 }  // namespace vtdge
 
 using namespace vtdge;
