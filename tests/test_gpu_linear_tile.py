@@ -1,0 +1,44 @@
+"""The bf16 Linear over long rows (K and N from 768 on) around the edges of its tiles: live rows at the ends of its 64-row units
+and of rounds of large tiles, each shape of the rest, output widths that end inside a tile, one slab of K more than twelve."""
+import pytest
+import torch
+
+from util import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("live", [0, 1, 63, 64, 65, 511, 513, 1700, 4200, 5500, 8190, 8193, 10700, 16390, 23000, None])
+@pytest.mark.parametrize("N,K", [(768, 768), (776, 832), (1664, 768), (3072, 768), (768, 3072)])
+@pytest.mark.parametrize("act,res", [("none", False), ("gelu", False), ("none", True)])
+def test_long_rows(dev, live, N, K, act, res):
+    from vtpack_amd import _lib, ops
+    cap = 25443
+    live = cap if live is None else live
+    g = torch.Generator(dev).manual_seed(live + N)
+    a, r = (torch.randn(*s, generator=g, device=dev).bfloat16() for s in ((cap, K), (cap, N)))
+    w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
+    bias = torch.randn(N, generator=g, device=dev).bfloat16() if live % 2 else None
+    out = torch.full((cap, N), 7.0, device=dev, dtype=torch.bfloat16)
+    ops.linear(a, w, bias, r if res else None, act=act, rows_dev=torch.tensor([live], device=dev), out=out)
+    assert "linear_tile_kernel" in _lib.last_kernel()
+    if live:
+        want = a[:live].float() @ w.float().T + (bias.float() if bias is not None else 0)
+        want = torch.nn.functional.gelu(want) if act == "gelu" else want
+        want = want + r[:live].float() if res else want
+        # one rounding of the result: 2^-9 of values up to about 6, against the largest of them
+        assert rel_err(out[:live], want) <= 2 ** -8
+    assert bool((out[live:] == 7.0).all())
+
+
+def test_rows_apart_and_a_result_in_the_residuals_place(dev):
+    from vtpack_amd import _lib, ops
+    g = torch.Generator(dev).manual_seed(1)
+    wide = torch.randn(3000, 1600, generator=g, device=dev).bfloat16()
+    w = (torch.randn(768, 768, generator=g, device=dev) * 768 ** -0.5).bfloat16()
+    r = torch.randn(3000, 768, generator=g, device=dev).bfloat16()
+    a = wide[:, 832:]
+    want = a.float() @ w.float().T + r.float()
+    ops.linear(a, w, None, r, out=r)
+    assert "linear_tile_kernel" in _lib.last_kernel()
+    assert rel_err(r, want) <= 2 ** -8

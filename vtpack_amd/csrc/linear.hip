@@ -215,6 +215,11 @@ int launch_linear_dma_split(const void *A, int64_t lda, const void *W, const voi
                       int64_t ldr, void *out, int64_t ldo, const int64_t *rows_dev, int64_t rows, int N, int K, int act,
                       hipStream_t st);
 
+// large tiles for bf16, long rows (linear_tile.hip)
+bool linear_tile_wanted(int64_t lda, int64_t rows, int N, int K, int act, const void *res);
+int launch_linear_tile(const void *A, int64_t lda, const void *W, const void *bias, const void *res, int64_t ldr, void *out,
+                       int64_t ldo, const int64_t *rows_dev, int64_t rows, int N, int K, int act, hipStream_t st);
+
 // weight-stationary variant for bf16, K = 384 (linear_ws8.hip)
 bool linear_ws_applicable(int64_t lda, int64_t ldr, int64_t ldo, int64_t rows, int N, int K, int esz, int act,
                           const void *bias, const void *res, const void *out);
@@ -461,6 +466,8 @@ extern "C" int vtdge_linear_prepacked(const void *A, int64_t lda, const void *W,
             return launch_linear_dma_split(A, lda, W, packed, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
         if (dtype == VTDGE_F32)
             return launch_linear_dma<float>(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
+        if (linear_tile_wanted(lda, rows, N, K, act, residual))
+            return launch_linear_tile(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
         return launch_linear_dma<bf16_t>(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
     }
     if (dtype == VTDGE_F32)
