@@ -504,6 +504,13 @@ int vtdge_layernorm_linear(const void *A0, int64_t lda0, const void *W0, const v
                            const void *ln_weight, const void *ln_bias, float ln_eps, int K, int act, int dtype,
                            void *stream);
 
+/* out0 = A0 W0^T + bias0 and out1 = A1 W1^T + bias1 over the same K in one launch, for few rows: the key/value and the query
+ * projection where the launch before them has written the LayerNorm of tokens and queries (vtdge_region_step).  Operands and
+ * sizes as in vtdge_layernorm_linear; the bits of two vtdge_linear calls. */
+int vtdge_linear_pair(const void *A0, int64_t lda0, const void *W0, const void *bias0, void *out0, const int64_t *rows_dev0,
+                      int64_t rows0, int N0, const void *A1, int64_t lda1, const void *W1, const void *bias1, void *out1,
+                      const int64_t *rows_dev1, int64_t rows1, int N1, int K, int dtype, void *stream);
+
 /* What a block does with its packed queries behind attention (vtpack/models/dge/deit_dge.py:127-128 with :74-75 and
  * :38-44), as one kernel without the hidden rows in memory:
  *   q1 = o proj_weight^T + proj_bias + comp,   out = q1 + fc2(gelu(fc1(LayerNorm(q1))))

@@ -63,6 +63,22 @@ def test_layernorm_inside(dev, dtype, vecs, rows, live):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("K,N0,N1", [(64, 128, 64), (192, 36, 192), (512, 1024, 512)])
+@pytest.mark.parametrize("rows,live", [(1, 1), (37, 0), (129, 64)])
+def test_two_products_in_one_launch(dev, dtype, K, N0, N1, rows, live):
+    from vtpack_amd import _lib, ops
+    x, c, w0, w1, b0 = _make(dev, dtype, K + rows, (rows, K), (rows, K), (N0, K), (N1, K), (N0,))
+    rd = torch.tensor([live], dtype=torch.int64, device=dev)
+    k, q = (torch.full((rows, n), 7.0, device=dev, dtype=dtype) for n in (N0, N1))
+    _lib.call("vtdge_linear_pair", x.data_ptr(), K, w0.data_ptr(), b0.data_ptr(), k.data_ptr(), 0, rows, N0, c.data_ptr(), K,
+              w1.data_ptr(), 0, q.data_ptr(), rd.data_ptr(), rows, N1, K, _lib.dtype_code(x), _lib.stream_ptr())
+    assert "linear_small" in _lib.last_kernel()
+    assert torch.equal(k, ops.linear(x, w0, b0))
+    assert torch.equal(q[:live], ops.linear(c, w1)[:live])
+    assert bool((q[live:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,H,C,k,N", [(1, 8, 64, 2, 32), (3, 8, 64, 8, 64), (2, 4, 128, 1, 8), (5, 12, 64, 4, 40)])
 def test_strided_convolution_of_few_rows(dev, dtype, B, H, C, k, N):
     from vtpack_amd import _lib, ops

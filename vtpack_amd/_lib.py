@@ -77,6 +77,7 @@ SIGNATURES = {
     "vtdge_layernorm_linear_fits": [_l, _i, _l, _i, _i, _i],
     "vtdge_layernorm_linear_wanted": [_l, _i, _l, _i, _i, _i],
     "vtdge_layernorm_linear": [_p, _l, _p, _p, _p, _p, _l, _i, _p, _l, _p, _p, _p, _p, _l, _i, _p, _p, _f, _i, _i, _i, _p],
+    "vtdge_linear_pair": [_p, _l, _p, _p, _p, _p, _l, _i, _p, _l, _p, _p, _p, _p, _l, _i, _i, _i, _p],
     "vtdge_block_tail_fits": [_l, _i, _i, _i],
     "vtdge_block_tail_wanted": [_l, _i, _i, _i],
     "vtdge_block_tail": [_p, _p, _p, _p, _p, _p, _f, _p, _p, _p, _p, _p, _p, _l, _i, _i, _i, _p],

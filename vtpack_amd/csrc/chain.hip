@@ -25,11 +25,6 @@ enum {
 };
 static_assert(P_COUNT == VTDGE_CHAIN_PARAMS, "the parameter table's documented length");
 
-// two Linears over few rows in one launch (linear_small.hip)
-int launch_linear_pair(const void *A0, const void *W0, const void *bias0, void *out0, int64_t rows0, int N0, const void *A1,
-                       const void *W1, const void *bias1, void *out1, const int64_t *rows_dev1, int64_t rows1, int N1, int K,
-                       int dtype, hipStream_t st);
-
 // first `n` rows of every sample of x [B, N, C] = rows [n, C] (the class tokens), 16 bytes a lane; `words` 64-bit words at
 // `clear` = 0 (the status words of the scatter-backs)
 __global__ __launch_bounds__(256) void front_rows_kernel(u32x4 *__restrict__ x, const u32x4 *__restrict__ rows,
@@ -352,8 +347,8 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
                 VT_TRY(split_block_weights(c, p, params, i, scratch, stream));
             if (p.ln_kvq && packed) {
                 // the scatter-back has left norm1 of tokens and queries
-                VT_TRY(launch_linear_pair(scratch + p.xln, P[P_KVW], P[P_KVB], kv, p.rows, 2 * C, scratch + p.comp_ln, P[P_QW],
-                                          P[P_QB], q, live, p.cap, C, C, dt, (hipStream_t)stream));
+                VT_TRY(vtdge_linear_pair(scratch + p.xln, C, P[P_KVW], P[P_KVB], kv, nullptr, p.rows, 2 * C, scratch + p.comp_ln,
+                                         C, P[P_QW], P[P_QB], q, live, p.cap, C, C, dt, stream));
             } else if (p.ln_kvq) {
                 VT_TRY(vtdge_layernorm_linear(x, C, P[P_KVW], P[P_KVB], kv, nullptr, p.rows, 2 * C, comp, C, P[P_QW], P[P_QB],
                                               q, live, p.cap, C, P[P_N1W], P[P_N1B], c->eps1, C, VTDGE_ACT_NONE, dt,

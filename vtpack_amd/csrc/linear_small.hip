@@ -440,25 +440,12 @@ static int launch_layernorm_linear(const void *A0, int64_t lda0, const void *W0,
 #undef VT_SMALL
 }
 
-// A0 W0^T + bias0 and A1 W1^T + bias1 over the same K in one launch: the key/value and the query projection of few rows whose
-// LayerNorm the kernel that produced them has written.  For sizes that layernorm_linear_fits takes.
+// A0 W0^T + bias0 and A1 W1^T + bias1 over the same K in one launch
 template <typename T>
-static int launch_pair(const void *A0, const void *W0, const void *bias0, void *out0, int64_t rows0, int N0, const void *A1,
-                       const void *W1, const void *bias1, void *out1, const int64_t *rows_dev1, int64_t rows1, int N1, int K,
-                       hipStream_t st)
+static int launch_pair(const SmallProblem &p0, const SmallProblem &p1, int K, hipStream_t st)
 {
     const PatchGeom none{0, 0, 0, 0, 0, 0, 0, 0};
-    const SmallProblem p0 = small_problem(A0, K, W0, bias0, nullptr, 0, out0, N0, nullptr, rows0, N0);
-    const SmallProblem p1 = small_problem(A1, K, W1, bias1, nullptr, 0, out1, N1, rows_dev1, rows1, N1);
     return go_small<T, 4, VTDGE_ACT_NONE, 0, false>(p0, p1, K, nullptr, nullptr, 0.f, none, st);
-}
-int launch_linear_pair(const void *A0, const void *W0, const void *bias0, void *out0, int64_t rows0, int N0, const void *A1,
-                       const void *W1, const void *bias1, void *out1, const int64_t *rows_dev1, int64_t rows1, int N1, int K,
-                       int dtype, hipStream_t st)
-{
-    if (dtype == VTDGE_F32)
-        return launch_pair<float>(A0, W0, bias0, out0, rows0, N0, A1, W1, bias1, out1, rows_dev1, rows1, N1, K, st);
-    return launch_pair<bf16_t>(A0, W0, bias0, out0, rows0, N0, A1, W1, bias1, out1, rows_dev1, rows1, N1, K, st);
 }
 
 }  // namespace vtdge
@@ -505,4 +492,26 @@ extern "C" int vtdge_layernorm_linear(const void *A0, int64_t lda0, const void *
                                               rows_dev1, rows1, N1, ln_weight, ln_bias, ln_eps, K, act, st);
     return launch_layernorm_linear<bf16_t>(A0, lda0, W0, bias0, out0, rows_dev0, rows0, N0, A1, lda1, W1, bias1, out1,
                                            rows_dev1, rows1, N1, ln_weight, ln_bias, ln_eps, K, act, st);
+}
+
+extern "C" int vtdge_linear_pair(const void *A0, int64_t lda0, const void *W0, const void *bias0, void *out0,
+                                 const int64_t *rows_dev0, int64_t rows0, int N0, const void *A1, int64_t lda1, const void *W1,
+                                 const void *bias1, void *out1, const int64_t *rows_dev1, int64_t rows1, int N1, int K, int dtype,
+                                 void *stream)
+{
+    VT_REQUIRE(A0 && W0 && out0 && A1 && W1 && out1, VTDGE_ERR_ARG, "linear_pair: NULL operand");
+    VT_REQUIRE(dtype == VTDGE_F32 || dtype == VTDGE_BF16, VTDGE_ERR_ARG, "linear_pair: unknown dtype %d", dtype);
+    const int esz = dtype == VTDGE_BF16 ? 2 : 4;
+    VT_REQUIRE(rows0 > 0 && rows1 > 0 && N0 > 0 && N1 > 0 && K > 0 && lda0 >= K && lda1 >= K, VTDGE_ERR_ARG,
+               "linear_pair: bad sizes");
+    VT_REQUIRE(layernorm_linear_fits(rows0, N0, rows1, N1, K, esz) && rows0 * lda0 * esz < (1ll << 31) &&
+                   rows1 * lda1 * esz < (1ll << 31) && (lda0 * esz) % 16 == 0 && (lda1 * esz) % 16 == 0,
+               VTDGE_ERR_UNSUPPORTED, "linear_pair: %lld x %d and %lld x %d outputs over %d values (see "
+               "vtdge_layernorm_linear_fits)", (long long)rows0, N0, (long long)rows1, N1, K);
+    VT_REQUIRE((((uintptr_t)A0 | (uintptr_t)W0 | (uintptr_t)out0 | (uintptr_t)A1 | (uintptr_t)W1 | (uintptr_t)out1) & 15) == 0,
+               VTDGE_ERR_ARG, "linear_pair: operands must be 16-byte aligned");
+    hipStream_t st = (hipStream_t)stream;
+    const SmallProblem p0 = small_problem(A0, lda0, W0, bias0, nullptr, 0, out0, N0, rows_dev0, rows0, N0);
+    const SmallProblem p1 = small_problem(A1, lda1, W1, bias1, nullptr, 0, out1, N1, rows_dev1, rows1, N1);
+    return dtype == VTDGE_F32 ? launch_pair<float>(p0, p1, K, st) : launch_pair<bf16_t>(p0, p1, K, st);
 }
