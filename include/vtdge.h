@@ -89,6 +89,14 @@ int vtdge_index_to_patch(const int64_t *indices, const int64_t *splits, int B, i
                          int R, int extra, int64_t *patches, int64_t capacity_rows, int64_t *offsets,
                          int64_t *lengths, void *stream);
 
+/* The same for up to 16384 regions with the lengths on the host when the call returns, as the reference's callers take them: the
+ * kernel writes them to `pinned` itself (int64 [B] of page-locked host memory that the GPU can write), the call waits for
+ * the stream and copies them to lengths_host int64 [B] and their sum to total_host int64 [1].  More regions:
+ * VTDGE_ERR_UNSUPPORTED.  Not for a stream that is being captured. */
+int vtdge_index_to_patch_host(const int64_t *indices, const int64_t *splits, int B, int Hr, int Wr, int S, int R, int extra,
+                              int64_t *patches, int64_t capacity_rows, int64_t *offsets, int64_t *pinned,
+                              int64_t *lengths_host, int64_t *total_host, void *stream);
+
 /* Every patch of every granularity (exported by the reference, unused by its
  * models).  Replaces grained_sample_index_to_patch_dense (grained_sample.cu:347-433).
  *   patches int64 [B * per_sample, 4], per_sample = extra + Hr*Wr*sum(splits^2)

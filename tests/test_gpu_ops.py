@@ -1020,3 +1020,30 @@ def test_patch_linear_refusals(dev):
     w = torch.zeros((64, 9 * 64), device=dev, dtype=torch.bfloat16)
     assert not ops.fits_patch_linear(x, 8, 8, 3, w, b)                   # the grid is not a multiple of the block
     assert not ops.fits_patch_linear(x, 8, 8, 2, w, None)
+
+
+@pytest.mark.parametrize("B,Hr,Wr", [(1, 1, 1), (64, 16, 16), (5, 64, 64), (4097, 2, 2)])
+def test_query_counts_on_the_host(dev, B, Hr, Wr):
+    """Counts that the kernel writes to host memory itself (up to 16384 regions) and counts that are copied; calls on two
+    streams and from two threads at once."""
+    import threading
+    from vtpack_amd import _C, ops
+    idx = random_indices(B + Hr, B, Hr, Wr)
+    sp = torch.tensor(SPLITS, device=dev)
+    want = orc.index_to_patch(idx, SPLITS, 4, 1)
+    bad = []
+
+    def check(stream):
+        with torch.cuda.stream(stream):
+            for _ in range(3):
+                patches, lengths = _C.grained_sample_index_to_patch(_t(idx, dev), sp, 4, 1)
+                if lengths.is_cuda or lengths.is_pinned() or not np.array_equal(lengths.numpy(), want[1]) or \
+                        not np.array_equal(patches.cpu().numpy(), want[0]):
+                    bad.append(stream)
+    threads = [threading.Thread(target=check, args=(s,)) for s in (torch.cuda.current_stream(), torch.cuda.Stream())]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    assert ops.index_to_patch_host(_t(idx, dev), sp, 4, 1)[2] == int(want[1].sum())

@@ -25,9 +25,7 @@ def grained_sample_index_to_patch(indices, split_sizes, region_size, num_extra_t
     vtpack/layers/csrc/grained_sample/grained_sample.cu:302-345."""
     if indices.dtype != torch.int64 or split_sizes.dtype != torch.int64:
         raise TypeError("indices and split_sizes must be int64")
-    patches, offsets, lengths = ops.index_to_patch(indices, split_sizes, int(region_size), int(num_extra_tokens))
-    batch_lengths = lengths.cpu()
-    total = int(batch_lengths.sum())
+    patches, batch_lengths, total = ops.index_to_patch_host(indices, split_sizes, int(region_size), int(num_extra_tokens))
     if total > patches.shape[0]:
         raise RuntimeError(
             f"split sizes produce {total} queries, more than one per token ({patches.shape[0]}): "
@@ -98,9 +96,10 @@ def batched_sparse_attention_forward(a, b, c, batch_lengths, scale):
     h, L, d = a.shape
     _, B, n, _ = b.shape
     offsets, lengths = ops.lengths_to_offsets(batch_lengths, a.device)
-    if lengths.numel() != B or int(lengths.sum()) != L:
+    counts = lengths.flatten().tolist()
+    if len(counts) != B or sum(counts) != L:
         raise ValueError("batch_lengths must have one entry per sample and sum to the number of query rows")
-    return ops.sparse_attention_heads(a, b, c, offsets, scale, int(lengths.max()) if B > 0 else 0)
+    return ops.sparse_attention_heads(a, b, c, offsets, scale, max(counts) if B > 0 else 0)
 
 
 def batched_sparse_gemm_forward(a, b, a_lengths, b_lengths, is_a_transposed, is_b_transposed):

@@ -28,6 +28,7 @@ SIGNATURES = {
     "vtdge_router": [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p],
     "vtdge_router_layernorm": [_p, _p, _p, _p, _p, _p, _p, _f, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p],
     "vtdge_index_to_patch": [_p, _p, _i, _i, _i, _i, _i, _i, _p, _l, _p, _p, _p],
+    "vtdge_index_to_patch_host": [_p, _p, _i, _i, _i, _i, _i, _i, _p, _l, _p, _p, _p, _p, _p],
     "vtdge_index_to_patch_dense": [_p, _i, _i, _i, _i, _i, _i, _p, _p],
     "vtdge_compress": [_p, _p, _p, _l, _p, _p, _p, _p, _f, _i, _i, _i, _i, _i, _i, _p],
     "vtdge_decompress": [_p, _p, _p, _p, _l, _p, _p, _i, _i, _i, _i, _i, _i, _p],
@@ -149,11 +150,12 @@ timer = None
 
 
 def call(name, *args, tag=None):
-    lib = load()
-    if timer is not None:
+    lib = _lib if _lib is not None else load()
+    if timer is None:
+        rc = getattr(lib, name)(*args)
+    else:
         timer.begin(name, tag)
-    rc = getattr(lib, name)(*args)
-    if timer is not None:
+        rc = getattr(lib, name)(*args)
         timer.end()
     if rc != 0:
         msg = lib.vtdge_last_error().decode("utf-8", "replace")

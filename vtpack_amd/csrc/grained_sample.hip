@@ -1600,6 +1600,8 @@ extern "C" int vtdge_router_layernorm(const void *x, const void *weight, const v
     return check_launch("router_layernorm");
 }
 
+constexpr int64_t ONE_LAUNCH_REGIONS = 16384;
+
 extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *splits, int B, int Hr, int Wr, int S,
                                     int R, int extra, int64_t *patches, int64_t capacity_rows, int64_t *offsets,
                                     int64_t *lengths, void *stream)
@@ -1612,7 +1614,7 @@ extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *split
     VT_REQUIRE((reinterpret_cast<uintptr_t>(patches) & 15u) == 0, VTDGE_ERR_ARG,
                "index_to_patch: patches must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
-    if (patches != nullptr && (int64_t)B * Hr * Wr <= 16384) {
+    if (patches != nullptr && (int64_t)B * Hr * Wr <= ONE_LAUNCH_REGIONS) {
         // small batches: one launch, every sample's workgroup sums the counts before it on its own
         note_kernel(reinterpret_cast<const void *>(patch_write_kernel<true>));
         patch_write_kernel<true><<<B, 256, 0, st>>>(indices, splits, offsets, lengths, Hr, Wr, S, R, extra, patches,
@@ -1638,6 +1640,26 @@ extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *split
                                                      capacity_rows, 0);
         return check_launch("index_to_patch(write)");
     }
+    return VTDGE_OK;
+}
+
+// A device-to-host copy behind the kernel costs its own launch and a round trip through the runtime's staging buffer: 15 to 20 us
+// a call on top of the wait itself.
+extern "C" int vtdge_index_to_patch_host(const int64_t *indices, const int64_t *splits, int B, int Hr, int Wr, int S, int R,
+                                         int extra, int64_t *patches, int64_t capacity_rows, int64_t *offsets, int64_t *pinned,
+                                         int64_t *lengths_host, int64_t *total_host, void *stream)
+{
+    VT_REQUIRE(patches && pinned && lengths_host && total_host, VTDGE_ERR_ARG, "index_to_patch: NULL operand");
+    VT_REQUIRE(B > 0 && Hr > 0 && Wr > 0 && (int64_t)B * Hr * Wr <= ONE_LAUNCH_REGIONS, VTDGE_ERR_UNSUPPORTED,
+               "index_to_patch: lengths on the host for %lld regions (at most %lld)", (long long)B * Hr * Wr,
+               (long long)ONE_LAUNCH_REGIONS);
+    const int rc = vtdge_index_to_patch(indices, splits, B, Hr, Wr, S, R, extra, patches, capacity_rows, offsets, pinned, stream);
+    if (rc != VTDGE_OK) return rc;
+    const hipError_t err = hipStreamSynchronize((hipStream_t)stream);
+    VT_REQUIRE(err == hipSuccess, VTDGE_ERR_LAUNCH, "index_to_patch: %s", hipGetErrorString(err));
+    int64_t total = 0;
+    for (int b = 0; b < B; b++) total += lengths_host[b] = pinned[b];
+    *total_host = total;
     return VTDGE_OK;
 }
 

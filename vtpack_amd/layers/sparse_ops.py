@@ -48,13 +48,13 @@ class _SparseAttentionTrain(Function):
     and again backward.  q [h, L, d], k and v [h, B, n, d] -> [L, h * d]."""
 
     @staticmethod
-    def forward(ctx, q, k, v, q_lengths, scale):
+    def forward(ctx, q, k, v, q_lengths, scale, max_rows):
         ops._need_gpu(q, k, v)
         q, k, v = (ops.on_boundary(t) for t in (ops.vector_rows(q), k.contiguous(), v.contiguous()))
         h, L, d = q.shape
-        offsets, lengths = ops.lengths_to_offsets(q_lengths, q.device)
+        offsets, _ = ops.lengths_to_offsets(q_lengths, q.device)
         out = torch.empty((L, h * d), dtype=q.dtype, device=q.device)
-        ctx.scale, ctx.max_rows = scale, int(lengths.max())
+        ctx.scale, ctx.max_rows = scale, max_rows
         ops.sparse_attention_heads(q, k, v, offsets, scale, ctx.max_rows, out=out.view(L, h, d).transpose(0, 1), train=True)
         ctx.save_for_backward(q, k, v, offsets)      # not the result: a caller may change that in place
         return out
@@ -68,7 +68,7 @@ class _SparseAttentionTrain(Function):
         q, k, v, grad = (ops.on_boundary(t) for t in (ops.vector_rows(q), *(t.contiguous() for t in (k, v, grad))))
         grad = grad.view(L, h, d).transpose(0, 1)
         dq, dk, dv = ops.sparse_attention_backward(q, k, v, None, grad, offsets, ctx.scale, ctx.max_rows)
-        return dq, dk, dv, None, None
+        return dq, dk, dv, None, None, None
 
 
 def sparse_attention_train(q, k, v, q_lengths, scale):
@@ -80,14 +80,15 @@ def sparse_attention_train(q, k, v, q_lengths, scale):
     a gradient or differ by head), compose two `batched_sparse_gemm` calls around a softmax over the keys."""
     h, L, d = q.shape
     B, n = k.shape[1], k.shape[2]
-    if int(q_lengths.max()) == int(q_lengths.min()):
+    counts = q_lengths.flatten().tolist()
+    if max(counts) == min(counts):
         scores = torch.matmul(q.reshape(h, B, -1, d), k.transpose(-1, -2)) * scale
         ctx = torch.matmul(scores.softmax(dim=-1, dtype=v.dtype), v)              # [h, B, Lq, d]
         return ctx.permute(1, 2, 0, 3).reshape(-1, h * d)
     if (d == 64 and not torch.is_tensor(scale) and q.is_cuda and q.dtype in (torch.float32, torch.bfloat16)
             and q.dtype == k.dtype == v.dtype and k.shape == v.shape and k.shape[0] == h and k.shape[3] == d
-            and q_lengths.numel() == B and int(q_lengths.sum()) == L):
-        return _SparseAttentionTrain.apply(q, k, v, q_lengths, float(scale))
+            and len(counts) == B and sum(counts) == L):
+        return _SparseAttentionTrain.apply(q, k, v, q_lengths, float(scale), int(max(counts)))
     kv_lengths = q_lengths.new_full([B], n)
     scores = batched_sparse_gemm(q, k.reshape(h, -1, d), q_lengths, kv_lengths, False, True) * scale
     ctx = batched_sparse_gemm(scores.softmax(dim=-1, dtype=v.dtype), v.reshape(h, -1, d), q_lengths, kv_lengths,

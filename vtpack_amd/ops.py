@@ -111,6 +111,31 @@ def index_to_patch(indices, splits, region_size, num_extra_tokens, capacity=None
     return patches, offsets, lengths
 
 
+def index_to_patch_host(indices, splits, region_size, num_extra_tokens):
+    """`index_to_patch` for callers that need the query counts now: (patches [capacity, 4], lengths [B] on the CPU, their
+    sum), behind a wait for the stream."""
+    _need_gpu(indices, splits)
+    if indices.dtype != torch.int64 or splits.dtype != torch.int64 or indices.dim() != 3:
+        raise TypeError("indices must be int64 [B, Hr, Wr] and splits int64")
+    B, Hr, Wr = indices.shape
+    if not 0 < B * Hr * Wr <= 16384:
+        patches, _, lengths = index_to_patch(indices, splits, region_size, num_extra_tokens)
+        lengths = lengths.cpu()
+        return patches, lengths, int(lengths.sum())
+    indices, splits = _contig(indices), _contig(splits)
+    capacity = B * (num_extra_tokens + Hr * Wr * region_size * region_size)
+    device = indices.device
+    patches = torch.empty((capacity, 4), dtype=torch.int64, device=device)
+    offsets = torch.empty((B + 1,), dtype=torch.int64, device=device)
+    pinned = torch.empty((B,), dtype=torch.int64, pin_memory=True)
+    lengths = torch.empty((B,), dtype=torch.int64)
+    total = ctypes.c_int64()
+    call("vtdge_index_to_patch_host", indices.data_ptr(), splits.data_ptr(), B, Hr, Wr, splits.numel(), region_size,
+         num_extra_tokens, patches.data_ptr(), capacity, offsets.data_ptr(), pinned.data_ptr(), lengths.data_ptr(),
+         ctypes.addressof(total), stream_ptr(), tag=("index_to_patch",))
+    return patches, lengths, total.value
+
+
 def compress(x, patches, width, num_extra_tokens, rows_dev=None, rows=None, ln_weight=None, ln_bias=None,
              ln_eps=1e-6):
     """x [B,N,C] -> comp [rows,C] (and LayerNorm(comp) when ln_weight is given)."""
@@ -936,7 +961,8 @@ def sparse_attention(q, k, v, offsets, scale, num_heads, max_rows_per_sample, ou
 
 def lengths_to_offsets(lengths, device):
     """CPU int64 lengths [B] -> device int64 offsets [B + 1], without a copy of host memory."""
-    lengths = lengths.detach().to("cpu", torch.int64).contiguous()
+    if lengths.dtype != torch.int64 or lengths.is_cuda or lengths.requires_grad or not lengths.is_contiguous():
+        lengths = lengths.detach().to("cpu", torch.int64).contiguous()
     offsets = torch.empty((lengths.numel() + 1,), dtype=torch.int64, device=device)
     call("vtdge_lengths_to_offsets", lengths.data_ptr(), lengths.numel(), ptr(offsets), stream_ptr(), tag=("offsets",))
     return offsets, lengths
