@@ -17,7 +17,8 @@
 // component of twice the spread in keys and values: 5.1e-2 from the rounded output, 3.6e-3 this way).
 //
 // Both are one scheme.  A wave keeps 16 rows of two operands in registers (Q and dO, or K and V) and walks the rows of
-// the other two, which the workgroup's four waves share through LDS in stages of 32 by direct loads (two buffers).  With
+// the other two, which the workgroup's four waves share through LDS in stages of 32 by direct loads (two buffers; over the queries
+// three or four, statistics among them: us, 64 samples, 3 heads, 257 keys, fp32 69.6 -> 60.7, 128, 6, bf16 46.2 -> 41.4).  With
 // the walked rows as rows of v_mfma_f32_16x16 tiles and the kept ones as columns, lane (l = lane % 16, g = lane / 16) holds
 // the score of walked rows 4 g + r (r < 4) with kept row l: the operand layout of the products over the walked rows, so
 // nothing moves between lanes.  Those products read the walked rows transposed: in fp32 a lane takes 4 consecutive channels
@@ -158,16 +159,23 @@ template <typename T> struct Stager {
     const unsigned char *base;
     uint32_t pitch, lds0;
     int rows, wid, lane;
-    __device__ __forceinline__ void load(int st) const
+    __device__ __forceinline__ void load(int st, int slot) const
     {
         const int r0 = st * AB_ROWS, last = rows - 1 - r0;
-        const uint32_t dst = lds0 + (uint32_t)((st & 1) * 2 * B::HALF + wid * NL * 1024);
+        const uint32_t dst = lds0 + (uint32_t)(slot * 2 * B::HALF + wid * NL * 1024);
         const void *src = uniform_ptr(base + (int64_t)r0 * pitch);
 #pragma unroll
         for (int i = 0; i < NL; i++) {
             const int row = ((wid & 1) * NL + i) * (64 / B::CPR) + lane / B::CPR;
             dma16(src, (uint32_t)min(row, last) * pitch + (uint32_t)B::slot(row, lane % B::CPR) * 16u, dst + i * 1024);
         }
+    }
+    // at most `younger` stages of this wave's loads, PER of them each, are outstanding
+    template <int PER> static __device__ __forceinline__ void wait(int younger)
+    {
+        if (younger >= 2) wait_vmcnt<2 * PER>();
+        else if (younger == 1) wait_vmcnt<PER>();
+        else wait_vmcnt<0>();
     }
 };
 
@@ -184,6 +192,73 @@ __device__ __forceinline__ void load_kept(typename BackMath<T>::Frag (&f)[BackTi
     }
 }
 
+// The (sample, head) pair and the chunk of 64 of its queries that this workgroup takes.  The pairs of an XCD (8 i + xcd) lie one
+// behind the other with as many workgroups each as it has chunks, found from the samples' offsets: a grid with room for the
+// longest sample's chunks in every pair, taken as it stands, leaves holes that the dispatcher deals out like work, and the last
+// live workgroups start when the first have ended (us, 64 samples, 3 heads, 257 keys, fp32: 72.6 -> 45.9; 128, 6, bf16: 45.9 ->
+// 41.9).  More pairs than are looked through in a few steps keep to that grid.
+constexpr int AB_SEARCH = 1024;
+__device__ __forceinline__ bool find_chunk(const int64_t *offsets, int pairs, int h, int &pair, int &chunk, int64_t &row0, int &Lb)
+{
+    const int rest = blockIdx.x >> 3, xcd = blockIdx.x & 7, pairs_x = (pairs + 7) / 8;
+    if (pairs_x > AB_SEARCH) {
+        pair = (rest % pairs_x) * 8 + xcd;
+        chunk = rest / pairs_x;
+        if (pair >= pairs) return false;
+        row0 = offsets[pair / h];
+        Lb = (int)(offsets[pair / h + 1] - row0);
+        return chunk * 16 * AB_WAVES < Lb;
+    }
+    __shared__ int totals[AB_SEARCH / 256][4], found[2];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    int mine[AB_SEARCH / 256], upto[AB_SEARCH / 256];
+    if (tid == 0) found[0] = -1;
+#pragma unroll
+    for (int k = 0; k < AB_SEARCH / 256; k++) {
+        const int p = (k * 256 + tid) * 8 + xcd;
+        mine[k] = 0;
+        if (k * 256 < pairs_x && p < pairs) {
+            const int b = p / h;
+            mine[k] = (int)((offsets[b + 1] - offsets[b] + 16 * AB_WAVES - 1) / (16 * AB_WAVES));
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < AB_SEARCH / 256; k++) {
+        int v = mine[k];
+        if (k * 256 < pairs_x) {
+#pragma unroll
+            for (int o = 1; o < WAVE; o <<= 1) {
+                const int up = __shfl_up(v, o, WAVE);
+                if (lane >= o) v += up;
+            }
+        }
+        upto[k] = v;
+        if (lane == 63) totals[k][wid] = v;
+    }
+    __syncthreads();
+    int before = 0;
+#pragma unroll
+    for (int k = 0; k < AB_SEARCH / 256; k++)
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            if (w == wid) {
+                const int first = before + upto[k] - mine[k];
+                if (rest >= first && rest < first + mine[k]) {
+                    found[0] = (k * 256 + tid) * 8 + xcd;
+                    found[1] = rest - first;
+                }
+            }
+            before += totals[k][w];
+        }
+    __syncthreads();
+    pair = __builtin_amdgcn_readfirstlane(found[0]);
+    chunk = __builtin_amdgcn_readfirstlane(found[1]);
+    if (pair < 0) return false;
+    row0 = offsets[pair / h];
+    Lb = (int)(offsets[pair / h + 1] - row0);
+    return true;
+}
+
 // The forward pass in bf16, from the same scores as the gradients: the inference kernels round the queries once more, times
 // the scale, and take their reference score from the first 32 keys, so that a row whose first scores are all -infinity comes
 // out as NaN.  Here a query's reference is its running maximum; until a finite score comes there is none and nothing is
@@ -192,14 +267,12 @@ __global__ __launch_bounds__(256, 4) void attention_train_kernel(AttnTrain a)
 {
     using B = BackTile<bf16_t>;
     using M = BackMath<bf16_t>;
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * B::HALF];
-    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8;
-    const int pair = (rest % pairs_x) * 8 + (blockIdx.x & 7), chunk = rest / pairs_x;
-    if (pair >= a.pairs) return;
+    constexpr int DEPTH = 2;                              // stages in LDS
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * B::HALF];
+    int pair, chunk, Lb;
+    int64_t row0;
+    if (!find_chunk(a.offsets, a.pairs, a.h, pair, chunk, row0, Lb)) return;
     const int b = pair / a.h, head = pair - b * a.h;
-    const int64_t row0 = a.offsets[b];
-    const int Lb = (int)(a.offsets[b + 1] - row0);
-    if (chunk * 16 * AB_WAVES >= Lb) return;
     const int lane = threadIdx.x & 63, l = lane & 15, g = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int row = (chunk * AB_WAVES + wid) * 16 + l;
@@ -209,7 +282,7 @@ __global__ __launch_bounds__(256, 4) void attention_train_kernel(AttnTrain a)
     const Stager<bf16_t> kv{reinterpret_cast<const unsigned char *>((wid < 2 ? a.k : a.v) + kv_at), (uint32_t)(a.kv_ts * 2),
                             (uint32_t)(uintptr_t)smem, a.n, wid, lane};
     const int stages = (a.n + AB_ROWS - 1) / AB_ROWS;
-    kv.load(0);
+    for (int st = 0; st < DEPTH - 1 && st < stages; st++) kv.load(st, st);
     typename M::Frag qf[B::NF];
     load_kept<bf16_t>(qf, a.q + (row0 + row) * a.q_rs + (int64_t)head * a.q_hs, live, g);
     f32x4 o[4];
@@ -217,10 +290,10 @@ __global__ __launch_bounds__(256, 4) void attention_train_kernel(AttnTrain a)
     for (int i = 0; i < 4; i++) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, s = 0.f;                         // of this lane's query; s of this lane's keys
     for (int st = 0; st < stages; st++) {
-        wait_vmcnt<0>();
+        Stager<bf16_t>::wait<Stager<bf16_t>::NL>(min(stages - 1 - st, DEPTH - 2));
         block_barrier();
-        if (st + 1 < stages) kv.load(st + 1);
-        unsigned char *Ks = smem + (st & 1) * 2 * B::HALF, *Vs = Ks + B::HALF;
+        if (st + DEPTH - 1 < stages) kv.load(st + DEPTH - 1, (st + DEPTH - 1) % DEPTH);
+        unsigned char *Ks = smem + st % DEPTH * 2 * B::HALF, *Vs = Ks + B::HALF;
         const int left = a.n - st * AB_ROWS;
         if (left < AB_ROWS) {                             // values past the last key: nothing of them, not even 0 * infinity
             for (int i = left * B::CPR + threadIdx.x; i < AB_ROWS * B::CPR; i += 64 * AB_WAVES)
@@ -267,14 +340,12 @@ template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 
 {
     using B = BackTile<T>;
     using M = BackMath<T>;
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * B::HALF];
-    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8;
-    const int pair = (rest % pairs_x) * 8 + (blockIdx.x & 7), chunk = rest / pairs_x;
-    if (pair >= a.pairs) return;
+    constexpr int DEPTH = 2;                              // stages in LDS
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * B::HALF];
+    int pair, chunk, Lb;
+    int64_t row0;
+    if (!find_chunk(a.offsets, a.pairs, a.h, pair, chunk, row0, Lb)) return;
     const int b = pair / a.h, head = pair - b * a.h;
-    const int64_t row0 = a.offsets[b];
-    const int Lb = (int)(a.offsets[b + 1] - row0);
-    if (chunk * 16 * AB_WAVES >= Lb) return;
     const int lane = threadIdx.x & 63, l = lane & 15, g = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int row = (chunk * AB_WAVES + wid) * 16 + l;
@@ -283,8 +354,16 @@ template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 
     const int64_t kv_at = (int64_t)b * a.kv_bs + (int64_t)head * a.kv_hs;
     const Stager<T> kv{reinterpret_cast<const unsigned char *>((const T *)(wid < 2 ? a.k : a.v) + kv_at),
                        (uint32_t)(a.kv_ts * sizeof(T)), (uint32_t)(uintptr_t)smem, a.n, wid, lane};
+    // the keys are walked twice, as one sequence of stages: the second walk's first ones are on their way when the first
+    // ends (of scores held it takes keys only)
     const int stages = (a.n + AB_ROWS - 1) / AB_ROWS;
-    kv.load(0);
+    const bool twice = HELD == 0 || wid < 2;
+    const int total = twice ? 2 * stages : stages;        // stages that this wave loads
+    auto load = [&](int u) {
+        if (u < total) kv.load(u < stages ? u : u - stages, u % DEPTH);
+    };
+    auto stage_at = [&](int u) { return smem + u % DEPTH * 2 * B::HALF; };
+    for (int u = 0; u < DEPTH - 1; u++) load(u);
 
     typename M::Frag qf[B::NF], df[B::NF];
     load_kept<T>(qf, (const T *)a.q + (row0 + row) * a.q_rs + (int64_t)head * a.q_hs, live, g);
@@ -294,7 +373,7 @@ template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 
     float m = -INFINITY, s = 0.f, sd = 0.f;
     f32x4 held_t[HELD > 0 ? HELD : 1][2], held_dp[HELD > 0 ? HELD : 1][2];
     auto sums = [&](int st, f32x4 (&t)[2], f32x4 (&dp)[2]) {
-        const unsigned char *Ks = smem + (st & 1) * 2 * B::HALF, *Vs = Ks + B::HALF;
+        const unsigned char *Ks = stage_at(st), *Vs = Ks + B::HALF;
         float mx = m;
 #pragma unroll
         for (int blk = 0; blk < 2; blk++) {
@@ -323,22 +402,22 @@ template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 
         sd = sd * down + (((ed[0][0] + ed[0][1]) + (ed[0][2] + ed[0][3])) + ((ed[1][0] + ed[1][1]) + (ed[1][2] + ed[1][3])));
         m = mx;
     };
-    auto next_stage = [&](int st, bool values) {
-        wait_vmcnt<0>();
+    auto next_stage = [&](int u) {
+        Stager<T>::template wait<Stager<T>::NL>(min(total - 1 - u, DEPTH - 2));
         block_barrier();
-        if (st + 1 < stages && (values || wid < 2)) kv.load(st + 1);
+        load(u + DEPTH - 1);
     };
     if constexpr (HELD > 0) {
         static_for<HELD>([&](auto st_c) {
             constexpr int st = decltype(st_c)::value;
             if (st < stages) {
-                next_stage(st, true);
+                next_stage(st);
                 if (wave_live) sums(st, held_t[st], held_dp[st]);
             }
         });
     } else {
         for (int st = 0; st < stages; st++) {
-            next_stage(st, true);
+            next_stage(st);
             if (wave_live) sums(st, held_t[0], held_dp[0]);
         }
     }
@@ -364,8 +443,6 @@ template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 
     f32x4 dq[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) dq[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    block_barrier();                                      // the last stage has been read
-    if (HELD == 0 || wid < 2) kv.load(0);                 // scores held: keys only
     auto add = [&](int st, const f32x4 (&t)[2], const f32x4 (&dp)[2]) {
         f32x4 ds[2];
 #pragma unroll
@@ -376,21 +453,21 @@ template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 
                 const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -all));
                 ds[blk][r] = in ? e * (dp[blk][r] - delta) * scale_s : 0.f;
             }
-        M::accumulate(smem + (st & 1) * 2 * B::HALF, ds, dq, l, g);
+        M::accumulate(stage_at(stages + st), ds, dq, l, g);
     };
     if constexpr (HELD > 0) {
         static_for<HELD>([&](auto st_c) {
             constexpr int st = decltype(st_c)::value;
             if (st < stages) {
-                next_stage(st, false);
+                next_stage(stages + st);
                 if (wave_live) add(st, held_t[st], held_dp[st]);
             }
         });
     } else {
         for (int st = 0; st < stages; st++) {
-            next_stage(st, true);
+            next_stage(stages + st);
             if (!wave_live) continue;
-            const unsigned char *Ks = smem + (st & 1) * 2 * B::HALF, *Vs = Ks + B::HALF;
+            const unsigned char *Ks = stage_at(stages + st), *Vs = Ks + B::HALF;
             f32x4 t[2], dp[2];
 #pragma unroll
             for (int blk = 0; blk < 2; blk++) {
@@ -408,9 +485,14 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
 {
     using B = BackTile<T>;
     using M = BackMath<T>;
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * B::HALF];
-    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8;
-    const int pair = (rest % pairs_x) * 8 + (blockIdx.x & 7), chunk = rest / pairs_x;
+    constexpr int DEPTH = sizeof(T) == 4 ? 3 : 4;         // stages in LDS
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * B::HALF];
+    __shared__ __attribute__((aligned(256))) float stats[DEPTH][3][64];      // m, 1 / s and delta of a stage's rows (twice)
+    // bf16: the chunks of a pair one behind the other (39.1 us at 128 samples of 6 heads and 257 keys, 40.9 chunk by chunk); fp32
+    // the other way round (60.7 us at 64 of 3; 63.1).  Pairs with most queries first: 48.2 and 57.0.
+    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8, chunks = (a.n + 16 * AB_WAVES - 1) / (16 * AB_WAVES);
+    const int chunk = sizeof(T) == 4 ? rest / pairs_x : rest % chunks;
+    const int pair = (sizeof(T) == 4 ? rest % pairs_x : rest / chunks) * 8 + (blockIdx.x & 7);
     if (pair >= a.pairs) return;
     const int b = pair / a.h, head = pair - b * a.h;
     const int64_t row0 = a.offsets[b];
@@ -427,23 +509,17 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
     const int64_t stat = (int64_t)head * a.L + row0;
     const bool apart = sizeof(T) == 4 && a.inv != nullptr;
     const float *rm = a.m + stat, *rinv = apart ? a.inv + stat : nullptr, *delta = a.delta + stat;
-    // m, 1 / s and delta of the lane's walked rows, one stage ahead; rows past the sample's last query: probability zero
-    f32x4 nm[2], niv[2], ndl[2];
-    auto fetch = [&](int st) {
-#pragma unroll
-        for (int blk = 0; blk < 2; blk++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int i = st * AB_ROWS + 16 * blk + 4 * g + r;
-                nm[blk][r] = i < Lb ? rm[i] : INFINITY;
-                niv[blk][r] = apart && i < Lb ? rinv[i] : 1.f;
-                ndl[blk][r] = i < Lb ? delta[i] : 0.f;
-            }
+    // waves 1 to 3 bring one of them each, behind their share of the rows
+    const float *mine = wid == 1 ? rm : wid == 2 ? rinv : delta;
+    const bool brings = wid == 1 || wid == 3 || (wid == 2 && apart);
+    auto load = [&](int st) {
+        const int slot = st % DEPTH;
+        qd.load(st, slot);
+        if (brings)
+            dma4(uniform_ptr(mine + st * AB_ROWS), (uint32_t)min(lane & 31, Lb - 1 - st * AB_ROWS) * 4u,
+                 (uint32_t)(uintptr_t)&stats[slot][wid - 1][0]);
     };
-    if (stages > 0) {
-        qd.load(0);
-        fetch(0);
-    }
+    for (int st = 0; st < DEPTH - 1 && st < stages; st++) load(st);
     typename M::Frag kf[B::NF], vf[B::NF];
     const int64_t kv_at = (int64_t)b * a.kv_bs + (int64_t)key * a.kv_ts + (int64_t)head * a.kv_hs;
     load_kept<T>(kf, (const T *)a.k + kv_at, live, g);
@@ -453,14 +529,12 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
     for (int i = 0; i < 4; i++) dk[i] = dv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     for (int st = 0; st < stages; st++) {
-        wait_vmcnt<0>();
+        const int younger = min(stages - 1 - st, DEPTH - 2);
+        if (brings) Stager<T>::template wait<Stager<T>::NL + 1>(younger);
+        else Stager<T>::template wait<Stager<T>::NL>(younger);
         block_barrier();
-        const f32x4 ms[2] = {nm[0], nm[1]}, iv[2] = {niv[0], niv[1]}, dl[2] = {ndl[0], ndl[1]};
-        if (st + 1 < stages) {
-            qd.load(st + 1);
-            if (wave_live) fetch(st + 1);
-        }
-        unsigned char *Qs = smem + (st & 1) * 2 * B::HALF, *Ds = Qs + B::HALF;
+        if (st + DEPTH - 1 < stages) load(st + DEPTH - 1);
+        unsigned char *Qs = smem + st % DEPTH * 2 * B::HALF, *Ds = Qs + B::HALF;
         const int left = Lb - st * AB_ROWS;
         if (left < AB_ROWS) {                             // dO past the last query: nothing of it, not even 0 * infinity
             for (int i = left * B::CPR + threadIdx.x; i < AB_ROWS * B::CPR; i += 64 * AB_WAVES)
@@ -468,6 +542,24 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
             lds_barrier();
         }
         if (!wave_live) continue;
+        f32x4 ms[2], iv[2], dl[2];                        // rows past the sample's last query: probability zero
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            const float (&of)[3][64] = stats[st % DEPTH];
+            const int i = 16 * blk + 4 * g;
+            ms[blk] = *reinterpret_cast<const f32x4 *>(&of[0][i]);
+            iv[blk] = f32x4{1.f, 1.f, 1.f, 1.f};
+            if (apart) iv[blk] = *reinterpret_cast<const f32x4 *>(&of[1][i]);
+            dl[blk] = *reinterpret_cast<const f32x4 *>(&of[2][i]);
+            if (left < AB_ROWS)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const bool in = i + r < left;
+                    ms[blk][r] = in ? ms[blk][r] : INFINITY;
+                    iv[blk][r] = in ? iv[blk][r] : 1.f;
+                    dl[blk][r] = in ? dl[blk][r] : 0.f;
+                }
+        }
         f32x4 p[2], ds[2];
 #pragma unroll
         for (int blk = 0; blk < 2; blk++) {

@@ -252,6 +252,12 @@ __device__ __forceinline__ void dma16(const void *base, uint32_t off, uint32_t l
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(off), "s"(base)
                  : "memory", "m0");
 }
+// four bytes a lane: LDS bytes [lds_addr, lds_addr + 256)
+__device__ __forceinline__ void dma4(const void *base, uint32_t off, uint32_t lds_addr)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_addr), "v"(off), "s"(base)
+                 : "memory", "m0");
+}
 // the same for data that is read once and not again (streamed past the caches' reuse-oriented replacement)
 __device__ __forceinline__ void dma16_nt(const void *base, uint32_t off, uint32_t lds_addr)
 {
