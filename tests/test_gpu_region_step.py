@@ -13,7 +13,9 @@ pytestmark = pytest.mark.gpu
     (5, 5, 13, 384, 3, "bf16", "records"), (96, 4, 4, 384, 1, "bf16", "records"), (1, 8, 8, 384, 1, "bf16", "plain"),
     (2, 4, 4, 512, 9, "bf16", "norm"), (7, 3, 3, 768, 1, "bf16", "norm"), (1, 4, 4, 1536, 1, "bf16", "norm"),
     (65, 1, 1, 192, 1, "f32", "norm"), (128, 4, 4, 192, 1, "f32", "norm"), (3, 4, 4, 132, 0, "f32", "plain"),
-    (2, 6, 4, 320, 0, "f32", "norm"), (3, 4, 4, 768, 64, "f32", "norm")])
+    (2, 6, 4, 320, 0, "f32", "norm"), (3, 4, 4, 768, 64, "f32", "norm"), (2, 4, 4, 8, 0, "bf16", "norm"),
+    (1, 16, 16, 64, 0, "bf16", "norm"), (3, 4, 4, 64, 1, "f32", "norm"), (96, 4, 4, 192, 1, "bf16", "norm"),
+    (2, 3, 5, 12, 0, "f32", "plain"), (5, 8, 8, 128, 0, "bf16", "plain"), (2, 4, 4, 256, 1, "bf16", "norm")])
 @pytest.mark.parametrize("placed", [False, True])
 def test_against_the_separate_operators(dev, B, Hr, Wr, C, extra, dtype, mode, placed):
     from vtpack_amd import _lib, ops

@@ -43,8 +43,42 @@ template <typename T> struct RegionStep {
     int B, H, W, C, extra, S, S2;
 };
 
+// The sums of NN rows, every lane a piece of each, in all lanes.  NARROW, rows of at most 32 vectors: in the order of the kernels
+// that give such a row to a group of 8, 16 or 32 lanes, the lane half a group away first (more than half a group away there is
+// nothing but zeros), so that both ways give the same bits.
+template <bool NARROW, int NN> __device__ __forceinline__ void row_sums(float (&v)[NN])
+{
+    if constexpr (!NARROW) {
+        wave_sum_n<NN>(v);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < NN; i++) {
+        const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i]), false, false);
+        v[i] = __uint_as_float(r16[0]) + __uint_as_float(r16[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < NN; i++) v[i] += dpp_move<0x128>(v[i]);                    // lane ^ 8
+#pragma unroll
+    for (int i = 0; i < NN; i++) v[i] += dpp_move<0x141>(dpp_move<0x1B>(v[i]));    // lane ^ 4
+#pragma unroll
+    for (int i = 0; i < NN; i++) v[i] += dpp_move<0x4E>(v[i]);                     // lane ^ 2
+#pragma unroll
+    for (int i = 0; i < NN; i++) v[i] += dpp_move<0xB1>(v[i]);                     // lane ^ 1
+#pragma unroll
+    for (int i = 0; i < NN; i++)
+        v[i] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[i]), 0));
+}
+template <bool NARROW> __device__ __forceinline__ float row_sum(float v)
+{
+    if constexpr (!NARROW) return wave_sum(v);
+    float one[1] = {v};
+    row_sums<NARROW, 1>(one);
+    return one[0];
+}
+
 // layernorm_kernel's arithmetic for one row held by a wave, a vector or several a lane
-template <typename T, int NV>
+template <typename T, int NV, bool NARROW>
 __device__ __forceinline__ void norm_row(const u32x4 (&row)[NV], const bool (&act)[NV], const u32x4 (&w)[NV],
                                          const u32x4 (&bb)[NV], float eps, int C, T *dst)
 {
@@ -58,7 +92,7 @@ __device__ __forceinline__ void norm_row(const u32x4 (&row)[NV], const bool (&ac
 #pragma unroll
             for (int c = 0; c < VEC; c++) s += vals[it][c];
         }
-    const float mean = wave_sum(s) / (float)C;
+    const float mean = row_sum<NARROW>(s) / (float)C;
 #pragma unroll
     for (int it = 0; it < NV; it++)
         if (act[it]) {
@@ -68,7 +102,7 @@ __device__ __forceinline__ void norm_row(const u32x4 (&row)[NV], const bool (&ac
                 q += dlt * dlt;
             }
         }
-    const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)C + eps);
+    const float rstd = 1.0f / sqrtf(row_sum<NARROW>(q) / (float)C + eps);
 #pragma unroll
     for (int it = 0; it < NV; it++)
         if (act[it]) {
@@ -85,7 +119,7 @@ __device__ __forceinline__ void norm_row(const u32x4 (&row)[NV], const bool (&ac
 // their quotients and roots are taken once, in four lanes side by side (the same operations on the same values).  With that,
 // the LayerNorm of a region that stays 16 queries taken over from its tokens, and registers for four waves a SIMD, a launch at
 // 2048 regions of 192 fp32 channels went from 39.9 to 36.3 us (119 MB), at 80 regions of 768 bf16 channels from 15.5 to 13.9.
-template <typename T, int NV>
+template <typename T, int NV, bool NARROW>
 __device__ __forceinline__ void norm_rows4(const u32x4 (&row)[4][NV], const bool (&act)[NV], const u32x4 (&w)[NV],
                                            const u32x4 (&bb)[NV], float eps, int C, T *dst, u32x4 (&y4)[4][NV])
 {
@@ -110,7 +144,7 @@ __device__ __forceinline__ void norm_rows4(const u32x4 (&row)[4][NV], const bool
                 for (int c = 0; c < VEC; c++) s[t] += vals[t][it][c];
             }
     }
-    wave_sum_n<4>(s);
+    row_sums<NARROW, 4>(s);
     per_row(s[0], s[1], s[2], s[3], [&](float v) { return v / (float)C; }, mean);
 #pragma unroll
     for (int t = 0; t < 4; t++) {
@@ -125,7 +159,7 @@ __device__ __forceinline__ void norm_rows4(const u32x4 (&row)[4][NV], const bool
                 }
             }
     }
-    wave_sum_n<4>(q);
+    row_sums<NARROW, 4>(q);
     per_row(q[0], q[1], q[2], q[3], [&](float v) { return 1.0f / sqrtf(v / (float)C + eps); }, rstd);
 #pragma unroll
     for (int t = 0; t < 4; t++)
@@ -157,10 +191,10 @@ __device__ __forceinline__ void record_row(const u32x4 &row, bool act, float eps
 
 }  // namespace
 
-template <typename T, int NV, bool REC>
+template <typename T, int NV, bool REC, bool NARROW>
 __global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_step_kernel(const RegionStep<T> a)
 {
-    static_assert(!REC || (NV == 1 && sizeof(T) == 2), "records: bf16 rows of one vector a lane");
+    static_assert(!REC || (NV == 1 && sizeof(T) == 2 && !NARROW), "records: bf16 rows of one vector a lane");
     constexpr int VEC = Elem<T>::VEC;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     u32x4 *const held = reinterpret_cast<u32x4 *>(smem);          // [16 tokens][vectors]
@@ -313,7 +347,7 @@ __global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_ste
             }
             const int64_t at = (int64_t)b * N + e;
             if constexpr (REC) record_row<T>(row[0], act[0], a.eps, C, a.records + at * 2);
-            else if (normed) norm_row<T, NV>(row, act, lw, lb, a.eps, C, a.out_ln + at * C + lane * VEC);
+            else if (normed) norm_row<T, NV, NARROW>(row, act, lw, lb, a.eps, C, a.out_ln + at * C + lane * VEC);
         }
     lds_barrier();
 
@@ -358,7 +392,7 @@ __global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_ste
         for (int s = 0; s < VTDGE_MAX_SPLITS; s++)
             if (s < a.S2) {
                 float logit =
-                    wave_sum(part[s]) + __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(rbias), s));
+                    row_sum<NARROW>(part[s]) + __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(rbias), s));
                 logit = Elem<T>::round(logit);
                 if (a.gate != nullptr && lane == 0) Elem<T>::store(a.gate + (int64_t)region * a.S2 + s, logit);
                 if (s == 0 || logit > best) {      // strict >: lowest index wins a tie
@@ -386,7 +420,7 @@ __global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_ste
         for (int t = 0; t < 4; t++) lane_sums<T>(tok[t][0], act[0], pivot[t], st[2 * t], st[2 * t + 1]);
         write_records4(st, pivot[0], pivot[1], pivot[2], pivot[3], C, a.eps, a.records + row0 * 2);
     } else if (normed) {
-        norm_rows4<T, NV>(tok, act, lw, lb, a.eps, C, a.out_ln + row0 * C + lane * VEC, y4);
+        norm_rows4<T, NV, NARROW>(tok, act, lw, lb, a.eps, C, a.out_ln + row0 * C + lane * VEC, y4);
     }
 
     // ---- the region's place among the next block's queries
@@ -424,7 +458,7 @@ __global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_ste
     };
     auto put = [&](const u32x4 (&row)[NV], int64_t r) {
         store(a.comp, row, r);
-        if (normed) norm_row<T, NV>(row, act, lw, lb, a.eps, C, a.comp_ln + r * C + lane * VEC);
+        if (normed) norm_row<T, NV, NARROW>(row, act, lw, lb, a.eps, C, a.comp_ln + r * C + lane * VEC);
     };
     if (ps_n == 4) {
         float pivot[4], st[8];
@@ -497,13 +531,15 @@ extern "C" int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int
     if (dtype != VTDGE_F32 && dtype != VTDGE_BF16) return 0;
     const int vec = dtype == VTDGE_BF16 ? 8 : 4, nvec = C / vec;
     const int64_t regions = (int64_t)B * (H / 4) * (W / 4);
-    if (C % vec != 0 || nvec <= 32 || nvec > 192) return 0;
+    if (C % vec != 0 || nvec > 192) return 0;
     // Up to where a wave for every four tokens is faster than one for sixteen that repeats nothing (the router's sums are
     // made from LDS again).  A forward, us, without it / with it (channels, regions): bf16 384: 256: 816 / 728, 512: 944 / 882,
     // 1024: 1348 / 1304, 1536: 1648 / 1628, 2048: 1874 / 1885, 4096: 3062 / 3258; 768: 512: 2204 / 2090, 1024: 3320 / 3286,
     // 1584: 4424 / 4426, 2560: 6495 / 6525; 320 (pyramid): 1024: 2320 / 2291, 2048: 3147 / 3170; fp32 192: 512: 1302 / 1196,
     // 1024: 1967 / 1900, 2048: 2964 / 2863; 384: 512: 2572 / 2509, 768: 3438 / 3452, 1600: 5715 / 5789; 768: 384: 5296 /
-    // 5280, 768: 8626 / 8675.
+    // 5280, 768: 8626 / 8675.  Narrow rows, whose other kernels give several regions to a wave, gain as long, most of a wave's
+    // lanes idle or not: bf16 192: 16: 543 / 435, 128: 749 / 630, 512: 996 / 848, 1024: 1182 / 1004, 1536: 1309 / 1195; pyramids of 64 to
+    // 512 channels by pictures of 256 px, bf16 2: 577 / 548, 16: 829 / 773, fp32 2: 745 / 720, 8: 1007 / 988.
     const int most = nvec <= WAVE ? (dtype == VTDGE_BF16 ? 1536 : 2048) : dtype == VTDGE_BF16 ? 1024 : 512;
     return regions <= most ? 1 : 0;
 }
@@ -534,8 +570,8 @@ extern "C" int vtdge_region_step(const void *in, const void *sub, const int64_t 
                    S2 <= VTDGE_MAX_SPLITS,
                VTDGE_ERR_UNSUPPORTED, "region_step: no kernel for %d samples of a %dx%d grid of %d channels (dtype %d)", B, H, W, C,
                dtype);
-    VT_REQUIRE(out_records == nullptr || (dtype == VTDGE_BF16 && C <= 512), VTDGE_ERR_UNSUPPORTED,
-               "region_step: statistics records are written for bf16 rows of up to 512 channels (C=%d)", C);
+    VT_REQUIRE(out_records == nullptr || (dtype == VTDGE_BF16 && C > 256 && C <= 512), VTDGE_ERR_UNSUPPORTED,
+               "region_step: statistics records are written for bf16 rows of 264 to 512 channels (C=%d)", C);
     VT_REQUIRE(capacity_rows >= (int64_t)B * (extra + (int64_t)H * W) && workspace_bytes >= vtdge_region_step_workspace(B, H, W),
                VTDGE_ERR_ARG, "region_step: buffers too small");
     VT_REQUIRE((((uintptr_t)in | (uintptr_t)sub | (uintptr_t)ref | (uintptr_t)out | (uintptr_t)next_weight | (uintptr_t)out_records |
@@ -544,8 +580,9 @@ extern "C" int vtdge_region_step(const void *in, const void *sub, const int64_t 
                VTDGE_ERR_ARG, "region_step: operands must be 16-byte aligned");
     const unsigned grid = (unsigned)(B * (H / 4) * (W / 4));
     const int vec = dtype == VTDGE_BF16 ? 8 : 4, nv = (C / vec + WAVE - 1) / WAVE;
+    const bool narrow = C / vec <= 32;
     const size_t lds = (size_t)16 * (C / vec) * 16;
-#define VT_GO(T, NV, REC)                                                                                                   \
+#define VT_GO(T, NV, REC, NARROW)                                                                                              \
     do {                                                                                                                    \
         const RegionStep<T> a{(const T *)in, (const T *)sub, (const T *)ref, cur_indices, splits, offsets, region_rows,     \
                               cur_counts, (T *)out, (const T *)next_weight, (const T *)next_bias, (T *)next_gate,           \
@@ -553,18 +590,20 @@ extern "C" int vtdge_region_step(const void *in, const void *sub, const int64_t 
                               (const T *)ln_weight, (const T *)ln_bias, eps, (T *)next_comp, (u32x4 *)next_comp_records,    \
                               (T *)next_comp_ln, next_patches, capacity_rows, next_offsets, next_region_rows,               \
                               (unsigned long long *)workspace, B, H, W, C, extra, S, S2};                                   \
-        note_kernel(reinterpret_cast<const void *>(region_step_kernel<T, NV, REC>));                                        \
-        region_step_kernel<T, NV, REC><<<grid, 256, lds, (hipStream_t)stream>>>(a);                                         \
+        note_kernel(reinterpret_cast<const void *>(region_step_kernel<T, NV, REC, NARROW>));                                        \
+        region_step_kernel<T, NV, REC, NARROW><<<grid, 256, lds, (hipStream_t)stream>>>(a);                                         \
         return check_launch("region_step");                                                                                 \
     } while (0)
     if (dtype == VTDGE_F32) {
-        if (nv == 1) VT_GO(float, 1, false);
-        if (nv == 2) VT_GO(float, 2, false);
-        VT_GO(float, 3, false);
+        if (narrow) VT_GO(float, 1, false, true);
+        if (nv == 1) VT_GO(float, 1, false, false);
+        if (nv == 2) VT_GO(float, 2, false, false);
+        VT_GO(float, 3, false, false);
     }
-    if (out_records != nullptr) VT_GO(bf16_t, 1, true);
-    if (nv == 1) VT_GO(bf16_t, 1, false);
-    if (nv == 2) VT_GO(bf16_t, 2, false);
-    VT_GO(bf16_t, 3, false);
+    if (out_records != nullptr) VT_GO(bf16_t, 1, true, false);
+    if (narrow) VT_GO(bf16_t, 1, false, true);
+    if (nv == 1) VT_GO(bf16_t, 1, false, false);
+    if (nv == 2) VT_GO(bf16_t, 2, false, false);
+    VT_GO(bf16_t, 3, false, false);
 #undef VT_GO
 }
