@@ -45,6 +45,29 @@ def test_few_pairs_many_tiles(dev):
     _check(dev, 2, 144, [1500], "two pairs of 47 tiles", _few(144))
 
 
+@pytest.mark.parametrize("n", [1, 33, 64, 257, 288])
+@pytest.mark.parametrize("h,most,lengths", [(41, 1300, [1300, 0, 257]), (40, 512, [511, 256, 1]), (150, 4000, [3000, 300])])
+def test_queries_dealt_out_in_chunks(dev, h, most, lengths, n):
+    """The resident kernel with a pair's queries in chunks, some of them empty, and in one piece (the same pairs among so many
+    that they fill the chip): a tile's arithmetic is the same, so the results are equal."""
+    from vtpack_amd import _C, _lib, ops
+    resident = f"sparse_attention_bf16_d64_pipelined_kernel<{-(-n // 32)}, "
+    lengths = torch.tensor(lengths, dtype=torch.int64)
+    L, B = int(lengths.sum()), len(lengths)
+    g = torch.Generator(dev).manual_seed(n)
+    q, k, v = (torch.randn(s, generator=g, device=dev).to(torch.bfloat16) for s in ((h, L, 64), (h, B, n, 64), (h, B, n, 64)))
+    off, _ = ops.lengths_to_offsets(lengths, q.device)
+    got = ops.sparse_attention_heads(q, k, v, off, 0.125, most)
+    assert resident + "true>" in _lib.last_kernel()
+    times = 1 + 512 // (h * B)
+    whole = _C.batched_sparse_attention_forward(q.repeat(times, 1, 1), k.repeat(times, 1, 1, 1), v.repeat(times, 1, 1, 1),
+                                                lengths, 0.125)
+    assert resident + "false>" in _lib.last_kernel()
+    assert torch.equal(got, whole.view(times, h, L, 64)[0]) and torch.equal(whole[-h:], whole[:h])
+    want = orc.attention(*(t[:2].float().cpu().numpy() for t in (q, k, v)), lengths.numpy(), 0.125)
+    assert_close(got[:2].float(), want, torch.bfloat16, f"{h} x {B} pairs of {n} keys in chunks")
+
+
 @pytest.mark.parametrize("n", [65, 145, 257, 401, 577])
 @pytest.mark.parametrize("size", [1.0, 4.0])
 def test_few_pairs_are_as_exact_as_many(dev, n, size):

@@ -4,7 +4,7 @@
 // restructured around what limits this operator at head_dim 64: the softmax's vector instructions (a wave issues
 // one every ~5 clocks, and there are about five per score against a quarter of an MFMA clock) and the K/V staging.
 //   * up to 288 keys (the 256 px models): K and V of a (sample, head) stay resident in LDS, double buffered across
-//     items by direct loads; V is transposed by the LDS read itself (ds_read_b64_tr_b16); the tile loop is a
+//     items - pairs, or chunks of their queries where the pairs alone leave the chip idle - by direct loads; V is transposed by the LDS read itself (ds_read_b64_tr_b16); the tile loop is a
 //     hand-ordered software pipeline in which the reference of the softmax rides in the MFMA accumulator;
 //   * longer sequences (512 px, spatially reduced PVT stages): K/V stages of 128 keys double buffered in LDS, K by
 //     direct loads, V through registers and transposed writes, online softmax in the log2 domain.
@@ -279,7 +279,7 @@ __device__ __forceinline__ void att_stage_fixed(const AttnTile &t, const int (&c
 
 // ---------------------------------------------------------------------------------------------------------
 // Short key sequences (n <= 288, e.g. 257 tokens at 256 px): one persistent workgroup of eight waves per compute
-// unit walks the (sample, head) items c, c + grid, c + 2 grid, ... with two buffers in LDS, each holding the item's K
+// unit walks the items - (sample, head) pairs, or chunks of their queries - c, c + grid, c + 2 grid, ... with two buffers in LDS, each holding the item's K
 // rows and V rows (128-byte rows, 16-byte chunks XOR-swizzled).  While the first four waves multiply item i out of
 // one buffer (a wave per 32-query tile; the other four join in for samples of more than 128 queries), the second
 // four bring item i+1 into the other buffer by direct loads; one barrier per item.  The staging of an item (its
@@ -287,12 +287,14 @@ __device__ __forceinline__ void att_stage_fixed(const AttnTile &t, const int (&c
 // Vector-memory operations retire in issue order: a wave asks for its first Q tile of the next item right after the
 // prefetch and nothing inside the tile arithmetic depends on either; only a sample with more than eight query
 // tiles (more than 256 queries) loads Q in between.
-// One instantiation per number of 32-key blocks (1 .. 9), so that the tile pipeline is fully unrolled.
-template <int NBLK>
+// One instantiation per number of 32-key blocks (1 .. 9), so that the tile pipeline is fully unrolled, and one for pairs in
+// chunks: with its loop, which asks for the next tile ahead, whole pairs of few tiles are slower (256 samples, 6 heads, 257
+// keys: 41.8 against 39.2 us; 1024 rows and more a sample gain nothing).
+template <int NBLK, bool CHUNKED>
 __global__ __launch_bounds__(512, 1) void sparse_attention_bf16_d64_pipelined_kernel(
     const bf16_t *__restrict__ q, int64_t q_rs, int64_t q_hs, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets,
-    bf16_t *__restrict__ out, int64_t o_rs, int64_t o_hs, int n, float scale, int items, int h)
+    bf16_t *__restrict__ out, int64_t o_rs, int64_t o_hs, int n, float scale, int items, int h, int chunks)
 {
     constexpr int NW = 8;                   // waves
     constexpr int npad = NBLK * 32;         // the host picks the instantiation: NBLK = ceil(n / 32)
@@ -305,14 +307,16 @@ __global__ __launch_bounds__(512, 1) void sparse_attention_bf16_d64_pipelined_ke
     const int64_t row_bytes = kv_ts * 2;
     const float c = scale * 1.44269504088896340736f;
 
-    // Items of this workgroup: blockIdx.x + li * gridDim.x, li = 0, 1, ...; item -> (sample, head) with the heads of a
-    // sample as neighbours, so the pieces of one token row are fetched by workgroups that run at the same time.
+    // Items of this workgroup: blockIdx.x + li * gridDim.x, li = 0, 1, ...; item -> (sample, chunk, head) with the heads of a
+    // sample as neighbours, so the pieces of one token row are fetched by workgroups that run at the same time.  Chunk c of
+    // a pair has its tiles 8 c .. 8 c + 7 (one for each wave), 8 (c + chunks) .. and so on.
     // First row and query count of every item are put into a small LDS table up front (up to ATT_TBL items per
     // workgroup; beyond that they are read from `offsets` when needed), so that no step of the loop waits for them.
     struct Item {
         int64_t row0;
-        int Lb, b, head;
+        int Lb, b, head, tile;      // tile: this wave's first
     };
+    const int per_sample = CHUNKED ? h * chunks : h, tile_step = CHUNKED ? NW * chunks : NW;
     int64_t *t_row0 = reinterpret_cast<int64_t *>(smem + 2 * bufsz);
     int *t_len = reinterpret_cast<int *>(t_row0 + ATT_TBL);
     const int grid = gridDim.x;
@@ -321,7 +325,7 @@ __global__ __launch_bounds__(512, 1) void sparse_attention_bf16_d64_pipelined_ke
     const bool tabled = my_items <= ATT_TBL;
     if (tabled) {
         for (int li = tid; li < my_items; li += 512) {
-            const int b = ((int)blockIdx.x + li * grid) / h;
+            const int b = ((int)blockIdx.x + li * grid) / per_sample;
             const int64_t r0 = offsets[b];
             t_row0[li] = r0;
             t_len[li] = (int)(offsets[b + 1] - r0);
@@ -330,8 +334,10 @@ __global__ __launch_bounds__(512, 1) void sparse_attention_bf16_d64_pipelined_ke
     auto item_of = [&](int li, bool from_table) {
         Item r;
         const int it = (int)blockIdx.x + li * grid;
-        r.b = it / h;
-        r.head = it - r.b * h;
+        r.b = it / per_sample;
+        const int of_sample = it - r.b * per_sample, chunk = CHUNKED ? of_sample / h : 0;
+        r.head = of_sample - chunk * h;
+        r.tile = chunk * NW + wid;
         if (from_table) {
             const int64_t r0 = t_row0[li];
             r.row0 = ((int64_t)__builtin_amdgcn_readfirstlane((int)(r0 >> 32)) << 32) |
@@ -397,7 +403,7 @@ __global__ __launch_bounds__(512, 1) void sparse_attention_bf16_d64_pipelined_ke
     Item cur = item_of(0, false);
     stage_issue(cur, smem, wid, NW);
     u32x4 qf[4], qn[4];
-    load_q(cur, wid, qf);
+    load_q(cur, cur.tile, qf);
     wait_vmcnt<0>();
     __syncthreads();
     Item nxt = cur;
@@ -406,26 +412,39 @@ __global__ __launch_bounds__(512, 1) void sparse_attention_bf16_d64_pipelined_ke
     for (int li = 0, par = 0; li < my_items; li++, par ^= 1) {
         unsigned char *buf = smem + par * bufsz;
         const bool has_next = li + 1 < my_items;
-        // The second half of the waves has a tile only in samples of more than 128 queries: it issues the prefetch
-        // of the next item, the first half goes straight to its tiles.  Every wave then asks for its first Q tile of
-        // the next item; nothing in the tile arithmetic depends on these loads.
-        if (has_next) {
-            if (wid >= NW / 2) stage_issue(nxt, smem + (par ^ 1) * bufsz, wid - NW / 2, NW / 2);
-            load_q(nxt, wid, qn);
-        }
+        // The second half of the waves has a tile only where there are more than 128 queries: it issues the prefetch of the
+        // next item, the first half goes straight to its tiles.  Every wave then asks for its next Q tile, of this item (CHUNKED) or
+        // the next; nothing in the tile arithmetic depends on these loads.
+        if (has_next && wid >= NW / 2) stage_issue(nxt, smem + (par ^ 1) * bufsz, wid - NW / 2, NW / 2);
+        if (!CHUNKED && has_next) load_q(nxt, nxt.tile, qn);
         const AttnTile tile = {buf + lr * 128, att_v_lane(buf + npad * 128, lane), nullptr, n, lg};
-        for (int rt = wid; rt * 32 < cur.Lb; rt += NW) {
+        auto take = [&](int rt) {
             const int qrow = rt * 32 + lr;
-            if (rt != wid) {        // a ninth tile and beyond (more than 256 queries): waits behind the prefetch
-                load_q(cur, rt, qf);
-                wait_vmcnt<0>();    // here, so that the common path carries no pending load into the arithmetic
-            }
             f32x16 o[2];
             float l_run;
             scale_q(qf);
             att_tile_fixed<NBLK>(tile, cs, qf, o, l_run);
             const float l_tot = l_run + __shfl_xor(l_run, 32, WAVE);
             if (qrow < cur.Lb) attn_store(out + (cur.row0 + qrow) * o_rs + (int64_t)cur.head * o_hs, o, l_tot, lg);
+        };
+        if constexpr (CHUNKED) {
+            for (int rt = cur.tile;; rt += tile_step) {
+                const bool more = (rt + tile_step) * 32 < cur.Lb;
+                if (more) load_q(cur, rt + tile_step, qn);
+                else if (has_next) load_q(nxt, nxt.tile, qn);
+                if (rt * 32 < cur.Lb) take(rt);
+                if (!more) break;
+#pragma unroll
+                for (int s = 0; s < 4; s++) qf[s] = qn[s];
+            }
+        } else {
+            for (int rt = wid; rt * 32 < cur.Lb; rt += NW) {
+                if (rt != wid) {        // a ninth tile and beyond (more than 256 queries): waits behind the prefetch
+                    load_q(cur, rt, qf);
+                    wait_vmcnt<0>();    // here, so that the common path carries no pending load into the arithmetic
+                }
+                take(rt);
+            }
         }
         cur = nxt;
         if (li + 2 < my_items) nxt = item_of(li + 2, tabled);
@@ -587,6 +606,29 @@ int launch_attention_split(const void *q, int64_t q_rs, int64_t q_hs, const void
                            int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs, int64_t o_hs, int B,
                            int h, int n, int max_rows, float scale, hipStream_t st);
 
+// Chunks that the resident kernel deals a pair's queries out in.  What a compute unit goes through, in tiles of a wave: its
+// items, each of them a share of the tiles (a third of what max_rows allows, as routed samples have) and one for bringing keys
+// and values in; a pair stays whole unless that says a tenth less, and where it has no sixteen tiles.  Us, whole / dealt out
+// (pairs, keys, rows a sample may have, has on average): 8, 256, 16384, 6000: 117.1 / 10.6; 24: 127.3 / 25.0; 140: 133.4 / 98.1;
+// 48, 256, 4096, 1500: 35.8 / 15.9; 120, 256, 1024, 400: 14.1 / 11.2; 12, 64, 4096, 1500: 21.0 / 6.9; 100: 26.7 / 17.5; 300:
+// 50.4 / 43.2.  Kept whole, whole / two chunks: 256, 64, 4096, 1500: 30.7 / 32.1; 512, 64, 1024, 380: 19.6 / 23.9; 300, 257, 257,
+// 110: 14.4 / 17.4.
+static int resident_chunks(int pairs, int max_rows, int cus)
+{
+    const int most = max_rows / 256;
+    const float tiles = (float)max_rows / (3.f * 256.f);
+    int best = 1;
+    float least = 0.9f * (float)ceil_div(pairs, cus) * (tiles + 1.f);
+    for (int c = 2; c <= most && c <= 2 + 2 * cus / pairs; c++) {
+        const float cost = (float)ceil_div((int64_t)pairs * c, cus) * (tiles / (float)c + 1.f);
+        if (cost < least) {
+            least = cost;
+            best = c;
+        }
+    }
+    return best;
+}
+
 int launch_attention_bf16_d64(const void *q, int64_t q_rs, int64_t q_hs, const void *k, const void *v, int64_t kv_bs,
                               int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs,
                               int64_t o_hs, int B, int h, int n, int max_rows, float scale, hipStream_t st)
@@ -598,17 +640,18 @@ int launch_attention_bf16_d64(const void *q, int64_t q_rs, int64_t q_hs, const v
         // keys and values resident in LDS: one persistent workgroup per compute unit, two buffers of K rows + V rows
         const int npad = (n + 31) & ~31;
         const size_t lds_p = 4 * (size_t)npad * 128 + ATT_TBL * 12;       // + the item table
-        const int items = B * h;
         const int cus = compute_units();
+        const int chunks = resident_chunks(B * h, max_rows, cus), items = B * h * chunks;
         dim3 grid_p((unsigned)(items < cus ? items : cus)), block_p(512);
 #define VT_ATT_PIPE(NB)                                                                                            \
     case NB: {                                                                                                     \
-        auto kern_p = sparse_attention_bf16_d64_pipelined_kernel<NB>;                                              \
+        auto kern_p = chunks > 1 ? sparse_attention_bf16_d64_pipelined_kernel<NB, true>                            \
+                                 : sparse_attention_bf16_d64_pipelined_kernel<NB, false>;                          \
         VT_RESERVE_LDS(kern_p, 160 * 1024, "sparse_attention");                                                    \
         note_kernel(reinterpret_cast<const void *>(kern_p)),                                                        \
         kern_p<<<grid_p, block_p, lds_p, st>>>((const bf16_t *)q, q_rs, q_hs, (const bf16_t *)k, (const bf16_t *)v, \
                                                kv_bs, kv_ts, kv_hs, offsets, (bf16_t *)out, o_rs, o_hs, n, scale,  \
-                                               items, h);                                                          \
+                                               items, h, chunks);                                                          \
         return check_launch("sparse_attention");                                                                   \
     }
         switch (npad / 32) {
