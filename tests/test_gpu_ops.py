@@ -52,6 +52,19 @@ def test_index_to_patch_bit_exact(dev, B, Hr, Wr, extra, splits):
     assert np.array_equal(got_p.cpu().numpy(), want_p)
 
 
+@pytest.mark.parametrize("R,splits", [(4, [4, 2, 1]), (8, [8, 1, 2, 4])])
+@pytest.mark.parametrize("B,Hr,Wr,extra", [(1, 15, 17, 0), (1, 16, 16, 300), (3, 1, 257, 1), (5, 32, 32, 2), (40, 23, 23, 1), (4097, 3, 3, 1)])
+def test_index_to_patch_over_several_workgroups(dev, B, Hr, Wr, extra, R, splits):
+    """Samples of a workgroup's 256 regions, one less and more, several workgroups; one launch, counts first, a scan first."""
+    from vtpack_amd import ops
+    idx = random_indices(B + Wr, B, Hr, Wr, len(splits))
+    want_p, want_l = orc.index_to_patch(idx, splits, R, extra)
+    got_p, off, got_l = ops.index_to_patch(_t(idx, dev), _t(np.array(splits, dtype=np.int64), dev), R, extra)
+    np.testing.assert_array_equal(got_l.cpu().numpy(), want_l)
+    np.testing.assert_array_equal(off.cpu().numpy(), np.concatenate([[0], np.cumsum(want_l)]))
+    np.testing.assert_array_equal(got_p.cpu().numpy()[:len(want_p)], want_p)
+
+
 def test_index_to_patch_uniform_gates(dev):
     from vtpack_amd import _C
     sp = _t(np.array(SPLITS, dtype=np.int64), dev)

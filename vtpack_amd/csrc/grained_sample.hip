@@ -313,153 +313,134 @@ __global__ __launch_bounds__(256) void patch_count_kernel(const int64_t *__restr
     if (lane == 0) lengths[b] = (int64_t)part + extra;
 }
 
-// Step 2: one workgroup per sample.  The per-region query counts go through an
-// LDS-staged wavefront prefix sum (256 regions per pass); then every thread emits
-// one descriptor per turn (row j of the sample: its region by binary search in the
-// prefix sums), so a workgroup writes 256 consecutive 32-byte rows at a time.
+// Step 2: a workgroup per 256 regions of a sample.  Their query counts go through a wavefront prefix sum, and sixteen threads
+// write the descriptors of a region (32 bytes each, consecutive), sixteen regions a turn.  What bounds it is latency.  Us, with one
+// workgroup per sample and the region of every row searched for in the prefix sums (eight dependent reads of LDS) / so (samples,
+// regions of each): 6, 576: 18.3 / 9.4; 8, 1024: 31.0 / 11.4; 64, 256: 17.9 / 15.0; 64, 16: 4.7 / 4.5; 256, 16: 5.4 / 5.2; 1024,
+// 16: 15.3 / 13.6; 5000, 16 (after a scan): 54.9 / 56.5.
 //
-// FUSED: the workgroup also finds its own first row, as the sum of the query counts of all samples before it (it
+// FUSED: the workgroup also finds its own first row, as the sum of the query counts of all regions before it (it
 // reads their gate indices itself: a few KB out of L2 for the batch sizes this variant is launched for), and writes
 // offsets / lengths; no first step then, and no dependency between workgroups.
-// Not FUSED: the first row comes from `offsets` (written by the scan kernel) or, with from_lengths, is the sum of
+// Not FUSED: the sample's first row comes from `offsets` (written by the scan kernel) or, with from_lengths, is the sum of
 // the lengths of the samples before this one (written by the count kernel), in which case the workgroup writes
-// offsets as well.
+// offsets as well; only its own sample's regions before it are added up.
 typedef long long i64x2 __attribute__((ext_vector_type(2)));
 
 template <bool FUSED>
 __global__ __launch_bounds__(256) void patch_write_kernel(const int64_t *__restrict__ indices,
                                                            const int64_t *__restrict__ splits,
                                                            int64_t *__restrict__ offsets, int64_t *__restrict__ lengths,
-                                                           int Hr, int Wr, int S, int R, int extra,
+                                                           int B, int Hr, int Wr, int S, int R, int extra,
                                                            int64_t *__restrict__ patches, int64_t capacity,
                                                            int from_lengths)
 {
     __shared__ int wave_tot[4];
-    __shared__ int carry_s;
     __shared__ int split_s[VTDGE_MAX_SPLITS];
-    __shared__ int64_t before_s[4];
+    __shared__ int64_t before_s[2][4];
     __shared__ int start_s[256], ps_s[256];
-    const int b = blockIdx.x;
+    const int nreg = Hr * Wr, chunks = (nreg + 255) / 256;
+    const int b = blockIdx.x / chunks, base = (blockIdx.x - b * chunks) * 256, nr = min(256, nreg - base);
+    const bool last_chunk = base + 256 >= nreg;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int nreg = Hr * Wr;
-    // everything the workgroup reads is requested before anything is used: the splits, the first gate indices of
-    // its own sample and (FUSED) sixteen per thread of the samples before it - one trip to memory instead of three
+    // everything the workgroup reads is requested before anything is used: the splits, the gate indices of
+    // its own regions and (FUSED) sixteen per thread of those before them - one trip to memory instead of three
     const int sp = threadIdx.x < S ? (int)splits[threadIdx.x] : 1;
-    int64_t g_first = 0;
-    if (threadIdx.x < nreg) g_first = indices[(int64_t)b * nreg + threadIdx.x];
-    constexpr int PRE = 16;
-    const int64_t nbefore = FUSED ? (int64_t)b * nreg : 0;
+    int64_t g_own = 0;
+    if (threadIdx.x < nr) g_own = indices[(int64_t)b * nreg + base + threadIdx.x];
+    constexpr int PRE = FUSED ? 16 : 1;
+    const int64_t sample0 = (int64_t)b * nreg, own0 = sample0 + base;
+    const int64_t *const from = FUSED ? indices : indices + sample0;
+    const int64_t nbefore = FUSED ? own0 : base;
     int64_t gq[PRE];
-    if constexpr (FUSED) {
 #pragma unroll
-        for (int i = 0; i < PRE; i++) {
-            const int64_t idx = threadIdx.x + 256 * (int64_t)i;
-            gq[i] = idx < nbefore ? indices[idx] : 0;
-        }
+    for (int i = 0; i < PRE; i++) {
+        const int64_t idx = threadIdx.x + 256 * (int64_t)i;
+        gq[i] = idx < nbefore ? from[idx] : 0;
     }
     if (threadIdx.x < VTDGE_MAX_SPLITS) split_s[threadIdx.x] = sp;
-    if (threadIdx.x == 0) carry_s = 0;
     __syncthreads();
-    int64_t row0;
-    if constexpr (FUSED) {
-        int64_t part = 0;
+    auto split_of = [&](int64_t g) { return split_s[g < 0 ? 0 : (g >= S ? S - 1 : g)]; };
+
+    // rows before the sample, and rows of its regions before these
+    int64_t sample_part = 0, own_part = 0;
+    auto count = [&](int64_t idx, int64_t g) {
+        const int ps = split_of(g), rows = ps * ps, own = !FUSED || idx >= sample0 ? rows : 0;
+        own_part += own;
+        sample_part += rows - own;
+    };
 #pragma unroll
-        for (int i = 0; i < PRE; i++) {
-            if (threadIdx.x + 256 * (int64_t)i < nbefore) {
-                const int64_t g = gq[i] < 0 ? 0 : (gq[i] >= S ? S - 1 : gq[i]);
-                const int ps = split_s[g];
-                part += ps * ps;
-            }
-        }
-        for (int64_t i = threadIdx.x + 256 * (int64_t)PRE; i < nbefore; i += 256) {
-            int64_t g = indices[i];
-            g = g < 0 ? 0 : (g >= S ? S - 1 : g);
-            const int ps = split_s[g];
-            part += ps * ps;
-        }
+    for (int i = 0; i < PRE; i++)
+        if (threadIdx.x + 256 * i < nbefore) count(threadIdx.x + 256 * i, gq[i]);
+    for (int64_t at = threadIdx.x + 256 * PRE; at < nbefore; at += 256 * 8) {
+        int64_t g[8];
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, WAVE);
-        if (lane == 0) before_s[wid] = part;
-        __syncthreads();
-        row0 = before_s[0] + before_s[1] + before_s[2] + before_s[3] + (int64_t)b * extra;
-        if (threadIdx.x == 0) offsets[b] = row0;
-    } else if (from_lengths) {
-        int64_t part = 0;
-        for (int i = threadIdx.x; i < b; i += 256) part += lengths[i];
+        for (int i = 0; i < 8; i++) g[i] = at + 256 * i < nbefore ? from[at + 256 * i] : 0;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, WAVE);
-        if (lane == 0) before_s[wid] = part;
-        __syncthreads();
-        row0 = before_s[0] + before_s[1] + before_s[2] + before_s[3];
-        if (threadIdx.x == 0) {
+        for (int i = 0; i < 8; i++)
+            if (at + 256 * i < nbefore) count(at + 256 * i, g[i]);
+    }
+    if (!FUSED && from_lengths)
+        for (int i = threadIdx.x; i < b; i += 256) sample_part += lengths[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        sample_part += __shfl_xor(sample_part, o, WAVE);
+        if (chunks > 1) own_part += __shfl_xor(own_part, o, WAVE);
+    }
+    const int ps = threadIdx.x < nr ? split_of(g_own) : 0;
+    const int cnt = ps * ps;
+    int inc = cnt;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+        int up = __shfl_up(inc, o, WAVE);
+        if (lane >= o) inc += up;
+    }
+    if (lane == 63) wave_tot[wid] = inc;
+    if (lane == 0) {
+        before_s[0][wid] = sample_part;
+        before_s[1][wid] = own_part;
+    }
+    __syncthreads();
+    int first = inc - cnt;
+    for (int w = 0; w < wid; w++) first += wave_tot[w];
+    start_s[threadIdx.x] = first;                  // first row of the region, of those of the workgroup
+    ps_s[threadIdx.x] = ps;
+    int64_t row0 = before_s[0][0] + before_s[0][1] + before_s[0][2] + before_s[0][3];
+    const int64_t in_sample = before_s[1][0] + before_s[1][1] + before_s[1][2] + before_s[1][3];
+    if constexpr (FUSED) row0 += (int64_t)b * extra;
+    else if (!from_lengths) row0 = offsets[b];
+    if (threadIdx.x == 0 && last_chunk) {
+        const int64_t len = extra + in_sample + wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
+        if constexpr (FUSED) lengths[b] = len;
+        if (FUSED || from_lengths) {
             offsets[b] = row0;
-            if (b == (int)gridDim.x - 1) offsets[b + 1] = row0 + lengths[b];
-        }
-    } else {
-        row0 = offsets[b];
-    }
-    for (int e = threadIdx.x; e < extra; e += 256) {
-        const int64_t row = row0 + e;
-        if (row < capacity) {
-            int64_t *p = patches + 4 * row;
-            p[0] = b; p[1] = -(int64_t)e - 1; p[2] = 0; p[3] = 1;
+            if (b == B - 1) offsets[B] = row0 + len;
         }
     }
-    for (int base = 0; base < nreg; base += 256) {
-        const int r = base + threadIdx.x;
-        int ps = 0;
-        if (r < nreg) {
-            int64_t g = base == 0 ? g_first : indices[(int64_t)b * nreg + r];
-            g = g < 0 ? 0 : (g >= S ? S - 1 : g);
-            ps = split_s[g];
-        }
-        const int cnt = ps * ps;
-        int inc = cnt;
-#pragma unroll
-        for (int o = 1; o < WAVE; o <<= 1) {
-            int up = __shfl_up(inc, o, WAVE);
-            if (lane >= o) inc += up;
-        }
-        if (lane == 63) wave_tot[wid] = inc;
-        __syncthreads();
-        const int first = carry_s;                 // rows of the regions of earlier passes
-        int before = first;
-        for (int w = 0; w < wid; w++) before += wave_tot[w];
-        // first row of the region (or, past the last region, one past the last row of the pass) and its split
-        start_s[threadIdx.x] = before + inc - cnt;
-        ps_s[threadIdx.x] = ps;
-        __syncthreads();
-        const int nr = min(256, nreg - base);
-        const int last = start_s[nr - 1] + ps_s[nr - 1] * ps_s[nr - 1];
-        // one descriptor per thread and turn: the region of row j is the last one that starts at or before j
-        for (int j = first + threadIdx.x; j < last; j += 256) {
-            int lo = 0, hi = nr - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (start_s[mid] <= j) lo = mid;
-                else hi = mid - 1;
-            }
-            const int rps = ps_s[lo], local = j - start_s[lo];
-            const int rg = base + lo, ry = rg / Wr, rx = rg % Wr;
-            const int step = R / rps, dy = local / rps, dx = local - dy * rps;
-            const int64_t row = row0 + extra + j;
+    if (base == 0)
+        for (int e = threadIdx.x; e < extra; e += 256) {
+            const int64_t row = row0 + e;
             if (row < capacity) {
-                i64x2 *p = reinterpret_cast<i64x2 *>(patches + 4 * row);
+                int64_t *p = patches + 4 * row;
+                p[0] = b; p[1] = -(int64_t)e - 1; p[2] = 0; p[3] = 1;
+            }
+        }
+    __syncthreads();
+    row0 += extra + in_sample;
+    for (int r = threadIdx.x >> 4; r < nr; r += 16) {
+        const int rps = ps_s[r], rows = rps * rps;
+        if ((threadIdx.x & 15) >= rows) continue;
+        const int rg = base + r, ry = rg / Wr, rx = rg - ry * Wr, step = R / rps;
+        const int64_t at = row0 + start_s[r];
+        for (int j = threadIdx.x & 15; j < rows; j += 16) {
+            const int dy = j / rps, dx = j - dy * rps;
+            if (at + j < capacity) {
+                i64x2 *p = reinterpret_cast<i64x2 *>(patches + 4 * (at + j));
                 const i64x2 lo2 = {(int64_t)b, (int64_t)ry * R + dy * step};
                 const i64x2 hi2 = {(int64_t)rx * R + dx * step, (int64_t)step};
                 p[0] = lo2;
                 p[1] = hi2;
             }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) carry_s = last;
-        __syncthreads();
-    }
-    if constexpr (FUSED) {
-        if (threadIdx.x == 0) {
-            const int64_t len = (int64_t)extra + carry_s;
-            lengths[b] = len;
-            if (b == (int)gridDim.x - 1) offsets[b + 1] = row0 + len;
         }
     }
 }
@@ -1615,10 +1596,11 @@ extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *split
     VT_REQUIRE((reinterpret_cast<uintptr_t>(patches) & 15u) == 0, VTDGE_ERR_ARG,
                "index_to_patch: patches must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
+    const unsigned chunks = (unsigned)ceil_div((int64_t)Hr * Wr, 256);
     if (patches != nullptr && (int64_t)B * Hr * Wr <= ONE_LAUNCH_REGIONS) {
         // small batches: one launch, every sample's workgroup sums the counts before it on its own
         note_kernel(reinterpret_cast<const void *>(patch_write_kernel<true>));
-        patch_write_kernel<true><<<B, 256, 0, st>>>(indices, splits, offsets, lengths, Hr, Wr, S, R, extra, patches,
+        patch_write_kernel<true><<<B * chunks, 256, 0, st>>>(indices, splits, offsets, lengths, B, Hr, Wr, S, R, extra, patches,
                                                     capacity_rows, 0);
         return check_launch("index_to_patch");
     }
@@ -1628,7 +1610,7 @@ extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *split
         patch_count_kernel<<<(B + 3) / 4, 256, 0, st>>>(indices, splits, B, Hr * Wr, S, extra, lengths);
         if (int rc = check_launch("index_to_patch(count)")) return rc;
         note_kernel(reinterpret_cast<const void *>(patch_write_kernel<false>));
-        patch_write_kernel<false><<<B, 256, 0, st>>>(indices, splits, offsets, lengths, Hr, Wr, S, R, extra, patches,
+        patch_write_kernel<false><<<B * chunks, 256, 0, st>>>(indices, splits, offsets, lengths, B, Hr, Wr, S, R, extra, patches,
                                                      capacity_rows, 1);
         return check_launch("index_to_patch(write)");
     }
@@ -1637,7 +1619,7 @@ extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *split
     if (int rc = check_launch("index_to_patch(count+scan)")) return rc;
     if (patches != nullptr) {
         note_kernel(reinterpret_cast<const void *>(patch_write_kernel<false>));
-        patch_write_kernel<false><<<B, 256, 0, st>>>(indices, splits, offsets, lengths, Hr, Wr, S, R, extra, patches,
+        patch_write_kernel<false><<<B * chunks, 256, 0, st>>>(indices, splits, offsets, lengths, B, Hr, Wr, S, R, extra, patches,
                                                      capacity_rows, 0);
         return check_launch("index_to_patch(write)");
     }
