@@ -299,6 +299,10 @@ int vtdge_patch_embed_norm(const void *images, const void *weight, const void *b
 int vtdge_layernorm_add(const void *x, const void *weight, const void *bias, const void *add, int64_t add_rows,
                         void *out, int64_t rows, int C, float eps, int dtype, void *stream);
 
+/* Token rows x [B, tokens, C] (rows dense, samples batch_stride elements apart) as feature maps out [B, C, tokens], dense: the
+ * permute(0, 3, 1, 2).contiguous() of vtpack/models/dge/pvt_dge.py's stage outputs. */
+int vtdge_rows_to_maps(const void *x, int64_t batch_stride, void *out, int B, int tokens, int C, int dtype, void *stream);
+
 /* Row-wise LayerNorm over the last dimension (biased variance, fp32 statistics).
  * Stands in for nn.LayerNorm(eps=1e-6) at vtpack/models/dge/deit_dge.py:127-128. */
 int vtdge_layernorm(const void *x, const void *weight, const void *bias, void *out, const int64_t *rows_dev,

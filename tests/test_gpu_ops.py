@@ -1060,3 +1060,16 @@ def test_query_counts_on_the_host(dev, B, Hr, Wr):
         t.join()
     assert not bad
     assert ops.index_to_patch_host(_t(idx, dev), sp, 4, 1)[2] == int(want[1].sum())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,H,W,C,extra,off", [(1, 1, 1, 1, 0, 0), (2, 8, 8, 64, 0, 0), (3, 7, 9, 65, 1, 0), (2, 12, 12, 512, 1, 0),
+                                               (2, 5, 13, 72, 0, 0), (4, 8, 16, 128, 0, 1), (1, 65, 1, 63, 2, 0)])
+def test_rows_to_maps(dev, B, H, W, C, extra, off, dtype):
+    """Whole and partial tiles, rows and maps on 16-byte boundaries and off them, samples apart: the same bits."""
+    from vtpack_amd import ops
+    store = torch.randint(-(1 << 15), 1 << 15, ((off + B * (extra + H * W) * C) * dtype.itemsize // 2,), dtype=torch.int16, device=dev)
+    x = store.view(dtype)[off:].view(B, extra + H * W, C)[:, extra:].view(B, H, W, C)
+    got, want = ops.rows_to_maps(x), x.permute(0, 3, 1, 2).contiguous()
+    assert got.shape == want.shape and got.is_contiguous()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))

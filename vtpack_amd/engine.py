@@ -819,6 +819,6 @@ def pvt_forward(model, images):
         elif model.num_classes == 0:
             outputs[f"res{i + 2}"] = x[:, 1:].reshape(B, H, W, C)
     if model.num_classes == 0:
-        return {name: t.permute(0, 3, 1, 2).contiguous() for name, t in outputs.items()}
+        return {name: ops.rows_to_maps(t) for name, t in outputs.items()}
     cls = ops.layernorm(x[:, 0, :], model.norm.weight, model.norm.bias, model.norm.eps)
     return ops.linear(cls, model.head.weight, model.head.bias)

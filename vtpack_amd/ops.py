@@ -512,6 +512,20 @@ def layernorm(x, weight, bias, eps=1e-6, rows_dev=None, out=None, add=None):
     return out
 
 
+def rows_to_maps(x):
+    """Tokens x [B, H, W, C] (rows dense, samples any distance apart) as feature maps [B, C, H, W]:
+    x.permute(0, 3, 1, 2).contiguous()."""
+    _need_gpu(x)
+    B, H, W, C = x.shape
+    if B and (not x[0].is_contiguous() or B > 1 and x.stride(0) < H * W * C):
+        x = x.contiguous()
+    out = torch.empty((B, C, H, W), dtype=x.dtype, device=x.device)
+    if out.numel():
+        call("vtdge_rows_to_maps", ptr(x), max(x.stride(0), H * W * C), ptr(out), B, H * W, C, dtype_code(x), stream_ptr(),
+             tag=("rows_to_maps", B * H * W, C))
+    return out
+
+
 def layernorm_front_rows(x, count, weight, bias, eps=1e-6):
     """LayerNorm of the first `count` rows of every sample of x [B, N, C] -> [B, count, C], read in place (no copy of
     the slice): the model's final norm on the class-token rows only."""
