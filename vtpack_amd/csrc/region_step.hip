@@ -537,10 +537,12 @@ extern "C" int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int
     // 1024: 1348 / 1304, 1536: 1648 / 1628, 2048: 1874 / 1885, 4096: 3062 / 3258; 768: 512: 2204 / 2090, 1024: 3320 / 3286,
     // 1584: 4424 / 4426, 2560: 6495 / 6525; 320 (pyramid): 1024: 2320 / 2291, 2048: 3147 / 3170; fp32 192: 512: 1302 / 1196,
     // 1024: 1967 / 1900, 2048: 2964 / 2863; 384: 512: 2572 / 2509, 768: 3438 / 3452, 1600: 5715 / 5789; 768: 384: 5296 /
-    // 5280, 768: 8626 / 8675.  Narrow rows, whose other kernels give several regions to a wave, gain as long, most of a wave's
-    // lanes idle or not: bf16 192: 16: 543 / 435, 128: 749 / 630, 512: 996 / 848, 1024: 1182 / 1004, 1536: 1309 / 1195; pyramids of 64 to
-    // 512 channels by pictures of 256 px, bf16 2: 577 / 548, 16: 829 / 773, fp32 2: 745 / 720, 8: 1007 / 988.
-    const int most = nvec <= WAVE ? (dtype == VTDGE_BF16 ? 1536 : 2048) : dtype == VTDGE_BF16 ? 1024 : 512;
+    // 5280, 768: 8626 / 8675.  Narrow rows, whose other kernels give several regions to a wave, gain longer, most of a wave's
+    // lanes idle or not: bf16 192: 16: 541 / 437, 128: 751 / 629, 512: 997 / 847, 1536: 1311 / 1202, 2048: 1393 / 1296, 2560: 1507 /
+    // 1415, 3072: 1712 / 1641, 4096: 2021 / 2024; pyramids of 64 to 512 channels by pictures of 256 px, bf16 2: 582 / 549, 16: 796 /
+    // 755, 48: 1024 / 994; fp32 8: 1004 / 980, with 2304 regions of 64 and 576 of 128 channels 1026 / 1028, 4096 and 1024:
+    // 1184 / 1207.
+    const int most = dtype == VTDGE_BF16 ? (nvec <= 32 ? 3072 : nvec <= WAVE ? 1536 : 1024) : nvec <= WAVE ? 2048 : 512;
     return regions <= most ? 1 : 0;
 }
 
