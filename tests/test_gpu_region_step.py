@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
     (2, 6, 4, 320, 0, "f32", "norm"), (3, 4, 4, 768, 64, "f32", "norm"), (2, 4, 4, 8, 0, "bf16", "norm"),
     (1, 16, 16, 64, 0, "bf16", "norm"), (3, 4, 4, 64, 1, "f32", "norm"), (96, 4, 4, 192, 1, "bf16", "norm"),
     (2, 3, 5, 12, 0, "f32", "plain"), (5, 8, 8, 128, 0, "bf16", "plain"), (2, 4, 4, 256, 1, "bf16", "norm"),
-    (192, 4, 4, 192, 1, "bf16", "norm"), (12, 16, 16, 64, 0, "bf16", "norm")])
+    (192, 4, 4, 192, 1, "bf16", "norm"), (12, 16, 16, 64, 0, "bf16", "norm"),
+    (192, 4, 4, 192, 1, "f32", "norm"), (80, 4, 4, 768, 1, "bf16", "norm"), (48, 4, 4, 384, 1, "f32", "norm")])
 @pytest.mark.parametrize("placed", [False, True])
 def test_against_the_separate_operators(dev, B, Hr, Wr, C, extra, dtype, mode, placed):
     from vtpack_amd import _lib, ops

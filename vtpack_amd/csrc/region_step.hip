@@ -534,15 +534,16 @@ extern "C" int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int
     if (C % vec != 0 || nvec > 192) return 0;
     // Up to where a wave for every four tokens is faster than one for sixteen that repeats nothing (the router's sums are
     // made from LDS again).  A forward, us, without it / with it (channels, regions): bf16 384: 256: 816 / 728, 512: 944 / 882,
-    // 1024: 1348 / 1304, 1536: 1648 / 1628, 2048: 1874 / 1885, 4096: 3062 / 3258; 768: 512: 2204 / 2090, 1024: 3320 / 3286,
-    // 1584: 4424 / 4426, 2560: 6495 / 6525; 320 (pyramid): 1024: 2320 / 2291, 2048: 3147 / 3170; fp32 192: 512: 1302 / 1196,
-    // 1024: 1967 / 1900, 2048: 2964 / 2863; 384: 512: 2572 / 2509, 768: 3438 / 3452, 1600: 5715 / 5789; 768: 384: 5296 /
-    // 5280, 768: 8626 / 8675.  Narrow rows, whose other kernels give several regions to a wave, gain longer, most of a wave's
-    // lanes idle or not: bf16 192: 16: 541 / 437, 128: 751 / 629, 512: 997 / 847, 1536: 1311 / 1202, 2048: 1393 / 1296, 2560: 1507 /
-    // 1415, 3072: 1712 / 1641, 4096: 2021 / 2024; pyramids of 64 to 512 channels by pictures of 256 px, bf16 2: 582 / 549, 16: 796 /
-    // 755, 48: 1024 / 994; fp32 8: 1004 / 980, with 2304 regions of 64 and 576 of 128 channels 1026 / 1028, 4096 and 1024:
-    // 1184 / 1207.
-    const int most = dtype == VTDGE_BF16 ? (nvec <= 32 ? 3072 : nvec <= WAVE ? 1536 : 1024) : nvec <= WAVE ? 2048 : 512;
+    // 1024: 1348 / 1304, 1568: 1552 / 1534, 2048: 1759 / 1777, 2560: 2056 / 2104; 768: 512: 2204 / 2090, 1040: 3262 / 3230, 1280:
+    // 3720 / 3664, 1584: 4325 / 4380; 320 (pyramid): 1024: 2320 / 2291, 2048: 3147 / 3170; fp32 192: 512: 1302 / 1196, 2080: 3200 /
+    // 3034, 3072: 4272 / 4138; 384: 528: 2418 / 2395, 768: 3002 / 2986, 1024: 3757 / 3713; 320 (pyramid): 768: 3865 / 3856, 1024:
+    // 4728 / 4745; 768: 384: 5296 / 5280, 528: 6572 / 6396, 768: 8303 / 8348.  Narrow rows, whose other kernels give several regions
+    // to a wave, gain longer in bf16, most of a wave's lanes idle or not: 192: 16: 541 / 437, 128: 751 / 629, 512: 997 / 847, 1536:
+    // 1311 / 1202, 2048: 1393 / 1296, 2560: 1507 / 1415, 3072: 1712 / 1641, 4096: 2021 / 2024; pyramids of 64 to 512 channels by
+    // pictures of 256 px, bf16 2: 582 / 549, 16: 796 / 755, 48: 1024 / 994; fp32 8: 1004 / 980, with 2304 regions of 64 and 576 of
+    // 128 channels 1026 / 1028, 4096 and 1024: 1184 / 1207.
+    const int most = dtype == VTDGE_BF16 ? (nvec <= 32 ? 3072 : nvec <= WAVE ? 1536 : 1280)
+                                         : (nvec <= 32 ? 2048 : nvec <= WAVE ? 3072 : nvec <= 128 ? 768 : 528);
     return regions <= most ? 1 : 0;
 }
 
