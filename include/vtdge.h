@@ -228,7 +228,7 @@ int vtdge_decompress_router_compress_static(const void *in, const void *sub, con
  *   out_records, next_comp_records (nullable, bf16 rows of 264 to 512 channels) or out_ln [B * (extra + H*W), C], next_comp_ln
  *   [capacity_rows, C] (nullable) with ln_weight, ln_bias; eps of either
  *   workspace: vtdge_region_step_workspace bytes, zero; its first word stays 0 unless the kernel gave up waiting
- * vtdge_region_step_fits: 1 for rows of 1 to 192 whole 16-byte vectors, up to 64 extra tokens and as many regions (512 to 3072, by
+ * vtdge_region_step_fits: 1 for rows of 1 to 192 whole 16-byte vectors, up to 64 extra tokens and as many regions (528 to 3072, by
  * width and type) as the launch is faster for than the separate ones. */
 int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int dtype);
 int64_t vtdge_region_step_workspace(int B, int H, int W);
