@@ -1073,3 +1073,40 @@ def test_rows_to_maps(dev, B, H, W, C, extra, off, dtype):
     got, want = ops.rows_to_maps(x), x.permute(0, 3, 1, 2).contiguous()
     assert got.shape == want.shape and got.is_contiguous()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("how", ["set_default_device", "with"])
+def test_operators_under_a_default_device(dev, how, train):
+    """A program whose default device is the GPU: counts still come to the CPU, and the results are those of one without."""
+    from vtpack_amd import layers
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    B, grid, h = 3, 12, 2
+    g = torch.Generator(dev).manual_seed(3)
+    x, k, v = (torch.randn(s, generator=g, device=dev).requires_grad_(train)
+               for s in ((B, 1 + grid * grid, 64 * h), (h, B, 20, 64), (h, B, 20, 64)))
+    idx, sp = _t(random_indices(5, B, 3, 3), dev), torch.tensor(SPLITS, device=dev)
+
+    def run():
+        patches, lengths = layers.grained_sample_index_to_patch(idx, sp, 4, 1)
+        assert lengths.device.type == "cpu"
+        comp = layers.grained_sample_compress(x, patches, grid, grid, 1)
+        q = comp.reshape(-1, h, 64).transpose(0, 1)
+        if train:
+            o = sparse_attention_train(q, k, v, lengths, 0.125)
+        else:
+            o = layers.batched_sparse_attention(q, k, v, lengths, 0.125).transpose(0, 1).reshape(-1, 64 * h)
+        out = layers.grained_sample_decompress(o - comp, patches, x, grid, grid, 1, True)
+        return (patches, lengths, out, *(torch.autograd.grad(out.square().sum(), (x, k, v)) if train else ()))
+    want = run()
+    if how == "with":
+        with torch.device(dev):
+            got = run()
+    else:
+        torch.set_default_device(dev)
+        try:
+            got = run()
+        finally:
+            torch.set_default_device(None)
+    for a, b in zip(got, want):
+        assert a.device == b.device and torch.equal(a, b)

@@ -127,8 +127,9 @@ def index_to_patch_host(indices, splits, region_size, num_extra_tokens):
     device = indices.device
     patches = torch.empty((capacity, 4), dtype=torch.int64, device=device)
     offsets = torch.empty((B + 1,), dtype=torch.int64, device=device)
-    pinned = torch.empty((B,), dtype=torch.int64, pin_memory=True)
-    lengths = torch.empty((B,), dtype=torch.int64)
+    # (on the CPU by name: under a default device both would go to the GPU)
+    pinned = torch.empty((B,), dtype=torch.int64, device="cpu", pin_memory=True)
+    lengths = torch.empty((B,), dtype=torch.int64, device="cpu")
     total = ctypes.c_int64()
     call("vtdge_index_to_patch_host", indices.data_ptr(), splits.data_ptr(), B, Hr, Wr, splits.numel(), region_size,
          num_extra_tokens, patches.data_ptr(), capacity, offsets.data_ptr(), pinned.data_ptr(), lengths.data_ptr(),
