@@ -1629,13 +1629,18 @@ extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *split
 // A device-to-host copy behind the kernel costs its own launch and a round trip through the runtime's staging buffer, and a wait
 // for the stream up to 50 us of a sleeping thread (a pass of sparse training, 64 samples, 192 channels fp32: 340 us with the
 // copy, 326 waiting for the stream, 303 looking at the counts themselves).
+extern "C" int vtdge_index_to_patch_host_fits(int B, int Hr, int Wr)
+{
+    return B > 0 && Hr > 0 && Wr > 0 && (int64_t)B * Hr <= ONE_LAUNCH_REGIONS && (int64_t)B * Hr * Wr <= ONE_LAUNCH_REGIONS ? 1 : 0;
+}
+
 extern "C" int vtdge_index_to_patch_host(const int64_t *indices, const int64_t *splits, int B, int Hr, int Wr, int S, int R,
                                          int extra, int64_t *patches, int64_t capacity_rows, int64_t *offsets, int64_t *pinned,
                                          int64_t *lengths_host, int64_t *total_host, void *stream)
 {
     VT_REQUIRE(patches && pinned && lengths_host && total_host, VTDGE_ERR_ARG, "index_to_patch: NULL operand");
-    VT_REQUIRE(B > 0 && Hr > 0 && Wr > 0 && (int64_t)B * Hr * Wr <= ONE_LAUNCH_REGIONS, VTDGE_ERR_UNSUPPORTED,
-               "index_to_patch: lengths on the host for %lld regions (at most %lld)", (long long)B * Hr * Wr,
+    VT_REQUIRE(vtdge_index_to_patch_host_fits(B, Hr, Wr), VTDGE_ERR_UNSUPPORTED,
+               "index_to_patch: lengths on the host for %d samples of %d x %d regions (1 to %lld in all)", B, Hr, Wr,
                (long long)ONE_LAUNCH_REGIONS);
     volatile int64_t *counts = pinned;
     for (int b = 0; b < B; b++) counts[b] = -1;

@@ -113,12 +113,13 @@ def index_to_patch(indices, splits, region_size, num_extra_tokens, capacity=None
 
 def index_to_patch_host(indices, splits, region_size, num_extra_tokens):
     """`index_to_patch` for callers that need the query counts now: (patches [capacity, 4], lengths [B] on the CPU, their
-    sum), behind a wait for the stream."""
+    sum).  Returns as soon as the counts have come; the patches belong to the current stream, like any result, and may
+    still be being written: another stream has to be ordered behind it."""
     _need_gpu(indices, splits)
     if indices.dtype != torch.int64 or splits.dtype != torch.int64 or indices.dim() != 3:
         raise TypeError("indices must be int64 [B, Hr, Wr] and splits int64")
     B, Hr, Wr = indices.shape
-    if not 0 < B * Hr * Wr <= 16384:
+    if not _lib.load().vtdge_index_to_patch_host_fits(B, Hr, Wr):
         patches, _, lengths = index_to_patch(indices, splits, region_size, num_extra_tokens)
         lengths = lengths.cpu()
         return patches, lengths, int(lengths.sum())
