@@ -93,8 +93,8 @@ int vtdge_index_to_patch(const int64_t *indices, const int64_t *splits, int B, i
  * `pinned` itself (int64 [B] of page-locked, coherent host memory), the call looks for them there for some time, waits for the
  * stream if they have not come by then, and copies them to lengths_host int64 [B] and their sum to total_host int64 [1].  Only
  * the lengths are there on return: patches and offsets are, like any result, ordered on `stream` and may still be being
- * written.  vtdge_index_to_patch_host_fits: 1 for the sizes that it takes (up to 16384 regions); others:
- * VTDGE_ERR_UNSUPPORTED.  Not for a stream that is being captured. */
+ * written.  vtdge_index_to_patch_host_fits: 1 for the sizes that it takes (up to 16384 regions); others, and a stream
+ * that is being captured: VTDGE_ERR_UNSUPPORTED, nothing launched. */
 int vtdge_index_to_patch_host_fits(int B, int Hr, int Wr);
 int vtdge_index_to_patch_host(const int64_t *indices, const int64_t *splits, int B, int Hr, int Wr, int S, int R, int extra,
                               int64_t *patches, int64_t capacity_rows, int64_t *offsets, int64_t *pinned,

@@ -1110,3 +1110,28 @@ def test_operators_under_a_default_device(dev, how, train):
             torch.set_default_device(None)
     for a, b in zip(got, want):
         assert a.device == b.device and torch.equal(a, b)
+
+
+def test_query_counts_during_a_capture(dev):
+    """Refused before anything is launched: the capture goes on, and its replays are right."""
+    from vtpack_amd import _C, _lib
+    idx, sp = _t(random_indices(2, 3, 4, 4), dev), torch.tensor(SPLITS, device=dev)
+    want = _C.grained_sample_index_to_patch(idx, sp, 4, 1)
+    patches, offsets = (torch.empty(s, dtype=torch.int64, device=dev) for s in ((3 * 257, 4), (4,)))
+    pinned, lengths, total = (torch.zeros(n, dtype=torch.int64).pin_memory() for n in (3, 3, 1))
+    x = torch.zeros(1000, device=dev)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = x + 1
+        with pytest.raises(RuntimeError, match="captured"):
+            _C.grained_sample_index_to_patch(idx, sp, 4, 1)
+        with pytest.raises(_lib.VtdgeError, match="captured"):
+            _lib.call("vtdge_index_to_patch_host", idx.data_ptr(), sp.data_ptr(), 3, 4, 4, 3, 4, 1, patches.data_ptr(), 3 * 257,
+                      offsets.data_ptr(), pinned.data_ptr(), lengths.data_ptr(), total.data_ptr(), _lib.stream_ptr())
+        y = y * 2
+    for i in range(3):
+        x.fill_(float(i))
+        graph.replay()
+        assert bool((y == 2 * i + 2).all())
+    got = _C.grained_sample_index_to_patch(idx, sp, 4, 1)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

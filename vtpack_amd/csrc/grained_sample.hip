@@ -1642,6 +1642,9 @@ extern "C" int vtdge_index_to_patch_host(const int64_t *indices, const int64_t *
     VT_REQUIRE(vtdge_index_to_patch_host_fits(B, Hr, Wr), VTDGE_ERR_UNSUPPORTED,
                "index_to_patch: lengths on the host for %d samples of %d x %d regions (1 to %lld in all)", B, Hr, Wr,
                (long long)ONE_LAUNCH_REGIONS);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    VT_REQUIRE(hipStreamIsCapturing((hipStream_t)stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone,
+               VTDGE_ERR_UNSUPPORTED, "index_to_patch: lengths on the host while the stream is being captured");
     volatile int64_t *counts = pinned;
     for (int b = 0; b < B; b++) counts[b] = -1;
     const int rc = vtdge_index_to_patch(indices, splits, B, Hr, Wr, S, R, extra, patches, capacity_rows, offsets, pinned, stream);

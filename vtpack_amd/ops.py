@@ -114,11 +114,13 @@ def index_to_patch(indices, splits, region_size, num_extra_tokens, capacity=None
 def index_to_patch_host(indices, splits, region_size, num_extra_tokens):
     """`index_to_patch` for callers that need the query counts now: (patches [capacity, 4], lengths [B] on the CPU, their
     sum).  Returns as soon as the counts have come; the patches belong to the current stream, like any result, and may
-    still be being written: another stream has to be ordered behind it."""
+    still be being written: another stream has to be ordered behind it.  Not for a stream that is being captured."""
     _need_gpu(indices, splits)
     if indices.dtype != torch.int64 or splits.dtype != torch.int64 or indices.dim() != 3:
         raise TypeError("indices must be int64 [B, Hr, Wr] and splits int64")
     B, Hr, Wr = indices.shape
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("the query counts cannot come to the host while the stream is being captured")
     if not _lib.load().vtdge_index_to_patch_host_fits(B, Hr, Wr):
         patches, _, lengths = index_to_patch(indices, splits, region_size, num_extra_tokens)
         lengths = lengths.cpu()
