@@ -1135,3 +1135,17 @@ def test_query_counts_during_a_capture(dev):
         assert bool((y == 2 * i + 2).all())
     got = _C.grained_sample_index_to_patch(idx, sp, 4, 1)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def test_query_counts_behind_a_long_queue(dev):
+    """Some milliseconds of products in front of the kernel: the call waits for the stream in the end."""
+    from vtpack_amd import _C
+    idx, sp = random_indices(4, 64, 4, 4), torch.tensor(SPLITS, device=dev)
+    want = orc.index_to_patch(idx, SPLITS, 4, 1)
+    a, at = torch.randn(8192, 8192, device=dev, dtype=torch.bfloat16), _t(idx, dev)
+    for _ in range(3):
+        for _ in range(4):
+            a @ a
+        patches, lengths = _C.grained_sample_index_to_patch(at, sp, 4, 1)
+        np.testing.assert_array_equal(lengths.numpy(), want[1])
+        np.testing.assert_array_equal(patches.cpu().numpy(), want[0])

@@ -1626,9 +1626,22 @@ extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *split
     return VTDGE_OK;
 }
 
-// A device-to-host copy behind the kernel costs its own launch and a round trip through the runtime's staging buffer, and a wait
-// for the stream up to 50 us of a sleeping thread (a pass of sparse training, 64 samples, 192 channels fp32: 340 us with the
-// copy, 326 waiting for the stream, 303 looking at the counts themselves).
+// A device-to-host copy behind the kernel costs its own launch and a round trip through the runtime's staging buffer, a wait for
+// the stream sees the kernel's end and not its first stores, and later (a pass of sparse training, 64 samples, 192 channels fp32:
+// 340 us with the copy, 326 waiting for the stream, 303 looking at the counts themselves; on another box 364 waiting, 311).
+// That is gained from 50 us of looking on, and not more with 2000 (nine cases of operators and training, 82 to 316 us a pass).  The
+// core is busy either way: with 0.3, 2.3 and 6.1 ms of products in front of it the thread's own time in the call is the whole
+// wait whether it looks for 0 or for 2000 us, as the runtime's wait for a stream does not sleep so soon.
+constexpr int COUNTS_US = 200;
+
+// leaves the core's execution units to its sibling thread
+static inline void cpu_pause()
+{
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+    __builtin_ia32_pause();
+#endif
+}
+
 extern "C" int vtdge_index_to_patch_host_fits(int B, int Hr, int Wr)
 {
     return B > 0 && Hr > 0 && Wr > 0 && (int64_t)B * Hr <= ONE_LAUNCH_REGIONS && (int64_t)B * Hr * Wr <= ONE_LAUNCH_REGIONS ? 1 : 0;
@@ -1650,19 +1663,23 @@ extern "C" int vtdge_index_to_patch_host(const int64_t *indices, const int64_t *
     const int rc = vtdge_index_to_patch(indices, splits, B, Hr, Wr, S, R, extra, patches, capacity_rows, offsets, pinned, stream);
     if (rc != VTDGE_OK) return rc;
     // every count is one store of its workgroup: seen here as soon as it is made.  What has a long queue before it is waited
-    // for as usual: the runtime may put the thread to sleep then, and it wakes up some 50 us late.
-    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    // for as usual.
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(COUNTS_US);
     int seen = 0;
     while (seen < B) {
         while (seen < B && counts[seen] >= 0) seen++;
         if (seen < B && std::chrono::steady_clock::now() > until) break;
+        cpu_pause();
     }
     if (seen < B) {
         const hipError_t err = hipStreamSynchronize((hipStream_t)stream);
         VT_REQUIRE(err == hipSuccess, VTDGE_ERR_LAUNCH, "index_to_patch: %s", hipGetErrorString(err));
     }
     int64_t total = 0;
-    for (int b = 0; b < B; b++) total += lengths_host[b] = counts[b];
+    for (int b = 0; b < B; b++) {
+        VT_REQUIRE(counts[b] >= 0, VTDGE_ERR_LAUNCH, "index_to_patch: the count of sample %d has not come", b);
+        total += lengths_host[b] = counts[b];
+    }
     *total_host = total;
     return VTDGE_OK;
 }
