@@ -65,6 +65,20 @@ def test_index_to_patch_over_several_workgroups(dev, B, Hr, Wr, extra, R, splits
     np.testing.assert_array_equal(got_p.cpu().numpy()[:len(want_p)], want_p)
 
 
+@pytest.mark.parametrize("B,Hr,Wr,extra", [(1, 128, 128, 1), (1, 1, 16385, 3), (1, 129, 129, 0), (3, 1, 33023, 257), (2, 200, 201, 1)])
+@pytest.mark.parametrize("fine", [0.0, 0.33, 0.34, 1.0])
+def test_index_to_patch_workgroups_of_several_chunks(dev, B, Hr, Wr, extra, fine):
+    """Samples of 64 times 256 regions, whose chunks have a workgroup each, and of more, which share one; last runs that are short.
+    Chunks of up to two queries a region on average, which a thread writes each, and of more."""
+    from vtpack_amd import ops
+    idx = (rng(Wr).random((B, Hr, Wr)) >= fine).astype(np.int64)
+    want_p, want_l = orc.index_to_patch(idx, [2, 1], 2, extra)
+    got_p, off, got_l = ops.index_to_patch(_t(idx, dev), _t(np.array([2, 1], dtype=np.int64), dev), 2, extra)
+    np.testing.assert_array_equal(got_l.cpu().numpy(), want_l)
+    np.testing.assert_array_equal(off.cpu().numpy(), np.concatenate([[0], np.cumsum(want_l)]))
+    np.testing.assert_array_equal(got_p.cpu().numpy()[:len(want_p)], want_p)
+
+
 def test_index_to_patch_uniform_gates(dev):
     from vtpack_amd import _C
     sp = _t(np.array(SPLITS, dtype=np.int64), dev)

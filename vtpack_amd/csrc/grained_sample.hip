@@ -313,21 +313,30 @@ __global__ __launch_bounds__(256) void patch_count_kernel(const int64_t *__restr
     if (lane == 0) lengths[b] = (int64_t)part + extra;
 }
 
-// Step 2: a workgroup per 256 regions of a sample.  Their query counts go through a wavefront prefix sum, and sixteen threads
-// write the descriptors of a region (32 bytes each, consecutive), sixteen regions a turn.  What bounds it is latency.  Us, with one
-// workgroup per sample and the region of every row searched for in the prefix sums (eight dependent reads of LDS) / so (samples,
-// regions of each): 6, 576: 18.3 / 9.4; 8, 1024: 31.0 / 11.4; 64, 256: 17.9 / 15.0; 64, 16: 4.7 / 4.5; 256, 16: 5.4 / 5.2; 1024,
-// 16: 15.3 / 13.6; 5000, 16 (after a scan): 54.9 / 56.5.
+// Step 2: a workgroup per chunk of 256 regions of a sample, or per run of chunks where a sample has more than PATCH_RUNS (RUNS).
+// The query counts of a chunk go through a wavefront prefix sum, every region's thread leaves its number at the region's rows in
+// LDS, and a thread writes a row's descriptor (32 bytes) at a time, consecutive ones side by side; with more rows than
+// that map holds sixteen threads write a region's.  What bounds it is latency, of large batches the stores.  Us, with one workgroup per
+// sample and the region of every row searched for in the prefix sums (eight dependent reads of LDS) / sixteen threads a
+// region throughout / so (samples, regions of each), regions of 1, 4 and 16 queries alike: 6, 576: 18.2 / 9.3 / 6.7; 8, 1024: 31.4 /
+// 11.2 / 8.8; 64, 256: 17.1 / 14.8 / 11.8; 256, 196: 12.9 / 11.4 / 9.6; 1024, 16: 14.8 / 13.0 / 13.1; 4096, 16: 16.7 / 16.0 / 16.6;
+// 5000, 16 (after a scan): 54.9 / 56.8 / 55.2; 256, 4096: 137 / 74 / 67; regions of one query: 64, 256: 12.2 / 15.6 / 9.5; 256, 196:
+// 7.3 / 10.4 / 6.7; 256, 4096: 51.9 / 70.8 / 37.7; 5000, 16: 52.5 / 55.5 / 51.4.
+// A workgroup adds up its sample's regions before its own, so that one per chunk takes a time that grows with the square of the
+// regions: 256, 65536 of one query: 953 us with one a sample, 1968 with one a chunk, 977 with 64 runs; 32, 2^20: 15524, 37796, 8973.
+// (The loop over chunks is an instantiation of its own: it takes 68 registers, a chunk alone 52, and eight waves a SIMD need 64.)
 //
 // FUSED: the workgroup also finds its own first row, as the sum of the query counts of all regions before it (it
-// reads their gate indices itself: a few KB out of L2 for the batch sizes this variant is launched for), and writes
-// offsets / lengths; no first step then, and no dependency between workgroups.
+// reads their gate indices itself: up to 128 KB out of L2, those of the first 4096 regions in one trip, with at most 16384 in all),
+// and writes offsets / lengths; no first step then, and no dependency between workgroups.
 // Not FUSED: the sample's first row comes from `offsets` (written by the scan kernel) or, with from_lengths, is the sum of
 // the lengths of the samples before this one (written by the count kernel), in which case the workgroup writes
 // offsets as well; only its own sample's regions before it are added up.
 typedef long long i64x2 __attribute__((ext_vector_type(2)));
+constexpr int PATCH_RUNS = 64;          // workgroups of a sample
+constexpr int PATCH_MAP = 4096;         // rows of a chunk that have their region looked up: all with splits of up to 4
 
-template <bool FUSED>
+template <bool FUSED, bool RUNS>
 __global__ __launch_bounds__(256) void patch_write_kernel(const int64_t *__restrict__ indices,
                                                            const int64_t *__restrict__ splits,
                                                            int64_t *__restrict__ offsets, int64_t *__restrict__ lengths,
@@ -339,19 +348,21 @@ __global__ __launch_bounds__(256) void patch_write_kernel(const int64_t *__restr
     __shared__ int split_s[VTDGE_MAX_SPLITS];
     __shared__ int64_t before_s[2][4];
     __shared__ int start_s[256], ps_s[256];
-    const int nreg = Hr * Wr, chunks = (nreg + 255) / 256;
-    const int b = blockIdx.x / chunks, base = (blockIdx.x - b * chunks) * 256, nr = min(256, nreg - base);
-    const bool last_chunk = base + 256 >= nreg;
+    __shared__ uint8_t region_s[PATCH_MAP];
+    static_assert(!FUSED || !RUNS, "one launch: samples of few chunks");
+    const int nreg = Hr * Wr, chunks = (nreg + 255) / 256, of_run = RUNS ? (chunks + gridDim.y - 1) / gridDim.y * 256 : 256;
+    const int b = blockIdx.x, base0 = blockIdx.y * of_run, end = base0 + min(of_run, nreg - base0);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     // everything the workgroup reads is requested before anything is used: the splits, the gate indices of
     // its own regions and (FUSED) sixteen per thread of those before them - one trip to memory instead of three
     const int sp = threadIdx.x < S ? (int)splits[threadIdx.x] : 1;
-    int64_t g_own = 0;
-    if (threadIdx.x < nr) g_own = indices[(int64_t)b * nreg + base + threadIdx.x];
     constexpr int PRE = FUSED ? 16 : 1;
-    const int64_t sample0 = (int64_t)b * nreg, own0 = sample0 + base;
+    const int64_t sample0 = (int64_t)b * nreg;
+    int64_t g_own = 0, row0 = 0;                   // row0: first row of the sample
+    if (!FUSED && !from_lengths) row0 = offsets[b];
+    if (threadIdx.x < end - base0) g_own = indices[sample0 + base0 + threadIdx.x];
     const int64_t *const from = FUSED ? indices : indices + sample0;
-    const int64_t nbefore = FUSED ? own0 : base;
+    const int64_t nbefore = FUSED ? sample0 + base0 : base0;
     int64_t gq[PRE];
 #pragma unroll
     for (int i = 0; i < PRE; i++) {
@@ -382,67 +393,95 @@ __global__ __launch_bounds__(256) void patch_write_kernel(const int64_t *__restr
     }
     if (!FUSED && from_lengths)
         for (int i = threadIdx.x; i < b; i += 256) sample_part += lengths[i];
+    if (FUSED || from_lengths) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        sample_part += __shfl_xor(sample_part, o, WAVE);
-        if (chunks > 1) own_part += __shfl_xor(own_part, o, WAVE);
+        for (int o = 32; o > 0; o >>= 1) sample_part += __shfl_xor(sample_part, o, WAVE);
     }
-    const int ps = threadIdx.x < nr ? split_of(g_own) : 0;
-    const int cnt = ps * ps;
-    int inc = cnt;
+    if (chunks > 1) {
 #pragma unroll
-    for (int o = 1; o < WAVE; o <<= 1) {
-        int up = __shfl_up(inc, o, WAVE);
-        if (lane >= o) inc += up;
+        for (int o = 32; o > 0; o >>= 1) own_part += __shfl_xor(own_part, o, WAVE);
     }
-    if (lane == 63) wave_tot[wid] = inc;
-    if (lane == 0) {
-        before_s[0][wid] = sample_part;
-        before_s[1][wid] = own_part;
-    }
-    __syncthreads();
-    int first = inc - cnt;
-    for (int w = 0; w < wid; w++) first += wave_tot[w];
-    start_s[threadIdx.x] = first;                  // first row of the region, of those of the workgroup
-    ps_s[threadIdx.x] = ps;
-    int64_t row0 = before_s[0][0] + before_s[0][1] + before_s[0][2] + before_s[0][3];
-    const int64_t in_sample = before_s[1][0] + before_s[1][1] + before_s[1][2] + before_s[1][3];
-    if constexpr (FUSED) row0 += (int64_t)b * extra;
-    else if (!from_lengths) row0 = offsets[b];
-    if (threadIdx.x == 0 && last_chunk) {
-        const int64_t len = extra + in_sample + wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
-        if constexpr (FUSED) lengths[b] = len;
-        if (FUSED || from_lengths) {
-            offsets[b] = row0;
-            if (b == B - 1) offsets[B] = row0 + len;
+    int64_t in_sample = 0;                         // rows of its regions before this chunk
+    int base = base0;
+    do {
+        const int nr = min(256, end - base);
+        if (RUNS && base > base0) {                // (the chunk before has been written)
+            g_own = threadIdx.x < nr ? indices[sample0 + base + threadIdx.x] : 0;
+            __syncthreads();
         }
-    }
-    if (base == 0)
-        for (int e = threadIdx.x; e < extra; e += 256) {
-            const int64_t row = row0 + e;
-            if (row < capacity) {
-                int64_t *p = patches + 4 * row;
-                p[0] = b; p[1] = -(int64_t)e - 1; p[2] = 0; p[3] = 1;
+        const int ps = threadIdx.x < nr ? split_of(g_own) : 0;
+        const int cnt = ps * ps;
+        int inc = cnt;
+#pragma unroll
+        for (int o = 1; o < WAVE; o <<= 1) {
+            int up = __shfl_up(inc, o, WAVE);
+            if (lane >= o) inc += up;
+        }
+        if (lane == 63) wave_tot[wid] = inc;
+        if (lane == 0 && base == base0) {
+            before_s[0][wid] = sample_part;
+            before_s[1][wid] = own_part;
+        }
+        __syncthreads();
+        int first = inc - cnt;
+        for (int w = 0; w < wid; w++) first += wave_tot[w];
+        start_s[threadIdx.x] = first;              // first row of the region, of those of the chunk
+        ps_s[threadIdx.x] = ps;
+        const int total = wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
+        const bool mapped = total <= PATCH_MAP;
+        if (mapped)
+#pragma clang loop vectorize(disable) unroll(disable)
+            for (int j = 0; j < min(cnt, PATCH_MAP - first); j++) region_s[first + j] = (uint8_t)threadIdx.x;
+        if (base == base0) {
+            row0 += before_s[0][0] + before_s[0][1] + before_s[0][2] + before_s[0][3];
+            in_sample = before_s[1][0] + before_s[1][1] + before_s[1][2] + before_s[1][3];
+            if constexpr (FUSED) row0 += (int64_t)b * extra;
+            if (base == 0)
+                for (int e = threadIdx.x; e < extra; e += 256) {
+                    const int64_t row = row0 + e;
+                    if (row < capacity) {
+                        int64_t *p = patches + 4 * row;
+                        p[0] = b; p[1] = -(int64_t)e - 1; p[2] = 0; p[3] = 1;
+                    }
+                }
+        }
+        const int64_t chunk0 = row0 + extra + in_sample;
+        in_sample += total;
+        if (threadIdx.x == 0 && base + nr == nreg) {
+            const int64_t len = extra + in_sample;
+            if constexpr (FUSED) lengths[b] = len;
+            if (FUSED || from_lengths) {
+                offsets[b] = row0;
+                if (b == B - 1) offsets[B] = row0 + len;
             }
         }
-    __syncthreads();
-    row0 += extra + in_sample;
-    for (int r = threadIdx.x >> 4; r < nr; r += 16) {
-        const int rps = ps_s[r], rows = rps * rps;
-        if ((threadIdx.x & 15) >= rows) continue;
-        const int rg = base + r, ry = rg / Wr, rx = rg - ry * Wr, step = R / rps;
-        const int64_t at = row0 + start_s[r];
-        for (int j = threadIdx.x & 15; j < rows; j += 16) {
+        __syncthreads();
+        auto write = [&](int r, int j) {
+            const int rps = ps_s[r], rg = base + r, ry = rg / Wr, rx = rg - ry * Wr, step = R / rps;
             const int dy = j / rps, dx = j - dy * rps;
-            if (at + j < capacity) {
-                i64x2 *p = reinterpret_cast<i64x2 *>(patches + 4 * (at + j));
+            const int64_t row = chunk0 + start_s[r] + j;
+            if (row < capacity) {
+                i64x2 *p = reinterpret_cast<i64x2 *>(patches + 4 * row);
                 const i64x2 lo2 = {(int64_t)b, (int64_t)ry * R + dy * step};
                 const i64x2 hi2 = {(int64_t)rx * R + dx * step, (int64_t)step};
                 p[0] = lo2;
                 p[1] = hi2;
             }
+        };
+        if (mapped) {
+#pragma unroll 1
+            for (int j = threadIdx.x; j < total; j += 256) {
+                const int r = region_s[j];
+                write(r, j - start_s[r]);
+            }
+        } else {
+#pragma unroll 1
+            for (int r = threadIdx.x >> 4; r < nr; r += 16)
+#pragma unroll 1
+                for (int j = threadIdx.x & 15; j < ps_s[r] * ps_s[r]; j += 16) write(r, j);
         }
-    }
+        base += 256;
+    } while (RUNS && base < end);
 }
 
 struct DenseSplits {
@@ -1596,11 +1635,13 @@ extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *split
     VT_REQUIRE((reinterpret_cast<uintptr_t>(patches) & 15u) == 0, VTDGE_ERR_ARG,
                "index_to_patch: patches must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
-    const unsigned chunks = (unsigned)ceil_div((int64_t)Hr * Wr, 256);
+    const int64_t chunks = ceil_div((int64_t)Hr * Wr, 256), of_run = ceil_div(chunks, PATCH_RUNS);
+    const dim3 grid((unsigned)B, (unsigned)ceil_div(chunks, of_run));
+    auto write = of_run > 1 ? patch_write_kernel<false, true> : patch_write_kernel<false, false>;
     if (patches != nullptr && (int64_t)B * Hr * Wr <= ONE_LAUNCH_REGIONS) {
         // small batches: one launch, every sample's workgroup sums the counts before it on its own
-        note_kernel(reinterpret_cast<const void *>(patch_write_kernel<true>));
-        patch_write_kernel<true><<<B * chunks, 256, 0, st>>>(indices, splits, offsets, lengths, B, Hr, Wr, S, R, extra, patches,
+        note_kernel(reinterpret_cast<const void *>(patch_write_kernel<true, false>));
+        patch_write_kernel<true, false><<<grid, 256, 0, st>>>(indices, splits, offsets, lengths, B, Hr, Wr, S, R, extra, patches,
                                                     capacity_rows, 0);
         return check_launch("index_to_patch");
     }
@@ -1609,8 +1650,8 @@ extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *split
         note_kernel(reinterpret_cast<const void *>(patch_count_kernel));
         patch_count_kernel<<<(B + 3) / 4, 256, 0, st>>>(indices, splits, B, Hr * Wr, S, extra, lengths);
         if (int rc = check_launch("index_to_patch(count)")) return rc;
-        note_kernel(reinterpret_cast<const void *>(patch_write_kernel<false>));
-        patch_write_kernel<false><<<B * chunks, 256, 0, st>>>(indices, splits, offsets, lengths, B, Hr, Wr, S, R, extra, patches,
+        note_kernel(reinterpret_cast<const void *>(write));
+        write<<<grid, 256, 0, st>>>(indices, splits, offsets, lengths, B, Hr, Wr, S, R, extra, patches,
                                                      capacity_rows, 1);
         return check_launch("index_to_patch(write)");
     }
@@ -1618,8 +1659,8 @@ extern "C" int vtdge_index_to_patch(const int64_t *indices, const int64_t *split
     patch_count_scan_kernel<<<1, 1024, 0, st>>>(indices, splits, B, Hr * Wr, S, extra, offsets, lengths);
     if (int rc = check_launch("index_to_patch(count+scan)")) return rc;
     if (patches != nullptr) {
-        note_kernel(reinterpret_cast<const void *>(patch_write_kernel<false>));
-        patch_write_kernel<false><<<B * chunks, 256, 0, st>>>(indices, splits, offsets, lengths, B, Hr, Wr, S, R, extra, patches,
+        note_kernel(reinterpret_cast<const void *>(write));
+        write<<<grid, 256, 0, st>>>(indices, splits, offsets, lengths, B, Hr, Wr, S, R, extra, patches,
                                                      capacity_rows, 0);
         return check_launch("index_to_patch(write)");
     }
