@@ -34,11 +34,36 @@ def test_long_rows(dev, live, N, K, act, res):
 def test_rows_apart_and_a_result_in_the_residuals_place(dev):
     from vtpack_amd import _lib, ops
     g = torch.Generator(dev).manual_seed(1)
-    wide = torch.randn(3000, 1600, generator=g, device=dev).bfloat16()
+    wide = torch.randn(11000, 1600, generator=g, device=dev).bfloat16()
     w = (torch.randn(768, 768, generator=g, device=dev) * 768 ** -0.5).bfloat16()
-    r = torch.randn(3000, 768, generator=g, device=dev).bfloat16()
+    r = torch.randn(11000, 768, generator=g, device=dev).bfloat16()
     a = wide[:, 832:]
     want = a.float() @ w.float().T + r.float()
     ops.linear(a, w, None, r, out=r)
     assert "linear_dma_tile_kernel" in _lib.last_kernel()
     assert rel_err(r, want) <= 2 ** -8
+
+
+@pytest.mark.parametrize("rows,N,K,act,res,packed,tile", [
+    (2056, 1536, 768, "none", False, False, True), (2047, 1536, 768, "none", False, False, False),
+    (10922, 768, 768, "none", True, False, False), (10923, 768, 768, "none", True, False, True),
+    (24966, 768, 768, "none", True, True, False), (24967, 768, 768, "none", True, True, True),
+    (5461, 768, 3072, "none", True, False, False), (5462, 768, 3072, "none", True, False, True),
+    (12484, 768, 3072, "none", True, True, False), (12485, 768, 3072, "none", True, True, True),
+    (4681, 3072, 768, "gelu", False, True, False), (4682, 3072, 768, "gelu", False, True, True),
+    (2730, 1536, 3072, "none", False, False, False), (2731, 1536, 3072, "none", False, False, True),
+    (4096, 2048, 832, "gelu", True, False, False)])
+def test_calls_that_take_it(dev, rows, N, K, act, res, packed, tile):
+    """Each line of the rule from both sides, with the result of either kernel."""
+    from vtpack_amd import _lib, ops
+    g = torch.Generator(dev).manual_seed(rows)
+    a, r = (torch.randn(*s, generator=g, device=dev).bfloat16() for s in ((rows, K), (rows, N)))
+    w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
+    rows_dev = torch.tensor([rows - 1], device=dev) if packed else None
+    out = ops.linear(a, w, None, r if res else None, act=act, rows_dev=rows_dev)
+    assert ("linear_dma_tile_kernel" if tile else "linear_dma_kernel") in _lib.last_kernel()
+    want = a.float() @ w.float().T
+    want = torch.nn.functional.gelu(want) if act == "gelu" else want
+    want = want + r.float() if res else want
+    # one rounding of the result, as above (two with an activation in front of the residual)
+    assert rel_err(out[:rows - packed], want[:rows - packed]) <= 2 ** -8

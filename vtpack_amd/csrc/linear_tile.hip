@@ -7,8 +7,8 @@
 // one is running: eight reads in a row cost 108 clocks on top of 512 of products (measured, registers and LDS only), single
 // ones between the products nothing.  So fragments of the next step and direct loads go out one at a time between the products,
 // across the stages' barriers too (11200 rows, 768, 3072: 72 us with reads and loads in a row, 63 like this).  A normal-valued
-// product loop alone, out of registers, runs at 1.65 PFLOP/s here (the clock falls to 1.65 GHz); this kernel reaches 0.96 to
-// 1.0 at K = 3072.
+// product loop alone, out of registers, runs at 1.65 PFLOP/s here (the clock falls to 1.65 GHz); this kernel reaches 0.93 to
+// 1.0 at K = 3072 with 25443 live rows, 0.87 with 11195, and 0.5 to 0.8 at K = 768.
 //   * A runs through a ring of three 64-value slabs, W of two (160 KB for 256 x 256), direct loads swizzled as in
 //     linear_dma.hip; one barrier a slab, before it a counted wait for this wave's loads of the next one.
 //   * An XCD takes an eighth of the rows, in units of 64, and walks the column tiles of a block of rows first.  As many whole
@@ -16,9 +16,10 @@
 //     known to the kernel only.
 //   * The sums start from the bias; the results leave in 16-byte pieces after half-wave swaps, residuals come a block of rows
 //     ahead.
-// Measured against the tiles of linear_dma.hip (rows, N, K, us before / now): 25443, 1536, 768: 77.3 / 70.5; 25443, 3072, 768 +
-// GELU: 159 / 149, 11200: 78 / 73; 25443, 768, 3072 + residual: 142 / 119, 11200: 83 / 65; 4200: 29 / 33; 1700: 28.3 / 27;
-// 25443, 768, 768 + residual: 48 / 45.5, 11200: 30 / 27, 4200: 12 / 13.
+// Measured against the tiles of linear_dma.hip (live rows, N, K, us there / here): 25443, 1536, 768: 69.8 / 67.8; 25443, 3072, 768 +
+// GELU: 160 / 150, 11195: 77.0 / 74.7; 25443, 768, 3072 + residual: 158 / 129, 11195: 78.6 / 61.0; 25443, 768, 768 + residual: 46.5 /
+// 44.3, 11195: 28.8 / 26.1; 32896, 4096, 1024 + GELU: 346 / 294; 25443, 1024, 4096 + residual: 277 / 204.  Which calls take
+// it: linear_tile_wanted below.
 #include "common.h"
 
 namespace vtdge {
@@ -341,14 +342,28 @@ template <int ACT, bool HAS_RES> static int go_tile(const TileArgs &a, hipStream
 // Which products the kernel is taken for (beyond what linear_dma_applicable asks and linear_small_wanted leaves).  Shorter rows
 // and narrower outputs leave its tiles few slabs and many epilogues: 28000, 1280, 320 + GELU: 48.0 / 49.4 us (linear_dma.hip /
 // here) with all rows live, 23.6 / 30.5 with 0.44 of them; 16640, 2048, 512 + GELU: 57.4 / 52.3 and 25.8 / 25.8; 16640, 512,
-// 2048: 58.1 / 47.0 and 22.5 / 24.6; 32896, 768, 192 + GELU: 23.7 / 30.5; few
-// rows: 1285, 1536, 768: 10.6 / 11.5; 1285, 3072, 768 + GELU: 21.4 / 19.9 and 12.8 / 13.8.  From 768 on, all rows and 0.44 of them: 2570, 1536, 768:
-// 18.9 / 16.7, 10.8 / 11.9; 2570, 768, 3072: 29.3 / 32.5, 27.2 / 26.0; 5140, 1536, 768: 25.6 / 22.9, 18.7 / 13.5; 5140, 3072, 768 +
-// GELU: 43.0 / 40.9, 31.1 / 24.8; 5140, 768, 3072: 53.1 / 46.8, 28.0 / 27.4; 10280, 768, 3072: 78.1 / 62.2, 30.3 / 32.3.
-bool linear_tile_wanted(int64_t lda, int64_t rows, int N, int K, int act, const void *res)
+// 2048: 58.1 / 47.0 and 22.5 / 24.6; 32896, 768, 192 + GELU: 23.7 / 30.5.
+// Above that it depends on the live rows, which only the device knows where they are packed (rows_dev): routed samples keep 7 of
+// 16 (regions of 16, 4 and 1 queries alike), untrained routers all of them, and a rule has to serve both.
+//   * Outputs that linear_dma.hip gives 128x128 tiles: while those fill the chip once at most and the 64x128 tiles of this kernel
+//     do not, its 128x128 tiles are slower (four waves against eight and four loaders): 4500 live rows of 768, 3072 + residual
+//     28.4 / 33.6, of 768, 768 + residual 11.9 / 14.5.  Taken from where 7 of 16 rows are past that, short K from twice as much on:
+//     12850 rows of 768, 3072 with 7 of 16 live 51.8 / 46.3, all 82.5 / 66.7; 25769 of 768, 768 + residual 29.6 / 26.8, 49.5 / 49.3.
+//     (A quarter of the rows live costs up to a fifth there: 14872 of 768, 3072: 27.6 / 33.3.)
+//   * Wider ones, 128x256 there: all rows live, always (28 sizes from 2056 to 40000 rows: 1536, 768 mean 0.92, the worst 1.01;
+//     2048, 1024 0.91, 1.04; 3072, 1536 0.88, 1.03).  Packed, 3072, 768 + GELU: with 7 of 16 and with all live 2056: 12.4 / 14.4, 27.6
+//     / 23.7; 3976: 17.8 / 19.8, 32.8 / 31.2; 4954: 29.5 / 24.0, 34.7 / 37.7; from there on the mean of 20 sizes is 0.98 (0.80 to 1.14), with 4096, 1024 0.92.
+// A pass of the 768-channel model, us, without this kernel / with it wherever K and N allow / so (256 px pictures): 5: 1033 / 1014 /
+// 1018; 12: 1496 / 1488 / 1499; 20: 1737 / 1694 / 1722; 32: 1977 / 2013 / 1981; 60: 2886 / 2943 / 2907; 64: 3108 / 3048 / 2999; 99: 4399 /
+// 4276 / 4283; 128: 5447 / 5175 / 5187.
+bool linear_tile_wanted(int64_t lda, bool packed, int64_t rows, int N, int K, int act, const void *res)
 {
-    return rows >= 2048 && N >= 768 && K >= 768 && K % 64 == 0 && (act == VTDGE_ACT_NONE || res == nullptr) && rows < (1ll << 30) &&
-           lda < (1 << 23) && K < (1 << 23);
+    if (rows < 2048 || N < 768 || K < 768 || K % 64 != 0 || (act != VTDGE_ACT_NONE && res != nullptr) || rows >= (1ll << 30) ||
+        lda >= (1 << 23) || K >= (1 << 23) || compute_units() != 256)      // its rounds are counted for a workgroup on each of 256
+        return false;
+    const int64_t live = (packed ? rows * 7 / 16 : rows) * N;
+    if (N < 1536 || K >= 2048 || res != nullptr) return live >= (K >= 1536 ? 1ll << 22 : 1ll << 23);
+    return !packed || live >= 6ll << 20;
 }
 
 int launch_linear_tile(const void *A, int64_t lda, const void *W, const void *bias, const void *res, int64_t ldr, void *out,
