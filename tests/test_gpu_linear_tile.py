@@ -21,7 +21,7 @@ def test_long_rows(dev, live, N, K, act, res):
     bias = torch.randn(N, generator=g, device=dev).bfloat16() if live % 2 else None
     out = torch.full((cap, N), 7.0, device=dev, dtype=torch.bfloat16)
     ops.linear(a, w, bias, r if res else None, act=act, rows_dev=torch.tensor([live], device=dev), out=out)
-    assert "linear_dma_tile_kernel" in _lib.last_kernel()
+    assert "linear_tile_kernel" in _lib.last_kernel()
     if live:
         want = a[:live].float() @ w.float().T + (bias.float() if bias is not None else 0)
         want = torch.nn.functional.gelu(want) if act == "gelu" else want
@@ -40,7 +40,7 @@ def test_rows_apart_and_a_result_in_the_residuals_place(dev):
     a = wide[:, 832:]
     want = a.float() @ w.float().T + r.float()
     ops.linear(a, w, None, r, out=r)
-    assert "linear_dma_tile_kernel" in _lib.last_kernel()
+    assert "linear_tile_kernel" in _lib.last_kernel()
     assert rel_err(r, want) <= 2 ** -8
 
 
@@ -61,7 +61,7 @@ def test_calls_that_take_it(dev, rows, N, K, act, res, packed, tile):
     w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
     rows_dev = torch.tensor([rows - 1], device=dev) if packed else None
     out = ops.linear(a, w, None, r if res else None, act=act, rows_dev=rows_dev)
-    assert ("linear_dma_tile_kernel" if tile else "linear_dma_kernel") in _lib.last_kernel()
+    assert ("linear_tile_kernel" if tile else "linear_dma_kernel") in _lib.last_kernel()
     want = a.float() @ w.float().T
     want = torch.nn.functional.gelu(want) if act == "gelu" else want
     want = want + r.float() if res else want

@@ -290,7 +290,7 @@ __device__ __forceinline__ void tile_phase(const TileArgs &p, unsigned char *sme
 }
 
 template <int ACT, bool HAS_RES>
-__global__ __launch_bounds__(256, 1) void linear_dma_tile_kernel(TileArgs p)
+__global__ __launch_bounds__(256, 1) void linear_tile_kernel(TileArgs p)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int64_t live = live_rows(p.rows_dev, p.rows);
@@ -332,7 +332,7 @@ __global__ __launch_bounds__(256, 1) void linear_dma_tile_kernel(TileArgs p)
 
 template <int ACT, bool HAS_RES> static int go_tile(const TileArgs &a, hipStream_t st)
 {
-    auto kern = linear_dma_tile_kernel<ACT, HAS_RES>;
+    auto kern = linear_tile_kernel<ACT, HAS_RES>;
     VT_RESERVE_LDS(kern, TILE_LDS, "linear");
     note_kernel(reinterpret_cast<const void *>(kern));
     kern<<<256, 256, TILE_LDS, st>>>(a);
