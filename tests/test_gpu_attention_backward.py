@@ -300,7 +300,7 @@ def test_scores_kept_between_the_walks(dev, n):
 @pytest.mark.parametrize("B,h", [(2051, 1), (1023, 8), (1025, 8), (4, 12)])
 def test_workgroups_find_their_queries(dev, dtype, B, h):
     """Ragged batches whose workgroups look through several steps of pairs for theirs, or through none: the bits of the same
-    samples in calls of 16, whose pairs are found in the first step."""
+    samples in calls of 16 (of 2), whose pairs are found in the first step, and a few samples, longest and last, against float64."""
     from vtpack_amd.layers.sparse_ops import sparse_attention_train
     n, d = 20, 64
     g = torch.Generator(dev).manual_seed(B)
@@ -316,9 +316,18 @@ def test_workgroups_find_their_queries(dev, dtype, B, h):
         out = sparse_attention_train(*args, lengths, 0.125)
         return out.detach(), *torch.autograd.grad(out, args, go.reshape(out.shape))
     out, dq, dk, dv = run(q, k, v, lengths, go)
-    at = 0
-    for b in range(0, B, max(16, B // 8 // 16 * 16)):
-        e = min(b + 16, B)
+    first = torch.cumsum(lengths, 0) - lengths
+    some = sorted({0, 1, min(97, B - 1), B // 2, B - 2, B - 1})
+    rows = torch.cat([torch.arange(first[b], first[b] + lengths[b]) for b in some])
+    want, grads = _reference(q[rows].cpu().transpose(0, 1), k[:, some].cpu(), v[:, some].cpu(), lengths[some].tolist(), 0.125,
+                             go[rows].cpu().reshape(len(rows), h * d))
+    assert float((out[rows].double().cpu() - want).abs().max()) <= TOL[dtype] * float(want.abs().max())
+    for name, a, b in zip("qkv", (dq[:, rows], dk[:, some], dv[:, some]), grads):
+        size = max(float(b.abs().max()), 24 * 0.125 if name != "v" else 0)       # as in test_against_float64
+        assert float((a.double().cpu() - b).abs().max()) <= TOL[dtype] * size, name
+    part = 16 if B > 16 else 2
+    for b in range(0, B, max(part, B // 8 // 16 * 16)):
+        e = min(b + part, B)
         at = int(lengths[:b].sum())
         to = at + int(lengths[b:e].sum())
         if int(lengths[b:e].max()) == int(lengths[b:e].min()):

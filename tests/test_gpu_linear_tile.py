@@ -44,6 +44,32 @@ def test_rows_apart_and_a_result_in_the_residuals_place(dev):
     assert rel_err(r, want) <= 2 ** -8
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("live", [24576, 25000, 25443])
+def test_rows_that_are_not_finite_stay_by_themselves(dev, bad, live):
+    """Rows of an infinity or NaN beside rows of another XCD's share of the live ones (whole 64-row units),
+    at tiles' edges and past the live rows: only their own results are not finite."""
+    from vtpack_amd import _lib, ops
+    g = torch.Generator(dev).manual_seed(live)
+    a = torch.randn(25443, 768, generator=g, device=dev).bfloat16()
+    w = (torch.randn(776, 768, generator=g, device=dev) * 768 ** -0.5).bfloat16()
+    units = -(-live // 64)
+    rows = {live - 1}
+    for share in range(8):
+        at = units * share // 8 * 64
+        rows |= {r for r in (at, at - 1, at + 255, at + 256) if 0 <= r < live}
+    rows = sorted(rows)
+    ops.linear(a, w, None, rows_dev=torch.tensor([live], device=dev), out=(want := torch.zeros(25443, 776, device=dev, dtype=a.dtype)))
+    a[rows, 5] = bad
+    a[live:] = bad
+    out = torch.full_like(want, 7.0)
+    ops.linear(a, w, None, rows_dev=torch.tensor([live], device=dev), out=out)
+    assert "linear_tile_kernel" in _lib.last_kernel()
+    assert not bool(out[rows].isfinite().any())
+    out[rows], want[rows] = 0, 0
+    assert torch.equal(out[:live], want[:live]) and bool((out[live:] == 7.0).all())
+
+
 @pytest.mark.parametrize("rows,N,K,act,res,packed,tile", [
     (2056, 1536, 768, "none", False, False, True), (2047, 1536, 768, "none", False, False, False),
     (10922, 768, 768, "none", True, False, False), (10923, 768, 768, "none", True, False, True),
