@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
 def test_long_rows(dev, live, N, K, act, res):
     from vtpack_amd import _lib, ops
     cap = 25443
+    K = max(K, 1600 if res else 1024 if act == "gelu" else 0)      # epilogues behind a shorter K are linear_dma.hip's
     live = cap if live is None else live
     g = torch.Generator(dev).manual_seed(live + N)
     a, r = (torch.randn(*s, generator=g, device=dev).bfloat16() for s in ((cap, K), (cap, N)))
@@ -34,9 +35,9 @@ def test_long_rows(dev, live, N, K, act, res):
 def test_rows_apart_and_a_result_in_the_residuals_place(dev):
     from vtpack_amd import _lib, ops
     g = torch.Generator(dev).manual_seed(1)
-    wide = torch.randn(11000, 1600, generator=g, device=dev).bfloat16()
-    w = (torch.randn(768, 768, generator=g, device=dev) * 768 ** -0.5).bfloat16()
-    r = torch.randn(11000, 768, generator=g, device=dev).bfloat16()
+    wide = torch.randn(6000, 2432, generator=g, device=dev).bfloat16()
+    w = (torch.randn(768, 1600, generator=g, device=dev) * 1600 ** -0.5).bfloat16()
+    r = torch.randn(6000, 768, generator=g, device=dev).bfloat16()
     a = wide[:, 832:]
     want = a.float() @ w.float().T + r.float()
     ops.linear(a, w, None, r, out=r)
@@ -70,15 +71,17 @@ def test_rows_that_are_not_finite_stay_by_themselves(dev, bad, live):
     assert torch.equal(out[:live], want[:live]) and bool((out[live:] == 7.0).all())
 
 
-@pytest.mark.parametrize("rows,N,K,act,res,packed,tile", [
-    (2056, 1536, 768, "none", False, False, True), (2047, 1536, 768, "none", False, False, False),
-    (10922, 768, 768, "none", True, False, False), (10923, 768, 768, "none", True, False, True),
-    (24966, 768, 768, "none", True, True, False), (24967, 768, 768, "none", True, True, True),
-    (5461, 768, 3072, "none", True, False, False), (5462, 768, 3072, "none", True, False, True),
-    (12484, 768, 3072, "none", True, True, False), (12485, 768, 3072, "none", True, True, True),
-    (4681, 3072, 768, "gelu", False, True, False), (4682, 3072, 768, "gelu", False, True, True),
-    (2730, 1536, 3072, "none", False, False, False), (2731, 1536, 3072, "none", False, False, True),
-    (4096, 2048, 832, "gelu", True, False, False)])
+@pytest.mark.parametrize("rows,N,K,act,res,tile", [
+    (2048, 1536, 768, "none", False, True), (2047, 1536, 768, "none", False, False),
+    (10922, 768, 768, "none", False, False), (10923, 768, 768, "none", False, True),
+    (25443, 768, 1472, "none", True, False), (25443, 768, 1600, "none", True, True),
+    (2730, 768, 3072, "none", True, True), (2731, 768, 3072, "none", True, False),
+    (5461, 768, 3072, "none", True, False), (5462, 768, 3072, "none", True, True),
+    (2730, 1536, 2048, "none", False, False), (2731, 1536, 2048, "none", False, True),
+    (3413, 1536, 768, "none", False, True), (3414, 1536, 768, "none", False, False),
+    (5120, 1536, 768, "none", False, False), (5121, 1536, 768, "none", False, True), (4096, 1536, 1024, "none", False, True),
+    (8192, 3072, 960, "gelu", False, False), (2056, 3072, 1024, "gelu", False, True), (4096, 2048, 832, "gelu", True, False)])
+@pytest.mark.parametrize("packed", [False, True])
 def test_calls_that_take_it(dev, rows, N, K, act, res, packed, tile):
     """Each line of the rule from both sides, with the result of either kernel."""
     from vtpack_amd import _lib, ops

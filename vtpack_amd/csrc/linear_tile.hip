@@ -16,10 +16,9 @@
 //     known to the kernel only.
 //   * The sums start from the bias; the results leave in 16-byte pieces after half-wave swaps, residuals come a block of rows
 //     ahead.
-// Measured against the tiles of linear_dma.hip (live rows, N, K, us there / here): 25443, 1536, 768: 69.8 / 67.8; 25443, 3072, 768 +
-// GELU: 160 / 150, 11195: 77.0 / 74.7; 25443, 768, 3072 + residual: 158 / 129, 11195: 78.6 / 61.0; 25443, 768, 768 + residual: 46.5 /
-// 44.3, 11195: 28.8 / 26.1; 32896, 4096, 1024 + GELU: 346 / 294; 25443, 1024, 4096 + residual: 277 / 204.  Which calls take
-// it: linear_tile_wanted below.
+// Launches one behind the other against the tiles of linear_dma.hip (live rows, N, K, us there / here): 25443, 1536, 768: 69.8 /
+// 67.8; 25443, 768, 3072 + residual: 158 / 129, 11195: 78.6 / 61.0; 32896, 4096, 1024 + GELU: 346 / 294; 25443, 1024, 4096 + residual:
+// 277 / 204.  Which calls take it: linear_tile_wanted below.
 #include "common.h"
 
 namespace vtdge {
@@ -343,27 +342,33 @@ template <int ACT, bool HAS_RES> static int go_tile(const TileArgs &a, hipStream
 // and narrower outputs leave its tiles few slabs and many epilogues: 28000, 1280, 320 + GELU: 48.0 / 49.4 us (linear_dma.hip /
 // here) with all rows live, 23.6 / 30.5 with 0.44 of them; 16640, 2048, 512 + GELU: 57.4 / 52.3 and 25.8 / 25.8; 16640, 512,
 // 2048: 58.1 / 47.0 and 22.5 / 24.6; 32896, 768, 192 + GELU: 23.7 / 30.5.
-// Above that it depends on the live rows, which only the device knows where they are packed (rows_dev): routed samples keep 7 of
-// 16 (regions of 16, 4 and 1 queries alike), untrained routers all of them, and a rule has to serve both.
-//   * Outputs that linear_dma.hip gives 128x128 tiles: while those fill the chip once at most and the 64x128 tiles of this kernel
-//     do not, its 128x128 tiles are slower (four waves against eight and four loaders): 4500 live rows of 768, 3072 + residual
-//     28.4 / 33.6, of 768, 768 + residual 11.9 / 14.5.  Taken from where 7 of 16 rows are past that, short K from twice as much on:
-//     12850 rows of 768, 3072 with 7 of 16 live 51.8 / 46.3, all 82.5 / 66.7; 25769 of 768, 768 + residual 29.6 / 26.8, 49.5 / 49.3.
-//     (A quarter of the rows live costs up to a fifth there: 14872 of 768, 3072: 27.6 / 33.3.)
-//   * Wider ones, 128x256 there: all rows live, always (28 sizes from 2056 to 40000 rows: 1536, 768 mean 0.92, the worst 1.01;
-//     2048, 1024 0.91, 1.04; 3072, 1536 0.88, 1.03).  Packed, 3072, 768 + GELU: with 7 of 16 and with all live 2056: 12.4 / 14.4, 27.6
-//     / 23.7; 3976: 17.8 / 19.8, 32.8 / 31.2; 4954: 29.5 / 24.0, 34.7 / 37.7; from there on the mean of 20 sizes is 0.98 (0.80 to 1.14), with 4096, 1024 0.92.
-// A pass of the 768-channel model, us, without this kernel / with it wherever K and N allow / so (256 px pictures): 5: 1033 / 1014 /
-// 1018; 12: 1496 / 1488 / 1499; 20: 1737 / 1694 / 1722; 32: 1977 / 2013 / 1981; 60: 2886 / 2943 / 2907; 64: 3108 / 3048 / 2999; 99: 4399 /
-// 4276 / 4283; 128: 5447 / 5175 / 5187.
-bool linear_tile_wanted(int64_t lda, bool packed, int64_t rows, int N, int K, int act, const void *res)
+// From 768 on, us of a launch inside a pass of the 768-channel model (256 px pictures of 257 rows, the mean of its blocks, whose
+// live rows are about 7 in 16), linear_dma.hip / here, at 8, 20, 44, 64, 99 and 128 pictures:
+//   keys and values (1536, 768, all rows live): 16.9 / 14.3, 25.1 / 22.7, 43.9 / 37.7, 55.2 / 49.0, 75.7 / 71.0, 98.4 / 89.8
+//   queries (768, 768):             10.0 / 9.7, 10.6 / 10.4, 16.8 / 13.8, 18.3 / 16.6, 24.7 / 21.4, 28.1 / 25.0; 40: 13.3 / 13.4
+//   proj (768, 768 + residual):     10.6 / 10.9, 11.2 / 11.8, 15.2 / 16.6, 17.4 / 19.8, 25.2 / 27.3, 30.2 / 32.2
+//   fc1 (3072, 768 + GELU):         13.6 / 15.1, 23.4 / 22.7, 36.4 / 36.6, 44.6 / 46.2, 64.4 / 68.0, 79.6 / 84.0
+//   fc2 (768, 3072 + residual):     26.3 / 25.1, 28.8 / 26.8, 39.9 / 37.4, 46.0 / 44.3, 67.5 / 59.3, 80.6 / 71.0; 32: 31.3 / 31.6
+// A long epilogue behind a short K costs four waves more than the products gain.  Launches one behind the other, with their
+// operands in the caches, say more for this kernel (fc1 77.0 / 74.7 at 99 pictures) except in one band: where the 128x128 tiles of
+// linear_dma.hip fill the chip once at most and 64x128 here do not, long K lose a fifth (4000 live rows of 768, 3072: 27.1 / 32.7).
+// Routed samples differ and only touch it (20 pictures: 28.8 / 26.8); with all rows live - an untrained router - outputs of 2 to 4 M
+// values lie in it altogether and are left out.  So are keys and values of 5 to 7.5 M, where 128x128 tiles there are one and a half
+// rounds (14 to 18 pictures: 18.7 / 19.3).  Wider K, launches one behind the other: 4096, 1024 + GELU: 0.91 of linear_dma.hip on average over 28 sizes with a quarter
+// to all rows live, 2048, 1024 and 3072, 1536 0.91 and 0.88.
+// A pass, us, without this kernel / with it wherever K and N allow / so: 5 pictures: 1034 / 1026 / 1029; 16: 1593 / 1571 / 1593; 32:
+// 1958 / 1994 / 1972; 44: 2574 / 2477 / 2470; 60: 2814 / 2892 / 2831; 80: 3512 / 3534 / 3474; 99: 4234 / 4147 / 4088; 128: 5152 / 4974 /
+// 4894.
+bool linear_tile_wanted(int64_t lda, int64_t rows, int N, int K, int act, const void *res)
 {
     if (rows < 2048 || N < 768 || K < 768 || K % 64 != 0 || (act != VTDGE_ACT_NONE && res != nullptr) || rows >= (1ll << 30) ||
         lda >= (1 << 23) || K >= (1 << 23) || compute_units() != 256)      // its rounds are counted for a workgroup on each of 256
         return false;
-    const int64_t live = (packed ? rows * 7 / 16 : rows) * N;
-    if (N < 1536 || K >= 2048 || res != nullptr) return live >= (K >= 1536 ? 1ll << 22 : 1ll << 23);
-    return !packed || live >= 6ll << 20;
+    if ((act != VTDGE_ACT_NONE && K < 1024) || (res != nullptr && K < 1536)) return false;
+    const bool square = N < 1536 || K >= 2048 || res != nullptr;           // 128x128 tiles there
+    const int64_t out = rows * N, M = 1 << 20;
+    if (square) return K >= 1536 ? out <= 2 * M || out > 4 * M : out >= 8 * M;
+    return K >= 1024 || out <= 5 * M || out > 7 * M + M / 2;
 }
 
 int launch_linear_tile(const void *A, int64_t lda, const void *W, const void *bias, const void *res, int64_t ldr, void *out,
