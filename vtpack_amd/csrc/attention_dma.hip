@@ -607,8 +607,9 @@ int launch_attention_split(const void *q, int64_t q_rs, int64_t q_hs, const void
                            int h, int n, int max_rows, float scale, hipStream_t st);
 
 // Chunks that the resident kernel deals a pair's queries out in.  What a compute unit goes through, in tiles of a wave: its
-// items, each of them a share of the tiles (a third of what max_rows allows, as routed samples have) and one for bringing keys
-// and values in; a pair stays whole unless that says a tenth less, and where it has no sixteen tiles.  Us, whole / dealt out
+// items, each of them a share of the tiles and one for bringing keys and values in; a pair has a third of the tiles that max_rows
+// allows, as in the models, which hand over a sample's tokens (the operators hand over the longest sample's queries, which are
+// dealt out as if there were a third of them); a pair stays whole unless that says a tenth less, and where it has no sixteen tiles.  Us, whole / dealt out
 // (pairs, keys, rows a sample may have, has on average): 8, 256, 16384, 6000: 117.1 / 10.6; 24: 127.3 / 25.0; 140: 133.4 / 98.1;
 // 48, 256, 4096, 1500: 35.8 / 15.9; 120, 256, 1024, 400: 14.1 / 11.2; 12, 64, 4096, 1500: 21.0 / 6.9; 100: 26.7 / 17.5; 300:
 // 50.4 / 43.2.  Kept whole, whole / two chunks: 256, 64, 4096, 1500: 30.7 / 32.1; 512, 64, 1024, 380: 19.6 / 23.9; 300, 257, 257,

@@ -99,12 +99,13 @@ FUSE_TAIL = True
 NATIVE_CHAIN = True
 # Values of a natively issued chain (tokens times channels) from which the routing half of a block goes to a second
 # stream, where the block has no folded kernels.  Below, the fork and the join cost more than the overlap gives: one
-# stream against two, GPU time of a forward, us: 1030 against 1088 (five 256 px pictures, 768 channels), 1505 against 1561
-# (12, 384 channels fp32).  Far above it gives more: 4531 against 4509 (99, 768 channels), 3203 against 3134 (128,
-# PVT-Small), 5176 against 5003 (256).  From the line to some 16 M values it depends on the model: 1698 against 1667 (12 of
-# 384 px, PVT-Tiny fp32), 2600 against 2545 (24), but 1737 against 1787 (32, PVT-Small) and, where few regions route the
-# next block in their scatter-back (`vtdge_region_step`) so that only the first block forks, 1462 against 1515 (12, 768
-# channels) and 2907 against 2926 (128, 192 channels fp32).
+# stream against two, GPU time of a forward, us: 1030 against 1088 (five 256 px pictures, 768 channels), 1419 against 1487
+# (12, 384 channels fp32).  Far above it gives more: 4098 against 4063 (99, 768 channels; the Linear of keys and values takes all
+# of a compute unit's LDS there, so that `patch_write` waits for its first workgroups and takes 14 us, not 10), 4885 against 4825
+# (128), 3110 against 3016 (128, PVT-Small), 5052 against 4946 (256).  From the line to some 16 M values it depends on the
+# model: 2402 against 2353 (24 of 384 px, PVT-Tiny fp32), but 1580 against 1589 (12), 1673 against 1725 (32, PVT-Small) and,
+# where few regions route the next block in their scatter-back (`vtdge_region_step`) so that only the first block forks, 1445
+# against 1497 (12, 768 channels), 2849 against 2872 (64) and 2690 against 2716 (128, 192 channels fp32).
 OVERLAP_FROM = 2 << 20
 _SWITCHES = ("OVERLAP", "FUSE_NEXT_NORM", "FUSE_ROUTER_NORM", "FUSE_NEXT_ROUTER", "FOLD_NORMS", "FUSE_PATCH_EMBED",
              "ROUTING_ON_SIDE", "Q_AFTER_JOIN", "REGION_COMPRESS", "SERIAL_BESIDE_WEIGHT_STATIONARY", "ROUTING_FIRST",
