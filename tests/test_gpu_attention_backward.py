@@ -298,11 +298,12 @@ def test_scores_kept_between_the_walks(dev, n):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,h", [(2051, 1), (1023, 8), (1025, 8), (4, 12)])
-def test_workgroups_find_their_queries(dev, dtype, B, h):
+@pytest.mark.parametrize("n", [20, 65, 130])       # searched for from 128 keys on; key chunks pair by pair and chunk by chunk
+def test_workgroups_find_their_queries(dev, dtype, B, h, n):
     """Ragged batches whose workgroups look through several steps of pairs for theirs, or through none: the bits of the same
     samples in calls of 16 (of 2), whose pairs are found in the first step, and a few samples, longest and last, against float64."""
     from vtpack_amd.layers.sparse_ops import sparse_attention_train
-    n, d = 20, 64
+    d = 64
     g = torch.Generator(dev).manual_seed(B)
     lengths = torch.randint(0, 9, (B,), generator=torch.Generator().manual_seed(h))
     lengths[::97] = 130
@@ -336,3 +337,30 @@ def test_workgroups_find_their_queries(dev, dtype, B, h):
         # (fp32: few workgroups have a forward kernel of their own, whose sums are in another order: a few roundings of 2^-24)
         assert torch.equal(o, out[at:to]) if dtype == torch.bfloat16 else float((o - out[at:to]).abs().max()) <= 2 ** -19
         assert torch.equal(q1, dq[:, at:to]) and torch.equal(k1, dk[:, b:e]) and torch.equal(v1, dv[:, b:e])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("low,high", [(1, 66), (60, 66), (128, 131)])
+def test_a_grid_with_holes_and_one_without(dev, dtype, low, high):
+    """As many pairs as the forward pass of bf16 searches for, too, with lengths that leave half the grid empty or none of it: the bits of
+    the same samples fifteen at a time, which the grid as it stands serves."""
+    from vtpack_amd.layers.sparse_ops import sparse_attention_train
+    B, h, n = 360, 8, 129
+    g = torch.Generator(dev).manual_seed(high)
+    lengths = torch.randint(low, high, (B,), generator=torch.Generator().manual_seed(low))
+    lengths[::90] = high - 1
+    L = int(lengths.sum())
+    q, go = (torch.randn(L, h, 64, generator=g, device=dev).to(dtype) for _ in range(2))
+    k, v = (torch.randn(h, B, n, 64, generator=g, device=dev).to(dtype) for _ in range(2))
+
+    def run(at, to, b, e):
+        args = [q[at:to].transpose(0, 1).requires_grad_(True), k[:, b:e].clone().requires_grad_(True), v[:, b:e].clone().requires_grad_(True)]
+        out = sparse_attention_train(*args, lengths[b:e], 0.125)
+        return out.detach(), *torch.autograd.grad(out, args, go[at:to].reshape(out.shape))
+    out, dq, dk, dv = run(0, L, 0, B)
+    for b in range(0, B, 15):
+        at, to = int(lengths[:b].sum()), int(lengths[:b + 15].sum())
+        o, q1, k1, v1 = run(at, to, b, b + 15)
+        # (fp32: few workgroups have a forward kernel of their own, as above)
+        assert torch.equal(o, out[at:to]) if dtype == torch.bfloat16 else float((o - out[at:to]).abs().max()) <= 2 ** -19
+        assert torch.equal(q1, dq[:, at:to]) and torch.equal(k1, dk[:, b:b + 15]) and torch.equal(v1, dv[:, b:b + 15])

@@ -150,6 +150,8 @@ struct AttnBack {
     int64_t q_rs, q_hs, kv_bs, kv_ts, kv_hs, o_rs, o_hs, dq_rs, dq_hs, dkv_bs, dkv_ts, dkv_hs, L;
     int pairs, h, n;
     float scale, scale_log2;
+    bool search;                                          // see find_chunk
+    bool by_chunk;                                        // see attention_dkv_kernel
 };
 
 // the stages of two operands' rows in LDS: `rows` of them from base0 / base1 with the given row pitches in bytes
@@ -192,16 +194,28 @@ __device__ __forceinline__ void load_kept(typename BackMath<T>::Frag (&f)[BackTi
     }
 }
 
-// The (sample, head) pair and the chunk of 64 of its queries that this workgroup takes.  The pairs of an XCD (8 i + xcd) lie one
-// behind the other with as many workgroups each as it has chunks, found from the samples' offsets: a grid with room for the
-// longest sample's chunks in every pair, taken as it stands, leaves holes that the dispatcher deals out like work, and the last
-// live workgroups start when the first have ended (us, 64 samples, 3 heads, 257 keys, fp32: 72.6 -> 45.9; 128, 6, bf16: 45.9 ->
-// 41.9).  More pairs than are looked through in a few steps keep to that grid.
-constexpr int AB_SEARCH = 1024;
-__device__ __forceinline__ bool find_chunk(const int64_t *offsets, int pairs, int h, int &pair, int &chunk, int64_t &row0, int &Lb)
+// The (sample, head) pair and the chunk of 64 of its queries that this workgroup takes: from a grid with room for the longest
+// sample's chunks in every pair, as it stands, or searched for: the pairs of an XCD (8 i + xcd) lie one behind the other then with as
+// many workgroups each as they have chunks, found from the samples' offsets.  The holes of the grid as it stands are dealt out by
+// the dispatcher like work, and the last live workgroups start when the first have ended; the search costs a workgroup 1 to 1.5
+// us, and that again for every 256 pairs of the XCD.  So it pays for the queries' gradients where there are holes, more
+// workgroups than compute units and enough keys (us inside a training pass, grid as it stands / searched; samples, heads, keys): fp32 64,
+// 3, 257: 63.4 / 46.3; 16, 6, 257: 42.4 / 31.0; 30, 5, 144: 25.9 / 20.5; 30, 3, 256: 73.6 / 63.7; bf16 128, 6, 257: 45.8 / 43.4; 60, 5,
+// 401: 43.6 / 39.5; 30, 3, 256: 26.5 / 22.9; and costs where there are not (launches one behind the other, both kernels): bf16 1024, 8, 20: 46.9 /
+// 67.0; 600, 12, 65: 134 / 162; 100, 8, 65 (inside a pass): 12.0 / 13.0; 128, 3, 257, no holes: 68.1 / 73.1; 4, 3, 257: 19.7 /
+// 21.1.  For the forward pass from 4096 workgroups on: 256, 6, 257: 46.6 / 39.8; with fewer 64, 6, 257: 16.0 / 17.2; 16, 6, 257: 10.4 /
+// 11.0; 64, 3, 257, no holes: 13.8 / 16.0; 2000, 4, 17: 12.7 / 35.1.
+constexpr int AB_SEARCH = 1024;                           // pairs of an XCD that are looked through
+// whether a grid of `chunks` for each pair has holes worth a search, with L queries in all: half a chunk of every pair is lost anyhow
+__host__ __device__ __forceinline__ bool has_holes(int64_t L, int64_t pairs, int h, int64_t chunks)
+{
+    return (L * h / (16 * AB_WAVES) + pairs / 2) * 100 < pairs * chunks * 88;
+}
+__device__ __forceinline__ bool find_chunk(bool search, const int64_t *offsets, int pairs, int h, int &pair, int &chunk, int64_t &row0,
+                                           int &Lb)
 {
     const int rest = blockIdx.x >> 3, xcd = blockIdx.x & 7, pairs_x = (pairs + 7) / 8;
-    if (pairs_x > AB_SEARCH) {
+    if (!search) {
         pair = (rest % pairs_x) * 8 + xcd;
         chunk = rest / pairs_x;
         if (pair >= pairs) return false;
@@ -263,7 +277,7 @@ __device__ __forceinline__ bool find_chunk(const int64_t *offsets, int pairs, in
 // the scale, and take their reference score from the first 32 keys, so that a row whose first scores are all -infinity comes
 // out as NaN.  Here a query's reference is its running maximum; until a finite score comes there is none and nothing is
 // added.  The row sum is taken of the probabilities as rounded for the product with the values.
-__global__ __launch_bounds__(256, 4) void attention_train_kernel(AttnTrain a)
+template <bool SEARCH> __global__ __launch_bounds__(256, 4) void attention_train_kernel(AttnTrain a)
 {
     using B = BackTile<bf16_t>;
     using M = BackMath<bf16_t>;
@@ -271,7 +285,8 @@ __global__ __launch_bounds__(256, 4) void attention_train_kernel(AttnTrain a)
     __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * B::HALF];
     int pair, chunk, Lb;
     int64_t row0;
-    if (!find_chunk(a.offsets, a.pairs, a.h, pair, chunk, row0, Lb)) return;
+    const bool search = SEARCH && has_holes(a.offsets[a.pairs / a.h], a.pairs, a.h, (int)(gridDim.x >> 3) / ((a.pairs + 7) / 8));
+    if (!find_chunk(search, a.offsets, a.pairs, a.h, pair, chunk, row0, Lb)) return;
     const int b = pair / a.h, head = pair - b * a.h;
     const int lane = threadIdx.x & 63, l = lane & 15, g = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -344,7 +359,7 @@ template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 
     __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * B::HALF];
     int pair, chunk, Lb;
     int64_t row0;
-    if (!find_chunk(a.offsets, a.pairs, a.h, pair, chunk, row0, Lb)) return;
+    if (!find_chunk(a.search, a.offsets, a.pairs, a.h, pair, chunk, row0, Lb)) return;
     const int b = pair / a.h, head = pair - b * a.h;
     const int lane = threadIdx.x & 63, l = lane & 15, g = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -488,12 +503,13 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
     constexpr int DEPTH = sizeof(T) == 4 ? 3 : 4;         // stages in LDS
     __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * B::HALF];
     __shared__ __attribute__((aligned(256))) float stats[DEPTH][3][64];      // m, 1 / s and delta of a stage's rows (twice)
-    // bf16: the chunks of a pair one behind the other (39.1 us at 128 samples of 6 heads and 257 keys, 40.9 chunk by chunk); fp32
-    // the other way round (60.7 us at 64 of 3; 63.1).  Samples are taken as they come; handed over with the longest first they
+    // bf16: the chunks of a pair one behind the other (39.1 us at 128 samples of 6 heads and 257 keys, 40.9 chunk by chunk), unless
+    // a small last chunk would then always fall to the same of an XCD's 32 compute units (both kernels, 600 samples of 6 heads, 65
+    // keys: 73.6 us, chunk by chunk 66.0; of 5 queries each 64.1 and 55.6); fp32 chunk by chunk (60.7 us at 64 of 3; 63.1).  Samples are taken as they come; handed over with the longest first they
     // would take 36.0 us where they take 37.2 (bf16), and 46.2 where they take 51.6 (fp32).
     const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8, chunks = (a.n + 16 * AB_WAVES - 1) / (16 * AB_WAVES);
-    const int chunk = sizeof(T) == 4 ? rest / pairs_x : rest % chunks;
-    const int pair = (sizeof(T) == 4 ? rest % pairs_x : rest / chunks) * 8 + (blockIdx.x & 7);
+    const int chunk = a.by_chunk ? rest / pairs_x : rest % chunks;
+    const int pair = (a.by_chunk ? rest % pairs_x : rest / chunks) * 8 + (blockIdx.x & 7);
     if (pair >= a.pairs) return;
     const int b = pair / a.h, head = pair - b * a.h;
     const int64_t row0 = a.offsets[b];
@@ -586,6 +602,8 @@ template <typename T> static int launch_backward(AttnBack a, int max_rows, hipSt
     const int64_t qc = ceil_div(max_rows, 16 * AB_WAVES), kc = ceil_div(a.n, 16 * AB_WAVES);
     VT_REQUIRE(pairs_x * 8 * (qc > kc ? qc : kc) < (1ll << 31), VTDGE_ERR_UNSUPPORTED,
                "sparse_attention_backward: too many workgroups for one launch");
+    a.search = qc >= 2 && a.n >= 128 && pairs_x <= AB_SEARCH && a.pairs * qc > compute_units() && has_holes(a.L, a.pairs, a.h, qc);
+    a.by_chunk = sizeof(T) == 4 || (32 % kc == 0 && (a.n - 1) % (16 * AB_WAVES) < 8 * AB_WAVES);
     if (qc > 0) {
         // fp32, whose products bound the kernel: up to 288 keys the scores and dP of the first walk are kept for the second, the
         // same bits in three products instead of five.  Us, both kernels, worked out again / kept (samples, heads, keys): 64, 3,
@@ -684,8 +702,10 @@ extern "C" int vtdge_sparse_attention_train(const void *q, int64_t q_row_stride,
     const AttnTrain a{(const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (bf16_t *)out, offsets, q_row_stride,
                       q_head_stride, kv_batch_stride, kv_tok_stride, kv_head_stride, o_row_stride, o_head_stride, B * h, h, n,
                       scale * 1.44269504088896340736f};
-    note_kernel(reinterpret_cast<const void *>(attention_train_kernel));
-    attention_train_kernel<<<dim3((unsigned)grid), dim3(64 * AB_WAVES), 0, (hipStream_t)stream>>>(a);
+    const bool search = chunks >= 2 && n >= 128 && B * h <= 8 * AB_SEARCH && B * h * chunks >= 16 * compute_units();
+    auto kern = search ? attention_train_kernel<true> : attention_train_kernel<false>;
+    note_kernel(reinterpret_cast<const void *>(kern));
+    kern<<<dim3((unsigned)grid), dim3(64 * AB_WAVES), 0, (hipStream_t)stream>>>(a);
     return check_launch("sparse_attention_train");
 }
 
