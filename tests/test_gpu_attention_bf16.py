@@ -68,6 +68,24 @@ def test_queries_dealt_out_in_chunks(dev, h, most, lengths, n):
     assert_close(got[:2].float(), want, torch.bfloat16, f"{h} x {B} pairs of {n} keys in chunks")
 
 
+@pytest.mark.parametrize("n", [33, 257])
+@pytest.mark.parametrize("lengths", [[511, 512], [512, 512], [0, 1], [4000, 1]])
+def test_pairs_of_few_live_rows_stay_whole(dev, lengths, n):
+    """300 pairs that may have 4000 rows each, in two chunks from 1024 live rows on, on either side of that: the bits of the same pairs
+    among 600, which no rule deals out."""
+    from vtpack_amd import _lib, ops
+    h, L = 150, sum(lengths)
+    g = torch.Generator(dev).manual_seed(n)
+    q, k, v = (torch.randn(s, generator=g, device=dev).to(torch.bfloat16) for s in ((h, L, 64), (h, 2, n, 64), (h, 2, n, 64)))
+    off, _ = ops.lengths_to_offsets(torch.tensor(lengths), q.device)
+    got = ops.sparse_attention_heads(q, k, v, off, 0.125, 4000)
+    assert f"pipelined_kernel<{-(-n // 32)}, true>" in _lib.last_kernel()
+    twice = ops.sparse_attention_heads(*(torch.cat((t, t)) for t in (q, k, v)), off, 0.125, 4000)
+    assert "false>" in _lib.last_kernel() and torch.equal(got, twice[:h]) and torch.equal(got, twice[h:])
+    want = orc.attention(*(t[:2].float().cpu().numpy() for t in (q, k, v)), np.array(lengths), 0.125)
+    assert_close(got[:2].float(), want, torch.bfloat16, f"{lengths} of {n} keys")
+
+
 @pytest.mark.parametrize("n", [65, 145, 257, 401, 577])
 @pytest.mark.parametrize("size", [1.0, 4.0])
 def test_few_pairs_are_as_exact_as_many(dev, n, size):

@@ -294,7 +294,7 @@ template <int NBLK, bool CHUNKED>
 __global__ __launch_bounds__(512, 1) void sparse_attention_bf16_d64_pipelined_kernel(
     const bf16_t *__restrict__ q, int64_t q_rs, int64_t q_hs, const bf16_t *__restrict__ k,
     const bf16_t *__restrict__ v, int64_t kv_bs, int64_t kv_ts, int64_t kv_hs, const int64_t *__restrict__ offsets,
-    bf16_t *__restrict__ out, int64_t o_rs, int64_t o_hs, int n, float scale, int items, int h, int chunks)
+    bf16_t *__restrict__ out, int64_t o_rs, int64_t o_hs, int n, float scale, int items, int h, int chunks, int64_t least_rows)
 {
     constexpr int NW = 8;                   // waves
     constexpr int npad = NBLK * 32;         // the host picks the instantiation: NBLK = ceil(n / 32)
@@ -316,6 +316,10 @@ __global__ __launch_bounds__(512, 1) void sparse_attention_bf16_d64_pipelined_ke
         int64_t row0;
         int Lb, b, head, tile;      // tile: this wave's first
     };
+    if (CHUNKED && least_rows > 0 && offsets[items / (h * chunks)] < least_rows) {       // few live rows: pairs stay whole
+        items /= chunks;
+        chunks = 1;
+    }
     const int per_sample = CHUNKED ? h * chunks : h, tile_step = CHUNKED ? NW * chunks : NW;
     int64_t *t_row0 = reinterpret_cast<int64_t *>(smem + 2 * bufsz);
     int *t_len = reinterpret_cast<int *>(t_row0 + ATT_TBL);
@@ -630,6 +634,19 @@ static int resident_chunks(int pairs, int max_rows, int cus)
     return best;
 }
 
+// Live rows from which that pays where the chunks take more rounds than the pairs: the kernel, which knows them, leaves the pairs
+// whole below.  Us, whole in a kernel of its own / in chunks whatever is live / so, about 256 of 4096 rows live (pairs, keys): 260, 64:
+// 10.8 / 16.3 / 12.2; 260, 257: 19.0 / 25.9 / 20.1; 300, 257: 21.4 / 25.5 / 21.9; 150, 257: 12.7 / 14.4 / 13.2; with 1800 live rows 260,
+// 257: 89.9 / 71.8 / 72.2.  (In one round the chunks cost up to a microsecond: 100, 257, 512 rows, 128 of them live: 9.4 / 10.3; 512: 15.8 /
+// 12.5.)
+static int64_t chunked_from_rows(int pairs, int chunks, int B, int cus)
+{
+    const float whole = (float)ceil_div(pairs, cus), dealt = (float)ceil_div((int64_t)pairs * chunks, cus);
+    if (dealt <= whole) return 0;
+    // whole (t + 1) = dealt (t / chunks + 1), t tiles of a wave in a pair
+    return (int64_t)((dealt - whole) / (whole - dealt / (float)chunks) * 256.f * (float)B);
+}
+
 int launch_attention_bf16_d64(const void *q, int64_t q_rs, int64_t q_hs, const void *k, const void *v, int64_t kv_bs,
                               int64_t kv_ts, int64_t kv_hs, const int64_t *offsets, void *out, int64_t o_rs,
                               int64_t o_hs, int B, int h, int n, int max_rows, float scale, hipStream_t st)
@@ -643,6 +660,7 @@ int launch_attention_bf16_d64(const void *q, int64_t q_rs, int64_t q_hs, const v
         const size_t lds_p = 4 * (size_t)npad * 128 + ATT_TBL * 12;       // + the item table
         const int cus = compute_units();
         const int chunks = resident_chunks(B * h, max_rows, cus), items = B * h * chunks;
+        const int64_t least_rows = chunks > 1 ? chunked_from_rows(B * h, chunks, B, cus) : 0;
         dim3 grid_p((unsigned)(items < cus ? items : cus)), block_p(512);
 #define VT_ATT_PIPE(NB)                                                                                            \
     case NB: {                                                                                                     \
@@ -652,7 +670,7 @@ int launch_attention_bf16_d64(const void *q, int64_t q_rs, int64_t q_hs, const v
         note_kernel(reinterpret_cast<const void *>(kern_p)),                                                        \
         kern_p<<<grid_p, block_p, lds_p, st>>>((const bf16_t *)q, q_rs, q_hs, (const bf16_t *)k, (const bf16_t *)v, \
                                                kv_bs, kv_ts, kv_hs, offsets, (bf16_t *)out, o_rs, o_hs, n, scale,  \
-                                               items, h, chunks);                                                          \
+                                               items, h, chunks, least_rows);                                              \
         return check_launch("sparse_attention");                                                                   \
     }
         switch (npad / 32) {
