@@ -521,11 +521,13 @@ def rows_to_maps(x):
     x.permute(0, 3, 1, 2).contiguous()."""
     _need_gpu(x)
     B, H, W, C = x.shape
-    if B and (not x[0].is_contiguous() or B > 1 and x.stride(0) < H * W * C):
+    stride, rows = x.stride(), H * W * C
+    if stride[1:] != (W * C, C, 1) or B > 1 and stride[0] < rows:
         x = x.contiguous()
+        stride = x.stride()
     out = torch.empty((B, C, H, W), dtype=x.dtype, device=x.device)
-    if out.numel():
-        call("vtdge_rows_to_maps", ptr(x), max(x.stride(0), H * W * C), ptr(out), B, H * W, C, dtype_code(x), stream_ptr(),
+    if B and rows:
+        call("vtdge_rows_to_maps", x.data_ptr(), max(stride[0], rows), out.data_ptr(), B, H * W, C, dtype_code(x), stream_ptr(),
              tag=("rows_to_maps", B * H * W, C))
     return out
 
