@@ -198,7 +198,9 @@ __global__ __launch_bounds__((WGM * WGN + NWP) * 64) void linear_dma_kernel(
         slot = slot + 1 == NSTAGE ? 0 : slot + 1;
         // the fragments of step s + 1 are requested between the products of step s, one at a time: in a row they hold up the
         // products that follow by about 14 clocks each (65536, 640, 320: 44.5 -> 39.8 us; 28000, 1280, 320 + GELU: 41.2 -> 37.8;
-        // 16640, 1024, 512: 27.6 -> 26.1).  Left to itself the compiler keeps one set of registers and waits in every step.
+        // 16640, 1024, 512: 27.6 -> 26.1), except in fp32, whose products are long and few a fragment (28000, 768, 192 + GELU: 89.4 us
+        // with the fragments ahead of the products, 90.6 between; 11000, 384, 384 + residual: 38.7, 39.5).  Left to itself the
+        // compiler keeps one set of registers and waits in every step.
         u32x4 fa[2][IM], fw[2][JN];
         auto fetch = [&](int s) {
 #pragma unroll
@@ -215,12 +217,16 @@ __global__ __launch_bounds__((WGM * WGN + NWP) * 64) void linear_dma_kernel(
         fetch(0);
         __builtin_amdgcn_sched_barrier(0);
         static_for<4>([&](auto S) {
-            constexpr int s = decltype(S)::value, P = IM * JN, R = IM + JN;
+            constexpr int s = decltype(S)::value, P = IM * JN, R = ESZ == 2 ? IM + JN : 0;
+            if constexpr (s < 3 && ESZ == 4) {
+                fetch(s + 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             static_for<P>([&](auto X) {
                 constexpr int x = decltype(X)::value;
                 Slab<T>::mma(fw[s & 1][x % JN], fa[s & 1][x / JN], acc[x / JN][x % JN]);      // D = W_blk * A_blk^T
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (s < 3) {
+                if constexpr (s < 3 && ESZ == 2) {
                     static_for<(x + 1) * R / P - x * R / P>([&](auto Y) { fetch1(s + 1, x * R / P + decltype(Y)::value); });
                     __builtin_amdgcn_sched_barrier(0);
                 }
