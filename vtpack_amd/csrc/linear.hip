@@ -216,7 +216,7 @@ int launch_linear_dma_split(const void *A, int64_t lda, const void *W, const voi
                       hipStream_t st);
 
 // large tiles for bf16, long rows (linear_tile.hip)
-bool linear_tile_wanted(int64_t lda, int64_t rows, int N, int K, int act, const void *res);
+bool linear_tile_wanted(int64_t lda, bool packed, int64_t rows, int N, int K, int act, const void *res);
 int launch_linear_tile(const void *A, int64_t lda, const void *W, const void *bias, const void *res, int64_t ldr, void *out,
                        int64_t ldo, const int64_t *rows_dev, int64_t rows, int N, int K, int act, hipStream_t st);
 
@@ -466,7 +466,7 @@ extern "C" int vtdge_linear_prepacked(const void *A, int64_t lda, const void *W,
             return launch_linear_dma_split(A, lda, W, packed, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
         if (dtype == VTDGE_F32)
             return launch_linear_dma<float>(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
-        if (linear_tile_wanted(lda, rows, N, K, act, residual))
+        if (linear_tile_wanted(lda, rows_dev != nullptr, rows, N, K, act, residual))
             return launch_linear_tile(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
         return launch_linear_dma<bf16_t>(A, lda, W, bias, residual, ldr, out, ldo, rows_dev, rows, N, K, act, st);
     }

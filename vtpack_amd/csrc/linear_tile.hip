@@ -344,31 +344,32 @@ template <int ACT, bool HAS_RES> static int go_tile(const TileArgs &a, hipStream
 // 2048: 58.1 / 47.0 and 22.5 / 24.6; 32896, 768, 192 + GELU: 23.7 / 30.5.
 // From 768 on, us of a launch inside a pass of the 768-channel model (256 px pictures of 257 rows, the mean of its blocks, whose
 // live rows are about 7 in 16), linear_dma.hip / here, at 8, 20, 44, 64, 99 and 128 pictures:
-//   keys and values (1536, 768, all rows live): 16.9 / 14.3, 25.1 / 22.7, 43.9 / 37.7, 55.2 / 49.0, 75.7 / 71.0, 98.4 / 89.8
+//   keys and values (1536, 768, all rows live): 16.9 / 14.3, 25.1 / 22.7, 43.9 / 37.7, 55.2 / 49.0, 75.7 / 71.0, 98.4 / 89.8; 16: 18.7 / 19.3
 //   queries (768, 768):             10.0 / 9.7, 10.6 / 10.4, 16.8 / 13.8, 18.3 / 16.6, 24.7 / 21.4, 28.1 / 25.0; 40: 13.3 / 13.4
 //   proj (768, 768 + residual):     10.6 / 10.9, 11.2 / 11.8, 15.2 / 16.6, 17.4 / 19.8, 25.2 / 27.3, 30.2 / 32.2
 //   fc1 (3072, 768 + GELU):         13.6 / 15.1, 23.4 / 22.7, 36.4 / 36.6, 44.6 / 46.2, 64.4 / 68.0, 79.6 / 84.0
 //   fc2 (768, 3072 + residual):     26.3 / 25.1, 28.8 / 26.8, 39.9 / 37.4, 46.0 / 44.3, 67.5 / 59.3, 80.6 / 71.0; 32: 31.3 / 31.6
-// A long epilogue behind a short K costs four waves more than the products gain.  Launches one behind the other, with their
-// operands in the caches, say more for this kernel (fc1 77.0 / 74.7 at 99 pictures) except in one band: where the 128x128 tiles of
-// linear_dma.hip fill the chip once at most and 64x128 here do not, long K lose a fifth (4000 live rows of 768, 3072: 27.1 / 32.7).
-// Routed samples differ and only touch it (20 pictures: 28.8 / 26.8); with all rows live - an untrained router - outputs of 2 to 4 M
-// values lie in it altogether and are left out.  So are keys and values of 5 to 7.5 M, where 128x128 tiles there are one and a half
-// rounds (14 to 18 pictures: 18.7 / 19.3).  Wider K, launches one behind the other: 4096, 1024 + GELU: 0.91 of linear_dma.hip on average over 28 sizes with a quarter
-// to all rows live, 2048, 1024 and 3072, 1536 0.91 and 0.88.
-// A pass, us, without this kernel / with it wherever K and N allow / so: 5 pictures: 1034 / 1026 / 1029; 16: 1593 / 1571 / 1593; 32:
-// 1958 / 1994 / 1972; 44: 2574 / 2477 / 2470; 60: 2814 / 2892 / 2831; 80: 3512 / 3534 / 3474; 99: 4234 / 4147 / 4088; 128: 5152 / 4974 /
-// 4894.
-bool linear_tile_wanted(int64_t lda, int64_t rows, int N, int K, int act, const void *res)
+// These are of a card that rests between a few passes; one that runs without a rest lowers its clock, by less for the fewer
+// instructions and loads of this kernel, and fc1 is ahead here too then.  A pass without a rest, us: without this kernel / with it wherever K and N
+// allow / without proj and fc1 / without proj, which is the rule: 10 pictures: 1396 / 1386 / 1379 / 1395; 28: 2018 / 1965 / 1975 /
+// 1953; 48: 2758 / 2670 / 2702 / 2664; 64: 3257 / 3138 / 3172 / 3133; 80: 3819 / 3743 / 3779 / 3725; 99: 4560 / 4418 / 4429 / 4403; 128: 5630 /
+// 5402 / 5360 / 5373.
+// Where the 128x128 tiles of linear_dma.hip fill the chip once at most and 64x128 here do not, long K lose a fifth (4000 live rows of
+// 768, 3072: 27.1 / 32.7).  With all rows live outputs of 2 to 4 M values lie in that band altogether and are left out.  Packed rows
+// are taken: blocks of routed samples only touch it (12 to 20 pictures, a pass: 1539 / 1499 to 1723 / 1695), a router that
+// keeps every row - an untrained one - loses about 3 percent of a pass there.  Left out are also keys and values of 5 to
+// 7.5 M, where 128x128 tiles there are one and a half rounds.  Wider K, launches one behind the other: 4096, 1024 + GELU: 0.91 of
+// linear_dma.hip on average over 28 sizes with a quarter to all rows live, 2048, 1024 and 3072, 1536 0.91 and 0.88.
+bool linear_tile_wanted(int64_t lda, bool packed, int64_t rows, int N, int K, int act, const void *res)
 {
     if (rows < 2048 || N < 768 || K < 768 || K % 64 != 0 || (act != VTDGE_ACT_NONE && res != nullptr) || rows >= (1ll << 30) ||
         lda >= (1 << 23) || K >= (1 << 23) || compute_units() != 256)      // its rounds are counted for a workgroup on each of 256
         return false;
-    if ((act != VTDGE_ACT_NONE && K < 1024) || (res != nullptr && K < 1536)) return false;
-    const bool square = N < 1536 || K >= 2048 || res != nullptr;           // 128x128 tiles there
+    if (res != nullptr && K < 1536) return false;
     const int64_t out = rows * N, M = 1 << 20;
-    if (square) return K >= 1536 ? out <= 2 * M || out > 4 * M : out >= 8 * M;
-    return K >= 1024 || out <= 5 * M || out > 7 * M + M / 2;
+    if (N < 1536 || K >= 2048 || res != nullptr)                           // 128x128 tiles there
+        return K >= 1536 ? packed || out <= 2 * M || out > 4 * M : out >= 8 * M;
+    return act != VTDGE_ACT_NONE || K >= 1024 || out <= 5 * M || out > 7 * M + M / 2;
 }
 
 int launch_linear_tile(const void *A, int64_t lda, const void *W, const void *bias, const void *res, int64_t ldr, void *out,
