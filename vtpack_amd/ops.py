@@ -6,6 +6,7 @@ packed operands may stay on the device (`rows_dev`), so nothing in this module
 synchronises with the GPU.
 """
 import ctypes
+import functools
 
 import torch
 
@@ -111,6 +112,11 @@ def index_to_patch(indices, splits, region_size, num_extra_tokens, capacity=None
     return patches, offsets, lengths
 
 
+@functools.lru_cache(maxsize=256)
+def _counts_to_host(B, Hr, Wr):
+    return bool(_lib.load().vtdge_index_to_patch_host_fits(B, Hr, Wr))
+
+
 def index_to_patch_host(indices, splits, region_size, num_extra_tokens):
     """`index_to_patch` for callers that need the query counts now: (patches [capacity, 4], lengths [B] on the CPU, their
     sum).  Returns as soon as the counts have come; the patches belong to the current stream, like any result, and may
@@ -121,7 +127,7 @@ def index_to_patch_host(indices, splits, region_size, num_extra_tokens):
     B, Hr, Wr = indices.shape
     if torch.cuda.is_current_stream_capturing():
         raise RuntimeError("the query counts cannot come to the host while the stream is being captured")
-    if not _lib.load().vtdge_index_to_patch_host_fits(B, Hr, Wr):
+    if not _counts_to_host(B, Hr, Wr):
         patches, _, lengths = index_to_patch(indices, splits, region_size, num_extra_tokens)
         lengths = lengths.cpu()
         return patches, lengths, int(lengths.sum())
