@@ -354,6 +354,13 @@ template <int ACT, bool HAS_RES> static int go_tile(const TileArgs &a, hipStream
 // allow / without proj and fc1 / without proj, which is the rule: 10 pictures: 1396 / 1386 / 1379 / 1395; 28: 2018 / 1965 / 1975 /
 // 1953; 48: 2758 / 2670 / 2702 / 2664; 64: 3257 / 3138 / 3172 / 3133; 80: 3819 / 3743 / 3779 / 3725; 99: 4560 / 4418 / 4429 / 4403; 128: 5630 /
 // 5402 / 5360 / 5373.
+// What the rule costs: with 2000 to 4700 rows of 768 and about 7 in 16 live, proj here as well takes 0.5 to 1 percent off a pass (one
+// model, builds in turn; 12 pictures 1497 / 1487, three of 512 px 1607 / 1595), and from 5100 rows on it adds as much (28 pictures
+// 1892 / 1900).  But where a router keeps every row it adds 1 to 2 percent from 2570 rows on (12 pictures 1808 / 1844), and queries
+// here as well 1 more (1857); the host does not know how many rows live, so that the rule takes the smaller loss.
+// Against a pass without this kernel, at 6168 to 12336 rows and 7 in 16, all or only the coarse ones live (48 passes): level or up to 11
+// percent faster, but for one in the band below (16 pictures of 384 px, 2297 / 2265 without), where fc2 elsewhere adds 2 percent if
+// every row lives.
 // Where the 128x128 tiles of linear_dma.hip fill the chip once at most and 64x128 here do not, long K lose a fifth (4000 live rows of
 // 768, 3072: 27.1 / 32.7).  With all rows live outputs of 2 to 4 M values lie in that band altogether and are left out.  Packed rows
 // are taken: blocks of routed samples only touch it (12 to 20 pictures, a pass: 1539 / 1499 to 1723 / 1695), a router that

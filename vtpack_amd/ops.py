@@ -2,8 +2,9 @@
 
 Every function here only checks shapes, allocates outputs with torch and hands
 raw device pointers plus the current HIP stream to libvtdge.  Row counts of
-packed operands may stay on the device (`rows_dev`), so nothing in this module
-synchronises with the GPU.
+packed operands may stay on the device (`rows_dev`), so no call here waits for
+the GPU but `index_to_patch_host`, which gives counts on the host, and the first
+use of a weight whose packed copy is kept (`done_before_shared`).
 """
 import ctypes
 import functools
