@@ -1,0 +1,113 @@
+"""The fp32 gradients of the packed-query attention on the bf16 matrix instructions: stages and tiles around their edges against
+float64, and operands that a sum of three bf16 values does not cover, which the fp32 instructions have to give as before."""
+import pytest
+import torch
+
+from util import randn
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [1, 0, 16, 17, 32, 33, 47, 48, 63, 64, 65, 97, 128, 129, 200]
+HEADS = 20                                 # 300 pairs, about 440 live workgroups: more than there are compute units
+
+
+def _reference(q, k, v, g, lengths, scale):
+    """-> gradients of q, g [h, L, 64] and k, v [h, B, n, 64] in float64 on the CPU."""
+    q, k, v, g = (t.cpu().double() for t in (q, k, v, g))
+    dq, dk, dv, at = torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v), 0
+    for b, m in enumerate(lengths):
+        qb, gb = q[:, at:at + m], g[:, at:at + m]
+        p = torch.softmax(qb @ k[:, b].transpose(1, 2) * scale, -1)
+        dp = gb @ v[:, b].transpose(1, 2)
+        ds = p * (dp - (p * dp).sum(-1, keepdim=True)) * scale
+        dq[:, at:at + m] = ds @ k[:, b]
+        dk[:, b], dv[:, b] = ds.transpose(1, 2) @ qb, p.transpose(1, 2) @ gb
+        at += m
+    return dq, dk, dv
+
+
+def _operands(dev, n, lengths=LENGTHS, h=HEADS):
+    L, B = sum(lengths), len(lengths)
+    return [torch.from_numpy(randn(n + i, *s)).to(dev) for i, s in enumerate([(h, L, 64), (h, B, n, 64), (h, B, n, 64), (h, L, 64)])]
+
+
+def _run(q, k, v, g, lengths=LENGTHS, scale=0.125, kernel="attention_dq_split_kernel<"):
+    from vtpack_amd import _lib, ops
+    offsets, _ = ops.lengths_to_offsets(torch.tensor(lengths), q.device)
+    out = ops.sparse_attention_backward(q, k, v, None, g, offsets, scale, max(lengths))
+    if kernel is None:
+        assert "split" not in _lib.last_kernel(1) + _lib.last_kernel()
+    else:
+        assert kernel in _lib.last_kernel(1) and "attention_dkv_split_kernel" in _lib.last_kernel()
+    return out
+
+
+@pytest.mark.parametrize("n", [161, 176, 177, 192, 193, 256, 257, 288, 289, 320, 321, 515])
+def test_tiles_and_stages(dev, n):
+    """As far off as the fp32 instructions at most, 4.2e-7 of dQ and 3.5e-7 of dK at 257 keys, growing with the square root of
+    the keys (6.7e-7 and 4.6e-7 at 1025)."""
+    q, k, v, g = _operands(dev, n)
+    kernel = f"attention_dq_split_kernel<{9 if n <= 288 else 0}>"
+    got = _run(q, k, v, g, kernel=kernel)
+    for name, a, b in zip("qkv", got, _reference(q, k, v, g, LENGTHS, 0.125)):
+        assert float((a.cpu().double() - b).norm() / b.norm()) <= 4.2e-7 * max(1.0, n / 257) ** 0.5, name
+    assert all(torch.equal(a, b) for a, b in zip(got, _run(q, k, v, g, kernel=kernel)))      # the same bytes on every call
+
+
+@pytest.mark.parametrize("size,common", [(1.0, 0.0), (4.0, 0.0), (16.0, 0.0), (1.0, 2.0)])
+def test_as_exact_as_the_fp32_instructions(dev, size, common):
+    """Large scores, and keys and values with a common component, beside the same samples in calls that are too small for the
+    split.  A twentieth is allowed for the spread of two rms errors over 940 rows, 1 / sqrt(2 * 940) each."""
+    q, k, v, g = _operands(dev, 257)
+    q, k, v = q * size, k + common * k[:, :1, :1], v + common * v[:, :1, :1]
+    got, at, parts = _run(q, k, v, g), 0, []
+    for b, m in enumerate(LENGTHS):
+        if m > 0:
+            parts.append(_run(q[:, at:at + m].contiguous(), k[:, b:b + 1].contiguous(), v[:, b:b + 1].contiguous(), g[:, at:at + m].contiguous(),
+                              [m], kernel=None))
+        at += m
+    plain = [torch.cat([p[i] for p in parts], dim=1) for i in range(3)]
+    some = [b for b, m in enumerate(LENGTHS) if m > 0]
+    for name, a, c, w in zip("qkv", got, plain, _reference(q, k, v, g, LENGTHS, 0.125)):
+        a, w = (t if name == "q" else t[:, some] for t in (a, w))
+        assert float((a.cpu().double() - w).norm()) <= 1.05 * float((c.cpu().double() - w).norm()), name
+
+
+@pytest.mark.parametrize("scale", [-0.3, 0.0, 0.9])
+def test_other_scales(dev, scale):
+    """A scale that is not positive goes to the fp32 instructions for dQ; at zero every key has the same probability."""
+    q, k, v, g = _operands(dev, 257)
+    for a, b in zip(_run(q, k, v, g, scale=scale), _reference(q, k, v, g, LENGTHS, scale)):
+        assert float((a.cpu().double() - b).norm()) <= 2e-6 * float(b.norm())
+
+
+@pytest.mark.parametrize("of_k,of_v,of_g", [(1.0, 1.0, 1e-12), (1.0, 1.0, 1e-20), (1.0, 1e-30, 1e-5), (1.0, 1e7, 1e-10), (1.0, 1e20, 1e-20),
+                                            (1e-3, 1e-25, 1e25), (1.0, 1.0, 65536.0)])
+def test_magnitudes(dev, of_k, of_v, of_g):
+    """Gradients of every magnitude that fp32 holds come out with its relative error, also where bf16 parts would fall below the
+    smallest bf16 numbers."""
+    q, k, v, g = _operands(dev, 257)
+    k, v, g = k * of_k, v * of_v, g * of_g
+    for name, a, b in zip("qkv", _run(q, k, v, g), _reference(q, k, v, g, LENGTHS, 0.125)):
+        assert float((a.cpu().double() - b).norm() / b.norm()) <= 6e-7, name
+
+
+@pytest.mark.parametrize("which,value", [(w, x) for x in (float("inf"), float("nan")) for w in "qkvg"] + [("v", 1e30), ("g", 1e30)])
+def test_values_outside_the_split(dev, which, value):
+    """One such value in a long sample: NaN where the composition has one, and everything else as it was.  (A query or key of
+    1e30 makes scores whose last fp32 bit is more than any exponent, on either instructions.)"""
+    t = dict(zip("qkvg", _operands(dev, 257)))
+    first = sum(LENGTHS[:12])
+    if which in "qg":
+        t[which][3, first + 100, 7] = value
+    else:
+        t[which][3, 12, 256, 7] = value
+    got, want = _run(*t.values()), _reference(*t.values(), LENGTHS, 0.125)
+    for name, a, b in zip("qkv", got, want):
+        a = a.cpu().double()
+        assert torch.equal(a.isnan() | a.isinf(), b.isnan() | b.isinf()), name
+        # what the large value multiplies and the rest, each in its own 2-norm (three times the 3.5e-7 of a whole gradient of unit
+        # normals: a few elements are left; one that cancels is off by its terms' last bits, not its own)
+        huge = b.abs() >= 1e9
+        for part in (b.isfinite() & huge, b.isfinite() & ~huge):
+            assert float((a - b)[part].norm()) <= 1e-6 * float(b[part].norm()), name

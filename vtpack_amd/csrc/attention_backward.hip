@@ -206,10 +206,12 @@ __device__ __forceinline__ void load_kept(typename BackMath<T>::Frag (&f)[BackTi
 // 21.1.  For the forward pass from 4096 workgroups on: 256, 6, 257: 46.6 / 39.8; with fewer 64, 6, 257: 16.0 / 17.2; 16, 6, 257: 10.4 /
 // 11.0; 64, 3, 257, no holes: 13.8 / 16.0; 2000, 4, 17: 12.7 / 35.1.
 constexpr int AB_SEARCH = 1024;                           // pairs of an XCD that are looked through
-// whether a grid of `chunks` for each pair has holes worth a search, with L queries in all: half a chunk of every pair is lost anyhow
+// about as many chunks of 64 queries as L queries in all make: half a chunk of every pair is lost
+__host__ __device__ __forceinline__ int64_t live_chunks(int64_t L, int64_t pairs, int h) { return L * h / (16 * AB_WAVES) + pairs / 2; }
+// whether a grid of `chunks` for each pair has holes worth a search
 __host__ __device__ __forceinline__ bool has_holes(int64_t L, int64_t pairs, int h, int64_t chunks)
 {
-    return (L * h / (16 * AB_WAVES) + pairs / 2) * 100 < pairs * chunks * 88;
+    return live_chunks(L, pairs, h) * 100 < pairs * chunks * 88;
 }
 __device__ __forceinline__ bool find_chunk(bool search, const int64_t *offsets, int pairs, int h, int &pair, int &chunk, int64_t &row0,
                                            int &Lb)
@@ -351,15 +353,12 @@ template <bool SEARCH> __global__ __launch_bounds__(256, 4) void attention_train
 
 // dQ of 64 query rows of one (sample, head), with their m, 1 / s and delta.
 // HELD: stages of keys whose scores and dP stay in registers between the two walks (0: they are worked out again)
-template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 : HELD <= 5 ? 3 : 2) void attention_dq_kernel(AttnBack a)
+template <typename T, int HELD>
+__device__ __forceinline__ void attention_dq_rows(const AttnBack &a, unsigned char *smem, int pair, int chunk, int64_t row0, int Lb)
 {
     using B = BackTile<T>;
     using M = BackMath<T>;
     constexpr int DEPTH = 2;                              // stages in LDS
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * B::HALF];
-    int pair, chunk, Lb;
-    int64_t row0;
-    if (!find_chunk(a.search, a.offsets, a.pairs, a.h, pair, chunk, row0, Lb)) return;
     const int b = pair / a.h, head = pair - b * a.h;
     const int lane = threadIdx.x & 63, l = lane & 15, g = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -495,18 +494,26 @@ template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 
     if (live) M::store((T *)a.dq + (row0 + row) * a.dq_rs + (int64_t)head * a.dq_hs, dq, g);
 }
 
-// dK and dV of 64 keys of one (sample, head)
-template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void attention_dkv_kernel(AttnBack a)
+template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 : HELD <= 5 ? 3 : 2) void attention_dq_kernel(AttnBack a)
+{
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * BackTile<T>::HALF];
+    int pair, chunk, Lb;
+    int64_t row0;
+    if (!find_chunk(a.search, a.offsets, a.pairs, a.h, pair, chunk, row0, Lb)) return;
+    attention_dq_rows<T, HELD>(a, smem, pair, chunk, row0, Lb);
+}
+
+// dK and dV of 64 keys of one (sample, head), from DEPTH stages of queries in LDS and their m, 1 / s and delta (of 32 rows, twice)
+template <typename T, int DEPTH>
+__device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned char *smem, float (*stats)[3][64])
 {
     using B = BackTile<T>;
     using M = BackMath<T>;
-    constexpr int DEPTH = sizeof(T) == 4 ? 3 : 4;         // stages in LDS
-    __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * B::HALF];
-    __shared__ __attribute__((aligned(256))) float stats[DEPTH][3][64];      // m, 1 / s and delta of a stage's rows (twice)
     // bf16: the chunks of a pair one behind the other (39.1 us at 128 samples of 6 heads and 257 keys, 40.9 chunk by chunk), unless
     // a small last chunk would then always fall to the same of an XCD's 32 compute units (both kernels, 600 samples of 6 heads, 65
-    // keys: 73.6 us, chunk by chunk 66.0; of 5 queries each 64.1 and 55.6); fp32 chunk by chunk (60.7 us at 64 of 3; 63.1).  Samples are taken as they come; handed over with the longest first they
-    // would take 36.0 us where they take 37.2 (bf16), and 46.2 where they take 51.6 (fp32).
+    // keys: 73.6 us, chunk by chunk 66.0; of 5 queries each 64.1 and 55.6); fp32 chunk by chunk (60.7 us at 64 of 3 on the fp32
+    // instructions; 63.1).  Samples are taken as they come; handed over with the longest first they would take 36.0 us where
+    // they take 37.2 (bf16), and 41.0 where they take 48.2 (fp32).
     const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8, chunks = (a.n + 16 * AB_WAVES - 1) / (16 * AB_WAVES);
     const int chunk = a.by_chunk ? rest / pairs_x : rest % chunks;
     const int pair = (a.by_chunk ? rest % pairs_x : rest / chunks) * 8 + (blockIdx.x & 7);
@@ -596,6 +603,453 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
     M::store((T *)a.dv + at, dv, g);
 }
 
+template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) void attention_dkv_kernel(AttnBack a)
+{
+    constexpr int DEPTH = sizeof(T) == 4 ? 3 : 4;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * BackTile<T>::HALF];
+    __shared__ __attribute__((aligned(256))) float stats[DEPTH][3][64];
+    attention_dkv_rows<T, DEPTH>(a, smem, stats);
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// fp32 on the bf16 matrix instructions, as exact: every operand of the products is the sum of three bf16 values, of whose nine
+// partial products the six large ones are multiplied and added in fp32 (linear_dma_split.hip).  A walked row is split once by
+// its workgroup on the way into LDS (planes of bf16 rows), a kept one once in its registers, P and dS where they arise.
+//
+// What bounds both kernels are the vector instructions (the splits: 44 for a fragment of 8 values a lane; they hide behind the
+// products only in part, two of them a matrix instruction) beside 96 (72) matrix instructions of 16 clocks a wave and stage, where the
+// fp32 ones were 128 (96) of 32.  Three (two) workgroups a compute unit fill each other's waits: one buffer of parts and two barriers a
+// stage; with two buffers and one barrier 155 -> 162 us (both kernels, 64 samples, 6 heads, 257 keys), with rows by direct loads
+// into a ring of three 153, two workgroups a compute unit for dK and dV 166.  Us, fp32 / bf16 instructions, 64 samples of 3 heads,
+// 257 keys, 7352 queries: dQ 42.7 / 33.8, dK and dV 61.7 / 48.2; 112 queries each: 41.8 / 33.2 and 42.2 / 35.8.  Relative errors against
+// float64 (2-norm): dQ 4.2e-7 / 3.1e-7, dK 3.5e-7 / 2.4e-7, dV 3.3e-7 / 2.2e-7.
+//
+// The values that this is not exact for take the fp32 instructions, the whole workgroup from the start: an operand that is not zero
+// and not in [2^-60, 2^20) in size (its third part, and products of parts, would reach below the smallest bf16 and fp32 numbers;
+// infinities and NaN are out of that range too), and a result that is not zero and below 2^-80, where what P and dS lose below 2^-134
+// shows.  The other workgroups of such a sample stay here, with scores of another order of sums than those that m and s are of.
+constexpr int BS_PLANE = AB_ROWS * 128, BS_BUF = 6 * BS_PLANE;      // bytes of a plane, and of two operands' three
+
+struct BackSplit {
+    static constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};      // partial products, the small ones first
+    // place of a row's 16-byte chunk: sixteen rows at one chunk (scores) and four rows at the two chunks of a block of channels
+    // (the transposing reads) both lie in different banks
+    static __device__ __forceinline__ int slot(int row, int chunk)
+    {
+        const int p = (row >> 1) & 7;
+        return chunk ^ (((p << 1) | (p >> 2)) & 7);
+    }
+    static __device__ __forceinline__ f32x4 mma(const u32x4 &a, const u32x4 &b, const f32x4 &c) { return BackMath<bf16_t>::mma(a, b, c); }
+    static __device__ __forceinline__ void split(const float (&x)[8], u32x4 (&p)[3])
+    {
+        float r[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) r[e] = x[e];
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                p[i][e] = pack_bf16x2(r[2 * e], r[2 * e + 1]);
+                if (i < 2) {
+                    r[2 * e] -= bf16lo(p[i][e]);
+                    r[2 * e + 1] -= bf16hi(p[i][e]);
+                }
+            }
+    }
+    // whether one of the bf16 values is not zero and not in [2^-60, 2^20)
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ bool outside(const u32x4 &a, const u32x4 &b)
+    {
+        u16x2 big = {0, 0}, small = {0xffff, 0xffff};
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const u16x2 m = __builtin_bit_cast(u16x2, (e < 4 ? a[e] : b[e - 4]) & 0x7fff7fffu);
+            big = __builtin_elementwise_max(big, m);
+            small = __builtin_elementwise_min(small, (u16x2)(m - (unsigned short)1));      // zero becomes the largest
+        }
+        constexpr unsigned short LOW = (127 - 60) << 7, HIGH = (127 + 20) << 7;
+        return (big[0] > big[1] ? big[0] : big[1]) >= HIGH || (small[0] < small[1] ? small[0] : small[1]) < LOW - 1;
+    }
+    // a kept row's 64 channels: step t of a contraction takes d = 32 t + 8 g + (0 .. 7)
+    static __device__ __forceinline__ bool load_kept(u32x4 (&f)[2][3], const float *row, bool live, int g)
+    {
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const f32x4 v = live ? *reinterpret_cast<const f32x4 *>(row + 32 * t + 8 * g + 4 * j) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[4 * j + e] = v[e];
+            }
+            split(x, f[t]);
+        }
+        return outside(f[0][0], f[1][0]);
+    }
+    // the three planes of 8 channels (chunk) of a walked row
+    static __device__ __forceinline__ void store_row(unsigned char *planes, int row, int chunk, const float (&x)[8], u32x4 (&p)[3])
+    {
+        split(x, p);
+#pragma unroll
+        for (int i = 0; i < 3; i++) *reinterpret_cast<u32x4 *>(planes + i * BS_PLANE + row * 128 + slot(row, chunk) * 16) = p[i];
+    }
+    // scores of walked rows 16 blk .. with the kept rows
+    static __device__ __forceinline__ f32x4 scores(const unsigned char *planes, int blk, const u32x4 (&x)[2][3], int l, int g)
+    {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            u32x4 f[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++)
+                f[i] = *reinterpret_cast<const u32x4 *>(planes + i * BS_PLANE + (16 * blk + l) * 128 + slot(l, 4 * t + g) * 16);
+#pragma unroll
+            for (int i = 0; i < 6; i++) acc = mma(f[PA[i]], x[t][PB[i]], acc);
+        }
+        return acc;
+    }
+    // out[db] += walked rows^T p; the layout of BackMath<bf16_t>::accumulate
+    static __device__ __forceinline__ void accumulate(const unsigned char *planes, const f32x4 (&p)[2], f32x4 (&out)[4], int l, int g)
+    {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[e] = p[e / 4][e % 4];
+        u32x4 b[3];
+        split(x, b);
+        const int row = 4 * g + (l >> 2);
+        const unsigned char *src = planes + row * 128 + 8 * (l & 1);
+#pragma unroll
+        for (int db = 0; db < 4; db++) {
+            u32x4 f[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                const unsigned char *at = src + i * BS_PLANE + slot(row, 2 * db + ((l & 3) >> 1)) * 16;
+                const u32x2 lo = lds_read_tr16(at), hi = lds_read_tr16(at + 16 * 128);
+                f[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
+            }
+#pragma unroll
+            for (int i = 0; i < 6; i++) out[db] = mma(f[PA[i]], b[PB[i]], out[db]);
+        }
+    }
+    // out[db][r] is channel 16 db + 4 g + r of kept row l
+    static __device__ __forceinline__ void store(float *row, const f32x4 (&o)[4], int g)
+    {
+#pragma unroll
+        for (int db = 0; db < 4; db++) *reinterpret_cast<f32x4 *>(row + 16 * db + 4 * g) = o[db];
+    }
+    // whether a result is not finite, or not zero and below 2^-80
+    static __device__ __forceinline__ bool lost(const f32x4 (&o)[4])
+    {
+        bool odd = false;
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const float m = fabsf(o[e / 4][e % 4]);
+            odd = odd || !(m < INFINITY) || (m < 0x1p-80f && m != 0.f);
+        }
+        return odd;
+    }
+};
+
+// attention_dq_rows on split operands -> whether it could
+template <int HELD>
+__device__ __forceinline__ bool attention_dq_split_rows(const AttnBack &a, unsigned char *smem, int *odd_seen, int pair, int chunk,
+                                                        int64_t row0, int Lb)
+{
+    using S = BackSplit;
+    if (!(a.scale_log2 > 0.f)) return false;              // keys past the last: a score of -infinity, below
+    const int b = pair / a.h, head = pair - b * a.h;
+    const int tid = threadIdx.x, lane = tid & 63, l = lane & 15, g = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row = (chunk * AB_WAVES + wid) * 16 + l;
+    const bool live = row < Lb, wave_live = (chunk * AB_WAVES + wid) * 16 < Lb;
+    if (tid == 0) *odd_seen = 0;
+
+    // the keys are walked twice, as one sequence of stages; this thread's part of one: 8 channels of a key and, on the first
+    // walk (on both where nothing is held), of a value
+    const int srow = tid >> 3, schunk = tid & 7;
+    const int64_t kv_at = (int64_t)b * a.kv_bs + (int64_t)head * a.kv_hs + 8 * schunk;
+    const int stages = (a.n + AB_ROWS - 1) / AB_ROWS;
+    float rk[8], rv[8];
+    auto load_stage = [&](int u) {                        // rows past the last key repeat it
+        const int64_t at = kv_at + (int64_t)min((u < stages ? u : u - stages) * AB_ROWS + srow, a.n - 1) * a.kv_ts;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const f32x4 x = *reinterpret_cast<const f32x4 *>((const float *)a.k + at + 4 * i);
+#pragma unroll
+            for (int e = 0; e < 4; e++) rk[4 * i + e] = x[e];
+            if (HELD == 0 || u < stages) {
+                const f32x4 y = *reinterpret_cast<const f32x4 *>((const float *)a.v + at + 4 * i);
+#pragma unroll
+                for (int e = 0; e < 4; e++) rv[4 * i + e] = y[e];
+            }
+        }
+    };
+    bool odd = false;
+    const unsigned char *Ks = smem, *Vs = smem + 3 * BS_PLANE;
+    // -> whether the operands are still such as the split covers
+    auto next_stage = [&](int u) {
+        lds_barrier();                                    // the stage before has been read (before the first: odd_seen is zero)
+        const int st = u < stages ? u : u - stages;
+        if (st * AB_ROWS + AB_ROWS > a.n) {               // nothing of a repeated row
+            const bool past = st * AB_ROWS + srow >= a.n;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                rk[e] = past ? 0.f : rk[e];
+                rv[e] = past ? 0.f : rv[e];
+            }
+        }
+        u32x4 p[2][3];
+        S::store_row(smem, srow, schunk, rk, p[0]);
+        if (HELD == 0 || u < stages) S::store_row(smem + 3 * BS_PLANE, srow, schunk, rv, p[1]);
+        if (u < stages) {                                 // (the second walk meets the same keys)
+            odd = odd || S::outside(p[0][0], p[1][0]);
+            if (odd) *odd_seen = 1;
+        }
+        if (u + 1 < 2 * stages) load_stage(u + 1);
+        lds_barrier();                                    // stage u is whole
+        return u >= stages || __builtin_amdgcn_readfirstlane(*odd_seen) == 0;
+    };
+
+    load_stage(0);
+    u32x4 qf[2][3], df[2][3];
+    odd = S::load_kept(qf, (const float *)a.q + (row0 + row) * a.q_rs + (int64_t)head * a.q_hs, live, g);
+    odd = S::load_kept(df, (const float *)a.dout + (row0 + row) * a.o_rs + (int64_t)head * a.o_hs, live, g) || odd;
+    // scores and dP of a stage; of a key past the last -infinity and (its value is zero) 0: nothing that is summed below
+    auto scores = [&](int st, f32x4 (&t)[2], f32x4 (&dp)[2]) {
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            t[blk] = S::scores(Ks, blk, qf, l, g);
+            dp[blk] = S::scores(Vs, blk, df, l, g);
+        }
+        const int left = a.n - st * AB_ROWS - 4 * g;      // keys from this lane's first one on
+        if (a.n - st * AB_ROWS < AB_ROWS)
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (16 * (e / 4) + e % 4 >= left) t[e / 4][e % 4] = -INFINITY;
+    };
+    // ---- m, s and delta as in attention_dq_rows
+    float m = -INFINITY, s = 0.f, sd = 0.f;
+    f32x4 held_t[HELD > 0 ? HELD : 1][2], held_dp[HELD > 0 ? HELD : 1][2];
+    auto sums = [&](int st, f32x4 (&t)[2], f32x4 (&dp)[2]) {
+        scores(st, t, dp);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 8; e++) mx = fmaxf(mx, t[e / 4][e % 4]);
+        mx = fmaxf(m, mx * a.scale_log2);
+        const float ref = mx == -INFINITY ? 0.f : mx, down = __builtin_amdgcn_exp2f(m - ref);
+        f32x4 e[2], ed[2];
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                e[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -ref));
+                ed[blk][r] = e[blk][r] * dp[blk][r];
+            }
+        s = s * down + (((e[0][0] + e[0][1]) + (e[0][2] + e[0][3])) + ((e[1][0] + e[1][1]) + (e[1][2] + e[1][3])));
+        sd = sd * down + (((ed[0][0] + ed[0][1]) + (ed[0][2] + ed[0][3])) + ((ed[1][0] + ed[1][1]) + (ed[1][2] + ed[1][3])));
+        m = mx;
+    };
+    if constexpr (HELD > 0) {
+        bool good = true;
+        static_for<HELD>([&](auto st_c) {
+            constexpr int st = decltype(st_c)::value;
+            if (good && st < stages) {
+                good = next_stage(st);
+                if (good && wave_live) sums(st, held_t[st], held_dp[st]);
+            }
+        });
+        if (!good) return false;
+    } else {
+        for (int st = 0; st < stages; st++) {
+            if (!next_stage(st)) return false;
+            if (wave_live) sums(st, held_t[0], held_dp[0]);
+        }
+    }
+    float all = fmaxf(m, __shfl_xor(m, 16, WAVE));
+    all = fmaxf(all, __shfl_xor(all, 32, WAVE));
+    const float down = __builtin_amdgcn_exp2f(m - all);   // a lane without keys: exp2(-inf) = 0 times 0
+    s *= down;
+    sd *= down;
+    s += __shfl_xor(s, 16, WAVE);
+    sd += __shfl_xor(sd, 16, WAVE);
+    s += __shfl_xor(s, 32, WAVE);
+    sd += __shfl_xor(sd, 32, WAVE);
+    const float inv = 1.0f / s, delta = sd / s, scale_s = a.scale * inv;
+
+    // ---- dQ^T += K^T dS^T
+    f32x4 dq[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) dq[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto add = [&](const f32x4 (&t)[2], const f32x4 (&dp)[2]) {
+        f32x4 ds[2];
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                ds[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -all)) * (dp[blk][r] - delta);
+        S::accumulate(Ks, ds, dq, l, g);
+    };
+    if constexpr (HELD > 0) {
+        static_for<HELD>([&](auto st_c) {
+            constexpr int st = decltype(st_c)::value;
+            if (st < stages) {
+                next_stage(stages + st);
+                if (wave_live) add(held_t[st], held_dp[st]);
+            }
+        });
+    } else {
+        for (int st = 0; st < stages; st++) {
+            next_stage(stages + st);
+            if (!wave_live) continue;
+            scores(st, held_t[0], held_dp[0]);
+            add(held_t[0], held_dp[0]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) dq[i] *= scale_s;         // this lane's query's
+    // (a row whose scores are all -infinity, or that met a NaN, has no finite delta)
+    if (__syncthreads_or(wave_live && (S::lost(dq) || (live && !(fabsf(delta) < INFINITY))) ? 1 : 0)) return false;
+    if (!live) return true;
+    if (g == 0) {
+        const int64_t at = (int64_t)head * a.L + row0 + row;
+        a.m[at] = a.inv != nullptr ? all : all + __builtin_amdgcn_logf(s);      // v_log_f32: base 2
+        if (a.inv != nullptr) a.inv[at] = inv;
+        a.delta[at] = delta;
+    }
+    S::store((float *)a.dq + (row0 + row) * a.dq_rs + (int64_t)head * a.dq_hs, dq, g);
+    return true;
+}
+
+template <int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 3 : 2) void attention_dq_split_kernel(AttnBack a)
+{
+    static_assert(4 * BackTile<float>::HALF >= BS_BUF, "one LDS for either");
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * BackTile<float>::HALF];
+    __shared__ int odd_seen;
+    int pair, chunk, Lb;
+    int64_t row0;
+    if (!find_chunk(a.search, a.offsets, a.pairs, a.h, pair, chunk, row0, Lb)) return;
+    if (attention_dq_split_rows<HELD>(a, smem, &odd_seen, pair, chunk, row0, Lb)) return;
+    __syncthreads();
+    attention_dq_rows<float, 0>(a, smem, pair, chunk, row0, Lb);
+}
+
+// attention_dkv_rows on split operands -> whether it could
+__device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsigned char *smem, float (*stats)[AB_ROWS], int *odd_seen)
+{
+    using S = BackSplit;
+    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8;
+    const int chunk = rest / pairs_x, pair = (rest % pairs_x) * 8 + (blockIdx.x & 7);
+    if (pair >= a.pairs) return true;
+    const int b = pair / a.h, head = pair - b * a.h;
+    const int64_t row0 = a.offsets[b];
+    const int Lb = (int)(a.offsets[b + 1] - row0);
+    const int tid = threadIdx.x, lane = tid & 63, l = lane & 15, g = lane >> 4;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int key = (chunk * AB_WAVES + wid) * 16 + l;
+    const bool live = key < a.n, wave_live = (chunk * AB_WAVES + wid) * 16 < a.n;
+    if (tid == 0) *odd_seen = 0;
+
+    // this thread's part of a stage: 8 channels of a query and of its dO, and one of the 96 statistics
+    const int srow = tid >> 3, schunk = tid & 7;
+    const float *qp = (const float *)a.q + row0 * a.q_rs + (int64_t)head * a.q_hs + 8 * schunk;
+    const float *dp_ = (const float *)a.dout + row0 * a.o_rs + (int64_t)head * a.o_hs + 8 * schunk;
+    const int64_t stat = (int64_t)head * a.L + row0;
+    const int which = tid >> 5;                           // 0: m, 1: 1 / s, 2: delta
+    const float *mine = (which == 0 ? a.m : which == 1 ? a.inv : a.delta);
+    const bool brings = which < 3 && mine != nullptr;
+    float rq[8], rd[8], rs = 1.f;
+    auto load_stage = [&](int st) {                       // rows past the last query repeat it
+        const int64_t r = min(st * AB_ROWS + srow, Lb - 1);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const f32x4 x = *reinterpret_cast<const f32x4 *>(qp + r * a.q_rs + 4 * i), y = *reinterpret_cast<const f32x4 *>(dp_ + r * a.o_rs + 4 * i);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                rq[4 * i + e] = x[e];
+                rd[4 * i + e] = y[e];
+            }
+        }
+        if (brings) rs = mine[stat + min(st * AB_ROWS + (tid & 31), Lb - 1)];
+    };
+    bool odd = false;
+    auto store_stage = [&](int st) {
+        if (st * AB_ROWS + AB_ROWS > Lb) {                // nothing of a repeated row: probability zero
+            const bool past = st * AB_ROWS + srow >= Lb;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                rq[e] = past ? 0.f : rq[e];
+                rd[e] = past ? 0.f : rd[e];
+            }
+            if (st * AB_ROWS + (tid & 31) >= Lb) rs = which == 0 ? INFINITY : which == 1 ? 1.f : 0.f;
+        }
+        u32x4 p[2][3];
+        S::store_row(smem, srow, schunk, rq, p[0]);
+        S::store_row(smem + 3 * BS_PLANE, srow, schunk, rd, p[1]);
+        odd = odd || S::outside(p[0][0], p[1][0]);
+        if (which < 3) stats[which][tid & 31] = rs;
+        if (odd) *odd_seen = 1;
+    };
+
+    const int stages = (Lb + AB_ROWS - 1) / AB_ROWS;      // none for a sample without queries: its gradients are zero
+    if (stages > 0) load_stage(0);
+    u32x4 kf[2][3], vf[2][3];
+    const int64_t kv_at = (int64_t)b * a.kv_bs + (int64_t)key * a.kv_ts + (int64_t)head * a.kv_hs;
+    odd = S::load_kept(kf, (const float *)a.k + kv_at, live, g);
+    odd = S::load_kept(vf, (const float *)a.v + kv_at, live, g) || odd;
+    f32x4 dk[4], dv[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) dk[i] = dv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    const unsigned char *Qs = smem, *Ds = smem + 3 * BS_PLANE;
+    for (int st = 0; st < stages; st++) {
+        lds_barrier();                                    // the stage before has been read (before the first: odd_seen is zero)
+        store_stage(st);
+        if (st + 1 < stages) load_stage(st + 1);
+        lds_barrier();                                    // stage st is whole
+        if (__builtin_amdgcn_readfirstlane(*odd_seen) != 0) return false;
+        if (!wave_live) continue;
+        f32x4 p[2], ds[2];
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            p[blk] = S::scores(Qs, blk, kf, l, g);
+            ds[blk] = S::scores(Ds, blk, vf, l, g);
+        }
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            const int i = 16 * blk + 4 * g;
+            const f32x4 ms = *reinterpret_cast<const f32x4 *>(&stats[0][i]), iv = *reinterpret_cast<const f32x4 *>(&stats[1][i]),
+                        dl = *reinterpret_cast<const f32x4 *>(&stats[2][i]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                p[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[blk][r], a.scale_log2, -ms[r])) * iv[r];
+                ds[blk][r] = p[blk][r] * (ds[blk][r] - dl[r]);
+            }
+        }
+        S::accumulate(Ds, p, dv, l, g);
+        S::accumulate(Qs, ds, dk, l, g);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) dk[i] *= a.scale;
+    if (__syncthreads_or(odd || S::lost(dk) || S::lost(dv) ? 1 : 0)) return false;
+    if (!live) return true;
+    const int64_t at = (int64_t)b * a.dkv_bs + (int64_t)key * a.dkv_ts + (int64_t)head * a.dkv_hs;
+    S::store((float *)a.dk + at, dk, g);
+    S::store((float *)a.dv + at, dv, g);
+    return true;
+}
+
+__global__ __launch_bounds__(256, 3) void attention_dkv_split_kernel(AttnBack a)
+{
+    constexpr int DEPTH = 2;                              // of the fp32 instructions
+    static_assert(DEPTH * 2 * BackTile<float>::HALF >= BS_BUF, "one LDS for either");
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * BackTile<float>::HALF];
+    __shared__ __attribute__((aligned(256))) float stats[DEPTH][3][64];
+    __shared__ int odd_seen;
+    if (attention_dkv_split_rows(a, smem, reinterpret_cast<float(*)[AB_ROWS]>(&stats[0][0][0]), &odd_seen)) return;
+    __syncthreads();
+    attention_dkv_rows<float, DEPTH>(a, smem, stats);
+}
+
 template <typename T> static int launch_backward(AttnBack a, int max_rows, hipStream_t st)
 {
     const int64_t pairs_x = ceil_div(a.pairs, 8);
@@ -604,15 +1058,22 @@ template <typename T> static int launch_backward(AttnBack a, int max_rows, hipSt
                "sparse_attention_backward: too many workgroups for one launch");
     a.search = qc >= 2 && a.n >= 128 && pairs_x <= AB_SEARCH && a.pairs * qc > compute_units() && has_holes(a.L, a.pairs, a.h, qc);
     a.by_chunk = sizeof(T) == 4 || (32 % kc == 0 && (a.n - 1) % (16 * AB_WAVES) < 8 * AB_WAVES);
+    // fp32 on the bf16 instructions: from 161 keys on, where live workgroups are about as many as compute units (below, one wave a
+    // SIMD waits for its own vector instructions, of which the split has more).  Both kernels or neither: dK and dV take m and s of
+    // dQ's scores, and other scores, of another order of sums, would double the error of dK where they are large.  Us, fp32 / bf16
+    // instructions (samples, heads, keys): 64, 3, 257: 108.3 / 88.4; 64, 6, 257: 176.7 / 143.9; 128, 6, 257: 323 / 260; 16, 3, 1025: 377 /
+    // 269; with few live workgroups 16, 6, 257 (212): 63.7 / 60.2; 8, 3, 257 (38): 44.4 / 44.4.
+    const bool split = sizeof(T) == 4 && a.n > 5 * AB_ROWS && live_chunks(a.L, a.pairs, a.h) >= compute_units();
     if (qc > 0) {
-        // fp32, whose products bound the kernel: up to 288 keys the scores and dP of the first walk are kept for the second, the
-        // same bits in three products instead of five.  Us, both kernels, worked out again / kept (samples, heads, keys): 64, 3,
+        // fp32: up to 288 keys the scores and dP of the first walk are kept for the second, the same bits in three products
+        // instead of five.  Us, both kernels on the fp32 instructions, worked out again / kept (samples, heads, keys): 64, 3,
         // 257: 161 / 127; 128, 6, 257: 366 / 322; 64, 6, 145: 104 / 80; 64, 3, 65: 36.5 / 31.3; 8, 3, 257: 58.4 / 51.6.  bf16
         // loses more by the registers than it gains: 128, 6, 257: 86 / 101; 64, 6, 145: 30.0 / 29.4.
         auto kern = attention_dq_kernel<T, 0>;
         if constexpr (sizeof(T) == 4) {
             if (a.n <= 3 * AB_ROWS) kern = attention_dq_kernel<T, 3>;
             else if (a.n <= 5 * AB_ROWS) kern = attention_dq_kernel<T, 5>;
+            else if (split) kern = a.n <= 9 * AB_ROWS ? attention_dq_split_kernel<9> : attention_dq_split_kernel<0>;
             else if (a.n <= 9 * AB_ROWS) kern = attention_dq_kernel<T, 9>;
         }
         note_kernel(reinterpret_cast<const void *>(kern));
@@ -620,8 +1081,11 @@ template <typename T> static int launch_backward(AttnBack a, int max_rows, hipSt
         const int rc = check_launch("sparse_attention_backward");
         if (rc != VTDGE_OK) return rc;
     }
-    note_kernel(reinterpret_cast<const void *>(attention_dkv_kernel<T>));
-    attention_dkv_kernel<T><<<dim3((unsigned)(pairs_x * 8 * kc)), dim3(64 * AB_WAVES), 0, st>>>(a);
+    auto kern = attention_dkv_kernel<T>;
+    if constexpr (sizeof(T) == 4)
+        if (split) kern = attention_dkv_split_kernel;
+    note_kernel(reinterpret_cast<const void *>(kern));
+    kern<<<dim3((unsigned)(pairs_x * 8 * kc)), dim3(64 * AB_WAVES), 0, st>>>(a);
     return check_launch("sparse_attention_backward");
 }
 
