@@ -59,6 +59,16 @@ template <> struct BackMath<float> {
         }
         return acc;
     }
+    // of both operands, for a stage's 32 walked rows
+    static __device__ __forceinline__ void both_scores(const unsigned char *S0, const unsigned char *S1, const Frag (&x)[4],
+                                                       const Frag (&y)[4], f32x4 (&t)[2], f32x4 (&dp)[2], int l, int g)
+    {
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            t[blk] = scores(S0, blk, x, l, g);
+            dp[blk] = scores(S1, blk, y, l, g);
+        }
+    }
     // out[channel][kept row] += walked rows^T p, p[blk][r] = lane's value of walked row 16 blk + 4 g + r
     static __device__ __forceinline__ void accumulate(const unsigned char *S, const f32x4 (&p)[2], f32x4 (&out)[4], int l, int g)
     {
@@ -97,6 +107,33 @@ template <> struct BackMath<bf16_t> {
                       x[j], acc);
         return acc;
     }
+    // All of the stage's fragments are asked for before the first product: left to itself the compiler keeps registers for two
+    // and waits for LDS in every step.  Us, with the masks of keys past the last in the last stage alone, before / now, dQ and dK with
+    // dV (samples, heads, keys): 128, 6, 257: 48.0 / 43.0 and 44.6 / 41.9; 64, 3, 257: 18.5 / 16.3 and 16.0 / 14.7; 30, 5, 401: 28.1 / 23.7 and
+    // 21.2 / 19.4; 16, 3, 1025: 48.0 / 37.2 and 36.4 / 33.1.
+    static __device__ __forceinline__ void both_scores(const unsigned char *S0, const unsigned char *S1, const Frag (&x)[2],
+                                                       const Frag (&y)[2], f32x4 (&t)[2], f32x4 (&dp)[2], int l, int g)
+    {
+        u32x4 f[2][2][2];
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int blk = 0; blk < 2; blk++) {
+                const int at = (16 * blk + l) * 128 + BackTile<bf16_t>::slot(l, 4 * j + g) * 16;
+                f[0][blk][j] = *reinterpret_cast<const u32x4 *>(S0 + at);
+                f[1][blk][j] = *reinterpret_cast<const u32x4 *>(S1 + at);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) t[blk] = dp[blk] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int blk = 0; blk < 2; blk++) {
+                t[blk] = mma(f[0][blk][j], x[j], t[blk]);
+                dp[blk] = mma(f[1][blk][j], y[j], dp[blk]);
+            }
+    }
     static __device__ __forceinline__ u32x4 pack(const f32x4 (&p)[2])
     {
         return u32x4{pack_bf16x2(p[0][0], p[0][1]), pack_bf16x2(p[0][2], p[0][3]), pack_bf16x2(p[1][0], p[1][1]),
@@ -112,12 +149,15 @@ template <> struct BackMath<bf16_t> {
         // this lane as a source of the transposing reads: row 4 g + l / 4, channels 16 db + 4 (l % 4) .. + 3
         const int row = 4 * g + (l >> 2);
         const unsigned char *src = S + row * 128 + 8 * (l & 1);
+        u32x2 lo[4], hi[4];
 #pragma unroll
         for (int db = 0; db < 4; db++) {
             const unsigned char *at = src + BackTile<bf16_t>::slot(row, 2 * db + ((l & 3) >> 1)) * 16;
-            const u32x2 lo = lds_read_tr16(at), hi = lds_read_tr16(at + 16 * 128);
-            out[db] = mma(u32x4{lo.x, lo.y, hi.x, hi.y}, b, out[db]);
+            lo[db] = lds_read_tr16(at);
+            hi[db] = lds_read_tr16(at + 16 * 128);
         }
+#pragma unroll
+        for (int db = 0; db < 4; db++) out[db] = mma(u32x4{lo[db].x, lo[db].y, hi[db].x, hi[db].y}, b, out[db]);
     }
     // out[db][r] is channel 16 db + 4 g + r of kept row l
     static __device__ __forceinline__ void store(bf16_t *row, const f32x4 (&o)[4], int g)
@@ -387,34 +427,39 @@ __device__ __forceinline__ void attention_dq_rows(const AttnBack &a, unsigned ch
     float m = -INFINITY, s = 0.f, sd = 0.f;
     f32x4 held_t[HELD > 0 ? HELD : 1][2], held_dp[HELD > 0 ? HELD : 1][2];
     auto sums = [&](int st, f32x4 (&t)[2], f32x4 (&dp)[2]) {
-        const unsigned char *Ks = stage_at(st), *Vs = Ks + B::HALF;
-        float mx = m;
+        M::both_scores(stage_at(st), stage_at(st) + B::HALF, qf, df, t, dp, l, g);
+        // keys past the last are left out by a mask: of the last stage alone where the code of a stage is there once
+        auto add_up = [&](auto partial) {
+            constexpr bool PARTIAL = decltype(partial)::value;
+            float hi = -INFINITY, lo = INFINITY;          // (one of them times the scale is the largest)
 #pragma unroll
-        for (int blk = 0; blk < 2; blk++) {
-            t[blk] = M::scores(Ks, blk, qf, l, g);
-            dp[blk] = M::scores(Vs, blk, df, l, g);
+            for (int blk = 0; blk < 2; blk++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const bool in = st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
-                dp[blk][r] = in ? dp[blk][r] : 0.f;
-                mx = fmaxf(mx, in ? t[blk][r] * a.scale_log2 : -INFINITY);
-            }
-        }
-        // (a maximum leaves NaN out, and a lane's keys may be one that is NaN and keys past the last: those are summed too)
-        const float ref = mx == -INFINITY ? 0.f : mx, down = __builtin_amdgcn_exp2f(m - ref);
-        // a stage's eight keys in pairs first: fewer roundings in a row than key by key
-        f32x4 e[2], ed[2];
+                for (int r = 0; r < 4; r++) {
+                    const bool in = !PARTIAL || st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
+                    dp[blk][r] = in ? dp[blk][r] : 0.f;
+                    hi = fmaxf(hi, in ? t[blk][r] : -INFINITY);
+                    lo = fminf(lo, in ? t[blk][r] : INFINITY);
+                }
+            const float mx = fmaxf(m, a.scale_log2 < 0.f ? lo * a.scale_log2 : hi * a.scale_log2);
+            // (a maximum leaves NaN out, and a lane's keys may be one that is NaN and keys past the last: those are summed too)
+            const float ref = mx == -INFINITY ? 0.f : mx, down = __builtin_amdgcn_exp2f(m - ref);
+            // a stage's eight keys in pairs first: fewer roundings in a row than key by key
+            f32x4 e[2], ed[2];
 #pragma unroll
-        for (int blk = 0; blk < 2; blk++)
+            for (int blk = 0; blk < 2; blk++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const bool in = st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
-                e[blk][r] = in ? __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -ref)) : 0.f;
-                ed[blk][r] = e[blk][r] * dp[blk][r];
-            }
-        s = s * down + (((e[0][0] + e[0][1]) + (e[0][2] + e[0][3])) + ((e[1][0] + e[1][1]) + (e[1][2] + e[1][3])));
-        sd = sd * down + (((ed[0][0] + ed[0][1]) + (ed[0][2] + ed[0][3])) + ((ed[1][0] + ed[1][1]) + (ed[1][2] + ed[1][3])));
-        m = mx;
+                for (int r = 0; r < 4; r++) {
+                    const bool in = !PARTIAL || st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
+                    e[blk][r] = in ? __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -ref)) : 0.f;
+                    ed[blk][r] = e[blk][r] * dp[blk][r];
+                }
+            s = s * down + (((e[0][0] + e[0][1]) + (e[0][2] + e[0][3])) + ((e[1][0] + e[1][1]) + (e[1][2] + e[1][3])));
+            sd = sd * down + (((ed[0][0] + ed[0][1]) + (ed[0][2] + ed[0][3])) + ((ed[1][0] + ed[1][1]) + (ed[1][2] + ed[1][3])));
+            m = mx;
+        };
+        if (HELD > 0 || a.n - st * AB_ROWS < AB_ROWS) add_up(std::true_type{});
+        else add_up(std::false_type{});
     };
     auto next_stage = [&](int u) {
         Stager<T>::template wait<Stager<T>::NL>(min(total - 1 - u, DEPTH - 2));
@@ -462,11 +507,12 @@ __device__ __forceinline__ void attention_dq_rows(const AttnBack &a, unsigned ch
 #pragma unroll
         for (int blk = 0; blk < 2; blk++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const bool in = st * AB_ROWS + 16 * blk + 4 * g + r < a.n;
-                const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -all));
-                ds[blk][r] = in ? e * (dp[blk][r] - delta) * scale_s : 0.f;
-            }
+            for (int r = 0; r < 4; r++)
+                ds[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -all)) * (dp[blk][r] - delta);
+        if (HELD > 0 || a.n - st * AB_ROWS < AB_ROWS)
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (st * AB_ROWS + 16 * (e / 4) + 4 * g + e % 4 >= a.n) ds[e / 4][e % 4] = 0.f;
         M::accumulate(stage_at(stages + st), ds, dq, l, g);
     };
     if constexpr (HELD > 0) {
@@ -481,16 +527,13 @@ __device__ __forceinline__ void attention_dq_rows(const AttnBack &a, unsigned ch
         for (int st = 0; st < stages; st++) {
             next_stage(stages + st);
             if (!wave_live) continue;
-            const unsigned char *Ks = stage_at(stages + st), *Vs = Ks + B::HALF;
             f32x4 t[2], dp[2];
-#pragma unroll
-            for (int blk = 0; blk < 2; blk++) {
-                t[blk] = M::scores(Ks, blk, qf, l, g);
-                dp[blk] = M::scores(Vs, blk, df, l, g);
-            }
+            M::both_scores(stage_at(stages + st), stage_at(stages + st) + B::HALF, qf, df, t, dp, l, g);
             add(st, t, dp);
         }
     }
+#pragma unroll
+    for (int i = 0; i < 4; i++) dq[i] *= scale_s;         // this lane's query's
     if (live) M::store((T *)a.dq + (row0 + row) * a.dq_rs + (int64_t)head * a.dq_hs, dq, g);
 }
 
@@ -585,13 +628,13 @@ __device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned c
                 }
         }
         f32x4 p[2], ds[2];
+        M::both_scores(Qs, Ds, kf, vf, p, ds, l, g);
 #pragma unroll
         for (int blk = 0; blk < 2; blk++) {
-            const f32x4 t = M::scores(Qs, blk, kf, l, g), dp = M::scores(Ds, blk, vf, l, g);
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                p[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[r], a.scale_log2, -ms[blk][r])) * iv[blk][r];
-                ds[blk][r] = p[blk][r] * (dp[r] - dl[blk][r]) * a.scale;
+                p[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[blk][r], a.scale_log2, -ms[blk][r])) * iv[blk][r];
+                ds[blk][r] = p[blk][r] * (ds[blk][r] - dl[blk][r]);
             }
         }
         M::accumulate(Ds, p, dv, l, g);
@@ -599,6 +642,8 @@ __device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned c
     }
     if (!live) return;
     const int64_t at = (int64_t)b * a.dkv_bs + (int64_t)key * a.dkv_ts + (int64_t)head * a.dkv_hs;
+#pragma unroll
+    for (int i = 0; i < 4; i++) dk[i] *= a.scale;
     M::store((T *)a.dk + at, dk, g);
     M::store((T *)a.dv + at, dv, g);
 }
@@ -619,10 +664,11 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
 // What bounds both kernels are the vector instructions (the splits: 44 for a fragment of 8 values a lane; they hide behind the
 // products only in part, two of them a matrix instruction) beside 96 (72) matrix instructions of 16 clocks a wave and stage, where the
 // fp32 ones were 128 (96) of 32.  Three (two) workgroups a compute unit fill each other's waits: one buffer of parts and two barriers a
-// stage; with two buffers and one barrier 155 -> 162 us (both kernels, 64 samples, 6 heads, 257 keys), with rows by direct loads
-// into a ring of three 153, two workgroups a compute unit for dK and dV 166.  Us, fp32 / bf16 instructions, 64 samples of 3 heads,
-// 257 keys, 7352 queries: dQ 42.7 / 33.8, dK and dV 61.7 / 48.2; 112 queries each: 41.8 / 33.2 and 42.2 / 35.8.  Relative errors against
-// float64 (2-norm): dQ 4.2e-7 / 3.1e-7, dK 3.5e-7 / 2.4e-7, dV 3.3e-7 / 2.2e-7.
+// stage.  Us, both kernels, 64 samples, 6 heads, 257 keys, as this one 144: two buffers and one barrier 162, rows by direct loads into a
+// ring of three 153, two workgroups a compute unit for dK and dV 148.  Us, fp32 / bf16 instructions, dQ and dK with dV (samples,
+// heads, keys, queries): 64, 3, 257, 7352: 45.6 / 36.3 and 63.5 / 49.3; 128, 6, 257, 15262: 159 / 124 and 167 / 121; 16, 3, 1025, 7598: 191 / 128
+// and 185 / 125.  Relative errors against float64 (2-norm): dQ 4.2e-7 / 2.9e-7, dK 3.5e-7 / 2.2e-7, dV 3.3e-7 / 2.0e-7; queries four times
+// as large: 9.0e-7 / 5.1e-7, 8.8e-7 / 4.8e-7, 7.3e-7 / 3.8e-7.
 //
 // The values that this is not exact for take the fp32 instructions, the whole workgroup from the start: an operand that is not zero
 // and not in [2^-60, 2^20) in size (its third part, and products of parts, would reach below the smallest bf16 and fp32 numbers;
@@ -693,22 +739,37 @@ struct BackSplit {
 #pragma unroll
         for (int i = 0; i < 3; i++) *reinterpret_cast<u32x4 *>(planes + i * BS_PLANE + row * 128 + slot(row, chunk) * 16) = p[i];
     }
-    // scores of walked rows 16 blk .. with the kept rows
-    static __device__ __forceinline__ f32x4 scores(const unsigned char *planes, int blk, const u32x4 (&x)[2][3], int l, int g)
+    // Fragments are asked for a batch of products ahead: left to itself the compiler keeps registers for one or two and waits for LDS
+    // before nearly every product.
+    // scores of a stage's 32 walked rows of two operands with the kept rows.  The walk over the queries adds the same products in
+    // the same order as the walk over the keys, so both have the same scores to the last bit.
+    template <bool QUERIES_WALKED>
+    static __device__ __forceinline__ void both_scores(const unsigned char *S0, const unsigned char *S1, const u32x4 (&x)[2][3],
+                                                       const u32x4 (&y)[2][3], f32x4 (&t)[2], f32x4 (&dp)[2], int l, int g)
     {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        u32x4 f[2][3];
+        auto read = [&](int k) {                          // batch k: rows 16 (k / 4) .., operand k / 2 % 2, channels 32 (k % 2) ..
+            const unsigned char *at = (k & 2 ? S1 : S0) + (16 * (k >> 2) + l) * 128 + slot(l, 4 * (k & 1) + g) * 16;
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            u32x4 f[3];
+            for (int i = 0; i < 3; i++) f[k & 1][i] = *reinterpret_cast<const u32x4 *>(at + i * BS_PLANE);
+        };
+        read(0);
+        f32x4 acc[2];
+        static_for<8>([&](auto k_c) {
+            constexpr int k = decltype(k_c)::value;
+            if constexpr (k < 7) read(k + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr ((k & 1) == 0) acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < 3; i++)
-                f[i] = *reinterpret_cast<const u32x4 *>(planes + i * BS_PLANE + (16 * blk + l) * 128 + slot(l, 4 * t + g) * 16);
-#pragma unroll
-            for (int i = 0; i < 6; i++) acc = mma(f[PA[i]], x[t][PB[i]], acc);
-        }
-        return acc;
+            for (int i = 0; i < 6; i++) {
+                const u32x4 &kept = (k & 2 ? y : x)[k & 1][QUERIES_WALKED ? PA[i] : PB[i]];
+                acc[i & 1] = mma(f[k & 1][QUERIES_WALKED ? PB[i] : PA[i]], kept, acc[i & 1]);
+            }
+            if constexpr ((k & 1) == 1) (k & 2 ? dp : t)[k >> 2] = acc[0] + acc[1];
+            __builtin_amdgcn_sched_barrier(0);
+        });
     }
-    // out[db] += walked rows^T p; the layout of BackMath<bf16_t>::accumulate
+    // out[db] += walked rows^T p; the layout of BackMath<bf16_t>::accumulate (a second set of fragments gains nothing here)
     static __device__ __forceinline__ void accumulate(const unsigned char *planes, const f32x4 (&p)[2], f32x4 (&out)[4], int l, int g)
     {
         float x[8];
@@ -727,6 +788,7 @@ struct BackSplit {
                 const u32x2 lo = lds_read_tr16(at), hi = lds_read_tr16(at + 16 * 128);
                 f[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
             }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < 6; i++) out[db] = mma(f[PA[i]], b[PB[i]], out[db]);
         }
@@ -816,11 +878,7 @@ __device__ __forceinline__ bool attention_dq_split_rows(const AttnBack &a, unsig
     odd = S::load_kept(df, (const float *)a.dout + (row0 + row) * a.o_rs + (int64_t)head * a.o_hs, live, g) || odd;
     // scores and dP of a stage; of a key past the last -infinity and (its value is zero) 0: nothing that is summed below
     auto scores = [&](int st, f32x4 (&t)[2], f32x4 (&dp)[2]) {
-#pragma unroll
-        for (int blk = 0; blk < 2; blk++) {
-            t[blk] = S::scores(Ks, blk, qf, l, g);
-            dp[blk] = S::scores(Vs, blk, df, l, g);
-        }
+        S::both_scores<false>(Ks, Vs, qf, df, t, dp, l, g);
         const int left = a.n - st * AB_ROWS - 4 * g;      // keys from this lane's first one on
         if (a.n - st * AB_ROWS < AB_ROWS)
 #pragma unroll
@@ -1009,11 +1067,7 @@ __device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsi
         if (__builtin_amdgcn_readfirstlane(*odd_seen) != 0) return false;
         if (!wave_live) continue;
         f32x4 p[2], ds[2];
-#pragma unroll
-        for (int blk = 0; blk < 2; blk++) {
-            p[blk] = S::scores(Qs, blk, kf, l, g);
-            ds[blk] = S::scores(Ds, blk, vf, l, g);
-        }
+        S::both_scores<true>(Qs, Ds, kf, vf, p, ds, l, g);
 #pragma unroll
         for (int blk = 0; blk < 2; blk++) {
             const int i = 16 * blk + 4 * g;
@@ -1061,8 +1115,8 @@ template <typename T> static int launch_backward(AttnBack a, int max_rows, hipSt
     // fp32 on the bf16 instructions: from 161 keys on, where live workgroups are about as many as compute units (below, one wave a
     // SIMD waits for its own vector instructions, of which the split has more).  Both kernels or neither: dK and dV take m and s of
     // dQ's scores, and other scores, of another order of sums, would double the error of dK where they are large.  Us, fp32 / bf16
-    // instructions (samples, heads, keys): 64, 3, 257: 108.3 / 88.4; 64, 6, 257: 176.7 / 143.9; 128, 6, 257: 323 / 260; 16, 3, 1025: 377 /
-    // 269; with few live workgroups 16, 6, 257 (212): 63.7 / 60.2; 8, 3, 257 (38): 44.4 / 44.4.
+    // instructions (samples, heads, keys): 64, 3, 257: 108.3 / 84.6; 64, 6, 257: 176.7 / 144; 128, 6, 257: 323 / 250; 16, 3, 1025: 377 / 252;
+    // with few live workgroups 16, 6, 257 (212): 63.7 / 60.2; 8, 3, 257 (38): 44.4 / 44.4.
     const bool split = sizeof(T) == 4 && a.n > 5 * AB_ROWS && live_chunks(a.L, a.pairs, a.h) >= compute_units();
     if (qc > 0) {
         // fp32: up to 288 keys the scores and dP of the first walk are kept for the second, the same bits in three products
