@@ -139,10 +139,15 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
         wait_vmcnt<0>();
         block_barrier();
         const int r0 = w * RW + (mine ? grp : 0) * RG;
-        // of four rows a division or square root is taken once, in four lanes side by side
+        // of four rows a division or square root is taken once, in four lanes side by side (the rows' values by value: behind a
+        // reference the selection turns into a load through a computed address, and the array into scratch memory, which every
+        // launch pays for: DeiT-Small, one picture, a pass: 483 us; 476 without)
+        auto in_one = [&](float v0, float v1, float v2, float v3, auto f) {
+            return f(lane & 2 ? (lane & 1 ? v3 : v2) : (lane & 1 ? v1 : v0));
+        };
         auto per_row = [&](const float (&v)[RG], auto f, float (&out)[RG]) {
             if constexpr (RG == 4) {
-                const float r = f(lane & 2 ? (lane & 1 ? v[3] : v[2]) : (lane & 1 ? v[1] : v[0]));
+                const float r = in_one(v[0], v[1], v[2], v[3], f);
 #pragma unroll
                 for (int t = 0; t < RG; t++)
                     out[t] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r), t));
@@ -217,11 +222,17 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
         const unsigned char *slot = smem + ring0 + (j % ring) * WROWS * SLAB_BYTES;
         const unsigned char *As = LN ? smem + (w + NW * j) * SM_BM * SLAB_BYTES : slot;
         const unsigned char *Ws = LN ? slot : slot + SM_BM * SLAB_BYTES;
+        // all fragments are asked for before the first product: left to itself the compiler waits for two at a time (DeiT-Base, 5
+        // pictures, a pass: 999 us; 989 this way).  Not in fp32, whose products are long (PVT-Tiny, 6 of 384 px: 1272; 1283)
+        u32x4 fa[4], fw[4];
 #pragma unroll
         for (int s = 0; s < 4; s++) {
-            const u32x4 fa = *reinterpret_cast<const u32x4 *>(As + cs[s]);
-            Slab<T>::mma(*reinterpret_cast<const u32x4 *>(Ws + cs[s]), fa, ac);
+            fa[s] = *reinterpret_cast<const u32x4 *>(As + cs[s]);
+            fw[s] = *reinterpret_cast<const u32x4 *>(Ws + cs[s]);
         }
+        if constexpr (ESZ == 2) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; s++) Slab<T>::mma(fw[s], fa[s], ac);
         if (j + ring < nj) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the slot has been read
             issue(j + ring);
