@@ -222,17 +222,25 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(SmallProblem p0, 
         const unsigned char *slot = smem + ring0 + (j % ring) * WROWS * SLAB_BYTES;
         const unsigned char *As = LN ? smem + (w + NW * j) * SM_BM * SLAB_BYTES : slot;
         const unsigned char *Ws = LN ? slot : slot + SM_BM * SLAB_BYTES;
-        // all fragments are asked for before the first product: left to itself the compiler waits for two at a time (DeiT-Base, 5
-        // pictures, a pass: 999 us; 989 this way).  Not in fp32, whose products are long (PVT-Tiny, 6 of 384 px: 1272; 1283)
-        u32x4 fa[4], fw[4];
+        if constexpr (ESZ == 2) {
+            // all fragments are asked for before the first product: left to itself the compiler waits for two at a time (DeiT-Base,
+            // 5 pictures, a pass: 999 us; 989 this way).  Not in fp32, whose products are long (PVT-Tiny, 6 of 384 px: 1272; 1283)
+            u32x4 fa[4], fw[4];
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-            fa[s] = *reinterpret_cast<const u32x4 *>(As + cs[s]);
-            fw[s] = *reinterpret_cast<const u32x4 *>(Ws + cs[s]);
+            for (int s = 0; s < 4; s++) {
+                fa[s] = *reinterpret_cast<const u32x4 *>(As + cs[s]);
+                fw[s] = *reinterpret_cast<const u32x4 *>(Ws + cs[s]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < 4; s++) Slab<T>::mma(fw[s], fa[s], ac);
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const u32x4 fa = *reinterpret_cast<const u32x4 *>(As + cs[s]);
+                Slab<T>::mma(*reinterpret_cast<const u32x4 *>(Ws + cs[s]), fa, ac);
+            }
         }
-        if constexpr (ESZ == 2) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int s = 0; s < 4; s++) Slab<T>::mma(fw[s], fa[s], ac);
         if (j + ring < nj) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // the slot has been read
             issue(j + ring);
