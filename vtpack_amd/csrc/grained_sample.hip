@@ -865,13 +865,13 @@ __device__ __forceinline__ void region_records(const u32x4 (&tok)[16], int W, in
 // router sums them, and finishes with the router's Linear + argmax on the NEXT block's gate weights: the indices
 // and logits it leaves are bit for bit those of router_kernel run on `out`, without a second pass over the tokens.
 // The group of a sample's first region also scatters the sample's extra tokens.
-// STAT (one wave per region, all 64 lanes present, `act` false for lanes past the row): also writes the
-// statistics records of the 16 stored rows, `rec` pointing at the record of the region's first token.
-template <typename T, int PS, bool SUB, bool STAT = false>
+// This one also writes the statistics records of the 16 stored rows, `rec` pointing at the record of the region's
+// first token: one wave per region, all 64 lanes present, `act` false for lanes past the row.
+template <typename T, int PS, bool SUB>
 __device__ __forceinline__ void region_scatter(const T *__restrict__ in, const T *__restrict__ sub, int64_t r0,
                                                const T *__restrict__ refp, T *__restrict__ outp, int W, int C,
-                                               float (&acc)[Elem<T>::VEC], bool act = true,
-                                               u32x4 *__restrict__ rec = nullptr, float eps = 0.f)
+                                               float (&acc)[Elem<T>::VEC], bool act,
+                                               u32x4 *__restrict__ rec, float eps)
 {
     constexpr int VEC = Elem<T>::VEC;
     constexpr int STEP = 4 / PS;
@@ -883,13 +883,11 @@ __device__ __forceinline__ void region_scatter(const T *__restrict__ in, const T
         const int j0 = (dy / STEP) * PS;
         float pivot[4], st[8];
         u32x4 xr[4], ir[NJ], sr[NJ];
-        if constexpr (STAT) {
-            const u32x4 z = {0u, 0u, 0u, 0u};
+        const u32x4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
-            for (int j = 0; j < NJ; j++) ir[j] = sr[j] = z;
+        for (int j = 0; j < NJ; j++) ir[j] = sr[j] = z;
 #pragma unroll
-            for (int dx = 0; dx < 4; dx++) xr[dx] = z;
-        }
+        for (int dx = 0; dx < 4; dx++) xr[dx] = z;
         if (act) {
 #pragma unroll
             for (int j = 0; j < NJ; j++) {
@@ -926,20 +924,63 @@ __device__ __forceinline__ void region_scatter(const T *__restrict__ in, const T
             Elem<T>::unpack(packed, f);                   // as stored: what the next block's router reads
 #pragma unroll
             for (int c = 0; c < VEC; c++) acc[c] += f[c];
-            if constexpr (STAT) {
-                pivot[dx] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(f[0])));
-                float a = 0.f, q = 0.f;
+            pivot[dx] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(f[0])));
+            float a = 0.f, q = 0.f;
 #pragma unroll
-                for (int c = 0; c < VEC; c++) {
-                    const float d = f[c] - pivot[dx];
-                    a += d;
-                    q += d * d;
-                }
-                st[2 * dx] = act ? a : 0.f;
-                st[2 * dx + 1] = act ? q : 0.f;
+            for (int c = 0; c < VEC; c++) {
+                const float d = f[c] - pivot[dx];
+                a += d;
+                q += d * d;
             }
+            st[2 * dx] = act ? a : 0.f;
+            st[2 * dx + 1] = act ? q : 0.f;
         }
-        if constexpr (STAT) write_records4(st, pivot[0], pivot[1], pivot[2], pivot[3], C, eps, rec + (int64_t)dy * W * 2);
+        write_records4(st, pivot[0], pivot[1], pivot[2], pivot[3], C, eps, rec + (int64_t)dy * W * 2);
+    }
+}
+
+// The same without records, for any split, `sh` its log2.  Rows of up to 32 vectors share a wave between regions whose splits
+// differ, and a branch a split takes the region's passes one after the other, each a trip to memory: every token fetches its
+// packed row by itself instead, four tokens' at a time, a row that four tokens share from the cache after the first.  The one
+// loop also needs 122 to 131 registers where the three splits' side by side needed 156, a wave more on a SIMD.  Bound by
+// memory: measured on bf16 rows, 256 x 64 x 64 tokens of 64 channels 118.6 -> 70.5 us (3.3 -> 5.5 TB/s, the first of a
+// region's rows found by all lanes below included), 256 x 32 x 32 of 128 53.0 -> 35.4, one region a wave 256 x 16 x 16 of 768
+// 66.4 -> 56.7, of 640 60.5 -> 48.8; fp32 64 x 64 x 64 of 64 56.7 -> 35.8, 64 x 32 x 32 of 256 42.3 -> 35.1.
+template <typename T, bool SUB>
+__device__ __forceinline__ void region_scatter_any(const T *__restrict__ in, const T *__restrict__ sub, int64_t r0, int sh,
+                                                   const T *__restrict__ refp, T *__restrict__ outp, int W, int C,
+                                                   float (&acc)[Elem<T>::VEC])
+{
+    constexpr int VEC = Elem<T>::VEC;
+    const T *in0 = in + r0 * (int64_t)C, *sub0 = SUB ? sub + r0 * (int64_t)C : nullptr;
+#pragma unroll 1
+    for (int dy = 0; dy < 4; dy++) {
+        u32x4 xr[4], ir[4], sr[4];
+#pragma unroll
+        for (int dx = 0; dx < 4; dx++) {
+            const int at = (((dy >> (2 - sh)) << sh) + (dx >> (2 - sh))) * C;
+            ir[dx] = *reinterpret_cast<const u32x4 *>(in0 + at);
+            if constexpr (SUB) sr[dx] = *reinterpret_cast<const u32x4 *>(sub0 + at);
+            xr[dx] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(refp + ((int64_t)dy * W + dx) * C));
+        }
+#pragma unroll
+        for (int dx = 0; dx < 4; dx++) {
+            float r[VEC], dv[VEC];
+            Elem<T>::unpack(ir[dx], dv);
+            if constexpr (SUB) {                          // in - sub, rounded to the storage type
+                float sv[VEC];
+                Elem<T>::unpack(sr[dx], sv);
+#pragma unroll
+                for (int c = 0; c < VEC; c++) dv[c] -= sv[c];
+                Elem<T>::unpack(Elem<T>::pack(dv), dv);
+            }
+            Elem<T>::unpack(xr[dx], r);
+#pragma unroll
+            for (int c = 0; c < VEC; c++) r[c] += dv[c];
+            const u32x4 packed = Elem<T>::pack(r);
+            *reinterpret_cast<u32x4 *>(outp + ((int64_t)dy * W + dx) * C) = packed;
+            add_vector<T>(acc, packed);                   // as stored: what the next block's router reads
+        }
     }
 }
 
@@ -1064,8 +1105,10 @@ struct ChainArgs {
 // token plus their position embedding, the same for every sample).
 // HELD: a region's reads are all in flight at once and its tokens stay in registers (region_scatter_held), from which the
 // chained variant packs them.
+// Not held, at least four waves a SIMD are asked for where the loop fits into 128 registers without scratch memory; with 131
+// the compiler's own choice was three, and the largest launches above took 74 and 39 us.
 template <typename T, int GS, bool SUB, bool STAT = false, bool SCATTER = true, bool CHAIN = false, bool HELD = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HELD ? 1 : CHAIN ? 4 : 1, HELD ? 2 : CHAIN ? 4 : 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HELD ? 1 : CHAIN || !STAT ? 4 : 1, HELD ? 2 : CHAIN ? 4 : 8)))
 void decompress_route_kernel(
     const T *__restrict__ in, const T *__restrict__ sub, const int64_t *__restrict__ cur_indices,
     const int64_t *__restrict__ splits, const int64_t *__restrict__ offsets, const T *__restrict__ ref,
@@ -1112,6 +1155,25 @@ void decompress_route_kernel(
             row_b = r0 - extra;          // read for a sample's first region only
             const int cnt = cur_counts[region];
             ps = cnt == 16 ? 4 : cnt == 4 ? 2 : 1;
+        } else if (GS < WAVE && nreg % (WAVE / GS) == 0) {
+            // the wave's regions are of one sample: all lanes add up what lies before the first of them, and each group what its
+            // neighbours before it take: a group by itself would walk nreg / GS gate indices one trip to memory after the other
+            ps = split_of(region);
+            const int wl = threadIdx.x & 63, first = rr - wl / GS;
+            float before = 0.f;
+#pragma unroll 4
+            for (int r2 = wl; r2 < first; r2 += WAVE) {
+                const int ps2 = split_of((int64_t)b * nreg + r2);
+                before += (float)(ps2 * ps2);
+            }
+            float upto = (float)(ps * ps);
+#pragma unroll
+            for (int o = GS; o < WAVE; o <<= 1) {
+                const float up = __shfl_up(upto, o, WAVE);
+                if (wl >= o) upto += up;
+            }
+            row_b = offsets[b];
+            r0 = row_b + extra + (int64_t)(wave_sum(before) + upto) - ps * ps;
         } else {
             float before = 0.f;
             for (int r2 = lane; r2 < rr; r2 += GS) {
@@ -1151,9 +1213,11 @@ void decompress_route_kernel(
                 region_scatter_held<T, 2, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, tok, act, rec, eps);
             else region_scatter_held<T, 1, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, tok, act, rec, eps);
         }
-        else if (ps == 4) region_scatter<T, 4, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
-        else if (ps == 2) region_scatter<T, 2, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
-        else region_scatter<T, 1, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
+        else if constexpr (!STAT)
+            region_scatter_any<T, SUB>(inv, subv, r0, ps == 4 ? 2 : ps == 2 ? 1 : 0, ref + off, out + off, W, C, acc);
+        else if (ps == 4) region_scatter<T, 4, SUB>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
+        else if (ps == 2) region_scatter<T, 2, SUB>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
+        else region_scatter<T, 1, SUB>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
         if (rr == 0) {          // the sample's extra tokens: packed rows row_b .. row_b + extra - 1
             for (int e = 0; e < extra; e++) {
                 float d[VEC], r[VEC];
