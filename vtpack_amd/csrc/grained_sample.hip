@@ -1082,10 +1082,9 @@ __device__ __forceinline__ void region_read(const T *__restrict__ refp, int W, i
 // CHAIN = true: the kernel goes on to pack the NEXT block's queries (what vtdge_compress_regions would do in a launch
 // of its own, reading the tokens back): the wave that has just written a region's tokens and chosen its next split has
 // everything for that but the region's first packed row, which is the number of queries of ALL regions before it.
-// The workgroups pass that number along in launch order through one 64-bit status word each (two flag bits + a
-// count): a workgroup publishes the queries of its four regions ("aggregate"), looks back over the words of the
-// workgroups before it - 64 of them per step, one per lane - until it meets one that already knows its total
-// ("prefix"), adds up what lies between and publishes its own prefix.  A workgroup only ever waits for workgroups
+// The workgroups pass that number along in launch order through one 64-bit status word each (a flag bit + a count): a
+// workgroup publishes the queries of its four regions, the last of every 64 the queries of them all, and each adds up
+// the words of its own group and the sums of the groups before it.  A workgroup only ever waits for workgroups
 // with smaller numbers, which were dispatched before it and wait for nobody behind them, so the chain always moves;
 // the wait is bounded all the same (a workgroup that gives up raises the error word and places its rows past the
 // capacity, where nothing is written).  The status words must be zero at launch; nothing else of them is kept.
