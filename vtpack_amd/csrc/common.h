@@ -385,6 +385,43 @@ template <int CTRL> __device__ __forceinline__ float dpp_move(float v)
 {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
+// v + the value of lane ^ O, in both
+template <int O> __device__ __forceinline__ float add_lane_xor(float v)
+{
+    if constexpr (O == 1) return v + dpp_move<0xB1>(v);
+    else if constexpr (O == 2) return v + dpp_move<0x4E>(v);
+    else if constexpr (O == 4) return v + dpp_move<0x141>(dpp_move<0x1B>(v));     // the quad reversed, then the half row mirrored
+    else if constexpr (O == 8) return v + dpp_move<0x128>(v);                     // the row rotated by eight
+    else {
+        static_assert(O == 16, "inside half a wave");
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);                     // odd rows swapped with even rows
+    }
+}
+// Sum over the GS lanes of a row's group, returned in each of them; farthest lanes first.
+template <int GS, int NV> __device__ __forceinline__ void group_sum_n(float (&v)[NV])
+{
+    if constexpr (GS == 64) {
+        wave_sum_n<NV>(v);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            if constexpr (GS > 16) v[i] = add_lane_xor<16>(v[i]);
+            if constexpr (GS > 8) v[i] = add_lane_xor<8>(v[i]);
+            v[i] = add_lane_xor<1>(add_lane_xor<2>(add_lane_xor<4>(v[i])));
+        }
+    }
+}
+template <int GS> __device__ __forceinline__ float group_sum(float v)
+{
+    if constexpr (GS == 64) {
+        return wave_sum(v);
+    } else {
+        float one[1] = {v};
+        group_sum_n<GS, 1>(one);
+        return one[0];
+    }
+}
 // v summed over the lanes that differ in bits 2..5 of the lane number (16 of them), returned in each of them
 __device__ __forceinline__ float sum_over_lane_bits_2_to_5(float v)
 {

@@ -20,29 +20,6 @@ constexpr int MAX_IT = 3;          // 16-byte vectors per lane: C <= 64*3*VEC
 // lanes per row for a row of nvec 16-byte vectors
 static int group_size(int nvec) { return nvec > 32 ? 64 : nvec > 16 ? 32 : nvec > 8 ? 16 : 8; }
 
-// sum over the GS lanes of a row's group, returned in each of them
-template <int GS, int NV> __device__ __forceinline__ void group_sum_n(float (&v)[NV])
-{
-    if constexpr (GS == 64) {
-        wave_sum_n<NV>(v);
-    } else {
-#pragma unroll
-        for (int o = GS / 2; o > 0; o >>= 1)
-#pragma unroll
-            for (int i = 0; i < NV; i++) v[i] += __shfl_xor(v[i], o, WAVE);
-    }
-}
-template <int GS> __device__ __forceinline__ float group_sum(float v)
-{
-    if constexpr (GS == 64) {
-        return wave_sum(v);
-    } else {
-#pragma unroll
-        for (int o = GS / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-        return v;
-    }
-}
-
 // LayerNorm of NR rows at once, one 16-byte vector of each row per lane of a GS-lane group (`active` false: the
 // lane holds no channels and only takes part in the sums).  dst(t) is where the lane's vector of row t goes.
 template <typename T, int GS, int NR, class F>
