@@ -390,6 +390,18 @@ int vtdge_patch_embed(const void *images, const void *weight, const void *bias, 
 int vtdge_patch_linear(const void *tokens, const void *weight, const void *bias, void *out, int B, int H, int W, int C,
                        int P, int N, int dtype, void *stream);
 
+/* vtdge_patch_linear on LayerNorm(tokens), each token normalised on its way (norm1 in front of the spatial reduction,
+ * vtpack/models/dge/pvt_dge.py:81-83): the LayerNorm rounded to the storage type, products of C columns with fp32 sums and
+ * one rounding, as the two calls would.  Taken where vtdge_layernorm_patch_linear_fits says 1 (bf16, 64 or 128 channels,
+ * P a multiple of 256 / C); VTDGE_ERR_UNSUPPORTED otherwise.  vtdge_layernorm_patch_linear_wanted: whether it is also the
+ * faster way. */
+int vtdge_layernorm_patch_linear_fits(int B, int H, int W, int C, int P, int dtype);
+int vtdge_layernorm_patch_linear_wanted(int B, int H, int W, int C, int P, int dtype);
+int64_t vtdge_layernorm_patch_linear_workspace(int C, int P);      /* bytes, written by the call */
+int vtdge_layernorm_patch_linear(const void *tokens, const void *ln_weight, const void *ln_bias, float eps,
+                                 const void *weight, const void *bias, void *out, void *workspace, int B, int H, int W, int C,
+                                 int P, int dtype, void *stream);
+
 /* LayerNorm folded into the Linear that consumes it: out = act(LayerNorm(A) W^T + bias) computed from the raw rows
  * of A, so that nn.LayerNorm followed by nn.Linear (norm1 -> kv and norm2 -> fc1,
  * vtpack/models/dge/deit_dge.py:127-128 with :73 and :38-44) costs no pass over the rows of its own:

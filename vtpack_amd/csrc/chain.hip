@@ -46,6 +46,7 @@ struct ChainPlan {
     bool step;                     // few regions: the scatter-back also writes what the next block's norm1 wants
     bool tail;                     // narrow bf16 rows: everything behind attention as one kernel
     bool ln_kvq, ln_fc1;           // few rows: norm1 inside the kv and q Linear, norm2 inside fc1
+    bool ln_sr;                    // many rows: norm1 inside the spatial reduction
     int64_t ws_words;
     bool split[LINEARS];           // fp32 Linears on split weights
     int split_blocks;              // blocks whose weights are split in one launch, 0: none are
@@ -54,7 +55,7 @@ struct ChainPlan {
     int64_t ints_total, big_total, scratch_total;
     int64_t gate0, off0, len0, ws0, gate_sz, off_sz, len_sz, ws_sz;      // in `ints`, block i at start + i * size
     int64_t tok0, comp0, q20, pat0, tok_sz, row_sz, pat_sz;              // in `big`
-    int64_t xln, red, kv, comp_ln, q, o, q1, q1_ln, hid, rec_x[2], rec_c[2], rec2, idx[2], cnt[2], rrows[2];   // in `scratch`
+    int64_t xln, red, srw, kv, comp_ln, q, o, q1, q1_ln, hid, rec_x[2], rec_c[2], rec2, idx[2], cnt[2], rrows[2];   // in `scratch`
 };
 
 #define VT_TRY(expr)                      \
@@ -134,6 +135,7 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
     p.folded = p.by_region && c->dtype == VTDGE_BF16 && c->C == 384 && p.rows >= 2048 && c->sr == 1 &&
                c->hidden % 384 == 0 && c->hidden <= 3072;
     p.ln_kvq = !p.folded && c->sr == 1 && vtdge_layernorm_linear_wanted(p.rows, 2 * c->C, p.cap, c->C, c->C, c->dtype);
+    p.ln_sr = c->sr > 1 && vtdge_layernorm_patch_linear_wanted(c->B, c->H, c->W, c->C, c->sr, c->dtype);
     p.tail = vtdge_block_tail_wanted(p.rows, c->C, c->hidden, c->dtype);
     p.ln_fc1 = !p.folded && !p.tail && vtdge_layernorm_linear_wanted(p.cap, c->hidden, 0, 0, c->C, c->dtype);
     p.step = c->depth > 1 && c->splits_124 && vtdge_region_step_fits(c->B, c->H, c->W, c->C, c->extra, c->dtype);
@@ -169,6 +171,7 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
     const int64_t row = p.rows * c->C * p.esz;
     p.xln = p.folded ? 0 : take(row);
     p.red = c->sr > 1 ? take((int64_t)c->B * p.n_kv * c->C * p.esz) : 0;
+    p.srw = p.ln_sr ? take(vtdge_layernorm_patch_linear_workspace(c->C, c->sr)) : 0;
     p.kv = take(2 * (int64_t)c->B * p.n_kv * c->C * p.esz);
     p.comp_ln = p.folded ? 0 : take(row);
     p.q = take(row);
@@ -354,12 +357,17 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
                                               q, live, p.cap, C, P[P_N1W], P[P_N1B], c->eps1, C, VTDGE_ACT_NONE, dt,
                                               stream));
             } else {
-                if (!packed)
+                const bool ln_sr = p.ln_sr && !packed;
+                if (!packed && !ln_sr)
                     VT_TRY(vtdge_layernorm(x, P[P_N1W], P[P_N1B], xln, nullptr, p.rows, C, c->eps1, dt, stream));
                 char *src = xln;
                 if (c->sr > 1) {
                     char *red = scratch + p.red;
-                    VT_TRY(vtdge_patch_linear(xln, P[P_SRW], P[P_SRB], red, B, H, W, C, c->sr, C, dt, stream));
+                    if (ln_sr)
+                        VT_TRY(vtdge_layernorm_patch_linear(x, P[P_N1W], P[P_N1B], c->eps1, P[P_SRW], P[P_SRB], red,
+                                                            scratch + p.srw, B, H, W, C, c->sr, dt, stream));
+                    else
+                        VT_TRY(vtdge_patch_linear(xln, P[P_SRW], P[P_SRB], red, B, H, W, C, c->sr, C, dt, stream));
                     // the normalised rows take the place of LN1(x), which nothing reads any more
                     VT_TRY(vtdge_layernorm(red, P[P_SRNW], P[P_SRNB], xln, nullptr, (int64_t)B * p.n_kv, C, c->sr_eps, dt,
                                            stream));
