@@ -842,13 +842,13 @@ __device__ __forceinline__ void region_records(const u32x4 (&tok)[16], int W, in
 // router sums them, and finishes with the router's Linear + argmax on the NEXT block's gate weights: the indices
 // and logits it leaves are bit for bit those of router_kernel run on `out`, without a second pass over the tokens.
 // The group of a sample's first region also scatters the sample's extra tokens.
-// This one also writes the statistics records of the 16 stored rows, `rec` pointing at the record of the region's
-// first token: one wave per region, all 64 lanes present, `act` false for lanes past the row.
-template <typename T, int PS, bool SUB>
+// STAT (one wave per region, all 64 lanes present, `act` false for lanes past the row): also writes the
+// statistics records of the 16 stored rows, `rec` pointing at the record of the region's first token.
+template <typename T, int PS, bool SUB, bool STAT = false>
 __device__ __forceinline__ void region_scatter(const T *__restrict__ in, const T *__restrict__ sub, int64_t r0,
                                                const T *__restrict__ refp, T *__restrict__ outp, int W, int C,
-                                               float (&acc)[Elem<T>::VEC], bool act,
-                                               u32x4 *__restrict__ rec, float eps)
+                                               float (&acc)[Elem<T>::VEC], bool act = true,
+                                               u32x4 *__restrict__ rec = nullptr, float eps = 0.f)
 {
     constexpr int VEC = Elem<T>::VEC;
     constexpr int STEP = 4 / PS;
@@ -860,11 +860,13 @@ __device__ __forceinline__ void region_scatter(const T *__restrict__ in, const T
         const int j0 = (dy / STEP) * PS;
         float pivot[4], st[8];
         u32x4 xr[4], ir[NJ], sr[NJ];
-        const u32x4 z = {0u, 0u, 0u, 0u};
+        if constexpr (STAT) {
+            const u32x4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int j = 0; j < NJ; j++) ir[j] = sr[j] = z;
+            for (int j = 0; j < NJ; j++) ir[j] = sr[j] = z;
 #pragma unroll
-        for (int dx = 0; dx < 4; dx++) xr[dx] = z;
+            for (int dx = 0; dx < 4; dx++) xr[dx] = z;
+        }
         if (act) {
 #pragma unroll
             for (int j = 0; j < NJ; j++) {
@@ -901,28 +903,31 @@ __device__ __forceinline__ void region_scatter(const T *__restrict__ in, const T
             Elem<T>::unpack(packed, f);                   // as stored: what the next block's router reads
 #pragma unroll
             for (int c = 0; c < VEC; c++) acc[c] += f[c];
-            pivot[dx] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(f[0])));
-            float a = 0.f, q = 0.f;
+            if constexpr (STAT) {
+                pivot[dx] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(f[0])));
+                float a = 0.f, q = 0.f;
 #pragma unroll
-            for (int c = 0; c < VEC; c++) {
-                const float d = f[c] - pivot[dx];
-                a += d;
-                q += d * d;
+                for (int c = 0; c < VEC; c++) {
+                    const float d = f[c] - pivot[dx];
+                    a += d;
+                    q += d * d;
+                }
+                st[2 * dx] = act ? a : 0.f;
+                st[2 * dx + 1] = act ? q : 0.f;
             }
-            st[2 * dx] = act ? a : 0.f;
-            st[2 * dx + 1] = act ? q : 0.f;
         }
-        write_records4(st, pivot[0], pivot[1], pivot[2], pivot[3], C, eps, rec + (int64_t)dy * W * 2);
+        if constexpr (STAT) write_records4(st, pivot[0], pivot[1], pivot[2], pivot[3], C, eps, rec + (int64_t)dy * W * 2);
     }
 }
 
 // The same without records, for any split, `sh` its log2.  Rows of up to 32 vectors share a wave between regions whose splits
 // differ, and a branch a split takes the region's passes one after the other, each a trip to memory: every token fetches its
 // packed row by itself instead, four tokens' at a time, a row that four tokens share from the cache after the first.  The one
-// loop also needs 122 to 131 registers where the three splits' side by side needed 156, a wave more on a SIMD.  Bound by
+// loop also needs up to 128 registers where the three splits' side by side needed 156, a wave more on a SIMD.  Bound by
 // memory: measured on bf16 rows, 256 x 64 x 64 tokens of 64 channels 118.6 -> 70.5 us (3.3 -> 5.5 TB/s, the first of a
-// region's rows found by all lanes below included), 256 x 32 x 32 of 128 53.0 -> 35.4, one region a wave 256 x 16 x 16 of 768
-// 66.4 -> 56.7, of 640 60.5 -> 48.8; fp32 64 x 64 x 64 of 64 56.7 -> 35.8, 64 x 32 x 32 of 256 42.3 -> 35.1.
+// region's rows found by all lanes below included), 256 x 32 x 32 of 128 53.0 -> 35.4; fp32 64 x 64 x 64 of 64 56.7 -> 35.8.
+// One region a wave the branch is one for all lanes and reads a row once: by itself a launch gains here too (256 x 16 x 16 of
+// 768 66.4 -> 56.7), in a forward, which leaves the rows in the caches, it loses (99 pictures of 768 channels 4394 -> 4409 us).
 template <typename T, bool SUB>
 __device__ __forceinline__ void region_scatter_any(const T *__restrict__ in, const T *__restrict__ sub, int64_t r0, int sh,
                                                    const T *__restrict__ refp, T *__restrict__ outp, int W, int C,
@@ -1081,10 +1086,10 @@ struct ChainArgs {
 // token plus their position embedding, the same for every sample).
 // HELD: a region's reads are all in flight at once and its tokens stay in registers (region_scatter_held), from which the
 // chained variant packs them.
-// Not held, at least four waves a SIMD are asked for where the loop fits into 128 registers without scratch memory; with 131
-// the compiler's own choice was three, and the largest launches above took 74 and 39 us.
+// Not held, at least four waves a SIMD are asked for where several regions share a wave, whose loop fits into 128 registers
+// without scratch memory; with 131 the compiler's own choice was three, and the first two launches above took 74 and 39 us.
 template <typename T, int GS, bool SUB, bool STAT = false, bool SCATTER = true, bool CHAIN = false, bool HELD = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HELD ? 1 : CHAIN || !STAT ? 4 : 1, HELD ? 2 : CHAIN ? 4 : 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HELD ? 1 : CHAIN || GS < WAVE ? 4 : 1, HELD ? 2 : CHAIN ? 4 : 8)))
 void decompress_route_kernel(
     const T *__restrict__ in, const T *__restrict__ sub, const int64_t *__restrict__ cur_indices,
     const int64_t *__restrict__ splits, const int64_t *__restrict__ offsets, const T *__restrict__ ref,
@@ -1189,11 +1194,11 @@ void decompress_route_kernel(
                 region_scatter_held<T, 2, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, tok, act, rec, eps);
             else region_scatter_held<T, 1, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, tok, act, rec, eps);
         }
-        else if constexpr (!STAT)
+        else if constexpr (GS < WAVE)
             region_scatter_any<T, SUB>(inv, subv, r0, ps == 4 ? 2 : ps == 2 ? 1 : 0, ref + off, out + off, W, C, acc);
-        else if (ps == 4) region_scatter<T, 4, SUB>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
-        else if (ps == 2) region_scatter<T, 2, SUB>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
-        else region_scatter<T, 1, SUB>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
+        else if (ps == 4) region_scatter<T, 4, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
+        else if (ps == 2) region_scatter<T, 2, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
+        else region_scatter<T, 1, SUB, STAT>(inv, subv, r0, ref + off, out + off, W, C, acc, act, rec, eps);
         if (rr == 0) {          // the sample's extra tokens: packed rows row_b .. row_b + extra - 1
             for (int e = 0; e < extra; e++) {
                 float d[VEC], r[VEC];
