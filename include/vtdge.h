@@ -392,15 +392,17 @@ int vtdge_patch_linear(const void *tokens, const void *weight, const void *bias,
 
 /* vtdge_patch_linear on LayerNorm(tokens), each token normalised on its way (norm1 in front of the spatial reduction,
  * vtpack/models/dge/pvt_dge.py:81-83): the LayerNorm rounded to the storage type, products of C columns with fp32 sums and
- * one rounding, as the two calls would.  Taken where vtdge_layernorm_patch_linear_fits says 1 (bf16, 64 or 128 channels,
- * P a multiple of 256 / C); VTDGE_ERR_UNSUPPORTED otherwise.  vtdge_layernorm_patch_linear_wanted: whether it is also the
- * faster way. */
+ * one rounding, and with out_ln_weight / out_ln_bias (nullable together) the LayerNorm of those rows in their place, as the
+ * separate calls would.  Taken where vtdge_layernorm_patch_linear_fits says 1 (bf16, 64 or 128 channels, P a multiple of
+ * 256 / C); VTDGE_ERR_UNSUPPORTED otherwise.  vtdge_layernorm_patch_linear_wanted: whether it is also the faster way.
+ *   packed   the weight [C, P*P*C] as vtdge_layernorm_patch_pack leaves it: `count` weights one behind the other, of
+ *            C * P*P*C values each */
 int vtdge_layernorm_patch_linear_fits(int B, int H, int W, int C, int P, int dtype);
 int vtdge_layernorm_patch_linear_wanted(int B, int H, int W, int C, int P, int dtype);
-int64_t vtdge_layernorm_patch_linear_workspace(int C, int P);      /* bytes, written by the call */
+int vtdge_layernorm_patch_pack(const void *const *weights_host, int count, void *packed, int C, int P, void *stream);
 int vtdge_layernorm_patch_linear(const void *tokens, const void *ln_weight, const void *ln_bias, float eps,
-                                 const void *weight, const void *bias, void *out, void *workspace, int B, int H, int W, int C,
-                                 int P, int dtype, void *stream);
+                                 const void *packed, const void *bias, const void *out_ln_weight, const void *out_ln_bias,
+                                 float out_eps, void *out, int B, int H, int W, int C, int P, int dtype, void *stream);
 
 /* LayerNorm folded into the Linear that consumes it: out = act(LayerNorm(A) W^T + bias) computed from the raw rows
  * of A, so that nn.LayerNorm followed by nn.Linear (norm1 -> kv and norm2 -> fc1,

@@ -1,6 +1,8 @@
 """LayerNorm inside the Linear over blocks of tokens, against the two operators it stands for: the normalised tokens are the
 LayerNorm's bit for bit, so what is left is the order of fp32 sums and one rounding, bounded beside the comparison.  Sizes
 around a workgroup's 32 rows, with steps of two and four tokens, two steps in all and many."""
+import ctypes
+
 import pytest
 import torch
 
@@ -21,13 +23,20 @@ def test_layernorm_inside_the_spatial_reduction(dev, B, H, W, C, P):
     nw, nb = ((torch.randn(C, generator=g, device=dev) * 0.3 + i).bfloat16() for i in (1, 0))
     w = (torch.randn(C, K, generator=g, device=dev) / K ** 0.5).bfloat16()
     b = torch.randn(C, generator=g, device=dev).bfloat16()
-    out = torch.full((rows + 1, C), 7.0, device=dev, dtype=torch.bfloat16)
-    size = lib.vtdge_layernorm_patch_linear_workspace(C, P)
-    assert size == w.numel() * 2
-    ws = torch.full((size // 2 + 8,), 7.0, device=dev, dtype=torch.bfloat16)
-    _lib.call("vtdge_layernorm_patch_linear", x.data_ptr(), nw.data_ptr(), nb.data_ptr(), 1e-6, w.data_ptr(), b.data_ptr(),
-              out.data_ptr(), ws.data_ptr(), B, H, W, C, P, _lib.BF16, _lib.stream_ptr())
-    assert (out[rows:] == 7).all() and (ws[size // 2:] == 7).all()      # nothing past the end
+    out, norm = (torch.full((rows + 1, C), 7.0, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    packed = torch.full((2 * w.numel() + 8,), 7.0, device=dev, dtype=torch.bfloat16)
+    two = (ctypes.c_void_p * 2)(torch.zeros_like(w).data_ptr(), w.data_ptr())
+    _lib.call("vtdge_layernorm_patch_pack", ctypes.cast(two, ctypes.c_void_p), 2, packed.data_ptr(), C, P, _lib.stream_ptr())
+    for to, n2 in ((out, (0, 0)), (norm, (nw.data_ptr(), nb.data_ptr()))):
+        _lib.call("vtdge_layernorm_patch_linear", x.data_ptr(), nw.data_ptr(), nb.data_ptr(), 1e-6,
+                  packed.data_ptr() + w.numel() * 2, b.data_ptr(), *n2, 1e-5, to.data_ptr(), B, H, W, C, P, _lib.BF16,
+                  _lib.stream_ptr())
+    assert (out[rows:] == 7).all() and (norm[rows:] == 7).all() and (packed[2 * w.numel():] == 7).all()    # nothing past the end
+    # the rows' own LayerNorm: the operator's on the rows it stands for, bit for bit
+    want = torch.empty_like(out[:rows])
+    _lib.call("vtdge_layernorm", out.data_ptr(), nw.data_ptr(), nb.data_ptr(), want.data_ptr(), None, rows, C, 1e-5, _lib.BF16,
+              _lib.stream_ptr())
+    assert torch.equal(norm[:rows], want)
     ln = torch.empty_like(x)
     _lib.call("vtdge_layernorm", x.data_ptr(), nw.data_ptr(), nb.data_ptr(), ln.data_ptr(), None, B * H * W, C, 1e-6, _lib.BF16,
               _lib.stream_ptr())

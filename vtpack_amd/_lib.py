@@ -53,7 +53,8 @@ SIGNATURES = {
     "vtdge_layernorm_rows": [_p, _l, _i, _p, _p, _p, _l, _i, _f, _i, _p],
     "vtdge_linear": [_p, _l, _p, _p, _p, _l, _p, _l, _p, _l, _i, _i, _i, _i, _p],
     "vtdge_patch_embed": [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p],
-    "vtdge_layernorm_patch_linear": [_p, _p, _p, _f, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p],
+    "vtdge_layernorm_patch_pack": [_p, _i, _p, _i, _i, _p],
+    "vtdge_layernorm_patch_linear": [_p, _p, _p, _f, _p, _p, _p, _p, _f, _p, _i, _i, _i, _i, _i, _i, _p],
     "vtdge_layernorm_patch_linear_fits": [_i, _i, _i, _i, _i, _i],
     "vtdge_layernorm_patch_linear_wanted": [_i, _i, _i, _i, _i, _i],
     "vtdge_patch_linear": [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p],
@@ -142,8 +143,6 @@ def load():
     lib.vtdge_decompress_router_compress_workspace.argtypes = [_i, _i, _i, _i]
     lib.vtdge_region_step_workspace.restype = _l
     lib.vtdge_region_step_workspace.argtypes = [_i, _i, _i]
-    lib.vtdge_layernorm_patch_linear_workspace.restype = _l
-    lib.vtdge_layernorm_patch_linear_workspace.argtypes = [_i, _i]
     for name, args in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.restype = _i

@@ -55,6 +55,7 @@ struct ChainPlan {
     int64_t ints_total, big_total, scratch_total;
     int64_t gate0, off0, len0, ws0, gate_sz, off_sz, len_sz, ws_sz;      // in `ints`, block i at start + i * size
     int64_t tok0, comp0, q20, pat0, tok_sz, row_sz, pat_sz;              // in `big`
+    int64_t srw_sz;                // a packed weight of the spatial reduction
     int64_t xln, red, srw, kv, comp_ln, q, o, q1, q1_ln, hid, rec_x[2], rec_c[2], rec2, idx[2], cnt[2], rrows[2];   // in `scratch`
 };
 
@@ -171,7 +172,8 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
     const int64_t row = p.rows * c->C * p.esz;
     p.xln = p.folded ? 0 : take(row);
     p.red = c->sr > 1 ? take((int64_t)c->B * p.n_kv * c->C * p.esz) : 0;
-    p.srw = p.ln_sr ? take(vtdge_layernorm_patch_linear_workspace(c->C, c->sr)) : 0;
+    p.srw_sz = (int64_t)c->sr * c->sr * c->C * c->C * p.esz;
+    p.srw = p.ln_sr ? take(c->depth * p.srw_sz) : 0;
     p.kv = take(2 * (int64_t)c->B * p.n_kv * c->C * p.esz);
     p.comp_ln = p.folded ? 0 : take(row);
     p.q = take(row);
@@ -274,6 +276,16 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
     int cur = 0;                 // which of the double buffers holds what the previous block left for this one
     bool routed = false, packed = false, have_counts = false;
     SideStream beside(stream, side);
+    if (p.ln_sr) {
+        // the weights of all blocks that use them packed at once: a launch for sixteen
+        const int blocks = p.pack ? 1 : c->depth;
+        for (int at = 0; at < blocks; at += 16) {
+            const void *weights[16];
+            int n = 0;
+            for (; n < 16 && at + n < blocks; n++) weights[n] = params[(int64_t)(at + n) * P_COUNT + P_SRW];
+            VT_TRY(vtdge_layernorm_patch_pack(weights, n, scratch + p.srw + at * p.srw_sz, C, c->sr, stream));
+        }
+    }
 
     for (int i = 0; i < c->depth; i++) {
         const void *const *P = params + (int64_t)i * P_COUNT;
@@ -364,13 +376,15 @@ static int run_chain(const vtdge_chain *c, const ChainPlan &p, const void *const
                 if (c->sr > 1) {
                     char *red = scratch + p.red;
                     if (ln_sr)
-                        VT_TRY(vtdge_layernorm_patch_linear(x, P[P_N1W], P[P_N1B], c->eps1, P[P_SRW], P[P_SRB], red,
-                                                            scratch + p.srw, B, H, W, C, c->sr, dt, stream));
-                    else
+                        VT_TRY(vtdge_layernorm_patch_linear(x, P[P_N1W], P[P_N1B], c->eps1, scratch + p.srw + i * p.srw_sz,
+                                                            P[P_SRB], P[P_SRNW], P[P_SRNB], c->sr_eps, xln, B, H, W, C, c->sr,
+                                                            dt, stream));
+                    else {
                         VT_TRY(vtdge_patch_linear(xln, P[P_SRW], P[P_SRB], red, B, H, W, C, c->sr, C, dt, stream));
-                    // the normalised rows take the place of LN1(x), which nothing reads any more
-                    VT_TRY(vtdge_layernorm(red, P[P_SRNW], P[P_SRNB], xln, nullptr, (int64_t)B * p.n_kv, C, c->sr_eps, dt,
-                                           stream));
+                        // the normalised rows take the place of LN1(x), which nothing reads any more
+                        VT_TRY(vtdge_layernorm(red, P[P_SRNW], P[P_SRNB], xln, nullptr, (int64_t)B * p.n_kv, C, c->sr_eps, dt,
+                                               stream));
+                    }
                 }
                 const int64_t kv_rows = (int64_t)B * p.n_kv;
                 VT_TRY(vtdge_linear_prepacked(src, C, P[P_KVW], copy_for(P_KVP, kv_rows), P[P_KVB], nullptr, 0, kv,

@@ -21,19 +21,23 @@ namespace vtdge {
 constexpr int LNP_ROWS = 32, LNP_K = 256, LNP_PITCH = LNP_K * 2 + 16;      // LDS row: the pad turns the banks a row further
 constexpr int LNP_THREADS = 256;
 
-// The weight [C, P P C] as the product reads it: fragment (step of 32 along K, 16 columns) after fragment, 64 vectors each.
-// In rows of a power of two of bytes a step's pieces all lie in the same two channels of an L2: 47 us whatever the batch, from
-// 64 channels and P = 8 on.
-__global__ __launch_bounds__(256) void patch_weight_pack_kernel(const u32x4 *__restrict__ weight, u32x4 *__restrict__ packed, int C, int K)
+// Weights [C, P P C] as the product reads them: fragment (step of 32 along K, 16 columns) after fragment, 64 vectors each, a
+// weight a grid row.  In rows of a power of two of bytes a step's pieces all lie in the same two channels of an L2: 47 us
+// whatever the batch, from 64 channels and P = 8 on.
+constexpr int LNP_WEIGHTS = 16;
+struct PatchWeights { const u32x4 *w[LNP_WEIGHTS]; };
+__global__ __launch_bounds__(256) void patch_weight_pack_kernel(const PatchWeights weights, u32x4 *__restrict__ packed, int C, int K)
 {
     const int i = blockIdx.x * 256 + threadIdx.x, lane = i & 63, tile = i / WAVE % (C / 16), k = i / WAVE / (C / 16);
-    if (k < K / 32) packed[i] = weight[(tile * 16 + (lane & 15)) * (K / 8) + k * 4 + (lane >> 4)];
+    if (k < K / 32)
+        packed[(int64_t)blockIdx.y * (C / 8) * K + i] = weights.w[blockIdx.y][(tile * 16 + (lane & 15)) * (K / 8) + k * 4 + (lane >> 4)];
 }
 
 template <int C>
 __global__ __launch_bounds__(LNP_THREADS, 2) void layernorm_patch_linear_kernel(
     const bf16_t *__restrict__ x, const bf16_t *__restrict__ ln_w, const bf16_t *__restrict__ ln_b, float eps,
-    const u32x4 *__restrict__ packed, const bf16_t *__restrict__ bias, bf16_t *__restrict__ out, int rows, int H, int W, int P)
+    const u32x4 *__restrict__ packed, const bf16_t *__restrict__ bias, const bf16_t *__restrict__ out_w,
+    const bf16_t *__restrict__ out_b, float out_eps, bf16_t *__restrict__ out, int rows, int H, int W, int P)
 {
     constexpr int TS = LNP_K / C;                                          // tokens of a block a step
     constexpr int GS = C / 8;                                              // lanes a token: a 16-byte vector each
@@ -162,6 +166,7 @@ __global__ __launch_bounds__(LNP_THREADS, 2) void layernorm_patch_linear_kernel(
         }
         lds_barrier();
     }
+    // the product's rows, rounded, through LDS: stored whole, or their LayerNorm instead
 #pragma unroll
     for (int j = 0; j < NT; j++) {
         const int n = (wave * NT + j) * 16 + fk * 4;
@@ -169,12 +174,36 @@ __global__ __launch_bounds__(LNP_THREADS, 2) void layernorm_patch_linear_kernel(
         const float b4[4] = {bf16lo(braw.x), bf16hi(braw.x), bf16lo(braw.y), bf16hi(braw.y)};
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            const int row = row0 + i * 16 + fr;
             u32x2 r;
             r.x = pack_bf16x2(acc[i][j][0] + b4[0], acc[i][j][1] + b4[1]);
             r.y = pack_bf16x2(acc[i][j][2] + b4[2], acc[i][j][3] + b4[3]);
-            if (row < rows) *reinterpret_cast<u32x2 *>(out + (int64_t)row * C + n) = r;
+            *reinterpret_cast<u32x2 *>(tile[0] + (i * 16 + fr) * LNP_PITCH + n * 2) = r;
         }
+    }
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < LNP_ROWS / (4 * RPW); i++) {
+        const int blk = (i * 4 + wave) * RPW + lane / GS, row = row0 + blk;
+        u32x4 r = *reinterpret_cast<const u32x4 *>(tile[0] + blk * LNP_PITCH + vec * 16);
+        if (out_w != nullptr) {
+            float f[8], w2[8], b2[8], s = 0.f, q = 0.f;
+            Elem<bf16_t>::unpack(r, f);
+            Elem<bf16_t>::unpack(*reinterpret_cast<const u32x4 *>(out_w + vec * 8), w2);
+            Elem<bf16_t>::unpack(*reinterpret_cast<const u32x4 *>(out_b + vec * 8), b2);
+#pragma unroll
+            for (int c = 0; c < 8; c++) s += f[c];
+            const float mean = group_sum<GS>(s) / (float)C;
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                f[c] -= mean;
+                q += f[c] * f[c];
+            }
+            const float rstd = 1.0f / sqrtf(group_sum<GS>(q) / (float)C + out_eps);
+#pragma unroll
+            for (int c = 0; c < 8; c++) f[c] = f[c] * rstd * w2[c] + b2[c];
+            r = Elem<bf16_t>::pack(f);
+        }
+        if (row < rows) *reinterpret_cast<u32x4 *>(out + (int64_t)row * C + vec * 8) = r;
     }
 }
 
@@ -196,30 +225,48 @@ extern "C" int vtdge_layernorm_patch_linear_wanted(int B, int H, int W, int C, i
     return vtdge_layernorm_patch_linear_fits(B, H, W, C, P, dtype) && (int64_t)B * (H / P) * (W / P) >= 192 * LNP_ROWS ? 1 : 0;
 }
 
-extern "C" int64_t vtdge_layernorm_patch_linear_workspace(int C, int P) { return (int64_t)P * P * C * C * 2; }
+extern "C" int vtdge_layernorm_patch_pack(const void *const *weights_host, int count, void *packed, int C, int P, void *stream)
+{
+    VT_REQUIRE(weights_host && packed && count > 0, VTDGE_ERR_ARG, "layernorm_patch_pack: NULL operand");
+    VT_REQUIRE((C == 64 || C == 128) && P > 0 && P <= 32, VTDGE_ERR_UNSUPPORTED, "layernorm_patch_pack: %d channels, P = %d", C, P);
+    VT_REQUIRE(((uintptr_t)packed & 15) == 0, VTDGE_ERR_ARG, "layernorm_patch_pack: operands must be 16-byte aligned");
+    const int K = P * P * C;
+    for (int at = 0; at < count; at += LNP_WEIGHTS) {
+        const int n = count - at < LNP_WEIGHTS ? count - at : LNP_WEIGHTS;
+        PatchWeights pw = {};
+        for (int i = 0; i < n; i++) {
+            VT_REQUIRE(weights_host[at + i] && ((uintptr_t)weights_host[at + i] & 15) == 0, VTDGE_ERR_ARG,
+                       "layernorm_patch_pack: operands must be 16-byte aligned");
+            pw.w[i] = (const u32x4 *)weights_host[at + i];
+        }
+        note_kernel(reinterpret_cast<const void *>(patch_weight_pack_kernel));
+        patch_weight_pack_kernel<<<dim3((unsigned)ceil_div(K / 8 * C, 256), (unsigned)n), 256, 0, (hipStream_t)stream>>>(
+            pw, (u32x4 *)packed + (int64_t)at * (C / 8) * K, C, K);
+        if (int rc = check_launch("layernorm_patch_pack")) return rc;
+    }
+    return VTDGE_OK;
+}
 
 extern "C" int vtdge_layernorm_patch_linear(const void *tokens, const void *ln_weight, const void *ln_bias, float eps,
-                                            const void *weight, const void *bias, void *out, void *workspace, int B, int H, int W,
-                                            int C, int P, int dtype, void *stream)
+                                            const void *packed, const void *bias, const void *out_ln_weight,
+                                            const void *out_ln_bias, float out_eps, void *out, int B, int H, int W, int C, int P,
+                                            int dtype, void *stream)
 {
-    VT_REQUIRE(tokens && ln_weight && ln_bias && weight && bias && out && workspace, VTDGE_ERR_ARG, "layernorm_patch_linear: NULL operand");
+    VT_REQUIRE(tokens && ln_weight && ln_bias && packed && bias && out && (out_ln_weight == nullptr) == (out_ln_bias == nullptr),
+               VTDGE_ERR_ARG, "layernorm_patch_linear: NULL operand");
     VT_REQUIRE(vtdge_layernorm_patch_linear_fits(B, H, W, C, P, dtype), VTDGE_ERR_UNSUPPORTED,
                "layernorm_patch_linear: no kernel for %d x %d blocks of a %d x %d grid of %d channels", P, P, H, W, C);
-    VT_REQUIRE((((uintptr_t)tokens | (uintptr_t)ln_weight | (uintptr_t)ln_bias | (uintptr_t)weight | (uintptr_t)bias |
-                 (uintptr_t)out | (uintptr_t)workspace) & 15) == 0, VTDGE_ERR_ARG,
+    VT_REQUIRE((((uintptr_t)tokens | (uintptr_t)ln_weight | (uintptr_t)ln_bias | (uintptr_t)packed | (uintptr_t)bias |
+                 (uintptr_t)out_ln_weight | (uintptr_t)out_ln_bias | (uintptr_t)out) & 15) == 0, VTDGE_ERR_ARG,
                "layernorm_patch_linear: operands must be 16-byte aligned");
     const int rows = B * (H / P) * (W / P);
     const unsigned grid = (unsigned)ceil_div(rows, LNP_ROWS);
     hipStream_t st = (hipStream_t)stream;
-    const int K = P * P * C;
-    note_kernel(reinterpret_cast<const void *>(patch_weight_pack_kernel));
-    patch_weight_pack_kernel<<<(unsigned)ceil_div(K / 8 * C, 256), 256, 0, st>>>((const u32x4 *)weight, (u32x4 *)workspace, C, K);
-    if (int rc = check_launch("layernorm_patch_linear")) return rc;
 #define VT_LAUNCH(CC)                                                                                               \
     note_kernel(reinterpret_cast<const void *>(layernorm_patch_linear_kernel<CC>)),                                 \
     layernorm_patch_linear_kernel<CC><<<grid, LNP_THREADS, 0, st>>>(                                                \
-        (const bf16_t *)tokens, (const bf16_t *)ln_weight, (const bf16_t *)ln_bias, eps, (const u32x4 *)workspace,  \
-        (const bf16_t *)bias, (bf16_t *)out, rows, H, W, P)
+        (const bf16_t *)tokens, (const bf16_t *)ln_weight, (const bf16_t *)ln_bias, eps, (const u32x4 *)packed,     \
+        (const bf16_t *)bias, (const bf16_t *)out_ln_weight, (const bf16_t *)out_ln_bias, out_eps, (bf16_t *)out, rows, H, W, P)
     if (C == 64) VT_LAUNCH(64); else VT_LAUNCH(128);
 #undef VT_LAUNCH
     return check_launch("layernorm_patch_linear");
