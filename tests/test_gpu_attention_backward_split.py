@@ -54,6 +54,18 @@ def test_tiles_and_stages(dev, n):
     assert all(torch.equal(a, b) for a, b in zip(got, _run(q, k, v, g, kernel=kernel)))      # the same bytes on every call
 
 
+@pytest.mark.parametrize("samples,n", [(1, 161), (2, 257), (63, 193), (64, 257), (65, 257)])
+def test_samples_in_any_order(dev, samples, n):
+    """Up to 64 samples are taken with the longest first, equal ones and empty ones among them; of more as they come.  The bound
+    of test_tiles_and_stages, dK and dV being fp32 sums over the queries as dQ is over the keys: an rms that grows with the
+    square root of the longer."""
+    lengths = [2000] if samples == 1 else [3 * LENGTHS[(7 * b) % 15] + (700 if samples == 2 else 0) for b in range(samples)]
+    h = {1: 20, 2: 20}.get(samples, 6)
+    q, k, v, g = _operands(dev, n, lengths, h)
+    for name, a, b in zip("qkv", _run(q, k, v, g, lengths), _reference(q, k, v, g, lengths, 0.125)):
+        assert float((a.cpu().double() - b).norm() / b.norm()) <= 4.2e-7 * max(1.0, n / 257, max(lengths) / 257) ** 0.5, name
+
+
 @pytest.mark.parametrize("size,common", [(1.0, 0.0), (4.0, 0.0), (16.0, 0.0), (1.0, 2.0)])
 def test_as_exact_as_the_fp32_instructions(dev, size, common):
     """Large scores, and keys and values with a common component, beside the same samples in calls that are too small for the

@@ -191,7 +191,7 @@ struct AttnBack {
     int pairs, h, n;
     float scale, scale_log2;
     bool search;                                          // see find_chunk
-    bool by_chunk;                                        // see attention_dkv_kernel
+    bool by_chunk;                                        // see dkv_place
 };
 
 // the stages of two operands' rows in LDS: `rows` of them from base0 / base1 with the given row pitches in bytes
@@ -546,21 +546,25 @@ template <typename T, int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 4 
     attention_dq_rows<T, HELD>(a, smem, pair, chunk, row0, Lb);
 }
 
+// The (sample, head), counted over the launch, and the 64 keys of it that a workgroup of the dK and dV kernels takes.
+// bf16: the chunks of a pair one behind the other (39.1 us at 128 samples of 6 heads and 257 keys, 40.9 chunk by chunk), unless
+// a small last chunk would then always fall to the same of an XCD's 32 compute units (both kernels, 600 samples of 6 heads, 65
+// keys: 73.6 us, chunk by chunk 66.0; of 5 queries each 64.1 and 55.6); fp32 chunk by chunk (60.7 us at 64 of 3 on the fp32
+// instructions; 63.1), on the bf16 instructions, with the longest samples first, behind one another (both kernels, 64, 3, 257: 77.5
+// us, chunk by chunk 80.5; 16, 3, 1025: 235 and 257; with a small last chunk, 64, 6, 200: 102.5 and 107).
+__device__ __forceinline__ void dkv_place(const AttnBack &a, int &pair, int &chunk)
+{
+    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8, chunks = (a.n + 16 * AB_WAVES - 1) / (16 * AB_WAVES);
+    chunk = a.by_chunk ? rest / pairs_x : rest % chunks;
+    pair = (a.by_chunk ? rest % pairs_x : rest / chunks) * 8 + (blockIdx.x & 7);
+}
+
 // dK and dV of 64 keys of one (sample, head), from DEPTH stages of queries in LDS and their m, 1 / s and delta (of 32 rows, twice)
 template <typename T, int DEPTH>
-__device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned char *smem, float (*stats)[3][64])
+__device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned char *smem, float (*stats)[3][64], int pair, int chunk)
 {
     using B = BackTile<T>;
     using M = BackMath<T>;
-    // bf16: the chunks of a pair one behind the other (39.1 us at 128 samples of 6 heads and 257 keys, 40.9 chunk by chunk), unless
-    // a small last chunk would then always fall to the same of an XCD's 32 compute units (both kernels, 600 samples of 6 heads, 65
-    // keys: 73.6 us, chunk by chunk 66.0; of 5 queries each 64.1 and 55.6); fp32 chunk by chunk (60.7 us at 64 of 3 on the fp32
-    // instructions; 63.1).  Samples are taken as they come; handed over with the longest first they would take 36.0 us where
-    // they take 37.2 (bf16), and 41.0 where they take 48.2 (fp32).
-    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8, chunks = (a.n + 16 * AB_WAVES - 1) / (16 * AB_WAVES);
-    const int chunk = a.by_chunk ? rest / pairs_x : rest % chunks;
-    const int pair = (a.by_chunk ? rest % pairs_x : rest / chunks) * 8 + (blockIdx.x & 7);
-    if (pair >= a.pairs) return;
     const int b = pair / a.h, head = pair - b * a.h;
     const int64_t row0 = a.offsets[b];
     const int Lb = (int)(a.offsets[b + 1] - row0);
@@ -653,7 +657,9 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
     constexpr int DEPTH = sizeof(T) == 4 ? 3 : 4;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * BackTile<T>::HALF];
     __shared__ __attribute__((aligned(256))) float stats[DEPTH][3][64];
-    attention_dkv_rows<T, DEPTH>(a, smem, stats);
+    int pair, chunk;                    // samples as they come; handed over with the longest first bf16 would take 36.0 us for 37.2
+    dkv_place(a, pair, chunk);
+    if (pair < a.pairs) attention_dkv_rows<T, DEPTH>(a, smem, stats, pair, chunk);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -991,13 +997,34 @@ template <int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 3 : 2) void at
     attention_dq_rows<float, 0>(a, smem, pair, chunk, row0, Lb);
 }
 
+// The sample in place `place` of the order by length, longest first: a lane a sample, of whose numbers (length, then the first
+// of equals) each wave finds the place-th from the top bit by bit.  A workgroup's time is its sample's queries, and those
+// that start last should be short (64 samples of 3 heads, 257 keys, both kernels: 85.3 -> 80.5 us).  Of more than 64 samples there
+// are workgroups enough to fill the end: as they come.
+__device__ __forceinline__ int longest_first(const AttnBack &a, int place)
+{
+    const int samples = a.pairs / a.h, t = threadIdx.x & 63;
+    if (samples > WAVE || a.L >= (1 << 26)) return place;
+    const uint32_t mine = t < samples ? ((uint32_t)(a.offsets[t + 1] - a.offsets[t]) << 6) + 63 - t : 0u;
+    unsigned long long left = ~0ull >> (WAVE - samples);
+    int k = __builtin_amdgcn_readfirstlane(place);
+    for (int bit = 31; bit >= 0; bit--) {
+        const unsigned long long ones = __builtin_amdgcn_ballot_w64((mine >> bit) & 1) & left;
+        const int count = __builtin_popcountll(ones);
+        if (k < count) left = ones;
+        else {
+            k -= count;
+            left &= ~ones;
+        }
+    }
+    return __builtin_ctzll(left);
+}
+
 // attention_dkv_rows on split operands -> whether it could
-__device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsigned char *smem, float (*stats)[AB_ROWS], int *odd_seen)
+__device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsigned char *smem, float (*stats)[AB_ROWS], int *odd_seen,
+                                                         int pair, int chunk)
 {
     using S = BackSplit;
-    const int rest = blockIdx.x >> 3, pairs_x = (a.pairs + 7) / 8;
-    const int chunk = rest / pairs_x, pair = (rest % pairs_x) * 8 + (blockIdx.x & 7);
-    if (pair >= a.pairs) return true;
     const int b = pair / a.h, head = pair - b * a.h;
     const int64_t row0 = a.offsets[b];
     const int Lb = (int)(a.offsets[b + 1] - row0);
@@ -1099,9 +1126,13 @@ __global__ __launch_bounds__(256, 3) void attention_dkv_split_kernel(AttnBack a)
     __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * BackTile<float>::HALF];
     __shared__ __attribute__((aligned(256))) float stats[DEPTH][3][64];
     __shared__ int odd_seen;
-    if (attention_dkv_split_rows(a, smem, reinterpret_cast<float(*)[AB_ROWS]>(&stats[0][0][0]), &odd_seen)) return;
+    int place, chunk;
+    dkv_place(a, place, chunk);
+    if (place >= a.pairs) return;
+    const int pair = longest_first(a, place / a.h) * a.h + place % a.h;
+    if (attention_dkv_split_rows(a, smem, reinterpret_cast<float(*)[AB_ROWS]>(&stats[0][0][0]), &odd_seen, pair, chunk)) return;
     __syncthreads();
-    attention_dkv_rows<float, DEPTH>(a, smem, stats);
+    attention_dkv_rows<float, DEPTH>(a, smem, stats, pair, chunk);
 }
 
 template <typename T> static int launch_backward(AttnBack a, int max_rows, hipStream_t st)
@@ -1111,13 +1142,13 @@ template <typename T> static int launch_backward(AttnBack a, int max_rows, hipSt
     VT_REQUIRE(pairs_x * 8 * (qc > kc ? qc : kc) < (1ll << 31), VTDGE_ERR_UNSUPPORTED,
                "sparse_attention_backward: too many workgroups for one launch");
     a.search = qc >= 2 && a.n >= 128 && pairs_x <= AB_SEARCH && a.pairs * qc > compute_units() && has_holes(a.L, a.pairs, a.h, qc);
-    a.by_chunk = sizeof(T) == 4 || (32 % kc == 0 && (a.n - 1) % (16 * AB_WAVES) < 8 * AB_WAVES);
     // fp32 on the bf16 instructions: from 161 keys on, where live workgroups are about as many as compute units (below, one wave a
     // SIMD waits for its own vector instructions, of which the split has more).  Both kernels or neither: dK and dV take m and s of
     // dQ's scores, and other scores, of another order of sums, would double the error of dK where they are large.  Us, fp32 / bf16
-    // instructions (samples, heads, keys): 64, 3, 257: 108.3 / 84.6; 64, 6, 257: 176.7 / 144; 128, 6, 257: 323 / 250; 16, 3, 1025: 377 / 252;
+    // instructions (samples, heads, keys): 64, 3, 257: 108.3 / 77.5; 64, 6, 257: 176.7 / 134; 128, 6, 257: 323 / 250; 16, 3, 1025: 377 / 235;
     // with few live workgroups 16, 6, 257 (212): 63.7 / 60.2; 8, 3, 257 (38): 44.4 / 44.4.
     const bool split = sizeof(T) == 4 && a.n > 5 * AB_ROWS && live_chunks(a.L, a.pairs, a.h) >= compute_units();
+    a.by_chunk = sizeof(T) == 4 ? !split : 32 % kc == 0 && (a.n - 1) % (16 * AB_WAVES) < 8 * AB_WAVES;
     if (qc > 0) {
         // fp32: up to 288 keys the scores and dP of the first walk are kept for the second, the same bits in three products
         // instead of five.  Us, both kernels on the fp32 instructions, worked out again / kept (samples, heads, keys): 64, 3,
