@@ -534,16 +534,17 @@ extern "C" int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int
     if (C % vec != 0 || nvec > 192) return 0;
     // Up to where a wave for every four tokens is faster than one for sixteen that repeats nothing (the router's sums are
     // made from LDS again).  A forward, us, without it / with it (channels, regions): bf16 384: 256: 816 / 728, 512: 944 / 882,
-    // 1024: 1348 / 1304, 1568: 1552 / 1534, 2048: 1759 / 1777, 2560: 2056 / 2104; 768: 512: 2204 / 2090, 1040: 3262 / 3230, 1280:
-    // 3720 / 3664, 1584: 4325 / 4380; 320 (pyramid): 1024: 2320 / 2291, 2048: 3147 / 3170; fp32 192: 512: 1302 / 1196, 2080: 3200 /
-    // 3034, 3072: 4272 / 4138; 384: 528: 2418 / 2395, 768: 3002 / 2986, 1024: 3757 / 3713; 320 (pyramid): 768: 3865 / 3856, 1024:
-    // 4728 / 4745; 768: 384: 5296 / 5280, 528: 6572 / 6396, 768: 8303 / 8348.  Narrow rows, whose other kernels give several regions
-    // to a wave, gain longer in bf16, most of a wave's lanes idle or not: 192: 16: 541 / 437, 128: 751 / 629, 512: 997 / 847, 1536:
-    // 1311 / 1202, 2048: 1393 / 1296, 2560: 1507 / 1415, 3072: 1712 / 1641, 4096: 2021 / 2024; pyramids of 64 to 512 channels by
-    // pictures of 256 px, bf16 2: 582 / 549, 16: 796 / 755, 48: 1024 / 994; fp32 8: 1004 / 980, with 2304 regions of 64 and 576 of
-    // 128 channels 1026 / 1028, 4096 and 1024: 1184 / 1207.
-    const int most = dtype == VTDGE_BF16 ? (nvec <= 32 ? 3072 : nvec <= WAVE ? 1536 : 1280)
-                                         : (nvec <= 32 ? 2048 : nvec <= WAVE ? 3072 : nvec <= 128 ? 768 : 528);
+    // 1024: 1348 / 1304, 1600: 1644 / 1619, 2048: 1872 / 1853, 2304: 2096 / 2072, 2560: 2184 / 2185, 3072: 2446 / 2478; 768: 512:
+    // 2204 / 2090, 1040: 3262 / 3230, 1408: 3965 / 3847, 2048: 5128 / 5078, 3072: 7152 / 7113, 4096: 9036 / 8924; 192: 16: 541 / 437,
+    // 128: 751 / 629, 512: 997 / 847, 1536: 1311 / 1202, 3328: 1583 / 1539, 4096: 1778 / 1758, 8192: 3177 / 3135, 11200: 4309 / 4341;
+    // fp32 192: 512: 1302 / 1196, 2080: 3200 / 3034, 3584: 4600 / 4363, 6400: 7892 / 7338, 11200: 13343 / 13022; 384: 528: 2418 / 2395,
+    // 800: 3415 / 3264, 1280: 4901 / 4749, 2048: 7207 / 7135; 768: 384: 5296 / 5280, 528: 6572 / 6396, 768: 8269 / 8182, 1024:
+    // 10488 / 10523; pyramids with 320 channels in their third stage, bf16 1600: 2507 / 2471, 2240: 3029 / 2996; fp32 864: 4626 /
+    // 4547, 1440: 6677 / 6562, 2048: 4673 / 4674.  Rows of up to 16 vectors, whose other kernels give several regions to a wave,
+    // lose sooner: pyramids of 64 to 512 channels by pictures of 256 px, bf16 2: 582 / 549, 16: 796 / 755; with 8192 regions of 64
+    // channels 1643 / 1728; fp32 with 2304 of 64 and 576 of 128 channels 1026 / 1028, 4096 and 1024: 1184 / 1207.
+    const int most = dtype == VTDGE_BF16 ? (nvec <= 16 ? 3072 : nvec <= 32 ? 8192 : nvec <= WAVE ? 2304 : 4096)
+                                         : (nvec <= 32 ? 2048 : nvec <= WAVE ? 11200 : nvec <= 128 ? 2048 : 768);
     return regions <= most ? 1 : 0;
 }
 
