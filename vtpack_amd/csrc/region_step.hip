@@ -192,7 +192,7 @@ __device__ __forceinline__ void record_row(const u32x4 &row, bool act, float eps
 }  // namespace
 
 template <typename T, int NV, bool REC, bool NARROW>
-__global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_step_kernel(const RegionStep<T> a)
+__global__ __launch_bounds__(256, NV == 1 ? 5 : NV == 2 ? 3 : 2) void region_step_kernel(const RegionStep<T> a)
 {
     static_assert(!REC || (NV == 1 && sizeof(T) == 2 && !NARROW), "records: bf16 rows of one vector a lane");
     constexpr int VEC = Elem<T>::VEC;
@@ -210,13 +210,19 @@ __global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_ste
     for (int it = 0; it < NV; it++) act[it] = it * WAVE + lane < nvec;
     const u32x4 z = {0u, 0u, 0u, 0u};
 
-    // ---- what depends on nothing before: the router (wave 0) and the LayerNorm's parameters
-    u32x4 rw[VTDGE_MAX_SPLITS][NV];
+    // ---- what depends on nothing before: the router (wave 0) and the LayerNorm's parameters.  The weights of more than four
+    // splits are read where they are used, and the LayerNorm's of rows of three vectors a lane behind the scatter: the registers,
+    // 96, 167 and 225 where all eight splits took 123, 201 and 290.  A forward with four and five workgroups a compute unit for rows
+    // of one vector, two and three for two, us (pictures): DeiT-S bf16 80: 1302 / 1260, 130: 1853 / 1840; DeiT-Ti bf16 200: 1492 /
+    // 1458, 400: 2581 / 2523; fp32 300: 5446 / 5412; DeiT-B bf16 99: 3965 / 3889, 5: 978 / 975; DeiT-S fp32 33: 2386 / 2351.  With
+    // scratch memory instead (three workgroups, all eight early) 99 pictures took 4266 where 4116 were taken.
+    constexpr int EARLY = 4;
+    u32x4 rw[EARLY][NV];
     float rbias = 0.f;
     int rsplit = 1;
     if (wv == 0) {
 #pragma unroll
-        for (int s = 0; s < VTDGE_MAX_SPLITS; s++)
+        for (int s = 0; s < EARLY; s++)
             if (s < a.S2) {
 #pragma unroll
                 for (int it = 0; it < NV; it++) {
@@ -232,14 +238,15 @@ __global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_ste
     }
     u32x4 lw[NV], lb[NV];
     const bool normed = !REC && a.out_ln != nullptr;
-    if (normed) {
+    auto norm_parameters = [&]() {
 #pragma unroll
         for (int it = 0; it < NV; it++)
             if (act[it]) {
                 lw[it] = *reinterpret_cast<const u32x4 *>(a.ln_w + (it * WAVE + lane) * VEC);
                 lb[it] = *reinterpret_cast<const u32x4 *>(a.ln_b + (it * WAVE + lane) * VEC);
             }
-    }
+    };
+    if (NV <= 2 && normed) norm_parameters();
 
     // ---- this block's place of the region
     int64_t r0, row_b;
@@ -321,7 +328,7 @@ __global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_ste
     if (ps == 4) scatter(std::integral_constant<int, 4>{});
     else if (ps == 2) scatter(std::integral_constant<int, 2>{});
     else scatter(std::integral_constant<int, 1>{});
-
+    if (NV > 2 && normed) norm_parameters();
     lds_barrier();
 
     // ---- the next router on the tokens as stored (wave 0), published at once
@@ -353,7 +360,8 @@ __global__ __launch_bounds__(256, NV == 1 ? 4 : NV == 2 ? 2 : 1) void region_ste
                 for (int s = 0; s < VTDGE_MAX_SPLITS; s++)
                     if (s < a.S2) {
                         float w[VEC];
-                        Elem<T>::unpack(rw[s][it], w);
+                        if (s < EARLY) Elem<T>::unpack(rw[s < EARLY ? s : 0][it], w);
+                        else Elem<T>::unpack(*reinterpret_cast<const u32x4 *>(a.weight + (int64_t)s * C + (it * WAVE + lane) * VEC), w);
 #pragma unroll
                         for (int c = 0; c < VEC; c++) part[s] += acc[c] * w[c];
                     }
