@@ -9,8 +9,8 @@ from util import random_indices
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("B,C,dtype,mode", [(144, 384, "bf16", "records"), (512, 192, "bf16", "norm"), (256, 768, "bf16", "norm"),
-                                            (700, 192, "f32", "norm"), (128, 384, "f32", "norm"), (48, 768, "f32", "norm")])
+@pytest.mark.parametrize("B,C,dtype,mode", [(176, 384, "bf16", "records"), (700, 192, "bf16", "norm"), (320, 768, "bf16", "norm"),
+                                            (800, 192, "f32", "norm"), (200, 384, "f32", "norm"), (80, 768, "f32", "norm")])
 def test_the_most_regions(dev, B, C, dtype, mode):
     from vtpack_amd import _lib
     step.test_against_the_separate_operators(dev, B, 4, 4, C, 1, dtype, mode, B % 32 == 0)

@@ -545,17 +545,16 @@ extern "C" int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int
     if (C % vec != 0 || nvec > 192) return 0;
     // Up to where a wave for every four tokens is faster than one for sixteen that repeats nothing (the router's sums are
     // made from LDS again).  A forward, us, without it / with it (channels, regions): bf16 384: 256: 816 / 728, 512: 944 / 882,
-    // 1024: 1348 / 1304, 1600: 1644 / 1619, 2048: 1872 / 1853, 2304: 2096 / 2072, 2560: 2184 / 2185, 3072: 2446 / 2478; 768: 512:
-    // 2204 / 2090, 1040: 3262 / 3230, 1408: 3965 / 3847, 2048: 5128 / 5078, 3072: 7152 / 7113, 4096: 9036 / 8924; 192: 16: 541 / 437,
-    // 128: 751 / 629, 512: 997 / 847, 1536: 1311 / 1202, 3328: 1583 / 1539, 4096: 1778 / 1758, 8192: 3177 / 3135, 11200: 4309 / 4341;
-    // fp32 192: 512: 1302 / 1196, 2080: 3200 / 3034, 3584: 4600 / 4363, 6400: 7892 / 7338, 11200: 13343 / 13022; 384: 528: 2418 / 2395,
-    // 800: 3415 / 3264, 1280: 4901 / 4749, 2048: 7207 / 7135; 768: 384: 5296 / 5280, 528: 6572 / 6396, 768: 8269 / 8182, 1024:
-    // 10488 / 10523; pyramids with 320 channels in their third stage, bf16 1600: 2507 / 2471, 2240: 3029 / 2996; fp32 864: 4626 /
-    // 4547, 1440: 6677 / 6562, 2048: 4673 / 4674.  Rows of up to 16 vectors, whose other kernels give several regions to a wave,
-    // lose sooner: pyramids of 64 to 512 channels by pictures of 256 px, bf16 2: 582 / 549, 16: 796 / 755; with 8192 regions of 64
-    // channels 1643 / 1728; fp32 with 2304 of 64 and 576 of 128 channels 1026 / 1028, 4096 and 1024: 1184 / 1207.
-    const int most = dtype == VTDGE_BF16 ? (nvec <= 16 ? 3072 : nvec <= 32 ? 8192 : nvec <= WAVE ? 2304 : 4096)
-                                         : (nvec <= 32 ? 2048 : nvec <= WAVE ? 11200 : nvec <= 128 ? 2048 : 768);
+    // 1024: 1348 / 1304, 2048: 1872 / 1853, 2560: 2126 / 2073, 2816: 2281 / 2256, 3072: 2387 / 2376
+    // and, of 512 px, 2671 / 2687, 4096: 2954 / 3003; 768: 512: 2204 / 2090, 1408: 3965 / 3847, 3072: 7152 / 7113, 5120: 10542 / 10259; 192: 16: 541 / 437, 512: 997 / 847, 1536: 1311 / 1202,
+    // 4096: 1778 / 1758, 8192: 3177 / 3135, 11200: 4287 / 4176, 14400: 5535 / 5626; fp32 192: 512: 1302 / 1196, 2080: 3200 / 3034,
+    // 6400: 7892 / 7338, 12800: 15009 / 14762; 384: 528: 2418 / 2395, 1280: 4901 / 4749, 2240: 7373 / 7166, 3200: 10060 / 9847, 4096:
+    // 12813 / 12864; 768: 384: 5296 / 5280, 768: 8269 / 8182, 1280: 12039 / 11820; pyramids with 320 channels in their third stage,
+    // bf16 1600: 2507 / 2471, 2240: 3029 / 2996; fp32 864: 4626 / 4547, 1440: 6677 / 6562.  Rows of up to 16 vectors, whose other
+    // kernels give several regions to a wave, lose sooner: pyramids of 64 to 512 channels by pictures of 256 px, bf16 2: 582 / 549,
+    // 14: 1419 / 1425, 20: 1479 / 1503; fp32 with 2304 regions of 64 and 576 of 128 channels 1049 / 1043, 3072 and 768: 1125 / 1126.
+    const int most = dtype == VTDGE_BF16 ? (nvec <= 16 ? 3072 : nvec <= 32 ? 11200 : nvec <= WAVE ? 2816 : 5120)
+                                         : (nvec <= 32 ? 2048 : nvec <= WAVE ? 12800 : nvec <= 128 ? 3200 : 1280);
     return regions <= most ? 1 : 0;
 }
 
