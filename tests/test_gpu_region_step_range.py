@@ -9,7 +9,7 @@ from util import random_indices
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("B,C,dtype,mode", [(176, 384, "bf16", "records"), (700, 192, "bf16", "norm"), (320, 768, "bf16", "norm"),
+@pytest.mark.parametrize("B,C,dtype,mode", [(640, 384, "bf16", "records"), (700, 192, "bf16", "norm"), (320, 768, "bf16", "norm"),
                                             (800, 192, "f32", "norm"), (200, 384, "f32", "norm"), (80, 768, "f32", "norm")])
 def test_the_most_regions(dev, B, C, dtype, mode):
     from vtpack_amd import _lib

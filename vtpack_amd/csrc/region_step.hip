@@ -192,7 +192,7 @@ __device__ __forceinline__ void record_row(const u32x4 &row, bool act, float eps
 }  // namespace
 
 template <typename T, int NV, bool REC, bool NARROW>
-__global__ __launch_bounds__(256, NV == 1 ? 5 : NV == 2 ? 3 : 2) void region_step_kernel(const RegionStep<T> a)
+__global__ __launch_bounds__(256, NV == 1 ? (REC ? 6 : 5) : NV == 2 ? 3 : 2) void region_step_kernel(const RegionStep<T> a)
 {
     static_assert(!REC || (NV == 1 && sizeof(T) == 2 && !NARROW), "records: bf16 rows of one vector a lane");
     constexpr int VEC = Elem<T>::VEC;
@@ -212,17 +212,18 @@ __global__ __launch_bounds__(256, NV == 1 ? 5 : NV == 2 ? 3 : 2) void region_ste
 
     // ---- what depends on nothing before: the router (wave 0) and the LayerNorm's parameters.  The weights of more than four
     // splits are read where they are used, and the LayerNorm's of rows of three vectors a lane behind the scatter: the registers,
-    // 96, 167 and 225 where all eight splits took 123, 201 and 290.  A forward with four and five workgroups a compute unit for rows
+    // 96, 167 and 225 where all eight splits took 123, 201 and 290; rows with records read two ahead and the third behind the scatter
+    // (80 registers, six workgroups: 120 pictures of 384 channels 1787 -> 1764 us, 176: 2323 -> 2280).  A forward with four and five workgroups a compute unit for rows
     // of one vector, two and three for two, us (pictures): DeiT-S bf16 80: 1302 / 1260, 130: 1853 / 1840; DeiT-Ti bf16 200: 1492 /
     // 1458, 400: 2581 / 2523; fp32 300: 5446 / 5412; DeiT-B bf16 99: 3965 / 3889, 5: 978 / 975; DeiT-S fp32 33: 2386 / 2351.  With
     // scratch memory instead (three workgroups, all eight early) 99 pictures took 4266 where 4116 were taken.
-    constexpr int EARLY = 4;
+    constexpr int EARLY = REC ? 3 : 4, FIRST = REC ? 2 : EARLY;
     u32x4 rw[EARLY][NV];
     float rbias = 0.f;
     int rsplit = 1;
     if (wv == 0) {
 #pragma unroll
-        for (int s = 0; s < EARLY; s++)
+        for (int s = 0; s < FIRST; s++)
             if (s < a.S2) {
 #pragma unroll
                 for (int it = 0; it < NV; it++) {
@@ -329,6 +330,15 @@ __global__ __launch_bounds__(256, NV == 1 ? 5 : NV == 2 ? 3 : 2) void region_ste
     else if (ps == 2) scatter(std::integral_constant<int, 2>{});
     else scatter(std::integral_constant<int, 1>{});
     if (NV > 2 && normed) norm_parameters();
+    if constexpr (FIRST < EARLY)
+        if (wv == 0) {
+#pragma unroll
+            for (int s = FIRST; s < EARLY; s++)
+                if (s < a.S2) {
+                    rw[s][0] = z;
+                    if (act[0]) rw[s][0] = *reinterpret_cast<const u32x4 *>(a.weight + (int64_t)s * C + lane * VEC);
+                }
+        }
     lds_barrier();
 
     // ---- the next router on the tokens as stored (wave 0), published at once
@@ -545,15 +555,15 @@ extern "C" int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int
     if (C % vec != 0 || nvec > 192) return 0;
     // Up to where a wave for every four tokens is faster than one for sixteen that repeats nothing (the router's sums are
     // made from LDS again).  A forward, us, without it / with it (channels, regions): bf16 384: 256: 816 / 728, 512: 944 / 882,
-    // 1024: 1348 / 1304, 2048: 1872 / 1853, 2560: 2126 / 2073, 2816: 2281 / 2256, 3072: 2387 / 2376
-    // and, of 512 px, 2671 / 2687, 4096: 2954 / 3003; 768: 512: 2204 / 2090, 1408: 3965 / 3847, 3072: 7152 / 7113, 5120: 10542 / 10259; 192: 16: 541 / 437, 512: 997 / 847, 1536: 1311 / 1202,
+    // 1024: 1348 / 1304, 2048: 1872 / 1853, 2560: 2126 / 2073, 3200: 2611 / 2573, 4800: 3588 / 3487, 6144: 4393 / 4327, 10240: 7188 /
+    // 7059 (at 4096 see chain.hip); 768: 512: 2204 / 2090, 1408: 3965 / 3847, 3072: 7152 / 7113, 5120: 10542 / 10259; 192: 16: 541 / 437, 512: 997 / 847, 1536: 1311 / 1202,
     // 4096: 1778 / 1758, 8192: 3177 / 3135, 11200: 4287 / 4176, 14400: 5535 / 5626; fp32 192: 512: 1302 / 1196, 2080: 3200 / 3034,
     // 6400: 7892 / 7338, 12800: 15009 / 14762; 384: 528: 2418 / 2395, 1280: 4901 / 4749, 2240: 7373 / 7166, 3200: 10060 / 9847, 4096:
     // 12813 / 12864; 768: 384: 5296 / 5280, 768: 8269 / 8182, 1280: 12039 / 11820; pyramids with 320 channels in their third stage,
-    // bf16 1600: 2507 / 2471, 2240: 3029 / 2996; fp32 864: 4626 / 4547, 1440: 6677 / 6562.  Rows of up to 16 vectors, whose other
+    // bf16 1600: 2507 / 2471, 2240: 3029 / 2996, 4096: 4597 / 4549, 9600: 9847 / 9805; fp32 864: 4626 / 4547, 1440: 6677 / 6562.  Rows of up to 16 vectors, whose other
     // kernels give several regions to a wave, lose sooner: pyramids of 64 to 512 channels by pictures of 256 px, bf16 2: 582 / 549,
     // 14: 1419 / 1425, 20: 1479 / 1503; fp32 with 2304 regions of 64 and 576 of 128 channels 1049 / 1043, 3072 and 768: 1125 / 1126.
-    const int most = dtype == VTDGE_BF16 ? (nvec <= 16 ? 3072 : nvec <= 32 ? 11200 : nvec <= WAVE ? 2816 : 5120)
+    const int most = dtype == VTDGE_BF16 ? (nvec <= 16 ? 3072 : nvec <= 32 ? 11200 : nvec <= WAVE ? 10240 : 5120)
                                          : (nvec <= 32 ? 2048 : nvec <= WAVE ? 12800 : nvec <= 128 ? 3200 : 1280);
     return regions <= most ? 1 : 0;
 }
