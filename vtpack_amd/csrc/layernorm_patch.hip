@@ -4,16 +4,16 @@
 // from memory through registers, where it is normalised and rounded as the LayerNorm kernel does it, into LDS.
 //
 // A workgroup of four waves makes 32 rows of the product, all C columns, two workgroups a compute unit whose phases fill each
-// other (one of eight waves and 64 rows: 44.7 us where this takes 41.4).  A step is TS tokens of each of its 32 blocks,
+// other (one of eight waves and 64 rows: 44.7 us where this took 41.4).  A step is TS tokens of each of its 32 blocks,
 // K = 256: the tokens of the next step are normalised into the other of two LDS tiles while the matrix instructions read
 // this one, those of the two steps after that are on their way to registers, and so are the next step's weights, fragments
 // straight from L2, which the workgroups of an XCD share.  The weights of a step are asked for before the tokens of a
 // later one: loads come back in order, and a fragment asked for behind a token would wait for memory.
 // Bound by memory with whole chips of work, the tokens at 3.6 TB/s (a forward's other stream reads them at the same time),
-// below by a step's chain of waits, 1.4 us.  Us, LayerNorm and Linear / this with its packing (rows, channels, P): 16384, 64, 8:
-// 78.7 / 41.4; 16384, 128, 4: 44.4 / 30.0; 8192: 41.3 / 27.8 and 27.7 / 21.4; 6144: 35.4 / 26.6 and 25.8 / 20.3; 4096: 24.6 / 26.0
-// and 27.1 / 19.7; 2048: 25.4 / 25.6 and 16.3 / 19.7; 50176, 64, 4: 56.1 / 38.8; 25088, 128, 2: 24.5 / 21.2; 4096, 128, 8: 52.6 /
-// 63.9.  PVT-Small at 256 pictures, a pass: 4786 -> 4517 us.
+// below by a step's chain of waits, 1.4 us.  Us, LayerNorm and Linear / this (rows, channels, P): 16384, 64, 8: 78.7 / 39.3;
+// 16384, 128, 4: 44.4 / 27.6; 8192: 41.3 / 25.2 and 27.7 / 19.0; 6144: 35.4 / 24.1 and 25.8 / 18.2; 4096: 24.6 / 23.7 and 27.1 / 17.5;
+// 2048: 25.4 / 23.3 and 16.3 / 17.4; 50176, 64, 4: 56.1 / 36.3; 25088, 128, 2: 24.5 / 18.6; 4096, 128, 8: 52.6 / 60.0.  PVT-Small at 256
+// pictures, a pass: 4786 -> 4517 us.
 #include "common.h"
 
 namespace vtdge {
@@ -221,8 +221,11 @@ extern "C" int vtdge_layernorm_patch_linear_fits(int B, int H, int W, int C, int
 
 extern "C" int vtdge_layernorm_patch_linear_wanted(int B, int H, int W, int C, int P, int dtype)
 {
-    // from three fourths of the compute units on: the times above
-    return vtdge_layernorm_patch_linear_fits(B, H, W, C, P, dtype) && (int64_t)B * (H / P) * (W / P) >= 192 * LNP_ROWS ? 1 : 0;
+    // from three eighths of a chip of workgroups on, with long sums from three fourths: the times above, and a forward of PVT-Small,
+    // two kernels / this (pictures, 64 rows each): 32: 1642 / 1643, 40: 1779 / 1772, 48: 1866 / 1853, 56: 1966 / 1913, 64: 2076 / 2011,
+    // 92: 2477 / 2349; 24: 1556 / 1570
+    return vtdge_layernorm_patch_linear_fits(B, H, W, C, P, dtype) &&
+                   (int64_t)B * (H / P) * (W / P) >= (P * P * C <= 4096 ? 96 : 192) * LNP_ROWS ? 1 : 0;
 }
 
 extern "C" int vtdge_layernorm_patch_pack(const void *const *weights_host, int count, void *packed, int C, int P, void *stream)
