@@ -364,3 +364,22 @@ def test_a_grid_with_holes_and_one_without(dev, dtype, low, high):
         # (fp32: few workgroups have a forward kernel of their own, as above)
         assert torch.equal(o, out[at:to]) if dtype == torch.bfloat16 else float((o - out[at:to]).abs().max()) <= 2 ** -19
         assert torch.equal(q1, dq[:, at:to]) and torch.equal(k1, dk[:, b:b + 15]) and torch.equal(v1, dv[:, b:b + 15])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("which", ["q", "k"])
+def test_sums_near_the_largest_number(dev, dtype, which):
+    """64 queries with the same score for each of 64 keys, dP of +-2^120: dS is 2^111 behind the scale, and dQ (of keys of 2^4) and dK
+    (of queries of 2^9) are 2^121 and 2^126 where dP's own products would add up to 2^130 and 2^129.  Powers of two: exact."""
+    from vtpack_amd import ops
+    sign = torch.tensor([1.0, -1.0]).repeat(32)[:, None].expand(64, 64)
+    q = torch.zeros(1, 64, 64) if which == "q" else torch.full((1, 64, 64), 2.0 ** 9)
+    k = (sign * 2.0 ** 4)[None, None] if which == "q" else torch.zeros(1, 1, 64, 64)
+    v, g = torch.zeros(1, 1, 64, 64), torch.zeros(1, 64, 64)
+    v[..., 0], g[..., 0] = sign[:, 0] * 2.0 ** 60, 2.0 ** 60
+    offsets, _ = ops.lengths_to_offsets(torch.tensor([64]), dev)
+    dq, dk, dv = ops.sparse_attention_backward(*(t.to(dev, dtype).contiguous() for t in (q, k, v)), None, g.to(dev, dtype), offsets,
+                                               0.125, 64)
+    assert torch.equal(dq.cpu().float(), torch.full((1, 64, 64), 2.0 ** 121 if which == "q" else 0.0))
+    assert torch.equal(dk.cpu().float()[0, 0], sign * 2.0 ** 126 if which == "k" else torch.zeros(64, 64))
+    assert torch.equal(dv.cpu().float()[0, 0], g[0])

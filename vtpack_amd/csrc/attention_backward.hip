@@ -498,7 +498,8 @@ __device__ __forceinline__ void attention_dq_rows(const AttnBack &a, unsigned ch
         a.delta[at] = delta;
     }
 
-    // ---- dQ^T += K^T dS^T
+    // ---- dQ^T += K^T dS^T, dS whole before it is rounded and added up: behind the sums, scale / s would come too late for those
+    // that pass the largest number without it
     f32x4 dq[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) dq[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -508,7 +509,7 @@ __device__ __forceinline__ void attention_dq_rows(const AttnBack &a, unsigned ch
         for (int blk = 0; blk < 2; blk++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                ds[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -all)) * (dp[blk][r] - delta);
+                ds[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -all)) * (dp[blk][r] - delta) * scale_s;
         if (HELD > 0 || a.n - st * AB_ROWS < AB_ROWS)
 #pragma unroll
             for (int e = 0; e < 8; e++)
@@ -532,8 +533,6 @@ __device__ __forceinline__ void attention_dq_rows(const AttnBack &a, unsigned ch
             add(st, t, dp);
         }
     }
-#pragma unroll
-    for (int i = 0; i < 4; i++) dq[i] *= scale_s;         // this lane's query's
     if (live) M::store((T *)a.dq + (row0 + row) * a.dq_rs + (int64_t)head * a.dq_hs, dq, g);
 }
 
@@ -638,7 +637,7 @@ __device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned c
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 p[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[blk][r], a.scale_log2, -ms[blk][r])) * iv[blk][r];
-                ds[blk][r] = p[blk][r] * (ds[blk][r] - dl[blk][r]);
+                ds[blk][r] = p[blk][r] * (ds[blk][r] - dl[blk][r]) * a.scale;
             }
         }
         M::accumulate(Ds, p, dv, l, g);
@@ -646,8 +645,6 @@ __device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned c
     }
     if (!live) return;
     const int64_t at = (int64_t)b * a.dkv_bs + (int64_t)key * a.dkv_ts + (int64_t)head * a.dkv_hs;
-#pragma unroll
-    for (int i = 0; i < 4; i++) dk[i] *= a.scale;
     M::store((T *)a.dk + at, dk, g);
     M::store((T *)a.dv + at, dv, g);
 }
