@@ -44,13 +44,12 @@ __device__ __forceinline__ void layernorm_rows(const u32x4 (&raw)[NR], bool acti
         float f[VEC];
         Elem<T>::unpack(raw[t], f);
         q[t] = 0.f;
-        if (active) {
 #pragma unroll
-            for (int c = 0; c < VEC; c++) {
-                const float dlt = f[c] - s[t];
-                q[t] += dlt * dlt;
-            }
+        for (int c = 0; c < VEC; c++) {
+            const float dlt = f[c] - s[t];
+            q[t] += dlt * dlt;
         }
+        q[t] = active ? q[t] : 0.f;
     }
     group_sum_n<GS, NR>(q);
     if (!active) return;          // after the last reduction
@@ -76,8 +75,13 @@ __device__ __forceinline__ void layernorm_rows(const u32x4 (&raw)[NR], bool acti
 // that of the sample's extra tokens): the block's first LayerNorm (vtpack/models/dge/deit_dge.py:127) without a
 // second pass over x.  Same arithmetic as layernorm_kernel (two-pass statistics in fp32, the same reduction
 // tree).  Needs RS > 0 and a row that fits one 16-byte vector per lane of the group.
+//
+// LNF, R = 4, keeps sixteen vectors a lane in up to 196 registers, two waves a SIMD; with the squares of the second pass in a branch of
+// their own the compiler took 402 of bf16 rows of 136 to 256 channels, one wave: 256 samples of 257 tokens of 136, 192 and 256
+// channels 23.2, 25.2 and 27.1 us, this way 13.9, 15.1 and 17.0.  R = 2 in fp32 fits 64 registers, eight waves (72: 96
+// channels 14.0 us, 13.1 this way).
 template <typename T, int RS, int GS, bool LNF = false>   // RS = region size known at compile time (all window loads in flight), 0 = generic
-__global__ __launch_bounds__(256) void router_kernel(const T *__restrict__ x, const T *__restrict__ weight,
+__global__ __launch_bounds__(256, LNF && RS == 2 && sizeof(T) == 4 ? 8 : 2) void router_kernel(const T *__restrict__ x, const T *__restrict__ weight,
                                                       const T *__restrict__ bias, T *__restrict__ gate,
                                                       int64_t *__restrict__ indices, int B, int H, int W,
                                                       int C, int extra, int R, int S,
