@@ -123,3 +123,37 @@ def test_values_outside_the_split(dev, which, value):
         huge = b.abs() >= 1e9
         for part in (b.isfinite() & huge, b.isfinite() & ~huge):
             assert float((a - b)[part].norm()) <= 1e-6 * float(b[part].norm()), name
+
+
+@pytest.mark.parametrize("odd", [None, "q", "k", "g"])
+@pytest.mark.parametrize("kind", ["x100", "x1000", "point"])
+def test_as_exact_where_few_keys_take_all(dev, kind, odd):
+    """Large scores, of which the largest key's P is 1 only if it comes from the scores that m and s are of: queries a hundred and a
+    thousand times as large, and queries that point at one key each (dV is then a copy of dO and all but exact: one rounding, 2^-24, is
+    allowed).  `odd`: a value too small for the split in one sample of a head, whose rows, or for a key all rows of the sample, take the
+    fp32 instructions while the rest of that sample does not.  Else the bound of test_as_exact_as_the_fp32_instructions."""
+    t = dict(zip("qkvg", _operands(dev, 257)))
+    at = [sum(LENGTHS[:b]) for b in range(len(LENGTHS))]
+    if kind == "point":
+        pick = torch.Generator().manual_seed(3)
+        for b, m in enumerate(LENGTHS):
+            t["q"][:, at[b]:at[b] + m] += 8 * t["k"][:, b, torch.randint(0, 257, (m,), generator=pick)]
+    else:
+        t["q"] *= float(kind[1:])
+    if odd in ("q", "g"):
+        for head in range(HEADS):
+            t[odd][head, at[14] + 70, 5] = 1e-25
+    elif odd == "k":
+        t["k"][:, 14, 7, 3] = 1e-25
+    got, parts = _run(*t.values()), []
+    some = [b for b, m in enumerate(LENGTHS) if m > 0]
+    for b in some:
+        rows = slice(at[b], at[b] + LENGTHS[b])
+        one = (t["q"][:, rows], t["k"][:, b:b + 1], t["v"][:, b:b + 1], t["g"][:, rows])
+        parts.append(_run(*(x.contiguous() for x in one), [LENGTHS[b]], kernel=None))
+    plain = [torch.cat([p[i] for p in parts], dim=1) for i in range(3)]
+    for name, a, c, w in zip("qkv", got, plain, _reference(*t.values(), LENGTHS, 0.125)):
+        a, w = (x if name == "q" else x[:, some] for x in (a, w))
+        off = float((a.cpu().double() - w).norm())
+        allowed = 2.0 ** -24 * float(w.norm()) if name == "v" and kind == "point" else 0.0
+        assert off <= max(allowed, 1.05 * float((c.cpu().double() - w).norm())), name

@@ -90,6 +90,15 @@ template <> struct BackMath<float> {
         for (int r = 0; r < 4; r++)
             *reinterpret_cast<f32x4 *>(row + 16 * g + 4 * r) = f32x4{o[0][r], o[1][r], o[2][r], o[3][r]};
     }
+    static __device__ __forceinline__ void add(const float *row, f32x4 (&o)[4], int g)
+    {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(row + 16 * g + 4 * r);
+#pragma unroll
+            for (int db = 0; db < 4; db++) o[db][r] += v[db];
+        }
+    }
 };
 template <> struct BackMath<bf16_t> {
     typedef u32x4 Frag;
@@ -109,8 +118,8 @@ template <> struct BackMath<bf16_t> {
     }
     // All of the stage's fragments are asked for before the first product: left to itself the compiler keeps registers for two
     // and waits for LDS in every step.  Us, with the masks of keys past the last in the last stage alone, before / now, dQ and dK with
-    // dV (samples, heads, keys): 128, 6, 257: 48.0 / 43.0 and 44.6 / 41.9; 64, 3, 257: 18.5 / 16.3 and 16.0 / 14.7; 30, 5, 401: 28.1 / 23.7 and
-    // 21.2 / 19.4; 16, 3, 1025: 48.0 / 37.2 and 36.4 / 33.1.
+    // dV (samples, heads, keys): 128, 6, 257: 48.5 / 44.5 and 45.2 / 43.6; 64, 3, 257: 18.2 / 16.2 and 15.6 / 14.8; 30, 5, 401: 27.2 / 23.5 and
+    // 20.4 / 19.3; 16, 3, 1025: 46.4 / 38.7 and 35.5 / 34.0.
     static __device__ __forceinline__ void both_scores(const unsigned char *S0, const unsigned char *S1, const Frag (&x)[2],
                                                        const Frag (&y)[2], f32x4 (&t)[2], f32x4 (&dp)[2], int l, int g)
     {
@@ -185,7 +194,7 @@ struct AttnTrain {
 struct AttnBack {
     const void *q, *k, *v, *dout;
     void *dq, *dk, *dv;
-    float *m, *inv, *delta;                               // [h, L] each; bf16, or inv NULL: m + log2(s) in m's place
+    float *m, *inv, *delta;                               // [h, L] each; bf16, or inv NULL: m + log2(s) in m's place; inv < 0: see BackSplit
     const int64_t *offsets;
     int64_t q_rs, q_hs, kv_bs, kv_ts, kv_hs, o_rs, o_hs, dq_rs, dq_hs, dkv_bs, dkv_ts, dkv_hs, L;
     int pairs, h, n;
@@ -393,7 +402,8 @@ template <bool SEARCH> __global__ __launch_bounds__(256, 4) void attention_train
 
 // dQ of 64 query rows of one (sample, head), with their m, 1 / s and delta.
 // HELD: stages of keys whose scores and dP stay in registers between the two walks (0: they are worked out again)
-template <typename T, int HELD>
+// MARKED: 1 / s is left with its sign set (see attention_dkv_split_rows)
+template <typename T, int HELD, bool MARKED = false>
 __device__ __forceinline__ void attention_dq_rows(const AttnBack &a, unsigned char *smem, int pair, int chunk, int64_t row0, int Lb)
 {
     using B = BackTile<T>;
@@ -494,7 +504,7 @@ __device__ __forceinline__ void attention_dq_rows(const AttnBack &a, unsigned ch
         const int64_t at = (int64_t)head * a.L + row0 + row;
         const bool apart = sizeof(T) == 4 && a.inv != nullptr;
         a.m[at] = apart ? all : all + __builtin_amdgcn_logf(s);                 // v_log_f32: base 2
-        if (apart) a.inv[at] = inv;
+        if (apart) a.inv[at] = MARKED ? __uint_as_float(__float_as_uint(inv) | 0x80000000u) : inv;
         a.delta[at] = delta;
     }
 
@@ -559,7 +569,8 @@ __device__ __forceinline__ void dkv_place(const AttnBack &a, int &pair, int &chu
 }
 
 // dK and dV of 64 keys of one (sample, head), from DEPTH stages of queries in LDS and their m, 1 / s and delta (of 32 rows, twice)
-template <typename T, int DEPTH>
+// MARKED: of the stages alone whose 1 / s has its sign set, and added to what this wave has stored before
+template <typename T, int DEPTH, bool MARKED = false>
 __device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned char *smem, float (*stats)[3][64], int pair, int chunk)
 {
     using B = BackTile<T>;
@@ -612,6 +623,7 @@ __device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned c
             lds_barrier();
         }
         if (!wave_live) continue;
+        if (MARKED && __builtin_amdgcn_readfirstlane(__float_as_int(stats[st % DEPTH][1][0])) >= 0) continue;
         f32x4 ms[2], iv[2], dl[2];                        // rows past the sample's last query: probability zero
 #pragma unroll
         for (int blk = 0; blk < 2; blk++) {
@@ -636,7 +648,8 @@ __device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned c
         for (int blk = 0; blk < 2; blk++) {
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                p[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[blk][r], a.scale_log2, -ms[blk][r])) * iv[blk][r];
+                p[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[blk][r], a.scale_log2, -ms[blk][r])) *
+                            (MARKED ? fabsf(iv[blk][r]) : iv[blk][r]);
                 ds[blk][r] = p[blk][r] * (ds[blk][r] - dl[blk][r]) * a.scale;
             }
         }
@@ -645,6 +658,10 @@ __device__ __forceinline__ void attention_dkv_rows(const AttnBack &a, unsigned c
     }
     if (!live) return;
     const int64_t at = (int64_t)b * a.dkv_bs + (int64_t)key * a.dkv_ts + (int64_t)head * a.dkv_hs;
+    if constexpr (MARKED) {
+        M::add((const T *)a.dk + at, dk, g);
+        M::add((const T *)a.dv + at, dv, g);
+    }
     M::store((T *)a.dk + at, dk, g);
     M::store((T *)a.dv + at, dv, g);
 }
@@ -667,16 +684,21 @@ template <typename T> __global__ __launch_bounds__(256, sizeof(T) == 4 ? 3 : 4) 
 // What bounds both kernels are the vector instructions (the splits: 44 for a fragment of 8 values a lane; they hide behind the
 // products only in part, two of them a matrix instruction) beside 96 (72) matrix instructions of 16 clocks a wave and stage, where the
 // fp32 ones were 128 (96) of 32.  Three (two) workgroups a compute unit fill each other's waits: one buffer of parts and two barriers a
-// stage.  Us, both kernels, 64 samples, 6 heads, 257 keys, as this one 144: two buffers and one barrier 162, rows by direct loads into a
-// ring of three 153, two workgroups a compute unit for dK and dV 148.  Us, fp32 / bf16 instructions, dQ and dK with dV (samples,
-// heads, keys, queries): 64, 3, 257, 7352: 45.6 / 36.3 and 63.5 / 49.3; 128, 6, 257, 15262: 159 / 124 and 167 / 121; 16, 3, 1025, 7598: 191 / 128
-// and 185 / 125.  Relative errors against float64 (2-norm): dQ 4.2e-7 / 2.9e-7, dK 3.5e-7 / 2.2e-7, dV 3.3e-7 / 2.0e-7; queries four times
-// as large: 9.0e-7 / 5.1e-7, 8.8e-7 / 4.8e-7, 7.3e-7 / 3.8e-7.
+// stage (both kernels, 64 samples, 6 heads, 257 keys: two buffers and one barrier an eighth slower, rows by direct loads into a ring of
+// three 6 %, two workgroups a compute unit for dK and dV 3 %).  Us, fp32 / bf16 instructions, dQ and dK with dV (samples, heads,
+// keys, queries): 64, 3, 257, 7352: 43.3 / 32.5 and 61.8 / 36.3; 64, 6: 82.0 / 61.1 and 95.1 / 56.2; 128, 6, 257, 15262: 157 / 120 and 165 / 107; 16, 3,
+// 1025, 7598: 190 / 125 and 186 / 98.  Relative errors against float64 (2-norm): dQ 4.2e-7 / 2.9e-7, dK 3.6e-7 / 2.2e-7, dV 3.4e-7 / 2.1e-7;
+// queries 16 times as large: 3.3e-6 / 1.7e-6, 3.4e-6 / 1.7e-6, 1.3e-6 / 6.3e-7; 1000 times: 1.8e-4 / 9.1e-5, 1.8e-4 / 9.4e-5, 9.6e-6 / 4.6e-6; queries
+// that point at one key each: 1.0e-2 / 7.9e-3, 8.8e-3 / 6.8e-3, 1.8e-8 / 4.2e-8 (a copy of dO, within a rounding).
 //
-// The values that this is not exact for take the fp32 instructions, the whole workgroup from the start: an operand that is not zero
-// and not in [2^-60, 2^20) in size (its third part, and products of parts, would reach below the smallest bf16 and fp32 numbers;
-// infinities and NaN are out of that range too), and a result that is not zero and below 2^-80, where what P and dS lose below 2^-134
-// shows.  The other workgroups of such a sample stay here, with scores of another order of sums than those that m and s are of.
+// The values that this is not exact for take the fp32 instructions: an operand that is not zero and not in [2^-60, 2^20) in size (its
+// third part, and products of parts, would reach below the smallest bf16 and fp32 numbers; infinities and NaN are out of that
+// range too).  A workgroup of 64 queries that meets one takes them from the start and marks its rows by the sign of 1 / s; the key
+// tiles leave the stages of such rows out and add them up by the fp32 instructions behind the others: the scores that P is made of
+// are always those, to the last bit, that m and s are of.  With other scores, of another order of sums, P of a row's largest key
+// would be exp2 of some last bits of the score (queries that point at one key each: dV 8.6e-6 and dK 0.51 off).  P and dS carry a factor of 2^32 into their parts and out of the results: their smallest values would
+// reach below 2^-134 otherwise.  Nothing can overflow: scores and dP stay below 2^46, sums of dS over rows below 2^120.
+constexpr float BS_UP = 0x1p32f, BS_DOWN = 0x1p-32f;
 constexpr int BS_PLANE = AB_ROWS * 128, BS_BUF = 6 * BS_PLANE;      // bytes of a plane, and of two operands' three
 
 struct BackSplit {
@@ -802,17 +824,6 @@ struct BackSplit {
 #pragma unroll
         for (int db = 0; db < 4; db++) *reinterpret_cast<f32x4 *>(row + 16 * db + 4 * g) = o[db];
     }
-    // whether a result is not finite, or not zero and below 2^-80
-    static __device__ __forceinline__ bool lost(const f32x4 (&o)[4])
-    {
-        bool odd = false;
-#pragma unroll
-        for (int e = 0; e < 16; e++) {
-            const float m = fabsf(o[e / 4][e % 4]);
-            odd = odd || !(m < INFINITY) || (m < 0x1p-80f && m != 0.f);
-        }
-        return odd;
-    }
 };
 
 // attention_dq_rows on split operands -> whether it could
@@ -821,7 +832,8 @@ __device__ __forceinline__ bool attention_dq_split_rows(const AttnBack &a, unsig
                                                         int64_t row0, int Lb)
 {
     using S = BackSplit;
-    if (!(a.scale_log2 > 0.f)) return false;              // keys past the last: a score of -infinity, below
+    // keys past the last: a score of -infinity, below; and what is said above of overflow
+    if (!(a.scale_log2 >= 0x1p-40f && a.scale_log2 <= 0x1p40f)) return false;
     const int b = pair / a.h, head = pair - b * a.h;
     const int tid = threadIdx.x, lane = tid & 63, l = lane & 15, g = lane >> 4;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -935,7 +947,13 @@ __device__ __forceinline__ bool attention_dq_split_rows(const AttnBack &a, unsig
     sd += __shfl_xor(sd, 16, WAVE);
     s += __shfl_xor(s, 32, WAVE);
     sd += __shfl_xor(sd, 32, WAVE);
-    const float inv = 1.0f / s, delta = sd / s, scale_s = a.scale * inv;
+    const float inv = 1.0f / s, delta = sd / s, scale_s = a.scale * inv * BS_DOWN, up_delta = BS_UP * delta;
+    if (live && g == 0) {
+        const int64_t at = (int64_t)head * a.L + row0 + row;
+        a.m[at] = all;
+        a.inv[at] = inv;
+        a.delta[at] = delta;
+    }
 
     // ---- dQ^T += K^T dS^T
     f32x4 dq[4];
@@ -947,7 +965,8 @@ __device__ __forceinline__ bool attention_dq_split_rows(const AttnBack &a, unsig
         for (int blk = 0; blk < 2; blk++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                ds[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -all)) * (dp[blk][r] - delta);
+                ds[blk][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[blk][r], a.scale_log2, -all)) *
+                             __builtin_fmaf(dp[blk][r], BS_UP, -up_delta);      // 2^32 (dP - delta), to the last bit
         S::accumulate(Ks, ds, dq, l, g);
     };
     if constexpr (HELD > 0) {
@@ -968,16 +987,7 @@ __device__ __forceinline__ bool attention_dq_split_rows(const AttnBack &a, unsig
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) dq[i] *= scale_s;         // this lane's query's
-    // (a row whose scores are all -infinity, or that met a NaN, has no finite delta)
-    if (__syncthreads_or(wave_live && (S::lost(dq) || (live && !(fabsf(delta) < INFINITY))) ? 1 : 0)) return false;
-    if (!live) return true;
-    if (g == 0) {
-        const int64_t at = (int64_t)head * a.L + row0 + row;
-        a.m[at] = a.inv != nullptr ? all : all + __builtin_amdgcn_logf(s);      // v_log_f32: base 2
-        if (a.inv != nullptr) a.inv[at] = inv;
-        a.delta[at] = delta;
-    }
-    S::store((float *)a.dq + (row0 + row) * a.dq_rs + (int64_t)head * a.dq_hs, dq, g);
+    if (live) S::store((float *)a.dq + (row0 + row) * a.dq_rs + (int64_t)head * a.dq_hs, dq, g);
     return true;
 }
 
@@ -991,7 +1001,7 @@ template <int HELD> __global__ __launch_bounds__(256, HELD == 0 ? 3 : 2) void at
     if (!find_chunk(a.search, a.offsets, a.pairs, a.h, pair, chunk, row0, Lb)) return;
     if (attention_dq_split_rows<HELD>(a, smem, &odd_seen, pair, chunk, row0, Lb)) return;
     __syncthreads();
-    attention_dq_rows<float, 0>(a, smem, pair, chunk, row0, Lb);
+    attention_dq_rows<float, 0, true>(a, smem, pair, chunk, row0, Lb);
 }
 
 // The sample in place `place` of the order by length, longest first: a lane a sample, of whose numbers (length, then the first
@@ -1017,9 +1027,9 @@ __device__ __forceinline__ int longest_first(const AttnBack &a, int place)
     return __builtin_ctzll(left);
 }
 
-// attention_dkv_rows on split operands -> whether it could
-__device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsigned char *smem, float (*stats)[AB_ROWS], int *odd_seen,
-                                                         int pair, int chunk)
+// attention_dkv_rows on split operands, of the stages whose rows are not marked -> whether any were.  A stage is of one workgroup's rows
+// of the queries' kernel, and one with an operand that the split does not cover is marked: the queries' own, or all for a key's.
+__device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsigned char *smem, float (*stats)[AB_ROWS], int pair, int chunk)
 {
     using S = BackSplit;
     const int b = pair / a.h, head = pair - b * a.h;
@@ -1029,7 +1039,6 @@ __device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsi
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int key = (chunk * AB_WAVES + wid) * 16 + l;
     const bool live = key < a.n, wave_live = (chunk * AB_WAVES + wid) * 16 < a.n;
-    if (tid == 0) *odd_seen = 0;
 
     // this thread's part of a stage: 8 channels of a query and of its dO, and one of the 96 statistics
     const int srow = tid >> 3, schunk = tid & 7;
@@ -1037,9 +1046,8 @@ __device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsi
     const float *dp_ = (const float *)a.dout + row0 * a.o_rs + (int64_t)head * a.o_hs + 8 * schunk;
     const int64_t stat = (int64_t)head * a.L + row0;
     const int which = tid >> 5;                           // 0: m, 1: 1 / s, 2: delta
-    const float *mine = (which == 0 ? a.m : which == 1 ? a.inv : a.delta);
-    const bool brings = which < 3 && mine != nullptr;
-    float rq[8], rd[8], rs = 1.f;
+    const float *mine = which == 0 ? a.m : which == 1 ? a.inv : a.delta;
+    float rq[8], rd[8], rs = 0.f;
     auto load_stage = [&](int st) {                       // rows past the last query repeat it
         const int64_t r = min(st * AB_ROWS + srow, Lb - 1);
 #pragma unroll
@@ -1051,9 +1059,8 @@ __device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsi
                 rd[4 * i + e] = y[e];
             }
         }
-        if (brings) rs = mine[stat + min(st * AB_ROWS + (tid & 31), Lb - 1)];
+        if (which < 3) rs = mine[stat + min(st * AB_ROWS + (tid & 31), Lb - 1)];
     };
-    bool odd = false;
     auto store_stage = [&](int st) {
         if (st * AB_ROWS + AB_ROWS > Lb) {                // nothing of a repeated row: probability zero
             const bool past = st * AB_ROWS + srow >= Lb;
@@ -1067,28 +1074,30 @@ __device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsi
         u32x4 p[2][3];
         S::store_row(smem, srow, schunk, rq, p[0]);
         S::store_row(smem + 3 * BS_PLANE, srow, schunk, rd, p[1]);
-        odd = odd || S::outside(p[0][0], p[1][0]);
-        if (which < 3) stats[which][tid & 31] = rs;
-        if (odd) *odd_seen = 1;
+        if (which < 3) stats[which][tid & 31] = which == 1 ? rs * BS_UP : rs;
     };
 
     const int stages = (Lb + AB_ROWS - 1) / AB_ROWS;      // none for a sample without queries: its gradients are zero
     if (stages > 0) load_stage(0);
     u32x4 kf[2][3], vf[2][3];
     const int64_t kv_at = (int64_t)b * a.kv_bs + (int64_t)key * a.kv_ts + (int64_t)head * a.kv_hs;
-    odd = S::load_kept(kf, (const float *)a.k + kv_at, live, g);
-    odd = S::load_kept(vf, (const float *)a.v + kv_at, live, g) || odd;
+    S::load_kept(kf, (const float *)a.k + kv_at, live, g);
+    S::load_kept(vf, (const float *)a.v + kv_at, live, g);
     f32x4 dk[4], dv[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) dk[i] = dv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const unsigned char *Qs = smem, *Ds = smem + 3 * BS_PLANE;
+    bool marked = false;
     for (int st = 0; st < stages; st++) {
-        lds_barrier();                                    // the stage before has been read (before the first: odd_seen is zero)
+        lds_barrier();                                    // the stage before has been read
         store_stage(st);
         if (st + 1 < stages) load_stage(st + 1);
         lds_barrier();                                    // stage st is whole
-        if (__builtin_amdgcn_readfirstlane(*odd_seen) != 0) return false;
+        if (__builtin_amdgcn_readfirstlane(__float_as_int(stats[1][0])) < 0) {
+            marked = true;
+            continue;
+        }
         if (!wave_live) continue;
         f32x4 p[2], ds[2];
         S::both_scores<true>(Qs, Ds, kf, vf, p, ds, l, g);
@@ -1106,14 +1115,16 @@ __device__ __forceinline__ bool attention_dkv_split_rows(const AttnBack &a, unsi
         S::accumulate(Ds, p, dv, l, g);
         S::accumulate(Qs, ds, dk, l, g);
     }
+    if (!live) return marked;
 #pragma unroll
-    for (int i = 0; i < 4; i++) dk[i] *= a.scale;
-    if (__syncthreads_or(odd || S::lost(dk) || S::lost(dv) ? 1 : 0)) return false;
-    if (!live) return true;
+    for (int i = 0; i < 4; i++) {
+        dk[i] *= a.scale * BS_DOWN;
+        dv[i] *= BS_DOWN;
+    }
     const int64_t at = (int64_t)b * a.dkv_bs + (int64_t)key * a.dkv_ts + (int64_t)head * a.dkv_hs;
     S::store((float *)a.dk + at, dk, g);
     S::store((float *)a.dv + at, dv, g);
-    return true;
+    return marked;
 }
 
 __global__ __launch_bounds__(256, 3) void attention_dkv_split_kernel(AttnBack a)
@@ -1122,14 +1133,13 @@ __global__ __launch_bounds__(256, 3) void attention_dkv_split_kernel(AttnBack a)
     static_assert(DEPTH * 2 * BackTile<float>::HALF >= BS_BUF, "one LDS for either");
     __shared__ __attribute__((aligned(1024))) unsigned char smem[DEPTH * 2 * BackTile<float>::HALF];
     __shared__ __attribute__((aligned(256))) float stats[DEPTH][3][64];
-    __shared__ int odd_seen;
     int place, chunk;
     dkv_place(a, place, chunk);
     if (place >= a.pairs) return;
     const int pair = longest_first(a, place / a.h) * a.h + place % a.h;
-    if (attention_dkv_split_rows(a, smem, reinterpret_cast<float(*)[AB_ROWS]>(&stats[0][0][0]), &odd_seen, pair, chunk)) return;
-    __syncthreads();
-    attention_dkv_rows<float, DEPTH>(a, smem, stats, pair, chunk);
+    if (!attention_dkv_split_rows(a, smem, reinterpret_cast<float(*)[AB_ROWS]>(&stats[0][0][0]), pair, chunk)) return;
+    __syncthreads();                                      // LDS has been read, and what the wave has stored can be
+    attention_dkv_rows<float, DEPTH, true>(a, smem, stats, pair, chunk);
 }
 
 template <typename T> static int launch_backward(AttnBack a, int max_rows, hipStream_t st)
@@ -1139,12 +1149,12 @@ template <typename T> static int launch_backward(AttnBack a, int max_rows, hipSt
     VT_REQUIRE(pairs_x * 8 * (qc > kc ? qc : kc) < (1ll << 31), VTDGE_ERR_UNSUPPORTED,
                "sparse_attention_backward: too many workgroups for one launch");
     a.search = qc >= 2 && a.n >= 128 && pairs_x <= AB_SEARCH && a.pairs * qc > compute_units() && has_holes(a.L, a.pairs, a.h, qc);
-    // fp32 on the bf16 instructions: from 161 keys on, where live workgroups are about as many as compute units (below, one wave a
-    // SIMD waits for its own vector instructions, of which the split has more).  Both kernels or neither: dK and dV take m and s of
-    // dQ's scores, and other scores, of another order of sums, would double the error of dK where they are large.  Us, fp32 / bf16
-    // instructions (samples, heads, keys): 64, 3, 257: 108.3 / 77.5; 64, 6, 257: 176.7 / 134; 128, 6, 257: 323 / 250; 16, 3, 1025: 377 / 235;
-    // with few live workgroups 16, 6, 257 (212): 63.7 / 60.2; 8, 3, 257 (38): 44.4 / 44.4.
-    const bool split = sizeof(T) == 4 && a.n > 5 * AB_ROWS && live_chunks(a.L, a.pairs, a.h) >= compute_units();
+    // fp32 on the bf16 instructions: from 161 keys on, where live workgroups are about as many as compute units.  Us, both kernels, fp32 /
+    // bf16 instructions (samples, heads, keys): 64, 3, 257: 106.6 / 74.2; 64, 6, 257: 177.7 / 122.1; 128, 6, 257: 321 / 231; 16, 3, 1025: 376 /
+    // 224.  With fewer, one wave a SIMD waits for its own vector instructions, of which the split has more: 16, 6, 257 (212 of them) 63.7 /
+    // 60.2, 8, 3, 257 (38) 44.4 / 44.4, less than the rest of a training pass waits.  Both kernels or neither, and with 1 / s to carry
+    // the marks: scores of another order of sums than those that m and s are of would be off where they are large.
+    const bool split = sizeof(T) == 4 && a.inv != nullptr && a.n > 5 * AB_ROWS && live_chunks(a.L, a.pairs, a.h) >= compute_units();
     a.by_chunk = sizeof(T) == 4 ? !split : 32 % kc == 0 && (a.n - 1) % (16 * AB_WAVES) < 8 * AB_WAVES;
     if (qc > 0) {
         // fp32: up to 288 keys the scores and dP of the first walk are kept for the second, the same bits in three products
