@@ -230,7 +230,8 @@ int vtdge_decompress_router_compress_static(const void *in, const void *sub, con
  *   next_*: of the block that follows, as in vtdge_decompress_router_compress; S and S2 split sizes, all of them 1, 2 or 4
  *   out_records, next_comp_records (nullable, bf16 rows of 264 to 512 channels) or out_ln [B * (extra + H*W), C], next_comp_ln
  *   [capacity_rows, C] (nullable) with ln_weight, ln_bias; eps of either
- *   workspace: vtdge_region_step_workspace bytes, zero; its first word stays 0 unless the kernel gave up waiting
+ *   workspace: vtdge_region_step_workspace bytes, zero; its first word stays 0 unless the kernel gave up waiting (rows are missing then
+ *   and next_offsets[B] exceeds capacity_rows)
  * vtdge_region_step_fits: 1 for rows of 1 to 192 whole 16-byte vectors, up to 64 extra tokens and as many regions (528 to 3072, by
  * width and type) as the launch is faster for than the separate ones. */
 int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int dtype);

@@ -1072,8 +1072,8 @@ __device__ __forceinline__ void region_read(const T *__restrict__ refp, int W, i
 // workgroup publishes the queries of its four regions, the last of every 64 the queries of them all, and each adds up
 // the words of its own group and the sums of the groups before it.  A workgroup only ever waits for workgroups
 // with smaller numbers, which were dispatched before it and wait for nobody behind them, so the chain always moves;
-// the wait is bounded all the same (a workgroup that gives up raises the error word and places its rows past the
-// capacity, where nothing is written).  The status words must be zero at launch; nothing else of them is kept.
+// the wait is bounded all the same (a workgroup that gives up raises the error word and the last offset and places its
+// rows past the capacity, where nothing is written; handover.h).  The status words must be zero at launch; nothing else of them is kept.
 struct ChainArgs {
     bf16_t *comp;                 // [capacity, C] the next block's packed queries
     u32x4 *comp_records;          // [capacity, 2] their statistics records
@@ -1303,7 +1303,7 @@ void decompress_route_kernel(
         if (wv == 0) {
             const int agg = cnt_s[0] + cnt_s[1] + cnt_s[2] + cnt_s[3];
             chain_publish(st, wg, agg);
-            const long long excl = chain_rows_before(chain.status, wg, agg, chain.capacity);
+            const long long excl = chain_rows_before(chain.status, wg, agg, chain.capacity, chain.offsets + B);
             if (lane == 0) excl_s = excl;
         }
         __syncthreads();
@@ -1329,7 +1329,7 @@ void decompress_route_kernel(
                 pp[0] = b; pp[1] = -(int64_t)lane - 1; pp[2] = 0; pp[3] = 1;
             }
         }
-        if (region == (int64_t)B * nreg - 1 && lane == 0) chain.offsets[B] = n0 + nq;
+        if (region == (int64_t)B * nreg - 1 && lane == 0) chain_total(chain.status, chain.offsets + B, n0 + nq, chain.capacity);
         if (n0 < extra || n0 + nq > chain.capacity) return;   // never outside the buffers
         // The tokens are read back by the lanes that stored them (a lane reads what it wrote itself, in program
         // order): plain loads, served by the caches the stores went through.

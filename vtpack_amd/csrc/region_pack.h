@@ -1,6 +1,7 @@
 // Packing the tokens of 4 x 4 regions into query rows, for the kernels that do it a wave per region.
 #pragma once
 #include "common.h"
+#include "handover.h"
 
 namespace vtdge {
 
@@ -186,66 +187,6 @@ __device__ __forceinline__ void pack_held(const u32x4 (&tok)[16], T *cp, u32x4 *
         lane_sums<T>(packed, act, pivot[w], st[2 * w], st[2 * w + 1]);
     }
     write_records4(st, pivot[0], pivot[1], pivot[2], pivot[3], C, eps, rec);
-}
-
-// ---------------------------------------------------------------- query counts handed from workgroup to workgroup
-// status[0]: error flag, status[1 + w]: what workgroup w has to say: a flag bit and its count, the last of every 64
-// workgroups the count of them all.  All zero at launch.
-constexpr int CHAIN_GROUP = 64;
-constexpr unsigned long long CHAIN_KNOWN = 1ull << 62;
-constexpr int CHAIN_SPIN_LIMIT = 1 << 20;
-
-// the queries of workgroup `wg`; one wave
-__device__ __forceinline__ void chain_publish(unsigned long long *words, int wg, int agg)
-{
-    if ((threadIdx.x & 63) == 0 && wg % CHAIN_GROUP != CHAIN_GROUP - 1)
-        __hip_atomic_store(words + wg, CHAIN_KNOWN | (unsigned long long)agg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// The queries of all workgroups before `wg`, whose own are `agg`.  One wave, the value in every lane; `capacity` where the wait
-// was given up.  A lane takes a workgroup of wg's own group and every 64th of the groups before it, and asks again only for
-// what it still lacks: two trips to memory once all have spoken, however many they are.  Looking back 64 words at a time took
-// 52.1 us for the scatter-back of 1024 workgroups (256 x 16 x 16 tokens of 384 channels) and 96.6 of 2048, this 49.1 and 88.8;
-// without any wait the first takes 48.3.  A group's sum made by atomic additions of all 64 instead: 58.9 us.
-__device__ __forceinline__ long long chain_rows_before(unsigned long long *status, int wg, int agg, int64_t capacity)
-{
-    const int lane = threadIdx.x & 63;
-    unsigned long long *st = status + 1;
-    const int groups = wg / CHAIN_GROUP, place = wg % CHAIN_GROUP;
-    int spins = 0, own = 0, before = 0, g = lane;
-    bool want_own = lane < place, to_say = place == CHAIN_GROUP - 1;
-    while (true) {
-        unsigned long long vo = 0, vg = 0;
-        if (want_own) vo = __hip_atomic_load(st + groups * CHAIN_GROUP + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (g < groups)
-            vg = __hip_atomic_load(st + (int64_t)g * CHAIN_GROUP + CHAIN_GROUP - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (vo & CHAIN_KNOWN) {
-            own = (int)(vo & 0xffffffffull);
-            want_own = false;
-        }
-        if (vg & CHAIN_KNOWN) {
-            before += (int)(vg & 0xffffffffull);
-            g += WAVE;
-        }
-        const bool own_done = __builtin_amdgcn_ballot_w64(want_own) == 0;
-        if (own_done && to_say) {
-            to_say = false;
-            const int all = agg + (int)wave_sum((float)own);                  // small integers: exact
-            if (lane == 0)
-                __hip_atomic_store(st + wg, CHAIN_KNOWN | (unsigned long long)all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (own_done && __builtin_amdgcn_ballot_w64(g < groups) == 0) return (long long)wave_sum((float)(own + before));
-        if (++spins > CHAIN_SPIN_LIMIT) {
-            // every row of this workgroup falls past the capacity, and of those that build on its group's count
-            if (lane == 0) {
-                __hip_atomic_store(status, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (to_say)
-                    __hip_atomic_store(st + wg, CHAIN_KNOWN | (unsigned long long)capacity, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            return capacity;
-        }
-        __builtin_amdgcn_s_sleep(1);
-    }
 }
 
 }  // namespace vtdge

@@ -10,7 +10,7 @@
 // results are theirs bit for bit.
 //
 // The first packed row of a region is the number of queries of all regions before it: handed along in launch order through
-// status words (region_pack.h), a workgroup waits for workgroups with smaller numbers only.
+// status words (handover.h), a workgroup waits for workgroups with smaller numbers only.
 #include "region_pack.h"
 
 namespace vtdge {
@@ -446,7 +446,7 @@ __global__ __launch_bounds__(256, NV == 1 ? (REC ? 6 : 5) : NV == 2 ? 3 : 2) voi
 
     // ---- the region's place among the next block's queries
     if (wv == 0) {
-        const long long before = chain_rows_before(a.status, region, nq, a.capacity);
+        const long long before = chain_rows_before(a.status, region, nq, a.capacity, a.next_offsets + a.B);
         if (lane == 0) s_before = before;
     }
     lds_barrier();
@@ -467,7 +467,7 @@ __global__ __launch_bounds__(256, NV == 1 ? (REC ? 6 : 5) : NV == 2 ? 3 : 2) voi
                 p[0] = b; p[1] = -(int64_t)lane - 1; p[2] = 0; p[3] = 1;
             }
         }
-        if (region == a.B * nreg - 1 && lane == 0) a.next_offsets[a.B] = n0 + nq;
+        if (region == a.B * nreg - 1 && lane == 0) chain_total(a.status, a.next_offsets + a.B, n0 + nq, a.capacity);
     }
     if (n0 + nq > a.capacity) return;                              // never outside the buffers
 
