@@ -350,3 +350,24 @@ def test_layernorm_linear_is_wanted_where_it_fits_and_not_beyond_its_lead():
         assert (lib.vtdge_layernorm_linear_wanted(*both), lib.vtdge_layernorm_linear_wanted(*one)) == (pair, fc1), (rows, C)
         assert lib.vtdge_layernorm_linear_fits(*both) >= pair and lib.vtdge_layernorm_linear_fits(*one) >= fc1
     assert lib.vtdge_layernorm_linear_fits(771, 1536, 771, 768, 768, _lib.BF16)      # what was taken before still is
+
+
+def test_region_step_is_planned_wherever_it_is_said_to_fit():
+    """A chain's status words, eight bytes a region where its blocks are joined by vtdge_region_step and a fourth of that by the
+    chained scatter-back: by the one rule of vtdge_region_step_fits, with no sizes of a chain's own in between."""
+    import ctypes
+    from vtpack_amd import _lib
+    lib = _lib.load()
+    for C, grid, batches in ((384, 16, (13, 192, 240, 241, 247, 250, 256, 257, 300, 511, 512, 640, 641, 700)),
+                             (384, 32, (60, 61, 63, 64, 65, 128, 160, 161))):
+        for B in batches:
+            desc = _lib.Chain(B=B, H=grid, W=grid, C=C, heads=C // 64, hidden=4 * C, extra=1, S=3, depth=3, dtype=_lib.BF16, sr=1,
+                              splits_124=1, eps1=1e-6, eps2=1e-6, sr_eps=0.0, scale=0.125)
+            words = (ctypes.c_int64 * (_lib.CHAIN_LAYOUT_HEAD + 3 * _lib.CHAIN_LAYOUT_BLOCK))()
+            assert lib.vtdge_chain_layout(ctypes.addressof(desc), ctypes.addressof(words)) == 0
+            regions = B * (grid // 4) ** 2
+            step = lib.vtdge_region_step_fits(B, grid, grid, C, 1, _lib.BF16)
+            assert step == (regions <= 10240)
+            want = lib.vtdge_region_step_workspace(B, grid, grid) if step else \
+                lib.vtdge_decompress_router_compress_workspace(B, grid, grid, 4)
+            assert words[3] == want, (grid, B)

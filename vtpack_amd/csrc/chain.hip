@@ -140,10 +140,6 @@ static int plan_chain(const vtdge_chain *c, ChainPlan &p)
     p.tail = vtdge_block_tail_wanted(p.rows, c->C, c->hidden, c->dtype);
     p.ln_fc1 = !p.folded && !p.tail && vtdge_layernorm_linear_wanted(p.cap, c->hidden, 0, 0, c->C, c->dtype);
     p.step = c->depth > 1 && c->splits_124 && vtdge_region_step_fits(c->B, c->H, c->W, c->C, c->extra, c->dtype);
-    // Where a wave for every region fills the chip once and all run at once, the chained scatter-back is as fast: 4096 regions, it /
-    // region_step, us: of 256 px 3093 / 3098, of 512 px 3427 / 3440 (3840: 2960 / 2956, 4800: 3588 / 3487).
-    constexpr int64_t WAVES = 256 * 16;       // compute units, and waves of its registers on one
-    if (p.folded && p.regions % 4 == 0 && p.regions > WAVES - WAVES / 16 && p.regions <= WAVES) p.step = false;
     p.pack = p.step || (p.folded && c->depth > 1 && p.regions % 4 == 0);
     p.ws_words = p.step   ? vtdge_region_step_workspace(c->B, c->H, c->W) / 8
                  : p.pack ? vtdge_decompress_router_compress_workspace(c->B, c->H, c->W, 4) / 8

@@ -555,8 +555,8 @@ extern "C" int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int
     if (C % vec != 0 || nvec > 192) return 0;
     // Up to where a wave for every four tokens is faster than one for sixteen that repeats nothing (the router's sums are
     // made from LDS again).  A forward, us, without it / with it (channels, regions): bf16 384: 256: 816 / 728, 512: 944 / 882,
-    // 1024: 1348 / 1304, 2048: 1872 / 1853, 2560: 2126 / 2073, 3200: 2611 / 2573, 4800: 3588 / 3487, 6144: 4393 / 4327, 10240: 7188 /
-    // 7059 (at 4096 see chain.hip); 768: 512: 2204 / 2090, 1408: 3965 / 3847, 3072: 7152 / 7113, 5120: 10542 / 10259; 192: 16: 541 / 437, 512: 997 / 847, 1536: 1311 / 1202,
+    // 1024: 1348 / 1304, 2048: 1872 / 1853, 2560: 2126 / 2073, 3200: 2486 / 2436, 3904: 2871 / 2853 (of 512 px 3254 / 3263), 4096: 2972 / 2968 (3394 / 3395), 4224: 3206 / 3090, 5120: 3738 / 3638, 6144: 4393 / 4327, 8192: 5739 / 5708, 10240: 7188 /
+    // 7059; 768: 512: 2204 / 2090, 1408: 3965 / 3847, 3072: 7152 / 7113, 5120: 10542 / 10259; 192: 16: 541 / 437, 512: 997 / 847, 1536: 1311 / 1202,
     // 4096: 1778 / 1758, 8192: 3177 / 3135, 11200: 4287 / 4176, 14400: 5535 / 5626; fp32 192: 512: 1302 / 1196, 2080: 3200 / 3034,
     // 6400: 7892 / 7338, 12800: 15009 / 14762; 384: 528: 2418 / 2395, 1280: 4901 / 4749, 2240: 7373 / 7166, 3200: 10060 / 9847, 4096:
     // 12813 / 12864; 768: 384: 5296 / 5280, 768: 8269 / 8182, 1280: 12039 / 11820; pyramids with 320 channels in their third stage,
