@@ -83,6 +83,38 @@ def test_pvt(dev, dtype, batch):
     assert all(_same(a[k], b[k]) for a, b in zip(st, wst) for k in KEYS)
 
 
+@pytest.mark.parametrize("two_streams", [False, True])
+@pytest.mark.parametrize("batch,img,depths,kernels", [
+    (48, 256, [3, 2, 1, 1], 4),       # 3072 rows: of 64 channels every block, of 128 (3072 regions too) the first, the second from region_step
+    (47, 256, [2, 2, 1, 1], 0), (52, 256, [18, 3, 1, 1], 21),          # a row short; more blocks than one launch packs weights for
+    (193, 128, [1, 2, 1, 1], 3)])
+def test_pvt_with_norm1_inside_the_reduction(dev, batch, img, depths, kernels, two_streams):
+    from vtpack_amd import _lib
+    torch.manual_seed(10)
+    m = PyramidVisionTransformer(img_size=img, patch_size=4, embed_dims=[64, 128, 320, 512], num_heads=[1, 2, 5, 8], mlp_ratios=[2] * 4,
+                                 qkv_bias=True, depths=depths, sr_ratios=[8, 4, 2, 1], split_sizes=[[4, 2, 1]] * 4, num_classes=30)
+    m = set_synthetic_router(m, 4).eval().to(dev).bfloat16()
+    with torch.no_grad():
+        for blk in _blocks(m):                   # no block's parameters like another's
+            for t in blk.parameters():
+                t += 0.02 * torch.randn_like(t) if t.is_floating_point() else 0
+    images = synthetic_images(batch, img, seed=6, dtype=torch.bfloat16, device=dev)
+    before, calls = engine.OVERLAP_FROM, []
+    engine.OVERLAP_FROM = 0 if two_streams else 1 << 62
+    whole = engine.ops.layernorm_patch_linear
+    engine.ops.layernorm_patch_linear = lambda *a: calls.append(a) or whole(*a)
+    try:
+        got, st = _run(m, images, True)
+        assert not calls
+        want, wst = _run(m, images, False)
+    finally:
+        engine.OVERLAP_FROM = before
+        engine.ops.layernorm_patch_linear = whole
+    assert len(calls) == kernels
+    assert torch.equal(got, want)
+    assert all(_same(a[k], b[k]) for a, b in zip(st, wst) for k in KEYS)
+
+
 def test_changes_of_the_parameters_are_seen(dev):
     """In-place edits, a parameter or a module replaced, another data type, a copy of the model: each call works with
     the parameters as they are then."""

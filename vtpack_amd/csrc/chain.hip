@@ -5,8 +5,8 @@
 // converting twenty arguments), more than most of them run for below a batch of some hundred pictures.  Here the
 // caller hands over three buffers and a table of parameter addresses once per call, and a launch costs what
 // hipLaunchKernel costs.  The kernels and their order are those that engine.block_forward issues, but for what it leaves to
-// separate launches: the scatter-back, sampling and LayerNorm of few regions (vtdge_region_step, the same bits) and the splits of
-// several blocks' fp32 weights (vtdge_linear_split_set).
+// separate launches: scatter-back, sampling and LayerNorm where regions are few enough (vtdge_region_step, the same bits), the splits
+// of several blocks' fp32 weights (vtdge_linear_split_set) and the packing of their reduction weights (vtdge_layernorm_patch_pack).
 //
 // Buffers: `ints` holds the small results a caller may read later (gate logits, offsets, lengths, and the status words
 // of the chained scatter-backs), `big` the tokens between blocks, the packed queries before and after the block and

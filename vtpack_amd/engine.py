@@ -205,6 +205,19 @@ def _key_value_source(attn, x_ln, H, W, extra):
     return ops.layernorm(red, attn.norm.weight, attn.norm.bias, attn.norm.eps).view(B, -1, C)
 
 
+def _reduced_raw(attn, norm1, x, H, W):
+    """`_key_value_source` from the raw tokens, norm1, the reduction and its norm in one kernel, or None where there is none or it is
+    not the faster way."""
+    sr = getattr(attn, "sr_ratio", 1)
+    if sr <= 1 or not FUSE_PATCH_EMBED or H % sr or W % sr or x.dtype != torch.bfloat16:
+        return None
+    args = (x, H, W, sr, _khwc_weight(attn.sr), attn.sr.bias)
+    ln, out_ln = (norm1.weight, norm1.bias), (attn.norm.weight, attn.norm.bias)
+    if not ops.fits_layernorm_patch_linear(*args, ln, out_ln):
+        return None
+    return ops.layernorm_patch_linear(*args, ln, norm1.eps, out_ln, attn.norm.eps).view(x.shape[0], -1, x.shape[-1])
+
+
 def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_block=None):
     """x [B, N, C] -> [B, N, C] for a DGE transformer block (`models.dge.deit_dge.Block` or
     `models.dge.pvt_dge.Block`) in eval mode.
@@ -226,6 +239,8 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
     routed = carry.get("routed") if gate is None else None
 
     n1, n2 = block.norm1, block.norm2
+    # whether a chain issued as one call has this block's norm1 from `vtdge_region_step`
+    steps = routed is not None and set(dge.router.split_sizes) <= {1, 2, 4} and ops.fits_region_step(x, H, W)
     fold1 = (FOLD_NORMS and x_ln is None and getattr(attn, "sr_ratio", 1) <= 1
              and ops.fits_linear_layernorm(x, attn.kv.weight))
     use_regions = REGION_COMPRESS and ops.fits_compress_regions(x, H, W, R, dge.router.split_sizes)
@@ -264,9 +279,11 @@ def block_forward(block, x, H, W, gate=None, overlap=True, carry=None, next_bloc
             if rec1 is None:
                 rec1 = ops.layernorm_stats(x, n1.eps)
             return x, ops.linear_layernorm(x, rec1, attn.kv.weight, attn.kv.bias, n1.weight, n1.bias)
-        if x_ln is None:
-            x_ln = ops.layernorm(x, n1.weight, n1.bias, n1.eps)
-        src = _key_value_source(attn, x_ln, H, W, extra)
+        src = _reduced_raw(attn, n1, x, H, W) if x_ln is None and not extra and not steps else None
+        if src is None:
+            if x_ln is None:
+                x_ln = ops.layernorm(x, n1.weight, n1.bias, n1.eps)
+            src = _key_value_source(attn, x_ln, H, W, extra)
         return src, ops.linear(src, attn.kv.weight, attn.kv.bias, keep_split=True)   # [B, n, 2C] = [B, n, 2, h, d]
 
     cap = B * N

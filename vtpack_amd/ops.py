@@ -306,6 +306,12 @@ def fits_pack_next(x, H, W, region_size, split_sizes):
             and (B * (H // region_size) * (W // region_size)) % 4 == 0)
 
 
+def fits_region_step(x, H, W):
+    """Whether a chain of blocks issued as one call joins them by `vtdge_region_step` on these tokens."""
+    return (x.is_cuda and x.dtype in (torch.float32, torch.bfloat16)
+            and _lib.load().vtdge_region_step_fits(x.shape[0], H, W, x.shape[2], x.shape[1] - H * W, dtype_code(x)) == 1)
+
+
 def decompress_router(inp, indices, splits, offsets, reference, H, W, region_size, sub=None, next_weight=None,
                       next_bias=None, want_gate=True, stats_eps=None, next_splits=None, region_rows=None,
                       cur_counts=None, pack_next=False, pack_eps=None, capacity=None, workspace=None):
@@ -830,6 +836,36 @@ def patch_linear(x, H, W, k, weight, bias, out=None):
         raise ValueError(f"out must be a contiguous tensor of shape {(rows, N)}")
     call("vtdge_patch_linear", ptr(x), ptr(_contig(weight)), ptr(_contig(bias)), ptr(out), B, H, W, C, k, N,
          dtype_code(x), stream_ptr(), tag=("patch_linear", B, H, W, C, k, N))
+    return out
+
+
+def fits_layernorm_patch_linear(x, H, W, k, weight, bias, ln, out_ln):
+    """Whether `layernorm_patch_linear` has a kernel for these operands (bf16, 64 or 128 channels kept, parameters on 16-byte
+    boundaries) and it is the faster way.  ln, out_ln = (weight, bias)."""
+    C = x.shape[-1]
+    return bool(x.is_cuda and x.dim() == 3 and x.shape[1] == H * W and x.dtype == torch.bfloat16 and tuple(weight.shape) == (C, k * k * C)
+                and all(t is not None and t.dtype == x.dtype and t.data_ptr() % 16 == 0 for t in (weight, bias, *ln, *out_ln))
+                and _lib.load().vtdge_layernorm_patch_linear_wanted(x.shape[0], H, W, C, k, dtype_code(x)))
+
+
+def layernorm_patch_linear(x, H, W, k, weight, bias, ln, ln_eps, out_ln, out_eps):
+    """LayerNorm(patch_linear(LayerNorm(x))) [B * (H/k) * (W/k), C] in one pass over the tokens: norm1, the spatial reduction and its
+    norm (vtpack/models/dge/pvt_dge.py:81-83), rounded in between as the three are.  See `fits_layernorm_patch_linear`."""
+    _need_gpu(x, weight, bias, *ln, *out_ln)
+    _check_like(x, weight=weight, bias=bias, ln_weight=ln[0], ln_bias=ln[1], out_ln_weight=out_ln[0], out_ln_bias=out_ln[1])
+    if not fits_layernorm_patch_linear(x, H, W, k, weight, bias, ln, out_ln):
+        raise ValueError("layernorm_patch_linear: no kernel for these operands (see fits_layernorm_patch_linear)")
+    B, _, C = x.shape
+    for name, t in (("bias", bias), ("ln_weight", ln[0]), ("ln_bias", ln[1]), ("out_ln_weight", out_ln[0]), ("out_ln_bias", out_ln[1])):
+        _check_vector(name, t, C)
+    x, weight = _contig(x), _contig(weight)
+    packed = torch.empty_like(weight)
+    one = (ctypes.c_void_p * 1)(ptr(weight))
+    call("vtdge_layernorm_patch_pack", ctypes.addressof(one), 1, ptr(packed), C, k, stream_ptr())
+    out = torch.empty((B * (H // k) * (W // k), C), dtype=x.dtype, device=x.device)
+    call("vtdge_layernorm_patch_linear", ptr(x), ptr(_contig(ln[0])), ptr(_contig(ln[1])), ln_eps, ptr(packed), ptr(_contig(bias)),
+         ptr(_contig(out_ln[0])), ptr(_contig(out_ln[1])), out_eps, ptr(out), B, H, W, C, k, dtype_code(x), stream_ptr(),
+         tag=("layernorm_patch_linear", B, H, W, C, k))
     return out
 
 
