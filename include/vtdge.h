@@ -222,7 +222,7 @@ int vtdge_decompress_router_compress_static(const void *in, const void *sub, con
                                             int B, int H, int W, int C, int extra, int R, int S, int S2, int dtype,
                                             void *stream);
 
-/* Few regions (see vtdge_region_step_fits): from the packed queries of one block to those of the next in one launch, a
+/* Up to some thousand regions (see vtdge_region_step_fits): from the packed queries of one block to those of the next in one launch, a
  * workgroup per 4 x 4 region - vtdge_decompress_router, vtdge_compress_regions (or vtdge_index_to_patch and vtdge_compress)
  * and, of tokens and packed rows, either the statistics records or the LayerNorm, each bit for bit.
  *   in, sub [.., C]: the packed queries after and before the block   cur_indices, splits, offsets: its gate indices, splits and
@@ -232,7 +232,7 @@ int vtdge_decompress_router_compress_static(const void *in, const void *sub, con
  *   [capacity_rows, C] (nullable) with ln_weight, ln_bias; eps of either
  *   workspace: vtdge_region_step_workspace bytes, zero; its first word stays 0 unless the kernel gave up waiting (rows are missing then
  *   and next_offsets[B] exceeds capacity_rows)
- * vtdge_region_step_fits: 1 for rows of 1 to 192 whole 16-byte vectors, up to 64 extra tokens and as many regions (528 to 3072, by
+ * vtdge_region_step_fits: 1 for rows of 1 to 192 whole 16-byte vectors, up to 64 extra tokens and as many regions (1280 to 12800, by
  * width and type) as the launch is faster for than the separate ones. */
 int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int dtype);
 int64_t vtdge_region_step_workspace(int B, int H, int W);

@@ -1,5 +1,5 @@
 """A block's scatter-back, the next router, index -> patch, compress and LayerNorm as one launch (vtdge_region_step) against the
-separate operators, bit for bit: region counts around its look-back window, rows of one to three vectors a lane, every split."""
+separate operators, bit for bit: region counts around the groups of 64 that hand their query counts along, rows of one to three vectors a lane, every split."""
 import pytest
 import torch
 

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,C,dtype,mode", [(640, 384, "bf16", "records"), (700, 192, "bf16", "norm"), (320, 768, "bf16", "norm"),
-                                            (800, 192, "f32", "norm"), (200, 384, "f32", "norm"), (80, 768, "f32", "norm")])
+                                            (192, 64, "bf16", "norm"), (128, 128, "f32", "norm"), (800, 192, "f32", "norm"), (200, 384, "f32", "norm"), (80, 768, "f32", "norm")])
 def test_the_most_regions(dev, B, C, dtype, mode):
     from vtpack_amd import _lib
     step.test_against_the_separate_operators(dev, B, 4, 4, C, 1, dtype, mode, B % 32 == 0)

@@ -43,7 +43,7 @@ struct ChainPlan {
     int esz, N, n_kv;              // tokens per sample, keys per sample
     bool folded;                   // norms folded into weight-stationary Linears, chained scatter-back (384-channel bf16)
     bool by_region, pack;          // compress by region; the scatter-back packs the next block's queries
-    bool step;                     // few regions: the scatter-back also writes what the next block's norm1 wants
+    bool step;                     // vtdge_region_step joins the blocks: the scatter-back also writes what the next block's norm1 wants
     bool tail;                     // narrow bf16 rows: everything behind attention as one kernel
     bool ln_kvq, ln_fc1;           // few rows: norm1 inside the kv and q Linear, norm2 inside fc1
     bool ln_sr;                    // many rows: norm1 inside the spatial reduction

@@ -1,9 +1,10 @@
 // From the packed queries of one block to those of the next in one launch, a workgroup per 4 x 4 region (gfx950): scatter
 // back, the next block's router, its index -> patch and compress, and whatever its first LayerNorm wants of tokens and rows.
 //
-// For few regions (up to a few a compute unit), where the launches this replaces - decompress_route_kernel, compress_regions or
-// patch_write + compress, layernorm - are chains of round trips to memory by four waves on four regions each: 300 instructions a
-// token one after the other in a wave that has its SIMD for itself.  Here a wave has one row of four tokens; the sixteen meet
+// With few regions the launches this replaces - decompress_route_kernel, compress_regions or patch_write + compress,
+// layernorm - are chains of round trips to memory by four waves on four regions each: 300 instructions a token one after the other
+// in a wave that has its SIMD for itself; with many, up to 50 a compute unit, they are the passes over the tokens that this one
+// does not repeat (vtdge_region_step_fits has the line).  Here a wave has one row of four tokens; the sixteen meet
 // in LDS, where wave 0 adds them up for the router in the one order all kernels use while the other waves write what
 // LayerNorm wants of theirs.  What the router needs is requested first of all, and its decision is published before
 // anything that can wait.  Every value has the arithmetic, the order and the rounding of the kernels named above: the
@@ -555,8 +556,8 @@ extern "C" int vtdge_region_step_fits(int B, int H, int W, int C, int extra, int
     if (C % vec != 0 || nvec > 192) return 0;
     // Up to where a wave for every four tokens is faster than one for sixteen that repeats nothing (the router's sums are
     // made from LDS again).  A forward, us, without it / with it (channels, regions): bf16 384: 256: 816 / 728, 512: 944 / 882,
-    // 1024: 1348 / 1304, 2048: 1872 / 1853, 2560: 2126 / 2073, 3200: 2486 / 2436, 3904: 2871 / 2853 (of 512 px 3254 / 3263), 4096: 2972 / 2968 (3394 / 3395), 4224: 3206 / 3090, 5120: 3738 / 3638, 6144: 4393 / 4327, 8192: 5739 / 5708, 10240: 7188 /
-    // 7059; 768: 512: 2204 / 2090, 1408: 3965 / 3847, 3072: 7152 / 7113, 5120: 10542 / 10259; 192: 16: 541 / 437, 512: 997 / 847, 1536: 1311 / 1202,
+    // 1024: 1348 / 1304, 2048: 1872 / 1853, 2560: 2126 / 2073, 3200: 2486 / 2436, 3904: 2871 / 2853 (of 512 px 3254 / 3263), 4096:
+    // 2972 / 2968 (3394 / 3395), 4224: 3206 / 3090, 5120: 3738 / 3638, 6144: 4393 / 4327, 8192: 5739 / 5708, 10240: 7188 / 7059; 768: 512: 2204 / 2090, 1408: 3965 / 3847, 3072: 7152 / 7113, 5120: 10542 / 10259; 192: 16: 541 / 437, 512: 997 / 847, 1536: 1311 / 1202,
     // 4096: 1778 / 1758, 8192: 3177 / 3135, 11200: 4287 / 4176, 14400: 5535 / 5626; fp32 192: 512: 1302 / 1196, 2080: 3200 / 3034,
     // 6400: 7892 / 7338, 12800: 15009 / 14762; 384: 528: 2418 / 2395, 1280: 4901 / 4749, 2240: 7373 / 7166, 3200: 10060 / 9847, 4096:
     // 12813 / 12864; 768: 384: 5296 / 5280, 768: 8269 / 8182, 1280: 12039 / 11820; pyramids with 320 channels in their third stage,
