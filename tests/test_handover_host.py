@@ -39,8 +39,10 @@ static std::function<void(void *, bool)> on_access;      // before a load or sto
 static void seen(const void *p, bool store) { if (threadIdx.x == 0 && on_access) on_access((void *)p, store); }
 template <typename T> T load(const T *p) { seen(p, false); return __atomic_load_n(p, __ATOMIC_SEQ_CST); }
 template <typename T, typename V> void store(T *p, V v) { seen(p, true); __atomic_store_n(p, (T)v, __ATOMIC_SEQ_CST); }
+template <typename T> T exchange(T *p, T v) { seen(p, true); return __atomic_exchange_n(p, v, __ATOMIC_SEQ_CST); }
 #define __hip_atomic_load(p, order, scope) load(p)
 #define __hip_atomic_store(p, v, order, scope) store(p, v)
+#define __hip_atomic_exchange(p, v, order, scope) exchange(p, v)
 static unsigned long long __builtin_amdgcn_ballot_w64(bool b)
 {
     wave->bits[threadIdx.x] = b;
@@ -112,7 +114,8 @@ int main(int argc, char **argv)
     memset(status, 0, sizeof(status));
     total = -7;                                                  // not cleared by anybody
     for (int i = 0; i < WGS; i++) publish(i);
-    if (when == 0) {                                             // nobody gives up
+    if (when == 0) {                                             // nobody gives up, whatever lay in the total's place
+        if (late) total = CAPACITY + 1;
         for (int i : {0, 1, 2, 62, 63, 64, 65, 126, 127, 128, 148, 149}) CHECK(run(i) == before(i));
         CHECK(status[0] == 0 && total == before(WGS));
         return 0;
@@ -125,7 +128,8 @@ int main(int argc, char **argv)
     auto once = [&](void *p, bool st, void *at, bool want) { return p == at && st == want && times++ == 0; };
     if (when == 1) run(last);
     if (when == 2) { run(last); give_up(late); }                 // after it
-    if (when == 3) {                                             // between its total and its look at the flag
+    if (when == 3) {                                             // another before it, this one between its total and its look at the flag
+        give_up(late == 40 ? 41 : 40);
         on_access = [&](void *p, bool st) { if (once(p, st, status, false)) give_up(late); };
         run(last);
         CHECK(times > 0);
@@ -169,8 +173,9 @@ def _go(program, when, late):
     assert r.returncode == 0, r.stdout + r.stderr
 
 
-def test_places(program):
-    _go(program, 0, 0)
+@pytest.mark.parametrize("past", [0, 1])
+def test_places(program, past):
+    _go(program, 0, past)
 
 
 @pytest.mark.parametrize("when", [1, 2, 3, 4, 5])

@@ -33,13 +33,13 @@ __device__ __forceinline__ void chain_publish(unsigned long long *words, int wg,
 }
 
 // `*total`, the rows of the whole launch, as its last workgroup knows them (one lane); past the capacity if a workgroup gave up
-// waiting.  That may happen before, during or after this: whoever gives up raises the flag first and the total then, and here
-// the total comes first and the look at the flag then, so one of the two stores past the capacity is the last.
+// waiting.  Whoever does raises the flag, then stores capacity + 1 in the total's place: behind this it stays, and before this
+// the exchange brings it back.  (What else may have lain there is told by the flag.)  One trip to memory where all went well: a store
+// that has to be there before a look at the flag would be two.
 __device__ __forceinline__ void chain_total(unsigned long long *status, int64_t *total, int64_t rows, int64_t capacity)
 {
-    chain_store(total, rows);
-    chain_stored();
-    if (chain_load(status) != 0 && rows <= capacity) chain_store(total, capacity + 1);
+    const int64_t was = __hip_atomic_exchange(total, rows, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (was == capacity + 1 && rows <= capacity && chain_load(status) != 0) chain_store(total, capacity + 1);
 }
 
 // The queries of all workgroups before `wg`, whose own are `agg`.  One wave, the value in every lane; `capacity`, with *total past
