@@ -1151,9 +1151,12 @@ template <typename T> static int launch_backward(AttnBack a, int max_rows, hipSt
     a.search = qc >= 2 && a.n >= 128 && pairs_x <= AB_SEARCH && a.pairs * qc > compute_units() && has_holes(a.L, a.pairs, a.h, qc);
     // fp32 on the bf16 instructions: from 161 keys on, where live workgroups are about as many as compute units.  Us, both kernels, fp32 /
     // bf16 instructions (samples, heads, keys): 64, 3, 257: 106.6 / 74.2; 64, 6, 257: 177.7 / 122.1; 128, 6, 257: 321 / 231; 16, 3, 1025: 376 /
-    // 224.  With fewer, one wave a SIMD waits for its own vector instructions, of which the split has more: 16, 6, 257 (212 of them) 63.7 /
-    // 60.2, 8, 3, 257 (38) 44.4 / 44.4, less than the rest of a training pass waits.  Both kernels or neither, and with 1 / s to carry
-    // the marks: scores of another order of sums than those that m and s are of would be off where they are large.
+    // 224.  With fewer, one wave a SIMD waits for its own vector instructions, of which the split has more, and gains less; out of a replayed
+    // graph, by live workgroups: 12: 35.9 / 34.6, 54: 39.4 / 37.0, 109: 40.7 / 38.0, 215: 49.2 / 44.5, 431: 86.8 / 65.3; of 161 keys 70: 30.0 /
+    // 29.1, 208: 36.9 / 35.6; of 1025 keys 38: 141 / 121, 89: 177 / 135, 180: 180 / 145, 357: 316 / 204.  The line is not where its
+    // lead ends but where it is a fifth and more (322, 257 keys: 72.3 / 55.9); one further down would be sound too.  Both kernels or
+    // neither, and with 1 / s to carry the marks: scores of another order of sums than those that m and s are of would be off where
+    // they are large.
     const bool split = sizeof(T) == 4 && a.inv != nullptr && a.n > 5 * AB_ROWS && live_chunks(a.L, a.pairs, a.h) >= compute_units();
     a.by_chunk = sizeof(T) == 4 ? !split : 32 % kc == 0 && (a.n - 1) % (16 * AB_WAVES) < 8 * AB_WAVES;
     if (qc > 0) {

@@ -104,7 +104,7 @@ NATIVE_CHAIN = True
 # of a compute unit's LDS there, so that `patch_write` waits for its first workgroups and takes 14 us, not 10), 4885 against 4825
 # (128), 3110 against 3016 (128, PVT-Small), 5052 against 4946 (256).  From the line to some 16 M values it depends on the
 # model: 2402 against 2353 (24 of 384 px, PVT-Tiny fp32), but 1580 against 1589 (12), 1673 against 1725 (32, PVT-Small) and,
-# where few regions route the next block in their scatter-back (`vtdge_region_step`) so that only the first block forks, 1445
+# where the scatter-back routes and packs the next block (`vtdge_region_step`) so that only the first block forks, 1445
 # against 1497 (12, 768 channels), 2849 against 2872 (64) and 2690 against 2716 (128, 192 channels fp32).
 OVERLAP_FROM = 2 << 20
 _SWITCHES = ("OVERLAP", "FUSE_NEXT_NORM", "FUSE_ROUTER_NORM", "FUSE_NEXT_ROUTER", "FOLD_NORMS", "FUSE_PATCH_EMBED",
